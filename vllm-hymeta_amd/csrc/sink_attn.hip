@@ -8,6 +8,8 @@
 // Rows of HYMETA_KV_SCALED_KEY hold ONE vector per key/value head that is both: the projected key, which is the value,
 // and its inverse root mean square, by which the score of the normed key differs from the score of the stored one (the
 // norm's weight rides in the queries).  A page then holds half of what keys and values apart would take.
+#include <algorithm>
+
 #include "act_types.h"
 
 namespace hymeta {
@@ -266,13 +268,10 @@ __device__ __forceinline__ f32x4v mfma16(bf16x8 a, bf16x8 b, f32x4v c) {
 constexpr int kTileKeys = 64;
 constexpr int kRowsPerWave = 32;
 
-// The value columns one launch computes: `first` .. `first` + DV of the `total` columns of a value row (and of an output
-// row).  Values wider than the kernels' DV run as several launches over slices (each repeats the scores).
-struct ValueSlice {
-  int first, total;
-  // (decode form) the query heads of a key/value head one launch takes as its rows: h_first .. h_first + h_count of the
-  // group; h_count 0: the whole group.  Groups of more than 32 heads run as several launches.
-  int h_first = 0, h_count = 0;
+// (decode form) the query heads of a key/value head one launch takes as its rows: first .. first + count of the group;
+// count 0: the whole group.  Groups of more than 32 heads run as several launches.
+struct HeadSlice {
+  int first = 0, count = 0;
 };
 
 template <int D, int DV>
@@ -307,7 +306,7 @@ struct TileStage {
   u32x4 rk[Scaled ? 1 : kKeyPerThread];
   u32x4 rv[4];
   float rs = 0.f;               // (SCALED_KEY) the scale of key j0 + threadIdx.x
-  int value_at = kValueAt;      // where the staged value columns start in a head's part of a row
+  int value_at = kValueAt;      // where the value starts in a head's part of a row
 
   // Pages hold a power of two of rows here (the host sends other sizes to the plain kernel).  A page of 64 rows or more
   // holds a whole tile (tiles start at multiples of 64): its number is one scalar load per tile, not a dependent vector
@@ -571,15 +570,15 @@ __device__ __forceinline__ void load_bias(WaveRows<D, DV, RB>& w, int rb, const 
 }
 
 // Waves of a prompt workgroup: 8, or 4 for keys longer than 192 elements, whose query fragments (D / 8 registers) and
-// staging registers do not leave a wave of 8 its accumulators within 256 registers (408 bytes of scratch per lane at
-// 576; a workgroup of 4 waves has 512 registers per wave).
+// staging registers do not leave a wave of 8 its accumulators within 256 registers (a workgroup of 4 waves has 512
+// registers per wave).
 template <int D> struct PrefillWaves { static constexpr int value = D > 192 ? 4 : 8; };
 template <int RB, int Waves> struct PrefillShape { static constexpr int kRows = 16 * RB * Waves; };
 
 // Portions of prompts: grid = (tiles of 16 RB rows per wave, heads, sequences); a wave holds RB blocks of 16 rows; sequences with
 // one row are left to the decode form.
 template <int D, int DV, int RB, int Layout>
-__global__ __launch_bounds__(64 * PrefillWaves<D>::value) void sink_attention_prefill_mfma_kernel(hymeta_sink_attention_args a, ValueSlice vs) {
+__global__ __launch_bounds__(64 * PrefillWaves<D>::value) void sink_attention_prefill_mfma_kernel(hymeta_sink_attention_args a) {
   constexpr int kPrefillWaves = PrefillWaves<D>::value;
   constexpr int kRows = PrefillShape<RB, kPrefillWaves>::kRows;
   constexpr int kImages = 2 * sizeof(MfmaSmem<D, DV>) <= 159 * 1024 ? 2 : 1;        // (160 KB of LDS)
@@ -625,7 +624,6 @@ __global__ __launch_bounds__(64 * PrefillWaves<D>::value) void sink_attention_pr
   // two LDS images: while the waves multiply tile t out of one, tile t + 1 goes into the other and the loads of tile
   // t + 2 are in flight; one barrier per tile
   TileStage<D, DV, 64 * kPrefillWaves, Layout> stage;
-  if (Layout == HYMETA_KV_VALUE_IN_KEY) stage.value_at = vs.first;
   if (Layout == HYMETA_KV_SHARED_KEY) stage.value_at = D + g * DV;
   stage.issue(a, bt, g, j_start, block_last);
   stage.commit(sm[0], s_scale[0]);
@@ -670,13 +668,13 @@ __global__ __launch_bounds__(64 * PrefillWaves<D>::value) void sink_attention_pr
     if (r >= q) continue;
     float inv = l > 0.f ? 1.f / l : 0.f;
     if (a.head_gate) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[static_cast<int64_t>(row0 + r) * a.head_gate_stride_t + h]));
-    uint16_t* out = static_cast<uint16_t*>(a.out) + (static_cast<int64_t>(row0 + r) * a.num_heads + h) * vs.total + vs.first;
+    uint16_t* out = static_cast<uint16_t*>(a.out) + (static_cast<int64_t>(row0 + r) * a.num_heads + h) * DV;
 #pragma unroll
     for (int cb = 0; cb < DV / 16; ++cb) {
       f32x4v o = w.o[rb][cb] * inv;
       if (a.elem_gate) {
         float gate[4];
-        ActBf16::ld4(static_cast<const uint16_t*>(a.elem_gate) + static_cast<int64_t>(row0 + r) * a.elem_gate_stride_t + static_cast<int64_t>(h) * vs.total + vs.first + 16 * cb + 4 * g4, gate);
+        ActBf16::ld4(static_cast<const uint16_t*>(a.elem_gate) + static_cast<int64_t>(row0 + r) * a.elem_gate_stride_t + static_cast<int64_t>(h) * DV + 16 * cb + 4 * g4, gate);
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] *= ActBf16::sigmoid(gate[e]);
       }
@@ -708,7 +706,7 @@ struct DecodeMerge {
 // four waves share the staged tiles and take a 16-key subtile each.  Every wave writes its (maximum, denominator,
 // weighted values) per head; the combine kernel merges them and the sink.
 template <int D, int DV, int RB, int Layout>
-__global__ __launch_bounds__(64 * kDecodeWaves) void sink_attention_decode_mfma_kernel(hymeta_sink_attention_args a, int splits, int tiles_per_split, ValueSlice vs) {
+__global__ __launch_bounds__(64 * kDecodeWaves) void sink_attention_decode_mfma_kernel(hymeta_sink_attention_args a, int splits, int tiles_per_split, HeadSlice hs) {
   constexpr int kImages = DecodeImages<D, DV>::value;
   constexpr bool kScaled = Layout == HYMETA_KV_SCALED_KEY;
   __shared__ MfmaSmem<D, DV> sm[kImages];
@@ -727,7 +725,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves) void sink_attention_decode_mfma_
   if (a.query_start_loc[s + 1] - t != 1) return;
   const int pos = a.seq_lens[s] - 1;
   const int group = a.num_heads / a.num_kv_heads;
-  const int HG = vs.h_count ? vs.h_count : group;            // this launch's rows
+  const int HG = hs.count ? hs.count : group;            // this launch's rows
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g4 = lane >> 4;
   // The sequence's tiles, numbered v = 0 ..: without a window tile v holds the keys from 64 v on, split as the host says.
   // With a window: the tiles of the kept first keys that lie before the window's first tile, then the window's tiles
@@ -752,7 +750,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves) void sink_attention_decode_mfma_
   for (int rb = 0; rb < RB; ++rb) {
     const int r = 16 * rb + n;
     const bool ok = r < HG;
-    const int h = g * group + vs.h_first + (ok ? r : 0);
+    const int h = g * group + hs.first + (ok ? r : 0);
     w.pos[rb] = ok ? pos : -1;
     w.first[rb] = first;
     load_bias<D, DV, RB>(w, rb, a, h);
@@ -763,7 +761,6 @@ __global__ __launch_bounds__(64 * kDecodeWaves) void sink_attention_decode_mfma_
     for (int cb = 0; cb < DV / 16; ++cb) w.o[rb][cb] = f32x4v{0.f, 0.f, 0.f, 0.f};
   }
   TileStage<D, DV, 64 * kDecodeWaves, Layout> stage;
-  if (Layout == HYMETA_KV_VALUE_IN_KEY) stage.value_at = vs.first;
   if (Layout == HYMETA_KV_SHARED_KEY) stage.value_at = D + g * DV;
   if (v_lo <= v_hi) {
     stage.issue(a, bt, g, tile(v_lo), pos);
@@ -854,51 +851,94 @@ __global__ __launch_bounds__(64 * kDecodeWaves) void sink_attention_decode_mfma_
   }
 }
 
-// grid = (sequences, heads), 64 threads: merge the slices of a decode row, add the sink, normalise, store bf16.
-__global__ __launch_bounds__(64) void sink_attention_decode_combine_kernel(hymeta_sink_attention_args a, int splits, ValueSlice vs) {
+// grid = (sequences, heads): merge the partials of a decode row, add the sink, normalise, store bf16.  Two round trips to
+// memory: the threads read the partials' statistics side by side (one each), agree on the row's maximum, and leave every
+// partial's factor in LDS; then groups of v_dim / 4 threads take the partials in turn, four columns a thread.  (As one
+// serial loop over the partials per column and statistic the launch took 11 us at 4 partials of 128 columns; now 6 at
+// 4 partials of 512.)
+constexpr int kCombineThreads = 128;
+constexpr int kMaxPartials = 512 * kDecodeWaves;
+
+__global__ __launch_bounds__(kCombineThreads) void sink_attention_decode_combine_kernel(hymeta_sink_attention_args a, int splits, HeadSlice hs) {
   // (splits: partials per (sequence, key/value head): one per slice, or one per wave of a slice)
+  __shared__ float s_f[kMaxPartials];
+  __shared__ float s_red[2][kCombineThreads / 64];
+  __shared__ __attribute__((aligned(16))) f32x4v s_acc[kCombineThreads];
   const int s = blockIdx.x;
   const int t = a.query_start_loc[s];
   if (a.query_start_loc[s + 1] - t != 1) return;
-  const int group = a.num_heads / a.num_kv_heads, HG = vs.h_count ? vs.h_count : group;
-  const int g = blockIdx.y / HG, r = blockIdx.y % HG, h = g * group + vs.h_first + r, DV = a.v_dim;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int group = a.num_heads / a.num_kv_heads, HG = hs.count ? hs.count : group;
+  const int g = blockIdx.y / HG, r = blockIdx.y % HG, h = g * group + hs.first + r, DV = a.v_dim;
   const size_t stride = HG * partial_row_floats(DV);
   const float* base = static_cast<const float*>(a.workspace) + (static_cast<size_t>(s) * a.num_kv_heads + g) * splits * stride +
                       r * partial_row_floats(DV);
   // (the partials' maxima are in the base-2 domain, as the waves kept them)
   const float sink2 = a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f;
   float m = a.sink ? sink2 : -INFINITY;
-  for (int sp = 0; sp < splits; ++sp) m = fmaxf(m, base[sp * stride + DV]);
-  float l = a.sink ? __builtin_amdgcn_exp2f(sink2 - m) : 0.f;
-  for (int sp = 0; sp < splits; ++sp) {
+  for (int sp = tid; sp < splits; sp += kCombineThreads) {
     const float ms = base[sp * stride + DV];
-    if (ms != -INFINITY) l += base[sp * stride + DV + 1] * __builtin_amdgcn_exp2f(ms - m);
+    s_f[sp] = ms;
+    m = fmaxf(m, ms);
   }
+  m = wave_max(m);
+  if (lane == 0) s_red[0][wave] = m;
+  __syncthreads();
+  m = fmaxf(s_red[0][0], s_red[0][1]);
+  float l = 0.f;
+  for (int sp = tid; sp < splits; sp += kCombineThreads) {      // (each thread's own entries of s_f)
+    const float f = s_f[sp] == -INFINITY ? -1.f : __builtin_amdgcn_exp2f(s_f[sp] - m);      // (-1: a partial without keys)
+    s_f[sp] = f;
+    if (!(f < 0.f)) l = fmaf(base[sp * stride + DV + 1], f, l);
+  }
+  l = wave_sum(l);
+  if (lane == 0) s_red[1][wave] = l;
+  __syncthreads();
+  l = (s_red[1][0] + s_red[1][1]) + (a.sink ? __builtin_amdgcn_exp2f(sink2 - m) : 0.f);
   float inv = l > 0.f ? 1.f / l : 0.f;
   if (a.head_gate) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[static_cast<int64_t>(t) * a.head_gate_stride_t + h]));
-  uint16_t* out = static_cast<uint16_t*>(a.out) + (static_cast<int64_t>(t) * a.num_heads + h) * vs.total + vs.first;
-  for (int c = threadIdx.x; c < DV; c += 64) {
-    float acc = 0.f;
-    for (int sp = 0; sp < splits; ++sp) {
-      const float ms = base[sp * stride + DV];
-      if (ms != -INFINITY) acc += base[sp * stride + c] * __builtin_amdgcn_exp2f(ms - m);
+  const int quads = DV / 4, turns = kCombineThreads / quads, turn = tid / quads, c = 4 * (tid % quads);
+  f32x4v acc = f32x4v{0.f, 0.f, 0.f, 0.f};
+  if (turn < turns) {
+#pragma unroll 4
+    for (int sp = turn; sp < splits; sp += turns) {
+      const float f = s_f[sp];
+      if (!(f < 0.f)) acc += *reinterpret_cast<const f32x4v*>(base + sp * stride + c) * f;
     }
-    acc *= inv;
-    if (a.elem_gate)
-      acc *= ActBf16::sigmoid(bf2f(static_cast<const uint16_t*>(a.elem_gate)[static_cast<int64_t>(t) * a.elem_gate_stride_t + static_cast<int64_t>(h) * vs.total + vs.first + c]));
-    out[c] = f2bf(acc);
   }
+  if (turns > 1) {
+    s_acc[tid] = acc;
+    __syncthreads();
+    if (turn == 0)
+      for (int k = 1; k < turns; ++k) acc += s_acc[tid + k * quads];
+  }
+  if (turn != 0) return;
+  acc *= inv;
+  if (a.elem_gate) {
+    float gate[4];
+    ActBf16::ld4(static_cast<const uint16_t*>(a.elem_gate) + static_cast<int64_t>(t) * a.elem_gate_stride_t + static_cast<int64_t>(h) * DV + c, gate);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] *= ActBf16::sigmoid(gate[e]);
+  }
+  *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.out) + (static_cast<int64_t>(t) * a.num_heads + h) * DV + c) =
+      u32x2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
 }
 
+}  // namespace
+}  // namespace hymeta
+
+#include "wide_latent.h"
+
+namespace hymeta {
+namespace {
+
 // Head sizes the matrix-core kernels are built for.  A value inside its key: a latent of 64 or 128 followed by a rotated
-// part of 32 or 64, or a latent of 256 / 384 / 512 followed by a rotated part of 64, which runs as 2 / 3 / 4 launches
-// over value slices of 128 (each repeats the scores over the whole key: 1.5 to 2.1 times the matrix work of one pass
-// with accumulators for all the value columns, which do not fit a wave's registers beside the query fragments).
+// part of 32 or 64 (the kernels above), or a latent of 256 / 384 / 512 followed by a rotated part of 64 (wide_latent.h).
 inline bool mfma_shape(const hymeta_sink_attention_args& a) {
   bool dims = (a.head_dim == 64 || a.head_dim == 128) && (a.v_dim == 64 || a.v_dim == 128);
   if (a.kv_layout == HYMETA_KV_VALUE_IN_KEY)
     dims = ((a.v_dim == 64 || a.v_dim == 128) && (a.head_dim == a.v_dim + 32 || a.head_dim == a.v_dim + 64)) ||
-           ((a.v_dim == 256 || a.v_dim == 384 || a.v_dim == 512) && a.head_dim == a.v_dim + 64);      // (in value slices of 128)
+           ((a.v_dim == 256 || a.v_dim == 384 || a.v_dim == 512) && a.head_dim == a.v_dim + 64);
   // one key for all heads: the concatenated keys of 1 / 2 / 4 / 8 key/value heads of 64 or 128
   if (a.kv_layout == HYMETA_KV_SHARED_KEY)
     dims = (a.head_dim == 64 || a.head_dim == 128 || a.head_dim == 256 || a.head_dim == 512) && (a.v_dim == 64 || a.v_dim == 128);
@@ -913,49 +953,70 @@ inline bool mfma_shape(const hymeta_sink_attention_args& a) {
          (reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.kv_cache) | reinterpret_cast<uintptr_t>(a.out)) % 16 == 0;
 }
 
-// span > 0 (a window's or a chunk's keys): a row reads the kept first keys' tiles and the span's, however long the sequence is.
-inline int decode_splits(int num_seqs, int num_heads, int num_kv_heads, int max_seq_len, int64_t span = 0, int keep_first = 0) {
-  int tiles = (max_seq_len + kTileKeys - 1) / kTileKeys;
-  if (span > 0) {
-    const int64_t seen = (static_cast<int64_t>(keep_first) + kTileKeys - 1) / kTileKeys + (span - 1) / kTileKeys + 2;
-    if (seen < tiles) tiles = static_cast<int>(seen);
-  }
+// Tiles of 64 keys a decode row reads at most: all of its sequence's, or with a window or a chunk the kept first keys' and
+// that span's, however long the sequence is.
+inline int decode_tiles(int max_seq_len, int64_t span = 0, int keep_first = 0) {
+  const int tiles = (max_seq_len + kTileKeys - 1) / kTileKeys;
+  if (span <= 0) return tiles;
+  const int64_t seen = (static_cast<int64_t>(keep_first) + kTileKeys - 1) / kTileKeys + (span - 1) / kTileKeys + 2;
+  return static_cast<int>(std::min<int64_t>(seen, tiles));
+}
+inline int decode_tiles(const hymeta_sink_attention_args& a) {
+  return decode_tiles(a.max_seq_len, a.chunk > 0 ? a.chunk : static_cast<int64_t>(a.window_left) + 1, a.keep_first);
+}
+
+inline int decode_splits(int num_seqs, int num_heads, int num_kv_heads, int tiles) {
   // Workgroups aimed at: a workgroup's fixed cost (query fragments, first tile, the merge of its waves, its partial) grows
   // with the query heads it carries, so fewer, longer workgroups pay.  Measured at 64 sequences x 4096 keys: 28 heads on
   // one row of 192: 93 / 67 / 56 / 87 us at 1024 / 512 / 256 / 128; 16 heads on it: 53 / 40 / 45; 4 key/value heads with
   // 7 query heads each: 125 / 114 / 168.
   const int target = num_heads / num_kv_heads > 16 ? 256 : 512;
-  int splits = (target + num_seqs * num_kv_heads - 1) / (num_seqs * num_kv_heads);
-  splits = splits < 1 ? 1 : splits;
-  return splits > tiles ? (tiles < 1 ? 1 : tiles) : splits;
+  const int splits = (target + num_seqs * num_kv_heads - 1) / (num_seqs * num_kv_heads);
+  return std::max(1, std::min(splits, tiles));
+}
+
+template <int C>
+int launch_wide_latent(const hymeta_sink_attention_args& a, hipStream_t st) {
+  const int group = a.num_heads / a.num_kv_heads;
+  if (a.max_query_len > 1) {
+    const int64_t rows = static_cast<int64_t>(a.max_query_len) * group;
+    const dim3 grid(static_cast<uint32_t>((rows + kWideRows - 1) / kWideRows), a.num_kv_heads, a.num_seqs);
+    hipLaunchKernelGGL((latent_prefill_kernel<C>), grid, dim3(64 * kWideWaves), 0, st, a);
+  }
+  // one workgroup per compute unit (its rings fill the LDS): as many as there are units
+  const int64_t slices = (group + kLatentHeads - 1) / kLatentHeads, items = static_cast<int64_t>(a.num_seqs) * a.num_kv_heads;
+  const int splits = static_cast<int>(std::min<int64_t>((256 + items * slices - 1) / (items * slices), decode_tiles(a)));
+  const dim3 grid(static_cast<uint32_t>((items * splits + 7) / 8 * 8 * slices));
+  hipLaunchKernelGGL((latent_decode_kernel<C>), grid, dim3(64 * kLatentWaves), 0, st, a, splits);
+  hipLaunchKernelGGL(sink_attention_decode_combine_kernel, dim3(a.num_seqs, a.num_heads), dim3(kCombineThreads), 0, st, a, splits, HeadSlice{});
+  return launch_status();
 }
 
 template <int D, int DV, int Layout = HYMETA_KV_KEY_THEN_VALUE>
-int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st, ValueSlice vs = ValueSlice{0, DV, 0, 0}) {
+int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st) {
   if (a.max_query_len > 1) {
     constexpr int kRB = PREFILL_RB;
     constexpr int kRows = PrefillShape<kRB, PrefillWaves<D>::value>::kRows;
     const dim3 grid((a.max_query_len + kRows - 1) / kRows, a.num_heads, a.num_seqs);
-    hipLaunchKernelGGL((sink_attention_prefill_mfma_kernel<D, DV, kRB, Layout>), grid, dim3(64 * PrefillWaves<D>::value), 0, st, a, vs);
+    hipLaunchKernelGGL((sink_attention_prefill_mfma_kernel<D, DV, kRB, Layout>), grid, dim3(64 * PrefillWaves<D>::value), 0, st, a);
   }
   // sequences with a single row: every step but a pure prompt step has some; a prompt of one token is one too
-  const int splits = decode_splits(a.num_seqs, a.num_heads, a.num_kv_heads, a.max_seq_len, a.chunk > 0 ? a.chunk : static_cast<int64_t>(a.window_left) + 1, a.keep_first);
+  const int splits = decode_splits(a.num_seqs, a.num_heads, a.num_kv_heads, decode_tiles(a));
   const int tiles = (a.max_seq_len + kTileKeys - 1) / kTileKeys;
   const int tiles_per_split = (tiles + splits - 1) / splits;
   const dim3 grid = Layout == HYMETA_KV_SHARED_KEY ? dim3((splits * a.num_seqs + 7) / 8 * 8 * a.num_kv_heads) : dim3(splits, a.num_kv_heads, a.num_seqs);
   const int group = a.num_heads / a.num_kv_heads;
   for (int first = 0; first < group; first += kRowsPerWave) {
-    vs.h_first = first;
-    vs.h_count = group - first < kRowsPerWave ? group - first : kRowsPerWave;
+    const HeadSlice hs{first, group - first < kRowsPerWave ? group - first : kRowsPerWave};
     int parts;
-    if (vs.h_count <= 16) {
-      hipLaunchKernelGGL((sink_attention_decode_mfma_kernel<D, DV, 1, Layout>), grid, dim3(64 * kDecodeWaves), 0, st, a, splits, tiles_per_split, vs);
+    if (hs.count <= 16) {
+      hipLaunchKernelGGL((sink_attention_decode_mfma_kernel<D, DV, 1, Layout>), grid, dim3(64 * kDecodeWaves), 0, st, a, splits, tiles_per_split, hs);
       parts = splits * (DecodeMerge<D, DV, 1>::value ? 1 : kDecodeWaves);
     } else {
-      hipLaunchKernelGGL((sink_attention_decode_mfma_kernel<D, DV, 2, Layout>), grid, dim3(64 * kDecodeWaves), 0, st, a, splits, tiles_per_split, vs);
+      hipLaunchKernelGGL((sink_attention_decode_mfma_kernel<D, DV, 2, Layout>), grid, dim3(64 * kDecodeWaves), 0, st, a, splits, tiles_per_split, hs);
       parts = splits * (DecodeMerge<D, DV, 2>::value ? 1 : kDecodeWaves);
     }
-    hipLaunchKernelGGL(sink_attention_decode_combine_kernel, dim3(a.num_seqs, a.num_kv_heads * vs.h_count), dim3(64), 0, st, a, parts, vs);
+    hipLaunchKernelGGL(sink_attention_decode_combine_kernel, dim3(a.num_seqs, a.num_kv_heads * hs.count), dim3(kCombineThreads), 0, st, a, parts, hs);
   }
   return launch_status();
 }
@@ -1015,7 +1076,7 @@ extern "C" int hymeta_scaled_key_cache(const hymeta_scaled_key_cache_args* args,
 extern "C" size_t hymeta_sink_attention_workspace_bytes(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads, int32_t v_dim,
                                                         int32_t max_seq_len) {
   if (num_seqs <= 0 || num_heads <= 0 || num_kv_heads <= 0 || v_dim <= 0) return 0;
-  const int splits = decode_splits(num_seqs, num_heads, num_kv_heads, max_seq_len < 1 ? 1 : max_seq_len);
+  const int splits = decode_splits(num_seqs, num_heads, num_kv_heads, decode_tiles(max_seq_len < 1 ? 1 : max_seq_len));
   return static_cast<size_t>(num_seqs) * splits * kDecodeWaves * num_heads * partial_row_floats(v_dim) * sizeof(float);
 }
 
@@ -1048,15 +1109,7 @@ extern "C" int hymeta_sink_attention(const hymeta_sink_attention_args* args, hym
     if (a.kv_layout == HYMETA_KV_VALUE_IN_KEY) {
       if (a.v_dim == 64) return a.head_dim == 96 ? launch_mfma<96, 64, HYMETA_KV_VALUE_IN_KEY>(a, st) : launch_mfma<128, 64, HYMETA_KV_VALUE_IN_KEY>(a, st);
       if (a.v_dim == 128) return a.head_dim == 160 ? launch_mfma<160, 128, HYMETA_KV_VALUE_IN_KEY>(a, st) : launch_mfma<192, 128, HYMETA_KV_VALUE_IN_KEY>(a, st);
-      hymeta_sink_attention_args b = a;
-      b.v_dim = 128;
-      for (int first = 0; first < a.v_dim; first += 128) {
-        const ValueSlice vs{first, a.v_dim, 0, 0};
-        const int rc = a.v_dim == 256 ? launch_mfma<320, 128, HYMETA_KV_VALUE_IN_KEY>(b, st, vs) : a.v_dim == 384 ? launch_mfma<448, 128, HYMETA_KV_VALUE_IN_KEY>(b, st, vs)
-                                                                                                 : launch_mfma<576, 128, HYMETA_KV_VALUE_IN_KEY>(b, st, vs);
-        if (rc != HYMETA_OK) return rc;
-      }
-      return HYMETA_OK;
+      return a.v_dim == 256 ? launch_wide_latent<256>(a, st) : a.v_dim == 384 ? launch_wide_latent<384>(a, st) : launch_wide_latent<512>(a, st);
     }
     if (a.kv_layout == HYMETA_KV_SCALED_KEY) {
       constexpr int kScaled = HYMETA_KV_SCALED_KEY;
