@@ -1194,7 +1194,8 @@ int hymeta_qk_norm_cache(const hymeta_qk_norm_cache_args* args, hymeta_stream_t 
  *   out_i = sum_j p_ij v_j
  * Scores and weights are fp32 in both activation types.  Query row t of sequence s stands at position
  * seq_lens[s] - (query_start_loc[s + 1] - t).  bf16 rows with head_dim and v_dim of 64 or 128 run on the
- * matrix cores: portions of prompts in tiles of 128 rows, sequences with one row (decode) per key/value
+ * matrix cores: portions of prompts in blocks of 128 (query, head) rows, short portions with their keys cut into slices as
+ * the workspace allows, sequences with one row (decode) per key/value
  * head with its query heads (32 to a launch), split over the keys into `workspace`
  * (hymeta_sink_attention_workspace_bytes) and merged by a second launch.
  * max_query_len / max_seq_len: upper bounds of the step's portion and sequence lengths (they size the
@@ -1248,6 +1249,11 @@ typedef struct hymeta_sink_attention_args {
 } hymeta_sink_attention_args;
 size_t hymeta_sink_attention_workspace_bytes(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads, int32_t v_dim,
                                              int32_t max_seq_len);
+/* The most a call whose longest portion has max_query_len > 1 rows can use for them: the keys of short portions are cut into
+ * slices.  span: the keys a row sees before keep_first, by a window (window_left + 1) or a chunk, 0: all.  With less, but at
+ * least the above, the call cuts them into fewer. */
+size_t hymeta_sink_attention_portion_workspace_bytes(int32_t num_tokens, int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads, int32_t v_dim,
+                                                     int32_t max_query_len, int32_t max_seq_len, int64_t span, int32_t keep_first);
 int hymeta_sink_attention(const hymeta_sink_attention_args* args, hymeta_stream_t stream);
 
 /* Mixture of experts whose choice is a table lookup by token id: table [vocab, top_k] names each

@@ -1,0 +1,107 @@
+"""Prompts' portions of the paged attention, keys of 32 to 192 elements in every layout of a cache row, at the edges of the
+kernel's tiles: 32 (query, head) rows a wave and 128 a workgroup, 64 keys a tile, pages that hold a tile and pages that do not,
+and portions short enough that their keys are cut into slices (more than 4 tiles a slice).
+
+Bound: the outputs are bf16 (2^-9 of each value at most); the weights are two bf16 parts (2^-17), exponentials, logarithms and
+products fp32 (below 2^-11 over these lengths and biases); together below 2^-9 + 2^-10 in the norm."""
+from itertools import accumulate
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BOUND = 2.0 ** -9 + 2.0 ** -10
+SLOPE, NEAR = 0.03, 0.25
+
+
+def reference(q, k, v, scale, ctx, o, sink, a, gate):
+    """One sequence in 64 bits: q [n, H, D] at positions ctx .., k [H, ctx + n, D], v [H, ctx + n, Dv]."""
+    n = q.shape[0]
+    i, j = torch.arange(ctx, ctx + n)[:, None], torch.arange(ctx + n)
+    seen = j <= i
+    if o["chunk"]:
+        seen = seen & (j >= i // o["chunk"] * o["chunk"])
+    elif o["window"]:
+        seen = seen & ((j > i - o["window"]) | (j < o["keep"]))
+    s = torch.einsum("nhd,hjd->hnj", q, k) * scale
+    if o["softcap"]:
+        s = o["softcap"] * torch.tanh(s / o["softcap"])
+    far = (i - j).clamp_min(0).double()
+    if o["bias"] == "log":
+        s = s - a[:, None, None] * torch.log1p(NEAR * far)
+    elif o["bias"] == "linear":
+        s = s - SLOPE * a[:, None, None] * far
+    s = s.masked_fill(~seen, float("-inf"))
+    if sink is not None:
+        s = torch.cat((s, sink[:, None, None].expand(len(sink), n, 1)), -1)
+    out = torch.einsum("hnj,hjc->nhc", torch.softmax(s, -1)[..., :ctx + n], v)
+    return out if gate is None else out * torch.sigmoid(gate)[:, :, None]
+
+
+@pytest.mark.parametrize("layout,D,Dv,H,G,page,lens,ctxs,opts", [
+    ("rows", 128, 128, 28, 4, 64, [18, 2, 19], [0, 64, 700], dict(sink=True, bias="log")),       # 126, 14 and 133 rows
+    ("rows", 128, 64, 4, 1, 16, [32, 33, 1], [31, 0, 70], dict(softcap=4.0)),                    # small pages
+    ("rows", 64, 128, 2, 2, 64, [129, 64], [1, 512], dict(window=70, keep=9)),                   # one head a key/value head, kept keys
+    ("rows", 64, 64, 6, 2, 128, [5, 3], [1000, 2000], dict(chunk=300, gate=True)),
+    ("rows", 128, 128, 8, 2, 64, [3, 2], [3000, 63], dict(softcap=6.0, bias="log", sink=True)),  # slices, of which some see nothing
+    ("latent", 192, 128, 16, 1, 64, [8, 9, 2], [0, 63, 1500], dict(sink=True)),
+    ("latent", 160, 128, 5, 1, 32, [70], [11], dict(bias="log")),
+    ("latent", 128, 64, 3, 1, 64, [90, 2], [0, 900], dict(window=200)),
+    ("latent", 96, 64, 7, 1, 8, [40, 64], [5, 64], dict(sink=True)),
+    ("shared", 128, 64, 4, 2, 64, [50, 2], [14, 800], dict(window=100, keep=4)),
+    ("shared", 64, 128, 4, 4, 64, [65], [64], {}),
+    ("scaled", 128, 128, 28, 4, 64, [20, 2], [0, 1200], dict(sink=True, bias="linear")),
+    ("scaled", 96, 96, 4, 2, 16, [33, 70], [100, 0], dict(bias="linear", window=50)),
+    ("scaled", 64, 64, 4, 1, 64, [64], [64], dict(sink=True)),
+    ("scaled", 32, 32, 3, 3, 64, [10, 11], [700, 0], dict(bias="linear")),
+])
+def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
+    from vllm_hymeta import hip_ops
+    dev, g = "cuda", torch.Generator().manual_seed(D + H)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
+    o = dict(dict(sink=False, window=0, keep=0, chunk=0, softcap=0.0, bias=None, gate=False), **opts)
+    key_heads = 1 if layout in ("latent", "shared") else G
+    total = [n + c for n, c in zip(lens, ctxs)]
+    keys = [torch.randn(t, key_heads, D, generator=g).bfloat16() for t in total]
+    values = [k[:, :, :Dv] if layout in ("latent", "scaled") else torch.randn(len(k), G, Dv, generator=g).bfloat16() for k in keys]
+    q = [torch.randn(n, H, D, generator=g).bfloat16() for n in lens]
+    sink = torch.randn(H, generator=g) if o["sink"] else None
+    a = 0.1 + torch.rand(H, generator=g)
+    gates = [torch.randn(n, H, generator=g).bfloat16() if o["gate"] else None for n in lens]
+    need = [(t + page - 1) // page for t in total]
+    order, at = torch.randperm(sum(need) + 1, generator=g).tolist(), 0
+    tail = {"rows": (G, D + Dv), "latent": (1, D), "shared": (1, D + G * Dv), "scaled": (1, hip_ops.scaled_key_row(G, D, torch.bfloat16))}[layout]
+    cache = torch.full((sum(need) + 1, page) + tail, float("nan"), dtype=torch.bfloat16, device=dev)
+    table = torch.zeros(len(lens), max(need), dtype=torch.int32)
+    for s in range(len(lens)):
+        pages = order[at:at + need[s]]
+        at += need[s]
+        table[s, :need[s]] = torch.tensor(pages, dtype=torch.int32)
+        slots = torch.tensor([pages[p // page] * page + p % page for p in range(total[s])], device=dev)
+        if layout == "scaled":
+            qk = torch.cat((torch.zeros(total[s], D).bfloat16(), keys[s].reshape(total[s], -1)), 1).to(dev)
+            ones = torch.ones(D, device=dev)
+            hip_ops.scaled_key_cache_(qk, 1, G, D, ones, ones, 1e-6, cache, slots)
+            continue
+        row = {"rows": lambda: torch.cat((keys[s], values[s]), 2), "latent": lambda: keys[s],
+               "shared": lambda: torch.cat((keys[s].reshape(total[s], 1, D), values[s].reshape(total[s], 1, -1)), 2)}[layout]()
+        cache.view((-1,) + tail)[slots] = row.to(dev)
+    out = hip_ops.sink_attention(
+        torch.cat(q).to(dev), cache, table.to(dev), i32([0] + list(accumulate(lens))), i32(total), G if layout != "latent" else 1, D, Dv, D ** -0.5,
+        max(lens), max(total), sink=sink is not None, sink_logits=None if sink is None else sink.to(dev), window_left=o["window"] - 1,
+        keep_first=o["keep"], chunk=o["chunk"], softcap=o["softcap"], value_in_key=layout == "latent", shared_key=layout == "shared",
+        scaled_key=layout == "scaled", bias_a=a.to(dev) if o["bias"] == "log" else None, slopes=(SLOPE * a).to(dev) if o["bias"] == "linear" else None,
+        bias_b=torch.full((H,), NEAR, device=dev) if o["bias"] == "log" else None,
+        head_gate=torch.cat(gates).to(dev) if o["gate"] else None).double().cpu()
+    at = 0
+    for s, n in enumerate(lens):
+        k, v = keys[s].double(), values[s].double()
+        if layout == "scaled":
+            k = k * torch.rsqrt(k.square().mean(-1, keepdim=True) + 1e-6)
+        spread = lambda x: x.permute(1, 0, 2).repeat_interleave(H // x.shape[1], 0)  # noqa: E731
+        ref = reference(q[s].double(), spread(k), spread(v), D ** -0.5, ctxs[s], o, None if sink is None else sink.double(), a.double(),
+                        None if gates[s] is None else gates[s].double())
+        got = out[at:at + n]
+        assert torch.isfinite(got).all()
+        assert (got - ref).norm() <= BOUND * ref.norm(), (s, float((got - ref).norm() / ref.norm()))
+        at += n

@@ -259,12 +259,6 @@ __device__ __forceinline__ f32x4v mfma16(bf16x8 a, bf16x8 b, f32x4v c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// Row blocks of 16 a prompt's wave holds.  Two halve the LDS reads per matrix instruction, but at about 250 registers
-// leave one workgroup per compute unit: measured on prompts of 2048 / 4096 / 8192 rows (28 heads of 128) 0.20 / 0.59 /
-// 2.10 ms against 0.21 / 0.64 / 1.86 ms with one.
-#ifndef PREFILL_RB
-#define PREFILL_RB 1
-#endif
 constexpr int kTileKeys = 64;
 constexpr int kRowsPerWave = 32;
 
@@ -569,18 +563,14 @@ __device__ __forceinline__ void load_bias(WaveRows<D, DV, RB>& w, int rb, const 
   w.bb[rb] = a.bias_mode == HYMETA_BIAS_LOG_DISTANCE ? a.bias_b[h] : 0.f;
 }
 
-// Waves of a prompt workgroup: 8, or 4 for keys longer than 192 elements, whose query fragments (D / 8 registers) and
-// staging registers do not leave a wave of 8 its accumulators within 256 registers (a workgroup of 4 waves has 512
-// registers per wave).
-template <int D> struct PrefillWaves { static constexpr int value = D > 192 ? 4 : 8; };
-template <int RB, int Waves> struct PrefillShape { static constexpr int kRows = 16 * RB * Waves; };
+// Portions of prompts with keys of more than 192 elements (shorter ones: row_attn.h): grid = (tiles of 16 rows per wave, heads,
+// sequences); sequences with one row are left to the decode form.  4 waves: the query fragments (D / 8 registers) and the
+// staging registers do not leave a wave of 8 its accumulators within 256 registers.
+constexpr int kPrefillWaves = 4;
 
-// Portions of prompts: grid = (tiles of 16 RB rows per wave, heads, sequences); a wave holds RB blocks of 16 rows; sequences with
-// one row are left to the decode form.
 template <int D, int DV, int RB, int Layout>
-__global__ __launch_bounds__(64 * PrefillWaves<D>::value) void sink_attention_prefill_mfma_kernel(hymeta_sink_attention_args a) {
-  constexpr int kPrefillWaves = PrefillWaves<D>::value;
-  constexpr int kRows = PrefillShape<RB, kPrefillWaves>::kRows;
+__global__ __launch_bounds__(64 * kPrefillWaves) void sink_attention_prefill_mfma_kernel(hymeta_sink_attention_args a) {
+  constexpr int kRows = 16 * RB * kPrefillWaves;
   constexpr int kImages = 2 * sizeof(MfmaSmem<D, DV>) <= 159 * 1024 ? 2 : 1;        // (160 KB of LDS)
   constexpr bool kScaled = Layout == HYMETA_KV_SCALED_KEY;
   __shared__ MfmaSmem<D, DV> sm[kImages];
@@ -851,28 +841,19 @@ __global__ __launch_bounds__(64 * kDecodeWaves) void sink_attention_decode_mfma_
   }
 }
 
-// grid = (sequences, heads): merge the partials of a decode row, add the sink, normalise, store bf16.  Two round trips to
-// memory: the threads read the partials' statistics side by side (one each), agree on the row's maximum, and leave every
-// partial's factor in LDS; then groups of v_dim / 4 threads take the partials in turn, four columns a thread.  (As one
-// serial loop over the partials per column and statistic the launch took 11 us at 4 partials of 128 columns; now 6 at
-// 4 partials of 512.)
+// Merge a row's partials (`splits` of them, `stride` floats apart from `base` on), add the sink, normalise, store bf16: one
+// workgroup per (row, head).  Two round trips to memory: the threads read the partials' statistics side by side (one each),
+// agree on the row's maximum, and leave every partial's factor in LDS; then groups of v_dim / 4 threads take the partials
+// in turn, four columns a thread.  (As one serial loop over the partials per column and statistic the launch took 11 us at
+// 4 partials of 128 columns of 64 x 16 rows; now 6 at 4 partials of 512.)
 constexpr int kCombineThreads = 128;
 constexpr int kMaxPartials = 512 * kDecodeWaves;
 
-__global__ __launch_bounds__(kCombineThreads) void sink_attention_decode_combine_kernel(hymeta_sink_attention_args a, int splits, HeadSlice hs) {
-  // (splits: partials per (sequence, key/value head): one per slice, or one per wave of a slice)
+__device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a, const float* base, size_t stride, int splits, int64_t t, int h) {
   __shared__ float s_f[kMaxPartials];
   __shared__ float s_red[2][kCombineThreads / 64];
   __shared__ __attribute__((aligned(16))) f32x4v s_acc[kCombineThreads];
-  const int s = blockIdx.x;
-  const int t = a.query_start_loc[s];
-  if (a.query_start_loc[s + 1] - t != 1) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int group = a.num_heads / a.num_kv_heads, HG = hs.count ? hs.count : group;
-  const int g = blockIdx.y / HG, r = blockIdx.y % HG, h = g * group + hs.first + r, DV = a.v_dim;
-  const size_t stride = HG * partial_row_floats(DV);
-  const float* base = static_cast<const float*>(a.workspace) + (static_cast<size_t>(s) * a.num_kv_heads + g) * splits * stride +
-                      r * partial_row_floats(DV);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, DV = a.v_dim;
   // (the partials' maxima are in the base-2 domain, as the waves kept them)
   const float sink2 = a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f;
   float m = a.sink ? sink2 : -INFINITY;
@@ -896,7 +877,7 @@ __global__ __launch_bounds__(kCombineThreads) void sink_attention_decode_combine
   __syncthreads();
   l = (s_red[1][0] + s_red[1][1]) + (a.sink ? __builtin_amdgcn_exp2f(sink2 - m) : 0.f);
   float inv = l > 0.f ? 1.f / l : 0.f;
-  if (a.head_gate) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[static_cast<int64_t>(t) * a.head_gate_stride_t + h]));
+  if (a.head_gate) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[t * a.head_gate_stride_t + h]));
   const int quads = DV / 4, turns = kCombineThreads / quads, turn = tid / quads, c = 4 * (tid % quads);
   f32x4v acc = f32x4v{0.f, 0.f, 0.f, 0.f};
   if (turn < turns) {
@@ -916,17 +897,38 @@ __global__ __launch_bounds__(kCombineThreads) void sink_attention_decode_combine
   acc *= inv;
   if (a.elem_gate) {
     float gate[4];
-    ActBf16::ld4(static_cast<const uint16_t*>(a.elem_gate) + static_cast<int64_t>(t) * a.elem_gate_stride_t + static_cast<int64_t>(h) * DV + c, gate);
+    ActBf16::ld4(static_cast<const uint16_t*>(a.elem_gate) + t * a.elem_gate_stride_t + static_cast<int64_t>(h) * DV + c, gate);
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] *= ActBf16::sigmoid(gate[e]);
   }
-  *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.out) + (static_cast<int64_t>(t) * a.num_heads + h) * DV + c) =
+  *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.out) + (t * a.num_heads + h) * DV + c) =
       u32x2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
+}
+
+// grid = (sequences, heads): the rows of a decode step.
+__global__ __launch_bounds__(kCombineThreads) void sink_attention_decode_combine_kernel(hymeta_sink_attention_args a, int splits, HeadSlice hs) {
+  // (splits: partials per (sequence, key/value head): one per slice, or one per wave of a slice)
+  const int s = blockIdx.x;
+  const int t = a.query_start_loc[s];
+  if (a.query_start_loc[s + 1] - t != 1) return;
+  const int group = a.num_heads / a.num_kv_heads, HG = hs.count ? hs.count : group;
+  const int g = blockIdx.y / HG, r = blockIdx.y % HG, h = g * group + hs.first + r;
+  const size_t row = partial_row_floats(a.v_dim), stride = HG * row;
+  combine_row(a, static_cast<const float*>(a.workspace) + (static_cast<size_t>(s) * a.num_kv_heads + g) * splits * stride + r * row, stride, splits, t, h);
+}
+
+// grid = (rows, heads): the rows of prompts' portions whose keys were cut into slices.
+__global__ __launch_bounds__(kCombineThreads) void sink_attention_rows_combine_kernel(hymeta_sink_attention_args a, int splits) {
+  const int t = blockIdx.x, h = blockIdx.y, s = seq_of_row(a.query_start_loc, a.num_seqs, t);
+  if (a.query_start_loc[s + 1] - a.query_start_loc[s] <= 1) return;
+  const size_t row = partial_row_floats(a.v_dim);
+  combine_row(a, static_cast<const float*>(a.workspace) + (static_cast<size_t>(t) * a.num_heads + h) * splits * row, row, splits, t, h);
 }
 
 }  // namespace
 }  // namespace hymeta
 
+#include "row_attn.h"
 #include "wide_latent.h"
 
 namespace hymeta {
@@ -975,13 +977,36 @@ inline int decode_splits(int num_seqs, int num_heads, int num_kv_heads, int tile
   return std::max(1, std::min(splits, tiles));
 }
 
+// Slices a portion's keys are cut into: where the blocks of 128 rows do not fill the chip (`target` workgroups) and the
+// workspace has room for the slices' partials, at least 4 tiles of 64 keys each (a slice's queries, its first tile and its
+// partial cost about two tiles).  7 rows x 28 heads behind 6000 keys: 299 -> 29 us; 40
+// rows x 28 heads on latents of 512 + 64, twice: 592 -> 77; 300 rows on latents of 128 + 64, twice: 233 -> 101.
+inline int64_t portion_partial_bytes(int num_tokens, int num_heads, int v_dim) {
+  return static_cast<int64_t>(num_tokens) * num_heads * static_cast<int64_t>(partial_row_floats(v_dim)) * 4;
+}
+inline int portion_target(int v_dim) { return v_dim > 128 ? 256 : 512; }       // one workgroup on a compute unit (wide_latent.h), or two
+inline int portion_splits(int num_tokens, int num_seqs, int num_heads, int num_kv_heads, int max_query_len, int tiles, int target) {
+  constexpr int64_t kRows = 128;
+  const int64_t group = std::max(1, num_heads / num_kv_heads);
+  const int64_t each = (max_query_len * group + kRows - 1) / kRows, all = (num_tokens * group + kRows - 1) / kRows + num_seqs;
+  const int64_t blocks = std::min(each * num_seqs, all) * num_kv_heads;
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(target / blocks, tiles / 4)));
+}
+inline int portion_splits(const hymeta_sink_attention_args& a) {
+  const int splits = portion_splits(a.num_tokens, a.num_seqs, a.num_heads, a.num_kv_heads, a.max_query_len, decode_tiles(a), portion_target(a.v_dim));
+  const int64_t room = static_cast<int64_t>(a.workspace_bytes) / portion_partial_bytes(a.num_tokens, a.num_heads, a.v_dim);
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(splits, room)));
+}
+
 template <int C>
 int launch_wide_latent(const hymeta_sink_attention_args& a, hipStream_t st) {
   const int group = a.num_heads / a.num_kv_heads;
   if (a.max_query_len > 1) {
     const int64_t rows = static_cast<int64_t>(a.max_query_len) * group;
-    const dim3 grid(static_cast<uint32_t>((rows + kWideRows - 1) / kWideRows), a.num_kv_heads, a.num_seqs);
-    hipLaunchKernelGGL((latent_prefill_kernel<C>), grid, dim3(64 * kWideWaves), 0, st, a);
+    const int splits = portion_splits(a);
+    const dim3 grid(static_cast<uint32_t>((rows + kWideRows - 1) / kWideRows * splits), a.num_kv_heads, a.num_seqs);
+    hipLaunchKernelGGL((latent_prefill_kernel<C>), grid, dim3(64 * kWideWaves), 0, st, a, splits);
+    if (splits > 1) hipLaunchKernelGGL(sink_attention_rows_combine_kernel, dim3(a.num_tokens, a.num_heads), dim3(kCombineThreads), 0, st, a, splits);
   }
   // one workgroup per compute unit (its rings fill the LDS): as many as there are units
   const int64_t slices = (group + kLatentHeads - 1) / kLatentHeads, items = static_cast<int64_t>(a.num_seqs) * a.num_kv_heads;
@@ -995,10 +1020,25 @@ int launch_wide_latent(const hymeta_sink_attention_args& a, hipStream_t st) {
 template <int D, int DV, int Layout = HYMETA_KV_KEY_THEN_VALUE>
 int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st) {
   if (a.max_query_len > 1) {
-    constexpr int kRB = PREFILL_RB;
-    constexpr int kRows = PrefillShape<kRB, PrefillWaves<D>::value>::kRows;
-    const dim3 grid((a.max_query_len + kRows - 1) / kRows, a.num_heads, a.num_seqs);
-    hipLaunchKernelGGL((sink_attention_prefill_mfma_kernel<D, DV, kRB, Layout>), grid, dim3(64 * PrefillWaves<D>::value), 0, st, a);
+    if constexpr (D <= 192) {
+      const int64_t rows = static_cast<int64_t>(a.max_query_len) * (a.num_heads / a.num_kv_heads);
+      constexpr int kRows = RowShape<D, DV, Layout>::kRows;
+      const int splits = portion_splits(a);
+      const dim3 grid(static_cast<uint32_t>((rows + kRows - 1) / kRows * splits), a.num_kv_heads, a.num_seqs);
+      auto launch = [&](auto rule) { hipLaunchKernelGGL((row_prefill_kernel<D, DV, Layout, decltype(rule)::value>), grid, dim3(256), 0, st, a, splits); };
+      const bool plain = a.softcap <= 0.f && a.bias_mode != HYMETA_BIAS_LOG_DISTANCE;
+      if constexpr (Layout == HYMETA_KV_SCALED_KEY) launch(std::integral_constant<int, kPlain>{});
+      else if (plain) launch(std::integral_constant<int, kPlain>{});
+      else if constexpr (Layout == HYMETA_KV_KEY_THEN_VALUE) {
+        if (a.softcap <= 0.f) launch(std::integral_constant<int, kLogBias>{});
+        else launch(std::integral_constant<int, kAnyRule>{});
+      } else launch(std::integral_constant<int, kAnyRule>{});
+      if (splits > 1) hipLaunchKernelGGL(sink_attention_rows_combine_kernel, dim3(a.num_tokens, a.num_heads), dim3(kCombineThreads), 0, st, a, splits);
+    } else {
+      constexpr int kRows = 16 * kPrefillWaves;
+      const dim3 grid((a.max_query_len + kRows - 1) / kRows, a.num_heads, a.num_seqs);
+      hipLaunchKernelGGL((sink_attention_prefill_mfma_kernel<D, DV, 1, Layout>), grid, dim3(64 * kPrefillWaves), 0, st, a);
+    }
   }
   // sequences with a single row: every step but a pure prompt step has some; a prompt of one token is one too
   const int splits = decode_splits(a.num_seqs, a.num_heads, a.num_kv_heads, decode_tiles(a));
@@ -1078,6 +1118,14 @@ extern "C" size_t hymeta_sink_attention_workspace_bytes(int32_t num_seqs, int32_
   if (num_seqs <= 0 || num_heads <= 0 || num_kv_heads <= 0 || v_dim <= 0) return 0;
   const int splits = decode_splits(num_seqs, num_heads, num_kv_heads, decode_tiles(max_seq_len < 1 ? 1 : max_seq_len));
   return static_cast<size_t>(num_seqs) * splits * kDecodeWaves * num_heads * partial_row_floats(v_dim) * sizeof(float);
+}
+
+extern "C" size_t hymeta_sink_attention_portion_workspace_bytes(int32_t num_tokens, int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads,
+                                                                int32_t v_dim, int32_t max_query_len, int32_t max_seq_len, int64_t span,
+                                                                int32_t keep_first) {
+  if (num_tokens <= 0 || num_seqs <= 0 || num_heads <= 0 || num_kv_heads <= 0 || v_dim <= 0 || max_query_len <= 1 || max_seq_len < 1) return 0;
+  const int splits = portion_splits(num_tokens, num_seqs, num_heads, num_kv_heads, max_query_len, decode_tiles(max_seq_len, span, keep_first), portion_target(v_dim));
+  return splits > 1 ? static_cast<size_t>(splits) * portion_partial_bytes(num_tokens, num_heads, v_dim) : 0;
 }
 
 extern "C" int hymeta_sink_attention(const hymeta_sink_attention_args* args, hymeta_stream_t stream) {

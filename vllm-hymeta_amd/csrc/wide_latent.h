@@ -16,27 +16,10 @@
 
 #include <type_traits>
 
-#include "common.h"
+#include "row_attn.h"
 
 namespace hymeta {
 namespace {
-
-typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
-
-// 16 bytes per lane from global memory into LDS at (wave-uniform) dst + 16 lane, without passing registers.  An asm
-// statement, its completion counted by hand: the compiler books such a load on the LDS counter as well and would turn
-// every wait for a fragment read into a wait for all of them.
-__device__ __forceinline__ void copy16_to_lds(const char* src, char* dst) {
-  const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)dst));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
-}
-
-// Lane (g4 = lane / 16, n = lane % 16) of the result: column n of the 16 x 4 keys block its 16 lanes address.
-__device__ __forceinline__ bf16x4 read_transposed(const char* p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4*)(p));
-}
-
-constexpr float kLazyMax2 = 8.f;     // the softmax reference may trail a row's maximum by a factor of 2^8
 
 // Scores of a lane's row against N keys at distances dist - i in the base-2 domain (scores times log2 e; the bias'
 // coefficient is the same in both), from the products of the query with the keys.
@@ -106,7 +89,7 @@ struct WideSmem {
   int moved[2][kWideWaves];                       // whether a row block has any factor but 1
 };
 
-// Portions of prompts: grid = (blocks of 128 rows, key/value heads, sequences); a row is a (query, head) pair, the heads of a
+// Portions of prompts: grid = (blocks of 128 rows x slices of the keys, key/value heads, sequences); a row is a (query, head) pair, the heads of a
 // key/value head side by side, so that a portion of a few tokens fills its blocks.  Sequences with one row are left to the
 // decode form.
 //
@@ -114,13 +97,14 @@ struct WideSmem {
 // the scores of tile t + 1 and adds tile t's values, which do not depend on each other: the two waves of a SIMD do them in
 // opposite order, so that one's softmax runs under the other's products.  One barrier per tile.  Bound by the matrix
 // pipe: 8192 rows x 16 heads on
-// 512 + 64: 1.62 ms = 1.06 PFLOP/s of the products issued (both parts of the weights counted), where launches over value
+// 512 + 64: 1.65 ms = 1.04 PFLOP/s of the products issued (both parts of the weights counted), where launches over value
 // slices of 128, each repeating the scores, took 11.3 ms.
 template <int C>
-__global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_sink_attention_args a) {
+__global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_sink_attention_args a, int splits) {
   constexpr int D = C + 64, kRowB = 2 * D, kSteps = D / 32, CB = C / 128;
   __shared__ __attribute__((aligned(16))) WideSmem<C> sm;
-  const int s = blockIdx.z, g = blockIdx.y, tile = gridDim.x - 1 - blockIdx.x;       // the longest rows first
+  const int turn = gridDim.x - 1 - blockIdx.x;              // the longest rows first
+  const int s = blockIdx.z, g = blockIdx.y, tile = turn / splits, split = turn % splits;
   const int row0 = a.query_start_loc[s];
   const int q = a.query_start_loc[s + 1] - row0;
   const int group = a.num_heads / a.num_kv_heads;
@@ -136,8 +120,9 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
   const int qi = ok ? r / group : 0, h = g * group + (ok ? r % group : 0);
   const int pos = ok ? ctx + qi : -1;
   const float ba = a.bias_mode ? a.bias_a[h] : 0.f, bb = a.bias_mode == HYMETA_BIAS_LOG_DISTANCE ? a.bias_b[h] : 0.f;
-  float m = a.sink ? (a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f) : -INFINITY;
-  float l = a.sink && g4 == 0 ? 1.f : 0.f;            // the sink's exp(m - m), counted once per row
+  const bool sink = a.sink && splits == 1;            // (of several slices of the keys none has the sink: the merge adds it)
+  float m = sink ? (a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f) : -INFINITY;
+  float l = sink && g4 == 0 ? 1.f : 0.f;              // the sink's exp(m - m), counted once per row
   bf16x8 qf[kSteps];
   {
     const uint16_t* qrow = static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(row0 + qi) * a.q_stride_t + static_cast<int64_t>(h) * D;
@@ -152,8 +137,9 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
   // the tiles: those of the kept first keys that lie before the window's first, then the window's
   const int from = first_key(a, p_lo) / kWideKeys * kWideKeys;
   const int kept = bounded(a) ? min((a.keep_first + kWideKeys - 1) / kWideKeys * kWideKeys, from) / kWideKeys : 0;
-  const int tiles = kept + (p_hi - from) / kWideKeys + 1;
-  auto key0 = [&](int t) { return t < kept ? t * kWideKeys : from + (t - kept) * kWideKeys; };
+  const int all = kept + (p_hi - from) / kWideKeys + 1, per = (all + splits - 1) / splits;
+  const int t0 = split * per, tiles = min(all - t0, per);          // this slice's
+  auto key0 = [&](int t) { return t0 + t < kept ? (t0 + t) * kWideKeys : from + (t0 + t - kept) * kWideKeys; };
 
   f32x4v o[kWideWaves][CB];                           // O^T: this wave's columns x the rows of block rb
 #pragma unroll
@@ -175,19 +161,18 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
   auto scores = [&](int t, const char* img, int buf) {
     const int j0 = key0(t);
     f32x4v acc[2] = {};
-    u32x4 kf[3][2];                                   // fragments two steps ahead, and no more: registers are short
+    u32x4 kf[2][2];                                   // fragments one step ahead, and no more: registers are short
     auto load = [&](int st) {
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) kf[st % 3][ks] = ld16(img + koff[st & 1] + ks * 16 * kRowB + (st >> 1) * 128);
+      for (int ks = 0; ks < 2; ++ks) kf[st & 1][ks] = ld16(img + koff[st & 1] + ks * 16 * kRowB + (st >> 1) * 128);
     };
     load(0);
-    load(1);
 #pragma unroll
     for (int st = 0; st < kSteps; ++st) {
-      if (st + 2 < kSteps) load(st + 2);
+      if (st + 1 < kSteps) load(st + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) acc[ks] = mfma16(__builtin_bit_cast(bf16x8, kf[st % 3][ks]), qf[st], acc[ks]);
+      for (int ks = 0; ks < 2; ++ks) acc[ks] = mfma16(__builtin_bit_cast(bf16x8, kf[st & 1][ks]), qf[st], acc[ks]);
     }
     // the lane holds the scores of its row against keys j0 + 16 ks + 4 g4 + e
     const bool masked = !(full && j0 + kWideKeys - 1 <= w_lo && j0 >= w_first);
@@ -274,13 +259,14 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
         for (int cb = 0; cb < CB; ++cb) o[rb][cb] = mfma16(vf[cb], __builtin_bit_cast(bf16x8, pf[rb & 1][part]), o[rb][cb]);
     }
   };
-  auto arrive = [&]() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-
-  copy.issue(key0(0), p_hi, sm.k[0]);
-  if (tiles > 1) copy.issue(key0(1), p_hi, sm.k[1]);
-  arrive();
-  scores(0, sm.k[0], 0);
-  arrive();
+  
+  if (tiles > 0) {
+    copy.issue(key0(0), p_hi, sm.k[0]);
+    if (tiles > 1) copy.issue(key0(1), p_hi, sm.k[1]);
+    copies_landed_barrier();
+    scores(0, sm.k[0], 0);
+    copies_landed_barrier();
+  }
   auto walk = [&](auto scores_first) {
     constexpr bool kScoresFirst = decltype(scores_first)::value;
     int i0 = 0, i1 = 1, i2 = 2;
@@ -290,7 +276,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
       if (!kScoresFirst) values(sm.k[i0], t & 1);
       if (t + 1 < tiles) scores(t + 1, sm.k[i1], (t + 1) & 1);
       if (kScoresFirst) values(sm.k[i0], t & 1);
-      arrive();
+      copies_landed_barrier();
       const int i = i0;
       i0 = i1, i1 = i2, i2 = i;
     }
@@ -299,6 +285,23 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
   else walk(std::false_type{});
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
+  if (splits > 1) {
+    float* parts = static_cast<float*>(a.workspace) + split * partial_row_floats(C);
+    const size_t stride = splits * partial_row_floats(C);
+    if (g4 == 0 && ok) {
+      float* part = parts + (static_cast<size_t>(row0 + qi) * a.num_heads + h) * stride;
+      part[C] = m, part[C + 1] = l;
+    }
+#pragma unroll
+    for (int rb = 0; rb < kWideWaves; ++rb) {
+      const int ro = r0 + 16 * rb + n;
+      if (ro >= rows) continue;
+      float* part = parts + (static_cast<size_t>(row0 + ro / group) * a.num_heads + g * group + ro % group) * stride + wave * 16 * CB;
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) *reinterpret_cast<f32x4v*>(part + 16 * cb + 4 * g4) = o[rb][cb];
+    }
+    return;
+  }
   if (g4 == 0) {
     float inv = l > 0.f ? 1.f / l : 0.f;
     if (a.head_gate && ok) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[static_cast<int64_t>(row0 + qi) * a.head_gate_stride_t + h]));

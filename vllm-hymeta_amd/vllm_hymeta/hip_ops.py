@@ -1693,10 +1693,6 @@ def sink_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_tables: torch.
     a = _C.SinkAttentionArgs()
     a.q, a.kv_cache, a.out, a.block_tables = _p(q), _p(kv_cache), _p(out), _p(block_tables)
     a.query_start_loc, a.seq_lens, a.bias_a, a.bias_b = _p(query_start_loc), _p(seq_lens), _p(bias_a), _p(bias_b)
-    nbytes = int(lib.hymeta_sink_attention_workspace_bytes(S, H, num_kv_heads, v_dim, max_seq_len))
-    if nbytes:
-        ws = _workspace(q.device, nbytes, "sink_attention")
-        a.workspace, a.workspace_bytes = _p(ws), ws.numel()
     a.num_tokens, a.num_seqs, a.num_heads, a.num_kv_heads, a.head_dim, a.v_dim = T, S, H, num_kv_heads, head_dim, v_dim
     a.block_size, a.act_dtype, a.num_blocks = kv_cache.shape[1], _act(q), kv_cache.shape[0]
     a.bias_mode = _C.BIAS_NONE if bias_a is None else _C.BIAS_LOG_DISTANCE
@@ -1714,6 +1710,13 @@ def sink_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_tables: torch.
     a.kv_layout = (_C.KV_SCALED_KEY if scaled_key else _C.KV_SHARED_KEY if shared_key else
                    _C.KV_VALUE_IN_KEY if value_in_key else _C.KV_KEY_THEN_VALUE)
     a.q_stride_t, a.block_table_stride = q.stride(0), block_tables.stride(0)
+    nbytes = int(lib.hymeta_sink_attention_workspace_bytes(S, H, num_kv_heads, v_dim, max_seq_len))
+    if max_query_len > 1:
+        nbytes = max(nbytes, int(lib.hymeta_sink_attention_portion_workspace_bytes(T, S, H, num_kv_heads, v_dim, max_query_len, max_seq_len,
+                                                                                   chunk if chunk > 0 else window_left + 1, keep_first)))
+    if nbytes:
+        ws = _workspace(q.device, nbytes, "sink_attention")
+        a.workspace, a.workspace_bytes = _p(ws), nbytes         # (not what the buffer has grown to: a call's slices follow from the call)
     _C.check(lib.hymeta_sink_attention(C.byref(a), _stream(q)), "hymeta_sink_attention")
     return out
 
