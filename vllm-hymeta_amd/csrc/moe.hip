@@ -13,6 +13,7 @@
 //   combine  out[t] = sum_k y[pos[t,k]] (+ shared[t]), y weighted in the down GEMM; pairs of non-local experts
 //            (expert parallelism) carry pos = -1 and add nothing
 #include "common.h"
+#include "lds_copy.h"
 #include "w8a8_quant.h"
 
 #include <algorithm>
@@ -692,6 +693,156 @@ __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void moe_gemm_t
   }
 }
 
+// int8 in tiles of 256 x 256 (8 waves of 64 rows x 128 columns), both operands copied from memory straight into LDS: nothing
+// of a step passes registers, so the fragments of the next quarter of a step are read while this one's are multiplied, and
+// v_mfma_i32_32x32x32_i8 needs 6 fragments of 1 KB for 8 instructions.  Two images of a step (128 bytes of every row); a
+// step's copies are asked for a whole step ahead.  The barrier that frees an image stands in front of the step's last
+// quarter: the first reads of the next image go out under that quarter's products.  The weights are the first operand: a
+// lane then holds four neighbouring columns of ONE row, which share its scales and go to the staged output together.
+// Bound by the matrix pipe and its power: 16 int8 experts on 8192 rows of 3584 columns took 779 us through
+// moe_gemm_tiled_kernel's 256 x 256 tile, 732 through this one (quantisation and activation included).  In bf16 the same structure takes 4% fewer cycles at a lower
+// clock: 0.99 to 1.02 of the tiled kernel's speed over 1500 to 8192 rows, so bf16 stays there.
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+constexpr int kBig = 256;                            // rows and columns of the tile
+constexpr int kBigImage = kBig * kTilePitch;         // bytes of one operand's step
+
+__global__ __launch_bounds__(512, 2) void moe_gemm_big_i8_kernel(hymeta_moe_gemm_args a) {
+  __shared__ __attribute__((aligned(16))) char sm[2][2 * kBigImage];   // [step parity][x | w]
+
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+
+  // which expert, which of its row tiles
+  int e = -1, row_lo = 0, row_hi = 0;
+  {
+    int t = blockIdx.y;
+    for (int i = a.local_expert_begin; i < a.local_expert_end; ++i) {
+      const int lo = a.expert_offsets[i], hi = a.expert_offsets[i + 1];
+      const int tiles = (hi - lo + kBig - 1) / kBig;
+      if (t < tiles) {
+        e = i;
+        row_lo = lo + t * kBig;
+        row_hi = hi;
+        break;
+      }
+      t -= tiles;
+    }
+  }
+  if (e < 0) return;                                 // workgroup-uniform
+  const int col0 = blockIdx.x * kBig;
+
+  // copies: an instruction of a wave brings 8 rows x 128 bytes; a row's 16-byte chunks lie XOR-ed with (row / 2) % 8, which
+  // with the pitch of 128 bytes spreads the rows of a fragment read over all banks
+  const int64_t kb = a.K;                          // bytes of an operand row
+  const char *xp[4], *wp[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = 8 * (4 * wave + j) + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
+    const int slot = min(row_lo + row, row_hi - 1);    // rows past the expert's end re-read its last row
+    xp[j] = static_cast<const char*>(a.x) + static_cast<int64_t>(moe_src_row(a, slot)) * a.x_stride_m + 16 * chunk;
+    wp[j] = static_cast<const char*>(a.weights) + static_cast<int64_t>(e) * a.w_stride_e + (col0 + row) * kb + 16 * chunk;
+  }
+  
+  auto issue = [&](int it, char* image) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      copy16_to_lds(xp[j] + it * kTilePitch, image + 1024 * (4 * wave + j));
+      copy16_to_lds(wp[j] + it * kTilePitch, image + kBigImage + 1024 * (4 * wave + j));
+    }
+  };
+  int off[4];                                        // a fragment's place for this lane: row r, chunk 2 ks + hh
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) off[ks] = r * kTilePitch + 16 * ((2 * ks + hh) ^ ((r >> 1) & 7));
+  const int xat = 64 * wm * kTilePitch, wat = kBigImage + 128 * wn * kTilePitch;
+
+  i32x16 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int k = 0; k < 16; ++k) acc[i][j][k] = 0;
+
+  i32x4 xf[2][2], wf[2][4];                          // [parity of the quarter]
+  auto read = [&](const char* image, int ks) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) xf[ks & 1][i] = __builtin_bit_cast(i32x4, ld16(image + xat + off[ks] + 32 * i * kTilePitch));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) wf[ks & 1][j] = __builtin_bit_cast(i32x4, ld16(image + wat + off[ks] + 32 * j * kTilePitch));
+  };
+  const int nk = static_cast<int>(kb / kTilePitch);
+  issue(0, sm[0]);
+  copies_landed_barrier();
+  if (nk > 1) issue(1, sm[1]);
+  read(sm[0], 0);
+  auto multiply = [&](int ks) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[ks & 1][j], xf[ks & 1][i], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // (the last step stands behind the loop: a branch around the barrier and the next step's reads would make the compiler
+  // wait for those reads in front of the last quarter's products)
+  for (int it = 0; it + 1 < nk; ++it) {
+    char* image = sm[it & 1];
+#pragma unroll
+    for (int ks = 0; ks < 3; ++ks) {
+      read(image, ks + 1);
+      multiply(ks);
+    }
+    copies_landed_barrier();                         // this step's last fragments are in registers, the next step's rows in LDS
+    read(sm[(it + 1) & 1], 0);
+    if (it + 2 < nk) issue(it + 2, image);
+    multiply(3);
+  }
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    if (ks < 3) read(sm[(nk - 1) & 1], ks + 1);
+    multiply(ks);
+  }
+  __syncthreads();
+
+  // acc[i][j][4 q + p] = C[row 64 wm + 32 i + r][col 128 wn + 32 j + 8 q + 4 hh + p]: routing weight on the fp32 sums, one
+  // rounding, staged through LDS 128 rows at a time and stored as whole rows
+  constexpr int kCPitch = 2 * kBig + 16, kStageRows = 128;
+  static_assert(kStageRows * kCPitch <= static_cast<int>(sizeof(sm)), "output staging fits the operand images");
+  char* cst = &sm[0][0];
+#pragma unroll
+  for (int half = 0; half < kBig / kStageRows; ++half) {
+    if (wm >> 1 == half) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = 64 * wm + 32 * i + r, slot = min(row_lo + row, row_hi - 1);
+        const float sc_row = a.row_scale != nullptr ? a.row_scale[a.scale_rows != nullptr ? a.scale_rows[slot] : slot] : 1.f;
+        const float xs = a.x_scale[moe_src_row(a, slot)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int col = 128 * wn + 32 * j + 8 * q + 4 * hh;
+            const f32x4 ws = *reinterpret_cast<const f32x4*>(a.w_scale + static_cast<int64_t>(e) * a.N + col0 + col);
+            f32x4 v;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) v[p] = w8a8_scaled(acc[i][j][4 * q + p], xs, ws[p], 0.f);
+            *reinterpret_cast<u32x2*>(cst + (row - kStageRows * half) * kCPitch + 2 * col) =
+                u32x2{pack_bf16x2(v[0] * sc_row, v[1] * sc_row), pack_bf16x2(v[2] * sc_row, v[3] * sc_row)};
+          }
+      }
+    }
+    __syncthreads();
+    constexpr int kChunksPerRow = kBig / 8;
+    for (int id = tid; id < kStageRows * kChunksPerRow; id += 512) {
+      const int row = id / kChunksPerRow, ch = id % kChunksPerRow, slot = row_lo + kStageRows * half + row;
+      if (slot < row_hi)
+        st16(reinterpret_cast<uint16_t*>(a.out) + static_cast<int64_t>(slot) * a.out_stride_m + col0 + 8 * ch, ld16(cst + row * kCPitch + 16 * ch));
+    }
+    if (half + 1 < kBig / kStageRows) __syncthreads();
+  }
+}
+
 // out[r, j] = silu(in[r, j]) * in[r, inter + j]; the product is formed in fp32 and rounded once.
 __global__ __launch_bounds__(256) void silu_and_mul_kernel(const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
                                                            const int32_t* __restrict__ num_rows_dev, int num_rows,
@@ -883,7 +1034,7 @@ extern "C" int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t
   if (kind == MoeGemmKind::kBigTiles) {
     const dim3 tgrid(a.N / 256, (a.max_rows + 255) / 256 + experts);
     HYMETA_MOE_BY_TYPE(hipLaunchKernelGGL((moe_gemm_tiled_kernel<256, 256, 4, 2, false>), tgrid, dim3(512), 0, s, a),
-                       hipLaunchKernelGGL((moe_gemm_tiled_kernel<256, 256, 4, 2, true>), tgrid, dim3(512), 0, s, a));
+                       hipLaunchKernelGGL(moe_gemm_big_i8_kernel, tgrid, dim3(512), 0, s, a));
     return launch_status();
   }
   if (kind == MoeGemmKind::kTiles) {

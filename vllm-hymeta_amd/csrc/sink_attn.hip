@@ -11,6 +11,7 @@
 #include <algorithm>
 
 #include "act_types.h"
+#include "row_copy.h"
 
 namespace hymeta {
 
@@ -414,8 +415,6 @@ struct WaveRows {
   int first[RB];               // the first key it sees
   float ba[RB], bb[RB];
 };
-
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
 
 // tanh through the hardware's exponential: 1 - 2 / (exp(2 x) + 1), exact at both ends (exp2 -> inf gives 1, -> 0 gives -1)
 __device__ __forceinline__ float tanh_fast(float x) {
