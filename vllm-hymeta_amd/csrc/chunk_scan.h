@@ -1,0 +1,441 @@
+// Linear attention with decays over the bf16 rows of prompts' portions, in chunks of 64 rows on the matrix cores: the
+// kernel behind lightning attention and the decay scan.  With S the state before a chunk, i and j rows of the chunk, n its
+// number of rows, l_j the log2 decays, c_i = l_0 + ... + l_i their running sums and b_j the input weights:
+//   o_i   = 2^(c_i) S^T q_i + sum_{j <= i} 2^(c_i - c_j) b_j (q_i . k_j) v_j + skip v_i
+//   S_new = 2^(c_{n-1}) S + sum_j k_j (2^(c_{n-1} - c_j) b_j v_j)^T
+#pragma once
+
+#include "act_types.h"
+#include "row_copy.h"
+
+namespace hymeta {
+namespace {
+
+struct ChunkScanArgs {
+  const uint16_t *q, *k, *v;               // rows of num_qk_heads x D, the same, num_heads x v_dim
+  int64_t q_stride, k_stride, v_stride;
+  const float *decay, *log2_decay;         // per head, or per row and head
+  const float *v_scale, *skip;             // b per row and head, skip per head, or NULL
+  float *state, *out, *workspace;          // state fp32 [slots, heads, D, v_dim]
+  const int32_t *query_start_loc, *context_lens, *slot_idx;
+  int num_seqs, num_heads, num_qk_heads, v_dim;
+};
+
+constexpr int kScanRows = 64;              // rows of a chunk
+constexpr int kScanMinRows = 8;            // shorter portions go token by token
+constexpr float kMinLog2 = -1.0e4f;        // a decay of 0 (or an overflowed step size): finite, so that differences of sums stay numbers
+
+// A workgroup takes as many value columns as there are, 128, 64 or 32 (16 to a wave): what is done once per workgroup, the
+// rows' silu and the chunk's weights, is then done once per head.  Where that gives few workgroups, half as wide ones: two
+// portions of 150 rows of 28 heads of 128 columns took 23.0 us in 56 workgroups, 21.1 in 112 and 27.6 in 224.
+inline int scan_waves(int64_t lanes, int v_dim) {
+  if (v_dim % 128 == 0 && lanes * (v_dim / 128) > 96) return 8;
+  return v_dim % 64 == 0 ? 4 : 2;
+}
+
+// A sequence's chunks follow each other in one workgroup per (head, value slice).  Where that leaves most of the chip idle,
+// the portions are cut into segments that run side by side: every segment but the last is summarised from a zero state (its
+// state and the sum of its log2 decays), the summaries are chained into the states in front of the segments, then every
+// segment runs from its state.  The summaries read the keys and values a second time, so fewer than three segments do not
+// pay.  As many segments as run at the same time, eight waves to a compute unit: one prompt of 8192 rows of 28 heads of 128
+// columns took 138 us (lightning) and 120 (plain decays) in 256 workgroups of eight waves, 152 and 136 in 512, 175 and 156
+// in 1024; of 64 columns 131 us in 512 workgroups of four, 189 in 256, 147 in 1024.  At least 192 rows each: three portions
+// of 700 rows of 16 heads took 39 us in three segments, 49 in one.
+struct ScanSegments { int rows, count; };
+inline ScanSegments scan_segments(int num_seqs, int num_heads, int v_dim, int max_query_len) {
+  const int64_t lanes = static_cast<int64_t>(num_seqs) * num_heads;
+  const int64_t wide = v_dim % 128 == 0 ? 128 : v_dim % 64 == 0 ? 64 : 32, slots = 256 * (128 / wide);
+  const int64_t want = std::min<int64_t>(slots / std::max<int64_t>(lanes * v_dim / wide, 1), max_query_len / 192);
+  if (want < 3) return ScanSegments{0, 1};
+  const int rows = static_cast<int>((max_query_len + want - 1) / want + kScanRows - 1) / kScanRows * kScanRows;
+  return ScanSegments{rows, (max_query_len + rows - 1) / rows};
+}
+inline size_t scan_workspace_bytes(int num_seqs, int num_heads, int head_dim, int v_dim, int max_query_len) {
+  if (num_seqs <= 0 || num_heads <= 0 || head_dim <= 0 || v_dim <= 0) return 0;
+  const ScanSegments sg = scan_segments(num_seqs, num_heads, v_dim, max_query_len);
+  return sg.count > 1 ? static_cast<size_t>(sg.count) * num_seqs * num_heads * (static_cast<size_t>(head_dim) * v_dim + 1) * sizeof(float) : 0;
+}
+
+// a chunk's rows at byte offsets below 2^31
+inline bool scan_offsets_fit(int64_t row_stride, int num_heads, int v_dim) {
+  return row_stride >= 0 && row_stride < (1 << 23) && static_cast<int64_t>(num_heads) * v_dim < (1 << 22);
+}
+
+typedef float f32x4s __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4s scan_mfma(bf16x8 a, bf16x8 b, f32x4s c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+
+// the hardware's exponential and reciprocal (about 1 ulp each): the input is bf16
+__device__ __forceinline__ float silu_fast(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
+
+// Two floats as hi + lo bf16 parts (16 bits of mantissa together).
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t& hi, uint32_t& lo) {
+  hi = pack_bf16x2(x, y);
+  lo = pack_bf16x2(x - lo_bf(hi), y - hi_bf(hi));
+}
+__device__ __forceinline__ bf16x8 frag_of(bf16x4 a, bf16x4 b) { return bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}; }
+
+// Rows behind a wave-uniform address, at byte offsets below 2^31: what a lane has no row for is read as zeros and not
+// written, without a branch (around branches the compiler waits for every load AND store in flight).
+template <int X> struct Const { static constexpr int value = X; };
+
+struct RowBuffer {
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ explicit RowBuffer(const void* base) : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000)) {}
+  __device__ __forceinline__ u32x4 load(bool valid, int offset) const {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, valid ? offset : INT32_MIN, 0, 0));
+  }
+  __device__ __forceinline__ float load1(bool valid, int offset) const {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, valid ? offset : INT32_MIN, 0, 0));
+  }
+  __device__ __forceinline__ void store(bool valid, int offset, f32x4s x) const {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, valid ? offset : INT32_MIN, 0, 0);
+  }
+};
+
+// grid = (heads, sequences x segments, value columns in slices of 16 NW); NW waves.
+//
+// Every wave owns 16 value columns of the state, fp32 in registers as the matrix instructions leave it (a lane holds runs of
+// four d of one column): that is also the layout in which the next chunk's product with the queries wants it, so the state
+// never goes through LDS.  The rows of a chunk go through their silu once per workgroup and lie in LDS as rows; what a product
+// needs transposed is read transposed.  The decays of the state's update go onto the values (a wave splits its own 16 columns
+// into hi + lo bf16 parts) and not onto the keys; the chunk's own weights are computed once per workgroup, a block of 16 rows
+// x 32 keys per wave, and handed over in LDS as fragments.  What enters a product from fp32 goes in as hi + lo parts, two
+// products, so that it keeps 16 bits of mantissa.
+// Bound by vector arithmetic between the barriers of a chunk: 2 x 16 cycles of exponential and reciprocal per silu'd value,
+// splits, scales; the matrix pipes are busy about a quarter of the time, memory far less.  One prompt of 8192 rows, 28 heads
+// of 128 x 128: lightning 351 -> 141 us (summaries 40, states 8, rows 88), plain decays 283 -> 121; with 64 value columns and
+// decays per row 316 -> 131; before, 4 waves to 32 value columns, each such workgroup with its own staging, weights and an
+// image of the state in LDS.
+template <int D, int NW, bool Silu, bool Summarise>
+__global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(ChunkScanArgs a, int seg_rows, int nseg) {
+  constexpr int NT = 64 * NW, KC = D / 8, VC = 2 * NW, KP = 2 * D, VP = 32 * NW, SD = D / 32, DB = D / 16;
+  constexpr int KPT = (kScanRows * KC + NT - 1) / NT, VPT = 2;
+  typedef ChunkOrder<KC> KOrder;
+  typedef ChunkOrder<VC> VOrder;
+  __shared__ __attribute__((aligned(16))) char s_k[kScanRows * KP], s_v[kScanRows * VP];
+  __shared__ __attribute__((aligned(16))) char s_q[Summarise ? 16 : kScanRows * KP], s_vlo[Silu ? kScanRows * VP : 16];
+  __shared__ __attribute__((aligned(16))) u32x4 s_p[Summarise ? 1 : 6][2][64];
+  __shared__ __attribute__((aligned(16))) float s_cum[kScanRows], s_b[kScanRows], s_w[kScanRows];
+  const int h = blockIdx.x, s = blockIdx.y / nseg, seg = blockIdx.y % nseg, vs = blockIdx.z;
+  const int r0 = a.query_start_loc[s], rows_all = a.query_start_loc[s + 1] - r0;
+  if (rows_all < kScanMinRows) return;
+  const bool whole = nseg == 1;
+  const int r_lo = whole ? 0 : seg * seg_rows;
+  if (r_lo >= rows_all) return;
+  const int rows = whole ? rows_all : min(rows_all, r_lo + seg_rows);        // (end of this workgroup's rows)
+  const bool last = rows == rows_all;
+  if (Summarise && last) return;                       // nothing comes behind the last segment
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int H = a.num_heads, Dv = a.v_dim, g = h / (H / a.num_qk_heads), col0 = vs * 16 * NW + 16 * wave;
+  const int slot = a.slot_idx[s];
+  float* st = slot >= 0 ? a.state + (static_cast<int64_t>(slot) * H + h) * D * Dv + col0 : nullptr;
+  const float l2_const = a.decay ? fmaxf(a.decay[h] > 0.f ? log2f(a.decay[h]) : -INFINITY, kMinLog2) : 0.f;
+  const float skip = a.skip ? a.skip[h] : 0.f;
+  // a segment's place in the workspace: its summary (Summarise writes it), then the state in front of it; the segments' sums
+  // of log2 decays lie behind all the states
+  const int64_t seg_at = (static_cast<int64_t>(s) * nseg + seg) * H + h;
+  float* wsp = whole ? nullptr : a.workspace + seg_at * D * Dv + col0;
+  const float* init = Summarise ? nullptr : whole ? (st != nullptr && a.context_lens[s] > 0 ? st : nullptr) : wsp;
+  float seg_total = 0.f;
+
+  const uint16_t* qp = a.q + static_cast<int64_t>(g) * D;
+  const uint16_t* kp = a.k + static_cast<int64_t>(g) * D;
+  const uint16_t* vp = a.v + static_cast<int64_t>(h) * Dv + vs * 16 * NW;
+  // a chunk's rows as they come from memory, a chunk ahead: this thread's 16-byte chunks of the keys, queries and values, and
+  // (first wave) row `lane`'s log2 decay and input weight
+  u32x4 rk[KPT], rq[Summarise ? 1 : KPT], rv[VPT];
+  float rl = 0.f, rb = 0.f;
+  auto fetch = [&](int c0) {
+    const int nrow = min(kScanRows, rows - c0);
+    const int64_t t0 = r0 + c0;
+    const RowBuffer kr(kp + t0 * a.k_stride), qr(qp + t0 * a.q_stride), vr(vp + t0 * a.v_stride);
+#pragma unroll
+    for (int u = 0; u < KPT; ++u) {
+      const int idx = tid + NT * u, j = idx / KC, ch = idx % KC;
+      rk[u] = kr.load(j < nrow, 2 * (j * static_cast<int>(a.k_stride) + 8 * ch));
+      if constexpr (!Summarise) rq[u] = qr.load(j < nrow, 2 * (j * static_cast<int>(a.q_stride) + 8 * ch));
+    }
+#pragma unroll
+    for (int u = 0; u < VPT; ++u) {
+      const int idx = tid + NT * u, j = idx / VC, ch = idx % VC;
+      rv[u] = vr.load(j < nrow, 2 * (j * static_cast<int>(a.v_stride) + 8 * ch));
+    }
+    const int at = 4 * lane * H;
+    if (a.log2_decay || a.v_scale) {
+      rl = RowBuffer(a.log2_decay + t0 * H + h).load1(a.log2_decay && lane < nrow, at);
+      rb = RowBuffer(a.v_scale + t0 * H + h).load1(a.v_scale && lane < nrow, at);
+    }
+  };
+  auto silu8 = [](u32x4 raw, u32x4& hi, u32x4& lo) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t x, y;
+      split_pair(silu_fast(lo_bf(raw[e])), silu_fast(hi_bf(raw[e])), x, y);
+      hi[e] = x, lo[e] = y;
+    }
+  };
+  // (rows past the portion were fetched as zeros, and silu(0) = 0: a whole chunk has no look at its rows)
+  auto stage_as = [&](int nrow, auto full) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < KPT; ++u) {
+      const int idx = tid + NT * u, j = idx / KC, ch = idx % KC;
+      if (kScanRows * KC % NT != 0 && j >= kScanRows) break;
+      const int at = j * KP + 16 * (ch ^ KOrder::twist(j));
+      u32x4 x = rk[u], lo;
+      if (Silu && (decltype(full)::value || j < nrow)) silu8(rk[u], x, lo);
+      st16(s_k + at, x);
+      if constexpr (!Summarise) {
+        x = rq[u];
+        if (Silu && (decltype(full)::value || j < nrow)) silu8(rq[u], x, lo);
+        st16(s_q + at, x);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < VPT; ++u) {
+      const int idx = tid + NT * u, j = idx / VC, ch = idx % VC, at = j * VP + 16 * (ch ^ VOrder::twist(j));
+      u32x4 x = rv[u], lo = u32x4{0u, 0u, 0u, 0u};
+      if constexpr (Silu) {
+        if (decltype(full)::value || j < nrow) silu8(rv[u], x, lo);
+        st16(s_vlo + at, lo);
+      }
+      st16(s_v + at, x);
+    }
+    if (wave == 0) {
+      // running sums of the chunk's log2 decays (rows past the portion add 0)
+      float cum;
+      if (a.log2_decay) {
+        cum = fmaxf(rl, kMinLog2);                     // (rows past the portion: 0)
+        // inclusive sums: within 16 lanes, then the rows of 16 lanes before
+        auto add = [&](auto ctrl, auto rows_mask) {
+          cum += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, cum), decltype(ctrl)::value, decltype(rows_mask)::value, 0xf, false));
+        };
+        add(Const<0x111>{}, Const<0xf>{}), add(Const<0x112>{}, Const<0xf>{}), add(Const<0x114>{}, Const<0xf>{}), add(Const<0x118>{}, Const<0xf>{});
+        add(Const<0x142>{}, Const<0xa>{}), add(Const<0x143>{}, Const<0xc>{});
+      } else {
+        cum = static_cast<float>(min(lane + 1, nrow)) * l2_const;
+      }
+      const float total = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cum), 63));
+      s_cum[lane] = cum;
+      const float b = a.v_scale ? rb : 1.f;
+      s_b[lane] = b;
+      s_w[lane] = lane < nrow ? __builtin_amdgcn_exp2f(total - cum) * b : 0.f;
+    }
+  };
+  auto stage = [&](int nrow) __attribute__((always_inline)) {
+    if (Silu && nrow < kScanRows) stage_as(nrow, std::false_type{});
+    else stage_as(nrow, std::true_type{});
+  };
+  // LDS offsets of this lane's fragments: rows n (16 bytes of a row, or two times 8 for the product with the state), and the
+  // transposed reads of 4 keys x 16 columns
+  const int kt = KOrder::twist(n), Rt = 4 * g4 + (n >> 2), kT = KOrder::twist(Rt), vT = VOrder::twist(Rt);
+  auto row_frag = [&](const char* img, int block, int sd) { return __builtin_bit_cast(bf16x8, ld16(img + (16 * block + n) * KP + 16 * ((4 * sd + g4) ^ kt))); };
+  auto row_frag_halves = [&](const char* img, int block, int sd) {
+    const char* row = img + (16 * block + n) * KP + 8 * (g4 & 1);
+    const u32x2 x = *reinterpret_cast<const u32x2*>(row + 16 * ((4 * sd + (g4 >> 1)) ^ kt));
+    const u32x2 y = *reinterpret_cast<const u32x2*>(row + 16 * ((4 * sd + 2 + (g4 >> 1)) ^ kt));
+    return __builtin_bit_cast(bf16x8, (u32x4{x[0], x[1], y[0], y[1]}));
+  };
+  // keys 32 kk + 4 g4 + e for e < 4, 32 kk + 16 + 4 g4 + e - 4 after, of column 16 db + n / of this wave's value column n
+  auto key_frag = [&](int db, int kk) {
+    const char* p = s_k + (32 * kk + Rt) * KP + 16 * ((2 * db + ((n & 3) >> 1)) ^ kT) + 8 * (n & 1);
+    return frag_of(read_transposed(p), read_transposed(p + 16 * KP));
+  };
+  auto value_frag = [&](const char* img, int kk) {
+    const char* p = img + (32 * kk + Rt) * VP + 16 * ((2 * wave + ((n & 3) >> 1)) ^ vT) + 8 * (n & 1);
+    return frag_of(read_transposed(p), read_transposed(p + 16 * VP));
+  };
+
+  fetch(r_lo);
+  f32x4s S[DB];                                        // S[16 db + 4 g4 + r][col0 + n]
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[db][r] = init ? init[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + n] : 0.f;
+  stage(min(kScanRows, rows - r_lo));
+  fetch(r_lo + kScanRows);
+  for (int c0 = r_lo; c0 < rows; c0 += kScanRows) {
+    const int nrow = min(kScanRows, rows - c0);
+    __syncthreads();
+    const float total = s_cum[kScanRows - 1];
+    seg_total += total;
+    bf16x8 vf[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) vf[kk] = value_frag(s_v, kk);
+    if constexpr (!Summarise) {
+      // weights of the chunk's own rows, as hi + lo fragments: rows 16 ib + n, keys 32 kk ..
+      for (int job = wave; job < 8; job += NW) {
+        const int ib = job >> 1, kk = job & 1;
+        if (2 * kk > ib) continue;
+        const int i = 16 * ib + n;
+        const float cum_i = s_cum[i];
+        u32x4 hi, lo;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const int jb = 2 * kk + t;
+          f32x4s sc = f32x4s{0.f, 0.f, 0.f, 0.f};
+          if (jb <= ib) {
+#pragma unroll
+            for (int sd = 0; sd < SD; ++sd) sc = scan_mfma(row_frag(s_k, jb, sd), row_frag(s_q, ib, sd), sc);
+          }
+          const f32x4s cj = *reinterpret_cast<const f32x4s*>(s_cum + 16 * jb + 4 * g4), bj = *reinterpret_cast<const f32x4s*>(s_b + 16 * jb + 4 * g4);
+          float p[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) p[r] = 16 * jb + 4 * g4 + r <= i ? sc[r] * __builtin_amdgcn_exp2f(cum_i - cj[r]) * bj[r] : 0.f;
+          uint32_t x, y;
+          split_pair(p[0], p[1], x, y), hi[2 * t] = x, lo[2 * t] = y;
+          split_pair(p[2], p[3], x, y), hi[2 * t + 1] = x, lo[2 * t + 1] = y;
+        }
+        const int at = ib < 2 ? ib : 2 * ib - 2 + kk;
+        s_p[at][0][lane] = hi;
+        s_p[at][1][lane] = lo;
+      }
+      // the state before the chunk
+      f32x4s o[4];
+#pragma unroll
+      for (int ib = 0; ib < 4; ++ib) o[ib] = f32x4s{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int sd = 0; sd < SD; ++sd) {
+        u32x4 sf[2];                                   // its d 32 sd + 4 g4 + e for e < 4, 32 sd + 16 + 4 g4 + e - 4 after, hi and lo
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          uint32_t x, y;
+          split_pair(S[2 * sd + (e >> 1)][2 * (e & 1)], S[2 * sd + (e >> 1)][2 * (e & 1) + 1], x, y);
+          sf[0][e] = x, sf[1][e] = y;
+        }
+        bf16x8 qf[4];
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) qf[ib] = row_frag_halves(s_q, ib, sd);
+#pragma unroll
+        for (int part = 0; part < 2; ++part)
+#pragma unroll
+          for (int ib = 0; ib < 4; ++ib) o[ib] = scan_mfma(__builtin_bit_cast(bf16x8, sf[part]), qf[ib], o[ib]);
+      }
+#pragma unroll
+      for (int ib = 0; ib < 4; ++ib) o[ib] *= __builtin_amdgcn_exp2f(s_cum[16 * ib + n]);
+      if (skip != 0.f) {
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) {
+          const u32x2 vi = *reinterpret_cast<const u32x2*>(s_v + (16 * ib + n) * VP + 16 * ((2 * wave + (g4 >> 1)) ^ VOrder::twist(n)) + 8 * (g4 & 1));
+          o[ib][0] = fmaf(skip, lo_bf(vi[0]), o[ib][0]), o[ib][1] = fmaf(skip, hi_bf(vi[0]), o[ib][1]);
+          o[ib][2] = fmaf(skip, lo_bf(vi[1]), o[ib][2]), o[ib][3] = fmaf(skip, hi_bf(vi[1]), o[ib][3]);
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int part = 0; part < 2; ++part)
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int ib = 2 * kk; ib < 4; ++ib) {
+            const int at = ib < 2 ? ib : 2 * ib - 2 + kk;
+            o[ib] = scan_mfma(vf[kk], __builtin_bit_cast(bf16x8, s_p[at][part][lane]), o[ib]);
+          }
+      const RowBuffer to(a.out + (static_cast<int64_t>(r0 + c0) * H + h) * Dv + col0);
+#pragma unroll
+      for (int ib = 0; ib < 4; ++ib) to.store(16 * ib + n < nrow, 4 * ((16 * ib + n) * H * Dv + 4 * g4), o[ib]);
+    }
+    // the state after the chunk
+    u32x4 wv[2][2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const u32x4 x = __builtin_bit_cast(u32x4, vf[kk]);
+      u32x4 y = u32x4{0u, 0u, 0u, 0u};
+      if constexpr (Silu) y = __builtin_bit_cast(u32x4, value_frag(s_vlo, kk));
+      const f32x4s w0 = *reinterpret_cast<const f32x4s*>(s_w + 32 * kk + 4 * g4), w1 = *reinterpret_cast<const f32x4s*>(s_w + 32 * kk + 16 + 4 * g4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float wa = e < 2 ? w0[2 * e] : w1[2 * e - 4], wb = e < 2 ? w0[2 * e + 1] : w1[2 * e - 3];
+        uint32_t hi, lo;
+        if constexpr (Silu) split_pair((lo_bf(x[e]) + lo_bf(y[e])) * wa, (hi_bf(x[e]) + hi_bf(y[e])) * wb, hi, lo);
+        else split_pair(lo_bf(x[e]) * wa, hi_bf(x[e]) * wb, hi, lo);
+        wv[kk][0][e] = hi, wv[kk][1][e] = lo;
+      }
+    }
+    const float chunk_decay = __builtin_amdgcn_exp2f(total);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      f32x4s acc = S[db] * chunk_decay;
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        const bf16x8 kf = key_frag(db, kk);
+        acc = scan_mfma(kf, __builtin_bit_cast(bf16x8, wv[kk][0]), acc);
+        acc = scan_mfma(kf, __builtin_bit_cast(bf16x8, wv[kk][1]), acc);
+      }
+      S[db] = acc;
+    }
+    __syncthreads();                                   // every wave is done with this chunk's rows
+    if (c0 + kScanRows < rows) {
+      stage(min(kScanRows, rows - c0 - kScanRows));
+      fetch(c0 + 2 * kScanRows);                       // (no row past the segment is read)
+    }
+  }
+  float* to = Summarise ? wsp : (last ? st : nullptr);
+  if (to != nullptr) {
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) to[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + n] = S[db][r];
+  }
+  if (Summarise && vs == 0 && tid == 0) a.workspace[static_cast<int64_t>(a.num_seqs) * nseg * H * D * Dv + seg_at] = seg_total;
+}
+
+// The segments' summaries (each segment's state had it started from zero) become the states in front of the segments:
+// run = carried state; per segment: place <- run, run <- 2^(segment's sum of log2 decays) run + summary.  An element per thread.
+// grid = (heads, sequences, parts of 1024 elements)
+__global__ __launch_bounds__(256) void chunk_scan_chain_kernel(ChunkScanArgs a, int head_dim, int seg_rows, int nseg) {
+  const int h = blockIdx.x, s = blockIdx.y, H = a.num_heads;
+  const int rows = a.query_start_loc[s + 1] - a.query_start_loc[s];
+  const int per_head = head_dim * a.v_dim, idx = 4 * (256 * static_cast<int>(blockIdx.z) + static_cast<int>(threadIdx.x));
+  if (rows < kScanMinRows || idx >= per_head) return;
+  const int slot = a.slot_idx[s];
+  f32x4s run = f32x4s{0.f, 0.f, 0.f, 0.f};
+  if (slot >= 0 && a.context_lens[s] > 0) run = *reinterpret_cast<const f32x4s*>(a.state + (static_cast<int64_t>(slot) * H + h) * per_head + idx);
+  const int segs = (rows + seg_rows - 1) / seg_rows;
+  const int64_t step = static_cast<int64_t>(H) * per_head;
+  float* p = a.workspace + (static_cast<int64_t>(s) * nseg * H + h) * per_head + idx;
+  const float* totals = a.workspace + a.num_seqs * nseg * step + static_cast<int64_t>(s) * nseg * H + h;
+  for (int seg0 = 0; seg0 < segs; seg0 += 8) {           // eight summaries in flight together (the last ones may lie past the end: read again)
+    f32x4s summary[8];
+    float decay[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int at = min(seg0 + u, segs - 1);
+      summary[u] = *reinterpret_cast<const f32x4s*>(p + at * step);
+      decay[u] = totals[at * H];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (seg0 + u < segs) {
+        *reinterpret_cast<f32x4s*>(p + (seg0 + u) * step) = run;
+        run = __builtin_amdgcn_exp2f(decay[u]) * run + summary[u];       // (behind the last segment: not used)
+      }
+  }
+}
+
+template <int D, int NW, bool Silu>
+void launch_chunk_scan_as(const ChunkScanArgs& a, ScanSegments sg, hipStream_t st) {
+  const dim3 grid(a.num_heads, a.num_seqs * sg.count, a.v_dim / (16 * NW)), block(64 * NW);
+  if (sg.count > 1) {
+    hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, true>), grid, block, 0, st, a, sg.rows, sg.count);
+    hipLaunchKernelGGL(chunk_scan_chain_kernel, dim3(a.num_heads, a.num_seqs, (D * a.v_dim + 1023) / 1024), dim3(256), 0, st, a, D, sg.rows, sg.count);
+  }
+  hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, false>), grid, block, 0, st, a, sg.rows, sg.count);
+}
+
+template <bool Silu>
+void launch_chunk_scan(const ChunkScanArgs& a, int head_dim, ScanSegments sg, hipStream_t st) {
+  const int nw = scan_waves(static_cast<int64_t>(a.num_seqs) * sg.count * a.num_heads, a.v_dim);
+  auto waves = [&](auto d) {
+    constexpr int D = decltype(d)::value;
+    if (nw == 8) launch_chunk_scan_as<D, 8, Silu>(a, sg, st);
+    else if (nw == 4) launch_chunk_scan_as<D, 4, Silu>(a, sg, st);
+    else launch_chunk_scan_as<D, 2, Silu>(a, sg, st);
+  };
+  if (head_dim == 32) waves(std::integral_constant<int, 32>{});
+  else if (head_dim == 64) waves(std::integral_constant<int, 64>{});
+  else waves(std::integral_constant<int, 128>{});
+}
+
+}  // namespace
+}  // namespace hymeta
