@@ -1,0 +1,34 @@
+"""The delta rule over many (sequence, head) pairs runs in slices of 128 value columns: against the same sequences one at a
+time, which run in narrow slices."""
+import pytest
+import torch
+
+from _util import gen
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("D,Dv,H,Hk", [(32, 128, 16, 4), (64, 256, 8, 8), (96, 128, 16, 16), (128, 128, 16, 8)])
+def test_wide_slices_equal_narrow_ones(D, Dv, H, Hk):
+    """Both multiply the same operands (fp32 as two bf16 parts, 2^-17 of the operand) and add in another order: 1e-5 of the
+    norm covers what that rounding grows to over three chunks.  Rows at a chunk's edges, several chunks, a portion that goes
+    token by token, carried states and one sequence without a slot."""
+    from vllm_hymeta import hip_ops
+    lens = [8, 63, 64, 65, 130, 7, 128, 129, 20, 1, 192]
+    T, S = sum(lens), len(lens)
+    g = gen(D + Dv)
+    q, k, v = (torch.randn(T, n, d, generator=g).bfloat16().to(DEV) for n, d in ((Hk, D), (Hk, D), (H, Dv)))
+    beta = torch.randn(T, H, generator=g).bfloat16().to(DEV)
+    l2 = (-torch.rand(T, H, generator=g) * 0.2).to(DEV)
+    state = (torch.randn(S, H, D, Dv, generator=g) * 0.1).to(DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    context, slots = [5 if i % 2 else 0 for i in range(S)], [i if i != 3 else -1 for i in range(S)]
+    wide, narrow = state.clone(), state.clone()
+    starts = [sum(lens[:i]) for i in range(S + 1)]
+    out = hip_ops.delta_rule(q, k, v, beta, l2, wide, i32(starts), i32(context), i32(slots), max(lens), D ** -0.5, 1e-6)
+    for s in range(S):
+        a, b = starts[s], starts[s + 1]
+        one = hip_ops.delta_rule(q[a:b], k[a:b], v[a:b], beta[a:b], l2[a:b], narrow, i32([0, b - a]), i32(context[s:s + 1]), i32(slots[s:s + 1]), b - a, D ** -0.5, 1e-6)
+        assert float((out[a:b] - one).norm() / one.norm()) < 1e-5, s
+        assert float((wide[s] - narrow[s]).norm() / narrow[s].norm()) < 1e-5, s

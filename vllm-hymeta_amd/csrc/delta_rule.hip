@@ -4,6 +4,7 @@
 // with unit-length queries and keys, the state fp32 and carried per sequence.  Beside the decayed scan (decay_scan.hip),
 // whose state only adds what a token brings.
 #include "act_types.h"
+#include "lds_copy.h"
 
 #include <type_traits>
 
@@ -197,6 +198,10 @@ constexpr int kChunk = HYMETA_DELTA_CHUNK;
 // Workgroups (with slices of 32 value columns) up to which the second launch runs slices of 16: measured for one prompt of 8192
 // with 28 heads of 128 x 128 (112 workgroups) 357 against 405 us, with 64 heads (256) 706 against 566 us.
 constexpr int kFewGroups = 128;
+// Workgroups of slices of 128 columns above which the second launch takes those: slices of 32 are then more than the 512
+// workgroups that run at the same time.  With 28 heads of 128 x 128 (16 for the last two): 5 portions of 1801 rows 310 us in
+// narrow slices, 281 in wide ones (140 workgroups); 16 of 500 250 and 191; 40 of 300 414 and 276; 8 of 700 (128) 102 and 108.
+constexpr int kManyWideGroups = 128;
 constexpr int kChunkMinRows = 8;            // shorter portions go token by token
 constexpr int kMat = kChunk * kChunk;
 // Where the second launch reads 64 x 64 matrices (or the chunk's keys) as matrix operands, they lie in the operand's own
@@ -617,6 +622,182 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(hymeta_delta_rule
   }
 }
 
+// The same over wide slices: grid = (heads, sequences, value columns in slices of 128), 8 waves of 16 columns.  Every step
+// of a chunk keeps to its columns, so a wave runs alone from barrier to barrier: the state, the right-hand side and U are
+// accumulators (a lane holds four consecutive rows of one column), and a pair of such blocks IS the operand of the next
+// product with the reduced index in the order 4 g4 + e, 16 + 4 g4 + e - 4; the other operand is read from LDS in that order.
+// What a chunk brings is copied to LDS a chunk ahead, once for all columns; a chunk's outputs are stored in the next one, so
+// that the wait for the copies does not wait for stores just issued.
+// Bound by LDS reads (every wave reads the chunk's 73 KB) and the matrix pipes, about alike.  About 6.7 us a chunk on a
+// compute unit, two waves on a SIMD; 4 workgroups of slices of 32 take 8.2.
+template <int D>
+__global__ __launch_bounds__(512) void delta_chunk_wide_kernel(hymeta_delta_rule_args a, int64_t chunks) {
+  constexpr int NW = 8;
+  constexpr int SD = D / 32, DB = D / 16, kRowsBytes = 3 * D * kChunk * 2, kMatBytes = 6 * 1024, kImage = kRowsBytes + 4 * kMatBytes + 1024;
+  constexpr int kCopies = kImage / 1024;
+  __shared__ __attribute__((aligned(16))) char images[2][kImage];       // keys, queries, transposed keys | T hi, lo, P hi, lo | beta, rhs, read, write
+  const int h = blockIdx.x, s = blockIdx.y, vs = blockIdx.z;
+  const int r0 = a.query_start_loc[s], rows = a.query_start_loc[s + 1] - r0;
+  if (rows < kChunkMinRows) return;
+  const int lane = threadIdx.x & 63, n = lane & 15, g4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int H = a.num_heads, G = a.num_qk_heads, Dv = a.v_dim, g = h / (H / G), col = vs * 16 * NW + 16 * wave + n;
+  const int64_t first = r0 / kChunk + s;
+  const ChunkPlace* places = static_cast<const ChunkPlace*>(a.workspace) + first * H + h;
+  const char* packed = static_cast<const char*>(a.workspace) + rows_at(chunks, H) + (first * G + g) * kRowsBytes;
+  const int num = (rows + kChunk - 1) / kChunk;
+  auto copy = [&](int c, char* image) __attribute__((always_inline)) {
+    const char* rows_from = packed + static_cast<int64_t>(c) * G * kRowsBytes + 16 * lane;
+    const char* place = reinterpret_cast<const char*>(places + static_cast<int64_t>(c) * H) + 16 * lane;
+#pragma unroll
+    for (int step = 0; step < (kCopies + NW - 1) / NW; ++step) {
+      const int i = wave + NW * step;
+      if (i >= kCopies) break;
+      // (of a lower triangular matrix the blocks of 16 rows and 32 columns that are not all zero: 0, 2, 4, 5, 6, 7)
+      const int m = i - kRowsBytes / 1024, b = m % 6;
+      const char* from = m < 0 ? rows_from + 1024 * i : m < 24 ? place + 8192 * (m / 6) + 1024 * (b < 2 ? 2 * b : b + 2) : place + 32768;
+      copy16_to_lds(from, image + 1024 * i);
+    }
+  };
+  const uint16_t* vp = static_cast<const uint16_t*>(a.v) + static_cast<int64_t>(h) * Dv + vs * 16 * NW;
+  const int v_stride = static_cast<int>(a.v_stride_t), HDv = H * Dv;
+  uint32_t vv[4][4];
+  float total = 0.f;
+  auto fetch = [&](int c) __attribute__((always_inline)) {
+    const int last = rows - 1 - c * kChunk;
+    const int64_t t0 = r0 + static_cast<int64_t>(c) * kChunk;
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) vv[ib][r] = vp[t0 * a.v_stride_t + static_cast<uint32_t>(min(16 * ib + 4 * g4 + r, last) * v_stride + 16 * wave + n)];
+    total = places[static_cast<int64_t>(c) * H].total;
+  };
+  copy(0, images[0]);
+  fetch(0);
+  const int slot = a.slot_idx[s];
+  float* st = slot >= 0 ? a.state + (static_cast<int64_t>(slot) * H + h) * D * Dv + col : nullptr;
+  const bool carry = st != nullptr && a.context_lens[s] > 0;
+  f32x4v S[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[db][r] = carry ? st[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv] : 0.f;
+  const int half = ((g4 >> 1) * 16 + n) * 16 + 8 * (g4 & 1);             // this lane's first half of a 1 KB operand block
+  auto operand = [&](const char* block) {
+    const u32x2 x = *reinterpret_cast<const u32x2*>(block + half), y = *reinterpret_cast<const u32x2*>(block + half + 512);
+    return frag(u32x4{x[0], x[1], y[0], y[1]});
+  };
+  auto split8 = [&](const f32x4v& x, const f32x4v& y, bf16x8& hi, bf16x8& lo) {
+    const float p[4] = {x[0], x[1], x[2], x[3]}, q[4] = {y[0], y[1], y[2], y[3]};
+    u32x2 ph, pl, qh, ql;
+    split4(p, ph, pl), split4(q, qh, ql);
+    hi = frag(u32x4{ph[0], ph[1], qh[0], qh[1]}), lo = frag(u32x4{pl[0], pl[1], ql[0], ql[1]});
+  };
+  float* out = static_cast<float*>(a.out) + static_cast<int64_t>(r0) * HDv + static_cast<int64_t>(h) * Dv + vs * 16 * NW;
+  f32x4v y[4];
+  auto store = [&](int c, auto full) __attribute__((always_inline)) {
+    const int live = rows - c * kChunk;
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * ib + 4 * g4 + r;
+        if (decltype(full)::value || i < live) out[static_cast<int64_t>(c) * kChunk * HDv + static_cast<uint32_t>(i * HDv + 16 * wave + n)] = y[ib][r];
+      }
+  };
+  for (int c = 0; c < num; ++c) {
+    const char* image = images[c & 1];
+    copies_landed_barrier();                 // this chunk's image is there, the other's readers are done
+    // what the compiler still counts as in flight has landed: it is used here, in front of the next copies, which it would
+    // otherwise wait for as well
+    float value[4][4], decay = total;
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        value[ib][r] = bf2f(static_cast<uint16_t>(vv[ib][r]));
+        asm volatile("" : "+v"(value[ib][r]));
+      }
+    asm volatile("" : "+v"(decay));
+    if (c > 0) store(c - 1, std::true_type{});
+    if (c + 1 < num) {
+      copy(c + 1, images[(c + 1) & 1]);
+      fetch(c + 1);
+    }
+    const char *keys = image, *queries = image + D * kChunk * 2, *transposed = image + 2 * D * kChunk * 2, *mats = image + kRowsBytes;
+    const float* scale = reinterpret_cast<const float*>(mats + 4 * kMatBytes) + 4 * g4;      // beta, rhs, read, write of rows 4 g4 ..
+    f32x4v x[4];
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib) x[ib] = y[ib] = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int sd = 0; sd < SD; ++sd) {
+      bf16x8 sh, sl;
+      split8(S[2 * sd], S[2 * sd + 1], sh, sl);
+#pragma unroll
+      for (int ib = 0; ib < 4; ++ib) {
+        const bf16x8 kf = operand(keys + 1024 * (ib * SD + sd)), qf = operand(queries + 1024 * (ib * SD + sd));
+        x[ib] = mfma16(kf, sh, x[ib]);
+        y[ib] = mfma16(qf, sh, y[ib]);
+        x[ib] = mfma16(kf, sl, x[ib]);
+        y[ib] = mfma16(qf, sl, y[ib]);
+      }
+    }
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib) {
+      const f32x4v beta = *reinterpret_cast<const f32x4v*>(scale + 16 * ib), rhs = *reinterpret_cast<const f32x4v*>(scale + kChunk + 16 * ib);
+      const f32x4v read = *reinterpret_cast<const f32x4v*>(scale + 2 * kChunk + 16 * ib);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[ib][r] = beta[r] * value[ib][r] - rhs[r] * x[ib][r];
+      y[ib] *= read;
+    }
+    // U = T x right-hand side; then U and U times the rows' write factors as operands
+    f32x4v u[4];
+    bf16x8 hi[2], lo[2], wh[2], wl[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) split8(x[2 * kk], x[2 * kk + 1], hi[kk], lo[kk]);
+    auto lower = [&](int matrix, f32x4v* to) __attribute__((always_inline)) {
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int ib = 2 * kk; ib < 4; ++ib) {
+          const char* block = mats + 2 * matrix * kMatBytes + 1024 * (ib < 2 ? ib : 2 * ib - 2 + kk);
+          const bf16x8 mh = operand(block), ml = operand(block + kMatBytes);
+          to[ib] = mfma16(mh, hi[kk], to[ib]);
+          to[ib] = mfma16(mh, lo[kk], to[ib]);
+          to[ib] = mfma16(ml, hi[kk], to[ib]);
+        }
+    };
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib) u[ib] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    lower(0, u);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      split8(u[2 * kk], u[2 * kk + 1], hi[kk], lo[kk]);
+      const f32x4v w0 = *reinterpret_cast<const f32x4v*>(scale + 3 * kChunk + 32 * kk), w1 = *reinterpret_cast<const f32x4v*>(scale + 3 * kChunk + 32 * kk + 16);
+      split8(u[2 * kk] * w0, u[2 * kk + 1] * w1, wh[kk], wl[kk]);
+    }
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      f32x4v acc = S[db] * decay;
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        const bf16x8 kt = operand(transposed + 1024 * (2 * db + kk));
+        acc = mfma16(kt, wh[kk], acc);
+        acc = mfma16(kt, wl[kk], acc);
+      }
+      S[db] = acc;
+    }
+    lower(1, y);
+  }
+  store(num - 1, std::false_type{});
+  if (st != nullptr) {
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) st[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv] = S[db][r];
+  }
+}
+
 inline bool chunk_dims(int head_dim, int v_dim, int act_dtype) {
   return act_dtype == HYMETA_BF16 && head_dim >= 32 && head_dim <= 128 && head_dim % 32 == 0 && v_dim % 32 == 0 && v_dim / 16 <= 65535;
 }
@@ -651,6 +832,11 @@ void launch_chunks(const hymeta_delta_rule_args& a, hipStream_t st, int64_t chun
       hipLaunchKernelGGL((delta_chunk_scan_kernel<D, 1>), dim3(a.num_heads, a.num_seqs, a.v_dim / 16), dim3(256), 0, st, a, chunks);
       return;
     }
+  }
+  const int64_t wide = static_cast<int64_t>(a.num_heads) * a.num_seqs * (a.v_dim / 128);
+  if (a.v_dim % 128 == 0 && wide > kManyWideGroups && a.v_stride_t < (1 << 23) && static_cast<int64_t>(a.num_heads) * a.v_dim < (1 << 22)) {
+    hipLaunchKernelGGL((delta_chunk_wide_kernel<D>), dim3(a.num_heads, a.num_seqs, a.v_dim / 128), dim3(512), 0, st, a, chunks);
+    return;
   }
   hipLaunchKernelGGL((delta_chunk_scan_kernel<D, 2>), dim3(a.num_heads, a.num_seqs, a.v_dim / 32), dim3(256), 0, st, a, chunks);
 }
