@@ -81,3 +81,24 @@ def test_lightning(D, Dv, H, lens):
     ref, after = _recurrence(x[:, :H * D].reshape(T, H, D), x[:, H * D:2 * H * D].reshape(T, H, D), x[:, 2 * H * D:].reshape(T, H, Dv),
                              one * torch.log2(decay.double()), one, torch.zeros(H, dtype=torch.float64), state.double(), lens, carried)
     assert _rel(out, ref) < 2 ** -8 and _rel(got, after) < 2 ** -8, (_rel(out, ref), _rel(got, after))
+
+
+@pytest.mark.parametrize("D,Dv,H,lens", [(128, 128, 2, [64, 200]), (64, 96, 2, [1300]), (32, 64, 3, [65, 8])])
+def test_lightning_state_holds_keys_in_two_parts(D, Dv, H, lens):
+    """The states against silu(k) in 64 bits and silu(v) as the bf16 it is rounded to: the keys' two parts leave 2^-17 of an
+    operand.  The silu's own error, 2^-21, flips the rounding of about 2^-12 of the values by 2^-8 of the value: 2^-14 of the
+    norm.  Twice their sum; keys in one part would leave 2^-9 / sqrt(3)."""
+    from vllm_hymeta import hip_ops
+    T, S = sum(lens), len(lens)
+    g = gen(D + Dv + H + 2)
+    qkv = torch.randn(T, H * (2 * D + Dv), generator=g).bfloat16()
+    state, carried = torch.randn(S, H, D, Dv, generator=g), [i % 2 == 0 for i in range(S)]
+    decay = torch.rand(H, generator=g) * 0.2 + 0.8
+    starts, context, slots = _layout(lens, carried)
+    got = state.to(DEV)
+    hip_ops.lightning_attention(qkv.to(DEV), got, decay.to(DEV), H, D, Dv, starts, context, slots, max(lens))
+    x = torch.nn.functional.silu(qkv.double())
+    one = torch.ones(T, H, dtype=torch.float64)
+    _, after = _recurrence(x[:, :H * D].reshape(T, H, D), x[:, H * D:2 * H * D].reshape(T, H, D), x[:, 2 * H * D:].bfloat16().double().reshape(T, H, Dv),
+                           one * torch.log2(decay.double()), one, torch.zeros(H, dtype=torch.float64), state.double(), lens, carried)
+    assert _rel(got, after) < 2 * (2 ** -17 + 2 ** -14), _rel(got, after)

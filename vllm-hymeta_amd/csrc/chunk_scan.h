@@ -38,7 +38,7 @@ inline int scan_waves(int64_t lanes, int v_dim) {
 // state and the sum of its log2 decays), the summaries are chained into the states in front of the segments, then every
 // segment runs from its state.  The summaries read the keys and values a second time, so fewer than three segments do not
 // pay.  As many segments as run at the same time, eight waves to a compute unit: one prompt of 8192 rows of 28 heads of 128
-// columns took 138 us (lightning) and 120 (plain decays) in 256 workgroups of eight waves, 152 and 136 in 512, 175 and 156
+// columns took 138 us (lightning, the keys in one part) and 120 (plain decays) in 256 workgroups of eight waves, 152 and 136 in 512, 175 and 156
 // in 1024; of 64 columns 131 us in 512 workgroups of four, 189 in 256, 147 in 1024.  At least 192 rows each: three portions
 // of 700 rows of 16 heads took 39 us in three segments, 49 in one.
 struct ScanSegments { int rows, count; };
@@ -100,10 +100,11 @@ struct RowBuffer {
 // needs transposed is read transposed.  The decays of the state's update go onto the values (a wave splits its own 16 columns
 // into hi + lo bf16 parts) and not onto the keys; the chunk's own weights are computed once per workgroup, a block of 16 rows
 // x 32 keys per wave, and handed over in LDS as fragments.  What enters a product from fp32 goes in as hi + lo parts, two
-// products, so that it keeps 16 bits of mantissa.
+// products, so that it keeps 16 bits of mantissa; so do the keys behind their silu in the state's update (three products: the
+// values, rounded to bf16 as in the outputs, carry the decays).
 // Bound by vector arithmetic between the barriers of a chunk: 2 x 16 cycles of exponential and reciprocal per silu'd value,
 // splits, scales; the matrix pipes are busy about a quarter of the time, memory far less.  One prompt of 8192 rows, 28 heads
-// of 128 x 128: lightning 351 -> 141 us (summaries 40, states 8, rows 88), plain decays 283 -> 121; with 64 value columns and
+// of 128 x 128: lightning 351 -> 152 us (141 with the keys in one part), plain decays 283 -> 121; with 64 value columns and
 // decays per row 316 -> 131; before, 4 waves to 32 value columns, each such workgroup with its own staging, weights and an
 // image of the state in LDS.
 template <int D, int NW, bool Silu, bool Summarise>
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
   typedef ChunkOrder<KC> KOrder;
   typedef ChunkOrder<VC> VOrder;
   __shared__ __attribute__((aligned(16))) char s_k[kScanRows * KP], s_v[kScanRows * VP];
-  __shared__ __attribute__((aligned(16))) char s_q[Summarise ? 16 : kScanRows * KP], s_vlo[Silu ? kScanRows * VP : 16];
+  __shared__ __attribute__((aligned(16))) char s_q[Summarise ? 16 : kScanRows * KP], s_klo[Silu ? kScanRows * KP : 16];
   __shared__ __attribute__((aligned(16))) u32x4 s_p[Summarise ? 1 : 6][2][64];
   __shared__ __attribute__((aligned(16))) float s_cum[kScanRows], s_b[kScanRows], s_w[kScanRows];
   const int h = blockIdx.x, s = blockIdx.y / nseg, seg = blockIdx.y % nseg, vs = blockIdx.z;
@@ -183,7 +184,11 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
       if (kScanRows * KC % NT != 0 && j >= kScanRows) break;
       const int at = j * KP + 16 * (ch ^ KOrder::twist(j));
       u32x4 x = rk[u], lo;
-      if (Silu && (decltype(full)::value || j < nrow)) silu8(rk[u], x, lo);
+      if constexpr (Silu) {
+        lo = u32x4{0u, 0u, 0u, 0u};
+        if (decltype(full)::value || j < nrow) silu8(rk[u], x, lo);
+        st16(s_klo + at, lo);
+      }
       st16(s_k + at, x);
       if constexpr (!Summarise) {
         x = rq[u];
@@ -194,11 +199,8 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
 #pragma unroll
     for (int u = 0; u < VPT; ++u) {
       const int idx = tid + NT * u, j = idx / VC, ch = idx % VC, at = j * VP + 16 * (ch ^ VOrder::twist(j));
-      u32x4 x = rv[u], lo = u32x4{0u, 0u, 0u, 0u};
-      if constexpr (Silu) {
-        if (decltype(full)::value || j < nrow) silu8(rv[u], x, lo);
-        st16(s_vlo + at, lo);
-      }
+      u32x4 x = rv[u], lo;
+      if (Silu && (decltype(full)::value || j < nrow)) silu8(rv[u], x, lo);
       st16(s_v + at, x);
     }
     if (wave == 0) {
@@ -219,7 +221,8 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
       s_cum[lane] = cum;
       const float b = a.v_scale ? rb : 1.f;
       s_b[lane] = b;
-      s_w[lane] = lane < nrow ? __builtin_amdgcn_exp2f(total - cum) * b : 0.f;
+      const float left = Silu ? static_cast<float>(nrow - 1 - lane) * l2_const : total - cum;
+      s_w[lane] = lane < nrow ? __builtin_amdgcn_exp2f(left) * b : 0.f;
     }
   };
   auto stage = [&](int nrow) __attribute__((always_inline)) {
@@ -237,8 +240,8 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
     return __builtin_bit_cast(bf16x8, (u32x4{x[0], x[1], y[0], y[1]}));
   };
   // keys 32 kk + 4 g4 + e for e < 4, 32 kk + 16 + 4 g4 + e - 4 after, of column 16 db + n / of this wave's value column n
-  auto key_frag = [&](int db, int kk) {
-    const char* p = s_k + (32 * kk + Rt) * KP + 16 * ((2 * db + ((n & 3) >> 1)) ^ kT) + 8 * (n & 1);
+  auto key_frag = [&](const char* img, int db, int kk) {
+    const char* p = img + (32 * kk + Rt) * KP + 16 * ((2 * db + ((n & 3) >> 1)) ^ kT) + 8 * (n & 1);
     return frag_of(read_transposed(p), read_transposed(p + 16 * KP));
   };
   auto value_frag = [&](const char* img, int kk) {
@@ -278,10 +281,17 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
 #pragma unroll
             for (int sd = 0; sd < SD; ++sd) sc = scan_mfma(row_frag(s_k, jb, sd), row_frag(s_q, ib, sd), sc);
           }
-          const f32x4s cj = *reinterpret_cast<const f32x4s*>(s_cum + 16 * jb + 4 * g4), bj = *reinterpret_cast<const f32x4s*>(s_b + 16 * jb + 4 * g4);
+          f32x4s span, bj;                             // log2 of the decay between row j and row i; j's input weight
+          if constexpr (Silu) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) span[r] = static_cast<float>(i - 16 * jb - 4 * g4 - r) * l2_const, bj[r] = 1.f;
+          } else {
+            span = cum_i - *reinterpret_cast<const f32x4s*>(s_cum + 16 * jb + 4 * g4);
+            bj = *reinterpret_cast<const f32x4s*>(s_b + 16 * jb + 4 * g4);
+          }
           float p[4];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) p[r] = 16 * jb + 4 * g4 + r <= i ? sc[r] * __builtin_amdgcn_exp2f(cum_i - cj[r]) * bj[r] : 0.f;
+          for (int r = 0; r < 4; ++r) p[r] = 16 * jb + 4 * g4 + r <= i ? sc[r] * __builtin_amdgcn_exp2f(span[r]) * bj[r] : 0.f;
           uint32_t x, y;
           split_pair(p[0], p[1], x, y), hi[2 * t] = x, lo[2 * t] = y;
           split_pair(p[2], p[3], x, y), hi[2 * t + 1] = x, lo[2 * t + 1] = y;
@@ -340,15 +350,12 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       const u32x4 x = __builtin_bit_cast(u32x4, vf[kk]);
-      u32x4 y = u32x4{0u, 0u, 0u, 0u};
-      if constexpr (Silu) y = __builtin_bit_cast(u32x4, value_frag(s_vlo, kk));
       const f32x4s w0 = *reinterpret_cast<const f32x4s*>(s_w + 32 * kk + 4 * g4), w1 = *reinterpret_cast<const f32x4s*>(s_w + 32 * kk + 16 + 4 * g4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float wa = e < 2 ? w0[2 * e] : w1[2 * e - 4], wb = e < 2 ? w0[2 * e + 1] : w1[2 * e - 3];
         uint32_t hi, lo;
-        if constexpr (Silu) split_pair((lo_bf(x[e]) + lo_bf(y[e])) * wa, (hi_bf(x[e]) + hi_bf(y[e])) * wb, hi, lo);
-        else split_pair(lo_bf(x[e]) * wa, hi_bf(x[e]) * wb, hi, lo);
+        split_pair(lo_bf(x[e]) * wa, hi_bf(x[e]) * wb, hi, lo);
         wv[kk][0][e] = hi, wv[kk][1][e] = lo;
       }
     }
@@ -358,9 +365,10 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
       f32x4s acc = S[db] * chunk_decay;
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
-        const bf16x8 kf = key_frag(db, kk);
+        const bf16x8 kf = key_frag(s_k, db, kk);
         acc = scan_mfma(kf, __builtin_bit_cast(bf16x8, wv[kk][0]), acc);
         acc = scan_mfma(kf, __builtin_bit_cast(bf16x8, wv[kk][1]), acc);
+        if constexpr (Silu) acc = scan_mfma(key_frag(s_klo, db, kk), __builtin_bit_cast(bf16x8, wv[kk][0]), acc);
       }
       S[db] = acc;
     }
