@@ -28,7 +28,7 @@ def reference(q, k, v, scale, ctx, o, sink, a, gate):
         s = o["softcap"] * torch.tanh(s / o["softcap"])
     far = (i - j).clamp_min(0).double()
     if o["bias"] == "log":
-        s = s - a[:, None, None] * torch.log1p(NEAR * far)
+        s = s - a[:, None, None] * torch.log1p(o["near"] * far)
     elif o["bias"] == "linear":
         s = s - SLOPE * a[:, None, None] * far
     s = s.masked_fill(~seen, float("-inf"))
@@ -44,6 +44,9 @@ def reference(q, k, v, scale, ctx, o, sink, a, gate):
     ("rows", 64, 128, 2, 2, 64, [129, 64], [1, 512], dict(window=70, keep=9)),                   # one head a key/value head, kept keys
     ("rows", 64, 64, 6, 2, 128, [5, 3], [1000, 2000], dict(chunk=300, gate=True)),
     ("rows", 128, 128, 8, 2, 64, [3, 2], [3000, 63], dict(softcap=6.0, bias="log", sink=True)),  # slices, of which some see nothing
+    ("rows", 128, 128, 8, 2, 64, [70, 3], [200, 0], dict(sink=True, bias="log", near=98765.43)),     # steep biases: the nearest keys'
+    ("rows", 128, 128, 8, 2, 64, [70, 3], [200, 0], dict(sink=True, bias="log", near=987654.3)),     # logarithms from exact distances
+    ("latent", 192, 128, 8, 1, 64, [33, 3], [100, 0], dict(sink=True, bias="log", near=98765.43)),
     ("latent", 192, 128, 16, 1, 64, [8, 9, 2], [0, 63, 1500], dict(sink=True)),
     ("latent", 160, 128, 5, 1, 32, [70], [11], dict(bias="log")),
     ("latent", 128, 64, 3, 1, 64, [90, 2], [0, 900], dict(window=200)),
@@ -59,7 +62,7 @@ def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
     from vllm_hymeta import hip_ops
     dev, g = "cuda", torch.Generator().manual_seed(D + H)
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
-    o = dict(dict(sink=False, window=0, keep=0, chunk=0, softcap=0.0, bias=None, gate=False), **opts)
+    o = dict(dict(sink=False, window=0, keep=0, chunk=0, softcap=0.0, bias=None, gate=False, near=NEAR), **opts)
     key_heads = 1 if layout in ("latent", "shared") else G
     total = [n + c for n, c in zip(lens, ctxs)]
     keys = [torch.randn(t, key_heads, D, generator=g).bfloat16() for t in total]
@@ -91,7 +94,7 @@ def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
         max(lens), max(total), sink=sink is not None, sink_logits=None if sink is None else sink.to(dev), window_left=o["window"] - 1,
         keep_first=o["keep"], chunk=o["chunk"], softcap=o["softcap"], value_in_key=layout == "latent", shared_key=layout == "shared",
         scaled_key=layout == "scaled", bias_a=a.to(dev) if o["bias"] == "log" else None, slopes=(SLOPE * a).to(dev) if o["bias"] == "linear" else None,
-        bias_b=torch.full((H,), NEAR, device=dev) if o["bias"] == "log" else None,
+        bias_b=torch.full((H,), o["near"], device=dev) if o["bias"] == "log" else None,
         head_gate=torch.cat(gates).to(dev) if o["gate"] else None).double().cpu()
     at = 0
     for s, n in enumerate(lens):

@@ -24,7 +24,7 @@ constexpr float kLazyMax2 = 8.f;     // the softmax reference may trail a row's 
 // pass over the output registers on most tiles.
 // Bound by the vector and the matrix pipe in turn: with a logarithm and an exponential per score they are busy 45 and 41 % of
 // the time and hardly at once, whatever the number of waves (one row block a wave and four waves a SIMD: 785 us).  8192 rows x
-// 28 heads of 128 with 4 key/value heads, logarithmic bias: 1400 -> 750 us; a latent of 128 + 64: 1632 -> 760; a window of 1024:
+// 28 heads of 128 with 4 key/value heads, logarithmic bias: 1400 -> 765 us; a latent of 128 + 64: 1632 -> 760; a window of 1024:
 // 410 -> 214; key and value in one vector, window of 1024: 345 -> 219.
 template <int D, int DV, int Layout>
 struct RowShape {
@@ -134,8 +134,9 @@ __global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attenti
     __builtin_amdgcn_s_setprio(0);
     const bool masked = !(full && j0 + kTileKeys - 1 <= w_lo && j0 >= w_first_hi);
     const float ref = m == -INFINITY ? 0.f : m;
-    // the scores, in the base-2 domain, less the reference
-    const float d0 = static_cast<float>(pos - j0 - 4 * hh), near = fmaf(bb, d0, 1.f), slope = fmaf(ba, d0, -ref);
+    // the scores, in the base-2 domain, less the reference (the logarithm's argument from the exact distance: formed from
+    // the tile's it would lose 64 of the coefficient's ulps, on the nearest keys of a steep bias all of itself)
+    const float d0 = static_cast<float>(pos - j0 - 4 * hh), slope = fmaf(ba, d0, -ref);
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -147,7 +148,7 @@ __global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attenti
           float x = sc[t][4 * i + e];
           const float away = static_cast<float>(32 * t + 8 * i + e);
           if (S::Scaled) x = fmaf(x, f[e], fmaf(-ba, away, slope));
-          else if (Rule == kLogBias) x = fmaf(x, scale2, fmaf(ba, __builtin_amdgcn_logf(fmaf(-bb, away, near)), -ref));
+          else if (Rule == kLogBias) x = fmaf(x, scale2, fmaf(ba, __builtin_amdgcn_logf(fmaf(bb, d0 - away, 1.f)), -ref));
           else if (Rule == kPlain) x = fmaf(x, scale2, -ref);
           sc[t][4 * i + e] = x;
         }
@@ -163,7 +164,7 @@ __global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attenti
       if (a.bias_mode == HYMETA_BIAS_LOG_DISTANCE) {
 #pragma unroll
         for (int i = 0; i < 32; ++i)
-          sc[i >> 4][i & 15] = fmaf(ba, __builtin_amdgcn_logf(fmaf(-bb, static_cast<float>(32 * (i >> 4) + 8 * ((i & 15) >> 2) + (i & 3)), near)), sc[i >> 4][i & 15]);
+          sc[i >> 4][i & 15] = fmaf(ba, __builtin_amdgcn_logf(fmaf(bb, d0 - static_cast<float>(32 * (i >> 4) + 8 * ((i & 15) >> 2) + (i & 3)), 1.f)), sc[i >> 4][i & 15]);
       }
     }
     if (masked) {
