@@ -34,7 +34,7 @@ def reference(q, k, v, scale, ctx, o, sink, a, gate):
     s = s.masked_fill(~seen, float("-inf"))
     if sink is not None:
         s = torch.cat((s, sink[:, None, None].expand(len(sink), n, 1)), -1)
-    out = torch.einsum("hnj,hjc->nhc", torch.softmax(s, -1)[..., :ctx + n], v)
+    out = torch.einsum("hnj,hjc->nhc", torch.softmax(s, -1)[..., :ctx + n].nan_to_num(), v)      # (no keys: 0)
     return out if gate is None else out * torch.sigmoid(gate)[:, :, None]
 
 
@@ -47,6 +47,9 @@ def reference(q, k, v, scale, ctx, o, sink, a, gate):
     ("rows", 128, 128, 8, 2, 64, [70, 3], [200, 0], dict(sink=True, bias="log", near=98765.43)),     # steep biases: the nearest keys'
     ("rows", 128, 128, 8, 2, 64, [70, 3], [200, 0], dict(sink=True, bias="log", near=987654.3)),     # logarithms from exact distances
     ("latent", 192, 128, 8, 1, 64, [33, 3], [100, 0], dict(sink=True, bias="log", near=98765.43)),
+    ("rows", 128, 128, 4, 2, 64, [3, 200, 1, 2], [-1, -150, -1, -2], {}),                        # rows in front of their sequence
+    ("rows", 64, 64, 4, 2, 16, [3, 70, 1], [-2, -30, -1], dict(chunk=20)),
+    ("scaled", 64, 64, 4, 2, 64, [2, 70, 1], [-1, -30, 3000], dict(sink=True, window=30)),
     ("latent", 192, 128, 16, 1, 64, [8, 9, 2], [0, 63, 1500], dict(sink=True)),
     ("latent", 160, 128, 5, 1, 32, [70], [11], dict(bias="log")),
     ("latent", 128, 64, 3, 1, 64, [90, 2], [0, 900], dict(window=200)),
@@ -80,7 +83,7 @@ def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
         pages = order[at:at + need[s]]
         at += need[s]
         table[s, :need[s]] = torch.tensor(pages, dtype=torch.int32)
-        slots = torch.tensor([pages[p // page] * page + p % page for p in range(total[s])], device=dev)
+        slots = torch.tensor([pages[p // page] * page + p % page for p in range(total[s])], dtype=torch.int64, device=dev)
         if layout == "scaled":
             qk = torch.cat((torch.zeros(total[s], D).bfloat16(), keys[s].reshape(total[s], -1)), 1).to(dev)
             ones = torch.ones(D, device=dev)

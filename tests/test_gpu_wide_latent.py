@@ -30,7 +30,7 @@ def reference(q, rows, C, scale, sink, window, keep, chunk, softcap, bias, gate,
     s = s.masked_fill(~seen, float("-inf"))
     if sink is not None:
         s = torch.cat((s, sink[:, None, None].expand(H, n, 1)), -1)
-    p = torch.softmax(s, -1)[..., :ctx + n]
+    p = torch.softmax(s, -1)[..., :ctx + n].nan_to_num()      # (no keys: 0)
     o = torch.einsum("hnj,jc->nhc", p, rows[:, :C])
     return o if gate is None else o * torch.sigmoid(gate)[:, :, None]
 
@@ -42,6 +42,8 @@ def reference(q, rows, C, scale, sink, window, keep, chunk, softcap, bias, gate,
     (384, 3, 32, [150, 1, 2], [0, 200, 1], dict(window=70, keep=5)),         # kept first keys ahead of the window
     (256, 4, 16, [64, 1, 1], [65, 0, 129], dict(chunk=48, gate=True)),
     (512, 1, 128, [129, 1], [0, 511], dict(softcap=5.0, bias=True)),
+    (512, 16, 64, [1, 3, 20, 1], [-1, -1, -10, 300], {}),                    # rows in front of their sequence
+    (256, 4, 16, [1, 70, 2], [-1, -30, -2], dict(chunk=20, sink=True)),
     (256, 33, 64, [1] * 5, [0, 15, 16, 1000, 63], dict(sink=True, window=33)),
 ])
 def test_against_64_bits(C, H, page, lens, ctxs, opts):

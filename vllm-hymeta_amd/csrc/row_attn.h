@@ -77,15 +77,15 @@ __global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attenti
   for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[cb][i] = 0.f;
-  // positions the block's and the wave's rows span
-  const int p_lo = ctx + r0 / group, p_hi = ctx + (min(rows, r0 + S::kRows) - 1) / group;
+  // positions the block's and the wave's rows span (rows in front of the sequence, at positions below 0, see nothing)
+  const int p_lo = max(0, ctx + r0 / group), p_hi = ctx + (min(rows, r0 + S::kRows) - 1) / group;
   const int w_lo = ctx + min(rows - 1, w0) / group, w_hi = ctx + min(rows - 1, w0 + 31) / group;
   const int w_first_lo = first_key(a, w_lo), w_first_hi = first_key(a, w_hi);
   const bool full = w0 + 32 <= rows, any = w0 < rows;
   // the tiles: those of the kept first keys that lie before the window's first, then the window's
   const int from = first_key(a, p_lo) / kTileKeys * kTileKeys;
   const int kept = bounded(a) ? min((a.keep_first + kTileKeys - 1) / kTileKeys * kTileKeys, from) / kTileKeys : 0;
-  const int tiles = kept + (p_hi - from) / kTileKeys + 1;
+  const int tiles = p_hi < 0 ? 0 : kept + (p_hi - from) / kTileKeys + 1;
   const int per = (tiles + splits - 1) / splits, t_lo = split * per, t_hi = min(tiles, t_lo + per);
   auto key0 = [&](int t) { return t < kept ? t * kTileKeys : from + (t - kept) * kTileKeys; };
 

@@ -129,15 +129,15 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
 #pragma unroll
     for (int st = 0; st < kSteps; ++st) qf[st] = ok ? __builtin_bit_cast(bf16x8, ld16g(qrow + 32 * st + 8 * g4)) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
   }
-  // positions the block's and the wave's rows span
-  const int p_lo = ctx + r0 / group, p_hi = ctx + (min(rows, r0 + kWideRows) - 1) / group;
+  // positions the block's and the wave's rows span (rows in front of the sequence, at positions below 0, see nothing)
+  const int p_lo = max(0, ctx + r0 / group), p_hi = ctx + (min(rows, r0 + kWideRows) - 1) / group;
   const int w_lo = ctx + min(rows - 1, r0 + 16 * wave) / group, w_hi = ctx + min(rows - 1, r0 + 16 * wave + 15) / group;
   const int w_first = first_key(a, w_hi);
   const bool full = r0 + 16 * wave + 16 <= rows;
   // the tiles: those of the kept first keys that lie before the window's first, then the window's
   const int from = first_key(a, p_lo) / kWideKeys * kWideKeys;
   const int kept = bounded(a) ? min((a.keep_first + kWideKeys - 1) / kWideKeys * kWideKeys, from) / kWideKeys : 0;
-  const int all = kept + (p_hi - from) / kWideKeys + 1, per = (all + splits - 1) / splits;
+  const int all = p_hi < 0 ? 0 : kept + (p_hi - from) / kWideKeys + 1, per = (all + splits - 1) / splits;
   const int t0 = split * per, tiles = min(all - t0, per);          // this slice's
   auto key0 = [&](int t) { return t0 + t < kept ? (t0 + t) * kWideKeys : from + (t0 + t - kept) * kWideKeys; };
 
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(64 * kLatentWaves) void latent_decode_kernel(hymeta
   const int first = first_key(a, pos);
   const int from = first / kTile * kTile;
   const int kept = bounded(a) ? min((a.keep_first + kTile - 1) / kTile * kTile, from) / kTile : 0;
-  const int tiles = kept + (pos - from) / kTile + 1, per = (tiles + splits - 1) / splits;
+  const int tiles = pos < 0 ? 0 : kept + (pos - from) / kTile + 1, per = (tiles + splits - 1) / splits;
   const int v_lo = split * per, v_hi = min(tiles, v_lo + per) - 1;
   auto key0 = [&](int v) { return (v < kept ? v * kTile : from + (v - kept) * kTile) + kLatentKeys * wave; };
 
