@@ -111,3 +111,17 @@ def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
         assert torch.isfinite(got).all()
         assert (got - ref).norm() <= BOUND * ref.norm(), (s, float((got - ref).norm() / ref.norm()))
         at += n
+
+
+@pytest.mark.parametrize("D,Dv", [(128, 128), (576, 512)])
+def test_rows_behind_the_last_portion_stay_untouched(D, Dv, monkeypatch):
+    """Six rows more than the portions have, with keys cut into slices: nothing is written for them."""
+    from vllm_hymeta import hip_ops
+    dev = "cuda"
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
+    inside, empty = D != Dv, torch.empty
+    q, cache = torch.randn(11, 4, D, device=dev).bfloat16(), torch.randn(32, 64, 1, D if inside else D + Dv, device=dev).bfloat16()
+    monkeypatch.setattr(torch, "empty", lambda *size, **kw: empty(*size, **kw).fill_(7))
+    out = hip_ops.sink_attention(q, cache, torch.arange(32, dtype=torch.int32, device=dev)[None], i32([0, 5]), i32([2048]), 1, D, Dv, D ** -0.5, 5, 2048,
+                                 value_in_key=inside)
+    assert (out[5:] == 7).all() and torch.isfinite(out).all() and not (out[:5] == 7).all()

@@ -919,7 +919,8 @@ __global__ __launch_bounds__(kCombineThreads) void sink_attention_decode_combine
 // grid = (rows, heads): the rows of prompts' portions whose keys were cut into slices.
 __global__ __launch_bounds__(kCombineThreads) void sink_attention_rows_combine_kernel(hymeta_sink_attention_args a, int splits) {
   const int t = blockIdx.x, h = blockIdx.y, s = seq_of_row(a.query_start_loc, a.num_seqs, t);
-  if (a.query_start_loc[s + 1] - a.query_start_loc[s] <= 1) return;
+  const int end = a.query_start_loc[s + 1];
+  if (end - a.query_start_loc[s] <= 1 || t >= end) return;      // (rows behind the last portion have no partials)
   const size_t row = partial_row_floats(a.v_dim);
   combine_row(a, static_cast<const float*>(a.workspace) + (static_cast<size_t>(t) * a.num_heads + h) * splits * row, row, splits, t, h);
 }
