@@ -1411,7 +1411,8 @@ typedef struct hymeta_lightning_attention_args {
   void* workspace;             /* hymeta_lightning_attention_workspace_bytes(...) bytes, or NULL when that is 0 */
   size_t workspace_bytes;
 } hymeta_lightning_attention_args;
-/* > 0 for steps with long portions: they run in segments side by side (summarise / chain / apply: three launches). */
+/* > 0 where a long portion beside single rows would run in segments side by side (summarise / chain / apply: three launches).
+ * Enough for steps of fewer sequences and shorter portions too. */
 size_t hymeta_lightning_attention_workspace_bytes(int32_t num_seqs, int32_t num_heads, int32_t head_dim, int32_t v_dim,
                                                   int32_t max_query_len);
 int hymeta_lightning_attention(const hymeta_lightning_attention_args* args, hymeta_stream_t stream);
@@ -1683,7 +1684,8 @@ typedef struct hymeta_decay_scan_args {
   void* workspace;             /* hymeta_decay_scan_workspace_bytes(...) bytes, or NULL when that is 0 */
   size_t workspace_bytes;
 } hymeta_decay_scan_args;
-/* > 0 for steps with long portions: they run in segments side by side (summarise / chain / apply: three launches). */
+/* > 0 where a long portion beside single rows would run in segments side by side (summarise / chain / apply: three launches).
+ * Enough for steps of fewer sequences and shorter portions too. */
 size_t hymeta_decay_scan_workspace_bytes(int32_t num_seqs, int32_t num_heads, int32_t head_dim, int32_t v_dim, int32_t max_query_len);
 int hymeta_decay_scan(const hymeta_decay_scan_args* args, hymeta_stream_t stream);
 

@@ -142,3 +142,17 @@ def test_shapes_the_bf16_entry_point_takes_above_128_rows():
     assert takes(256, 3584, 3584, 0) == 1 and takes(256, 3584, 37888, 1) == 1         # K slices; whole tiles with the activation
     assert takes(256, 3584, 9472, 1) == 0 and takes(256, 256, 1024, 0) == 0 and takes(256, 3584, 152064, 2) == 1 and takes(256, 3584, 3584, 2) == 0              # too few workgroups: a library GEMM
     assert takes(128, 3584, 3584, 0) == 1 and takes(257, 18944, 3584, 0) == 0 and takes(64, 96, 64, 0) == 1
+
+
+@pytest.mark.parametrize("name", ["decay_scan", "lightning_attention"])
+def test_scan_workspace_covers_smaller_steps(name):
+    """A workspace for the largest step serves every smaller one, and a long portion has its segments whatever number of
+    sequences decode beside it."""
+    from vllm_hymeta import _C
+
+    size = getattr(_C.load(), f"hymeta_{name}_workspace_bytes")
+    for heads, v_dim in ((28, 128), (16, 64), (1, 32)):
+        by_seqs = [[size(s, heads, 128, v_dim, rows) for s in (1, 2, 5, 64, 256, 4096)] for rows in (1, 575, 576, 2048, 8192, 32768)]
+        assert all(a <= b for row in by_seqs for a, b in zip(row, row[1:]))
+        assert all(a <= b for col in zip(*by_seqs) for a, b in zip(col, col[1:]))
+        assert by_seqs[0][-1] == 0 and by_seqs[4][3] > 0

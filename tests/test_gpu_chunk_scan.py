@@ -36,6 +36,8 @@ def _rel(x, ref):
 SHAPES = [
     (128, 128, 2, [8, 63, 64, 65]), (128, 128, 32, [130, 9, 64, 100]), (128, 256, 2, [577, 40]), (64, 64, 3, [576, 640, 8]),
     (32, 32, 2, [1, 200, 600, 7]), (64, 96, 2, [129, 701]), (32, 128, 24, [70, 64, 9, 65, 66]), (128, 64, 2, [1200]),
+    # a long portion among single rows and short ones; long ones side by side, whose cuts have neighbouring numbers
+    (128, 128, 2, [1] * 9 + [1300] + [1] * 20 + [600, 7, 8, 400]), (32, 32, 2, [705, 1, 700, 1, 577, 640, 1]),
 ]
 
 

@@ -2,6 +2,8 @@
 // structs): loads widen to fp32, stores round once.
 #pragma once
 
+#include <algorithm>
+
 #include "common.h"
 
 namespace hymeta {
@@ -76,6 +78,13 @@ __device__ __forceinline__ int seq_of_row(const int32_t* query_start_loc, int nu
     if (query_start_loc[mid] <= t) lo = mid; else hi = mid - 1;
   }
   return lo;
+}
+
+// How many portions of max_query_len rows the rows of a step are worth, beyond the one row that every sequence has: the work
+// beside which single rows (decode) and short portions count for what they are.
+inline int64_t long_portions(int num_tokens, int num_seqs, int max_query_len) {
+  const int64_t more = std::max(max_query_len - 1, 1);
+  return std::max<int64_t>(1, std::min<int64_t>(num_seqs, (static_cast<int64_t>(num_tokens) - num_seqs + more - 1) / more));
 }
 
 __device__ __forceinline__ float sigmoid_exact(float x) { return 1.f / (1.f + expf(-x)); }

@@ -27,7 +27,8 @@ constexpr float kMinLog2 = -1.0e4f;        // a decay of 0 (or an overflowed ste
 
 // A workgroup takes as many value columns as there are, 128, 64 or 32 (16 to a wave): what is done once per workgroup, the
 // rows' silu and the chunk's weights, is then done once per head.  Where that gives few workgroups, half as wide ones: two
-// portions of 150 rows of 28 heads of 128 columns took 23.0 us in 56 workgroups, 21.1 in 112 and 27.6 in 224.
+// portions of 150 rows of 28 heads of 128 columns took 23.0 us in 56 workgroups, 21.1 in 112 and 27.6 in 224.  (lanes: the
+// workgroups that have rows, per 128 columns or fewer)
 inline int scan_waves(int64_t lanes, int v_dim) {
   if (v_dim % 128 == 0 && lanes * (v_dim / 128) > 96) return 8;
   return v_dim % 64 == 0 ? 4 : 2;
@@ -37,23 +38,50 @@ inline int scan_waves(int64_t lanes, int v_dim) {
 // the portions are cut into segments that run side by side: every segment but the last is summarised from a zero state (its
 // state and the sum of its log2 decays), the summaries are chained into the states in front of the segments, then every
 // segment runs from its state.  The summaries read the keys and values a second time, so fewer than three segments do not
-// pay.  As many segments as run at the same time, eight waves to a compute unit: one prompt of 8192 rows of 28 heads of 128
+// pay.  What counts is the work there is (long_portions), not the sequences: single rows and short portions leave the chip to
+// a long prompt beside them.  8192 rows of 28 heads of 128 columns beside 63 single rows: lightning 198 us (705 with the
+// sequences counted), plain decays 159 (565); 6000 rows beside six portions of 700: 225 (495) and 157 (392).
+// As many segments as run at the same time, eight waves to a compute unit: one prompt of 8192 rows of 28 heads of 128
 // columns took 138 us (lightning, the keys in one part) and 120 (plain decays) in 256 workgroups of eight waves, 152 and 136 in 512, 175 and 156
 // in 1024; of 64 columns 131 us in 512 workgroups of four, 189 in 256, 147 in 1024.  At least 192 rows each: three portions
 // of 700 rows of 16 heads took 39 us in three segments, 49 in one.
-struct ScanSegments { int rows, count; };
-inline ScanSegments scan_segments(int num_seqs, int num_heads, int v_dim, int max_query_len) {
-  const int64_t lanes = static_cast<int64_t>(num_seqs) * num_heads;
+//
+// The segments of the portions of more than `rows` rows are numbered one behind the other (segment_at); there are no more than
+// one per `rows` rows of the step and one per such portion.  What has no rows comes behind what has: a workgroup that ends at
+// once in front of others leaves its compute unit idle while those share one (16 heads: 90 -> 145 us).
+struct ScanSegments {
+  int rows = 0x7fffffff, count = 0;        // rows of a segment; bound on the segments' numbers
+  int64_t lanes = 0;                       // (segment, head) pairs that run side by side
+};
+// Segments of a step of `portions` long ones: how many of a head's fit on the chip beside the others.
+inline int64_t scan_segments_wanted(int64_t portions, int num_heads, int v_dim, int max_query_len) {
   const int64_t wide = v_dim % 128 == 0 ? 128 : v_dim % 64 == 0 ? 64 : 32, slots = 256 * (128 / wide);
-  const int64_t want = std::min<int64_t>(slots / std::max<int64_t>(lanes * v_dim / wide, 1), max_query_len / 192);
-  if (want < 3) return ScanSegments{0, 1};
-  const int rows = static_cast<int>((max_query_len + want - 1) / want + kScanRows - 1) / kScanRows * kScanRows;
-  return ScanSegments{rows, (max_query_len + rows - 1) / rows};
+  return std::min<int64_t>(slots / (portions * num_heads * std::max<int64_t>(v_dim / wide, 1)), max_query_len / 192);
 }
+inline ScanSegments scan_segments(int num_tokens, int num_seqs, int num_heads, int v_dim, int max_query_len) {
+  const int64_t portions = long_portions(num_tokens, num_seqs, max_query_len);
+  const int64_t want = scan_segments_wanted(portions, num_heads, v_dim, max_query_len);
+  ScanSegments sg;
+  sg.lanes = portions * num_heads;
+  if (want < 3) return sg;
+  const int rows = static_cast<int>((max_query_len + want - 1) / want + kScanRows - 1) / kScanRows * kScanRows;
+  const int64_t cuts = (std::min<int64_t>(num_tokens, static_cast<int64_t>(num_seqs) * max_query_len) - 1) / rows;
+  const int64_t count = cuts + std::min<int64_t>(num_seqs, cuts);
+  if (num_seqs + count > 65535) return sg;
+  sg.rows = rows, sg.count = static_cast<int>(count), sg.lanes *= (max_query_len + rows - 1) / rows;
+  return sg;
+}
+// The workspace: per segment and head its summary, then the state in front of it; the segments' sums of log2 decays.
+inline size_t scan_segment_bytes(int64_t count, int num_heads, int head_dim, int v_dim) {
+  return static_cast<size_t>(count) * num_heads * (static_cast<size_t>(head_dim) * v_dim + 1) * sizeof(float);
+}
+// Enough for any number of tokens, and for fewer sequences and shorter portions too.  With p long portions of m rows at most
+// in segments of at least m / w rows there are no more than (p m + num_seqs) w / m cuts: p w is at most what one portion would
+// be cut into, w / m at most 1 / 192.
 inline size_t scan_workspace_bytes(int num_seqs, int num_heads, int head_dim, int v_dim, int max_query_len) {
-  if (num_seqs <= 0 || num_heads <= 0 || head_dim <= 0 || v_dim <= 0) return 0;
-  const ScanSegments sg = scan_segments(num_seqs, num_heads, v_dim, max_query_len);
-  return sg.count > 1 ? static_cast<size_t>(sg.count) * num_seqs * num_heads * (static_cast<size_t>(head_dim) * v_dim + 1) * sizeof(float) : 0;
+  if (num_seqs <= 0 || num_heads <= 0 || head_dim <= 0 || v_dim <= 0 || scan_segments_wanted(1, num_heads, v_dim, max_query_len) < 3) return 0;
+  const int64_t cuts = scan_segments_wanted(1, num_heads, v_dim, 0x7fffffff) + num_seqs / 192 + 1;
+  return scan_segment_bytes(cuts + std::min<int64_t>(num_seqs, cuts), num_heads, head_dim, v_dim);
 }
 
 // a chunk's rows at byte offsets below 2^31
@@ -74,10 +102,10 @@ __device__ __forceinline__ void split_pair(float x, float y, uint32_t& hi, uint3
 }
 __device__ __forceinline__ bf16x8 frag_of(bf16x4 a, bf16x4 b) { return bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}; }
 
-// Rows behind a wave-uniform address, at byte offsets below 2^31: what a lane has no row for is read as zeros and not
-// written, without a branch (around branches the compiler waits for every load AND store in flight).
 template <int X> struct Const { static constexpr int value = X; };
 
+// Rows behind a wave-uniform address, at byte offsets below 2^31: what a lane has no row for is read as zeros and not
+// written, without a branch (around branches the compiler waits for every load AND store in flight).
 struct RowBuffer {
   __amdgpu_buffer_rsrc_t r;
   __device__ __forceinline__ explicit RowBuffer(const void* base) : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000)) {}
@@ -92,7 +120,37 @@ struct RowBuffer {
   }
 };
 
-// grid = (heads, sequences x segments, value columns in slices of 16 NW); NW waves.
+// Inclusive sums over a wave's lanes: within 16 lanes, then the rows of 16 lanes before.
+template <typename T>
+__device__ __forceinline__ T lane_sums(T x) {
+  auto add = [&](auto ctrl, auto rows_mask) {
+    x += __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, decltype(rows_mask)::value, 0xf, false));
+  };
+  add(Const<0x111>{}, Const<0xf>{}), add(Const<0x112>{}, Const<0xf>{}), add(Const<0x114>{}, Const<0xf>{}), add(Const<0x118>{}, Const<0xf>{});
+  add(Const<0x142>{}, Const<0xa>{}), add(Const<0x143>{}, Const<0xc>{});
+  return x;
+}
+
+// Segment `number` of the step (wave-uniform): its sequence (-1: there is no such segment), that one's rows, and which of its
+// segments.  A wave takes 64 sequences at a time.
+struct SegmentAt { int seq, row0, rows, index; };
+__device__ __forceinline__ SegmentAt segment_at(const ChunkScanArgs& a, int seg_rows, int number) {
+  const int lane = threadIdx.x & 63;
+  for (int s0 = 0; s0 < a.num_seqs; s0 += 64) {
+    const int s = min(s0 + lane, a.num_seqs - 1), row0 = a.query_start_loc[s], rows = s0 + lane < a.num_seqs ? a.query_start_loc[s + 1] - row0 : 0;
+    const int mine = rows > seg_rows ? (rows - 1) / seg_rows + 1 : 0, upto = lane_sums(mine);
+    const uint64_t past = __ballot(number < upto);
+    if (past != 0) {
+      const int at = __builtin_ctzll(past);
+      return SegmentAt{s0 + at, __builtin_amdgcn_readlane(row0, at), __builtin_amdgcn_readlane(rows, at), number - __builtin_amdgcn_readlane(upto - mine, at)};
+    }
+    number -= __builtin_amdgcn_readlane(upto, 63);
+  }
+  return SegmentAt{-1, 0, 0, 0};
+}
+
+// grid = (heads, value columns in slices of 16 NW, segments + sequences (Summarise: segments)); NW waves.  A workgroup takes a
+// segment of a portion that has several, or a portion that has one.
 //
 // Every wave owns 16 value columns of the state, fp32 in registers as the matrix instructions leave it (a lane holds runs of
 // four d of one column): that is also the layout in which the next chunk's product with the queries wants it, so the state
@@ -108,7 +166,7 @@ struct RowBuffer {
 // decays per row 316 -> 131; before, 4 waves to 32 value columns, each such workgroup with its own staging, weights and an
 // image of the state in LDS.
 template <int D, int NW, bool Silu, bool Summarise>
-__global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(ChunkScanArgs a, int seg_rows, int nseg) {
+__global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(ChunkScanArgs a, int seg_rows, int segments) {
   constexpr int NT = 64 * NW, KC = D / 8, VC = 2 * NW, KP = 2 * D, VP = 32 * NW, SD = D / 32, DB = D / 16;
   constexpr int KPT = (kScanRows * KC + NT - 1) / NT, VPT = 2;
   typedef ChunkOrder<KC> KOrder;
@@ -117,13 +175,19 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
   __shared__ __attribute__((aligned(16))) char s_q[Summarise ? 16 : kScanRows * KP], s_klo[Silu ? kScanRows * KP : 16];
   __shared__ __attribute__((aligned(16))) u32x4 s_p[Summarise ? 1 : 6][2][64];
   __shared__ __attribute__((aligned(16))) float s_cum[kScanRows], s_b[kScanRows], s_w[kScanRows];
-  const int h = blockIdx.x, s = blockIdx.y / nseg, seg = blockIdx.y % nseg, vs = blockIdx.z;
-  const int r0 = a.query_start_loc[s], rows_all = a.query_start_loc[s + 1] - r0;
-  if (rows_all < kScanMinRows) return;
-  const bool whole = nseg == 1;
-  const int r_lo = whole ? 0 : seg * seg_rows;
-  if (r_lo >= rows_all) return;
-  const int rows = whole ? rows_all : min(rows_all, r_lo + seg_rows);        // (end of this workgroup's rows)
+  const int h = blockIdx.x, vs = blockIdx.y, number = blockIdx.z;
+  const bool whole = number >= segments;
+  SegmentAt seg;
+  if (!whole) {
+    seg = segment_at(a, seg_rows, number);
+    if (seg.seq < 0) return;
+  } else {
+    seg.seq = number - segments, seg.index = 0;
+    seg.row0 = a.query_start_loc[seg.seq], seg.rows = a.query_start_loc[seg.seq + 1] - seg.row0;
+  }
+  const int s = seg.seq, r0 = seg.row0, rows_all = seg.rows;
+  if (rows_all < kScanMinRows || (whole && rows_all > seg_rows)) return;
+  const int r_lo = whole ? 0 : seg.index * seg_rows, rows = r_lo + min(rows_all - r_lo, seg_rows);        // (end of this workgroup's rows)
   const bool last = rows == rows_all;
   if (Summarise && last) return;                       // nothing comes behind the last segment
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
@@ -135,8 +199,8 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
   const float skip = a.skip ? a.skip[h] : 0.f;
   // a segment's place in the workspace: its summary (Summarise writes it), then the state in front of it; the segments' sums
   // of log2 decays lie behind all the states
-  const int64_t seg_at = (static_cast<int64_t>(s) * nseg + seg) * H + h;
-  float* wsp = whole ? nullptr : a.workspace + seg_at * D * Dv + col0;
+  const int64_t place = static_cast<int64_t>(number) * H + h;
+  float* wsp = whole ? nullptr : a.workspace + place * D * Dv + col0;
   const float* init = Summarise ? nullptr : whole ? (st != nullptr && a.context_lens[s] > 0 ? st : nullptr) : wsp;
   float seg_total = 0.f;
 
@@ -207,13 +271,7 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
       // running sums of the chunk's log2 decays (rows past the portion add 0)
       float cum;
       if (a.log2_decay) {
-        cum = fmaxf(rl, kMinLog2);                     // (rows past the portion: 0)
-        // inclusive sums: within 16 lanes, then the rows of 16 lanes before
-        auto add = [&](auto ctrl, auto rows_mask) {
-          cum += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, cum), decltype(ctrl)::value, decltype(rows_mask)::value, 0xf, false));
-        };
-        add(Const<0x111>{}, Const<0xf>{}), add(Const<0x112>{}, Const<0xf>{}), add(Const<0x114>{}, Const<0xf>{}), add(Const<0x118>{}, Const<0xf>{});
-        add(Const<0x142>{}, Const<0xa>{}), add(Const<0x143>{}, Const<0xc>{});
+        cum = lane_sums(fmaxf(rl, kMinLog2));          // (rows past the portion: 0)
       } else {
         cum = static_cast<float>(min(lane + 1, nrow)) * l2_const;
       }
@@ -385,55 +443,60 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) to[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + n] = S[db][r];
   }
-  if (Summarise && vs == 0 && tid == 0) a.workspace[static_cast<int64_t>(a.num_seqs) * nseg * H * D * Dv + seg_at] = seg_total;
+  if (Summarise && vs == 0 && tid == 0) a.workspace[static_cast<int64_t>(segments) * H * D * Dv + place] = seg_total;
 }
 
 // The segments' summaries (each segment's state had it started from zero) become the states in front of the segments:
-// run = carried state; per segment: place <- run, run <- 2^(segment's sum of log2 decays) run + summary.  An element per thread.
-// grid = (heads, sequences, parts of 1024 elements)
-__global__ __launch_bounds__(256) void chunk_scan_chain_kernel(ChunkScanArgs a, int head_dim, int seg_rows, int nseg) {
-  const int h = blockIdx.x, s = blockIdx.y, H = a.num_heads;
-  const int rows = a.query_start_loc[s + 1] - a.query_start_loc[s];
-  const int per_head = head_dim * a.v_dim, idx = 4 * (256 * static_cast<int>(blockIdx.z) + static_cast<int>(threadIdx.x));
-  if (rows < kScanMinRows || idx >= per_head) return;
-  const int slot = a.slot_idx[s];
-  f32x4s run = f32x4s{0.f, 0.f, 0.f, 0.f};
-  if (slot >= 0 && a.context_lens[s] > 0) run = *reinterpret_cast<const f32x4s*>(a.state + (static_cast<int64_t>(slot) * H + h) * per_head + idx);
-  const int segs = (rows + seg_rows - 1) / seg_rows;
-  const int64_t step = static_cast<int64_t>(H) * per_head;
-  float* p = a.workspace + (static_cast<int64_t>(s) * nseg * H + h) * per_head + idx;
-  const float* totals = a.workspace + a.num_seqs * nseg * step + static_cast<int64_t>(s) * nseg * H + h;
-  for (int seg0 = 0; seg0 < segs; seg0 += 8) {           // eight summaries in flight together (the last ones may lie past the end: read again)
-    f32x4s summary[8];
-    float decay[8];
+// run = carried state; per segment: place <- run, run <- 2^(segment's sum of log2 decays) run + summary.  Four elements per
+// thread.  grid = (heads, segments, parts per segment): a portion's workgroups deal the parts of 1024 elements among them.
+__global__ __launch_bounds__(256) void chunk_scan_chain_kernel(ChunkScanArgs a, int head_dim, int seg_rows, int segments) {
+  const int h = blockIdx.x, H = a.num_heads, per_head = head_dim * a.v_dim;
+  const SegmentAt seg = segment_at(a, seg_rows, blockIdx.y);
+  const int s = seg.seq;
+  if (s < 0) return;
+  const int slot = a.slot_idx[s], segs = (seg.rows - 1) / seg_rows + 1;
+  const int64_t step = static_cast<int64_t>(H) * per_head, first = static_cast<int64_t>(blockIdx.y - seg.index) * H + h;
+  const float* totals = a.workspace + segments * step + first;
+  const bool carry = slot >= 0 && a.context_lens[s] > 0;
+  for (int part = seg.index + segs * blockIdx.z; 1024 * part < per_head; part += segs * gridDim.z) {
+    const int idx = 1024 * part + 4 * threadIdx.x;
+    if (idx >= per_head) return;
+    f32x4s run = f32x4s{0.f, 0.f, 0.f, 0.f};
+    if (carry) run = *reinterpret_cast<const f32x4s*>(a.state + (static_cast<int64_t>(slot) * H + h) * per_head + idx);
+    float* p = a.workspace + first * per_head + idx;
+    for (int seg0 = 0; seg0 < segs; seg0 += 8) {         // eight summaries in flight together (the last ones may lie past the end: read again)
+      f32x4s summary[8];
+      float decay[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int at = min(seg0 + u, segs - 1);
-      summary[u] = *reinterpret_cast<const f32x4s*>(p + at * step);
-      decay[u] = totals[at * H];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (seg0 + u < segs) {
-        *reinterpret_cast<f32x4s*>(p + (seg0 + u) * step) = run;
-        run = __builtin_amdgcn_exp2f(decay[u]) * run + summary[u];       // (behind the last segment: not used)
+      for (int u = 0; u < 8; ++u) {
+        const int at = min(seg0 + u, segs - 1);
+        summary[u] = *reinterpret_cast<const f32x4s*>(p + at * step);
+        decay[u] = totals[at * H];
       }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (seg0 + u < segs) {
+          *reinterpret_cast<f32x4s*>(p + (seg0 + u) * step) = run;
+          run = __builtin_amdgcn_exp2f(decay[u]) * run + summary[u];     // (behind the last segment: not used)
+        }
+    }
   }
 }
 
 template <int D, int NW, bool Silu>
 void launch_chunk_scan_as(const ChunkScanArgs& a, ScanSegments sg, hipStream_t st) {
-  const dim3 grid(a.num_heads, a.num_seqs * sg.count, a.v_dim / (16 * NW)), block(64 * NW);
-  if (sg.count > 1) {
-    hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, true>), grid, block, 0, st, a, sg.rows, sg.count);
-    hipLaunchKernelGGL(chunk_scan_chain_kernel, dim3(a.num_heads, a.num_seqs, (D * a.v_dim + 1023) / 1024), dim3(256), 0, st, a, D, sg.rows, sg.count);
+  const dim3 block(64 * NW);
+  const unsigned slices = a.v_dim / (16 * NW);
+  if (sg.count > 0) {
+    hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, true>), dim3(a.num_heads, slices, sg.count), block, 0, st, a, sg.rows, sg.count);
+    hipLaunchKernelGGL(chunk_scan_chain_kernel, dim3(a.num_heads, sg.count, (D * a.v_dim + 3071) / 3072), dim3(256), 0, st, a, D, sg.rows, sg.count);
   }
-  hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, false>), grid, block, 0, st, a, sg.rows, sg.count);
+  hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, false>), dim3(a.num_heads, slices, sg.count + a.num_seqs), block, 0, st, a, sg.rows, sg.count);
 }
 
 template <bool Silu>
 void launch_chunk_scan(const ChunkScanArgs& a, int head_dim, ScanSegments sg, hipStream_t st) {
-  const int nw = scan_waves(static_cast<int64_t>(a.num_seqs) * sg.count * a.num_heads, a.v_dim);
+  const int nw = scan_waves(sg.lanes, a.v_dim);
   auto waves = [&](auto d) {
     constexpr int D = decltype(d)::value;
     if (nw == 8) launch_chunk_scan_as<D, 8, Silu>(a, sg, st);

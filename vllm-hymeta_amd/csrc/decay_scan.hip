@@ -185,10 +185,9 @@ extern "C" int hymeta_decay_scan(const hymeta_decay_scan_args* args, hymeta_stre
   hipStream_t st = begin_launches(stream);
   int max_rows = 0x7fffffff;
   if (chunk_shape(a) && a.max_query_len >= kScanMinRows) {
-    const size_t need = hymeta_decay_scan_workspace_bytes(a.num_seqs, a.num_heads, a.head_dim, a.v_dim, a.max_query_len);
+    const ScanSegments sg = scan_segments(a.num_tokens, a.num_seqs, a.num_heads, a.v_dim, a.max_query_len);
+    const size_t need = scan_segment_bytes(sg.count, a.num_heads, a.head_dim, a.v_dim);
     if (need > 0 && (!a.workspace || a.workspace_bytes < need)) return HYMETA_ERR_WORKSPACE;
-    const ScanSegments sg = scan_segments(a.num_seqs, a.num_heads, a.v_dim, a.max_query_len);
-    if (static_cast<int64_t>(a.num_seqs) * sg.count > 65535) return HYMETA_ERR_UNSUPPORTED;
     const ChunkScanArgs c{static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.k), static_cast<const uint16_t*>(a.v), a.q_stride_t, a.k_stride_t,
                           a.v_stride_t, a.log2_decay ? nullptr : a.decay, a.log2_decay, a.v_scale, a.skip, a.state, a.out, static_cast<float*>(a.workspace),
                           a.query_start_loc, a.context_lens, a.slot_idx, a.num_seqs, a.num_heads, a.num_qk_heads, a.v_dim};

@@ -249,10 +249,9 @@ extern "C" int hymeta_lightning_attention(const hymeta_lightning_attention_args*
   hipStream_t st = begin_launches(stream);
   int max_rows = 0x7fffffff;
   if (chunk_shape(a) && a.max_query_len >= kScanMinRows) {
-    const size_t need = hymeta_lightning_attention_workspace_bytes(a.num_seqs, a.num_heads, a.head_dim, a.v_dim, a.max_query_len);
+    const ScanSegments sg = scan_segments(a.num_tokens, a.num_seqs, a.num_heads, a.v_dim, a.max_query_len);
+    const size_t need = scan_segment_bytes(sg.count, a.num_heads, a.head_dim, a.v_dim);
     if (need > 0 && (!a.workspace || a.workspace_bytes < need)) return HYMETA_ERR_WORKSPACE;
-    const ScanSegments sg = scan_segments(a.num_seqs, a.num_heads, a.v_dim, a.max_query_len);
-    if (static_cast<int64_t>(a.num_seqs) * sg.count > 65535) return HYMETA_ERR_UNSUPPORTED;
     const uint16_t* qkv = static_cast<const uint16_t*>(a.qkv);
     const int64_t keys = static_cast<int64_t>(a.num_heads) * a.head_dim;
     const ChunkScanArgs c{qkv, qkv + keys, qkv + 2 * keys, a.qkv_stride_t, a.qkv_stride_t, a.qkv_stride_t, a.decay, nullptr, nullptr, nullptr,
