@@ -39,8 +39,8 @@ inline int scan_waves(int64_t lanes, int v_dim) {
 // state and the sum of its log2 decays), the summaries are chained into the states in front of the segments, then every
 // segment runs from its state.  The summaries read the keys and values a second time, so fewer than three segments do not
 // pay.  What counts is the work there is (long_portions), not the sequences: single rows and short portions leave the chip to
-// a long prompt beside them.  8192 rows of 28 heads of 128 columns beside 63 single rows: lightning 198 us (705 with the
-// sequences counted), plain decays 159 (565); 6000 rows beside six portions of 700: 225 (495) and 157 (392).
+// a long prompt beside them.  8192 rows of 28 heads of 128 columns beside 63 single rows: lightning 194 us (705 with the
+// sequences counted), plain decays 159 (565); 6000 rows beside six portions of 700: 218 (495) and 157 (392).
 // As many segments as run at the same time, eight waves to a compute unit: one prompt of 8192 rows of 28 heads of 128
 // columns took 138 us (lightning, the keys in one part) and 120 (plain decays) in 256 workgroups of eight waves, 152 and 136 in 512, 175 and 156
 // in 1024; of 64 columns 131 us in 512 workgroups of four, 189 in 256, 147 in 1024.  At least 192 rows each: three portions
@@ -162,7 +162,7 @@ __device__ __forceinline__ SegmentAt segment_at(const ChunkScanArgs& a, int seg_
 // values, rounded to bf16 as in the outputs, carry the decays).
 // Bound by vector arithmetic between the barriers of a chunk: 2 x 16 cycles of exponential and reciprocal per silu'd value,
 // splits, scales; the matrix pipes are busy about a quarter of the time, memory far less.  One prompt of 8192 rows, 28 heads
-// of 128 x 128: lightning 351 -> 152 us (141 with the keys in one part), plain decays 283 -> 121; with 64 value columns and
+// of 128 x 128: lightning 351 -> 151 us (141 with the keys in one part), plain decays 283 -> 121; with 64 value columns and
 // decays per row 316 -> 131; before, 4 waves to 32 value columns, each such workgroup with its own staging, weights and an
 // image of the state in LDS.
 template <int D, int NW, bool Silu, bool Summarise>
@@ -418,15 +418,28 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
       }
     }
     const float chunk_decay = __builtin_amdgcn_exp2f(total);
+    // fragments a block ahead of their products, where there are registers for them (a read in front of every product: lightning
+    // over 512 rows of 28 heads 52 us, so 47)
+    constexpr int kAhead = Summarise ? 0 : 1;
+    bf16x8 kf[1 + kAhead][Silu ? 2 : 1][2];
+    auto read_keys = [&](int db) __attribute__((always_inline)) {
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        kf[db & kAhead][0][kk] = key_frag(s_k, db, kk);
+        if constexpr (Silu) kf[db & kAhead][1][kk] = key_frag(s_klo, db, kk);
+      }
+    };
+    if (kAhead) read_keys(0);
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
+      if (db + kAhead < DB) read_keys(db + kAhead);
+      if (kAhead) __builtin_amdgcn_sched_barrier(0);
       f32x4s acc = S[db] * chunk_decay;
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
-        const bf16x8 kf = key_frag(s_k, db, kk);
-        acc = scan_mfma(kf, __builtin_bit_cast(bf16x8, wv[kk][0]), acc);
-        acc = scan_mfma(kf, __builtin_bit_cast(bf16x8, wv[kk][1]), acc);
-        if constexpr (Silu) acc = scan_mfma(key_frag(s_klo, db, kk), __builtin_bit_cast(bf16x8, wv[kk][0]), acc);
+        acc = scan_mfma(kf[db & kAhead][0][kk], __builtin_bit_cast(bf16x8, wv[kk][0]), acc);
+        acc = scan_mfma(kf[db & kAhead][0][kk], __builtin_bit_cast(bf16x8, wv[kk][1]), acc);
+        if constexpr (Silu) acc = scan_mfma(kf[db & kAhead][1][kk], __builtin_bit_cast(bf16x8, wv[kk][0]), acc);
       }
       S[db] = acc;
     }
