@@ -1,5 +1,5 @@
-"""The delta rule over many (sequence, head) pairs runs in slices of 128 value columns: against the same sequences one at a
-time, which run in narrow slices."""
+"""The delta rule over many (portion, head) pairs runs in slices of 128 value columns: against the same sequences one at a
+time, which run in narrow slices.  A long portion among single rows runs in narrow slices too."""
 import pytest
 import torch
 
@@ -9,13 +9,17 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-@pytest.mark.parametrize("D,Dv,H,Hk", [(32, 128, 16, 4), (64, 256, 8, 8), (96, 128, 16, 16), (128, 128, 16, 8)])
-def test_wide_slices_equal_narrow_ones(D, Dv, H, Hk):
+EDGES = [8, 63, 64, 65, 130, 7, 128, 129, 20, 1, 130, 97, 126, 127, 128]        # worth ten portions of 130: 160 wide slices
+
+
+@pytest.mark.parametrize("D,Dv,H,Hk,lens", [
+    (32, 128, 16, 4, EDGES), (64, 256, 8, 8, EDGES), (96, 128, 16, 16, EDGES), (128, 128, 16, 8, EDGES),
+    (128, 128, 16, 8, [1] * 20 + [300] + [1] * 12 + [9, 130]), (96, 128, 12, 12, [1] * 20 + [300] + [1] * 12 + [9, 130])])
+def test_wide_slices_equal_narrow_ones(D, Dv, H, Hk, lens):
     """Both multiply the same operands (fp32 as two bf16 parts, 2^-17 of the operand) and add in another order: 1e-5 of the
-    norm covers what that rounding grows to over three chunks.  Rows at a chunk's edges, several chunks, a portion that goes
+    norm covers what that rounding grows to over a few chunks.  Rows at a chunk's edges, several chunks, a portion that goes
     token by token, carried states and one sequence without a slot."""
     from vllm_hymeta import hip_ops
-    lens = [8, 63, 64, 65, 130, 7, 128, 129, 20, 1, 192]
     T, S = sum(lens), len(lens)
     g = gen(D + Dv)
     q, k, v = (torch.randn(T, n, d, generator=g).bfloat16().to(DEV) for n, d in ((Hk, D), (Hk, D), (H, Dv)))

@@ -201,6 +201,8 @@ constexpr int kFewGroups = 128;
 // Workgroups of slices of 128 columns above which the second launch takes those: slices of 32 are then more than the 512
 // workgroups that run at the same time.  With 28 heads of 128 x 128 (16 for the last two): 5 portions of 1801 rows 310 us in
 // narrow slices, 281 in wide ones (140 workgroups); 16 of 500 250 and 191; 40 of 300 414 and 276; 8 of 700 (128) 102 and 108.
+// Both count the portions that the step's rows are worth (long_portions): one of 8192 rows beside 63 single rows took 960 us in
+// the wide slices that 64 sequences asked for, 420 in slices of 16 (single rows and the solving launch included).
 constexpr int kManyWideGroups = 128;
 constexpr int kChunkMinRows = 8;            // shorter portions go token by token
 constexpr int kMat = kChunk * kChunk;
@@ -826,15 +828,16 @@ void launch_rows(const hymeta_delta_rule_args& a, hipStream_t st, int min_rows, 
 template <int D>
 void launch_chunks(const hymeta_delta_rule_args& a, hipStream_t st, int64_t chunks) {
   hipLaunchKernelGGL(delta_chunk_solve_kernel<D>, dim3(static_cast<unsigned>(chunks), a.num_heads), dim3(256), 0, st, a, chunks);
-  // slices of 32 columns reread a chunk's matrices half as often; slices of 16 double the workgroups where they are few
+  // slices of 32 columns reread a chunk's matrices half as often; slices of 16 double the workgroups where they are few.  Few
+  // and many of those that have work for the time the longest takes: single rows and short portions end at once or soon
+  const int64_t lanes = a.num_heads * long_portions(a.num_tokens, a.num_seqs, a.max_query_len);
   if constexpr (D % 64 == 0) {
-    if (static_cast<int64_t>(a.num_heads) * a.num_seqs * (a.v_dim / 32) <= kFewGroups) {
+    if (lanes * (a.v_dim / 32) <= kFewGroups) {
       hipLaunchKernelGGL((delta_chunk_scan_kernel<D, 1>), dim3(a.num_heads, a.num_seqs, a.v_dim / 16), dim3(256), 0, st, a, chunks);
       return;
     }
   }
-  const int64_t wide = static_cast<int64_t>(a.num_heads) * a.num_seqs * (a.v_dim / 128);
-  if (a.v_dim % 128 == 0 && wide > kManyWideGroups && a.v_stride_t < (1 << 23) && static_cast<int64_t>(a.num_heads) * a.v_dim < (1 << 22)) {
+  if (a.v_dim % 128 == 0 && lanes * (a.v_dim / 128) > kManyWideGroups && a.v_stride_t < (1 << 23) && static_cast<int64_t>(a.num_heads) * a.v_dim < (1 << 22)) {
     hipLaunchKernelGGL((delta_chunk_wide_kernel<D>), dim3(a.num_heads, a.num_seqs, a.v_dim / 128), dim3(512), 0, st, a, chunks);
     return;
   }
