@@ -56,6 +56,12 @@ def reference(q, k, v, scale, ctx, o, sink, a, gate):
     ("latent", 96, 64, 7, 1, 8, [40, 64], [5, 64], dict(sink=True)),
     ("shared", 128, 64, 4, 2, 64, [50, 2], [14, 800], dict(window=100, keep=4)),
     ("shared", 64, 128, 4, 4, 64, [65], [64], {}),
+    # keys cut into slices: a window with kept first keys and both gates, beside single rows, some blocks cut and some whole
+    ("rows", 128, 128, 8, 2, 64, [40, 1, 1, 3, 1], [3000, 900, 64, 10, 2000], dict(window=2100, keep=70, gate=True, elem=True)),
+    ("rows", 64, 64, 4, 2, 16, [1, 9, 1], [70, 2500, 1300], dict(window=1500, keep=9, elem=True, sink=True)),
+    ("rows", 128, 64, 6, 2, 64, [5, 1, 50], [2900, 100, 0], dict(chunk=1000, gate=True, elem=True)),
+    ("latent", 192, 128, 40, 1, 64, [7, 1, 4], [2000, 1500, 0], dict(elem=True, gate=True)),      # two launches of heads for single rows
+    ("scaled", 64, 64, 4, 2, 64, [3, 1, 17], [2500, 3000, 600], dict(sink=True, bias="linear", window=2000, keep=5, elem=True)),
     ("scaled", 128, 128, 28, 4, 64, [20, 2], [0, 1200], dict(sink=True, bias="linear")),
     ("scaled", 96, 96, 4, 2, 16, [33, 70], [100, 0], dict(bias="linear", window=50)),
     ("scaled", 64, 64, 4, 1, 64, [64], [64], dict(sink=True)),
@@ -65,7 +71,7 @@ def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
     from vllm_hymeta import hip_ops
     dev, g = "cuda", torch.Generator().manual_seed(D + H)
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
-    o = dict(dict(sink=False, window=0, keep=0, chunk=0, softcap=0.0, bias=None, gate=False, near=NEAR), **opts)
+    o = dict(dict(sink=False, window=0, keep=0, chunk=0, softcap=0.0, bias=None, gate=False, elem=False, near=NEAR), **opts)
     key_heads = 1 if layout in ("latent", "shared") else G
     total = [n + c for n, c in zip(lens, ctxs)]
     keys = [torch.randn(t, key_heads, D, generator=g).bfloat16() for t in total]
@@ -74,6 +80,7 @@ def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
     sink = torch.randn(H, generator=g) if o["sink"] else None
     a = 0.1 + torch.rand(H, generator=g)
     gates = [torch.randn(n, H, generator=g).bfloat16() if o["gate"] else None for n in lens]
+    elems = [torch.randn(n, H * Dv, generator=g).bfloat16() if o["elem"] else None for n in lens]
     need = [(t + page - 1) // page for t in total]
     order, at = torch.randperm(sum(need) + 1, generator=g).tolist(), 0
     tail = {"rows": (G, D + Dv), "latent": (1, D), "shared": (1, D + G * Dv), "scaled": (1, hip_ops.scaled_key_row(G, D, torch.bfloat16))}[layout]
@@ -98,7 +105,7 @@ def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
         keep_first=o["keep"], chunk=o["chunk"], softcap=o["softcap"], value_in_key=layout == "latent", shared_key=layout == "shared",
         scaled_key=layout == "scaled", bias_a=a.to(dev) if o["bias"] == "log" else None, slopes=(SLOPE * a).to(dev) if o["bias"] == "linear" else None,
         bias_b=torch.full((H,), o["near"], device=dev) if o["bias"] == "log" else None,
-        head_gate=torch.cat(gates).to(dev) if o["gate"] else None).double().cpu()
+        head_gate=torch.cat(gates).to(dev) if o["gate"] else None, elem_gate=torch.cat(elems).to(dev) if o["elem"] else None).double().cpu()
     at = 0
     for s, n in enumerate(lens):
         k, v = keys[s].double(), values[s].double()
@@ -107,6 +114,8 @@ def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
         spread = lambda x: x.permute(1, 0, 2).repeat_interleave(H // x.shape[1], 0)  # noqa: E731
         ref = reference(q[s].double(), spread(k), spread(v), D ** -0.5, ctxs[s], o, None if sink is None else sink.double(), a.double(),
                         None if gates[s] is None else gates[s].double())
+        if elems[s] is not None:
+            ref = ref * torch.sigmoid(elems[s].double()).reshape(ref.shape)
         got = out[at:at + n]
         assert torch.isfinite(got).all()
         assert (got - ref).norm() <= BOUND * ref.norm(), (s, float((got - ref).norm() / ref.norm()))
@@ -125,3 +134,19 @@ def test_rows_behind_the_last_portion_stay_untouched(D, Dv, monkeypatch):
     out = hip_ops.sink_attention(q, cache, torch.arange(32, dtype=torch.int32, device=dev)[None], i32([0, 5]), i32([2048]), 1, D, Dv, D ** -0.5, 5, 2048,
                                  value_in_key=inside)
     assert (out[5:] == 7).all() and torch.isfinite(out).all() and not (out[:5] == 7).all()
+
+
+@pytest.mark.parametrize("D,Dv", [(128, 128), (576, 512)])
+@pytest.mark.parametrize("lens", [[1], [0, 2], [1, 0, 1]])
+def test_bounds_larger_than_the_step(D, Dv, lens):
+    """The step's lengths are bounds: fewer rows than the longest portion may have, and sequences without rows."""
+    from vllm_hymeta import hip_ops
+    dev, T = "cuda", sum(lens)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
+    inside = D != Dv
+    q, cache = torch.randn(T, 4, D, device=dev).bfloat16(), torch.randn(8, 64, 1, D if inside else D + Dv, device=dev).bfloat16()
+    table = torch.arange(8, dtype=torch.int32, device=dev)[None].repeat(len(lens), 1)
+    starts, ends = i32([0] + list(accumulate(lens))), i32([300 + n for n in lens])
+    run = lambda most_rows, most_keys: hip_ops.sink_attention(q, cache, table, starts, ends, 1, D, Dv, D ** -0.5, most_rows, most_keys, value_in_key=inside)  # noqa: E731
+    a, b = run(max(lens), 300 + max(lens)).double(), run(500, 512).double()
+    assert torch.isfinite(a).all() and (a - b).norm() <= BOUND * a.norm()

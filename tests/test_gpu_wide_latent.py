@@ -44,6 +44,9 @@ def reference(q, rows, C, scale, sink, window, keep, chunk, softcap, bias, gate,
     (512, 1, 128, [129, 1], [0, 511], dict(softcap=5.0, bias=True)),
     (512, 16, 64, [1, 3, 20, 1], [-1, -1, -10, 300], {}),                    # rows in front of their sequence
     (256, 4, 16, [1, 70, 2], [-1, -30, -2], dict(chunk=20, sink=True)),
+    # keys cut into slices beside single rows: a window, kept first keys, a gate; some blocks whole
+    (512, 16, 64, [9, 1, 3, 1], [2500, 700, 5, 64], dict(window=1600, keep=40, gate=True, sink=True)),
+    (256, 40, 16, [1, 5, 1], [900, 1400, 31], dict(chunk=700, gate=True)),
     (256, 33, 64, [1] * 5, [0, 15, 16, 1000, 63], dict(sink=True, window=33)),
 ])
 def test_against_64_bits(C, H, page, lens, ctxs, opts):

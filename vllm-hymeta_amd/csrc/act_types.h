@@ -87,6 +87,38 @@ inline int64_t long_portions(int num_tokens, int num_seqs, int max_query_len) {
   return std::max<int64_t>(1, std::min<int64_t>(num_seqs, (static_cast<int64_t>(num_tokens) - num_seqs + more - 1) / more));
 }
 
+template <int X> struct Const { static constexpr int value = X; };
+
+// Inclusive sums over a wave's lanes: within 16 lanes, then the rows of 16 lanes before.
+template <typename T>
+__device__ __forceinline__ T lane_sums(T x) {
+  auto add = [&](auto ctrl, auto rows_mask) {
+    x += __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, decltype(rows_mask)::value, 0xf, false));
+  };
+  add(Const<0x111>{}, Const<0xf>{}), add(Const<0x112>{}, Const<0xf>{}), add(Const<0x114>{}, Const<0xf>{}), add(Const<0x118>{}, Const<0xf>{});
+  add(Const<0x142>{}, Const<0xa>{}), add(Const<0x143>{}, Const<0xc>{});
+  return x;
+}
+
+// Every sequence of a step falls into pieces(its rows) pieces, numbered through: the sequence of piece `number` (wave-uniform;
+// -1: there is no such piece), that one's rows, and which of its pieces it is.  A wave takes 64 sequences at a time.
+struct PieceAt { int seq, row0, rows, index; };
+template <typename F>
+__device__ __forceinline__ PieceAt piece_at(const int32_t* query_start_loc, int num_seqs, int number, const F& pieces) {
+  const int lane = threadIdx.x & 63;
+  for (int s0 = 0; s0 < num_seqs; s0 += 64) {
+    const int s = min(s0 + lane, num_seqs - 1), row0 = query_start_loc[s], rows = s0 + lane < num_seqs ? query_start_loc[s + 1] - row0 : 0;
+    const int mine = pieces(rows), upto = lane_sums(mine);
+    const uint64_t past = __ballot(number < upto);
+    if (past != 0) {
+      const int at = __builtin_ctzll(past);
+      return PieceAt{s0 + at, __builtin_amdgcn_readlane(row0, at), __builtin_amdgcn_readlane(rows, at), number - __builtin_amdgcn_readlane(upto - mine, at)};
+    }
+    number -= __builtin_amdgcn_readlane(upto, 63);
+  }
+  return PieceAt{-1, 0, 0, 0};
+}
+
 __device__ __forceinline__ float sigmoid_exact(float x) { return 1.f / (1.f + expf(-x)); }
 
 }  // namespace hymeta

@@ -102,8 +102,6 @@ __device__ __forceinline__ void split_pair(float x, float y, uint32_t& hi, uint3
 }
 __device__ __forceinline__ bf16x8 frag_of(bf16x4 a, bf16x4 b) { return bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}; }
 
-template <int X> struct Const { static constexpr int value = X; };
-
 // Rows behind a wave-uniform address, at byte offsets below 2^31: what a lane has no row for is read as zeros and not
 // written, without a branch (around branches the compiler waits for every load AND store in flight).
 struct RowBuffer {
@@ -120,33 +118,10 @@ struct RowBuffer {
   }
 };
 
-// Inclusive sums over a wave's lanes: within 16 lanes, then the rows of 16 lanes before.
-template <typename T>
-__device__ __forceinline__ T lane_sums(T x) {
-  auto add = [&](auto ctrl, auto rows_mask) {
-    x += __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, decltype(rows_mask)::value, 0xf, false));
-  };
-  add(Const<0x111>{}, Const<0xf>{}), add(Const<0x112>{}, Const<0xf>{}), add(Const<0x114>{}, Const<0xf>{}), add(Const<0x118>{}, Const<0xf>{});
-  add(Const<0x142>{}, Const<0xa>{}), add(Const<0x143>{}, Const<0xc>{});
-  return x;
-}
-
 // Segment `number` of the step (wave-uniform): its sequence (-1: there is no such segment), that one's rows, and which of its
-// segments.  A wave takes 64 sequences at a time.
-struct SegmentAt { int seq, row0, rows, index; };
-__device__ __forceinline__ SegmentAt segment_at(const ChunkScanArgs& a, int seg_rows, int number) {
-  const int lane = threadIdx.x & 63;
-  for (int s0 = 0; s0 < a.num_seqs; s0 += 64) {
-    const int s = min(s0 + lane, a.num_seqs - 1), row0 = a.query_start_loc[s], rows = s0 + lane < a.num_seqs ? a.query_start_loc[s + 1] - row0 : 0;
-    const int mine = rows > seg_rows ? (rows - 1) / seg_rows + 1 : 0, upto = lane_sums(mine);
-    const uint64_t past = __ballot(number < upto);
-    if (past != 0) {
-      const int at = __builtin_ctzll(past);
-      return SegmentAt{s0 + at, __builtin_amdgcn_readlane(row0, at), __builtin_amdgcn_readlane(rows, at), number - __builtin_amdgcn_readlane(upto - mine, at)};
-    }
-    number -= __builtin_amdgcn_readlane(upto, 63);
-  }
-  return SegmentAt{-1, 0, 0, 0};
+// segments.
+__device__ __forceinline__ PieceAt segment_at(const ChunkScanArgs& a, int seg_rows, int number) {
+  return piece_at(a.query_start_loc, a.num_seqs, number, [=](int rows) { return rows > seg_rows ? (rows - 1) / seg_rows + 1 : 0; });
 }
 
 // grid = (heads, value columns in slices of 16 NW, segments + sequences (Summarise: segments)); NW waves.  A workgroup takes a
@@ -177,7 +152,7 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
   __shared__ __attribute__((aligned(16))) float s_cum[kScanRows], s_b[kScanRows], s_w[kScanRows];
   const int h = blockIdx.x, vs = blockIdx.y, number = blockIdx.z;
   const bool whole = number >= segments;
-  SegmentAt seg;
+  PieceAt seg;
   if (!whole) {
     seg = segment_at(a, seg_rows, number);
     if (seg.seq < 0) return;
@@ -464,7 +439,7 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
 // thread.  grid = (heads, segments, parts per segment): a portion's workgroups deal the parts of 1024 elements among them.
 __global__ __launch_bounds__(256) void chunk_scan_chain_kernel(ChunkScanArgs a, int head_dim, int seg_rows, int segments) {
   const int h = blockIdx.x, H = a.num_heads, per_head = head_dim * a.v_dim;
-  const SegmentAt seg = segment_at(a, seg_rows, blockIdx.y);
+  const PieceAt seg = segment_at(a, seg_rows, blockIdx.y);
   const int s = seg.seq;
   if (s < 0) return;
   const int slot = a.slot_idx[s], segs = (seg.rows - 1) / seg_rows + 1;

@@ -12,7 +12,7 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return 
 
 constexpr float kLazyMax2 = 8.f;     // the softmax reference may trail a row's maximum by a factor of 2^8
 
-// Grid = (blocks of 128 rows x slices of the keys, key/value heads, sequences); a row is a (query, head) pair, the heads of a key/value head side by
+// Grid = the portions' blocks of 128 rows x slices of the keys at most x key/value heads; a row is a (query, head) pair, the heads of a key/value head side by
 // side: they share every key, so that a portion of a few tokens fills its blocks and a block's causal edge is one tile.
 // Sequences with one row are left to the decode form.
 //
@@ -32,6 +32,7 @@ struct RowShape {
   static constexpr int kKeyChunks = D / 8, kValueChunks = Inside ? 0 : DV / 8, kChunks = kKeyChunks + kValueChunks;
   static constexpr int kPitch = 16 * kChunks, kImage = kTileKeys * kPitch;
   static constexpr int kWaves = 4, kRows = 32 * kWaves;
+  static_assert(kRows == kPortionRows, "the merge finds a row's block");
 };
 
 // How a score follows from its product, in kernels of their own where a design's every layer asks for it: a branch per row
@@ -39,21 +40,22 @@ struct RowShape {
 enum ScoreRule { kPlain, kLogBias, kAnyRule };
 
 template <int D, int DV, int Layout, int Rule>
-__global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attention_args a, int splits) {
+__global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attention_args a, PortionSlices ps) {
   typedef RowShape<D, DV, Layout> S;
   constexpr int kSteps = D / 16, CB = DV / 32;
   __shared__ __attribute__((aligned(16))) char s_rows[2][S::kImage];
   __shared__ __attribute__((aligned(16))) float s_scale[2][S::Scaled ? kTileKeys : 4];
-  const int turn = gridDim.x - 1 - blockIdx.x;              // the longest rows first
-  const int s = blockIdx.z, g = blockIdx.y, tile = turn / splits, split = turn % splits;
-  const int row0 = a.query_start_loc[s];
-  const int q = a.query_start_loc[s + 1] - row0;
-  const int group = a.num_heads / a.num_kv_heads;
-  const int rows = q * group, r0 = tile * S::kRows;
-  if (q <= 1 || r0 >= rows) return;
+  const int group = a.num_heads / a.num_kv_heads, g = blockIdx.x % a.num_kv_heads, item = blockIdx.x / a.num_kv_heads, split = item % ps.splits;
+  const PieceAt block = portion_block(a, item / ps.splits);
+  const int s = block.seq, row0 = block.row0, q = block.rows, rows = q * group;
+  if (s < 0) return;
+  const int r0 = ((rows - 1) / S::kRows - block.index) * S::kRows;        // (the longest rows first)
   const int lane = threadIdx.x & 63, n = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ctx = a.seq_lens[s] - q, w0 = r0 + 32 * wave;
+  const BlockKeys keys = block_keys<kTileKeys>(a, ctx + r0 / group, ctx + (min(rows, r0 + S::kRows) - 1) / group);
+  const int splits = keys.slices(ps);
+  if (split >= splits) return;
 
   // this lane's row; it holds the row's scores against half of a tile's keys, its partner lane +- 32 the others
   const int r = w0 + n;
@@ -77,17 +79,13 @@ __global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attenti
   for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[cb][i] = 0.f;
-  // positions the block's and the wave's rows span (rows in front of the sequence, at positions below 0, see nothing)
-  const int p_lo = max(0, ctx + r0 / group), p_hi = ctx + (min(rows, r0 + S::kRows) - 1) / group;
+  // positions the block's and the wave's rows span
+  const int p_hi = ctx + (min(rows, r0 + S::kRows) - 1) / group;
   const int w_lo = ctx + min(rows - 1, w0) / group, w_hi = ctx + min(rows - 1, w0 + 31) / group;
   const int w_first_lo = first_key(a, w_lo), w_first_hi = first_key(a, w_hi);
   const bool full = w0 + 32 <= rows, any = w0 < rows;
-  // the tiles: those of the kept first keys that lie before the window's first, then the window's
-  const int from = first_key(a, p_lo) / kTileKeys * kTileKeys;
-  const int kept = bounded(a) ? min((a.keep_first + kTileKeys - 1) / kTileKeys * kTileKeys, from) / kTileKeys : 0;
-  const int tiles = p_hi < 0 ? 0 : kept + (p_hi - from) / kTileKeys + 1;
-  const int per = (tiles + splits - 1) / splits, t_lo = split * per, t_hi = min(tiles, t_lo + per);
-  auto key0 = [&](int t) { return t < kept ? t * kTileKeys : from + (t - kept) * kTileKeys; };
+  const int per = (keys.tiles + splits - 1) / splits, t_lo = split * per, t_hi = min(keys.tiles, t_lo + per);
+  auto key0 = [&](int t) { return keys.first(t); };
 
   const ScaledRow lay = scaled_row(a.num_kv_heads, D, 2);
   const int64_t row_elems = S::Scaled ? lay.elems : S::Shared ? D + static_cast<int64_t>(a.num_kv_heads) * DV : static_cast<int64_t>(a.num_kv_heads) * (S::Inside ? D : D + DV);
@@ -224,7 +222,7 @@ __global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attenti
   if (!ok) return;
   const int64_t token = row0 + qi;
   if (splits > 1) {
-    float* part = static_cast<float*>(a.workspace) + ((token * a.num_heads + h) * splits + split) * partial_row_floats(DV);
+    float* part = ps.parts + ((token * a.num_heads + h) * ps.splits + split) * partial_row_floats(DV);
     if (hh == 0) part[DV] = m, part[DV + 1] = l;
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb)

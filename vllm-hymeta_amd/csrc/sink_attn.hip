@@ -875,8 +875,6 @@ __device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a,
   if (lane == 0) s_red[1][wave] = l;
   __syncthreads();
   l = (s_red[1][0] + s_red[1][1]) + (a.sink ? __builtin_amdgcn_exp2f(sink2 - m) : 0.f);
-  float inv = l > 0.f ? 1.f / l : 0.f;
-  if (a.head_gate) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[t * a.head_gate_stride_t + h]));
   const int quads = DV / 4, turns = kCombineThreads / quads, turn = tid / quads, c = 4 * (tid % quads);
   f32x4v acc = f32x4v{0.f, 0.f, 0.f, 0.f};
   if (turn < turns) {
@@ -893,6 +891,8 @@ __device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a,
       for (int k = 1; k < turns; ++k) acc += s_acc[tid + k * quads];
   }
   if (turn != 0) return;
+  float inv = l > 0.f ? 1.f / l : 0.f;
+  if (a.head_gate) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[t * a.head_gate_stride_t + h]));
   acc *= inv;
   if (a.elem_gate) {
     float gate[4];
@@ -904,25 +904,59 @@ __device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a,
       u32x2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
 }
 
-// grid = (sequences, heads): the rows of a decode step.
-__global__ __launch_bounds__(kCombineThreads) void sink_attention_decode_combine_kernel(hymeta_sink_attention_args a, int splits, HeadSlice hs) {
-  // (splits: partials per (sequence, key/value head): one per slice, or one per wave of a slice)
-  const int s = blockIdx.x;
-  const int t = a.query_start_loc[s];
-  if (a.query_start_loc[s + 1] - t != 1) return;
-  const int group = a.num_heads / a.num_kv_heads, HG = hs.count ? hs.count : group;
-  const int g = blockIdx.y / HG, r = blockIdx.y % HG, h = g * group + hs.first + r;
-  const size_t row = partial_row_floats(a.v_dim), stride = HG * row;
-  combine_row(a, static_cast<const float*>(a.workspace) + (static_cast<size_t>(s) * a.num_kv_heads + g) * splits * stride + r * row, stride, splits, t, h);
-}
+// How the keys of portions are cut: into `splits` slices at most, whose partials lie at `parts`, [row][head][splits]; blocks of
+// up to `whole` tiles of 64 keys are not cut.
+struct PortionSlices {
+  int splits = 1, whole = 0, least = 0;           // (least: the keys of a slice at least)
+  float* parts = nullptr;
+};
+constexpr int kPortionRows = 128;              // (query, head) rows of a block, the heads of a key/value head side by side
 
-// grid = (rows, heads): the rows of prompts' portions whose keys were cut into slices.
-__global__ __launch_bounds__(kCombineThreads) void sink_attention_rows_combine_kernel(hymeta_sink_attention_args a, int splits) {
-  const int t = blockIdx.x, h = blockIdx.y, s = seq_of_row(a.query_start_loc, a.num_seqs, t);
-  const int end = a.query_start_loc[s + 1];
-  if (end - a.query_start_loc[s] <= 1 || t >= end) return;      // (rows behind the last portion have no partials)
+// The keys that rows at positions p_first .. p_hi see, in tiles of Keys: first the kept first keys that lie before the window's
+// first tile, then the window's.  Rows in front of the sequence, at positions below 0, see nothing.
+struct BlockKeys {
+  int from, kept, tiles, size;
+  __device__ __forceinline__ int first(int t) const { return t < kept ? t * size : from + (t - kept) * size; }
+  __device__ __forceinline__ int slices(const PortionSlices& ps) const {
+    return tiles * size <= ps.whole * kTileKeys ? 1 : max(1, min(ps.splits, tiles * size / ps.least));
+  }
+};
+template <int Keys>
+__device__ __forceinline__ BlockKeys block_keys(const hymeta_sink_attention_args& a, int p_first, int p_hi) {
+  BlockKeys b;
+  b.size = Keys;
+  b.from = first_key(a, max(0, p_first)) / Keys * Keys;
+  b.kept = bounded(a) ? min((a.keep_first + Keys - 1) / Keys * Keys, b.from) / Keys : 0;
+  b.tiles = p_hi < 0 ? 0 : b.kept + (p_hi - b.from) / Keys + 1;
+  return b;
+}
+// Block `number` of the step's portions.
+__device__ __forceinline__ PieceAt portion_block(const hymeta_sink_attention_args& a, int number) {
+  const int group = a.num_heads / a.num_kv_heads;
+  return piece_at(a.query_start_loc, a.num_seqs, number, [=](int q) { return q > 1 ? (q * group + kPortionRows - 1) / kPortionRows : 0; });
+}
+constexpr int kWideKeys = 32;                  // a tile of the kernels over wide latents
+
+// grid = (sequences + rows where portions' keys were cut, heads): the rows of single-row sequences, and the rows of portions whose
+// blocks were cut.  One launch for both: a step of both takes no more launches than without slices.
+__global__ __launch_bounds__(kCombineThreads) void sink_attention_combine_kernel(hymeta_sink_attention_args a, int splits, HeadSlice hs, PortionSlices ps) {
+  // (splits: partials per (sequence, key/value head): one per slice, or one per wave of a slice)
+  const int group = a.num_heads / a.num_kv_heads, HG = hs.count ? hs.count : group;
+  const int g = blockIdx.y / HG, r = blockIdx.y % HG, in_group = hs.first + r, h = g * group + in_group;
   const size_t row = partial_row_floats(a.v_dim);
-  combine_row(a, static_cast<const float*>(a.workspace) + (static_cast<size_t>(t) * a.num_heads + h) * splits * row, row, splits, t, h);
+  if (blockIdx.x < a.num_seqs) {
+    const int s = blockIdx.x, t = a.query_start_loc[s];
+    if (a.query_start_loc[s + 1] - t != 1) return;
+    const size_t stride = HG * row;
+    combine_row(a, static_cast<const float*>(a.workspace) + (static_cast<size_t>(s) * a.num_kv_heads + g) * splits * stride + r * row, stride, splits, t, h);
+    return;
+  }
+  const int t = blockIdx.x - a.num_seqs, s = seq_of_row(a.query_start_loc, a.num_seqs, t), row0 = a.query_start_loc[s], end = a.query_start_loc[s + 1];
+  if (end - row0 <= 1 || t >= end) return;             // (rows behind the last portion have no partials)
+  const int ctx = a.seq_lens[s] - (end - row0), rows = (end - row0) * group, r0 = ((t - row0) * group + in_group) / kPortionRows * kPortionRows;
+  const int p_first = ctx + r0 / group, p_hi = ctx + (min(rows, r0 + kPortionRows) - 1) / group;
+  const int n = a.v_dim > 128 ? block_keys<kWideKeys>(a, p_first, p_hi).slices(ps) : block_keys<kTileKeys>(a, p_first, p_hi).slices(ps);
+  if (n > 1) combine_row(a, ps.parts + (static_cast<size_t>(t) * a.num_heads + h) * ps.splits * row, row, n, t, h);
 }
 
 }  // namespace
@@ -977,55 +1011,88 @@ inline int decode_splits(int num_seqs, int num_heads, int num_kv_heads, int tile
   return std::max(1, std::min(splits, tiles));
 }
 
-// Slices a portion's keys are cut into: where the blocks of 128 rows do not fill the chip (`target` workgroups) and the
-// workspace has room for the slices' partials, at least 4 tiles of 64 keys each (a slice's queries, its first tile and its
-// partial cost about two tiles).  7 rows x 28 heads behind 6000 keys: 299 -> 29 us; 40
-// rows x 28 heads on latents of 512 + 64, twice: 592 -> 77; 300 rows on latents of 128 + 64, twice: 233 -> 101.
+inline int64_t decode_partial_bytes(int num_seqs, int num_heads, int num_kv_heads, int v_dim, int max_seq_len) {
+  const int splits = decode_splits(num_seqs, num_heads, num_kv_heads, decode_tiles(max_seq_len < 1 ? 1 : max_seq_len));
+  return static_cast<int64_t>(num_seqs) * splits * kDecodeWaves * num_heads * static_cast<int64_t>(partial_row_floats(v_dim)) * 4;
+}
+
+// Bound on the portions' blocks of 128 rows: as many of the longest as there are sequences, or the rows' and one begun per
+// portion of two rows or more.
+inline int64_t portion_blocks(int num_tokens, int num_seqs, int group, int max_query_len) {
+  const int64_t each = (static_cast<int64_t>(max_query_len) * group + kPortionRows - 1) / kPortionRows;
+  return std::max<int64_t>(1, std::min<int64_t>(each * num_seqs, static_cast<int64_t>(num_tokens) * group / kPortionRows + std::min(num_seqs, num_tokens / 2)));
+}
+// Slices a portion's keys are cut into: where the blocks that the step's portions are worth (long_portions) do not fill the chip
+// (`target` workgroups) and the workspace has room for the partials (bounded: every row of the step has a place).  A slice's
+// queries, its first tile and its partial cost about two tiles of 64 keys, and a (row, head) of the merge about 1 / 768 of one,
+// so that blocks of fewer tiles stay whole.  7 rows x 28 heads behind 6000 keys: 299 -> 29 us; 40 rows x 28 heads on latents of
+// 512 + 64, twice: 592 -> 77; 300 rows on latents of 128 + 64, twice: 233 -> 101.
+//
+// Beside single rows, whose keys say nothing of the portion's, the merge's look at every row of the step (2 to 6 us) is lost on a
+// portion that begins its sequence.  Up to kFewBlocks, where one behind many keys would have nothing but its own tiles to wait
+// for, it is worth it (with at most kMostNumbers numbers of blocks, most of which have none): 40 rows x 28 heads behind 6000
+// keys beside 63 single rows take 164 us where they took 417, with a window of 1024 57 where they took 85 (331 and 77 with a
+// workgroup per head); without keys in front of them 43 where they took 41.  Above, only where all numbers fit the chip.
+constexpr int64_t kMostPartialBytes = 96 << 20, kFewBlocks = 32, kMostNumbers = 2048;
 inline int64_t portion_partial_bytes(int num_tokens, int num_heads, int v_dim) {
   return static_cast<int64_t>(num_tokens) * num_heads * static_cast<int64_t>(partial_row_floats(v_dim)) * 4;
 }
-inline int portion_target(int v_dim) { return v_dim > 128 ? 256 : 512; }       // one workgroup on a compute unit (wide_latent.h), or two
-inline int portion_splits(int num_tokens, int num_seqs, int num_heads, int num_kv_heads, int max_query_len, int tiles, int target) {
-  constexpr int64_t kRows = 128;
-  const int64_t group = std::max(1, num_heads / num_kv_heads);
-  const int64_t each = (max_query_len * group + kRows - 1) / kRows, all = (num_tokens * group + kRows - 1) / kRows + num_seqs;
-  const int64_t blocks = std::min(each * num_seqs, all) * num_kv_heads;
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(target / blocks, tiles / 4)));
+inline PortionSlices portion_slices(int num_tokens, int num_seqs, int num_heads, int num_kv_heads, int v_dim, int max_query_len, int tiles) {
+  PortionSlices ps;
+  ps.least = (v_dim > 128 ? 2 : 4) * kTileKeys;        // (a tile of a wide latent takes four times as long)
+  const int group = std::max(1, num_heads / num_kv_heads), target = v_dim > 128 ? 256 : 512;       // one workgroup on a compute unit (wide_latent.h), or two
+  const int64_t each = (static_cast<int64_t>(max_query_len) * group + kPortionRows - 1) / kPortionRows, portions = long_portions(num_tokens, num_seqs, max_query_len);
+  const int64_t blocks = each * portions * num_kv_heads;
+  int64_t most = std::min<int64_t>(tiles / (ps.least / kTileKeys), kMostPartialBytes / portion_partial_bytes(num_tokens, num_heads, v_dim));
+  if (num_seqs > portions) most = std::min<int64_t>(most, (blocks > kFewBlocks ? target : kMostNumbers) / (portion_blocks(num_tokens, num_seqs, group, max_query_len) * num_kv_heads));
+  ps.whole = static_cast<int>(std::min<int64_t>(tiles, std::max<int64_t>(2 * ps.least / kTileKeys - 1, portions * max_query_len * num_heads / 768)));
+  if (tiles > ps.whole) ps.splits = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(target / blocks, most)));
+  // (an odd stride: the first slices alone, where blocks stay whole, are on all of the chip's 8 dies)
+  if (num_seqs > portions && blocks <= kFewBlocks && ps.splits > 2) ps.splits -= 1 - ps.splits % 2;
+  return ps;
 }
-inline int portion_splits(const hymeta_sink_attention_args& a) {
-  const int splits = portion_splits(a.num_tokens, a.num_seqs, a.num_heads, a.num_kv_heads, a.max_query_len, decode_tiles(a), portion_target(a.v_dim));
-  const int64_t room = static_cast<int64_t>(a.workspace_bytes) / portion_partial_bytes(a.num_tokens, a.num_heads, a.v_dim);
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(splits, room)));
+inline PortionSlices portion_slices(const hymeta_sink_attention_args& a) {
+  PortionSlices ps;
+  if (a.max_query_len <= 1) return ps;
+  ps = portion_slices(a.num_tokens, a.num_seqs, a.num_heads, a.num_kv_heads, a.v_dim, a.max_query_len, decode_tiles(a));
+  const int64_t decode = decode_partial_bytes(a.num_seqs, a.num_heads, a.num_kv_heads, a.v_dim, a.max_seq_len);
+  const int64_t room = (static_cast<int64_t>(a.workspace_bytes) - decode) / portion_partial_bytes(a.num_tokens, a.num_heads, a.v_dim);
+  ps.splits = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(ps.splits, room)));
+  ps.parts = static_cast<float*>(a.workspace) + decode / 4;
+  return ps;
+}
+inline dim3 portion_grid(const hymeta_sink_attention_args& a, const PortionSlices& ps) {
+  return dim3(static_cast<uint32_t>(portion_blocks(a.num_tokens, a.num_seqs, a.num_heads / a.num_kv_heads, a.max_query_len) * ps.splits * a.num_kv_heads));
+}
+void launch_combine(const hymeta_sink_attention_args& a, hipStream_t st, int splits, HeadSlice hs, const PortionSlices& ps) {
+  const dim3 grid(a.num_seqs + (ps.splits > 1 ? a.num_tokens : 0), hs.count ? hs.count * a.num_kv_heads : a.num_heads);
+  hipLaunchKernelGGL(sink_attention_combine_kernel, grid, dim3(kCombineThreads), 0, st, a, splits, hs, ps);
 }
 
 template <int C>
 int launch_wide_latent(const hymeta_sink_attention_args& a, hipStream_t st) {
   const int group = a.num_heads / a.num_kv_heads;
+  const PortionSlices ps = portion_slices(a);
   if (a.max_query_len > 1) {
-    const int64_t rows = static_cast<int64_t>(a.max_query_len) * group;
-    const int splits = portion_splits(a);
-    const dim3 grid(static_cast<uint32_t>((rows + kWideRows - 1) / kWideRows * splits), a.num_kv_heads, a.num_seqs);
-    hipLaunchKernelGGL((latent_prefill_kernel<C>), grid, dim3(64 * kWideWaves), 0, st, a, splits);
-    if (splits > 1) hipLaunchKernelGGL(sink_attention_rows_combine_kernel, dim3(a.num_tokens, a.num_heads), dim3(kCombineThreads), 0, st, a, splits);
+    hipLaunchKernelGGL((latent_prefill_kernel<C>), portion_grid(a, ps), dim3(64 * kWideWaves), 0, st, a, ps);
   }
   // one workgroup per compute unit (its rings fill the LDS): as many as there are units
   const int64_t slices = (group + kLatentHeads - 1) / kLatentHeads, items = static_cast<int64_t>(a.num_seqs) * a.num_kv_heads;
   const int splits = static_cast<int>(std::min<int64_t>((256 + items * slices - 1) / (items * slices), decode_tiles(a)));
   const dim3 grid(static_cast<uint32_t>((items * splits + 7) / 8 * 8 * slices));
   hipLaunchKernelGGL((latent_decode_kernel<C>), grid, dim3(64 * kLatentWaves), 0, st, a, splits);
-  hipLaunchKernelGGL(sink_attention_decode_combine_kernel, dim3(a.num_seqs, a.num_heads), dim3(kCombineThreads), 0, st, a, splits, HeadSlice{});
+  launch_combine(a, st, splits, HeadSlice{}, ps);
   return launch_status();
 }
 
 template <int D, int DV, int Layout = HYMETA_KV_KEY_THEN_VALUE>
 int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st) {
+  PortionSlices ps;
   if (a.max_query_len > 1) {
     if constexpr (D <= 192) {
-      const int64_t rows = static_cast<int64_t>(a.max_query_len) * (a.num_heads / a.num_kv_heads);
-      constexpr int kRows = RowShape<D, DV, Layout>::kRows;
-      const int splits = portion_splits(a);
-      const dim3 grid(static_cast<uint32_t>((rows + kRows - 1) / kRows * splits), a.num_kv_heads, a.num_seqs);
-      auto launch = [&](auto rule) { hipLaunchKernelGGL((row_prefill_kernel<D, DV, Layout, decltype(rule)::value>), grid, dim3(256), 0, st, a, splits); };
+      ps = portion_slices(a);
+      const dim3 grid = portion_grid(a, ps);
+      auto launch = [&](auto rule) { hipLaunchKernelGGL((row_prefill_kernel<D, DV, Layout, decltype(rule)::value>), grid, dim3(256), 0, st, a, ps); };
       const bool plain = a.softcap <= 0.f && a.bias_mode != HYMETA_BIAS_LOG_DISTANCE;
       if constexpr (Layout == HYMETA_KV_SCALED_KEY) launch(std::integral_constant<int, kPlain>{});
       else if (plain) launch(std::integral_constant<int, kPlain>{});
@@ -1033,7 +1100,6 @@ int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st) {
         if (a.softcap <= 0.f) launch(std::integral_constant<int, kLogBias>{});
         else launch(std::integral_constant<int, kAnyRule>{});
       } else launch(std::integral_constant<int, kAnyRule>{});
-      if (splits > 1) hipLaunchKernelGGL(sink_attention_rows_combine_kernel, dim3(a.num_tokens, a.num_heads), dim3(kCombineThreads), 0, st, a, splits);
     } else {
       constexpr int kRows = 16 * kPrefillWaves;
       const dim3 grid((a.max_query_len + kRows - 1) / kRows, a.num_heads, a.num_seqs);
@@ -1056,7 +1122,7 @@ int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st) {
       hipLaunchKernelGGL((sink_attention_decode_mfma_kernel<D, DV, 2, Layout>), grid, dim3(64 * kDecodeWaves), 0, st, a, splits, tiles_per_split, hs);
       parts = splits * (DecodeMerge<D, DV, 2>::value ? 1 : kDecodeWaves);
     }
-    hipLaunchKernelGGL(sink_attention_decode_combine_kernel, dim3(a.num_seqs, a.num_kv_heads * hs.count), dim3(kCombineThreads), 0, st, a, parts, hs);
+    launch_combine(a, st, parts, hs, ps);
   }
   return launch_status();
 }
@@ -1116,16 +1182,15 @@ extern "C" int hymeta_scaled_key_cache(const hymeta_scaled_key_cache_args* args,
 extern "C" size_t hymeta_sink_attention_workspace_bytes(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads, int32_t v_dim,
                                                         int32_t max_seq_len) {
   if (num_seqs <= 0 || num_heads <= 0 || num_kv_heads <= 0 || v_dim <= 0) return 0;
-  const int splits = decode_splits(num_seqs, num_heads, num_kv_heads, decode_tiles(max_seq_len < 1 ? 1 : max_seq_len));
-  return static_cast<size_t>(num_seqs) * splits * kDecodeWaves * num_heads * partial_row_floats(v_dim) * sizeof(float);
+  return static_cast<size_t>(decode_partial_bytes(num_seqs, num_heads, num_kv_heads, v_dim, max_seq_len));
 }
 
 extern "C" size_t hymeta_sink_attention_portion_workspace_bytes(int32_t num_tokens, int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads,
                                                                 int32_t v_dim, int32_t max_query_len, int32_t max_seq_len, int64_t span,
                                                                 int32_t keep_first) {
   if (num_tokens <= 0 || num_seqs <= 0 || num_heads <= 0 || num_kv_heads <= 0 || v_dim <= 0 || max_query_len <= 1 || max_seq_len < 1) return 0;
-  const int splits = portion_splits(num_tokens, num_seqs, num_heads, num_kv_heads, max_query_len, decode_tiles(max_seq_len, span, keep_first), portion_target(v_dim));
-  return splits > 1 ? static_cast<size_t>(splits) * portion_partial_bytes(num_tokens, num_heads, v_dim) : 0;
+  const int splits = portion_slices(num_tokens, num_seqs, num_heads, num_kv_heads, v_dim, max_query_len, decode_tiles(max_seq_len, span, keep_first)).splits;
+  return splits > 1 ? static_cast<size_t>(decode_partial_bytes(num_seqs, num_heads, num_kv_heads, v_dim, max_seq_len) + splits * portion_partial_bytes(num_tokens, num_heads, v_dim)) : 0;
 }
 
 extern "C" int hymeta_sink_attention(const hymeta_sink_attention_args* args, hymeta_stream_t stream) {

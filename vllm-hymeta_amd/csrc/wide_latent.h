@@ -78,7 +78,8 @@ struct LatentCopy {
   }
 };
 
-constexpr int kWideWaves = 8, kWideRows = 16 * kWideWaves, kWideKeys = 32;
+constexpr int kWideWaves = 8, kWideRows = 16 * kWideWaves;
+static_assert(kWideRows == kPortionRows, "the merge finds a row's block");
 
 template <int C>
 struct WideSmem {
@@ -89,7 +90,7 @@ struct WideSmem {
   int moved[2][kWideWaves];                       // whether a row block has any factor but 1
 };
 
-// Portions of prompts: grid = (blocks of 128 rows x slices of the keys, key/value heads, sequences); a row is a (query, head) pair, the heads of a
+// Portions of prompts: grid = their blocks of 128 rows x slices of the keys at most x key/value heads; a row is a (query, head) pair, the heads of a
 // key/value head side by side, so that a portion of a few tokens fills its blocks.  Sequences with one row are left to the
 // decode form.
 //
@@ -100,16 +101,14 @@ struct WideSmem {
 // 512 + 64: 1.65 ms = 1.04 PFLOP/s of the products issued (both parts of the weights counted), where launches over value
 // slices of 128, each repeating the scores, took 11.3 ms.
 template <int C>
-__global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_sink_attention_args a, int splits) {
+__global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_sink_attention_args a, PortionSlices ps) {
   constexpr int D = C + 64, kRowB = 2 * D, kSteps = D / 32, CB = C / 128;
   __shared__ __attribute__((aligned(16))) WideSmem<C> sm;
-  const int turn = gridDim.x - 1 - blockIdx.x;              // the longest rows first
-  const int s = blockIdx.z, g = blockIdx.y, tile = turn / splits, split = turn % splits;
-  const int row0 = a.query_start_loc[s];
-  const int q = a.query_start_loc[s + 1] - row0;
-  const int group = a.num_heads / a.num_kv_heads;
-  const int rows = q * group, r0 = tile * kWideRows;
-  if (q <= 1 || r0 >= rows) return;
+  const int group = a.num_heads / a.num_kv_heads, g = blockIdx.x % a.num_kv_heads, item = blockIdx.x / a.num_kv_heads, split = item % ps.splits;
+  const PieceAt block = portion_block(a, item / ps.splits);
+  const int s = block.seq, row0 = block.row0, q = block.rows, rows = q * group;
+  if (s < 0) return;
+  const int r0 = ((rows - 1) / kWideRows - block.index) * kWideRows;        // (the longest rows first)
   const int lane = threadIdx.x & 63, n = lane & 15, g4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ctx = a.seq_lens[s] - q;
@@ -120,26 +119,25 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
   const int qi = ok ? r / group : 0, h = g * group + (ok ? r % group : 0);
   const int pos = ok ? ctx + qi : -1;
   const float ba = a.bias_mode ? a.bias_a[h] : 0.f, bb = a.bias_mode == HYMETA_BIAS_LOG_DISTANCE ? a.bias_b[h] : 0.f;
-  const bool sink = a.sink && splits == 1;            // (of several slices of the keys none has the sink: the merge adds it)
-  float m = sink ? (a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f) : -INFINITY;
-  float l = sink && g4 == 0 ? 1.f : 0.f;              // the sink's exp(m - m), counted once per row
   bf16x8 qf[kSteps];
   {
     const uint16_t* qrow = static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(row0 + qi) * a.q_stride_t + static_cast<int64_t>(h) * D;
 #pragma unroll
     for (int st = 0; st < kSteps; ++st) qf[st] = ok ? __builtin_bit_cast(bf16x8, ld16g(qrow + 32 * st + 8 * g4)) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
   }
-  // positions the block's and the wave's rows span (rows in front of the sequence, at positions below 0, see nothing)
-  const int p_lo = max(0, ctx + r0 / group), p_hi = ctx + (min(rows, r0 + kWideRows) - 1) / group;
+  // positions the block's and the wave's rows span
+  const int p_hi = ctx + (min(rows, r0 + kWideRows) - 1) / group;
   const int w_lo = ctx + min(rows - 1, r0 + 16 * wave) / group, w_hi = ctx + min(rows - 1, r0 + 16 * wave + 15) / group;
   const int w_first = first_key(a, w_hi);
   const bool full = r0 + 16 * wave + 16 <= rows;
-  // the tiles: those of the kept first keys that lie before the window's first, then the window's
-  const int from = first_key(a, p_lo) / kWideKeys * kWideKeys;
-  const int kept = bounded(a) ? min((a.keep_first + kWideKeys - 1) / kWideKeys * kWideKeys, from) / kWideKeys : 0;
-  const int all = p_hi < 0 ? 0 : kept + (p_hi - from) / kWideKeys + 1, per = (all + splits - 1) / splits;
-  const int t0 = split * per, tiles = min(all - t0, per);          // this slice's
-  auto key0 = [&](int t) { return t0 + t < kept ? (t0 + t) * kWideKeys : from + (t0 + t - kept) * kWideKeys; };
+  const BlockKeys keys = block_keys<kWideKeys>(a, ctx + r0 / group, p_hi);
+  const int splits = keys.slices(ps);
+  if (split >= splits) return;
+  const bool sink = a.sink && splits == 1;            // (of several slices of the keys none has the sink: the merge adds it)
+  float m = sink ? (a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f) : -INFINITY;
+  float l = sink && g4 == 0 ? 1.f : 0.f;              // the sink's exp(m - m), counted once per row
+  const int per = (keys.tiles + splits - 1) / splits, t0 = split * per, tiles = min(keys.tiles - t0, per);          // this slice's
+  auto key0 = [&](int t) { return keys.first(t0 + t); };
 
   f32x4v o[kWideWaves][CB];                           // O^T: this wave's columns x the rows of block rb
 #pragma unroll
@@ -286,8 +284,8 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
   if (splits > 1) {
-    float* parts = static_cast<float*>(a.workspace) + split * partial_row_floats(C);
-    const size_t stride = splits * partial_row_floats(C);
+    float* parts = ps.parts + split * partial_row_floats(C);
+    const size_t stride = ps.splits * partial_row_floats(C);
     if (g4 == 0 && ok) {
       float* part = parts + (static_cast<size_t>(row0 + qi) * a.num_heads + h) * stride;
       part[C] = m, part[C + 1] = l;
