@@ -150,3 +150,14 @@ def test_bounds_larger_than_the_step(D, Dv, lens):
     run = lambda most_rows, most_keys: hip_ops.sink_attention(q, cache, table, starts, ends, 1, D, Dv, D ** -0.5, most_rows, most_keys, value_in_key=inside)  # noqa: E731
     a, b = run(max(lens), 300 + max(lens)).double(), run(500, 512).double()
     assert torch.isfinite(a).all() and (a - b).norm() <= BOUND * a.norm()
+
+
+@pytest.mark.parametrize("D,dtype", [(512, torch.bfloat16), (128, torch.float32)])
+def test_kernels_without_slices_ask_for_no_room_for_them(D, dtype, monkeypatch):
+    from vllm_hymeta import _C, hip_ops
+    dev, asked, workspace = "cuda", [], hip_ops._workspace
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
+    monkeypatch.setattr(hip_ops, "_workspace", lambda device, nbytes, tag: asked.append(nbytes) or workspace(device, nbytes, tag))
+    q, cache = torch.randn(5, 4, D, device=dev).to(dtype), torch.randn(64, 64, 1, D + 2 * 64, device=dev).to(dtype)
+    out = hip_ops.sink_attention(q, cache, torch.arange(64, dtype=torch.int32, device=dev)[None], i32([0, 5]), i32([4096]), 2, D, 64, D ** -0.5, 5, 4096, shared_key=True)
+    assert asked == [_C.load().hymeta_sink_attention_workspace_bytes(1, 4, 2, 64, 4096)] and torch.isfinite(out).all()
