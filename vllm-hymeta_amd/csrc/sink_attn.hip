@@ -562,18 +562,17 @@ __device__ __forceinline__ void load_bias(WaveRows<D, DV, RB>& w, int rb, const 
   w.bb[rb] = a.bias_mode == HYMETA_BIAS_LOG_DISTANCE ? a.bias_b[h] : 0.f;
 }
 
-// Portions of prompts with keys of more than 192 elements (shorter ones: row_attn.h): grid = (tiles of 16 rows per wave, heads,
-// sequences); sequences with one row are left to the decode form.  4 waves: the query fragments (D / 8 registers) and the
+// Portions of prompts over rows of HYMETA_KV_SHARED_KEY with keys of more than 192 elements (shorter keys and other rows:
+// row_attn.h, wide_latent.h): grid = (tiles of 16 rows per wave, heads, sequences); sequences with one row are left to the decode
+// form.  4 waves: the query fragments (D / 8 registers) and the
 // staging registers do not leave a wave of 8 its accumulators within 256 registers.
 constexpr int kPrefillWaves = 4;
 
-template <int D, int DV, int RB, int Layout>
-__global__ __launch_bounds__(64 * kPrefillWaves) void sink_attention_prefill_mfma_kernel(hymeta_sink_attention_args a) {
-  constexpr int kRows = 16 * RB * kPrefillWaves;
+template <int D, int DV>
+__global__ __launch_bounds__(64 * kPrefillWaves) void sink_attention_prefill_shared_kernel(hymeta_sink_attention_args a) {
+  constexpr int kRows = 16 * kPrefillWaves;
   constexpr int kImages = 2 * sizeof(MfmaSmem<D, DV>) <= 159 * 1024 ? 2 : 1;        // (160 KB of LDS)
-  constexpr bool kScaled = Layout == HYMETA_KV_SCALED_KEY;
   __shared__ MfmaSmem<D, DV> sm[kImages];
-  __shared__ __attribute__((aligned(16))) float s_scale[kImages][kScaled ? kTileKeys : 4];
   // A prompt's later rows (of the sequence, or of a chunk) see more keys.  The row blocks are handed out from the last on, all
   // heads of a block side by side: what runs at the end is short, and the chip's 8 dies, which take workgroups round robin,
   // get the same mix of blocks (with the blocks side by side a die gets every eighth block of every head: measured at 8192
@@ -587,23 +586,19 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void sink_attention_prefill_mfm
   const int g = h / (a.num_heads / a.num_kv_heads);
   const int ctx = a.seq_lens[s] - q;
   const int32_t* bt = a.block_tables + static_cast<int64_t>(s) * a.block_table_stride;
-  WaveRows<D, DV, RB> w;
-  const int wrow = tile * kRows + wave * 16 * RB;
+  WaveRows<D, DV, 1> w;
+  const int wrow = tile * kRows + wave * 16, r = wrow + n;
+  const bool ok = r < q;
+  w.pos[0] = ok ? ctx + r : -1;
+  w.first[0] = first_key(a, ctx + r);
+  load_bias<D, DV, 1>(w, 0, a, h);
+  w.m[0] = a.sink ? (a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f) : -INFINITY;
+  w.l[0] = (a.sink && g4 == 0) ? 1.f : 0.f;          // the sink's exp(m - m), counted once per row
+  load_q<D, DV, 1>(w, 0, ok ? static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(row0 + r) * a.q_stride_t + static_cast<int64_t>(h) * D : nullptr);
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const int r = wrow + 16 * rb + n;
-    const bool ok = r < q;
-    w.pos[rb] = ok ? ctx + r : -1;
-    w.first[rb] = first_key(a, ctx + r);
-    load_bias<D, DV, RB>(w, rb, a, h);
-    w.m[rb] = a.sink ? (a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f) : -INFINITY;
-    w.l[rb] = (a.sink && g4 == 0) ? 1.f : 0.f;        // the sink's exp(m - m), counted once per row
-    load_q<D, DV, RB>(w, rb, ok ? static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(row0 + r) * a.q_stride_t + static_cast<int64_t>(h) * D : nullptr);
-#pragma unroll
-    for (int cb = 0; cb < DV / 16; ++cb) w.o[rb][cb] = f32x4v{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int cb = 0; cb < DV / 16; ++cb) w.o[0][cb] = f32x4v{0.f, 0.f, 0.f, 0.f};
   const int block_last = ctx + min(q, tile * kRows + kRows) - 1;      // last key any row of the block sees
-  const int wave_last = ctx + min(q, wrow + 16 * RB) - 1;
+  const int wave_last = ctx + min(q, wrow + 16) - 1;
   const int first_lo = first_key(a, ctx + wrow), first_hi = first_key(a, wave_last);           // of the wave's rows
   const int j_first = first_key(a, ctx + tile * kRows) / kTileKeys * kTileKeys;
   // the tiles of the kept first keys that lie before the window's first tile come first, then the window's
@@ -612,22 +607,22 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void sink_attention_prefill_mfm
   auto next = [&](int j0) { return (j0 < keep_end && j0 + kTileKeys >= keep_end) ? j_first : j0 + kTileKeys; };
   // two LDS images: while the waves multiply tile t out of one, tile t + 1 goes into the other and the loads of tile
   // t + 2 are in flight; one barrier per tile
-  TileStage<D, DV, 64 * kPrefillWaves, Layout> stage;
-  if (Layout == HYMETA_KV_SHARED_KEY) stage.value_at = D + g * DV;
+  TileStage<D, DV, 64 * kPrefillWaves, HYMETA_KV_SHARED_KEY> stage;
+  stage.value_at = D + g * DV;
   stage.issue(a, bt, g, j_start, block_last);
-  stage.commit(sm[0], s_scale[0]);
+  stage.commit(sm[0], nullptr);
   if (kImages == 2 && next(j_start) <= block_last) stage.issue(a, bt, g, next(j_start), block_last);
   __syncthreads();
   if constexpr (kImages == 2) {
     int buf = 0;
     for (int j0 = j_start; j0 <= block_last; j0 = next(j0), buf ^= 1) {
       const int j1 = next(j0), j2 = next(j1);
-      if (j1 <= block_last) stage.commit(sm[buf ^ 1], s_scale[buf ^ 1]);
+      if (j1 <= block_last) stage.commit(sm[buf ^ 1], nullptr);
       if (j2 <= block_last) stage.issue(a, bt, g, j2, block_last);
       if (wrow < q && j0 <= wave_last && !tile_shut(a, j0, first_lo)) {
         // tiles whose every key is visible to every row of the wave need no mask
-        if (tile_open(j0, ctx + wrow, first_hi)) attend_tile<D, DV, RB, 4, false, kScaled>(w, sm[buf], s_scale[buf], a, j0, 0);
-        else attend_tile<D, DV, RB, 4, true, kScaled>(w, sm[buf], s_scale[buf], a, j0, 0);
+        if (tile_open(j0, ctx + wrow, first_hi)) attend_tile<D, DV, 1, 4, false, false>(w, sm[buf], nullptr, a, j0, 0);
+        else attend_tile<D, DV, 1, 4, true, false>(w, sm[buf], nullptr, a, j0, 0);
       }
       __syncthreads();
     }
@@ -638,37 +633,33 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void sink_attention_prefill_mfm
       const bool more = next(j0) <= block_last;
       if (more) stage.issue(a, bt, g, next(j0), block_last);
       if (wrow < q && j0 <= wave_last && !tile_shut(a, j0, first_lo)) {
-        if (tile_open(j0, ctx + wrow, first_hi)) attend_tile<D, DV, RB, 4, false, kScaled>(w, sm[0], s_scale[0], a, j0, 0);
-        else attend_tile<D, DV, RB, 4, true, kScaled>(w, sm[0], s_scale[0], a, j0, 0);
+        if (tile_open(j0, ctx + wrow, first_hi)) attend_tile<D, DV, 1, 4, false, false>(w, sm[0], nullptr, a, j0, 0);
+        else attend_tile<D, DV, 1, 4, true, false>(w, sm[0], nullptr, a, j0, 0);
       }
       __syncthreads();
       if (more) {
-        stage.commit(sm[0], s_scale[0]);
+        stage.commit(sm[0], nullptr);
         __syncthreads();
       }
     }
   }
+  float l = w.l[0];
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (r >= q) return;
+  float inv = l > 0.f ? 1.f / l : 0.f;
+  if (a.head_gate) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[static_cast<int64_t>(row0 + r) * a.head_gate_stride_t + h]));
+  uint16_t* out = static_cast<uint16_t*>(a.out) + (static_cast<int64_t>(row0 + r) * a.num_heads + h) * DV;
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    float l = w.l[rb];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    const int r = wrow + 16 * rb + n;
-    if (r >= q) continue;
-    float inv = l > 0.f ? 1.f / l : 0.f;
-    if (a.head_gate) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[static_cast<int64_t>(row0 + r) * a.head_gate_stride_t + h]));
-    uint16_t* out = static_cast<uint16_t*>(a.out) + (static_cast<int64_t>(row0 + r) * a.num_heads + h) * DV;
+  for (int cb = 0; cb < DV / 16; ++cb) {
+    f32x4v o = w.o[0][cb] * inv;
+    if (a.elem_gate) {
+      float gate[4];
+      ActBf16::ld4(static_cast<const uint16_t*>(a.elem_gate) + static_cast<int64_t>(row0 + r) * a.elem_gate_stride_t + static_cast<int64_t>(h) * DV + 16 * cb + 4 * g4, gate);
 #pragma unroll
-    for (int cb = 0; cb < DV / 16; ++cb) {
-      f32x4v o = w.o[rb][cb] * inv;
-      if (a.elem_gate) {
-        float gate[4];
-        ActBf16::ld4(static_cast<const uint16_t*>(a.elem_gate) + static_cast<int64_t>(row0 + r) * a.elem_gate_stride_t + static_cast<int64_t>(h) * DV + 16 * cb + 4 * g4, gate);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] *= ActBf16::sigmoid(gate[e]);
-      }
-      *reinterpret_cast<u32x2*>(out + 16 * cb + 4 * g4) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+      for (int e = 0; e < 4; ++e) o[e] *= ActBf16::sigmoid(gate[e]);
     }
+    *reinterpret_cast<u32x2*>(out + 16 * cb + 4 * g4) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
   }
 }
 
@@ -1103,7 +1094,7 @@ int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st) {
     } else {
       constexpr int kRows = 16 * kPrefillWaves;
       const dim3 grid((a.max_query_len + kRows - 1) / kRows, a.num_heads, a.num_seqs);
-      hipLaunchKernelGGL((sink_attention_prefill_mfma_kernel<D, DV, 1, Layout>), grid, dim3(64 * kPrefillWaves), 0, st, a);
+      hipLaunchKernelGGL((sink_attention_prefill_shared_kernel<D, DV>), grid, dim3(64 * kPrefillWaves), 0, st, a);
     }
   }
   // sequences with a single row: every step but a pure prompt step has some; a prompt of one token is one too

@@ -29,6 +29,7 @@
 //     [slice][M][N], summed by the reduce kernel or by the consumer (the same contract as the decode-sized kernel).
 #include <cstdlib>
 
+#include "lds_copy.h"
 #include "stream_gemm.h"
 
 namespace hymeta {
@@ -49,16 +50,9 @@ __device__ __forceinline__ typename Acc<I8>::type mma(const u32x4& a, const u32x
   }
 }
 
-// 16 bytes per lane from global memory into LDS at (wave-uniform) dst + 16 lane.  Written as an asm statement, with
-// the waits for it counted by hand (wait_loads_then_barrier): the compiler books such a load on the LDS counter as
-// well, and while one is in flight -- here: always -- every wait for a fragment read becomes a wait for ALL of them.
-// (The non-temporal hint on the weight requests, which the decode-sized kernel's register loads gain from, was measured
-// here too: level on whole-K tiles, 3 to 5 us slower per launch on the K-sliced 7B shapes.)
-__device__ __forceinline__ void glds16(const char* src, char* dst) {
-  const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)dst));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
-}
-
+// The copies to LDS (copy16_to_lds) are always in flight here, the waits for them counted by hand.  (The non-temporal hint on
+// the weight requests, which the decode-sized kernel's register loads gain from, was measured here too: level on whole-K tiles,
+// 3 to 5 us slower per launch on the K-sliced 7B shapes.)
 template <int N>
 __device__ __forceinline__ void wait_loads_then_barrier() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
@@ -135,9 +129,9 @@ __device__ __forceinline__ void tall_wave(const StreamArgs& a, char* smem, const
   auto request = [&](int q, int g) {
     if (q >= kReq) return;
     if (q < kXInstr) {
-      glds16(src[q] + pair_off(g + 1), xbuf + ((g + 1) & 1) * kXBuf + dst[q]);
+      copy16_to_lds(src[q] + pair_off(g + 1), xbuf + ((g + 1) & 1) * kXBuf + dst[q]);
     } else {
-      glds16(src[q] + pair_off(g + 2), wbuf + ((g + 2) % kRing) * kWSlot + dst[q]);
+      copy16_to_lds(src[q] + pair_off(g + 2), wbuf + ((g + 2) % kRing) * kWSlot + dst[q]);
     }
   };
   // every wave: until all but its newest weight requests have landed, then until every wave's have -- at which point

@@ -41,7 +41,8 @@ __device__ __forceinline__ void finish_scores(const hymeta_sink_attention_args& 
 }
 
 // Keys [j0, j0 + Keys) of a sequence's key/value head into an LDS image of Keys rows of D elements, by waves `wave` of
-// `Waves`; keys past `last` repeat it (their weights are zero).  Pages hold a power of two of rows.
+// `Waves`; keys past `last` repeat it (their weights are zero).  Pages hold a power of two of rows.  Beside RowCopy, which keeps
+// the lanes' places in registers: none are left here (512 + 64: all 256, with 18 spilled).
 template <int D, int Keys, int Waves>
 struct LatentCopy {
   static constexpr int kChunks = D / 8, kInstr = Keys * kChunks / 64, kPerWave = (kInstr + Waves - 1) / Waves;
