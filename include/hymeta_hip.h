@@ -1193,11 +1193,12 @@ int hymeta_qk_norm_cache(const hymeta_qk_norm_cache_args* args, hymeta_stream_t 
  *   sink_logits, that has no value and is neither scaled nor biased) or 0
  *   out_i = sum_j p_ij v_j
  * Scores and weights are fp32 in both activation types.  Query row t of sequence s stands at position
- * seq_lens[s] - (query_start_loc[s + 1] - t).  bf16 rows with head_dim and v_dim of 64 or 128 run on the
+ * seq_lens[s] - (query_start_loc[s + 1] - t); a row in front of position 0 sees nothing and its output is 0.  bf16 rows with
+ * head_dim and v_dim of 64 or 128 run on the
  * matrix cores: portions of prompts in blocks of 128 (query, head) rows, short portions with their keys cut into slices as
  * the workspace allows, sequences with one row (decode) per key/value
  * head with its query heads (32 to a launch), split over the keys into `workspace`
- * (hymeta_sink_attention_workspace_bytes) and merged by a second launch.
+ * (hymeta_sink_attention_workspace_bytes); a last launch merges what was split.
  * max_query_len / max_seq_len: upper bounds of the step's portion and sequence lengths (they size the
  * grids).  Everything else runs a wave per (row, head). */
 enum hymeta_bias_mode { HYMETA_BIAS_NONE = 0, HYMETA_BIAS_LOG_DISTANCE = 1, HYMETA_BIAS_LINEAR_DISTANCE = 2 };
@@ -1205,8 +1206,9 @@ enum hymeta_bias_mode { HYMETA_BIAS_NONE = 0, HYMETA_BIAS_LOG_DISTANCE = 1, HYME
  * elements (hymeta_qk_norm_cache).  VALUE_IN_KEY: head_dim elements, of which the first v_dim are also the value (a
  * latent shared by keys and values followed by a rotated key part: hymeta_latent_kv_prep); v_dim <= head_dim.  With
  * VALUE_IN_KEY bf16 rows with v_dim 64 or 128 and head_dim = v_dim + 32 or v_dim + 64 run on the matrix cores (the
- * kernels of KEY_THEN_VALUE with another staging of the tiles), and so do v_dim 256 / 384 / 512 with head_dim = v_dim + 64,
- * as 2 / 3 / 4 launches over value slices of 128; other sizes a wave per (row, head).
+ * kernels of KEY_THEN_VALUE, which read the values from the keys' image), and so do v_dim 256 / 384 / 512 with head_dim = v_dim
+ * + 64 (kernels of their own, one pass over the keys for all value columns, 16 query heads of a decode row at a time); other
+ * sizes a wave per (row, head).
  * SHARED_KEY: a row is ONE key of head_dim elements that every query head reads, followed by num_kv_heads values of
  * v_dim elements; query head h reads value h / (num_heads / num_kv_heads) (hymeta_talk_qkv_prep: queries that were
  * mixed across heads against the concatenated keys of the key/value heads).  bf16 rows with head_dim 128 / 256 / 512 and

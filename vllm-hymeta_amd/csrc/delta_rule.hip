@@ -630,7 +630,8 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(hymeta_delta_rule
 // product with the reduced index in the order 4 g4 + e, 16 + 4 g4 + e - 4; the other operand is read from LDS in that order.
 // What a chunk brings is copied to LDS a chunk ahead, once for all columns; a chunk's outputs are stored in the next one, so
 // that the wait for the copies does not wait for stores just issued.
-// Bound by LDS reads (every wave reads the chunk's 73 KB) and the matrix pipes, about alike.  About 6.7 us a chunk on a
+// Bound by the chain of a chunk's products: with a workgroup on 55 % of the compute units LDS (every wave reads the chunk's 73
+// KB) is busy 28 % of the time of all of them, the matrix pipes 12 %, and the waves wait half of theirs.  About 6.7 us a chunk on a
 // compute unit, two waves on a SIMD; 4 workgroups of slices of 32 take 8.2.
 template <int D>
 __global__ __launch_bounds__(512) void delta_chunk_wide_kernel(hymeta_delta_rule_args a, int64_t chunks) {

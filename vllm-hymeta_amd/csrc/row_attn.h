@@ -12,20 +12,21 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return 
 
 constexpr float kLazyMax2 = 8.f;     // the softmax reference may trail a row's maximum by a factor of 2^8
 
-// Grid = the portions' blocks of 128 rows x slices of the keys at most x key/value heads; a row is a (query, head) pair, the heads of a key/value head side by
-// side: they share every key, so that a portion of a few tokens fills its blocks and a block's causal edge is one tile.
+// Grid = the portions' blocks of 128 rows x slices of the keys at most x key/value heads (fastest, so that workgroups without
+// rows come last); a row is a (query, head) pair, the heads of a key/value head side by side: they share every key, so that a
+// portion of a few tokens fills its blocks and a block's causal edge is one tile.
 // Sequences with one row are left to the decode form.
 //
 // Four waves of 32 rows, keys in tiles of 64 copied to two LDS images without passing registers, the values read transposed
 // from the rows as they lie; one barrier per tile; two workgroups on a compute unit, so that one's softmax runs under the
 // other's products.  v_mfma_f32_32x32x16 holds the issue port for a quarter of its time, the 16 x 16 form for half, and the
-// kernel needs the port for its scores (measured level, with less to read from LDS and fewer registers).  The scores are formed relative to the row's running reference, which moves
-// only when a score exceeds it by 2^8 (or at the row's first visible key): no maximum across lanes, no subtraction and no
-// pass over the output registers on most tiles.
-// Bound by the vector and the matrix pipe in turn: with a logarithm and an exponential per score they are busy 45 and 41 % of
+// kernel needs the port for its scores (measured level, with less to read from LDS and fewer registers).  The scores are
+// formed relative to the row's running reference, which moves only when a score exceeds it by 2^8 (or at the row's first
+// visible key): no maximum across lanes, no subtraction and no pass over the output registers on most tiles.
+// Bound by the vector and the matrix pipe in turn: with a logarithm and an exponential per score they are busy 56 and 43 % of
 // the time and hardly at once, whatever the number of waves (one row block a wave and four waves a SIMD: 785 us).  8192 rows x
-// 28 heads of 128 with 4 key/value heads, logarithmic bias: 1400 -> 765 us; a latent of 128 + 64: 1632 -> 760; a window of 1024:
-// 410 -> 214; key and value in one vector, window of 1024: 345 -> 219.
+// 28 heads of 128 with 4 key/value heads, logarithmic bias: 1398 -> 759 us; a latent of 128 + 64: 1629 -> 745; a window of 1024:
+// 406 -> 198; key and value in one vector, window of 1024: 357 -> 230; chunks of 2048: 414 -> 199.
 template <int D, int DV, int Layout>
 struct RowShape {
   static constexpr bool Scaled = Layout == HYMETA_KV_SCALED_KEY, Inside = Layout == HYMETA_KV_VALUE_IN_KEY || Scaled, Shared = Layout == HYMETA_KV_SHARED_KEY;

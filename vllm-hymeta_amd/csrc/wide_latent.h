@@ -91,16 +91,15 @@ struct WideSmem {
   int moved[2][kWideWaves];                       // whether a row block has any factor but 1
 };
 
-// Portions of prompts: grid = their blocks of 128 rows x slices of the keys at most x key/value heads; a row is a (query, head) pair, the heads of a
-// key/value head side by side, so that a portion of a few tokens fills its blocks.  Sequences with one row are left to the
-// decode form.
+// Portions of prompts: grid = their blocks of 128 rows x slices of the keys at most x key/value heads; a row is a (query, head)
+// pair, the heads of a key/value head side by side, so that a portion of a few tokens fills its blocks.  Sequences with one row
+// are left to the decode form.
 //
 // Per tile of 32 keys a workgroup issues 800 matrix instructions (C = 512) against 480 LDS reads of 1 KB; a step computes
 // the scores of tile t + 1 and adds tile t's values, which do not depend on each other: the two waves of a SIMD do them in
 // opposite order, so that one's softmax runs under the other's products.  One barrier per tile.  Bound by the matrix
-// pipe: 8192 rows x 16 heads on
-// 512 + 64: 1.65 ms = 1.04 PFLOP/s of the products issued (both parts of the weights counted), where launches over value
-// slices of 128, each repeating the scores, took 11.3 ms.
+// and the vector pipes, busy 43 and 39 % of the time: 8192 rows x 16 heads on 512 + 64: 1.61 ms = 1.07 PFLOP/s of the products
+// issued (both parts of the weights counted), where launches over value slices of 128, each repeating the scores, took 11.3 ms.
 template <int C>
 __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_sink_attention_args a, PortionSlices ps) {
   constexpr int D = C + 64, kRowB = 2 * D, kSteps = D / 32, CB = C / 128;
@@ -335,8 +334,8 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
 // The waves' sums are merged through LDS (a tree of two steps) into one partial per slice.  Two row blocks in a wave (28
 // heads) need 400 registers, of which 256 can be addressed by everything but the matrix instructions: the compiler spills
 // 460.  The head slices of a (sequence, slice of keys) follow each other on one die instead, whose L2 has the keys for the
-// second.  Bound by memory: 64 sequences x 4097 keys of 512 + 64, 16 heads: 57 us = 5.3 TB/s, where four
-// launches over value slices took 280.
+// second.  Bound by memory, and by what stands around a slice's few tiles (queries, first tile, merge): 64 sequences x 4096 keys
+// of 512 + 64, 16 heads: 69 us = 4.4 TB/s, where four launches over value slices took 280.
 constexpr int kLatentWaves = 4, kLatentKeys = 16, kLatentHeads = 16;
 
 template <int C>
