@@ -929,7 +929,8 @@ __device__ __forceinline__ PieceAt portion_block(const hymeta_sink_attention_arg
 constexpr int kWideKeys = 32;                  // a tile of the kernels over wide latents
 
 // grid = (sequences + rows where portions' keys were cut, heads): the rows of single-row sequences, and the rows of portions whose
-// blocks were cut.  One launch for both: a step of both takes no more launches than without slices.
+// blocks were cut.  One launch for both: a step of both takes no more launches than without slices.  A row's portion is found in
+// one round trip for 64 sequences (one read behind the other: 300 whole rows beside 63 single ones took 78.2 us, so 76.2).
 __global__ __launch_bounds__(kCombineThreads) void sink_attention_combine_kernel(hymeta_sink_attention_args a, int splits, HeadSlice hs, PortionSlices ps) {
   // (splits: partials per (sequence, key/value head): one per slice, or one per wave of a slice)
   const int group = a.num_heads / a.num_kv_heads, HG = hs.count ? hs.count : group;
@@ -942,9 +943,9 @@ __global__ __launch_bounds__(kCombineThreads) void sink_attention_combine_kernel
     combine_row(a, static_cast<const float*>(a.workspace) + (static_cast<size_t>(s) * a.num_kv_heads + g) * splits * stride + r * row, stride, splits, t, h);
     return;
   }
-  const int t = blockIdx.x - a.num_seqs, s = seq_of_row(a.query_start_loc, a.num_seqs, t), row0 = a.query_start_loc[s], end = a.query_start_loc[s + 1];
-  if (end - row0 <= 1 || t >= end) return;             // (rows behind the last portion have no partials)
-  const int ctx = a.seq_lens[s] - (end - row0), rows = (end - row0) * group, r0 = ((t - row0) * group + in_group) / kPortionRows * kPortionRows;
+  const PieceAt at = piece_at(a.query_start_loc, a.num_seqs, blockIdx.x - a.num_seqs, [](int q) { return q; });
+  if (at.seq < 0 || at.rows <= 1) return;              // (rows behind the last portion have no partials)
+  const int t = at.row0 + at.index, ctx = a.seq_lens[at.seq] - at.rows, rows = at.rows * group, r0 = (at.index * group + in_group) / kPortionRows * kPortionRows;
   const int p_first = ctx + r0 / group, p_hi = ctx + (min(rows, r0 + kPortionRows) - 1) / group;
   const int n = a.v_dim > 128 ? block_keys<kWideKeys>(a, p_first, p_hi).slices(ps) : block_keys<kTileKeys>(a, p_first, p_hi).slices(ps);
   if (n > 1) combine_row(a, ps.parts + (static_cast<size_t>(t) * a.num_heads + h) * ps.splits * row, row, n, t, h);
@@ -1019,11 +1020,11 @@ inline int64_t portion_blocks(int num_tokens, int num_seqs, int group, int max_q
 // so that blocks of fewer tiles stay whole.  7 rows x 28 heads behind 6000 keys: 299 -> 29 us; 40 rows x 28 heads on latents of
 // 512 + 64, twice: 592 -> 77; 300 rows on latents of 128 + 64, twice: 233 -> 101.
 //
-// Beside single rows, whose keys say nothing of the portion's, the merge's look at every row of the step (2 to 6 us) is lost on a
+// Beside single rows, whose keys say nothing of the portion's, the merge's look at every row of the step (1 to 3 us) is lost on a
 // portion that begins its sequence.  Up to kFewBlocks, where one behind many keys would have nothing but its own tiles to wait
 // for, it is worth it (with at most kMostNumbers numbers of blocks, most of which have none): 40 rows x 28 heads behind 6000
-// keys beside 63 single rows take 164 us where they took 417, with a window of 1024 57 where they took 85 (331 and 77 with a
-// workgroup per head); without keys in front of them 43 where they took 41.  Above, only where all numbers fit the chip.
+// keys beside 63 single rows take 161 us where they took 417 whole, with a window of 1024 54 where they took 85 (329 and 75 with
+// a workgroup per head); without keys in front of them 41 (38).  Above, only where all numbers fit the chip.
 constexpr int64_t kMostPartialBytes = 96 << 20, kFewBlocks = 32, kMostNumbers = 2048;
 inline int64_t portion_partial_bytes(int num_tokens, int num_heads, int v_dim) {
   return static_cast<int64_t>(num_tokens) * num_heads * static_cast<int64_t>(partial_row_floats(v_dim)) * 4;
