@@ -66,6 +66,11 @@ def reference(q, k, v, scale, ctx, o, sink, a, gate):
     ("scaled", 96, 96, 4, 2, 16, [33, 70], [100, 0], dict(bias="linear", window=50)),
     ("scaled", 64, 64, 4, 1, 64, [64], [64], dict(sink=True)),
     ("scaled", 32, 32, 3, 3, 64, [10, 11], [700, 0], dict(bias="linear")),
+    # single rows: as many partials as a thread of the merge holds, and one more; head groups that are not full
+    *[("rows", 64, 64, 10, 2, 64, [1, 0, 1, 1], [64 * n - 1, 5, 0, 70], dict(sink=True, gate=True, elem=True)) for n in (2, 3, 4, 5, 8, 9)],
+    ("rows", 64, 128, 3, 1, 64, [1, 1], [63, -1], {}),
+    ("latent", 192, 128, 37, 1, 64, [1, 1], [127, 3], dict(sink=True, elem=True)),
+    ("scaled", 96, 96, 7, 7, 64, [1, 1], [200, 3], dict(sink=True, bias="linear")),
 ])
 def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
     from vllm_hymeta import hip_ops

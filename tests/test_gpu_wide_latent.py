@@ -48,6 +48,7 @@ def reference(q, rows, C, scale, sink, window, keep, chunk, softcap, bias, gate,
     (512, 16, 64, [9, 1, 3, 1], [2500, 700, 5, 64], dict(window=1600, keep=40, gate=True, sink=True)),
     (256, 40, 16, [1, 5, 1], [900, 1400, 31], dict(chunk=700, gate=True)),
     (256, 33, 64, [1] * 5, [0, 15, 16, 1000, 63], dict(sink=True, window=33)),
+    *[(c, 16, 64, [1, 1], [64 * n - 1, 20], dict(sink=True, gate=True)) for c, n in ((384, 2), (512, 3), (256, 8), (512, 9))],      # partials of a row
 ])
 def test_against_64_bits(C, H, page, lens, ctxs, opts):
     from vllm_hymeta import hip_ops

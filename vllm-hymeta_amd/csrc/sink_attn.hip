@@ -834,10 +834,28 @@ __global__ __launch_bounds__(64 * kDecodeWaves) void sink_attention_decode_mfma_
 // Merge a row's partials (`splits` of them, `stride` floats apart from `base` on), add the sink, normalise, store bf16: one
 // workgroup per (row, head).  Two round trips to memory: the threads read the partials' statistics side by side (one each),
 // agree on the row's maximum, and leave every partial's factor in LDS; then groups of v_dim / 4 threads take the partials
-// in turn, four columns a thread.  (As one serial loop over the partials per column and statistic the launch took 11 us at
-// 4 partials of 128 columns of 64 x 16 rows; now 6 at 4 partials of 512.)
+// in turn, four columns a thread.  (One serial loop over the partials per column and statistic: 3 rows of 28 heads with 20
+// partials of 128 columns 25.7 us with the kernel in front of it, so 21.3.)
 constexpr int kCombineThreads = 128;
 constexpr int kMaxPartials = 512 * kDecodeWaves;
+// Up to as many partials a (row, head) goes to the kernel that holds them all in registers: more partials are for few rows, which
+// leave the chip room for a workgroup each.
+constexpr int kFewPartials = 8;
+
+// Columns c .. c + 3 of row t's head h, from the weighted values and the weights' sum.
+__device__ __forceinline__ void store_row(const hymeta_sink_attention_args& a, f32x4v acc, float l, int64_t t, int h, int c) {
+  float inv = l > 0.f ? 1.f / l : 0.f;
+  if (a.head_gate) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[t * a.head_gate_stride_t + h]));
+  acc *= inv;
+  if (a.elem_gate) {
+    float gate[4];
+    ActBf16::ld4(static_cast<const uint16_t*>(a.elem_gate) + t * a.elem_gate_stride_t + static_cast<int64_t>(h) * a.v_dim + c, gate);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] *= ActBf16::sigmoid(gate[e]);
+  }
+  *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.out) + (t * a.num_heads + h) * a.v_dim + c) =
+      u32x2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
+}
 
 __device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a, const float* base, size_t stride, int splits, int64_t t, int h) {
   __shared__ float s_f[kMaxPartials];
@@ -881,18 +899,7 @@ __device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a,
     if (turn == 0)
       for (int k = 1; k < turns; ++k) acc += s_acc[tid + k * quads];
   }
-  if (turn != 0) return;
-  float inv = l > 0.f ? 1.f / l : 0.f;
-  if (a.head_gate) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[t * a.head_gate_stride_t + h]));
-  acc *= inv;
-  if (a.elem_gate) {
-    float gate[4];
-    ActBf16::ld4(static_cast<const uint16_t*>(a.elem_gate) + t * a.elem_gate_stride_t + static_cast<int64_t>(h) * DV + c, gate);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] *= ActBf16::sigmoid(gate[e]);
-  }
-  *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.out) + (t * a.num_heads + h) * DV + c) =
-      u32x2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
+  if (turn == 0) store_row(a, acc, l, t, h, c);
 }
 
 // How the keys of portions are cut: into `splits` slices at most, whose partials lie at `parts`, [row][head][splits]; blocks of
@@ -949,6 +956,45 @@ __global__ __launch_bounds__(kCombineThreads) void sink_attention_combine_kernel
   const int p_first = ctx + r0 / group, p_hi = ctx + (min(rows, r0 + kPortionRows) - 1) / group;
   const int n = a.v_dim > 128 ? block_keys<kWideKeys>(a, p_first, p_hi).slices(ps) : block_keys<kTileKeys>(a, p_first, p_hi).slices(ps);
   if (n > 1) combine_row(a, ps.parts + (static_cast<size_t>(t) * a.num_heads + h) * ps.splits * row, row, n, t, h);
+}
+
+// The same for single rows of at most N partials where no portion's keys were cut: every thread reads all of its four columns'
+// partials and their statistics at once, v_dim / 4 threads to a (row, head), as many heads as fit in a workgroup; no LDS, no
+// barriers.  grid = (sequences, head groups).  A workgroup per (row, head) needs four round trips and two barriers for them, and
+// more than 3840 of them (LDS) are not on the chip at once.  28 heads of 128 with the kernel in front, a workgroup each -> so (and
+// with the serial loop), us: 236 rows at 79 keys 27.4 -> 23.1 (24.9), 256 at 1024 111.0 -> 105.3 (108.5), 64 at 4096 101.6 ->
+// 99.9 (102.1), 16 at 4096 (8 partials) 30.5 -> 29.2 (36.1); 64 x 16 heads of 512 at 4096 70.9 -> 69.8.
+template <int N>
+__global__ __launch_bounds__(kCombineThreads) void sink_attention_combine_few_kernel(hymeta_sink_attention_args a, int splits, HeadSlice hs) {
+  const int s = blockIdx.x, t = a.query_start_loc[s];
+  const int group = a.num_heads / a.num_kv_heads, HG = hs.count ? hs.count : group, DV = a.v_dim;
+  const int quads = DV / 4, each = kCombineThreads / quads, at = blockIdx.y * each + threadIdx.x / quads, c = 4 * (threadIdx.x % quads);
+  if (a.query_start_loc[s + 1] - t != 1 || threadIdx.x >= each * quads || at >= HG * a.num_kv_heads) return;
+  const int g = at / HG, r = at % HG, h = g * group + hs.first + r;
+  const size_t row = partial_row_floats(DV), stride = HG * row;
+  const float* base = static_cast<const float*>(a.workspace) + (static_cast<size_t>(s) * a.num_kv_heads + g) * splits * stride + r * row;
+  f32x4v x[N];
+  float2 stat[N];                                      // a partial's maximum (base-2 domain) and denominator
+#pragma unroll
+  for (int sp = 0; sp < N; ++sp) {                     // (past the last one: read again)
+    const float* part = base + min(sp, splits - 1) * stride;
+    stat[sp] = *reinterpret_cast<const float2*>(part + DV);
+    x[sp] = *reinterpret_cast<const f32x4v*>(part + c);
+  }
+  const float sink2 = a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f;
+  float m = a.sink ? sink2 : -INFINITY;
+#pragma unroll
+  for (int sp = 0; sp < N; ++sp) m = fmaxf(m, stat[sp].x);
+  float l = a.sink ? __builtin_amdgcn_exp2f(sink2 - m) : 0.f;
+  f32x4v acc = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int sp = 0; sp < N; ++sp)
+    if (sp < splits && stat[sp].x != -INFINITY) {      // (a partial without keys)
+      const float f = __builtin_amdgcn_exp2f(stat[sp].x - m);
+      l = fmaf(stat[sp].y, f, l);
+      acc += x[sp] * f;
+    }
+  store_row(a, acc, l, t, h, c);
 }
 
 }  // namespace
@@ -1057,7 +1103,16 @@ inline dim3 portion_grid(const hymeta_sink_attention_args& a, const PortionSlice
   return dim3(static_cast<uint32_t>(portion_blocks(a.num_tokens, a.num_seqs, a.num_heads / a.num_kv_heads, a.max_query_len) * ps.splits * a.num_kv_heads));
 }
 void launch_combine(const hymeta_sink_attention_args& a, hipStream_t st, int splits, HeadSlice hs, const PortionSlices& ps) {
-  const dim3 grid(a.num_seqs + (ps.splits > 1 ? a.num_tokens : 0), hs.count ? hs.count * a.num_kv_heads : a.num_heads);
+  const int heads = hs.count ? hs.count * a.num_kv_heads : a.num_heads;
+  if (ps.splits == 1 && splits <= kFewPartials) {
+    const int each = kCombineThreads / (a.v_dim / 4);
+    const dim3 grid(a.num_seqs, (heads + each - 1) / each);
+    if (splits <= 2) hipLaunchKernelGGL(sink_attention_combine_few_kernel<2>, grid, dim3(kCombineThreads), 0, st, a, splits, hs);
+    else if (splits <= 4) hipLaunchKernelGGL(sink_attention_combine_few_kernel<4>, grid, dim3(kCombineThreads), 0, st, a, splits, hs);
+    else hipLaunchKernelGGL(sink_attention_combine_few_kernel<kFewPartials>, grid, dim3(kCombineThreads), 0, st, a, splits, hs);
+    return;
+  }
+  const dim3 grid(a.num_seqs + (ps.splits > 1 ? a.num_tokens : 0), heads);
   hipLaunchKernelGGL(sink_attention_combine_kernel, grid, dim3(kCombineThreads), 0, st, a, splits, hs, ps);
 }
 
