@@ -1235,9 +1235,10 @@ extern "C" size_t hymeta_sink_attention_workspace_bytes(int32_t num_seqs, int32_
 extern "C" size_t hymeta_sink_attention_portion_workspace_bytes(int32_t num_tokens, int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads,
                                                                 int32_t v_dim, int32_t max_query_len, int32_t max_seq_len, int64_t span,
                                                                 int32_t keep_first) {
-  if (num_tokens <= 0 || num_seqs <= 0 || num_heads <= 0 || num_kv_heads <= 0 || v_dim <= 0 || max_query_len <= 1 || max_seq_len < 1) return 0;
+  const size_t single = hymeta_sink_attention_workspace_bytes(num_seqs, num_heads, num_kv_heads, v_dim, max_seq_len);
+  if (num_tokens <= 0 || single == 0 || max_query_len <= 1 || max_seq_len < 1) return single;
   const int splits = portion_slices(num_tokens, num_seqs, num_heads, num_kv_heads, v_dim, max_query_len, decode_tiles(max_seq_len, span, keep_first)).splits;
-  return splits > 1 ? static_cast<size_t>(decode_partial_bytes(num_seqs, num_heads, num_kv_heads, v_dim, max_seq_len) + splits * portion_partial_bytes(num_tokens, num_heads, v_dim)) : 0;
+  return single + (splits > 1 ? static_cast<size_t>(splits * portion_partial_bytes(num_tokens, num_heads, v_dim)) : 0);
 }
 
 extern "C" int hymeta_sink_attention(const hymeta_sink_attention_args* args, hymeta_stream_t stream) {
