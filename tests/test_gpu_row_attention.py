@@ -1,6 +1,6 @@
 """Prompts' portions of the paged attention, keys of 32 to 192 elements in every layout of a cache row, at the edges of the
 kernel's tiles: 32 (query, head) rows a wave and 128 a workgroup, 64 keys a tile, pages that hold a tile and pages that do not,
-and portions short enough that their keys are cut into slices (more than 4 tiles a slice).
+and portions short enough that their keys are cut into slices (2 tiles a slice or more).
 
 Bound: the outputs are bf16 (2^-9 of each value at most); the weights are two bf16 parts (2^-17), exponentials, logarithms and
 products fp32 (below 2^-11 over these lengths and biases); together below 2^-9 + 2^-10 in the norm."""
@@ -66,6 +66,8 @@ def reference(q, k, v, scale, ctx, o, sink, a, gate):
     ("scaled", 96, 96, 4, 2, 16, [33, 70], [100, 0], dict(bias="linear", window=50)),
     ("scaled", 64, 64, 4, 1, 64, [64], [64], dict(sink=True)),
     ("scaled", 32, 32, 3, 3, 64, [10, 11], [700, 0], dict(bias="linear")),
+    # the shortest keys that are cut: 3, 4 and 5 tiles
+    *[("rows", 128, 128, 8, 2, 64, [8, 2], [c, 63], dict(sink=True, gate=True)) for c in (184, 185, 248, 249)],
     # single rows: as many partials as a thread of the merge holds, and one more; head groups that are not full
     *[("rows", 64, 64, 10, 2, 64, [1, 0, 1, 1], [64 * n - 1, 5, 0, 70], dict(sink=True, gate=True, elem=True)) for n in (2, 3, 4, 5, 8, 9)],
     ("rows", 64, 128, 3, 1, 64, [1, 1], [63, -1], {}),

@@ -904,8 +904,9 @@ __device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a,
 
 // How the keys of portions are cut: into `splits` slices at most, whose partials lie at `parts`, [row][head][splits]; blocks of
 // up to `whole` tiles of 64 keys are not cut.
+constexpr int kLeastTiles = 2;                 // of a slice
 struct PortionSlices {
-  int splits = 1, whole = 0, least = 0;           // (least: the keys of a slice at least)
+  int splits = 1, whole = 0;
   float* parts = nullptr;
 };
 constexpr int kPortionRows = 128;              // (query, head) rows of a block, the heads of a key/value head side by side
@@ -916,7 +917,7 @@ struct BlockKeys {
   int from, kept, tiles, size;
   __device__ __forceinline__ int first(int t) const { return t < kept ? t * size : from + (t - kept) * size; }
   __device__ __forceinline__ int slices(const PortionSlices& ps) const {
-    return tiles * size <= ps.whole * kTileKeys ? 1 : max(1, min(ps.splits, tiles * size / ps.least));
+    return tiles * size <= ps.whole * kTileKeys ? 1 : max(1, min(ps.splits, tiles * size / (kLeastTiles * kTileKeys)));
   }
 };
 template <int Keys>
@@ -1063,13 +1064,15 @@ inline int64_t portion_blocks(int num_tokens, int num_seqs, int group, int max_q
 // Slices a portion's keys are cut into: where the blocks that the step's portions are worth (long_portions) do not fill the chip
 // (`target` workgroups) and the workspace has room for the partials (bounded: every row of the step has a place).  A slice's
 // queries, its first tile and its partial cost about two tiles of 64 keys, and a (row, head) of the merge about 1 / 768 of one,
-// so that blocks of fewer tiles stay whole.  7 rows x 28 heads behind 6000 keys: 299 -> 29 us; 40 rows x 28 heads on latents of
-// 512 + 64, twice: 592 -> 77; 300 rows on latents of 128 + 64, twice: 233 -> 101.
+// so that blocks of fewer tiles stay whole.  7 rows x 28 heads behind 6000 keys: 299 -> 25 us; 40 rows x 28 heads on latents of
+// 512 + 64, twice: 592 -> 77; 300 rows on latents of 128 + 64, twice: 233 -> 101.  Slices of two tiles and more: of four, 64 rows
+// x 28 heads behind 400 keys took 29.0 us (26.0 with a workgroup per head), three times 40 28.3 (24.5), 8 behind 650 27.4 (30.6);
+// of two 23.4, 24.9 and 23.9, at which the host's call stands; of three between them.
 //
 // Beside single rows, whose keys say nothing of the portion's, the merge's look at every row of the step (1 to 3 us) is lost on a
 // portion that begins its sequence.  Up to kFewBlocks, where one behind many keys would have nothing but its own tiles to wait
 // for, it is worth it (with at most kMostNumbers numbers of blocks, most of which have none): 40 rows x 28 heads behind 6000
-// keys beside 63 single rows take 161 us where they took 417 whole, with a window of 1024 54 where they took 85 (329 and 75 with
+// keys beside 63 single rows take 161 us where they took 417 whole, with a window of 1024 47 where they took 85 (329 and 75 with
 // a workgroup per head); without keys in front of them 41 (38).  Above, only where all numbers fit the chip.
 constexpr int64_t kMostPartialBytes = 96 << 20, kFewBlocks = 32, kMostNumbers = 2048;
 inline int64_t portion_partial_bytes(int num_tokens, int num_heads, int v_dim) {
@@ -1077,13 +1080,12 @@ inline int64_t portion_partial_bytes(int num_tokens, int num_heads, int v_dim) {
 }
 inline PortionSlices portion_slices(int num_tokens, int num_seqs, int num_heads, int num_kv_heads, int v_dim, int max_query_len, int tiles) {
   PortionSlices ps;
-  ps.least = (v_dim > 128 ? 2 : 4) * kTileKeys;        // (a tile of a wide latent takes four times as long)
   const int group = std::max(1, num_heads / num_kv_heads), target = v_dim > 128 ? 256 : 512;       // one workgroup on a compute unit (wide_latent.h), or two
   const int64_t each = (static_cast<int64_t>(max_query_len) * group + kPortionRows - 1) / kPortionRows, portions = long_portions(num_tokens, num_seqs, max_query_len);
   const int64_t blocks = each * portions * num_kv_heads;
-  int64_t most = std::min<int64_t>(tiles / (ps.least / kTileKeys), kMostPartialBytes / portion_partial_bytes(num_tokens, num_heads, v_dim));
+  int64_t most = std::min<int64_t>(tiles / kLeastTiles, kMostPartialBytes / portion_partial_bytes(num_tokens, num_heads, v_dim));
   if (num_seqs > portions) most = std::min<int64_t>(most, (blocks > kFewBlocks ? target : kMostNumbers) / (portion_blocks(num_tokens, num_seqs, group, max_query_len) * num_kv_heads));
-  ps.whole = static_cast<int>(std::min<int64_t>(tiles, std::max<int64_t>(2 * ps.least / kTileKeys - 1, portions * max_query_len * num_heads / 768)));
+  ps.whole = static_cast<int>(std::min<int64_t>(tiles, std::max<int64_t>(2 * kLeastTiles - 1, portions * max_query_len * num_heads / 768)));
   if (tiles > ps.whole) ps.splits = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(target / blocks, most)));
   // (an odd stride: the first slices alone, where blocks stay whole, are on all of the chip's 8 dies)
   if (num_seqs > portions && blocks <= kFewBlocks && ps.splits > 2) ps.splits -= 1 - ps.splits % 2;
