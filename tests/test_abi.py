@@ -156,3 +156,15 @@ def test_scan_workspace_covers_smaller_steps(name):
         assert all(a <= b for row in by_seqs for a, b in zip(row, row[1:]))
         assert all(a <= b for col in zip(*by_seqs) for a, b in zip(col, col[1:]))
         assert by_seqs[0][-1] == 0 and by_seqs[4][3] > 0
+
+
+def test_attention_workspace_with_slices_holds_the_single_rows():
+    """One question covers a step: room for slices comes on top of the room that single rows take."""
+    from vllm_hymeta import _C
+
+    lib = _C.load()
+    single, both = lib.hymeta_sink_attention_workspace_bytes, lib.hymeta_sink_attention_portion_workspace_bytes
+    for tokens, seqs, rows, keys in ((64, 64, 1, 4096), (103, 64, 40, 6040), (8192, 1, 8192, 8192), (2, 1, 2, 2), (0, 3, 5, 100)):
+        for v_dim in (64, 512):
+            assert both(tokens, seqs, 28, 4, v_dim, rows, keys, 0, 0) >= single(seqs, 28, 4, v_dim, keys) > 0
+    assert both(7, 1, 28, 4, 128, 7, 6007, 0, 0) > single(1, 28, 4, 128, 6007)
