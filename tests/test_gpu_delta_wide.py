@@ -14,7 +14,8 @@ EDGES = [8, 63, 64, 65, 130, 7, 128, 129, 20, 1, 130, 97, 126, 127, 128]        
 
 @pytest.mark.parametrize("D,Dv,H,Hk,lens", [
     (32, 128, 16, 4, EDGES), (64, 256, 8, 8, EDGES), (96, 128, 16, 16, EDGES), (128, 128, 16, 8, EDGES),
-    (128, 128, 16, 8, [1] * 20 + [300] + [1] * 12 + [9, 130]), (96, 128, 12, 12, [1] * 20 + [300] + [1] * 12 + [9, 130])])
+    (128, 128, 16, 8, [1] * 20 + [300] + [1] * 12 + [9, 130]), (96, 128, 12, 12, [1] * 20 + [300] + [1] * 12 + [9, 130]),
+    (128, 128, 16, 8, [1] * 60 + [300] + [1] * 30)])
 def test_wide_slices_equal_narrow_ones(D, Dv, H, Hk, lens):
     """Both multiply the same operands (fp32 as two bf16 parts, 2^-17 of the operand) and add in another order: 1e-5 of the
     norm covers what that rounding grows to over a few chunks.  Rows at a chunk's edges, several chunks, a portion that goes

@@ -196,8 +196,12 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(hymeta_delta_rule_
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 constexpr int kChunk = HYMETA_DELTA_CHUNK;
 // Workgroups (with slices of 32 value columns) up to which the second launch runs slices of 16: measured for one prompt of 8192
-// with 28 heads of 128 x 128 (112 workgroups) 357 against 405 us, with 64 heads (256) 706 against 566 us.
-constexpr int kFewGroups = 128;
+// with 28 heads of 128 x 128 (112 workgroups) 357 against 405 us, with 64 heads (256) 706 against 566 us.  They also double the
+// workgroups of the sequences without a chunk, which end at once but take about 0.65 ns each to come and go, and save about 0.55
+// us a chunk of 64 rows: not where those are more than 10 per row of the longest portion.  28 heads, slices of 16 and of 32, us:
+// 100 rows beside 63 single ones 52.1 and 49.1, 400 beside 63 72.1 and 67.2, 700 beside 63 78.4 and 76.3, 2048 beside 63 122 and
+// 133, 1000 beside 200 170 and 157, 2048 beside 255 246 and 222.
+constexpr int kFewGroups = 128, kIdleGroupsPerRow = 10;
 // Workgroups of slices of 128 columns above which the second launch takes those: slices of 32 are then more than the 512
 // workgroups that run at the same time.  With 28 heads of 128 x 128 (16 for the last two): 5 portions of 1801 rows 310 us in
 // narrow slices, 281 in wide ones (140 workgroups); 16 of 500 250 and 191; 40 of 300 414 and 276; 8 of 700 (128) 102 and 108.
@@ -831,9 +835,10 @@ void launch_chunks(const hymeta_delta_rule_args& a, hipStream_t st, int64_t chun
   hipLaunchKernelGGL(delta_chunk_solve_kernel<D>, dim3(static_cast<unsigned>(chunks), a.num_heads), dim3(256), 0, st, a, chunks);
   // slices of 32 columns reread a chunk's matrices half as often; slices of 16 double the workgroups where they are few.  Few
   // and many of those that have work for the time the longest takes: single rows and short portions end at once or soon
-  const int64_t lanes = a.num_heads * long_portions(a.num_tokens, a.num_seqs, a.max_query_len);
+  const int64_t portions = long_portions(a.num_tokens, a.num_seqs, a.max_query_len), lanes = a.num_heads * portions;
+  const int64_t idle = a.num_heads * (a.num_seqs - portions) * (a.v_dim / 32);
   if constexpr (D % 64 == 0) {
-    if (lanes * (a.v_dim / 32) <= kFewGroups) {
+    if (lanes * (a.v_dim / 32) <= kFewGroups && idle <= static_cast<int64_t>(kIdleGroupsPerRow) * a.max_query_len) {
       hipLaunchKernelGGL((delta_chunk_scan_kernel<D, 1>), dim3(a.num_heads, a.num_seqs, a.v_dim / 16), dim3(256), 0, st, a, chunks);
       return;
     }
