@@ -1,27 +1,37 @@
 // Varlen prefill attention: causal sliding window over the real keys plus an
 // always-visible block of meta keys, one softmax (flash-attention forward).
 //
-// MFMA-bound.  A 512-thread workgroup owns 256 consecutive queries of one
-// (sequence, q-head); each of its 8 waves owns 32 of them as two 16-row MFMA
-// tiles.  The workgroup walks the visible keys in tiles of 64: all threads
-// stage the tile's K and V rows once (global -> registers one tile ahead,
-// registers -> LDS right after the barrier that frees the buffer, one barrier
-// per tile, two LDS buffers), and every wave reads its operands from that
-// shared image:
-//   S^T = K Q^T   A = 16 key rows x 32 channels, ds_read_b128 from the K image
-//                 (256-byte rows, 16-byte chunks XOR-ed with the row so the
-//                 sixteen rows of a read hit distinct banks);
-//                 B = the wave's resident Q fragments.
-//   O  += P V     A = the S^T accumulators re-packed to bf16: the query is on
-//                 the lane and the keys are in registers, which is the
-//                 A-operand layout up to a fixed permutation of the key slots;
-//                 B = V in the same permuted key order, two transposed 8-byte
-//                 LDS reads (ds_read_b64_tr_b16) per fragment from the V image
-//                 (288-byte rows: the four rows of a read sit 8 banks apart).
+// A workgroup owns 128 (query, head) rows of one (sequence, kv-head): the
+// query heads of a kv-head lie side by side, so that they share every key and
+// a chunk of a few queries still fills its waves.  Each wave owns 32 rows; the
+// keys are walked in tiles of 64, copied straight into LDS images (256-byte
+// rows, 16-byte chunks permuted within the row).  Two workgroups run on a
+// compute unit, in steps of their own.
+//
+// A wave's step is a software pipeline over three tiles: the products of the
+// scores of tile t + 1 (S^T = K Q^T) and of the output of tile t - 1 (O^T +=
+// V^T P^T), with the exponentials of tile t and the maximum of tile t + 1
+// placed between them, so that the matrix pipe runs under the wave's own vector
+// work.  S^T leaves row n's scores of 32 of the 64 keys on lane n and the
+// others on lane n + 32; packed to bf16 they are the second product's operand
+// as they lie, the values being read transposed (ds_read_b64_tr_b16) in the
+// same order of keys.
+//
+// Bound by the matrix pipe and its clock: with nothing but the products left in
+// the loop, one prompt of 8192 x 28 heads (4 kv-heads, window 4097) takes 263 us,
+// with everything 359 (1.0 PFLOP/s); copies cost 6 %, barriers and the look at
+// the reference 3 % each.  Against a workgroup per head with operands through
+// registers, one tile at a time: 647 -> 359 us here, a chunk of 2048 at 32k of
+// 7 heads on one kv-head 368 -> 248, one prompt of 32768 (window 4097) 1968 ->
+// 1709, eight of 4096 1739 -> 962, four chunks of 5 tokens behind 7922 65 -> 26.
+// Eight waves to a workgroup, which read the keys half as often: level at
+// prompts of 8192 and more, 3 to 20 % slower below and with few heads.  The
+// step's scalar work counts as much as its vector work (twice as many scalar
+// instructions and branches per tile: 415 us): what a tile needs is worked out
+// in front of the loop.
 // Keys are read through a block table (chunked / prefix prefill) or from the
-// packed [token, kv-head, dim] tensor of the step.  Outputs are normalised,
-// staged through LDS and stored as whole 256-byte rows.
-#include "common.h"
+// packed [token, kv-head, dim] tensor of the step.
+#include "lds_copy.h"
 
 namespace hymeta {
 namespace {
@@ -29,28 +39,20 @@ namespace {
 constexpr int kTile = 32;            // granularity required of the meta-key count
 constexpr int kTileK = 64;           // keys per step
 constexpr int kRowsPerWave = 32;
-constexpr int kMaxWaves = 8;
-constexpr int kKPitch = 256;
-constexpr int kVPitch = 288;
-constexpr int kKBytes = kTileK * kKPitch;
-constexpr int kVBytes = kTileK * kVPitch;
-constexpr int kOPitch = 272;         // output staging rows (bf16 x 128 + pad)
+constexpr int kWaves = 4, kRows = kRowsPerWave * kWaves;
+constexpr int kCopies = 16 / kWaves;  // copies of 4 rows a wave makes per image
+constexpr int kPitch = 2 * kHeadDim;
+constexpr int kImage = kTileK * kPitch;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazyLog2 = 8.f;     // the softmax reference may trail the true row maximum by a factor 2^8
 
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
-struct Smem {
-  char k[2][kKBytes];
-  char v[2][kVBytes];
-};
-static_assert(sizeof(Smem) >= kMaxWaves * kRowsPerWave * kOPitch, "output staging aliases the K/V images");
-
-__device__ __forceinline__ f32x4 mfma16(const bf16x8& a, const bf16x8& b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+__device__ __forceinline__ f32x16 mfma32(const u32x4& a, const u32x4& b, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
-__device__ __forceinline__ bf16x8 as_frag(const u32x4& v) { return __builtin_bit_cast(bf16x8, v); }
 
 // max of three as ONE instruction: v_maximum3_f32 (NaN-propagating, so the compiler adds no
 // canonicalising v_max per MFMA output as it does for fmaxf, and no wait states as after inline asm).
@@ -59,54 +61,60 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
 }
 
 // 4 keys x 16 dims block read column-major: lane i of a 16-lane group gets dim i of the 4 keys.
-__device__ __forceinline__ s16x4 tr_read(const char* p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
+__device__ __forceinline__ u32x2 tr_read(const char* p) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p)));
 }
+
+// Sum of a packed bf16 pair and c, in fp32.
+__device__ __forceinline__ float add_pair(uint32_t pair, float c) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, 0x3f803f80u), c, false);
+}
+
+// 16-byte chunks of a row are permuted so that the rows of one fragment read hit distinct banks: a key read asks for one chunk
+// of 16 rows, a transposed value read for four neighbouring chunks of four rows.
+__device__ __forceinline__ int key_twist(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+__device__ __forceinline__ int value_twist(int row) { return (row & 3) << 2; }
+
+// A quotient of wave-uniform values as one: the division runs on the vector unit, and what follows from it would stay there.
+__device__ __forceinline__ int quotient(int a, int b) { return __builtin_amdgcn_readfirstlane(a / b); }
 
 }  // namespace
 
-// grid = (ceil(max_seqlen_q / (32 NW)), num_seqs (+1: the meta-query rows), num_heads); NW waves of
-// 32 queries per workgroup: 8 by default, 4 when that leaves compute units without a workgroup.
+// grid = (blocks of 128 rows x key slices x kv-heads (fastest), num_seqs (+1: the meta-query rows)).
 //
-// splits > 1 (few workgroups, long key ranges: a short chunk of a long sequence): blockIdx.x also
-// numbers the key slice; a workgroup walks only its share of the tiles and leaves an un-normalised
-// partial (fp32 O, the reference exponent and the row sum per query) in the workspace; a second
-// launch merges the slices in slice order.
-template <bool PAGED, int NW>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void swa_prefill_kernel(hymeta_swa_prefill_args a, float scale_log2, int splits,
-                                                                      int64_t part_rows) {
-  constexpr int kRowsPerBlock = kRowsPerWave * NW;
-  constexpr int kPasses = 16 / NW;     // staging passes: 4 NW key rows of a 64-key tile per pass
+// splits > 1 (few workgroups, long key ranges: a short chunk of a long sequence): a workgroup walks
+// only its share of the tiles and leaves an un-normalised partial (fp32 O, the reference exponent
+// and the row sum per row) in the workspace; a second launch merges the slices in slice order.
+template <bool PAGED>
+__global__ __launch_bounds__(64 * kWaves, 2) void swa_prefill_kernel(hymeta_swa_prefill_args a, float scale_log2, int splits,
+                                                                 int64_t part_rows) {
+  __shared__ __attribute__((aligned(16))) char s_k[2][kImage];
+  __shared__ __attribute__((aligned(16))) char s_v[2][kImage];
 
-  __shared__ __attribute__((aligned(16))) Smem sm;
-
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int c = lane >> 4;
-  const int n = lane & 15;
-
+  const int lane = threadIdx.x & 63, n = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int seq = blockIdx.y;
-  const int h = blockIdx.z;
-  const int kvh = h / (a.num_heads / a.num_kv_heads);
+  const int group = quotient(a.num_heads, a.num_kv_heads);
+  const int item = quotient(blockIdx.x, a.num_kv_heads), kvh = blockIdx.x - item * a.num_kv_heads;
+  const int block = quotient(item, splits), split = item - block * splits;
   const bool meta_rows = seq == a.num_seqs;  // this workgroup computes the meta-query rows
   const int M = a.meta_key != nullptr ? a.num_meta : 0;
   const int meta_tiles = (M + kTileK - 1) / kTileK;
   const int out_row0 = a.meta_query != nullptr ? a.num_meta : 0;
 
-  int Lq, Lk, q_first;        // query count, key count, first query row of the sequence
+  int Lq, Lk;                 // query count, key count
   const uint16_t* qbase;
-  int64_t q_stride_t;
+  int64_t q_stride_t, q_stride_h;
   int64_t out_first;          // output row of the sequence's first query
   int64_t k_first = 0;        // un-paged: first key row of the sequence
   if (meta_rows) {
     Lq = a.num_meta;
     Lk = 0;
-    qbase = reinterpret_cast<const uint16_t*>(a.meta_query) + static_cast<int64_t>(h) * a.meta_q_stride_h;
-    q_stride_t = a.meta_q_stride_t;
+    qbase = static_cast<const uint16_t*>(a.meta_query);
+    q_stride_t = a.meta_q_stride_t, q_stride_h = a.meta_q_stride_h;
     out_first = 0;
   } else {
-    q_first = a.cu_seqlens_q[seq];
+    const int q_first = a.cu_seqlens_q[seq];
     Lq = a.cu_seqlens_q[seq + 1] - q_first;
     if constexpr (PAGED) {
       Lk = a.seq_lens_k[seq];
@@ -114,375 +122,330 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void swa_prefill_kernel(hymeta_swa
       k_first = a.cu_seqlens_k[seq];
       Lk = a.cu_seqlens_k[seq + 1] - static_cast<int>(k_first);
     }
-    qbase = reinterpret_cast<const uint16_t*>(a.q) + static_cast<int64_t>(q_first) * a.q_stride_t + static_cast<int64_t>(h) * a.q_stride_h;
-    q_stride_t = a.q_stride_t;
+    qbase = static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(q_first) * a.q_stride_t;
+    q_stride_t = a.q_stride_t, q_stride_h = a.q_stride_h;
     out_first = out_row0 + q_first;
   }
-  const int split = splits > 1 ? blockIdx.x % splits : 0;
-  const int blk0 = (splits > 1 ? blockIdx.x / splits : blockIdx.x) * kRowsPerBlock;
-  if (blk0 >= Lq) return;                      // workgroup-uniform
-  const int row0 = blk0 + wave * kRowsPerWave;  // first query of this wave
-  const bool active = row0 < Lq;               // idle waves still stage tiles and meet the barriers
-  const int pos_shift = Lk - Lq;  // query r sits at key position r + pos_shift (bottom-right aligned)
+  const int rows = Lq * group;
+  const int r0 = ((rows + kRows - 1) / kRows - 1 - block) * kRows;   // the blocks with the most keys first
+  if (r0 < 0) return;                        // workgroup-uniform
+  const int w0 = r0 + wave * kRowsPerWave;   // first row of this wave
+  const bool active = w0 < rows;             // idle waves still copy tiles and meet the barriers
+  const int pos_shift = Lk - Lq;             // query i sits at key position i + pos_shift (bottom-right aligned)
 
-  // Q fragments: qf[qt][ks] = Q[row0 + 16qt + n][32ks + 8c .. +7]
-  bf16x8 qf[2][4];
+  // this lane's row
+  const int r = w0 + n;
+  const bool ok = r < rows;
+  const int qi = ok ? r / group : 0, h = kvh * group + (ok ? r - qi * group : 0);
+  u32x4 qf[8];
+  {
+    const uint16_t* qrow = qbase + static_cast<int64_t>(qi) * q_stride_t + static_cast<int64_t>(h) * q_stride_h + 8 * hh;
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
-    const int r = row0 + 16 * qt + n;
-    const uint16_t* qp = qbase + static_cast<int64_t>(r) * q_stride_t + 8 * c;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      u32x4 raw = {0u, 0u, 0u, 0u};
-      if (r < Lq) raw = ld16(qp + 32 * ks);
-      qf[qt][ks] = as_frag(raw);
+    for (int st = 0; st < 8; ++st) {
+      qf[st] = u32x4{0u, 0u, 0u, 0u};
+      if (ok) qf[st] = ld16g(qrow + 16 * st);
     }
   }
 
-  f32x4 o[2][8];
-#pragma unroll
-  for (int qt = 0; qt < 2; ++qt)
-#pragma unroll
-    for (int t = 0; t < 8; ++t) o[qt][t] = {0.f, 0.f, 0.f, 0.f};
-  float m_run[2] = {-INFINITY, -INFINITY};   // reference score of the exponentials (a lazy running maximum)
-  float ms_run[2] = {0.f, 0.f};              // m_run * scale_log2, 0 while m_run is -inf
-  f32x4 l_acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};   // l_acc[qt][r]: softmax denominator of query 16qt + 4c + r
-  const bf16x8 ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80};
-
-  // Real-key tile ranges: of this wave's 32 queries and of the workgroup's 256.
-  const int last_row = min(row0 + kRowsPerWave, Lq) - 1;
-  const int p_lo = row0 + pos_shift, p_hi = last_row + pos_shift;
+  // Tile ranges: of the workgroup's rows and (real keys) of this wave's.
+  const int p_lo = quotient(min(w0, rows - 1), group) + pos_shift, p_hi = quotient(min(w0 + kRowsPerWave - 1, rows - 1), group) + pos_shift;
   int tw_lo = 0, tw_hi = -1, T_lo = 0, T_hi = -1;
   if (!meta_rows && Lk > 0) {
-    if (active && p_hi >= 0) {
-      const int k_lo = (a.window_left >= 0 && p_lo - a.window_left > 0) ? p_lo - a.window_left : 0;
-      const int k_hi = p_hi < Lk - 1 ? p_hi : Lk - 1;
-      tw_lo = k_lo / kTileK;
-      tw_hi = k_hi / kTileK;
-    }
-    const int P_lo = blk0 + pos_shift, P_hi = min(blk0 + kRowsPerBlock, Lq) - 1 + pos_shift;
-    if (P_hi >= 0) {
-      const int k_lo = (a.window_left >= 0 && P_lo - a.window_left > 0) ? P_lo - a.window_left : 0;
-      const int k_hi = P_hi < Lk - 1 ? P_hi : Lk - 1;
-      T_lo = k_lo / kTileK;
-      T_hi = k_hi / kTileK;
-    }
+    auto tiles_of = [&](int first, int last, int& lo, int& hi) __attribute__((always_inline)) {
+      if (last < 0) return;
+      lo = (a.window_left >= 0 && first - a.window_left > 0 ? first - a.window_left : 0) / kTileK;
+      hi = min(last, Lk - 1) / kTileK;
+    };
+    if (active) tiles_of(p_lo, p_hi, tw_lo, tw_hi);
+    tiles_of(quotient(r0, group) + pos_shift, quotient(min(r0 + kRows - 1, rows - 1), group) + pos_shift, T_lo, T_hi);
   }
   const int all_tiles = meta_tiles + (T_hi - T_lo + 1);
   // this workgroup's share of the tile sequence (all of it when there is one slice)
-  const int per_split = (all_tiles + splits - 1) / splits;
+  const int per_split = quotient(all_tiles + splits - 1, splits);
   const int t_begin = min(split * per_split, all_tiles);
-  const int ntiles = min(t_begin + per_split, all_tiles);     // one past the last tile walked here
+  const int t_end = min(t_begin + per_split, all_tiles);
+  // Tile t holds the real keys from 64 (t + t_real) on, if t >= meta_tiles.
+  const int t_real = T_lo - meta_tiles;
+  // first and last tile that this wave's rows see (with meta keys: from the first on)
+  const int seen_lo = active ? (meta_tiles > 0 ? 0 : tw_lo - t_real) : all_tiles + 1, seen_hi = active && tw_hi >= 0 ? tw_hi - t_real : meta_tiles - 1;
+  // real tiles that every row of the wave sees whole: [clear_lo, clear_hi)
+  const int clear_lo = max(meta_tiles, (a.window_left >= 0 ? max(p_hi - a.window_left + kTileK - 1, 0) / kTileK : 0) - t_real);
+  const int clear_hi = max(min(p_lo + 1, Lk), 0) / kTileK - t_real;
 
-  const uint16_t* kglob = nullptr;
-  const uint16_t* vglob = nullptr;
-  const int32_t* bt = nullptr;
+  // ---- copies: an instruction takes four rows of an image, lane = row lane / 16, chunk lane % 16 as it lies in LDS; the
+  // wave's i-th the rows 4 (wave + 4 i) ..
+  const int32_t* bt = PAGED ? a.block_tables + static_cast<int64_t>(seq) * a.block_table_stride : nullptr;
+  const int64_t k_row = 2 * (PAGED ? a.cache_stride_pos : a.k_stride_t), v_row = 2 * (PAGED ? a.cache_stride_pos : a.v_stride_t);
+  const char* kglob;
+  const char* vglob;
   if constexpr (PAGED) {
-    kglob = reinterpret_cast<const uint16_t*>(a.key_cache) + static_cast<int64_t>(kvh) * a.cache_stride_h;
-    vglob = reinterpret_cast<const uint16_t*>(a.value_cache) + static_cast<int64_t>(kvh) * a.cache_stride_h;
-    bt = a.block_tables + static_cast<int64_t>(seq) * a.block_table_stride;
-  } else if (!meta_rows) {
-    kglob = reinterpret_cast<const uint16_t*>(a.key) + k_first * a.k_stride_t + static_cast<int64_t>(kvh) * a.k_stride_h;
-    vglob = reinterpret_cast<const uint16_t*>(a.value) + k_first * a.v_stride_t + static_cast<int64_t>(kvh) * a.v_stride_h;
+    kglob = static_cast<const char*>(a.key_cache) + 2 * kvh * a.cache_stride_h;
+    vglob = static_cast<const char*>(a.value_cache) + 2 * kvh * a.cache_stride_h;
+  } else {
+    kglob = static_cast<const char*>(a.key) + 2 * kvh * a.k_stride_h + k_first * k_row;
+    vglob = static_cast<const char*>(a.value) + 2 * kvh * a.v_stride_h + k_first * v_row;
   }
-
-  // ---- staging role: thread = 16-byte chunk sc of key rows sr + 4 NW i (i < kPasses) of the tile
-  const int sr = tid >> 4, sc = tid & 15;
-  constexpr int kRowStep = 4 * NW;
-  // Loads are unconditional (rows past the end are clamped to the last valid row and zeroed when
-  // they are committed), so nothing has to wait for them before the tile's compute.
-  u32x4 kreg[kPasses], vreg[kPasses];
-  bool rok[kPasses] = {};
-  // Un-paged keys: the thread's two row pointers walk down the tile sequence (one 64-bit add per
-  // pointer and tile); they are rebuilt only where the sequence of tiles changes tensor (first
-  // tile, first real tile after the meta tiles).  klast / vlast: the last valid row of the tensor
-  // being walked, what a row past the end reads instead.
-  const uint16_t* kptr[kPasses] = {};
-  const uint16_t* vptr[kPasses] = {};
-  const uint16_t* klast = nullptr;
-  const uint16_t* vlast = nullptr;
-  int64_t kstep = 0, vstep = 0;
-  int prow = 0, plimit = 0;            // row index of kptr[0] in its tensor, and that tensor's row count
-  auto issue = [&](int tile) {
-    if constexpr (PAGED) {
+  auto chunk_of = [&](int ln, bool value) __attribute__((always_inline)) -> uint32_t {      // (16 rows on: the same)
+    return 16 * ((ln & 15) ^ (value ? value_twist(ln >> 4) : key_twist(4 * wave + (ln >> 4))));
+  };
+  const uint32_t kplace = (lane >> 4) * static_cast<uint32_t>(k_row) + chunk_of(lane, false);
+  const uint32_t vplace = (lane >> 4) * static_cast<uint32_t>(v_row) + chunk_of(lane, true);
+  const char* kwave = kglob + 4 * wave * k_row;
+  const char* vwave = vglob + 4 * wave * v_row;
+  // Tiles [whole_lo, whole_hi) are 64 rows at one stride (whole tiles within a page, four rows within 32 bits): a base per tile
+  // and an offset per lane.  Every other one's rows are found one by one.
+  const bool regular = (PAGED ? a.block_size % kTileK == 0 : true) && max(k_row, v_row) < (1 << 27);
+  const int whole_lo = meta_tiles, whole_hi = regular ? Lk / kTileK - t_real : 0;
+  // Paged: lane = tile % 64 holds where a tile's first row lies, for 64 tiles from the last refill on.
+  int64_t tile_at = 0;
+  auto refill = [&](int t) __attribute__((always_inline)) {
+    if (!PAGED) return;
+    const int tile = t + ((lane - t) & 63);
+    if (tile < whole_lo || tile >= min(whole_hi, t_end)) return;
+    const int j = (tile + t_real) * kTileK, at = j / a.block_size;
+    tile_at = 2 * (bt[at] * a.cache_stride_block + (j - at * a.block_size) * a.cache_stride_pos);
+  };
+  auto place_of = [&](int t, int64_t row_bytes) __attribute__((always_inline)) -> int64_t {
+    if (!PAGED) return static_cast<int64_t>(t + t_real) * kTileK * row_bytes;
+    const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int>(tile_at), t & 63);
+    const int hi = __builtin_amdgcn_readlane(static_cast<int>(tile_at >> 32), t & 63);
+    return (static_cast<int64_t>(hi) << 32) | lo;
+  };
+  auto copy_tile = [&](int t, bool value, char* image) __attribute__((always_inline)) {
+    if (t >= whole_lo && t < whole_hi) {
+      const int64_t row_bytes = value ? v_row : k_row;
+      const char* base = (value ? vwave : kwave) + place_of(t, row_bytes);
 #pragma unroll
-      for (int i = 0; i < kPasses; ++i) {
-        const int r = sr + kRowStep * i;
-        const uint16_t* kp;
-        const uint16_t* vp;
-        if (tile < meta_tiles) {
-          const int idx = tile * kTileK + r;
-          rok[i] = idx < M;
-          const int64_t off = static_cast<int64_t>(min(idx, M - 1)) * a.meta_stride_t + static_cast<int64_t>(kvh) * a.meta_stride_h + 8 * sc;
-          kp = reinterpret_cast<const uint16_t*>(a.meta_key) + off;
-          vp = reinterpret_cast<const uint16_t*>(a.meta_value) + off;
+      for (int i = 0; i < kCopies; ++i) {
+        copy16_to_lds(base, value ? vplace : kplace, image + 1024 * (wave + kWaves * i));
+        base += 4 * kWaves * row_bytes;
+      }
+      return;
+    }
+    // rows past the last repeat it (their weights are zero)
+    int ln = lane;
+    asm volatile("" : "+v"(ln));               // (nothing of this is kept in registers over the other tiles)
+    for (int i = 0; i < kCopies; ++i) {
+      const int row = 4 * (wave + kWaves * i) + (ln >> 4);
+      const char* from;
+      if (t < meta_tiles) {
+        from = static_cast<const char*>(value ? a.meta_value : a.meta_key) + 2 * (min(t * kTileK + row, M - 1) * a.meta_stride_t + kvh * a.meta_stride_h);
+      } else {
+        const int j = min((t + t_real) * kTileK + row, Lk - 1);
+        from = value ? vglob : kglob;
+        if (PAGED) {
+          const int at = j / a.block_size;
+          from += 2 * (bt[at] * a.cache_stride_block + (j - at * a.block_size) * a.cache_stride_pos);
         } else {
-          const int p_raw = (T_lo + tile - meta_tiles) * kTileK + r;
-          rok[i] = p_raw < Lk;   // rows past the sequence end: stale cache
-          const int p = min(p_raw, Lk - 1);
-          const int64_t off = static_cast<int64_t>(bt[p / a.block_size]) * a.cache_stride_block +
-                              static_cast<int64_t>(p % a.block_size) * a.cache_stride_pos + 8 * sc;
-          kp = kglob + off;
-          vp = vglob + off;
+          from += j * (value ? v_row : k_row);
         }
-        kreg[i] = ld16(kp);
-        vreg[i] = ld16(vp);
       }
-    } else {
-      if (tile == t_begin || tile == meta_tiles) { // workgroup-uniform, at most twice per workgroup
-        const bool meta = tile < meta_tiles;
-        const uint16_t* kb = meta ? reinterpret_cast<const uint16_t*>(a.meta_key) + static_cast<int64_t>(kvh) * a.meta_stride_h : kglob;
-        const uint16_t* vb = meta ? reinterpret_cast<const uint16_t*>(a.meta_value) + static_cast<int64_t>(kvh) * a.meta_stride_h : vglob;
-        const int64_t ks = meta ? a.meta_stride_t : a.k_stride_t, vs = meta ? a.meta_stride_t : a.v_stride_t;
-        plimit = meta ? M : Lk;
-        prow = (meta ? tile : T_lo + tile - meta_tiles) * kTileK + sr;
-        kstep = ks * kTileK, vstep = vs * kTileK;
-#pragma unroll
-        for (int i = 0; i < kPasses; ++i) {
-          kptr[i] = kb + static_cast<int64_t>(prow + kRowStep * i) * ks + 8 * sc;
-          vptr[i] = vb + static_cast<int64_t>(prow + kRowStep * i) * vs + 8 * sc;
-        }
-        klast = kb + static_cast<int64_t>(plimit - 1) * ks + 8 * sc;
-        vlast = vb + static_cast<int64_t>(plimit - 1) * vs + 8 * sc;
-      }
-#pragma unroll
-      for (int i = 0; i < kPasses; ++i) {
-        rok[i] = prow + kRowStep * i < plimit;           // rows past the end: next sequence, or outside the tensor
-        kreg[i] = ld16(rok[i] ? kptr[i] : klast);
-        vreg[i] = ld16(rok[i] ? vptr[i] : vlast);
-        kptr[i] += kstep;
-        vptr[i] += vstep;
-      }
-      prow += kTileK;
-    }
-  };
-  auto commit = [&](int buf) {
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    bool all_ok = true;
-#pragma unroll
-    for (int i = 0; i < kPasses; ++i) all_ok = all_ok && rok[i];
-    if (__all(all_ok)) {
-#pragma unroll
-      for (int i = 0; i < kPasses; ++i) {
-        const int r = sr + kRowStep * i;
-        st16(&sm.k[buf][r * kKPitch + 16 * (sc ^ (r & 15))], kreg[i]);
-        st16(&sm.v[buf][r * kVPitch + 16 * sc], vreg[i]);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < kPasses; ++i) {
-        const int r = sr + kRowStep * i;
-        st16(&sm.k[buf][r * kKPitch + 16 * (sc ^ (r & 15))], rok[i] ? kreg[i] : z);
-        st16(&sm.v[buf][r * kVPitch + 16 * sc], rok[i] ? vreg[i] : z);
-      }
+      copy16_to_lds(from + chunk_of(ln, value), image + 1024 * (wave + kWaves * i));
     }
   };
 
-  if (ntiles > t_begin) {
-    issue(t_begin);
-    commit(0);
+  // ---- LDS offsets of this lane's fragments
+  int koff[8], voff[4];
+#pragma unroll
+  for (int st = 0; st < 8; ++st) koff[st] = n * kPitch + 16 * ((2 * st + hh) ^ key_twist(n));
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) {
+    const int R = 4 * hh + ((lane & 15) >> 2), chunk = 4 * cb + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+    voff[cb] = R * kPitch + 16 * (chunk ^ value_twist(R)) + 8 * (lane & 1);
   }
-  if (ntiles > t_begin + 1) issue(t_begin + 1);
-  // Pin the Q fragments as landed here: otherwise the first MFMA of EVERY tile waits for all
-  // outstanding global loads (the just-issued next tile included) on behalf of the Q loads above.
-#pragma unroll
-  for (int qt = 0; qt < 2; ++qt)
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(qf[qt][ks]));
-  __syncthreads();
 
-  for (int tile = t_begin; tile < ntiles; ++tile) {
-    const int buf = (tile - t_begin) & 1;
-    // Tile t + 1 (loaded during the previous tile) goes to the other buffer now, behind the barrier
-    // that ended its last reads, and tile t + 2 is requested at once: the stores overlap the
-    // other waves' matrix work instead of standing between every wave's last MFMA and the barrier.
-    if (tile + 1 < ntiles) commit(buf ^ 1);
-    if (tile + 2 < ntiles) issue(tile + 2);
+  f32x16 o[4];                               // O^T: columns 32 cb + 8 i + 4 hh + e of the lane's row, i, e < 4
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[cb][i] = 0.f;
+  float ref = 0.f, l = 0.f;                  // reference of the exponentials (base 2, a lazy running maximum), sum of the weights
+  bool unset = true;                         // the row has not seen a key
+  f32x16 sa[2], sb[2];                       // scores: keys 32 x + 8 i + 4 hh + e of a tile, element 4 i + e of [x]
+  u32x4 pa[4], pb[4];                        // weights: keys 8 i + 4 hh + e and 32 further, e < 4, of [i]
 
-    const bool is_meta = tile < meta_tiles;
-    const int rt = T_lo + tile - meta_tiles;   // real tile index
-    if (active && (is_meta || (rt >= tw_lo && rt <= tw_hi))) {
-      const int pos0 = is_meta ? tile * kTileK : rt * kTileK;
-      // Every (query, key) pair of the tile visible?  (wave-uniform)
-      const bool full = is_meta ? (pos0 + kTileK <= M)
-                                : (pos0 + kTileK - 1 <= p_lo && pos0 + kTileK <= Lk &&
-                                   (a.window_left < 0 || p_hi - pos0 <= a.window_left));
-      const char* kimg = sm.k[buf];
-      const char* vimg = sm.v[buf];
-
-      // S^T tiles: st[qt][s][r] = score(key 16s + 4c + r, query 16qt + n)
-      f32x4 st[2][4];
+  // fragment f of a step: f < 16 of the keys (step f / 2 of the head, half f % 2 of the tile), else of the values (16 keys
+  // (f - 16) / 4, columns 32 (f % 4) ..)
+  auto fragment = [&](const char* kimg, const char* vimg, int f) __attribute__((always_inline)) {
+    if (f < 16) return ld16(kimg + koff[f >> 1] + (f & 1) * 32 * kPitch);
+    const char* v = vimg + voff[f & 3] + ((f - 16) >> 2) * 8 * kPitch;
+    const u32x2 lo = tr_read(v), hi = tr_read(v + 32 * kPitch);
+    return u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
+  // After the scores of tile t: mask them, move the reference where they ask for it.  `p` holds the weights that are not in
+  // `o` yet; steps of the reference are whole powers of two, so that they scale exactly.
+  auto settle = [&](int t, f32x16 (&s)[2], float mx, u32x4 (&p)[4]) __attribute__((always_inline)) {
+    if (t < clear_lo || t >= clear_hi) {
+      const bool is_meta = t < meta_tiles;
+      const int pos0 = (is_meta ? t : t + t_real) * kTileK;
+      // visible key positions of this lane's query: [lo, hi], as one unsigned range test
+      const int qp = qi + pos_shift;
+      const int lo = is_meta || a.window_left < 0 ? 0 : max(qp - a.window_left, 0), hi = is_meta ? M - 1 : min(qp, Lk - 1);
+      const unsigned span = static_cast<unsigned>(hi - lo);
+      int ahead = pos0 + 4 * hh - lo;
+      asm volatile("" : "+v"(ahead));          // (keeps the compiler from working this out on every tile)
+      mx = -INFINITY;
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        bf16x8 kf[4];
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) kf[ks] = as_frag(ld16(kimg + (16 * s + n) * kKPitch + 16 * ((4 * ks + c) ^ n)));
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt) {
-          st[qt][s] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ks = 0; ks < 4; ++ks) st[qt][s] = mfma16(kf[ks], qf[qt][ks], st[qt][s]);
-        }
-      }
-
-      if (!full) {
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt) {
-          // visible key positions of this lane's query: [lo, hi], as one unsigned range test
-          const int qp = row0 + 16 * qt + n + pos_shift;
-          int lo = 0, hi = M - 1;
-          if (!is_meta) {
-            lo = a.window_left >= 0 ? max(qp - a.window_left, 0) : 0;
-            hi = min(qp, Lk - 1);
-          }
-          const bool any = hi >= lo;
-          const unsigned span = static_cast<unsigned>(hi - lo);
-#pragma unroll
-          for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int kp = pos0 + 16 * s + 4 * c + r;
-              const bool ok = any & (static_cast<unsigned>(kp - lo) <= span);
-              st[qt][s][r] = ok ? st[qt][s][r] : -INFINITY;
-            }
-        }
-      }
-
-      // online softmax per query column
-      bf16x8 pf[2][2];
-      float tnew[2];
-#pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        float tmax = max3(st[qt][0][0], st[qt][0][1], st[qt][0][2]);
-        tmax = max3(tmax, st[qt][0][3], st[qt][1][0]);
-        tmax = max3(tmax, st[qt][1][1], st[qt][1][2]);
-        tmax = max3(tmax, st[qt][1][3], st[qt][2][0]);
-        tmax = max3(tmax, st[qt][2][1], st[qt][2][2]);
-        tmax = max3(tmax, st[qt][2][3], st[qt][3][0]);
-        tmax = max3(tmax, st[qt][3][1], st[qt][3][2]);
-        tmax = max3(tmax, st[qt][3][3], st[qt][3][3]);
-        // across the four 16-lane groups (the tile's other keys) with the two row-swap
-        // instructions: ALU latency on the tile's critical path instead of two LDS round trips
-        const auto h16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
-        tmax = max3(__uint_as_float(h16[0]), __uint_as_float(h16[1]), tmax);
-        const auto h32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
-        tnew[qt] = max3(__uint_as_float(h32[0]), __uint_as_float(h32[1]), tmax);
-      }
-      // The running reference m_run follows the row maximum lazily: it moves (and the running
-      // output is rescaled) only when some query's scores exceed it by more than 2^kLazyLog2, so
-      // P stays <= 2^kLazyLog2 and most tiles skip the pass over the 64 output registers.  The
-      // decision precedes this tile's exponentials and follows the previous tile's P V.
-      const bool grow = (tnew[0] - m_run[0]) * scale_log2 > kLazyLog2 || (tnew[1] - m_run[1]) * scale_log2 > kLazyLog2;
-      if (__any(grow)) {
-        float alpha[2];
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt) {
-          const float m_new = max3(m_run[qt], tnew[qt], tnew[qt]);
-          const float m_use = m_new == -INFINITY ? 0.f : m_new;
-          alpha[qt] = __builtin_amdgcn_exp2f((m_run[qt] - m_use) * scale_log2);
-          m_run[qt] = m_new;
-          ms_run[qt] = m_use * scale_log2;
-        }
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float ar = __shfl(alpha[qt], 4 * c + r);  // o rows are queries 4c + r
-#pragma unroll
-            for (int t = 0; t < 8; ++t) o[qt][t][r] *= ar;
-            l_acc[qt][r] *= ar;
-          }
-      }
-      // P re-packed as the A operand of P V:
-      // fragment kh, slot j <-> key 32kh + (j < 4 ? 4c + j : 16 + 4c + j - 4)
-#pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        const float ms = ms_run[qt];
-#pragma unroll
-        for (int kh = 0; kh < 2; ++kh) {
-          float p[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            p[j] = __builtin_amdgcn_exp2f(fmaf(st[qt][2 * kh + (j >> 2)][j & 3], scale_log2, -ms));
-          u32x4 pw;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) pw[i] = pack_bf16x2(p[2 * i], p[2 * i + 1]);
-          pf[qt][kh] = as_frag(pw);
-        }
-      }
-
-      // O += P V : o[qt][t][r] = O[query 16qt + 4c + r][dim 16t + n]
-      const char* vlane = vimg + (4 * c + (n >> 2)) * kVPitch + 8 * (n & 3);
-#pragma unroll
-      for (int kh = 0; kh < 2; ++kh) {
-        // row sums of the bf16 P that enters P V, on the matrix cores (B = ones)
-        l_acc[0] = mfma16(pf[0][kh], ones, l_acc[0]);
-        l_acc[1] = mfma16(pf[1][kh], ones, l_acc[1]);
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const s16x4 lo = tr_read(vlane + (32 * kh) * kVPitch + 32 * t);
-          const s16x4 hi = tr_read(vlane + (32 * kh + 16) * kVPitch + 32 * t);
-          const bf16x8 vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          o[0][t] = mfma16(pf[0][kh], vf, o[0][t]);
-          o[1][t] = mfma16(pf[1][kh], vf, o[1][t]);
-        }
+      for (int i = 0; i < 32; ++i) {
+        const bool in = hi >= lo && static_cast<unsigned>(ahead + 32 * (i >> 4) + 8 * ((i & 15) >> 2) + (i & 3)) <= span;
+        s[i >> 4][i & 15] = in ? s[i >> 4][i & 15] : -INFINITY;
+        mx = __builtin_elementwise_maximum(mx, s[i >> 4][i & 15]);
       }
     }
+    const float over = fmaf(mx, scale_log2, -ref);
+    if (__any(over > kLazyLog2 || (unset && mx > -INFINITY))) {
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float top = fmaf(mx, scale_log2, -ref);
+      const bool up = top > kLazyLog2 || (unset && mx > -INFINITY);
+      const float step = up ? ceilf(top) : 0.f, corr = up ? (unset ? 0.f : __builtin_amdgcn_exp2f(-step)) : 1.f;
+      ref += step;
+      unset = unset && !up;
+      l *= corr;
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) o[cb] *= corr;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p[i][e] = pack_bf16x2(lo_bf(p[i][e]) * corr, hi_bf(p[i][e]) * corr);
+    }
+  };
+  // One step: scores of tile t + 1 into `next`, weights of tile t (scores `cur`) into `p`, output of tile t - 1 (weights `q`).
+  // A slot is one product, the read of a fragment a few products ahead and a slice of the vector work.
+  constexpr int kAhead = 4;
+  auto step = [&](const char* kimg, const char* vimg, f32x16 (&cur)[2], f32x16 (&next)[2], u32x4 (&p)[4], u32x4 (&q)[4]) __attribute__((always_inline)) -> float {
+    u32x4 fr[32];
+    float mx = 0.f;
+#pragma unroll
+    for (int f = 0; f < kAhead; ++f) fr[f] = fragment(kimg, vimg, f);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) next[x][i] = 0.f;
+#pragma unroll
+    for (int f = 0; f < 32; ++f) {
+      if (f + kAhead < 32) fr[f + kAhead] = fragment(kimg, vimg, f + kAhead);
+      if (f < 16) next[f & 1] = mfma32(fr[f], qf[f >> 1], next[f & 1]);
+      else o[f & 3] = mfma32(fr[f], q[(f - 16) >> 2], o[f & 3]);
+      // weights: 16 pairs of scores, ten of them under the first product, six under the second
+      const int lo = f < 16 ? f * 10 / 16 : 10 + (f - 16) * 6 / 10, hi = f < 16 ? (f + 1) * 10 / 16 : 10 + (f - 15) * 6 / 10;
+#pragma unroll
+      for (int j = lo; j < (hi < 16 ? hi : 16); ++j) {
+        const int i = j >> 2, e = j & 3;
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(cur[e >> 1][4 * i + 2 * (e & 1)], scale_log2, -ref));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(cur[e >> 1][4 * i + 2 * (e & 1) + 1], scale_log2, -ref));
+        p[i][e] = pack_bf16x2(p0, p1);
+        l = add_pair(p[i][e], l);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (lo <= 4 * i + 3 && 4 * i + 3 < hi) asm volatile("" : "+v"(p[i]), "+v"(l));      // here, not where they are used
+      // the next tile's maximum
+      if (f == 20) mx = __builtin_elementwise_maximum(next[0][0], next[1][0]);
+      if (f > 20) {
+#pragma unroll
+        for (int j = 1 + (f - 21) * 15 / 11; j < 1 + (f - 20) * 15 / 11; ++j) mx = max3(mx, next[0][j], next[1][j]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("" : "+v"(mx));
+    return mx;
+  };
+  // The same without a tile t - 1 that this wave's rows see.
+  auto lead = [&](const char* kimg, f32x16 (&cur)[2], f32x16 (&next)[2], u32x4 (&p)[4]) __attribute__((always_inline)) -> float {
+#pragma unroll
+    for (int i = 0; i < 32; ++i) next[i >> 4][i & 15] = 0.f;
+#pragma unroll
+    for (int f = 0; f < 16; ++f) next[f & 1] = mfma32(fragment(kimg, kimg, f), qf[f >> 1], next[f & 1]);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int i = j >> 2, e = j & 3;
+      const float p0 = __builtin_amdgcn_exp2f(fmaf(cur[e >> 1][4 * i + 2 * (e & 1)], scale_log2, -ref));
+      const float p1 = __builtin_amdgcn_exp2f(fmaf(cur[e >> 1][4 * i + 2 * (e & 1) + 1], scale_log2, -ref));
+      p[i][e] = pack_bf16x2(p0, p1);
+      l = add_pair(p[i][e], l);
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mx = max3(mx, next[0][i], next[1][i]);
+    return mx;
+  };
+  auto blank = [&](f32x16 (&s)[2], u32x4 (&p)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 32; ++i) s[i >> 4][i & 15] = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p[i] = u32x4{0u, 0u, 0u, 0u};
+  };
 
-    __syncthreads();
+  blank(sa, pa), blank(sb, pb);
+  if (t_begin < t_end) {
+    refill(t_begin);
+    copy_tile(t_begin, false, s_k[0]);
+    copies_landed_barrier();
+    if (t_begin + 1 < t_end) copy_tile(t_begin + 1, false, s_k[1]);
+    settle(t_begin, sa, lead(s_k[0], sb, sa, pa), pa);     // the first tile's scores
+    // tile t: keys and values in images (t - t_begin) & 1
+    auto arrive = [&](int t, int even) __attribute__((always_inline)) {
+      copies_landed_barrier();               // keys of t + 1 and values of t - 1 are there, and nobody reads the images they leave
+      if (t + 2 < t_end) copy_tile(t + 2, false, s_k[even]);
+      copy_tile(t, true, s_v[even]);
+    };
+    auto iterate = [&](int t, int even, f32x16 (&cur)[2], f32x16 (&next)[2], u32x4 (&p)[4], u32x4 (&q)[4]) __attribute__((always_inline)) {
+      arrive(t, even);
+      if (t + 1 < seen_lo || t - 1 > seen_hi) {
+        blank(next, p);
+        return;
+      }
+      const float mx = step(s_k[1 - even], s_v[1 - even], cur, next, p, q);
+      if (t + 1 < t_end) settle(t + 1, next, mx, p);
+    };
+    auto finish = [&](int last, u32x4 (&p)[4]) __attribute__((always_inline)) {
+      copies_landed_barrier();
+#pragma unroll
+      for (int f = 16; f < 32; ++f) o[f & 3] = mfma32(fragment(s_v[last], s_v[last], f), p[(f - 16) >> 2], o[f & 3]);
+    };
+    arrive(t_begin, 0);
+    {
+      const float mx = lead(s_k[1], sa, sb, pa);
+      if (t_begin + 1 < t_end) settle(t_begin + 1, sb, mx, pa);
+    }
+    int t = t_begin + 1;
+    for (; t + 1 < t_end; t += 2) {
+      if (((t - t_begin) & 31) == 31) refill(t);
+      iterate(t, 1, sb, sa, pb, pa);
+      iterate(t + 1, 0, sa, sb, pa, pb);
+    }
+    if (t < t_end) {
+      iterate(t, 1, sb, sa, pb, pa);
+      finish(1, pb);
+    } else {
+      finish(0, pa);
+    }
   }
+  l += __shfl_xor(l, 32, 64);
+  if (!ok) return;
 
   if (splits > 1) {
-    // partial of this key slice: O un-normalised (fp32), per query its reference exponent (the
-    // lanes of the first 16-lane group hold the queries' references) and its row sum
+    // partial of this key slice: O un-normalised (fp32), the row's reference exponent and its sum
+    const int64_t prow = (split * part_rows + out_first + qi) * a.num_heads + h;
     float* po = static_cast<float*>(a.workspace);
     float* pm = po + static_cast<int64_t>(splits) * part_rows * a.num_heads * kHeadDim;
     float* pl = pm + static_cast<int64_t>(splits) * part_rows * a.num_heads;
+    if (hh == 0) pm[prow] = unset ? -INFINITY : ref, pl[prow] = l;
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
-      if (c == 0) {
-        const int qr = row0 + 16 * qt + n;
-        if (qr < Lq) pm[(split * part_rows + out_first + qr) * a.num_heads + h] = m_run[qt] == -INFINITY ? -INFINITY : ms_run[qt];
-      }
+    for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int qr = row0 + 16 * qt + 4 * c + r;
-        if (qr >= Lq) continue;
-        const int64_t prow_ = (split * part_rows + out_first + qr) * a.num_heads + h;
-        if (n == 0) pl[prow_] = l_acc[qt][r];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) po[prow_ * kHeadDim + 16 * t + n] = o[qt][t][r];
-      }
-    }
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<f32x4*>(po + prow * kHeadDim + 32 * cb + 8 * i + 4 * hh) = f32x4{o[cb][4 * i], o[cb][4 * i + 1], o[cb][4 * i + 2], o[cb][4 * i + 3]};
     return;
   }
-
-  // epilogue: normalise, stage the wave's 32 x 128 outputs in LDS (the K/V images are free after
-  // the loop's last barrier), store whole rows.
-  char* ost = reinterpret_cast<char*>(&sm) + wave * (kRowsPerWave * kOPitch);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  uint16_t* out = static_cast<uint16_t*>(a.out) + (out_first + qi) * a.out_stride_t + static_cast<int64_t>(h) * a.out_stride_h;
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
+  for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float lr = l_acc[qt][r];
-      const float inv = lr > 0.f ? 1.f / lr : 0.f;
-      uint16_t* orow = reinterpret_cast<uint16_t*>(ost + (16 * qt + 4 * c + r) * kOPitch) + n;
-#pragma unroll
-      for (int t = 0; t < 8; ++t) orow[16 * t] = f2bf(o[qt][t][r] * inv);
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int id = lane + 64 * i;
-    const int row = id >> 4, ch = id & 15;
-    const int qr = row0 + row;
-    if (qr < Lq) {
-      uint16_t* op = reinterpret_cast<uint16_t*>(a.out) + (out_first + qr) * a.out_stride_t +
-                     static_cast<int64_t>(h) * a.out_stride_h + 8 * ch;
-      st16(op, ld16(ost + row * kOPitch + 16 * ch));
-    }
-  }
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<u32x2*>(out + 32 * cb + 8 * i + 4 * hh) =
+          u32x2{pack_bf16x2(o[cb][4 * i] * inv, o[cb][4 * i + 1] * inv), pack_bf16x2(o[cb][4 * i + 2] * inv, o[cb][4 * i + 3] * inv)};
 }
 
 // One wave per (output row, head): out = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s, slices in order.
@@ -587,14 +550,6 @@ extern "C" int hymeta_meta_swa_prefill(const hymeta_swa_prefill_args* args, hyme
   if (a.meta_query != nullptr && a.num_meta > max_rows) max_rows = a.num_meta;
   const int seqs = have_rows ? a.num_seqs : 0;
   if (!have_rows) a.num_seqs = 0;
-  // 256-query workgroups, unless they would leave more than half of the compute units idle:
-  // then 128-query ones (the same tiles staged by half as many threads, two workgroups per
-  // compute unit; measured 13 % faster on a 2048-query chunk of one 7-head shard, slower once the
-  // 256-query workgroups already fill the chip)
-  const int64_t wgs256 = (static_cast<int64_t>(have_rows ? a.total_q : 0) + 255) / 256 * a.num_heads +
-                         (a.meta_query != nullptr ? static_cast<int64_t>(a.num_heads) * ((a.num_meta + 255) / 256) : 0);
-  const int nw = wgs256 < 128 ? 4 : 8;
-  const int rows_per_block = kRowsPerWave * nw;
   // key slices: the library's choice needs a workspace that holds it (without one: a single slice)
   const int64_t out_rows = static_cast<int64_t>(have_rows ? a.total_q : 0) + (a.meta_query != nullptr ? a.num_meta : 0);
   int splits = a.num_splits > 0 ? a.num_splits
@@ -606,16 +561,12 @@ extern "C" int hymeta_meta_swa_prefill(const hymeta_swa_prefill_args* args, hyme
     splits = 1;
   }
   if (splits > 1 && reinterpret_cast<uintptr_t>(a.workspace) % 16 != 0) return HYMETA_ERR_UNSUPPORTED;
-  dim3 grid((max_rows + rows_per_block - 1) / rows_per_block * splits, seqs + (a.meta_query != nullptr ? 1 : 0), a.num_heads);
+  const int64_t blocks = (static_cast<int64_t>(max_rows) * (a.num_heads / a.num_kv_heads) + kRows - 1) / kRows;
+  dim3 grid(static_cast<unsigned>(blocks * splits * a.num_kv_heads), seqs + (a.meta_query != nullptr ? 1 : 0));
   hipStream_t s = begin_launches(stream);
   const float sl2 = scale * kLog2e;
-  if (paged) {
-    if (nw == 8) hipLaunchKernelGGL((swa_prefill_kernel<true, 8>), grid, dim3(512), 0, s, a, sl2, splits, out_rows);
-    else hipLaunchKernelGGL((swa_prefill_kernel<true, 4>), grid, dim3(256), 0, s, a, sl2, splits, out_rows);
-  } else {
-    if (nw == 8) hipLaunchKernelGGL((swa_prefill_kernel<false, 8>), grid, dim3(512), 0, s, a, sl2, splits, out_rows);
-    else hipLaunchKernelGGL((swa_prefill_kernel<false, 4>), grid, dim3(256), 0, s, a, sl2, splits, out_rows);
-  }
+  if (paged) hipLaunchKernelGGL((swa_prefill_kernel<true>), grid, dim3(64 * kWaves), 0, s, a, sl2, splits, out_rows);
+  else hipLaunchKernelGGL((swa_prefill_kernel<false>), grid, dim3(64 * kWaves), 0, s, a, sl2, splits, out_rows);
   if (splits > 1) {
     if (hipGetLastError() != hipSuccess) return HYMETA_ERR_LAUNCH;
     const int64_t pairs = out_rows * a.num_heads;
