@@ -168,3 +168,31 @@ def test_kernels_without_slices_ask_for_no_room_for_them(D, dtype, monkeypatch):
     q, cache = torch.randn(5, 4, D, device=dev).to(dtype), torch.randn(64, 64, 1, D + 2 * 64, device=dev).to(dtype)
     out = hip_ops.sink_attention(q, cache, torch.arange(64, dtype=torch.int32, device=dev)[None], i32([0, 5]), i32([4096]), 2, D, 64, D ** -0.5, 5, 4096, shared_key=True)
     assert asked == [_C.load().hymeta_sink_attention_workspace_bytes(1, 4, 2, 64, 4096)] and torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("layout,D,Dv,H,G,rows,ctx,scale,opts", [
+    ("rows", 64, 128, 8, 8, 4300, 0, 0.125, dict(sink=True, bias=True)),          # more tiles than a lane table holds
+    ("rows", 128, 64, 14, 2, 2500, 2100, -0.08, dict(keep=9, window=2200)),       # scores that fall with their products
+    ("rows", 128, 128, 4, 4, 4500, 1, 0.1, dict(softcap=3.0, chunk=4300)),
+    ("shared", 64, 64, 6, 6, 4400, 77, 0.125, dict(sink=True)),
+])
+def test_long_portions_against_the_general_kernel(layout, D, Dv, H, G, rows, ctx, scale, opts):
+    """Pages of 64 against pages of 48, which only the kernel of one row per wave reads."""
+    from vllm_hymeta import hip_ops
+    dev, g, total = "cuda", torch.Generator().manual_seed(D + rows), rows + ctx
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
+    tail = (1, D + G * Dv) if layout == "shared" else (G, D + Dv)
+    keys, q = torch.randn((total,) + tail, generator=g).bfloat16().to(dev), torch.randn(rows, H, D, generator=g).bfloat16().to(dev)
+    bias = dict(bias_a=(0.1 + torch.rand(H, generator=g)).to(dev), bias_b=torch.full((H,), NEAR, device=dev)) if opts.get("bias") else {}
+    outs = []
+    for page in (64, 48):
+        pages = (total + page - 1) // page
+        table = torch.randperm(pages, generator=g).to(torch.int32).to(dev)
+        cache = torch.full((pages * page,) + tail, float("nan"), dtype=torch.bfloat16, device=dev)
+        j = torch.arange(total, device=dev)
+        cache[table[j // page].long() * page + j % page] = keys
+        outs.append(hip_ops.sink_attention(q, cache.view((pages, page) + tail), table[None], i32([0, rows]), i32([total]), G, D, Dv, scale, rows, total,
+                                           sink=opts.get("sink", False), softcap=opts.get("softcap", 0.0), chunk=opts.get("chunk", 0),
+                                           window_left=opts.get("window", 0) - 1, keep_first=opts.get("keep", 0), shared_key=layout == "shared", **bias).double())
+    assert all(torch.isfinite(o).all() for o in outs)
+    assert (outs[0] - outs[1]).norm() <= 2 * BOUND * outs[1].norm()             # (each within BOUND of the exact result)

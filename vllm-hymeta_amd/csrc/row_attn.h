@@ -1,4 +1,5 @@
-// Prompts' portions of the attention over paged rows, keys of up to 192 elements: included by sink_attn.hip.
+// Prompts' portions of the attention over paged rows, keys of up to 192 elements, where the value lies inside the key or a cap
+// meets a bias (the others: row_pipe.h): included by sink_attn.hip.
 #pragma once
 
 #include "row_copy.h"
@@ -38,7 +39,7 @@ struct RowShape {
 
 // How a score follows from its product, in kernels of their own where a design's every layer asks for it: a branch per row
 // block in the middle of a tile keeps the compiler from overlapping what stands on its two sides.
-enum ScoreRule { kPlain, kLogBias, kAnyRule };
+enum ScoreRule { kPlain, kLogBias, kCapped, kAnyRule };
 
 template <int D, int DV, int Layout, int Rule>
 __global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attention_args a, PortionSlices ps) {

@@ -1002,6 +1002,7 @@ __global__ __launch_bounds__(kCombineThreads) void sink_attention_combine_few_ke
 }  // namespace hymeta
 
 #include "row_attn.h"
+#include "row_pipe.h"
 #include "wide_latent.h"
 
 namespace hymeta {
@@ -1141,14 +1142,22 @@ int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st) {
     if constexpr (D <= 192) {
       ps = portion_slices(a);
       const dim3 grid = portion_grid(a, ps);
-      auto launch = [&](auto rule) { hipLaunchKernelGGL((row_prefill_kernel<D, DV, Layout, decltype(rule)::value>), grid, dim3(256), 0, st, a, ps); };
-      const bool plain = a.softcap <= 0.f && a.bias_mode != HYMETA_BIAS_LOG_DISTANCE;
-      if constexpr (Layout == HYMETA_KV_SCALED_KEY) launch(std::integral_constant<int, kPlain>{});
-      else if (plain) launch(std::integral_constant<int, kPlain>{});
+      // a kernel per rule of the scores; a cap and a bias together, which no design has, in the general one
+      auto launch = [&](auto rule) {
+        constexpr int Rule = decltype(rule)::value;
+        if constexpr ((Layout == HYMETA_KV_KEY_THEN_VALUE || Layout == HYMETA_KV_SHARED_KEY) && Rule != kAnyRule)
+          hipLaunchKernelGGL((row_pipe_kernel<D, DV, Layout, Rule>), grid, dim3(256), 0, st, a, ps);
+        else hipLaunchKernelGGL((row_prefill_kernel<D, DV, Layout, Rule>), grid, dim3(256), 0, st, a, ps);
+      };
+      const bool log_bias = a.bias_mode == HYMETA_BIAS_LOG_DISTANCE, capped = a.softcap > 0.f;
+      if (Layout == HYMETA_KV_SCALED_KEY || (!log_bias && !capped)) launch(std::integral_constant<int, kPlain>{});
       else if constexpr (Layout == HYMETA_KV_KEY_THEN_VALUE) {
-        if (a.softcap <= 0.f) launch(std::integral_constant<int, kLogBias>{});
+        if (!capped) launch(std::integral_constant<int, kLogBias>{});
+        else if (!log_bias) launch(std::integral_constant<int, kCapped>{});
         else launch(std::integral_constant<int, kAnyRule>{});
-      } else launch(std::integral_constant<int, kAnyRule>{});
+      } else if constexpr (Layout != HYMETA_KV_SCALED_KEY) {
+        launch(std::integral_constant<int, kAnyRule>{});
+      }
     } else {
       constexpr int kRows = 16 * kPrefillWaves;
       const dim3 grid((a.max_query_len + kRows - 1) / kRows, a.num_heads, a.num_seqs);
