@@ -4,9 +4,11 @@
 // with unit-length queries and keys, the state fp32 and carried per sequence.  Beside the decayed scan (decay_scan.hip),
 // whose state only adds what a token brings.
 #include "act_types.h"
-#include "lds_copy.h"
+#include "row_copy.h"
 
+#include <algorithm>
 #include <type_traits>
+#include <utility>
 
 namespace hymeta {
 
@@ -76,22 +78,19 @@ __global__ __launch_bounds__(256) void delta_rule_rows_kernel(hymeta_delta_rule_
   }
 }
 
-// Sequences with one row (decode).  grid = (heads, sequences), 256 threads over the state in fours of value columns: a
-// thread takes the columns 4 c4 .. 4 c4 + 3 of the rows d0, d0 + dstep, ... of S and keeps them in registers (16-byte loads,
-// all in flight together).  S^T k and S^T q of the OLD state are reduced over the row groups in one go; what the token's own
-// write adds to the output is u (k . q), so the state is read once and written once with one reduction between.  Norm: the
-// head's output row goes through its RMS norm, weight and silu gate in the same launch.
+// The rows t0 .. t1 - 1 of a sequence, one after the other, by 256 threads over the state in fours of value columns: a thread
+// takes the columns 4 c4 .. 4 c4 + 3 of the rows d0, d0 + dstep, ... of S and keeps them in registers (16-byte loads, all in
+// flight together).  S^T k and S^T q of the OLD state are reduced over the row groups in one go; what the token's own write
+// adds to the output is u (k . q), so the state is read once and written once with one reduction per row between.  Norm: the
+// head's output rows go through their RMS norm, weight and silu gate as well.
 constexpr int kStepMaxD = 256, kStepRows = 16;
+struct StepScratch {
+  __attribute__((aligned(16))) float a[256 * 4], c[256 * 4], u[1024];
+  float q[kStepMaxD], k[kStepMaxD], red[4];
+};
 template <typename A, bool Norm>
-__global__ __launch_bounds__(256) void delta_rule_step_kernel(hymeta_delta_rule_args a) {
+__device__ __forceinline__ void delta_rows(const hymeta_delta_rule_args& a, int h, int s, int t0, int t1, StepScratch& m) {
   typedef typename A::elem elem;
-  __shared__ float s_q[kStepMaxD], s_k[kStepMaxD];
-  __shared__ __attribute__((aligned(16))) float s_a[256 * 4], s_c[256 * 4];
-  __shared__ __attribute__((aligned(16))) float s_u[1024];
-  __shared__ float red[4];
-  const int h = blockIdx.x, s = blockIdx.y;
-  const int t = a.query_start_loc[s];
-  if (a.query_start_loc[s + 1] - t != 1) return;
   const int H = a.num_heads, D = a.head_dim, Dv = a.v_dim, Dv4 = Dv / 4;
   const int g = h / (H / a.num_qk_heads);
   const int c4 = threadIdx.x % Dv4, d0 = threadIdx.x / Dv4, dstep = 256 / Dv4, lane = threadIdx.x & 63;
@@ -104,79 +103,91 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(hymeta_delta_rule_
     const int d = d0 + u * dstep;
     S[u] = (carry && d < D) ? *reinterpret_cast<const f32x4*>(st + static_cast<int64_t>(d) * Dv + 4 * c4) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  const elem* q = static_cast<const elem*>(a.q) + static_cast<int64_t>(t) * a.q_stride_t + static_cast<int64_t>(g) * D;
-  const elem* k = static_cast<const elem*>(a.k) + static_cast<int64_t>(t) * a.k_stride_t + static_cast<int64_t>(g) * D;
-  const float decay = exp2_act<A>(fmaxf(a.log2_decay[static_cast<int64_t>(t) * H + h], kMinLog2));
-  const float beta = sigmoid_exact(A::ld(static_cast<const elem*>(a.beta_logit) + static_cast<int64_t>(t) * a.beta_stride_t + h));
-  // every wave sums the lengths and the product for itself
-  float kk = 0.f, qq = 0.f, kq = 0.f;
-  for (int d = lane; d < D; d += 64) {
-    const float kd = A::ld(k + d), qd = A::ld(q + d);
-    if (threadIdx.x < 64) s_k[d] = kd, s_q[d] = qd;
-    kk = fmaf(kd, kd, kk);
-    qq = fmaf(qd, qd, qq);
-    kq = fmaf(kd, qd, kq);
-  }
-  kk = wave_sum(kk), qq = wave_sum(qq), kq = wave_sum(kq);
-  const float ik = 1.f / sqrtf(kk + a.unit_eps), iq = a.q_scale / sqrtf(qq + a.unit_eps);
-  __syncthreads();
-  f32x4 pa = f32x4{0.f, 0.f, 0.f, 0.f}, pc = pa;
-#pragma unroll
-  for (int u = 0; u < kStepRows; ++u) {
-    const int d = d0 + u * dstep;
-    if (d >= D) continue;
-    const float kd = s_k[d], qd = s_q[d];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) pa[e] = fmaf(S[u][e], kd, pa[e]), pc[e] = fmaf(S[u][e], qd, pc[e]);
-  }
-  *reinterpret_cast<f32x4*>(&s_a[threadIdx.x * 4]) = pa;          // [d0][4 c4 + e]
-  *reinterpret_cast<f32x4*>(&s_c[threadIdx.x * 4]) = pc;
-  __syncthreads();
-  float o[4] = {0.f, 0.f, 0.f, 0.f}, ss = 0.f;                    // columns threadIdx.x, + 256, ...
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int c = threadIdx.x + 256 * i;
-    if (c >= Dv) continue;
-    float da = 0.f, dc = 0.f;
-    for (int gg = 0; gg < dstep; ++gg) da += s_a[gg * Dv + c], dc += s_c[gg * Dv + c];
-    const float v = A::ld(static_cast<const elem*>(a.v) + static_cast<int64_t>(t) * a.v_stride_t + static_cast<int64_t>(h) * Dv + c);
-    const float u = beta * (v - decay * (da * ik)) * ik;          // (with the key's length: what multiplies the raw key)
-    s_u[c] = u;
-    o[i] = iq * fmaf(u, kq, decay * dc);
-    ss = fmaf(o[i], o[i], ss);
-  }
-  __syncthreads();
-  if (st != nullptr) {
-    const f32x4 u4 = *reinterpret_cast<const f32x4*>(&s_u[4 * c4]);
+  for (int t = t0; t < t1; ++t) {
+    const elem* q = static_cast<const elem*>(a.q) + static_cast<int64_t>(t) * a.q_stride_t + static_cast<int64_t>(g) * D;
+    const elem* k = static_cast<const elem*>(a.k) + static_cast<int64_t>(t) * a.k_stride_t + static_cast<int64_t>(g) * D;
+    const float decay = exp2_act<A>(fmaxf(a.log2_decay[static_cast<int64_t>(t) * H + h], kMinLog2));
+    const float beta = sigmoid_exact(A::ld(static_cast<const elem*>(a.beta_logit) + static_cast<int64_t>(t) * a.beta_stride_t + h));
+    if (t > t0) __syncthreads();                                  // (the state's update reads the last row's key)
+    // every wave sums the lengths and the product for itself
+    float kk = 0.f, qq = 0.f, kq = 0.f;
+    for (int d = lane; d < D; d += 64) {
+      const float kd = A::ld(k + d), qd = A::ld(q + d);
+      if (threadIdx.x < 64) m.k[d] = kd, m.q[d] = qd;
+      kk = fmaf(kd, kd, kk);
+      qq = fmaf(qd, qd, qq);
+      kq = fmaf(kd, qd, kq);
+    }
+    kk = wave_sum(kk), qq = wave_sum(qq), kq = wave_sum(kq);
+    const float ik = 1.f / sqrtf(kk + a.unit_eps), iq = a.q_scale / sqrtf(qq + a.unit_eps);
+    __syncthreads();
+    f32x4 pa = f32x4{0.f, 0.f, 0.f, 0.f}, pc = pa;
 #pragma unroll
     for (int u = 0; u < kStepRows; ++u) {
       const int d = d0 + u * dstep;
       if (d >= D) continue;
-      const float kd = s_k[d];
+      const float kd = m.k[d], qd = m.q[d];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) S[u][e] = fmaf(decay, S[u][e], kd * u4[e]);
-      *reinterpret_cast<f32x4*>(st + static_cast<int64_t>(d) * Dv + 4 * c4) = S[u];
+      for (int e = 0; e < 4; ++e) pa[e] = fmaf(S[u][e], kd, pa[e]), pc[e] = fmaf(S[u][e], qd, pc[e]);
     }
-  }
-  const int64_t at = (static_cast<int64_t>(t) * H + h) * Dv;
-  if constexpr (Norm) {
-    ss = block_sum<4>(ss, red);
-    const float inv = 1.f / sqrtf(ss / static_cast<float>(Dv) + a.norm_eps);
-    const elem* gate = static_cast<const elem*>(a.gate) + static_cast<int64_t>(t) * a.gate_stride_t + static_cast<int64_t>(h) * Dv;
+    *reinterpret_cast<f32x4*>(&m.a[threadIdx.x * 4]) = pa;        // [d0][4 c4 + e]
+    *reinterpret_cast<f32x4*>(&m.c[threadIdx.x * 4]) = pc;
+    __syncthreads();
+    float o[4] = {0.f, 0.f, 0.f, 0.f}, ss = 0.f;                  // columns threadIdx.x, + 256, ...
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int c = threadIdx.x + 256 * i;
       if (c >= Dv) continue;
-      const float gv = A::ld(gate + c);
-      A::st(static_cast<elem*>(a.out) + at + c, o[i] * inv * a.norm_weight[c] * gv * sigmoid_exact(gv));
+      float da = 0.f, dc = 0.f;
+      for (int gg = 0; gg < dstep; ++gg) da += m.a[gg * Dv + c], dc += m.c[gg * Dv + c];
+      const float v = A::ld(static_cast<const elem*>(a.v) + static_cast<int64_t>(t) * a.v_stride_t + static_cast<int64_t>(h) * Dv + c);
+      const float u = beta * (v - decay * (da * ik)) * ik;        // (with the key's length: what multiplies the raw key)
+      m.u[c] = u;
+      o[i] = iq * fmaf(u, kq, decay * dc);
+      ss = fmaf(o[i], o[i], ss);
     }
-  } else {
+    __syncthreads();
+    if (st != nullptr || t + 1 < t1) {
+      const f32x4 u4 = *reinterpret_cast<const f32x4*>(&m.u[4 * c4]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = threadIdx.x + 256 * i;
-      if (c < Dv) static_cast<float*>(a.out)[at + c] = o[i];
+      for (int u = 0; u < kStepRows; ++u) {
+        const int d = d0 + u * dstep;
+        if (d >= D) continue;
+        const float kd = m.k[d];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[u][e] = fmaf(decay, S[u][e], kd * u4[e]);
+        if (st != nullptr && t + 1 == t1) *reinterpret_cast<f32x4*>(st + static_cast<int64_t>(d) * Dv + 4 * c4) = S[u];
+      }
+    }
+    const int64_t at = (static_cast<int64_t>(t) * H + h) * Dv;
+    if constexpr (Norm) {
+      ss = block_sum<4>(ss, m.red);
+      const float inv = 1.f / sqrtf(ss / static_cast<float>(Dv) + a.norm_eps);
+      const elem* gate = static_cast<const elem*>(a.gate) + static_cast<int64_t>(t) * a.gate_stride_t + static_cast<int64_t>(h) * Dv;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int c = threadIdx.x + 256 * i;
+        if (c >= Dv) continue;
+        const float gv = A::ld(gate + c);
+        A::st(static_cast<elem*>(a.out) + at + c, o[i] * inv * a.norm_weight[c] * gv * sigmoid_exact(gv));
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int c = threadIdx.x + 256 * i;
+        if (c < Dv) static_cast<float*>(a.out)[at + c] = o[i];
+      }
     }
   }
+}
+
+// Sequences with one row (decode).  grid = (heads, sequences).
+template <typename A, bool Norm>
+__global__ __launch_bounds__(256) void delta_rule_step_kernel(hymeta_delta_rule_args a) {
+  __shared__ StepScratch m;
+  const int h = blockIdx.x, s = blockIdx.y, t = a.query_start_loc[s];
+  if (a.query_start_loc[s + 1] - t != 1) return;
+  delta_rows<A, Norm>(a, h, s, t, t + 1, m);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -195,19 +206,16 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(hymeta_delta_rule_
 // ------------------------------------------------------------------------------------------------
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 constexpr int kChunk = HYMETA_DELTA_CHUNK;
-// Workgroups (with slices of 32 value columns) up to which the second launch runs slices of 16: measured for one prompt of 8192
-// with 28 heads of 128 x 128 (112 workgroups) 357 against 405 us, with 64 heads (256) 706 against 566 us.  They also double the
-// workgroups of the sequences without a chunk, which end at once but take about 0.65 ns each to come and go, and save about 0.55
-// us a chunk of 64 rows: not where those are more than 10 per row of the longest portion.  28 heads, slices of 16 and of 32, us:
-// 100 rows beside 63 single ones 52.1 and 49.1, 400 beside 63 72.1 and 67.2, 700 beside 63 78.4 and 76.3, 2048 beside 63 122 and
-// 133, 1000 beside 200 170 and 157, 2048 beside 255 246 and 222.
-constexpr int kFewGroups = 128, kIdleGroupsPerRow = 10;
-// Workgroups of slices of 128 columns above which the second launch takes those: slices of 32 are then more than the 512
-// workgroups that run at the same time.  With 28 heads of 128 x 128 (16 for the last two): 5 portions of 1801 rows 310 us in
-// narrow slices, 281 in wide ones (140 workgroups); 16 of 500 250 and 191; 40 of 300 414 and 276; 8 of 700 (128) 102 and 108.
-// Both count the portions that the step's rows are worth (long_portions): one of 8192 rows beside 63 single rows took 960 us in
-// the wide slices that 64 sequences asked for, 420 in slices of 16 (single rows and the solving launch included).
-constexpr int kManyWideGroups = 128;
+// Workgroups with slices of 32 value columns up to which the second launch runs slices of 16 whose waves share a chunk's rows
+// (delta_chunk_narrow_kernel), about 2 us a chunk against 2.6 where a wave takes all rows of its columns: one prompt of 8192
+// rows with 28 heads of 128 x 128 (112 workgroups) 327 us against 388, with 16 heads 216 against 345.  They also double the
+// workgroups of the sequences without a chunk, which end at once but take about 0.65 ns each to come and go, and save about 0.6
+// us a chunk of 64 rows: not where those are more than 10 per row of the longest portion.
+// Workgroups with slices of 64 columns up to which the other kernel takes those: its images leave room for one workgroup on a
+// compute unit, where four waves take 2.6 us a chunk and eight (slices of 128) 4.4.  28 heads: three portions of 2700 (168)
+// 177 us, 301 before; five of 1801 (280, in slices of 128) 182, 280 before.
+// All count the portions that the step's rows are worth (long_portions): single rows leave the chip to a long prompt.
+constexpr int kFewGroups = 128, kIdleGroupsPerRow = 10, kManyGroups = 256;
 constexpr int kChunkMinRows = 8;            // shorter portions go token by token
 constexpr int kMat = kChunk * kChunk;
 // Where the second launch reads 64 x 64 matrices (or the chunk's keys) as matrix operands, they lie in the operand's own
@@ -224,6 +232,12 @@ struct ChunkPlace {
 };
 static_assert(sizeof(ChunkPlace) % 16 == 0, "16-byte loads of every place");
 
+// f(0), f(1), ... f(N - 1) with constants
+template <int N, typename F, int... I>
+__device__ __forceinline__ void unrolled(const F& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void unrolled(const F& f) { unrolled<N>(f, std::make_integer_sequence<int, N>{}); }
+
 __device__ __forceinline__ f32x4v mfma16(bf16x8 a, bf16x8 b, f32x4v c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ bf16x8 frag(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
@@ -236,16 +250,22 @@ __device__ __forceinline__ void split4(const float* v, u32x2& hi, u32x2& lo) {
   }
 }
 
-// Workspace: the chunks' places ([chunk][head]), then per chunk and query / key head the chunk's keys [64][D], queries [64][D]
-// and transposed keys [D][64], bf16 in operand order.
+// Workspace: the chunks' places ([chunk][head]), then (narrow slices) per chunk and query / key head the chunk's keys [64][D],
+// queries [64][D] and transposed keys [D][64], bf16 in operand order.
 __host__ __device__ inline size_t rows_at(int64_t chunks, int heads) { return static_cast<size_t>(chunks) * heads * sizeof(ChunkPlace); }
 
 // grid = (chunk numbers, heads), 4 waves with 16 rows of the chunk each.
-template <int D>
-__global__ __launch_bounds__(256) void delta_chunk_solve_kernel(hymeta_delta_rule_args a, int64_t chunks) {
+// Portions shorter than kChunkMinRows go token by token here (short_too: the state fits the threads' registers), so that they
+// need no launch of their own: two launches with nothing to do took 9 of the 280 us of five portions of 1801 rows.
+template <int D, bool Pack>
+__global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hymeta_delta_rule_args a, int64_t chunks, int short_too) {
   constexpr int PK = D + 8, PF = kChunk + 4;
-  __shared__ __attribute__((aligned(16))) uint16_t sk[kChunk * PK];
-  __shared__ __attribute__((aligned(16))) float sA[kChunk * PF], sT[kChunk * PF];
+  // (the keys and T share their place where nothing asks for the keys again: four workgroups to a compute unit)
+  constexpr int kKeyBytes = kChunk * PK * 2, kMatrixBytes = kChunk * PF * 4;
+  __shared__ __attribute__((aligned(16))) char s_keys[Pack ? kKeyBytes + kMatrixBytes : kKeyBytes > kMatrixBytes ? kKeyBytes : kMatrixBytes];
+  uint16_t* sk = reinterpret_cast<uint16_t*>(s_keys);
+  float* sT = reinterpret_cast<float*>(s_keys + (Pack ? kKeyBytes : 0));
+  __shared__ __attribute__((aligned(16))) float sA[kChunk * PF];
   __shared__ float s_hi[kChunk], s_lo[kChunk], s_beta[kChunk], s_ik[kChunk], s_iq[kChunk];
   // the sequence: the last one whose first number is not past this one
   const int number = blockIdx.x;
@@ -257,7 +277,12 @@ __global__ __launch_bounds__(256) void delta_chunk_solve_kernel(hymeta_delta_rul
   }
   const int r0 = a.query_start_loc[s], rows = a.query_start_loc[s + 1] - r0;
   const int c0 = (number - (r0 / kChunk + s)) * kChunk;
-  if (rows < kChunkMinRows || c0 >= rows) return;
+  if (c0 >= rows) return;
+  if (rows < kChunkMinRows) {
+    static_assert(sizeof(StepScratch) <= sizeof(sA), "the scratch lies where A would");
+    if (short_too) delta_rows<ActBf16, false>(a, blockIdx.y, s, r0, r0 + rows, *reinterpret_cast<StepScratch*>(sA));
+    return;
+  }
   const int nrow = min(kChunk, rows - c0), h = blockIdx.y, H = a.num_heads, group = H / a.num_qk_heads, g = h / group;
   const int64_t t0 = r0 + c0;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g4 = lane >> 4;
@@ -327,9 +352,9 @@ __global__ __launch_bounds__(256) void delta_chunk_solve_kernel(hymeta_delta_rul
       }
       *reinterpret_cast<f32x4v*>(&sA[i * PF + 16 * jb + 4 * g4]) = f32x4v{av[0], av[1], av[2], av[3]};
     }
-    // (the blocks behind the diagonal are stored as zeros: every wave multiplies all 64 rows)
     u32x2 hi, lo;
     split4(pv, hi, lo);
+    if (!Pack && wave < 2 && jb >= 2) continue;         // (rows up to 31, columns from 32 on: narrow slices alone multiply these zeros)
     *reinterpret_cast<u32x2*>(&place->p[0][operand_at(i, 16 * jb + 4 * g4, kChunk)]) = hi;
     *reinterpret_cast<u32x2*>(&place->p[1][operand_at(i, 16 * jb + 4 * g4, kChunk)]) = lo;
   }
@@ -375,6 +400,7 @@ __global__ __launch_bounds__(256) void delta_chunk_solve_kernel(hymeta_delta_rul
     const int row = tid >> 2, jb = tid & 3, rb = row >> 4;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
+      if (!Pack && rb < 2 && jb >= 2) break;
       float v[4] = {0.f, 0.f, 0.f, 0.f};
       if (jb <= rb) {
         const f32x4v tv = *reinterpret_cast<const f32x4v*>(&sT[row * PF + 16 * jb + 4 * u]);
@@ -387,7 +413,7 @@ __global__ __launch_bounds__(256) void delta_chunk_solve_kernel(hymeta_delta_rul
       *reinterpret_cast<u32x2*>(&place->t[1][operand_at(row, 16 * jb + 4 * u, kChunk)]) = lo;
     }
   }
-  if (h % group == 0) {
+  if (Pack && h % group == 0) {
     uint16_t* kr = reinterpret_cast<uint16_t*>(static_cast<char*>(a.workspace) + rows_at(chunks, H)) +
                    (static_cast<int64_t>(number) * a.num_qk_heads + g) * 3 * D * kChunk;
     uint16_t *qr = kr + D * kChunk, *kt = qr + D * kChunk;
@@ -416,15 +442,15 @@ __global__ __launch_bounds__(256) void delta_chunk_solve_kernel(hymeta_delta_rul
   }
 }
 
-// grid = (heads, sequences, value columns in slices of 16 CB), 4 waves.  The state slice stays fp32 in registers in blocks of
+// grid = (heads, sequences, value columns in slices of 16), 4 waves.  The state slice stays fp32 in registers in blocks of
 // 16 x 16 dealt over the waves (a lane holds 4 consecutive rows d of one column); its bf16 parts, the right-hand side and
 // U pass through LDS with the reduced index consecutive; everything a chunk brings comes from memory in the matrix
 // operands' own layout, loaded two chunks ahead (the loads of two chunks are in flight, each in registers of its own).  Rows past the portion read its last row (beta, and with it what they would
 // write, is 0 there), and the last chunk fetches itself once more, so that no load stands under a condition.
-template <int D, int CB>
-__global__ __launch_bounds__(256) void delta_chunk_scan_kernel(hymeta_delta_rule_args a, int64_t chunks) {
-  constexpr int SV = 16 * CB, PK = D + 8, PT = kChunk + 8, NBW = (D / 16) * CB / 4;
-  static_assert((D / 16) * CB % 4 == 0, "the state's blocks deal evenly over the waves");
+template <int D>
+__global__ __launch_bounds__(256) void delta_chunk_narrow_kernel(hymeta_delta_rule_args a, int64_t chunks) {
+  constexpr int SV = 16, PK = D + 8, PT = kChunk + 8, NBW = D / 16 / 4;
+  static_assert(D / 16 % 4 == 0, "the state's blocks deal evenly over the waves");
   __shared__ __attribute__((aligned(16))) uint16_t sst[2][SV * PK];                                      // state, [c][d]
   __shared__ __attribute__((aligned(16))) uint16_t srt[2][SV * PT], su[2][SV * PT], sw[2][SV * PT];      // [c][row]
   const int h = blockIdx.x, s = blockIdx.y, vs = blockIdx.z;
@@ -438,19 +464,19 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(hymeta_delta_rule
   f32x4v S[NBW];
 #pragma unroll
   for (int ib = 0; ib < NBW; ++ib) {
-    const int b = wave + 4 * ib, cb = b % CB, db = b / CB;
+    const int db = wave + 4 * ib;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) S[ib][r] = carry ? st[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + 16 * cb + n] : 0.f;
+    for (int r = 0; r < 4; ++r) S[ib][r] = carry ? st[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + n] : 0.f;
   }
   auto state_to_lds = [&]() {
 #pragma unroll
     for (int ib = 0; ib < NBW; ++ib) {
-      const int b = wave + 4 * ib, cb = b % CB, db = b / CB;
+      const int db = wave + 4 * ib;
       const float v[4] = {S[ib][0], S[ib][1], S[ib][2], S[ib][3]};
       u32x2 hi, lo;
       split4(v, hi, lo);
-      *reinterpret_cast<u32x2*>(&sst[0][(16 * cb + n) * PK + 16 * db + 4 * g4]) = hi;
-      *reinterpret_cast<u32x2*>(&sst[1][(16 * cb + n) * PK + 16 * db + 4 * g4]) = lo;
+      *reinterpret_cast<u32x2*>(&sst[0][n * PK + 16 * db + 4 * g4]) = hi;
+      *reinterpret_cast<u32x2*>(&sst[1][n * PK + 16 * db + 4 * g4]) = lo;
     }
   };
   state_to_lds();
@@ -463,7 +489,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(hymeta_delta_rule
   // what a chunk brings: row fragments of the keys, queries, T and P, the transposed keys of this wave's state blocks, values
   struct Chunk {
     u32x4 kf[D / 32], qf[D / 32], tf[2][2], pf[2][2], wf[NBW][2];
-    uint16_t vv[CB][4];
+    uint16_t vv[4];
     f32x4v beta, rhs, read, write;
     float total;
   };
@@ -474,11 +500,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(hymeta_delta_rule
 #pragma unroll
     for (int sd = 0; sd < D / 32; ++sd) m.kf[sd] = ld16g(kr + 512 * sd), m.qf[sd] = ld16g(kr + D * kChunk + 512 * sd);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const uint16_t* vr = vp + (t0 + min(iq + r, last)) * a.v_stride_t;
-#pragma unroll
-      for (int cb = 0; cb < CB; ++cb) m.vv[cb][r] = vr[16 * cb];
-    }
+    for (int r = 0; r < 4; ++r) m.vv[r] = vp[(t0 + min(iq + r, last)) * a.v_stride_t];
   };
   auto fetch_t = [&](Chunk& m, int c) {
     const ChunkPlace* p = places + static_cast<int64_t>(c) * H;
@@ -503,7 +525,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(hymeta_delta_rule
     m.total = places[static_cast<int64_t>(c) * H].total;
 #pragma unroll
     for (int ib = 0; ib < NBW; ++ib) {
-      const int db = (wave + 4 * ib) / CB;
+      const int db = wave + 4 * ib;
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) m.wf[ib][kk] = ld16g(kt + (2 * db + kk) * 512);
     }
@@ -513,42 +535,39 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(hymeta_delta_rule
   auto advance = [&](Chunk& m, int c, auto full) {         // full: a whole chunk (every row is the portion's)
     const int next = min(c + 2, num - 1);
     __syncthreads();                        // the state's parts are in place
-    f32x4v x[CB], y[CB];
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      x[cb] = y[cb] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    f32x4v x, y;
+    {
+      x = y = f32x4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int sd = 0; sd < D / 32; ++sd) {
-        const bf16x8 sh = frag(ld16(&sst[0][(16 * cb + n) * PK + 32 * sd + 8 * g4]));
-        const bf16x8 sl = frag(ld16(&sst[1][(16 * cb + n) * PK + 32 * sd + 8 * g4]));
-        x[cb] = mfma16(frag(m.kf[sd]), sh, x[cb]);
-        y[cb] = mfma16(frag(m.qf[sd]), sh, y[cb]);
-        x[cb] = mfma16(frag(m.kf[sd]), sl, x[cb]);
-        y[cb] = mfma16(frag(m.qf[sd]), sl, y[cb]);
+        const bf16x8 sh = frag(ld16(&sst[0][n * PK + 32 * sd + 8 * g4]));
+        const bf16x8 sl = frag(ld16(&sst[1][n * PK + 32 * sd + 8 * g4]));
+        x = mfma16(frag(m.kf[sd]), sh, x);
+        y = mfma16(frag(m.qf[sd]), sh, y);
+        x = mfma16(frag(m.kf[sd]), sl, x);
+        y = mfma16(frag(m.qf[sd]), sl, y);
       }
     }
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
+    {
       float v[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        v[r] = m.beta[r] * bf2f(m.vv[cb][r]) - m.rhs[r] * x[cb][r];
-        y[cb][r] *= m.read[r];
+        v[r] = m.beta[r] * bf2f(m.vv[r]) - m.rhs[r] * x[r];
+        y[r] *= m.read[r];
       }
       u32x2 hi, lo;
       split4(v, hi, lo);
-      *reinterpret_cast<u32x2*>(&srt[0][(16 * cb + n) * PT + iq]) = hi;
-      *reinterpret_cast<u32x2*>(&srt[1][(16 * cb + n) * PT + iq]) = lo;
+      *reinterpret_cast<u32x2*>(&srt[0][n * PT + iq]) = hi;
+      *reinterpret_cast<u32x2*>(&srt[1][n * PT + iq]) = lo;
     }
     fetch_rows(m, next);
     __syncthreads();
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
+    {
       f32x4v u = f32x4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
-        const bf16x8 rh = frag(ld16(&srt[0][(16 * cb + n) * PT + 32 * kk + 8 * g4]));
-        const bf16x8 rl = frag(ld16(&srt[1][(16 * cb + n) * PT + 32 * kk + 8 * g4]));
+        const bf16x8 rh = frag(ld16(&srt[0][n * PT + 32 * kk + 8 * g4]));
+        const bf16x8 rl = frag(ld16(&srt[1][n * PT + 32 * kk + 8 * g4]));
         u = mfma16(frag(m.tf[0][kk]), rh, u);
         u = mfma16(frag(m.tf[0][kk]), rl, u);
         u = mfma16(frag(m.tf[1][kk]), rh, u);
@@ -556,38 +575,36 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(hymeta_delta_rule
       float v[4] = {u[0], u[1], u[2], u[3]};
       u32x2 hi, lo;
       split4(v, hi, lo);
-      *reinterpret_cast<u32x2*>(&su[0][(16 * cb + n) * PT + iq]) = hi;
-      *reinterpret_cast<u32x2*>(&su[1][(16 * cb + n) * PT + iq]) = lo;
+      *reinterpret_cast<u32x2*>(&su[0][n * PT + iq]) = hi;
+      *reinterpret_cast<u32x2*>(&su[1][n * PT + iq]) = lo;
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[r] *= m.write[r];
       split4(v, hi, lo);
-      *reinterpret_cast<u32x2*>(&sw[0][(16 * cb + n) * PT + iq]) = hi;
-      *reinterpret_cast<u32x2*>(&sw[1][(16 * cb + n) * PT + iq]) = lo;
+      *reinterpret_cast<u32x2*>(&sw[0][n * PT + iq]) = hi;
+      *reinterpret_cast<u32x2*>(&sw[1][n * PT + iq]) = lo;
     }
     fetch_t(m, next);
     __syncthreads();
 #pragma unroll
     for (int ib = 0; ib < NBW; ++ib) {
-      const int cb = (wave + 4 * ib) % CB;
       f32x4v acc = S[ib] * m.total;
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
-        acc = mfma16(frag(m.wf[ib][kk]), frag(ld16(&sw[0][(16 * cb + n) * PT + 32 * kk + 8 * g4])), acc);
-        acc = mfma16(frag(m.wf[ib][kk]), frag(ld16(&sw[1][(16 * cb + n) * PT + 32 * kk + 8 * g4])), acc);
+        acc = mfma16(frag(m.wf[ib][kk]), frag(ld16(&sw[0][n * PT + 32 * kk + 8 * g4])), acc);
+        acc = mfma16(frag(m.wf[ib][kk]), frag(ld16(&sw[1][n * PT + 32 * kk + 8 * g4])), acc);
       }
       S[ib] = acc;
     }
     fetch_transposed(m, next);
     state_to_lds();                         // (its last readers passed the barrier before)
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
+    {
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
-        const bf16x8 uh = frag(ld16(&su[0][(16 * cb + n) * PT + 32 * kk + 8 * g4]));
-        const bf16x8 ul = frag(ld16(&su[1][(16 * cb + n) * PT + 32 * kk + 8 * g4]));
-        y[cb] = mfma16(frag(m.pf[0][kk]), uh, y[cb]);
-        y[cb] = mfma16(frag(m.pf[0][kk]), ul, y[cb]);
-        y[cb] = mfma16(frag(m.pf[1][kk]), uh, y[cb]);
+        const bf16x8 uh = frag(ld16(&su[0][n * PT + 32 * kk + 8 * g4]));
+        const bf16x8 ul = frag(ld16(&su[1][n * PT + 32 * kk + 8 * g4]));
+        y = mfma16(frag(m.pf[0][kk]), uh, y);
+        y = mfma16(frag(m.pf[0][kk]), ul, y);
+        y = mfma16(frag(m.pf[1][kk]), uh, y);
       }
     }
     fetch_p(m, next);
@@ -596,8 +613,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(hymeta_delta_rule
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       if (decltype(full)::value || r < live) {
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) to[static_cast<int64_t>(r) * H * Dv + 16 * cb] = y[cb][r];
+        to[static_cast<int64_t>(r) * H * Dv ] = y[r];
       }
   };
   Chunk even, odd;
@@ -621,187 +637,291 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(hymeta_delta_rule
   if (st != nullptr) {
 #pragma unroll
     for (int ib = 0; ib < NBW; ++ib) {
-      const int b = wave + 4 * ib, cb = b % CB, db = b / CB;
+      const int db = wave + 4 * ib;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) st[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + 16 * cb + n] = S[ib][r];
+      for (int r = 0; r < 4; ++r) st[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + n] = S[ib][r];
     }
   }
 }
 
-// The same over wide slices: grid = (heads, sequences, value columns in slices of 128), 8 waves of 16 columns.  Every step
-// of a chunk keeps to its columns, so a wave runs alone from barrier to barrier: the state, the right-hand side and U are
-// accumulators (a lane holds four consecutive rows of one column), and a pair of such blocks IS the operand of the next
-// product with the reduced index in the order 4 g4 + e, 16 + 4 g4 + e - 4; the other operand is read from LDS in that order.
-// What a chunk brings is copied to LDS a chunk ahead, once for all columns; a chunk's outputs are stored in the next one, so
-// that the wait for the copies does not wait for stores just issued.
-// Bound by the chain of a chunk's products: with a workgroup on 55 % of the compute units LDS (every wave reads the chunk's 73
-// KB) is busy 28 % of the time of all of them, the matrix pipes 12 %, and the waves wait half of theirs.  About 6.7 us a chunk on a
-// compute unit, two waves on a SIMD; 4 workgroups of slices of 32 take 8.2.
-template <int D>
-__global__ __launch_bounds__(512) void delta_chunk_wide_kernel(hymeta_delta_rule_args a, int64_t chunks) {
-  constexpr int NW = 8;
-  constexpr int SD = D / 32, DB = D / 16, kRowsBytes = 3 * D * kChunk * 2, kMatBytes = 6 * 1024, kImage = kRowsBytes + 4 * kMatBytes + 1024;
-  constexpr int kCopies = kImage / 1024;
-  __shared__ __attribute__((aligned(16))) char images[2][kImage];       // keys, queries, transposed keys | T hi, lo, P hi, lo | beta, rhs, read, write
+// grid = (heads, sequences, value columns in slices of 16 NW), NW waves of 16 columns.  Every step of a chunk keeps to
+// its columns, so a wave runs alone from barrier to barrier: the state, the right-hand side and U are accumulators (a lane
+// holds four consecutive rows of a column), and a pair of such blocks IS the operand of the next product.  Which row of 32 a
+// block's row m stands for is free: block 0 of a pair takes 8 (m / 4) + m % 4, block 1 the ones 4 further on, so that a lane's
+// eight values of a pair are consecutive and the other operand is the plain one, a 16-byte read.  What a chunk brings is copied
+// to LDS a chunk ahead, once for all columns, the keys' and queries' rows as they lie in memory; transposed keys are read
+// transposed.  A chunk's outputs are stored in the next one, so that the wait for the copies does not wait for stores just
+// issued.
+// Bound by what a wave can issue: 132 matrix and 450 vector instructions a chunk of 64 rows x 128 keys, on a SIMD with one wave
+// or two.  Left to itself the compiler reads a fragment in front of its product and waits (3.9 us a chunk with four waves), so
+// the step is laid out by hand: fragments six ahead, vector work and copies dealt between the products.  LDS is busy about 60 %
+// of the time with eight waves, as each reads the chunk's 72 KB; waves of 32 columns would halve that, but their state and
+// operands do not fit 256 registers (5.5 us a chunk instead of 4.4).  Earlier forms: operands packed by the first launch, in
+// halves of 8 bytes, no fragment ahead: 6.7 us.
+//
+// LDS: blocks of 16 rows x 32 columns, 1 KB, in operand order but for the rows: chunk (16 bytes) ch of the block's row m lies
+// at 16 ch + (m ^ 4 ch), so that the transposed reads of 4 rows x 4 chunks spread over the banks too.
+template <int D, int NW>
+__global__ __launch_bounds__(64 * NW, NW / 4 > 0 ? NW / 4 : 1) void delta_chunk_wide_kernel(hymeta_delta_rule_args a) {
+  constexpr bool Direct = NW == 2;                          // values of any alignment, read by the lanes that want them
+  constexpr int SD = D / 32, DB = D / 16, VC = 2 * NW, kRowsBytes = kChunk * D * 2, kMatBytes = 6 * 1024;
+  constexpr int kMatsAt = 2 * kRowsBytes, kScaleAt = kMatsAt + 4 * kMatBytes, kValuesAt = kScaleAt + 1024, kImage = kValuesAt + (Direct ? 0 : kChunk * 16 * VC);
+  static_assert(NW == 2 || NW == 4 || NW == 8, "the copies deal evenly over the waves");
+  typedef ChunkOrder<VC> VOrder;
+  typedef f32x4v f32x4_any __attribute__((aligned(4)));
+  __shared__ __attribute__((aligned(16))) char images[2][kImage];       // keys, queries | T hi, lo, P hi, lo | beta, rhs, read, write | values
   const int h = blockIdx.x, s = blockIdx.y, vs = blockIdx.z;
   const int r0 = a.query_start_loc[s], rows = a.query_start_loc[s + 1] - r0;
   if (rows < kChunkMinRows) return;
   const int lane = threadIdx.x & 63, n = lane & 15, g4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int H = a.num_heads, G = a.num_qk_heads, Dv = a.v_dim, g = h / (H / G), col = vs * 16 * NW + 16 * wave + n;
-  const int64_t first = r0 / kChunk + s;
-  const ChunkPlace* places = static_cast<const ChunkPlace*>(a.workspace) + first * H + h;
-  const char* packed = static_cast<const char*>(a.workspace) + rows_at(chunks, H) + (first * G + g) * kRowsBytes;
+  const int H = a.num_heads, Dv = a.v_dim, g = h / (H / a.num_qk_heads), col0 = (vs * NW + wave) * 16;
+  const ChunkPlace* places = static_cast<const ChunkPlace*>(a.workspace) + static_cast<int64_t>(r0 / kChunk + s) * H + h;
   const int num = (rows + kChunk - 1) / kChunk;
-  auto copy = [&](int c, char* image) __attribute__((always_inline)) {
-    const char* rows_from = packed + static_cast<int64_t>(c) * G * kRowsBytes + 16 * lane;
-    const char* place = reinterpret_cast<const char*>(places + static_cast<int64_t>(c) * H) + 16 * lane;
-#pragma unroll
-    for (int step = 0; step < (kCopies + NW - 1) / NW; ++step) {
-      const int i = wave + NW * step;
-      if (i >= kCopies) break;
-      // (of a lower triangular matrix the blocks of 16 rows and 32 columns that are not all zero: 0, 2, 4, 5, 6, 7)
-      const int m = i - kRowsBytes / 1024, b = m % 6;
-      const char* from = m < 0 ? rows_from + 1024 * i : m < 24 ? place + 8192 * (m / 6) + 1024 * (b < 2 ? 2 * b : b + 2) : place + 32768;
-      copy16_to_lds(from, image + 1024 * i);
+  auto row_of = [](int ib, int m) __attribute__((always_inline)) { return 32 * (ib >> 1) + 4 * (ib & 1) + 8 * (m >> 2) + (m & 3); };
+  // ---- copies: number i of a wave's; chunk c's rows past the portion's last one read that again
+  constexpr int kRowCopies = 8 * SD / NW, kMatCopies = 24 / NW, kCopies = kRowCopies + kMatCopies + (Direct ? 0 : 2) + 1;
+  const int ch = lane >> 4, m = (lane & 15) ^ (4 * ch);     // this lane's place in a block: row m, chunk ch
+  const uint32_t mat_lane = (m >> 3) * 2048 + (8 * ((m >> 2) & 1) + (m & 3)) * 16 + ch * 256;
+  const int k_stride = static_cast<int>(a.k_stride_t), q_stride = static_cast<int>(a.q_stride_t), v_stride = static_cast<int>(a.v_stride_t);
+  struct Source { const char *k, *q, *v, *place; int last; };
+  auto source = [&](int c) __attribute__((always_inline)) {
+    const int64_t t0 = r0 + static_cast<int64_t>(c) * kChunk;
+    return Source{reinterpret_cast<const char*>(static_cast<const uint16_t*>(a.k) + t0 * a.k_stride_t + static_cast<int64_t>(g) * D),
+                  reinterpret_cast<const char*>(static_cast<const uint16_t*>(a.q) + t0 * a.q_stride_t + static_cast<int64_t>(g) * D),
+                  reinterpret_cast<const char*>(static_cast<const uint16_t*>(a.v) + t0 * a.v_stride_t + static_cast<int64_t>(h) * Dv + vs * 8 * VC),
+                  reinterpret_cast<const char*>(places + static_cast<int64_t>(c) * H), rows - 1 - c * kChunk};
+  };
+  auto copy = [&](const Source& from, char* image, int i) __attribute__((always_inline)) {
+    if (i < kRowCopies) {                                   // 16 rows x 32 columns of the keys or the queries
+      const int sd = i % SD, block = wave + NW * (i / SD), ib = block & 3, row = min(row_of(ib, m), from.last);
+      const bool keys = block < 4;
+      copy16_to_lds((keys ? from.k : from.q) + 64 * sd, 2 * (__umul24(row, keys ? k_stride : q_stride) + 8 * ch), image + (keys ? 0 : kRowsBytes) + 1024 * (ib * SD + sd));
+    } else if (i < kRowCopies + kMatCopies) {               // a lower triangular matrix's blocks of 16 x 32 that are not all zero
+      const int j = kMatCopies * wave + i - kRowCopies, which = j / 6, b = j % 6, ib = b < 2 ? b : b / 2 + 1, kk = b < 2 ? 0 : b & 1;
+      copy16_to_lds(from.place + 8192 * which + 4096 * (ib >> 1) + 64 * (ib & 1) + 1024 * kk, mat_lane, image + kMatsAt + 1024 * j);
+    } else if (i < kCopies - 1) {                           // rows of the slice's values
+      const int j = wave + NW * (i - kRowCopies - kMatCopies), row = (64 * j + lane) / VC;
+      copy16_to_lds(from.v, 2 * __umul24(min(row, from.last), v_stride) + 16 * ((lane % VC) ^ VOrder::twist(row)), image + kValuesAt + 1024 * j);
+    } else if (wave == 0) {
+      copy16_to_lds(from.place + 32768, 16 * lane, image + kScaleAt);
     }
   };
-  const uint16_t* vp = static_cast<const uint16_t*>(a.v) + static_cast<int64_t>(h) * Dv + vs * 16 * NW;
-  const int v_stride = static_cast<int>(a.v_stride_t), HDv = H * Dv;
-  uint32_t vv[4][4];
+  uint32_t vv[4][4];                                        // Direct: values of rows row_of(ib, 4 g4 + r)
   float total = 0.f;
-  auto fetch = [&](int c) __attribute__((always_inline)) {
-    const int last = rows - 1 - c * kChunk;
-    const int64_t t0 = r0 + static_cast<int64_t>(c) * kChunk;
+  auto fetch = [&](const Source& from) __attribute__((always_inline)) {
+    if constexpr (Direct) {
 #pragma unroll
-    for (int ib = 0; ib < 4; ++ib)
+      for (int ib = 0; ib < 4; ++ib)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) vv[ib][r] = vp[t0 * a.v_stride_t + static_cast<uint32_t>(min(16 * ib + 4 * g4 + r, last) * v_stride + 16 * wave + n)];
-    total = places[static_cast<int64_t>(c) * H].total;
+        for (int r = 0; r < 4; ++r)
+          vv[ib][r] = reinterpret_cast<const uint16_t*>(from.v)[__umul24(min(row_of(ib, 4 * g4 + r), from.last), v_stride) + 16 * wave + n];
+    }
+    total = reinterpret_cast<const ChunkPlace*>(from.place)->total;
   };
-  copy(0, images[0]);
-  fetch(0);
-  const int slot = a.slot_idx[s];
-  float* st = slot >= 0 ? a.state + (static_cast<int64_t>(slot) * H + h) * D * Dv + col : nullptr;
+  {
+    const Source from = source(0);
+#pragma unroll
+    for (int i = 0; i < kCopies; ++i) copy(from, images[0], i);
+    fetch(from);
+  }
+  const int slot_ = a.slot_idx[s];
+  float* st = slot_ >= 0 ? a.state + (static_cast<int64_t>(slot_) * H + h) * D * Dv + col0 + n : nullptr;
   const bool carry = st != nullptr && a.context_lens[s] > 0;
-  f32x4v S[DB];
+  f32x4v S[DB];                                             // rows d row_of(db, 4 g4 + r) of its pair's 32, column n
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) S[db][r] = carry ? st[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv] : 0.f;
-  const int half = ((g4 >> 1) * 16 + n) * 16 + 8 * (g4 & 1);             // this lane's first half of a 1 KB operand block
-  auto operand = [&](const char* block) {
-    const u32x2 x = *reinterpret_cast<const u32x2*>(block + half), y = *reinterpret_cast<const u32x2*>(block + half + 512);
-    return frag(u32x4{x[0], x[1], y[0], y[1]});
+    for (int r = 0; r < 4; ++r) S[db][r] = carry ? st[static_cast<int64_t>(row_of(db, 4 * g4 + r)) * Dv] : 0.f;
+  const int place_of = 16 * (16 * g4 + (n ^ (4 * g4)));     // this lane's 16 bytes of an operand block
+  auto operand = [&](const char* block) __attribute__((always_inline)) { return ld16(block + place_of); };
+  // transposed keys: rows 32 kk + 8 g4 + e of the chunk (positions 4 g4 .. of the blocks 2 kk, 2 kk + 1), column n of block db
+  const int across = 16 * (16 * (n & 3) + ((4 * g4 + (n >> 2)) ^ (4 * (n & 3))));
+  auto transposed = [&](const char* keys, int db, int kk) __attribute__((always_inline)) {
+    const char* p = keys + 1024 * (2 * kk * SD + (db >> 1)) + 8 * (db & 1) + across;
+    const u32x2 x = __builtin_bit_cast(u32x2, read_transposed(p)), y = __builtin_bit_cast(u32x2, read_transposed(p + 1024 * SD));
+    return u32x4{x[0], x[1], y[0], y[1]};
   };
-  auto split8 = [&](const f32x4v& x, const f32x4v& y, bf16x8& hi, bf16x8& lo) {
-    const float p[4] = {x[0], x[1], x[2], x[3]}, q[4] = {y[0], y[1], y[2], y[3]};
-    u32x2 ph, pl, qh, ql;
-    split4(p, ph, pl), split4(q, qh, ql);
-    hi = frag(u32x4{ph[0], ph[1], qh[0], qh[1]}), lo = frag(u32x4{pl[0], pl[1], ql[0], ql[1]});
+  // values: rows row_of(ib, 4 g4 + r), r < 4, of column n, in pairs
+  auto value_at = [&](const char* values, int ib) __attribute__((always_inline)) {
+    const int row = row_of(ib, 4 * g4 + (n >> 2)), chunk = 2 * wave + ((n >> 1) & 1);
+    return __builtin_bit_cast(u32x2, read_transposed(values + row * 16 * VC + 16 * (chunk ^ VOrder::twist(row)) + 8 * (n & 1)));
   };
-  float* out = static_cast<float*>(a.out) + static_cast<int64_t>(r0) * HDv + static_cast<int64_t>(h) * Dv + vs * 16 * NW;
-  f32x4v y[4];
-  auto store = [&](int c, auto full) __attribute__((always_inline)) {
-    const int live = rows - c * kChunk;
+  f32x4v x[4], y[4];                        // right-hand side, then U; the outputs: columns 4 g4 + r of row row_of(ib, n)
+  bf16x8 sh[SD], sl[SD], hi[2], lo[2], wh[2], wl[2];
+  // four values as half of an operand's parts (block ib of pairs)
+  auto split_half = [&](const f32x4v& v, int ib, bf16x8& to_hi, bf16x8& to_lo) __attribute__((always_inline)) {
+    const float p[4] = {v[0], v[1], v[2], v[3]};
+    u32x2 ph, pl;
+    split4(p, ph, pl);
+    u32x4 h4 = __builtin_bit_cast(u32x4, to_hi), l4 = __builtin_bit_cast(u32x4, to_lo);
+    h4[2 * (ib & 1)] = ph[0], h4[2 * (ib & 1) + 1] = ph[1], l4[2 * (ib & 1)] = pl[0], l4[2 * (ib & 1) + 1] = pl[1];
+    to_hi = frag(h4), to_lo = frag(l4);
+  };
+  auto split_state = [&](int i) __attribute__((always_inline)) { split_half(S[i], i, sh[i / 2], sl[i / 2]); };
 #pragma unroll
-    for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = 16 * ib + 4 * g4 + r;
-        if (decltype(full)::value || i < live) out[static_cast<int64_t>(c) * kChunk * HDv + static_cast<uint32_t>(i * HDv + 16 * wave + n)] = y[ib][r];
-      }
+  for (int i = 0; i < DB; ++i) split_state(i);
+  const int64_t row_floats = static_cast<int64_t>(H) * Dv;
+  float* out = static_cast<float*>(a.out) + static_cast<int64_t>(r0) * row_floats + static_cast<int64_t>(h) * Dv + col0 + 4 * g4;
+  auto store = [&](int c, int ib, int live) __attribute__((always_inline)) {
+    const int row = row_of(ib, n);
+    float* to = out + static_cast<int64_t>(c) * kChunk * row_floats + __umul24(row, static_cast<int>(row_floats));
+    if (row < live) *reinterpret_cast<f32x4_any*>(to) = y[ib];
   };
   for (int c = 0; c < num; ++c) {
     const char* image = images[c & 1];
+    char* next = images[(c + 1) & 1];
+    const Source from = source(min(c + 1, num - 1));        // (the last chunk fetches itself once more: no copy under a condition)
     copies_landed_barrier();                 // this chunk's image is there, the other's readers are done
     // what the compiler still counts as in flight has landed: it is used here, in front of the next copies, which it would
     // otherwise wait for as well
-    float value[4][4], decay = total;
-#pragma unroll
-    for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        value[ib][r] = bf2f(static_cast<uint16_t>(vv[ib][r]));
-        asm volatile("" : "+v"(value[ib][r]));
-      }
+    float decay = total;
     asm volatile("" : "+v"(decay));
-    if (c > 0) store(c - 1, std::true_type{});
-    if (c + 1 < num) {
-      copy(c + 1, images[(c + 1) & 1]);
-      fetch(c + 1);
+    if constexpr (Direct) {
+#pragma unroll
+      for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(vv[ib][r]));
     }
-    const char *keys = image, *queries = image + D * kChunk * 2, *transposed = image + 2 * D * kChunk * 2, *mats = image + kRowsBytes;
-    const float* scale = reinterpret_cast<const float*>(mats + 4 * kMatBytes) + 4 * g4;      // beta, rhs, read, write of rows 4 g4 ..
-    f32x4v x[4];
-#pragma unroll
-    for (int ib = 0; ib < 4; ++ib) x[ib] = y[ib] = f32x4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int sd = 0; sd < SD; ++sd) {
-      bf16x8 sh, sl;
-      split8(S[2 * sd], S[2 * sd + 1], sh, sl);
-#pragma unroll
-      for (int ib = 0; ib < 4; ++ib) {
-        const bf16x8 kf = operand(keys + 1024 * (ib * SD + sd)), qf = operand(queries + 1024 * (ib * SD + sd));
-        x[ib] = mfma16(kf, sh, x[ib]);
-        y[ib] = mfma16(qf, sh, y[ib]);
-        x[ib] = mfma16(kf, sl, x[ib]);
-        y[ib] = mfma16(qf, sl, y[ib]);
-      }
-    }
-#pragma unroll
-    for (int ib = 0; ib < 4; ++ib) {
-      const f32x4v beta = *reinterpret_cast<const f32x4v*>(scale + 16 * ib), rhs = *reinterpret_cast<const f32x4v*>(scale + kChunk + 16 * ib);
-      const f32x4v read = *reinterpret_cast<const f32x4v*>(scale + 2 * kChunk + 16 * ib);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) x[ib][r] = beta[r] * value[ib][r] - rhs[r] * x[ib][r];
-      y[ib] *= read;
-    }
-    // U = T x right-hand side; then U and U times the rows' write factors as operands
-    f32x4v u[4];
-    bf16x8 hi[2], lo[2], wh[2], wl[2];
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) split8(x[2 * kk], x[2 * kk + 1], hi[kk], lo[kk]);
-    auto lower = [&](int matrix, f32x4v* to) __attribute__((always_inline)) {
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-        for (int ib = 2 * kk; ib < 4; ++ib) {
-          const char* block = mats + 2 * matrix * kMatBytes + 1024 * (ib < 2 ? ib : 2 * ib - 2 + kk);
-          const bf16x8 mh = operand(block), ml = operand(block + kMatBytes);
-          to[ib] = mfma16(mh, hi[kk], to[ib]);
-          to[ib] = mfma16(mh, lo[kk], to[ib]);
-          to[ib] = mfma16(ml, hi[kk], to[ib]);
-        }
+    const char *keys = image, *queries = image + kRowsBytes, *mats = image + kMatsAt;
+    // beta, rhs, write of this lane's rows of block ib
+    auto scale = [&](int which, int ib) __attribute__((always_inline)) {
+      return *reinterpret_cast<const f32x4v*>(image + kScaleAt + 4 * (kChunk * which + 32 * (ib >> 1) + 4 * (ib & 1) + 8 * g4));
     };
+    // Fragments in the order of their use, four to a slot, read kAhead of them ahead: keys (slots of 32 columns), half of the
+    // queries, T, the other queries, transposed keys, P.
+    constexpr int kQa = SD / 2, kT = SD + kQa, kQb = kT + 3, kK = kQb + SD - kQa, kP = kK + SD, kSlots = kP + 3, kAhead = 6;
+    u32x4 fr[4 * kSlots + kAhead];
+    auto read = [&](int f) __attribute__((always_inline)) {
+      const int slot = f / 4, i = f % 4;
+      auto matrix = [&](int which, int pair) __attribute__((always_inline)) {       // blocks (0, 0) (1, 0), (2, 0) (3, 0), (2, 1) (3, 1): hi, then lo
+        const int ib = (pair == 0 ? 0 : 2) + (i & 1), kk = pair == 2;
+        return operand(mats + kMatBytes * (2 * which + (i >> 1)) + 1024 * (ib < 2 ? ib : 2 * ib - 2 + kk));
+      };
+      if (slot < SD) fr[f] = operand(keys + 1024 * (i * SD + slot));
+      else if (slot < kT) fr[f] = operand(queries + 1024 * (i * SD + slot - SD));
+      else if (slot < kQb) fr[f] = matrix(0, slot - kT);
+      else if (slot < kK) fr[f] = operand(queries + 1024 * (i * SD + slot - kQb + kQa));
+      else if (slot < kP) fr[f] = transposed(keys, 2 * (slot - kK) + (i & 1), i >> 1);
+      else if (slot < kSlots) fr[f] = matrix(1, slot - kP);
+    };
+    // pieces of other work of `count`, dealt evenly over the steps [0, of) of a phase
+    auto pieces = [&](int step, int of, int count, auto&& piece) __attribute__((always_inline)) {
 #pragma unroll
-    for (int ib = 0; ib < 4; ++ib) u[ib] = f32x4v{0.f, 0.f, 0.f, 0.f};
-    lower(0, u);
+      for (int i = step * count / of; i < (step + 1) * count / of; ++i) piece(i);
+    };
+    // the next chunk's copies, dealt over the steps (products) up to the middle of the state's update: issued side by side they
+    // hold the wave up (25 cycles of the compute unit's address path each)
+    auto copies = [&](int step) __attribute__((always_inline)) {
+      pieces(step, 20 * SD + 18, kCopies, [&](int i) __attribute__((always_inline)) { if (i < kCopies) copy(from, next, i); });
+    };
+    f32x4v beta[4], rhs[4], write[4];
+    u32x2 value[4];
+    float reads[4];
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      split8(u[2 * kk], u[2 * kk + 1], hi[kk], lo[kk]);
-      const f32x4v w0 = *reinterpret_cast<const f32x4v*>(scale + 3 * kChunk + 32 * kk), w1 = *reinterpret_cast<const f32x4v*>(scale + 3 * kChunk + 32 * kk + 16);
-      split8(u[2 * kk] * w0, u[2 * kk + 1] * w1, wh[kk], wl[kk]);
-    }
+    for (int f = 0; f < kAhead; ++f) read(f);
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
-      f32x4v acc = S[db] * decay;
+    for (int ib = 0; ib < 4; ++ib) x[ib] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    auto right_hand_side = [&](int b) __attribute__((always_inline)) {
+      const float v[4] = {lo_bf(value[b][0]), hi_bf(value[b][0]), lo_bf(value[b][1]), hi_bf(value[b][1])};
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        const bf16x8 kt = operand(transposed + 1024 * (2 * db + kk));
-        acc = mfma16(kt, wh[kk], acc);
-        acc = mfma16(kt, wl[kk], acc);
+      for (int r = 0; r < 4; ++r) x[b][r] = beta[b][r] * v[r] - rhs[b][r] * x[b][r];
+      split_half(x[b], b, hi[b >> 1], lo[b >> 1]);
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    unrolled<kSlots>([&](auto number) __attribute__((always_inline)) {
+      constexpr int slot = decltype(number)::value;
+#pragma unroll
+      for (int f = 4 * slot + kAhead; f < 4 * slot + 4 + kAhead; ++f) read(f);
+      const u32x4* fs = fr + 4 * slot;
+      if constexpr (slot == SD) {
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) y[ib] = f32x4v{0.f, 0.f, 0.f, 0.f};
+        if constexpr (kQa == 0) {                           // (a head of 32: the right-hand side in front of T)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) right_hand_side(i);
+        }
       }
-      S[db] = acc;
-    }
-    lower(1, y);
+      if constexpr (slot == kT) {
+        if constexpr (Direct) fetch(from);
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) x[ib] = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) write[ib] = scale(3, ib), reads[ib] = *reinterpret_cast<const float*>(image + kScaleAt + 4 * (2 * kChunk + row_of(ib, n)));
+      }
+      if constexpr (slot == SD - 1) {
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) {
+          beta[ib] = scale(0, ib), rhs[ib] = scale(1, ib);
+          if constexpr (Direct) value[ib] = u32x2{vv[ib][0] | (vv[ib][1] << 16), vv[ib][2] | (vv[ib][3] << 16)};
+          else value[ib] = value_at(image + kValuesAt, ib);
+        }
+      }
+      if constexpr (slot < kT || (slot >= kQb && slot < kK)) {        // keys times the state; the state times queries, transposed
+        constexpr int sd = slot < SD ? slot : slot < kT ? slot - SD : slot - kQb + kQa;
+#pragma unroll
+        for (int part = 0; part < 2; ++part)
+#pragma unroll
+          for (int ib = 0; ib < 4; ++ib) {
+            const bf16x8 state = part == 0 ? sh[sd] : sl[sd];
+            if constexpr (slot < SD) x[ib] = mfma16(frag(fs[ib]), state, x[ib]);
+            else y[ib] = mfma16(state, frag(fs[ib]), y[ib]);
+            constexpr int from_step = 8 * (slot < SD ? slot : slot < kT ? slot - SD : slot - kQb);
+            const int step = from_step + 4 * part + ib;
+            copies((slot < kT ? 0 : 8 * kT + 18) + from_step + (slot >= SD && slot < kT ? 8 * SD : 0) + 4 * part + ib);
+            if constexpr (slot < SD) {
+              pieces(step, 4 * SD, 4, [&](int i) __attribute__((always_inline)) {
+                if (i < 4 && c > 0) store(c - 1, i, kChunk);
+              });
+            } else if constexpr (slot < kT) pieces(step, 8 * kQa, 4, right_hand_side);
+            else {
+              pieces(step, 8 * (SD - kQa), 4, [&](int b) __attribute__((always_inline)) { split_half(x[b] * write[b], b, wh[b >> 1], wl[b >> 1]); });
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+      } else if constexpr (slot < kQb || slot >= kP) {      // T times the right-hand side; U times P, transposed
+        constexpr int pair = slot < kQb ? slot - kT : slot - kP, kk = pair == 2;
+#pragma unroll
+        for (int part = 0; part < 3; ++part) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int ib = (pair == 0 ? 0 : 2) + i;
+            const bf16x8 mat = frag(fs[part == 2 ? 2 + i : i]), other = part == 1 ? lo[kk] : hi[kk];
+            if constexpr (slot < kQb) x[ib] = mfma16(mat, other, x[ib]), copies(8 * kT + 6 * pair + 2 * part + i);
+            else y[ib] = mfma16(other, mat, y[ib]);
+            if constexpr (slot >= kP) pieces(6 * pair + 2 * part + i, 18, DB, split_state);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        if constexpr (slot == kT && !Direct) fetch(from);
+      } else {                                              // the state's update, two blocks at a time
+        constexpr int db = 2 * (slot - kK);
+        f32x4v acc[2] = {S[db] * decay, S[db + 1] * decay};
+#pragma unroll
+        for (int part = 0; part < 4; ++part)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            acc[i] = mfma16(frag(fs[2 * (part >> 1) + i]), part & 1 ? wl[part >> 1] : wh[part >> 1], acc[i]);
+            copies(8 * 2 * SD + 18 + 8 * (slot - kK) + 2 * part + i);
+            pieces(8 * (slot - kK) + 2 * part + i, 8 * SD, 4, [&](int b) __attribute__((always_inline)) {
+              split_half(x[b], b, hi[b >> 1], lo[b >> 1]);
+              y[b] *= reads[b];
+            });
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        S[db] = acc[0], S[db + 1] = acc[1];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
   }
-  store(num - 1, std::false_type{});
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // (the last copies, which nobody waits for, end before the workgroup)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) store(num - 1, i, rows - (num - 1) * kChunk);
   if (st != nullptr) {
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) st[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv] = S[db][r];
+      for (int r = 0; r < 4; ++r) st[static_cast<int64_t>(row_of(db, 4 * g4 + r)) * Dv] = S[db][r];
   }
 }
 
@@ -810,7 +930,9 @@ inline bool chunk_dims(int head_dim, int v_dim, int act_dtype) {
 }
 inline bool chunk_shape(const hymeta_delta_rule_args& a) {
   auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  return chunk_dims(a.head_dim, a.v_dim, a.act_dtype) && a.q_stride_t % 8 == 0 && a.k_stride_t % 8 == 0 && aligned(a.q) && aligned(a.k);
+  // (a chunk's rows at 24-bit products of row and stride)
+  const bool offsets = std::max(a.q_stride_t, std::max(a.k_stride_t, a.v_stride_t)) < (1 << 23) && static_cast<int64_t>(a.num_heads) * a.v_dim < (1 << 22);
+  return chunk_dims(a.head_dim, a.v_dim, a.act_dtype) && offsets && a.q_stride_t % 8 == 0 && a.k_stride_t % 8 == 0 && aligned(a.q) && aligned(a.k);
 }
 inline int64_t chunk_numbers(int num_tokens, int num_seqs) { return static_cast<int64_t>(num_tokens) / kChunk + num_seqs; }
 
@@ -831,23 +953,29 @@ void launch_rows(const hymeta_delta_rule_args& a, hipStream_t st, int min_rows, 
 }
 
 template <int D>
-void launch_chunks(const hymeta_delta_rule_args& a, hipStream_t st, int64_t chunks) {
-  hipLaunchKernelGGL(delta_chunk_solve_kernel<D>, dim3(static_cast<unsigned>(chunks), a.num_heads), dim3(256), 0, st, a, chunks);
-  // slices of 32 columns reread a chunk's matrices half as often; slices of 16 double the workgroups where they are few.  Few
-  // and many of those that have work for the time the longest takes: single rows and short portions end at once or soon
+void launch_chunks(const hymeta_delta_rule_args& a, hipStream_t st, int64_t chunks, bool short_too) {
   const int64_t portions = long_portions(a.num_tokens, a.num_seqs, a.max_query_len), lanes = a.num_heads * portions;
   const int64_t idle = a.num_heads * (a.num_seqs - portions) * (a.v_dim / 32);
+  const bool narrow = D % 64 == 0 && lanes * (a.v_dim / 32) <= kFewGroups && idle <= static_cast<int64_t>(kIdleGroupsPerRow) * a.max_query_len;
+  const dim3 solve(static_cast<unsigned>(chunks), a.num_heads);
   if constexpr (D % 64 == 0) {
-    if (lanes * (a.v_dim / 32) <= kFewGroups && idle <= static_cast<int64_t>(kIdleGroupsPerRow) * a.max_query_len) {
-      hipLaunchKernelGGL((delta_chunk_scan_kernel<D, 1>), dim3(a.num_heads, a.num_seqs, a.v_dim / 16), dim3(256), 0, st, a, chunks);
+    if (narrow && a.max_query_len >= kChunkMinRows) {
+      hipLaunchKernelGGL((delta_chunk_solve_kernel<D, true>), solve, dim3(256), 0, st, a, chunks, short_too ? 1 : 0);
+      hipLaunchKernelGGL(delta_chunk_narrow_kernel<D>, dim3(a.num_heads, a.num_seqs, a.v_dim / 16), dim3(256), 0, st, a, chunks);
       return;
     }
   }
-  if (a.v_dim % 128 == 0 && lanes * (a.v_dim / 128) > kManyWideGroups && a.v_stride_t < (1 << 23) && static_cast<int64_t>(a.num_heads) * a.v_dim < (1 << 22)) {
-    hipLaunchKernelGGL((delta_chunk_wide_kernel<D>), dim3(a.num_heads, a.num_seqs, a.v_dim / 128), dim3(512), 0, st, a, chunks);
-    return;
-  }
-  hipLaunchKernelGGL((delta_chunk_scan_kernel<D, 2>), dim3(a.num_heads, a.num_seqs, a.v_dim / 32), dim3(256), 0, st, a, chunks);
+  hipLaunchKernelGGL((delta_chunk_solve_kernel<D, false>), solve, dim3(256), 0, st, a, chunks, short_too ? 1 : 0);
+  if (a.max_query_len < kChunkMinRows) return;
+  auto launch = [&](auto nw) {
+    constexpr int NW = decltype(nw)::value;
+    hipLaunchKernelGGL((delta_chunk_wide_kernel<D, NW>), dim3(a.num_heads, a.num_seqs, a.v_dim / (16 * NW)), dim3(64 * NW), 0, st, a);
+  };
+  using std::integral_constant;
+  const bool aligned = a.v_stride_t % 8 == 0 && reinterpret_cast<uintptr_t>(a.v) % 16 == 0;      // (values copied to LDS)
+  if (aligned && a.v_dim % 128 == 0 && lanes * (a.v_dim / 64) > kManyGroups) launch(integral_constant<int, 8>{});
+  else if (aligned && a.v_dim % 64 == 0) launch(integral_constant<int, 4>{});
+  else launch(integral_constant<int, 2>{});
 }
 
 }  // namespace
@@ -881,19 +1009,18 @@ extern "C" int hymeta_delta_rule(const hymeta_delta_rule_args* args, hymeta_stre
   }
   hipStream_t st = begin_launches(stream);
   const bool bf = a.act_dtype == HYMETA_BF16;
-  int max_rows = 0x7fffffff;
-  if (chunk_shape(a) && a.max_query_len >= kChunkMinRows) {
+  int min_rows = 1, max_rows = 0x7fffffff;
+  if (chunk_shape(a) && a.max_query_len >= (step ? 2 : kChunkMinRows)) {
     const size_t need = hymeta_delta_rule_workspace_bytes(a.num_tokens, a.num_seqs, a.num_heads, a.num_qk_heads, a.head_dim, a.v_dim, a.act_dtype, a.max_query_len);
-    if (!a.workspace || a.workspace_bytes < need || reinterpret_cast<uintptr_t>(a.workspace) % 16 != 0) return HYMETA_ERR_WORKSPACE;
+    if (need > 0 && (!a.workspace || a.workspace_bytes < need || reinterpret_cast<uintptr_t>(a.workspace) % 16 != 0)) return HYMETA_ERR_WORKSPACE;
     const int64_t chunks = chunk_numbers(a.num_tokens, a.num_seqs);
-    if (a.head_dim == 32) launch_chunks<32>(a, st, chunks);
-    else if (a.head_dim == 64) launch_chunks<64>(a, st, chunks);
-    else if (a.head_dim == 96) launch_chunks<96>(a, st, chunks);
-    else launch_chunks<128>(a, st, chunks);
+    if (a.head_dim == 32) launch_chunks<32>(a, st, chunks, step);
+    else if (a.head_dim == 64) launch_chunks<64>(a, st, chunks, step);
+    else if (a.head_dim == 96) launch_chunks<96>(a, st, chunks, step);
+    else launch_chunks<128>(a, st, chunks, step);
+    if (step) return launch_status();
     max_rows = kChunkMinRows - 1;
-  }
-  int min_rows = 1;
-  if (step) {
+  } else if (step) {
     const dim3 grid(a.num_heads, a.num_seqs), block(256);
     if (a.norm_weight) {
       if (bf) hipLaunchKernelGGL((delta_rule_step_kernel<ActBf16, true>), grid, block, 0, st, a);
