@@ -1,0 +1,57 @@
+"""Portions too short for a chunk of the lightning attention and the decay scan, beside longer ones and alone: against the
+recurrence in 64 bits."""
+import pytest
+import torch
+
+from _util import gen
+
+pytestmark = pytest.mark.gpu
+MIXED = [7, 1, 8, 2, 65, 3, 1, 130, 6]
+
+
+def _recurrence(q, k, v, w, decay, state, starts, context, slots):
+    out, states = [], state.double().clone()
+    for s in range(len(starts) - 1):
+        S = states[slots[s]].clone() if slots[s] >= 0 and context[s] > 0 else torch.zeros_like(states[0])
+        for t in range(starts[s], starts[s + 1]):
+            S = S * decay[t][:, None, None] + k[t][:, :, None] * w[t][:, None]
+            out.append((S * q[t][:, :, None]).sum(1))
+        if slots[s] >= 0:
+            states[slots[s]] = S
+    return torch.stack(out), states
+
+
+@pytest.mark.parametrize("silu", [True, False])
+@pytest.mark.parametrize("D,Dv,H,lens", [
+    (128, 128, 14, MIXED + [100] * 6), (64, 64, 4, MIXED), (32, 96, 4, MIXED), (128, 256, 4, [2, 7, 1, 3]),
+    (64, 128, 2, [700, 1, 5, 300]),               # cut into segments
+])
+def test_short_portions(D, Dv, H, lens, silu):
+    """Rows of portions of up to 7 stay in fp32: 1e-6 of the norm.  The others' operands enter as two bf16 parts, 2e-5, behind a
+    silu rounded to bf16 on the way, 3e-3."""
+    from vllm_hymeta import hip_ops
+    T, n, g = sum(lens), len(lens), gen(D + Dv + silu)
+    Hk = H if silu else H // 2
+    qkv = torch.randn(T, 2 * Hk * D + H * Dv, generator=g).bfloat16()
+    q, k, v = (x.unflatten(1, (h, d)) for x, h, d in zip(qkv.split([Hk * D, Hk * D, H * Dv], 1), (Hk, Hk, H), (D, D, Dv)))
+    state, decay = torch.randn(n, H, D, Dv, generator=g) * 0.1, 1 - torch.rand(H, generator=g) * 0.1
+    l2, b, skip = -torch.rand(T, H, generator=g) * 0.2, torch.rand(T, H, generator=g), torch.randn(H, generator=g)
+    starts, context, slots = [sum(lens[:i]) for i in range(n + 1)], [5 * (i % 2) for i in range(n)], [i if i != 3 else -1 for i in range(n)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    got, dev, where = state.cuda(), qkv.cuda(), (i32(starts), i32(context), i32(slots), max(lens))
+    if silu:
+        out = hip_ops.lightning_attention(dev, got, decay.cuda(), H, D, Dv, *where)
+        act = torch.nn.functional.silu
+        want, states = _recurrence(act(q.double()), act(k.double()), act(v.double()), act(v.double()), decay.double().expand(T, H), state, starts, context, slots)
+    else:
+        dq, dk, dv = (x.unflatten(1, (h, d)) for x, h, d in zip(dev.split([Hk * D, Hk * D, H * Dv], 1), (Hk, Hk, H), (D, D, Dv)))
+        out = hip_ops.decay_scan(dq, dk, dv, got, *where, log2_decay=l2.cuda(), v_scale=b.cuda(), skip=skip.cuda())
+        qd, kd, vd = q.double().repeat_interleave(2, 1), k.double().repeat_interleave(2, 1), v.double()
+        want, states = _recurrence(qd, kd, vd, vd * b.double()[:, :, None], torch.exp2(l2.double()), state, starts, context, slots)
+        want = want + skip.double()[None, :, None] * vd
+    out, got = out.view(T, H, Dv).double().cpu(), got.double().cpu()
+    for s in range(n):
+        rows, bound = slice(starts[s], starts[s + 1]), 1e-6 if lens[s] < 8 else 3e-3 if silu else 2e-5
+        assert float((out[rows] - want[rows]).norm() / want[rows].norm()) < bound, s
+        assert slots[s] < 0 or float((got[s] - states[s]).norm() / states[s].norm()) < bound, s
+    assert torch.equal(got[3], state[3].double())

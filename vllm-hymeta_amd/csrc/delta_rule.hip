@@ -97,11 +97,12 @@ __device__ __forceinline__ void delta_rows(const hymeta_delta_rule_args& a, int 
   const int slot = a.slot_idx[s];
   float* st = slot >= 0 ? a.state + ((static_cast<int64_t>(slot) * H + h) * D) * Dv : nullptr;
   const bool carry = st != nullptr && a.context_lens[s] > 0;
+  const uint32_t lane_at = d0 * Dv + 4 * c4;                      // (rows of S further on: a wave-uniform step)
   f32x4 S[kStepRows];
 #pragma unroll
   for (int u = 0; u < kStepRows; ++u) {
     const int d = d0 + u * dstep;
-    S[u] = (carry && d < D) ? *reinterpret_cast<const f32x4*>(st + static_cast<int64_t>(d) * Dv + 4 * c4) : f32x4{0.f, 0.f, 0.f, 0.f};
+    S[u] = (carry && d < D) ? *reinterpret_cast<const f32x4*>(st + u * dstep * Dv + lane_at) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   for (int t = t0; t < t1; ++t) {
     const elem* q = static_cast<const elem*>(a.q) + static_cast<int64_t>(t) * a.q_stride_t + static_cast<int64_t>(g) * D;
@@ -156,7 +157,7 @@ __device__ __forceinline__ void delta_rows(const hymeta_delta_rule_args& a, int 
         const float kd = m.k[d];
 #pragma unroll
         for (int e = 0; e < 4; ++e) S[u][e] = fmaf(decay, S[u][e], kd * u4[e]);
-        if (st != nullptr && t + 1 == t1) *reinterpret_cast<f32x4*>(st + static_cast<int64_t>(d) * Dv + 4 * c4) = S[u];
+        if (st != nullptr && t + 1 == t1) *reinterpret_cast<f32x4*>(st + u * dstep * Dv + lane_at) = S[u];
       }
     }
     const int64_t at = (static_cast<int64_t>(t) * H + h) * Dv;
@@ -216,6 +217,9 @@ constexpr int kChunk = HYMETA_DELTA_CHUNK;
 // 177 us, 301 before; five of 1801 (280, in slices of 128) 182, 280 before.
 // All count the portions that the step's rows are worth (long_portions): single rows leave the chip to a long prompt.
 constexpr int kFewGroups = 128, kIdleGroupsPerRow = 10, kManyGroups = 256;
+// (head, short portion) pairs up to which those run in the first launch and not in their own, which have more workgroups on a
+// compute unit: 28 heads, 2048 rows beside 63 single ones (1764 pairs) 129 against 141 us, 40 beside 255 (7140) 246 against 230.
+constexpr int kManyShort = 4096;
 constexpr int kChunkMinRows = 8;            // shorter portions go token by token
 constexpr int kMat = kChunk * kChunk;
 // Where the second launch reads 64 x 64 matrices (or the chunk's keys) as matrix operands, they lie in the operand's own
@@ -1010,17 +1014,20 @@ extern "C" int hymeta_delta_rule(const hymeta_delta_rule_args* args, hymeta_stre
   hipStream_t st = begin_launches(stream);
   const bool bf = a.act_dtype == HYMETA_BF16;
   int min_rows = 1, max_rows = 0x7fffffff;
-  if (chunk_shape(a) && a.max_query_len >= (step ? 2 : kChunkMinRows)) {
+  const int64_t idle = static_cast<int64_t>(a.num_heads) * (a.num_seqs - long_portions(a.num_tokens, a.num_seqs, a.max_query_len));
+  const bool short_too = step && idle <= kManyShort;
+  if (chunk_shape(a) && a.max_query_len >= (short_too ? 2 : kChunkMinRows)) {
     const size_t need = hymeta_delta_rule_workspace_bytes(a.num_tokens, a.num_seqs, a.num_heads, a.num_qk_heads, a.head_dim, a.v_dim, a.act_dtype, a.max_query_len);
     if (need > 0 && (!a.workspace || a.workspace_bytes < need || reinterpret_cast<uintptr_t>(a.workspace) % 16 != 0)) return HYMETA_ERR_WORKSPACE;
     const int64_t chunks = chunk_numbers(a.num_tokens, a.num_seqs);
-    if (a.head_dim == 32) launch_chunks<32>(a, st, chunks, step);
-    else if (a.head_dim == 64) launch_chunks<64>(a, st, chunks, step);
-    else if (a.head_dim == 96) launch_chunks<96>(a, st, chunks, step);
-    else launch_chunks<128>(a, st, chunks, step);
-    if (step) return launch_status();
+    if (a.head_dim == 32) launch_chunks<32>(a, st, chunks, short_too);
+    else if (a.head_dim == 64) launch_chunks<64>(a, st, chunks, short_too);
+    else if (a.head_dim == 96) launch_chunks<96>(a, st, chunks, short_too);
+    else launch_chunks<128>(a, st, chunks, short_too);
+    if (short_too) return launch_status();
     max_rows = kChunkMinRows - 1;
-  } else if (step) {
+  }
+  if (step) {
     const dim3 grid(a.num_heads, a.num_seqs), block(256);
     if (a.norm_weight) {
       if (bf) hipLaunchKernelGGL((delta_rule_step_kernel<ActBf16, true>), grid, block, 0, st, a);

@@ -14,14 +14,14 @@ __device__ __forceinline__ float silu_f(float x) { return x / (1.f + expf(-x)); 
 // Token by token.  grid = (heads, sequences, value columns in runs of 256); a thread owns one value column c and keeps
 // that column of the state, S[:, c], in registers; q_t and k_t go through LDS.
 template <typename A, int DMAX>
-__global__ __launch_bounds__(256) void lightning_rows_kernel(hymeta_lightning_attention_args a, int min_rows, int max_rows) {
+__global__ __launch_bounds__(256) void lightning_rows_kernel(hymeta_lightning_attention_args a, int min_rows) {
   typedef typename A::elem elem;
   __shared__ float s_q[2][DMAX], s_k[2][DMAX];
   const int h = blockIdx.x, s = blockIdx.y;
   const int c = blockIdx.z * 256 + threadIdx.x;
   const int H = a.num_heads, D = a.head_dim, Dv = a.v_dim;
   const int r0 = a.query_start_loc[s], r1 = a.query_start_loc[s + 1];
-  if (r1 - r0 < min_rows || r1 - r0 > max_rows) return;          // single rows / longer portions: the other kernels'
+  if (r1 - r0 < min_rows) return;          // single rows: the other kernel's
   const int slot = a.slot_idx[s];
   const bool live = c < Dv;
   float* st = (slot >= 0) ? a.state + ((static_cast<int64_t>(slot) * H + h) * D) * Dv : nullptr;
@@ -217,13 +217,13 @@ inline bool step_shape(const hymeta_lightning_attention_args& a) {
 }
 
 template <typename A>
-void launch_rows(const hymeta_lightning_attention_args& a, hipStream_t st, int min_rows, int max_rows) {
+void launch_rows(const hymeta_lightning_attention_args& a, hipStream_t st, int min_rows) {
   const dim3 grid(a.num_heads, a.num_seqs, (a.v_dim + 255) / 256);
   const dim3 block(a.v_dim >= 256 ? 256 : (a.v_dim + 63) / 64 * 64);
-  if (a.head_dim <= 32) hipLaunchKernelGGL((lightning_rows_kernel<A, 32>), grid, block, 0, st, a, min_rows, max_rows);
-  else if (a.head_dim <= 64) hipLaunchKernelGGL((lightning_rows_kernel<A, 64>), grid, block, 0, st, a, min_rows, max_rows);
-  else if (a.head_dim <= 128) hipLaunchKernelGGL((lightning_rows_kernel<A, 128>), grid, block, 0, st, a, min_rows, max_rows);
-  else hipLaunchKernelGGL((lightning_rows_kernel<A, 256>), grid, block, 0, st, a, min_rows, max_rows);
+  if (a.head_dim <= 32) hipLaunchKernelGGL((lightning_rows_kernel<A, 32>), grid, block, 0, st, a, min_rows);
+  else if (a.head_dim <= 64) hipLaunchKernelGGL((lightning_rows_kernel<A, 64>), grid, block, 0, st, a, min_rows);
+  else if (a.head_dim <= 128) hipLaunchKernelGGL((lightning_rows_kernel<A, 128>), grid, block, 0, st, a, min_rows);
+  else hipLaunchKernelGGL((lightning_rows_kernel<A, 256>), grid, block, 0, st, a, min_rows);
 }
 
 }  // namespace
@@ -247,8 +247,8 @@ extern "C" int hymeta_lightning_attention(const hymeta_lightning_attention_args*
   if (!a.qkv || !a.state || !a.decay || !a.out || !a.query_start_loc || !a.context_lens || !a.slot_idx) return HYMETA_ERR_INVALID_ARG;
   if (a.qkv_stride_t < static_cast<int64_t>(a.num_heads) * (2 * a.head_dim + a.v_dim)) return HYMETA_ERR_INVALID_ARG;
   hipStream_t st = begin_launches(stream);
-  int max_rows = 0x7fffffff;
-  if (chunk_shape(a) && a.max_query_len >= kScanMinRows) {
+  // (portions shorter than a chunk's least run in the same launch)
+  if (chunk_shape(a) && a.max_query_len >= 2) {
     const ScanSegments sg = scan_segments(a.num_tokens, a.num_seqs, a.num_heads, a.v_dim, a.max_query_len);
     const size_t need = scan_segment_bytes(sg.count, a.num_heads, a.head_dim, a.v_dim);
     if (need > 0 && (!a.workspace || a.workspace_bytes < need)) return HYMETA_ERR_WORKSPACE;
@@ -258,7 +258,7 @@ extern "C" int hymeta_lightning_attention(const hymeta_lightning_attention_args*
                           a.state, a.out, static_cast<float*>(a.workspace), a.query_start_loc, a.context_lens, a.slot_idx,
                           a.num_seqs, a.num_heads, a.num_heads, a.v_dim};
     launch_chunk_scan<true>(c, a.head_dim, sg, st);
-    max_rows = kScanMinRows - 1;
+    return launch_status();
   }
   int min_rows = 1;
   if (step_shape(a)) {
@@ -267,9 +267,9 @@ extern "C" int hymeta_lightning_attention(const hymeta_lightning_attention_args*
     else hipLaunchKernelGGL(lightning_step_kernel<ActF32>, grid, dim3(256), 0, st, a);
     min_rows = 2;
   }
-  if (a.max_query_len >= min_rows && max_rows >= min_rows) {
-    if (a.act_dtype == HYMETA_BF16) launch_rows<ActBf16>(a, st, min_rows, max_rows);
-    else launch_rows<ActF32>(a, st, min_rows, max_rows);
+  if (a.max_query_len >= min_rows) {
+    if (a.act_dtype == HYMETA_BF16) launch_rows<ActBf16>(a, st, min_rows);
+    else launch_rows<ActF32>(a, st, min_rows);
   }
   return launch_status();
 }
