@@ -86,3 +86,29 @@ def test_against_64_bits(C, H, page, lens, ctxs, opts):
         assert torch.isfinite(got).all()
         assert (got - ref).norm() <= BOUND * ref.norm(), (s, float((got - ref).norm() / ref.norm()))
         at += n
+
+
+@pytest.mark.parametrize("C,H,page,lens,keys", [(256, 8, 64, [1100], 5300), (512, 16, 32, [600, 500], 3000), (256, 3, 16, [1] * 300, 4600), (384, 16, 64, [1] * 270, 4400)])
+def test_more_tiles_than_a_look_up_holds(C, H, page, lens, keys):
+    """Sequences over the same pages, so many that their keys are not cut: more than 64 tiles one behind the other."""
+    from vllm_hymeta import hip_ops
+    g, D, T = torch.Generator().manual_seed(C + keys), C + 64, sum(lens)
+    rows, q = torch.randn(keys, D, generator=g).bfloat16(), torch.randn(T, H, D, generator=g).bfloat16()
+    pages = (keys + page - 1) // page
+    order = torch.randperm(pages, generator=g)
+    cache = torch.full((pages, page, 1, D), float("nan"), dtype=torch.bfloat16)
+    for b in range(pages):
+        piece = rows[b * page:(b + 1) * page]
+        cache[order[b], :len(piece), 0] = piece
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    out = hip_ops.sink_attention(q.cuda(), cache.cuda(), order.to(torch.int32)[None].expand(len(lens), -1).contiguous().cuda(), i32([0] + list(accumulate(lens))),
+                                 i32([keys] * len(lens)), 1, D, C, D ** -0.5, max(lens), keys, value_in_key=True).double().cpu()
+    starts = [0] + list(accumulate(lens))
+    for s in range(0, len(lens), 1 if len(lens) < 9 else 89):
+        some = sorted({0, lens[s] // 2, lens[s] - 1})
+        for i in some:                                    # (a row over the keys up to its own)
+            n = keys - lens[s] + i + 1
+            ref = reference(q[starts[s] + i:starts[s] + i + 1].double(), rows[:n].double(), C, D ** -0.5, None, 0, 0, 0, 0.0, None, None, n - 1)
+            got = out[starts[s] + i:starts[s] + i + 1]
+            assert (got - ref).norm() <= BOUND * ref.norm(), (s, i)
+    assert torch.isfinite(out).all()

@@ -1124,7 +1124,8 @@ int launch_wide_latent(const hymeta_sink_attention_args& a, hipStream_t st) {
   const int group = a.num_heads / a.num_kv_heads;
   const PortionSlices ps = portion_slices(a);
   if (a.max_query_len > 1) {
-    hipLaunchKernelGGL((latent_prefill_kernel<C>), portion_grid(a, ps), dim3(64 * kWideWaves), 0, st, a, ps);
+    if (a.softcap <= 0.f && a.bias_mode == 0) hipLaunchKernelGGL((latent_prefill_kernel<C, true>), portion_grid(a, ps), dim3(64 * kWideWaves), 0, st, a, ps);
+    else hipLaunchKernelGGL((latent_prefill_kernel<C, false>), portion_grid(a, ps), dim3(64 * kWideWaves), 0, st, a, ps);
   }
   // one workgroup per compute unit (its rings fill the LDS): as many as there are units
   const int64_t slices = (group + kLatentHeads - 1) / kLatentHeads, items = static_cast<int64_t>(a.num_seqs) * a.num_kv_heads;

@@ -40,41 +40,93 @@ __device__ __forceinline__ void finish_scores(const hymeta_sink_attention_args& 
   }
 }
 
-// Keys [j0, j0 + Keys) of a sequence's key/value head into an LDS image of Keys rows of D elements, by waves `wave` of
-// `Waves`; keys past `last` repeat it (their weights are zero).  Pages hold a power of two of rows.  Beside RowCopy, which keeps
-// the lanes' places in registers: none are left here (512 + 64: all 256, with 18 spilled).
+// Tiles of Keys keys of a sequence's key/value head into LDS images of Keys rows of D elements, by waves `wave` of `Waves`.  Pages
+// hold a power of two of rows.  An instruction takes 64 chunks of 16 bytes; those of 8 rows (D / 64 instructions) repeat from 8
+// rows to 8 rows but for a chunk's place, and with the row pitch an odd multiple of 128 bytes that differs in one bit: the lanes'
+// places of 8 rows are enough.  Where a tile's first row lies is looked up for 64 tiles at once:
+// a load in front of every tile's copies waits for all that are on their way.  So does a register that lies in scratch memory;
+// with 512 + 64 the prompts' form has none left over, works its places out on every tile and parks the queries' last two steps in
+// LDS.  8192 rows x 16 heads on 512 + 64 1614 -> 1404 us, a decode step of 64 sequences x 4096 71.2 -> 66.4 (the look-ups and
+// places alone 1615 -> 1441 and all of 5 us).
 template <int D, int Keys, int Waves>
 struct LatentCopy {
-  static constexpr int kChunks = D / 8, kInstr = Keys * kChunks / 64, kPerWave = (kInstr + Waves - 1) / Waves;
-  static_assert(kChunks % 16 == 8 && Keys * kChunks % 64 == 0, "the row pitch is an odd multiple of 128 bytes");
+  static constexpr int kChunks = D / 8, kInstr = Keys * kChunks / 64, kEight = kChunks / 8;
+  static constexpr int kShare = Waves == 1 ? 1 : Waves / (Keys / 8), kPlaces = (kEight + kShare - 1) / kShare;       // waves to 8 rows
+  static_assert(kChunks % 16 == 8 && Keys % 8 == 0 && (Waves == 1 || Waves == kShare * (Keys / 8)), "the row pitch is an odd multiple of 128 bytes");
   const char* cache;
   const int32_t* bt;
   int64_t row_bytes;
   int shift, mask, wave;
+  static constexpr bool kKept = Waves == 1;       // the lanes' places are kept: where eight waves share a tile, registers are short
+  uint32_t place[kKept ? kPlaces : 1];
+  int tile_row;                   // lane = tile % 64: the cache row of a tile's first key, for 64 tiles from the last refill on
 
   __device__ __forceinline__ LatentCopy(const hymeta_sink_attention_args& a, const int32_t* tables, int g, int wave_)
       : cache(static_cast<const char*>(a.kv_cache) + static_cast<int64_t>(g) * D * 2), bt(tables),
-        row_bytes(static_cast<int64_t>(a.num_kv_heads) * D * 2), shift(__builtin_ctz(a.block_size)), mask(a.block_size - 1), wave(wave_) {}
-  __device__ __forceinline__ void issue(int j0, int last, char* image) const {
-    const bool whole = mask + 1 >= Keys;          // a tile (tiles start at multiples of Keys) lies in one page
-    int lane = threadIdx.x & 63;
-    asm volatile("" : "+v"(lane));                // the lanes' places are computed here each time: registers are short
-    if (!whole) {                                 // small pages: every row's page is looked up
-      for (int at = wave; at < kInstr; at += Waves) {
-        const int chunk = 64 * at + lane, row = chunk / kChunks, j = min(j0 + row, last);
-        const int64_t src = (static_cast<int64_t>(bt[j >> shift]) << shift) + (j & mask);
-        copy16_to_lds(cache + src * row_bytes + 16 * ((chunk % kChunks) ^ ((row >> 1) & 7)), image + 1024 * at);
-      }
-      return;
+        row_bytes(static_cast<int64_t>(a.num_kv_heads) * D * 2), shift(__builtin_ctz(a.block_size)), mask(a.block_size - 1), wave(wave_), tile_row(0) {
+  }
+  // this lane's byte offset from the tile's first row in the wave's i-th instruction over its 8 rows
+  __device__ __forceinline__ uint32_t place_of(int i, int lane) const {
+    const int eight = wave / kShare, chunk = 64 * (wave % kShare + kShare * i) + lane;
+    const int r = static_cast<int>(__umul24(chunk >> 3, (512 + kEight - 1) / kEight) >> 9);          // chunk / kChunks below 8 rows
+    const int pos = chunk - r * kChunks;
+    return __umul24(8 * eight + r, static_cast<uint32_t>(row_bytes)) + 16 * (pos ^ ((4 * eight + (r >> 1)) & 7));
+  }
+  // whether tiles of Keys rows of one page can be copied from lanes' 32-bit offsets
+  __device__ __forceinline__ bool fits() const { return mask + 1 >= Keys && row_bytes < (1 << 24); }
+  // (a tile behind the last key: that one's row)
+  template <typename F>
+  __device__ __forceinline__ void refill(int t, int tiles, int last, const F& key_of, bool begin = false) {
+    const int tile = t + ((static_cast<int>(threadIdx.x) - t) & 63);
+    if (tile < tiles) {
+      const int j = min(key_of(tile), last);
+      tile_row = (bt[j >> shift] << shift) + (j & mask);
     }
-    const int64_t base = (static_cast<int64_t>(__builtin_amdgcn_readfirstlane(bt[j0 >> shift])) << shift) + (j0 & mask);
+    if constexpr (kKept) {
+      if (begin) {                                // (under the load)
 #pragma unroll
-    for (int i = 0; i < kPerWave; ++i) {
-      const int at = wave + Waves * i;
-      if (kInstr % Waves != 0 && at >= kInstr) break;
+        for (int i = 0; i < kPlaces; ++i) place[i] = place_of(i, threadIdx.x & 63);
+      }
+    }
+    asm volatile("" : "+v"(tile_row));            // (waited for here and not on every tile)
+  }
+  // tile t, all of it in one page and seen by some row
+  __device__ __forceinline__ void issue_whole(int t, char* image) const {
+    const char* base = cache + static_cast<int64_t>(__builtin_amdgcn_readlane(tile_row, t & 63)) * row_bytes;
+    if constexpr (Waves == 1) {
+#pragma unroll
+      for (int e = 0; e < Keys / 8; ++e) {
+#pragma unroll
+        for (int i = 0; i < kEight; ++i) copy16_to_lds(base, e & 1 ? place[i] ^ 64 : place[i], image + 1024 * (kEight * e + i));
+        base += 8 * row_bytes;
+      }
+    } else {
+      char* rows = image + 1024 * (kEight * (wave / kShare) + wave % kShare);
+      int lane = threadIdx.x & 63;
+      asm volatile("" : "+v"(lane));              // (worked out here each time)
+#pragma unroll
+      for (int i = 0; i < kPlaces; ++i)
+        if (kEight % kShare == 0 || i + 1 < kPlaces || wave % kShare < kEight % kShare) copy16_to_lds(base, place_of(i, lane), rows + 1024 * kShare * i);
+    }
+  }
+  // tile t with its rows past the first `rows` repeating the last of those (their weights are zero)
+  __device__ __forceinline__ void issue_part(int t, int rows, char* image) const {
+    const char* base = cache + static_cast<int64_t>(__builtin_amdgcn_readlane(tile_row, t & 63)) * row_bytes;
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));                // (nothing of this is kept in registers over the other tiles)
+    for (int at = wave; at < kInstr; at += Waves) {
       const int chunk = 64 * at + lane, row = chunk / kChunks;
-      const int off = 16 * ((chunk % kChunks) ^ ((row >> 1) & 7));
-      copy16_to_lds(cache + (base + min(row, last - j0)) * row_bytes + off, image + 1024 * at);
+      copy16_to_lds(base, __umul24(min(row, rows - 1), static_cast<uint32_t>(row_bytes)) + 16 * ((chunk % kChunks) ^ ((row >> 1) & 7)), image + 1024 * at);
+    }
+  }
+  // pages that do not fit: keys [j0, j0 + Keys), those past `last` repeating it
+  __device__ __forceinline__ void issue(int j0, int last, char* image) const {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));                // (nothing of this is kept in registers over the other tiles)
+    for (int at = wave; at < kInstr; at += Waves) {
+      const int chunk = 64 * at + lane, row = chunk / kChunks, j = min(j0 + row, last);
+      const int64_t src = (static_cast<int64_t>(bt[j >> shift]) << shift) + (j & mask);
+      copy16_to_lds(cache + src * row_bytes + 16 * ((chunk % kChunks) ^ ((row >> 1) & 7)), image + 1024 * at);
     }
   }
 };
@@ -85,7 +137,9 @@ static_assert(kWideRows == kPortionRows, "the merge finds a row's block");
 template <int C>
 struct WideSmem {
   static constexpr int kImage = kWideKeys * (C + 64) * 2;
+  static constexpr int kParked = C == 512 ? 2 : 0;      // the queries' last steps that find no registers
   char k[3][kImage];                              // tiles t, t + 1 and, on its way, t + 2
+  u32x4 q[kParked ? kWideWaves : 1][kParked ? kParked : 1][64];
   u32x4 p[2][kWideWaves][2][64];                  // weights of a tile, high and low bf16 parts, by row block and lane
   float corr[2][kWideRows];                       // what a row's sums so far are multiplied with before the tile
   int moved[2][kWideWaves];                       // whether a row block has any factor but 1
@@ -98,11 +152,12 @@ struct WideSmem {
 // Per tile of 32 keys a workgroup issues 800 matrix instructions (C = 512) against 480 LDS reads of 1 KB; a step computes
 // the scores of tile t + 1 and adds tile t's values, which do not depend on each other: the two waves of a SIMD do them in
 // opposite order, so that one's softmax runs under the other's products.  One barrier per tile.  Bound by the matrix
-// and the vector pipes, busy 43 and 39 % of the time: 8192 rows x 16 heads on 512 + 64: 1.61 ms = 1.07 PFLOP/s of the products
-// issued (both parts of the weights counted), where launches over value slices of 128, each repeating the scores, took 11.3 ms.
-template <int C>
+// and the vector pipes, busy 51 and 40 % of the time at 2.05 GHz: 8192 rows x 16 heads on 512 + 64: 1.40 ms = 1.23 PFLOP/s of the
+// products issued (both parts of the weights counted), where launches over value slices of 128, each repeating the scores, took
+// 11.3 ms.  Fragments of the keys three ahead (two: 1.408, five: 1.406).  Plain: neither a bias nor a cap on the scores.
+template <int C, bool Plain>
 __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_sink_attention_args a, PortionSlices ps) {
-  constexpr int D = C + 64, kRowB = 2 * D, kSteps = D / 32, CB = C / 128;
+  constexpr int D = C + 64, kRowB = 2 * D, kSteps = D / 32, CB = C / 128, kParked = WideSmem<C>::kParked, kAhead = 3;
   __shared__ __attribute__((aligned(16))) WideSmem<C> sm;
   const int group = a.num_heads / a.num_kv_heads, g = blockIdx.x % a.num_kv_heads, item = blockIdx.x / a.num_kv_heads, split = item % ps.splits;
   const PieceAt block = portion_block(a, item / ps.splits);
@@ -118,12 +173,16 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
   const bool ok = r < rows;
   const int qi = ok ? r / group : 0, h = g * group + (ok ? r % group : 0);
   const int pos = ok ? ctx + qi : -1;
-  const float ba = a.bias_mode ? a.bias_a[h] : 0.f, bb = a.bias_mode == HYMETA_BIAS_LOG_DISTANCE ? a.bias_b[h] : 0.f;
-  bf16x8 qf[kSteps];
+  const float ba = !Plain && a.bias_mode ? a.bias_a[h] : 0.f, bb = !Plain && a.bias_mode == HYMETA_BIAS_LOG_DISTANCE ? a.bias_b[h] : 0.f;
+  bf16x8 qf[kSteps - kParked];
   {
     const uint16_t* qrow = static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(row0 + qi) * a.q_stride_t + static_cast<int64_t>(h) * D;
 #pragma unroll
-    for (int st = 0; st < kSteps; ++st) qf[st] = ok ? __builtin_bit_cast(bf16x8, ld16g(qrow + 32 * st + 8 * g4)) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    for (int st = 0; st < kSteps; ++st) {
+      const u32x4 x = ok ? ld16g(qrow + 32 * st + 8 * g4) : u32x4{0u, 0u, 0u, 0u};
+      if (st < kSteps - kParked) qf[st] = __builtin_bit_cast(bf16x8, x);
+      else sm.q[wave][st - (kSteps - kParked)][lane] = x;
+    }
   }
   // positions the block's and the wave's rows span
   const int p_hi = ctx + (min(rows, r0 + kWideRows) - 1) / group;
@@ -145,32 +204,39 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) o[rb][cb] = f32x4v{0.f, 0.f, 0.f, 0.f};
 
-  const LatentCopy<D, kWideKeys, kWideWaves> copy(a, a.block_tables + static_cast<int64_t>(s) * a.block_table_stride, g, wave);
+  LatentCopy<D, kWideKeys, kWideWaves> copy(a, a.block_tables + static_cast<int64_t>(s) * a.block_table_stride, g, wave);
   // LDS offsets of this lane's fragments: keys (even and odd 32-element steps), values
   const int swz = (n >> 1) & 7;
-  const int koff[2] = {n * kRowB + 16 * (g4 ^ swz), n * kRowB + 16 * ((4 + g4) ^ swz)};
-  int voff[CB];
-#pragma unroll
-  for (int cb = 0; cb < CB; ++cb) {
-    const int R = 4 * g4 + (n >> 2), chunk = 2 * (wave * CB + cb) + ((n & 3) >> 1);
-    voff[cb] = R * kRowB + 16 * (chunk ^ ((R >> 1) & 7)) + 8 * (n & 1);
-  }
-
+  // (the others are one bit away, and worked out where they are used: registers are short)
+  const int koff = n * kRowB + 16 * (g4 ^ swz);
+  const int vrow = 4 * g4 + (n >> 2);
+  auto value_place = [&](int block) __attribute__((always_inline)) {
+    return vrow * kRowB + 16 * ((2 * block + ((n & 3) >> 1)) ^ ((vrow >> 1) & 7)) + 8 * (n & 1);
+  };
+  const int voff = value_place(wave * CB);
+  const float scale2 = a.scale * 1.4426950408889634f;
   auto scores = [&](int t, const char* img, int buf) {
     const int j0 = key0(t);
     f32x4v acc[2] = {};
-    u32x4 kf[2][2];                                   // fragments one step ahead, and no more: registers are short
-    auto load = [&](int st) {
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) kf[st & 1][ks] = ld16(img + koff[st & 1] + ks * 16 * kRowB + (st >> 1) * 128);
+    // fragment f: step f / 2 of the head, keys 16 (f % 2) ..; kAhead of them ahead
+    u32x4 kf[kAhead + 1];
+    bf16x8 parked[kParked + 1];
+    int even = koff;
+    asm volatile("" : "+v"(even));
+    const int odd = even ^ 64;
+    auto load = [&](int f) __attribute__((always_inline)) {
+      const int st = f >> 1, late = st - (kSteps - kParked);
+      kf[f % (kAhead + 1)] = ld16(img + (st & 1 ? odd : even) + (f & 1) * 16 * kRowB + (st >> 1) * 128);
+      if (late >= 0 && (f & 1) == 0) parked[late < 0 ? 0 : late] = __builtin_bit_cast(bf16x8, sm.q[wave][late < 0 ? 0 : late][lane]);
     };
-    load(0);
 #pragma unroll
-    for (int st = 0; st < kSteps; ++st) {
-      if (st + 1 < kSteps) load(st + 1);
+    for (int f = 0; f < kAhead; ++f) load(f);
+#pragma unroll
+    for (int f = 0; f < 2 * kSteps; ++f) {
+      if (f + kAhead < 2 * kSteps) load(f + kAhead);
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) acc[ks] = mfma16(__builtin_bit_cast(bf16x8, kf[st & 1][ks]), qf[st], acc[ks]);
+      const int st = f >> 1, late = st - (kSteps - kParked);
+      acc[f & 1] = mfma16(__builtin_bit_cast(bf16x8, kf[f % (kAhead + 1)]), late < 0 ? qf[late < 0 ? st : 0] : parked[late < 0 ? 0 : late], acc[f & 1]);
     }
     // the lane holds the scores of its row against keys j0 + 16 ks + 4 g4 + e
     const bool masked = !(full && j0 + kWideKeys - 1 <= w_lo && j0 >= w_first);
@@ -179,7 +245,12 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
     for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) sc[ks][e] = acc[ks][e];
-      finish_scores(a, sc[ks], static_cast<float>(pos - (j0 + 16 * ks + 4 * g4)), ba, bb);
+      if constexpr (Plain) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sc[ks][e] *= scale2;
+      } else {
+        finish_scores(a, sc[ks], static_cast<float>(pos - (j0 + 16 * ks + 4 * g4)), ba, bb);
+      }
     }
     if (masked) {
       const int first = first_key(a, pos);
@@ -225,9 +296,13 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
   };
   auto values = [&](const char* img, int buf) {
     bf16x8 vf[CB];
+    int at = voff;
+    asm volatile("" : "+v"(at));
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
-      const bf16x4 v0 = read_transposed(img + voff[cb]), v1 = read_transposed(img + voff[cb] + 16 * kRowB);
+      // columns 16 (wave CB + cb) ..: CB runs of 2 chunks, 4 runs to a group of 8 chunks (CB = 3: not on its boundary)
+      const int col = 4 % CB == 0 ? at ^ (32 * cb) : value_place(wave * CB + cb);
+      const bf16x4 v0 = read_transposed(img + col), v1 = read_transposed(img + col + 16 * kRowB);
       vf[cb] = bf16x8{v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
     }
     int moved = 0;
@@ -257,10 +332,18 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
         for (int cb = 0; cb < CB; ++cb) o[rb][cb] = mfma16(vf[cb], __builtin_bit_cast(bf16x8, pf[rb & 1][part]), o[rb][cb]);
     }
   };
-  
+
+  const bool fits = copy.fits();
+  const int whole = p_hi + 1 - key0(tiles - 1) >= kWideKeys ? tiles : tiles - 1, looked_up = fits ? tiles : 0;
+  auto copy_tile = [&](int t, char* image) __attribute__((always_inline)) {
+    if (!fits) copy.issue(key0(t), p_hi, image);
+    else if (t < whole) copy.issue_whole(t, image);
+    else copy.issue_part(t, p_hi + 1 - key0(t), image);
+  };
   if (tiles > 0) {
-    copy.issue(key0(0), p_hi, sm.k[0]);
-    if (tiles > 1) copy.issue(key0(1), p_hi, sm.k[1]);
+    copy.refill(0, looked_up, p_hi, key0);
+    copy_tile(0, sm.k[0]);
+    if (tiles > 1) copy_tile(1, sm.k[1]);
     copies_landed_barrier();
     scores(0, sm.k[0], 0);
     copies_landed_barrier();
@@ -270,10 +353,11 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
     int i0 = 0, i1 = 1, i2 = 2;
     for (int t = 0; t < tiles; ++t) {
       // image i2 held tile t - 1, read for the last time before the barrier
-      if (t + 2 < tiles) copy.issue(key0(t + 2), p_hi, sm.k[i2]);
+      if (t + 2 < tiles) copy_tile(t + 2, sm.k[i2]);
       if (!kScoresFirst) values(sm.k[i0], t & 1);
       if (t + 1 < tiles) scores(t + 1, sm.k[i1], (t + 1) & 1);
       if (kScoresFirst) values(sm.k[i0], t & 1);
+      if ((t & 31) == 29) copy.refill(t + 3, looked_up, p_hi, key0);
       copies_landed_barrier();
       const int i = i0;
       i0 = i1, i1 = i2, i2 = i;
@@ -335,7 +419,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
 // heads) need 400 registers, of which 256 can be addressed by everything but the matrix instructions: the compiler spills
 // 460.  The head slices of a (sequence, slice of keys) follow each other on one die instead, whose L2 has the keys for the
 // second.  Bound by memory, and by what stands around a slice's few tiles (queries, first tile, merge): 64 sequences x 4096 keys
-// of 512 + 64, 16 heads: 69 us = 4.4 TB/s, where four launches over value slices took 280.
+// of 512 + 64, 16 heads: 66 us = 4.6 TB/s, where four launches over value slices took 280.
 constexpr int kLatentWaves = 4, kLatentKeys = 16, kLatentHeads = 16;
 
 template <int C>
@@ -382,7 +466,7 @@ __global__ __launch_bounds__(64 * kLatentWaves) void latent_decode_kernel(hymeta
   }
 #pragma unroll
   for (int cb = 0; cb < C / 16; ++cb) o[cb] = f32x4v{0.f, 0.f, 0.f, 0.f};
-  const LatentCopy<D, kLatentKeys, 1> copy(a, a.block_tables + static_cast<int64_t>(s) * a.block_table_stride, g, 0);
+  LatentCopy<D, kLatentKeys, 1> copy(a, a.block_tables + static_cast<int64_t>(s) * a.block_table_stride, g, 0);
   constexpr int kLoads = LatentCopy<D, kLatentKeys, 1>::kInstr;
   char* ring = sm.bytes + wave * 2 * Smem::kStage;
   const int swz = (n >> 1) & 7;
@@ -395,9 +479,17 @@ __global__ __launch_bounds__(64 * kLatentWaves) void latent_decode_kernel(hymeta
   }
 
   // (a wave whose 16 keys lie past the last one copies the last one and skips them)
+  const bool fits = copy.fits();
+  const int whole = key0(tiles - 1) + kLatentKeys - 1 <= pos ? tiles : tiles - 1, looked_up = fits ? v_hi + 1 : 0;
+  auto copy_tile = [&](int v, char* image) __attribute__((always_inline)) {
+    if (!fits) copy.issue(min(key0(v), pos), pos, image);
+    else if (v < whole) copy.issue_whole(v, image);
+    else copy.issue_part(v, max(1, pos + 1 - key0(v)), image);
+  };
   if (v_lo <= v_hi) {
-    copy.issue(min(key0(v_lo), pos), pos, ring);
-    if (v_lo < v_hi) copy.issue(min(key0(v_lo + 1), pos), pos, ring + Smem::kStage);
+    copy.refill(v_lo, looked_up, pos, key0, true);
+    copy_tile(v_lo, ring);
+    if (v_lo < v_hi) copy_tile(v_lo + 1, ring + Smem::kStage);
   }
   for (int v = v_lo; v <= v_hi; ++v) {
     const int j0 = key0(v);
@@ -452,7 +544,8 @@ __global__ __launch_bounds__(64 * kLatentWaves) void latent_decode_kernel(hymeta
     }
     if (v + 2 <= v_hi) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // the tile's last reads are in registers
-      copy.issue(min(key0(v + 2), pos), pos, img);
+      if (((v - v_lo) & 31) == 30) copy.refill(v + 2, looked_up, pos, key0);
+      copy_tile(v + 2, img);
     }
   }
   l += __shfl_xor(l, 16, 64);
