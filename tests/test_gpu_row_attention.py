@@ -73,6 +73,11 @@ def reference(q, k, v, scale, ctx, o, sink, a, gate):
     ("rows", 64, 128, 3, 1, 64, [1, 1], [63, -1], {}),
     ("latent", 192, 128, 37, 1, 64, [1, 1], [127, 3], dict(sink=True, elem=True)),
     ("scaled", 96, 96, 7, 7, 64, [1, 1], [200, 3], dict(sink=True, bias="linear")),
+    # few keys: single rows among the portions' blocks, up to the last such length and one key past it
+    *[("rows", 128, 128, 28, 4, 64, [1, 5, 0, 1, 40, 1], [0, 3, 0, c, 100, -1], dict(sink=True, bias="log", gate=True)) for c in (1023, 1024)],
+    ("latent", 192, 128, 16, 1, 64, [1, 1, 9], [511, 63, 0], dict(sink=True, elem=True)),
+    ("scaled", 64, 64, 4, 2, 64, [1, 2, 1], [700, 30, 5000], dict(sink=True, bias="linear", window=500, keep=7)),
+    ("shared", 128, 64, 4, 2, 16, [3, 1], [100, 255], {}),
 ])
 def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
     from vllm_hymeta import hip_ops

@@ -42,6 +42,8 @@ def reference(q, rows, C, scale, sink, window, keep, chunk, softcap, bias, gate,
     (384, 3, 32, [150, 1, 2], [0, 200, 1], dict(window=70, keep=5)),         # kept first keys ahead of the window
     (256, 4, 16, [64, 1, 1], [65, 0, 129], dict(chunk=48, gate=True)),
     (512, 1, 128, [129, 1], [0, 511], dict(softcap=5.0, bias=True)),
+    (512, 16, 64, [3, 1, 1], [100, 127, 0], dict(sink=True, gate=True)),      # few keys: single rows among the portions' blocks
+    (384, 5, 16, [2, 1, 1], [100, 128, -1], {}),                              # one key past that
     (512, 16, 64, [1, 3, 20, 1], [-1, -1, -10, 300], {}),                    # rows in front of their sequence
     (256, 4, 16, [1, 70, 2], [-1, -30, -2], dict(chunk=20, sink=True)),
     # keys cut into slices beside single rows: a window, kept first keys, a gate; some blocks whole

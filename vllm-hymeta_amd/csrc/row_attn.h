@@ -16,7 +16,7 @@ constexpr float kLazyMax2 = 8.f;     // the softmax reference may trail a row's 
 // Grid = the portions' blocks of 128 rows x slices of the keys at most x key/value heads (fastest, so that workgroups without
 // rows come last); a row is a (query, head) pair, the heads of a key/value head side by side: they share every key, so that a
 // portion of a few tokens fills its blocks and a block's causal edge is one tile.
-// Sequences with one row are left to the decode form.
+// Sequences with one row are left to the decode form, but where the step's keys are few (one_launch).
 //
 // Four waves of 32 rows, keys in tiles of 64 copied to two LDS images without passing registers, the values read transposed
 // from the rows as they lie; one barrier per tile; two workgroups on a compute unit, so that one's softmax runs under the
@@ -48,7 +48,7 @@ __global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attenti
   __shared__ __attribute__((aligned(16))) char s_rows[2][S::kImage];
   __shared__ __attribute__((aligned(16))) float s_scale[2][S::Scaled ? kTileKeys : 4];
   const int group = a.num_heads / a.num_kv_heads, g = blockIdx.x % a.num_kv_heads, item = blockIdx.x / a.num_kv_heads, split = item % ps.splits;
-  const PieceAt block = portion_block(a, item / ps.splits);
+  const PieceAt block = portion_block(a, item / ps.splits, ps);
   const int s = block.seq, row0 = block.row0, q = block.rows, rows = q * group;
   if (s < 0) return;
   const int r0 = ((rows - 1) / S::kRows - block.index) * S::kRows;        // (the longest rows first)

@@ -31,7 +31,7 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
   const int group = uniform(a.num_heads / a.num_kv_heads);
   const int item = uniform(blockIdx.x / a.num_kv_heads), g = blockIdx.x - item * a.num_kv_heads;
   const int number = uniform(item / ps.splits), split = item - number * ps.splits;
-  const PieceAt block = portion_block(a, number);
+  const PieceAt block = portion_block(a, number, ps);
   const int s = uniform(block.seq), row0 = block.row0, q = block.rows, rows = q * group;
   if (s < 0) return;
   const int r0 = ((rows - 1) / kRows - uniform(block.index)) * kRows;     // (the longest rows first)

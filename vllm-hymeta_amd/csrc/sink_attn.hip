@@ -906,7 +906,7 @@ __device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a,
 // up to `whole` tiles of 64 keys are not cut.
 constexpr int kLeastTiles = 2;                 // of a slice
 struct PortionSlices {
-  int splits = 1, whole = 0;
+  int splits = 1, whole = 0, least = 2;        // least: rows from which a sequence is a portion
   float* parts = nullptr;
 };
 constexpr int kPortionRows = 128;              // (query, head) rows of a block, the heads of a key/value head side by side
@@ -930,9 +930,9 @@ __device__ __forceinline__ BlockKeys block_keys(const hymeta_sink_attention_args
   return b;
 }
 // Block `number` of the step's portions.
-__device__ __forceinline__ PieceAt portion_block(const hymeta_sink_attention_args& a, int number) {
+__device__ __forceinline__ PieceAt portion_block(const hymeta_sink_attention_args& a, int number, const PortionSlices& ps) {
   const int group = a.num_heads / a.num_kv_heads;
-  return piece_at(a.query_start_loc, a.num_seqs, number, [=](int q) { return q > 1 ? (q * group + kPortionRows - 1) / kPortionRows : 0; });
+  return piece_at(a.query_start_loc, a.num_seqs, number, [=, least = ps.least](int q) { return q >= least ? (q * group + kPortionRows - 1) / kPortionRows : 0; });
 }
 constexpr int kWideKeys = 32;                  // a tile of the kernels over wide latents
 
@@ -1057,10 +1057,10 @@ inline int64_t decode_partial_bytes(int num_seqs, int num_heads, int num_kv_head
 }
 
 // Bound on the portions' blocks of 128 rows: as many of the longest as there are sequences, or the rows' and one begun per
-// portion of two rows or more.
-inline int64_t portion_blocks(int num_tokens, int num_seqs, int group, int max_query_len) {
+// portion of `least` rows or more.
+inline int64_t portion_blocks(int num_tokens, int num_seqs, int group, int max_query_len, int least = 2) {
   const int64_t each = (static_cast<int64_t>(max_query_len) * group + kPortionRows - 1) / kPortionRows;
-  return std::max<int64_t>(1, std::min<int64_t>(each * num_seqs, static_cast<int64_t>(num_tokens) * group / kPortionRows + std::min(num_seqs, num_tokens / 2)));
+  return std::max<int64_t>(1, std::min<int64_t>(each * num_seqs, static_cast<int64_t>(num_tokens) * group / kPortionRows + std::min(num_seqs, num_tokens / least)));
 }
 // Slices a portion's keys are cut into: where the blocks that the step's portions are worth (long_portions) do not fill the chip
 // (`target` workgroups) and the workspace has room for the partials (bounded: every row of the step has a place).  A slice's
@@ -1103,7 +1103,18 @@ inline PortionSlices portion_slices(const hymeta_sink_attention_args& a) {
   return ps;
 }
 inline dim3 portion_grid(const hymeta_sink_attention_args& a, const PortionSlices& ps) {
-  return dim3(static_cast<uint32_t>(portion_blocks(a.num_tokens, a.num_seqs, a.num_heads / a.num_kv_heads, a.max_query_len) * ps.splits * a.num_kv_heads));
+  return dim3(static_cast<uint32_t>(portion_blocks(a.num_tokens, a.num_seqs, a.num_heads / a.num_kv_heads, a.max_query_len, ps.least) * ps.splits * a.num_kv_heads));
+}
+// Whether the portions' launch takes the single rows as well, as portions of one row: neither the decode form nor its merge is
+// launched then, which cost 5 to 8 us where a step has no single row.  Only where no row sees more than `most` tiles of 64 keys,
+// which a workgroup walks alone (about 1.5 us each), and the single rows that there may be find room beside each other.  28 heads
+// of 128 with 4 key/value heads: six portions of 147 rows 28.9 -> 22.2 us, three of 100 behind 100 25.8 -> 19.3 (at which the host's
+// call stands); 40 rows beside 63 single ones, behind 400 36.6 -> 34.7, behind 900 47.4 -> 47.0.  A tile of the wide latents' kernel
+// costs three times as much: six portions of 33 rows on 512 + 64 27.5 -> 21.3.
+constexpr int kFewTiles = 16, kFewWideTiles = 2, kManySingleRows = 512;
+inline bool one_launch(const hymeta_sink_attention_args& a, const PortionSlices& ps, int most) {
+  return a.max_query_len > 1 && ps.splits == 1 && decode_tiles(a) <= most &&
+         static_cast<int64_t>(a.num_seqs - long_portions(a.num_tokens, a.num_seqs, a.max_query_len)) * a.num_kv_heads <= kManySingleRows;
 }
 void launch_combine(const hymeta_sink_attention_args& a, hipStream_t st, int splits, HeadSlice hs, const PortionSlices& ps) {
   const int heads = hs.count ? hs.count * a.num_kv_heads : a.num_heads;
@@ -1122,11 +1133,14 @@ void launch_combine(const hymeta_sink_attention_args& a, hipStream_t st, int spl
 template <int C>
 int launch_wide_latent(const hymeta_sink_attention_args& a, hipStream_t st) {
   const int group = a.num_heads / a.num_kv_heads;
-  const PortionSlices ps = portion_slices(a);
+  PortionSlices ps = portion_slices(a);
+  const bool alone = one_launch(a, ps, kFewWideTiles);
+  if (alone) ps.least = 1;
   if (a.max_query_len > 1) {
     if (a.softcap <= 0.f && a.bias_mode == 0) hipLaunchKernelGGL((latent_prefill_kernel<C, true>), portion_grid(a, ps), dim3(64 * kWideWaves), 0, st, a, ps);
     else hipLaunchKernelGGL((latent_prefill_kernel<C, false>), portion_grid(a, ps), dim3(64 * kWideWaves), 0, st, a, ps);
   }
+  if (alone) return launch_status();
   // one workgroup per compute unit (its rings fill the LDS): as many as there are units
   const int64_t slices = (group + kLatentHeads - 1) / kLatentHeads, items = static_cast<int64_t>(a.num_seqs) * a.num_kv_heads;
   const int splits = static_cast<int>(std::min<int64_t>((256 + items * slices - 1) / (items * slices), decode_tiles(a)));
@@ -1142,6 +1156,8 @@ int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st) {
   if (a.max_query_len > 1) {
     if constexpr (D <= 192) {
       ps = portion_slices(a);
+      const bool alone = one_launch(a, ps, kFewTiles);
+      if (alone) ps.least = 1;
       const dim3 grid = portion_grid(a, ps);
       // a kernel per rule of the scores; a cap and a bias together, which no design has, in the general one
       auto launch = [&](auto rule) {
@@ -1159,6 +1175,7 @@ int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st) {
       } else if constexpr (Layout != HYMETA_KV_SCALED_KEY) {
         launch(std::integral_constant<int, kAnyRule>{});
       }
+      if (alone) return launch_status();
     } else {
       constexpr int kRows = 16 * kPrefillWaves;
       const dim3 grid((a.max_query_len + kRows - 1) / kRows, a.num_heads, a.num_seqs);

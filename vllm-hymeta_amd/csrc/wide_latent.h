@@ -160,7 +160,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
   constexpr int D = C + 64, kRowB = 2 * D, kSteps = D / 32, CB = C / 128, kParked = WideSmem<C>::kParked, kAhead = 3;
   __shared__ __attribute__((aligned(16))) WideSmem<C> sm;
   const int group = a.num_heads / a.num_kv_heads, g = blockIdx.x % a.num_kv_heads, item = blockIdx.x / a.num_kv_heads, split = item % ps.splits;
-  const PieceAt block = portion_block(a, item / ps.splits);
+  const PieceAt block = portion_block(a, item / ps.splits, ps);
   const int s = block.seq, row0 = block.row0, q = block.rows, rows = q * group;
   if (s < 0) return;
   const int r0 = ((rows - 1) / kWideRows - block.index) * kWideRows;        // (the longest rows first)
