@@ -18,12 +18,19 @@ from . import _C
 _DT = {torch.bfloat16: _C.HYMETA_BF16, torch.float32: _C.HYMETA_F32}
 
 
-def _stream(t: torch.Tensor):
-    return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# What stands around every call.  A small step's kernels take less than the call does (attention over two portions of 125 rows 22 us
+# of host time against 15 on the GPU), so addresses go into the structs as plain numbers, the current stream is asked for
+# without building a Stream object, and messages are put together when they are needed.
+def _raw_stream(device: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
-def _p(t: Optional[torch.Tensor]):
-    return None if t is None else C.c_void_p(t.data_ptr())
+def _stream(t: torch.Tensor) -> int:
+    return _raw_stream(t.device)
+
+
+def _p(t: Optional[torch.Tensor]) -> Optional[int]:
+    return None if t is None else t.data_ptr()
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -36,9 +43,12 @@ def _dev(*ts):
     for t in ts:
         if t is None:
             continue
-        _require(t.is_cuda, "hymeta ops need HIP device tensors")
-        dev = dev or t.device
-        _require(t.device == dev, "all tensors must live on one device")
+        if dev is None:
+            _require(t.is_cuda, "hymeta ops need HIP device tensors")
+            dev = t.device
+        elif t.device != dev:
+            _require(t.is_cuda, "hymeta ops need HIP device tensors")
+            _require(False, "all tensors must live on one device")
     return dev
 
 
@@ -353,9 +363,9 @@ class _Workspace:
         self.buf, self.eager_clean, self.captures, self.uses = buf, eager_clean, set(), 0
 
 
-def _capture_id(stream) -> int:
+def _capture_id(stream: int) -> int:
     cid = C.c_uint64(0)
-    _C.check(_C.load().hymeta_stream_capture_id(C.c_void_p(stream.cuda_stream), C.byref(cid)), "hymeta_stream_capture_id")
+    _C.check(_C.load().hymeta_stream_capture_id(stream, C.byref(cid)), "hymeta_stream_capture_id")
     return int(cid.value)
 
 
@@ -370,8 +380,8 @@ def _workspace(device: torch.device, nbytes: int, tag: str = "paged_decode") -> 
     capture (told apart by its capture id) records its own clearing kernel in front of its first use of a
     ticketed workspace: each replay then starts from zero tickets whatever ran before it, and a buffer
     made during a capture is cleared eagerly before its first eager use."""
-    stream = torch.cuda.current_stream(device)
-    key = (device, stream.cuda_stream, tag)
+    stream = _raw_stream(device)
+    key = (device, stream, tag)
     cid = _capture_id(stream) if torch.cuda.is_current_stream_capturing() else 0
     ticketed = tag in _TICKETED
     ws = _workspaces.get(key)
@@ -419,14 +429,13 @@ class PartialSums:
             out = torch.empty(M, N, dtype=torch.bfloat16, device=self.device)
         _require(out.shape == (M, N) and out.dtype == torch.bfloat16 and out.stride(1) == 1, "out must be bf16 [M, N]")
         _C.check(_C.load().hymeta_gemm_partials_reduce(C.byref(self.desc), _p(out), out.stride(0),
-                                                       C.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)),
+                                                       _raw_stream(self.device)),
                  "hymeta_gemm_partials_reduce")
         return out
 
 
 def _partials(desc, M, N, device, tag, *keep):
-    stream = torch.cuda.current_stream(device)
-    key = (device, stream.cuda_stream, tag)
+    key = (device, _raw_stream(device), tag)
     return PartialSums(desc, (M, N), device, key, (_workspaces[key].buf,) + keep)
 
 
@@ -1469,11 +1478,13 @@ def _act(t: torch.Tensor) -> int:
 
 
 def _f32vec(t: Optional[torch.Tensor], n: int, name: str) -> None:
-    _require(t is None or (t.dtype == torch.float32 and t.is_contiguous() and t.numel() == n), f"{name} must be contiguous fp32 [{n}]")
+    if t is not None and not (t.dtype == torch.float32 and t.is_contiguous() and t.numel() == n):
+        raise ValueError(f"{name} must be contiguous fp32 [{n}]")
 
 
 def _i32vec(t: torch.Tensor, n: int, name: str) -> None:
-    _require(t.dtype == torch.int32 and t.is_contiguous() and t.numel() >= n, f"{name} must be contiguous int32 [{n}]")
+    if not (t.dtype == torch.int32 and t.is_contiguous() and t.numel() >= n):
+        raise ValueError(f"{name} must be contiguous int32 [{n}]")
 
 
 def embed_rows(token_ids: torch.Tensor, table: torch.Tensor, add: Optional[torch.Tensor] = None, scale: float = 1.0,
@@ -1673,8 +1684,8 @@ def sink_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_tables: torch.
     if scaled_key:
         _require(v_dim == head_dim, "a scaled key is its value")
         cache_tail = (1, scaled_key_row(num_kv_heads, head_dim, q.dtype))
-    _require(kv_cache.dtype == q.dtype and kv_cache.is_contiguous() and kv_cache.dim() == 4
-             and kv_cache.shape[2:] == cache_tail, f"kv_cache must be contiguous [blocks, block_size, {cache_tail[0]}, {cache_tail[1]}]")
+    if not (kv_cache.dtype == q.dtype and kv_cache.is_contiguous() and kv_cache.dim() == 4 and kv_cache.shape[2:] == cache_tail):
+        raise ValueError(f"kv_cache must be contiguous [blocks, block_size, {cache_tail[0]}, {cache_tail[1]}]")
     _require(keep_first >= 0, "keep_first counts tokens")
     _require(chunk >= 0 and (chunk == 0 or (window_left < 0 and keep_first == 0)), "a chunk goes without a window and kept first keys")
     _f32vec(sink_logits, H, "sink_logits")
