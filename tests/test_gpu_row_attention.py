@@ -78,6 +78,9 @@ def reference(q, k, v, scale, ctx, o, sink, a, gate):
     ("latent", 192, 128, 16, 1, 64, [1, 1, 9], [511, 63, 0], dict(sink=True, elem=True)),
     ("scaled", 64, 64, 4, 2, 64, [1, 2, 1], [700, 30, 5000], dict(sink=True, bias="linear", window=500, keep=7)),
     ("shared", 128, 64, 4, 2, 16, [3, 1], [100, 255], {}),
+    # keys cut into slices beside more single rows than go among the portions' blocks
+    ("rows", 64, 64, 4, 2, 64, [9] + [1] * 40, [2500] + [31 * i for i in range(40)], dict(sink=True, gate=True)),
+    ("latent", 192, 128, 8, 1, 64, [30] + [1] * 70, [1500] + [17 * i for i in range(70)], {}),
 ])
 def test_against_64_bits(layout, D, Dv, H, G, page, lens, ctxs, opts):
     from vllm_hymeta import hip_ops

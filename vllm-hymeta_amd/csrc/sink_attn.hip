@@ -944,15 +944,16 @@ __global__ __launch_bounds__(kCombineThreads) void sink_attention_combine_kernel
   const int group = a.num_heads / a.num_kv_heads, HG = hs.count ? hs.count : group;
   const int g = blockIdx.y / HG, r = blockIdx.y % HG, in_group = hs.first + r, h = g * group + in_group;
   const size_t row = partial_row_floats(a.v_dim);
-  if (blockIdx.x < a.num_seqs) {
+  const int singles = ps.least > 1 ? a.num_seqs : 0;   // (else single rows are portions)
+  if (blockIdx.x < singles) {
     const int s = blockIdx.x, t = a.query_start_loc[s];
     if (a.query_start_loc[s + 1] - t != 1) return;
     const size_t stride = HG * row;
     combine_row(a, static_cast<const float*>(a.workspace) + (static_cast<size_t>(s) * a.num_kv_heads + g) * splits * stride + r * row, stride, splits, t, h);
     return;
   }
-  const PieceAt at = piece_at(a.query_start_loc, a.num_seqs, blockIdx.x - a.num_seqs, [](int q) { return q; });
-  if (at.seq < 0 || at.rows <= 1) return;              // (rows behind the last portion have no partials)
+  const PieceAt at = piece_at(a.query_start_loc, a.num_seqs, blockIdx.x - singles, [](int q) { return q; });
+  if (at.seq < 0 || at.rows < ps.least) return;              // (rows behind the last portion have no partials)
   const int t = at.row0 + at.index, ctx = a.seq_lens[at.seq] - at.rows, rows = at.rows * group, r0 = (at.index * group + in_group) / kPortionRows * kPortionRows;
   const int p_first = ctx + r0 / group, p_hi = ctx + (min(rows, r0 + kPortionRows) - 1) / group;
   const int n = a.v_dim > 128 ? block_keys<kWideKeys>(a, p_first, p_hi).slices(ps) : block_keys<kTileKeys>(a, p_first, p_hi).slices(ps);
@@ -1105,16 +1106,21 @@ inline PortionSlices portion_slices(const hymeta_sink_attention_args& a) {
 inline dim3 portion_grid(const hymeta_sink_attention_args& a, const PortionSlices& ps) {
   return dim3(static_cast<uint32_t>(portion_blocks(a.num_tokens, a.num_seqs, a.num_heads / a.num_kv_heads, a.max_query_len, ps.least) * ps.splits * a.num_kv_heads));
 }
-// Whether the portions' launch takes the single rows as well, as portions of one row: neither the decode form nor its merge is
-// launched then, which cost 5 to 8 us where a step has no single row.  Only where no row sees more than `most` tiles of 64 keys,
-// which a workgroup walks alone (about 1.5 us each), and the single rows that there may be find room beside each other.  28 heads
-// of 128 with 4 key/value heads: six portions of 147 rows 28.9 -> 22.2 us, three of 100 behind 100 25.8 -> 19.3 (at which the host's
-// call stands); 40 rows beside 63 single ones, behind 400 36.6 -> 34.7, behind 900 47.4 -> 47.0.  A tile of the wide latents' kernel
-// costs three times as much: six portions of 33 rows on 512 + 64 27.5 -> 21.3.
-constexpr int kFewTiles = 16, kFewWideTiles = 2, kManySingleRows = 512;
+// Whether the portions' launch takes the single rows as well, as portions of one row: the decode form is not launched then, nor,
+// where no keys are cut, its merge, which cost 5 to 8 us where a step has no single row.  Without cut keys only where no row sees
+// more than `most` tiles of 64 keys, which a workgroup walks alone (about 1.5 us each), and the single rows that there may be find
+// room beside each other.  28 heads of 128 with 4 key/value heads: six portions of 147 rows 28.9 -> 22.2 us, three of 100 behind 100
+// 25.8 -> 19.3 (at which the host's call stood); 40 rows beside 63 single ones, behind 400 36.6 -> 34.7, behind 900 47.4 -> 47.0.  A
+// tile of the wide latents' kernel costs three times as much: six portions of 33 rows on 512 + 64 27.5 -> 21.3.  Where keys are cut
+// the single rows' are as well; few of them, as a slice of theirs has a workgroup of 128 rows to itself: 7 rows behind 6000 26.8 ->
+// 20.6 us, 40 beside 8 single ones 50.3 -> 46.4 (latents of 128 + 64: 48.0 -> 38.3), 8 beside 15 behind 3000 40.7 -> 34.5 (of each
+// about 5 the host's shorter call).  With one key/value head, whose single rows fill a fifth of a block, a quarter as many: 300 rows beside 8
+// single ones of 4096 keys on latents of 128 + 64 46 -> 49, beside 63 75 -> 86.
+constexpr int kFewTiles = 16, kFewWideTiles = 2, kManySingleRows = 512, kFewSingleRows = 4;
 inline bool one_launch(const hymeta_sink_attention_args& a, const PortionSlices& ps, int most) {
-  return a.max_query_len > 1 && ps.splits == 1 && decode_tiles(a) <= most &&
-         static_cast<int64_t>(a.num_seqs - long_portions(a.num_tokens, a.num_seqs, a.max_query_len)) * a.num_kv_heads <= kManySingleRows;
+  const int64_t singles = a.num_seqs - long_portions(a.num_tokens, a.num_seqs, a.max_query_len);
+  if (a.max_query_len <= 1) return false;
+  return ps.splits > 1 ? singles <= kFewSingleRows * std::min(a.num_kv_heads, 4) : decode_tiles(a) <= most && singles * a.num_kv_heads <= kManySingleRows;
 }
 void launch_combine(const hymeta_sink_attention_args& a, hipStream_t st, int splits, HeadSlice hs, const PortionSlices& ps) {
   const int heads = hs.count ? hs.count * a.num_kv_heads : a.num_heads;
@@ -1126,7 +1132,7 @@ void launch_combine(const hymeta_sink_attention_args& a, hipStream_t st, int spl
     else hipLaunchKernelGGL(sink_attention_combine_few_kernel<kFewPartials>, grid, dim3(kCombineThreads), 0, st, a, splits, hs);
     return;
   }
-  const dim3 grid(a.num_seqs + (ps.splits > 1 ? a.num_tokens : 0), heads);
+  const dim3 grid((ps.least > 1 ? a.num_seqs : 0) + (ps.splits > 1 ? a.num_tokens : 0), heads);
   hipLaunchKernelGGL(sink_attention_combine_kernel, grid, dim3(kCombineThreads), 0, st, a, splits, hs, ps);
 }
 
@@ -1140,7 +1146,10 @@ int launch_wide_latent(const hymeta_sink_attention_args& a, hipStream_t st) {
     if (a.softcap <= 0.f && a.bias_mode == 0) hipLaunchKernelGGL((latent_prefill_kernel<C, true>), portion_grid(a, ps), dim3(64 * kWideWaves), 0, st, a, ps);
     else hipLaunchKernelGGL((latent_prefill_kernel<C, false>), portion_grid(a, ps), dim3(64 * kWideWaves), 0, st, a, ps);
   }
-  if (alone) return launch_status();
+  if (alone) {
+    if (ps.splits > 1) launch_combine(a, st, 0, HeadSlice{}, ps);
+    return launch_status();
+  }
   // one workgroup per compute unit (its rings fill the LDS): as many as there are units
   const int64_t slices = (group + kLatentHeads - 1) / kLatentHeads, items = static_cast<int64_t>(a.num_seqs) * a.num_kv_heads;
   const int splits = static_cast<int>(std::min<int64_t>((256 + items * slices - 1) / (items * slices), decode_tiles(a)));
@@ -1175,7 +1184,10 @@ int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st) {
       } else if constexpr (Layout != HYMETA_KV_SCALED_KEY) {
         launch(std::integral_constant<int, kAnyRule>{});
       }
-      if (alone) return launch_status();
+      if (alone) {
+        if (ps.splits > 1) launch_combine(a, st, 0, HeadSlice{}, ps);
+        return launch_status();
+      }
     } else {
       constexpr int kRows = 16 * kPrefillWaves;
       const dim3 grid((a.max_query_len + kRows - 1) / kRows, a.num_heads, a.num_seqs);
