@@ -1,5 +1,7 @@
 """Prefill attention where its blocks of (query, head) rows, its tiles of keys and its copies can go wrong, against the dense
 definition in 64 bits."""
+import math
+
 import pytest
 import torch
 
@@ -80,3 +82,29 @@ def test_packed_rows(splits, rows, lens, H, G, M, window):
                                    max_seqlen_k=max(lens), num_splits=splits,
                                    **(dict(meta_key=meta[0].cuda(), meta_value=meta[1].cuda()) if M else {}))
     assert_bf16_close(out.cpu(), torch.cat(want), f"{splits} slices")
+
+
+@pytest.mark.parametrize("splits", [1, 4])
+def test_weight_of_the_greatest_score_is_not_rounded(splits):
+    """Every row sees one key of weight 1 and one of 3/4, both exact in bf16, beside keys of weights below 2^-40; their values are 1
+    and -1, so that an error of the weights' quotient shows 24/7 times as large.  The result, 1/7, is off by its own rounding (2^-9 at most)
+    and the scores' errors (fp32: below 2^-18 in the exponent, 2^-16 in the result)."""
+    from vllm_hymeta import hip_ops
+    n, L, scale = 512, 2048, 2.0 ** -4
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    # scores in base 2: c + 0 and c + log2(3/4) for the two keys, c = 48 .. 56 by row: q = (x, y, 0 ..), keys (1, 0, ..) and (1, 1, 0 ..)
+    g = gen(5)
+    x = (48 + 8 * torch.rand(n, generator=g)) * math.log(2) / scale
+    x = x.bfloat16()
+    parts, rest = [], torch.full((n,), math.log(0.75) / scale, dtype=torch.float64)
+    for _ in range(3):                                       # log(3/4) in three bf16 parts
+        parts.append(rest.bfloat16())
+        rest = rest - parts[-1].double()
+    q = torch.zeros(n, 1, D).bfloat16()
+    q[:, 0, 0] = x
+    q[:, 0, 1:4] = torch.stack(parts, 1)
+    k, v = torch.zeros(L, 1, D).bfloat16(), torch.zeros(L, 1, D).bfloat16()
+    k[5, 0, 0], k[9, 0, :4], v[5], v[9] = 1, 1, 1, -1
+    out = hip_ops.meta_swa_prefill(q.cuda(), i32([0, n]), n, key=k.cuda(), value=v.cuda(), cu_seqlens_k=i32([0, L]), scale=scale, num_splits=splits,
+                                   max_seqlen_k=L).double().cpu()
+    assert (out * 7 - 1).abs().max() < 2.0 ** -9 + 2.0 ** -15
