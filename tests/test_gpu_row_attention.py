@@ -204,3 +204,19 @@ def test_long_portions_against_the_general_kernel(layout, D, Dv, H, G, rows, ctx
                                            window_left=opts.get("window", 0) - 1, keep_first=opts.get("keep", 0), shared_key=layout == "shared", **bias).double())
     assert all(torch.isfinite(o).all() for o in outs)
     assert (outs[0] - outs[1]).norm() <= 2 * BOUND * outs[1].norm()             # (each within BOUND of the exact result)
+
+
+@pytest.mark.parametrize("D,Dv,lens", [(128, 128, [4]), (192, 128, [4]), (576, 512, [4]), (128, 128, [1]), (576, 512, [1])])
+@pytest.mark.parametrize("every", [1, 4])
+def test_keys_that_are_not_numbers_stay_in_a_row_of_cut_keys(D, Dv, lens, every):
+    """NaN in every tile of the first 1536 keys, where slices of 2, 3 and 4 tiles of 64 end, so that none sees both kinds: the row's
+    result is NaN, as where its keys are not cut."""
+    from vllm_hymeta import hip_ops
+    dev, total = "cuda", 3000
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
+    inside = D != Dv
+    q, cache = torch.randn(sum(lens), 4, D, device=dev).bfloat16(), torch.randn(47, 64, 1, D if inside else D + Dv, device=dev).bfloat16()
+    cache.view(-1, cache.shape[-1])[:1536:every, :64] = float("nan")           # (of a key alone; where it holds the value, of that too)
+    out = hip_ops.sink_attention(q, cache, torch.arange(47, dtype=torch.int32, device=dev)[None], i32([0] + list(accumulate(lens))), i32([total]), 1, D, Dv,
+                                 D ** -0.5, max(lens), total, value_in_key=inside)
+    assert out.isnan().all()

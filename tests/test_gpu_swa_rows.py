@@ -108,3 +108,14 @@ def test_weight_of_the_greatest_score_is_not_rounded(splits):
     out = hip_ops.meta_swa_prefill(q.cuda(), i32([0, n]), n, key=k.cuda(), value=v.cuda(), cu_seqlens_k=i32([0, L]), scale=scale, num_splits=splits,
                                    max_seqlen_k=L).double().cpu()
     assert (out * 7 - 1).abs().max() < 2.0 ** -9 + 2.0 ** -15
+
+
+@pytest.mark.parametrize("every", [1, 4])
+def test_keys_that_are_not_numbers_stay_in_a_row_of_cut_keys(every):
+    """NaN in every tile of the first two of four slices: the row's result is NaN, as where its keys are not cut."""
+    from vllm_hymeta import hip_ops
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    q, k, v = (torch.randn(n, h, D, device="cuda").bfloat16() for n, h in ((4, 7), (2048, 1), (2048, 1)))
+    k[:1024:every] = float("nan")
+    out = hip_ops.meta_swa_prefill(q, i32([0, 4]), 4, key=k, value=v, cu_seqlens_k=i32([0, 2048]), num_splits=4, max_seqlen_k=2048)
+    assert out.isnan().all()

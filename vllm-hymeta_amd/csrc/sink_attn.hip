@@ -857,6 +857,10 @@ __device__ __forceinline__ void store_row(const hymeta_sink_attention_args& a, f
       u32x2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
 }
 
+// Whether a partial has seen no key, by its maximum and the sum of its weights: where every tile it saw held a NaN it has no
+// maximum either, but a NaN for a sum, which the row's result keeps.
+__device__ __forceinline__ bool no_keys(float m, float l) { return m == -INFINITY && l == 0.f; }
+
 __device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a, const float* base, size_t stride, int splits, int64_t t, int h) {
   __shared__ float s_f[kMaxPartials];
   __shared__ float s_red[2][kCombineThreads / 64];
@@ -876,9 +880,9 @@ __device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a,
   m = fmaxf(s_red[0][0], s_red[0][1]);
   float l = 0.f;
   for (int sp = tid; sp < splits; sp += kCombineThreads) {      // (each thread's own entries of s_f)
-    const float f = s_f[sp] == -INFINITY ? -1.f : __builtin_amdgcn_exp2f(s_f[sp] - m);      // (-1: a partial without keys)
+    const float lp = base[sp * stride + DV + 1], f = no_keys(s_f[sp], lp) ? -1.f : __builtin_amdgcn_exp2f(s_f[sp] - m);
     s_f[sp] = f;
-    if (!(f < 0.f)) l = fmaf(base[sp * stride + DV + 1], f, l);
+    if (!(f < 0.f)) l = fmaf(lp, f, l);
   }
   l = wave_sum(l);
   if (lane == 0) s_red[1][wave] = l;
@@ -991,7 +995,7 @@ __global__ __launch_bounds__(kCombineThreads) void sink_attention_combine_few_ke
   f32x4v acc = f32x4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int sp = 0; sp < N; ++sp)
-    if (sp < splits && stat[sp].x != -INFINITY) {      // (a partial without keys)
+    if (sp < splits && !no_keys(stat[sp].x, stat[sp].y)) {
       const float f = __builtin_amdgcn_exp2f(stat[sp].x - m);
       l = fmaf(stat[sp].y, f, l);
       acc += x[sp] * f;

@@ -462,13 +462,13 @@ __global__ __launch_bounds__(256) void swa_prefill_merge_kernel(hymeta_swa_prefi
   for (int s = 0; s < splits; ++s) m = fmaxf(m, pm[s * part_rows * a.num_heads + pair]);
   float o0 = 0.f, o1 = 0.f, l = 0.f;
   for (int s = 0; s < splits; ++s) {
-    const float ms = pm[s * part_rows * a.num_heads + pair];
-    if (ms == -INFINITY) continue;           // a slice without a visible key for this query
+    const float ms = pm[s * part_rows * a.num_heads + pair], ls = pl[s * part_rows * a.num_heads + pair];
+    if (ms == -INFINITY && ls == 0.f) continue;           // a slice without a visible key for this query (of nothing but NaN: its sum is one)
     const float w = __builtin_amdgcn_exp2f(ms - m);
     const f32x2 v = *reinterpret_cast<const f32x2*>(po + (s * part_rows * a.num_heads + pair) * kHeadDim + 2 * lane);
     o0 += w * v[0];
     o1 += w * v[1];
-    l += w * pl[s * part_rows * a.num_heads + pair];
+    l += w * ls;
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;
   const int64_t row = pair / a.num_heads;
