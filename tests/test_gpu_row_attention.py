@@ -220,3 +220,19 @@ def test_keys_that_are_not_numbers_stay_in_a_row_of_cut_keys(D, Dv, lens, every)
     out = hip_ops.sink_attention(q, cache, torch.arange(47, dtype=torch.int32, device=dev)[None], i32([0] + list(accumulate(lens))), i32([total]), 1, D, Dv,
                                  D ** -0.5, max(lens), total, value_in_key=inside)
     assert out.isnan().all()
+
+
+@pytest.mark.parametrize("layout", ["rows", "shared"])
+@pytest.mark.parametrize("opts", [{}, dict(softcap=5.0), dict(window_left=20)])
+def test_scale_of_zero_weighs_all_keys_alike(layout, opts):
+    """Scores of 0: a row is the mean of the values it sees."""
+    from vllm_hymeta import hip_ops
+    dev, n, D = "cuda", 100, 128
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
+    q, cache = torch.randn(n, 4, D, device=dev).bfloat16(), torch.randn(2, 64, 1, 2 * D, device=dev).bfloat16()
+    out = hip_ops.sink_attention(q, cache, i32([[0, 1]]), i32([0, n]), i32([n]), 1, D, D, 0.0, n, n, sink=False,
+                                 shared_key=layout == "shared", **opts).double()
+    i = torch.arange(n, device=dev)
+    seen = ((i[None] <= i[:, None]) & (i[None] >= i[:, None] - opts.get("window_left", n))).double()
+    want = (seen @ cache.view(-1, 2 * D)[:n, D:].double() / seen.sum(1, keepdim=True))[:, None].expand(n, 4, D)
+    assert (out - want).norm() <= BOUND * want.norm()

@@ -56,17 +56,18 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
   bool unset = !sink;                                 // the row has seen neither a key nor a sink
   float ref = sink && a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f;      // of the exponentials, base 2
   float l = sink && hh == 0 ? 1.f : 0.f;              // the sink's exp(ref - ref), counted once per row
-  const float scale = fabsf(a.scale), scale2 = scale * 1.4426950408889634f;
+  // (a scale of 0: the queries are 0 and the scale 1, so that a masked score's -inf is not multiplied by 0)
+  const float scale = a.scale == 0.f ? 1.f : fabsf(a.scale), scale2 = scale * 1.4426950408889634f;
   const float cap_in = a.softcap > 0.f ? scale / a.softcap : 0.f, cap2 = a.softcap * 1.4426950408889634f;
   u32x4 qf[kSteps];                                   // (with the scale's sign, so that scores grow with their products)
   {
     const uint16_t* qrow = static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(row0 + qi) * a.q_stride_t + static_cast<int64_t>(h) * D + 8 * hh;
-    const uint32_t sign = a.scale < 0.f ? 0x80008000u : 0u;
+    const uint32_t sign = a.scale < 0.f ? 0x80008000u : 0u, kept_bits = a.scale == 0.f ? 0u : ~0u;
 #pragma unroll
     for (int st = 0; st < kSteps; ++st) {
       qf[st] = ld16g(qrow + 16 * st);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) qf[st][e] ^= sign;
+      for (int e = 0; e < 4; ++e) qf[st][e] = (qf[st][e] & kept_bits) ^ sign;
     }
   }
   f32x16 o[CB];                                       // O^T: columns 32 cb + 8 i + 4 hh + e of the lane's row, i, e < 4
