@@ -55,3 +55,19 @@ def test_short_portions(D, Dv, H, lens, silu):
         assert float((out[rows] - want[rows]).norm() / want[rows].norm()) < bound, s
         assert slots[s] < 0 or float((got[s] - states[s]).norm() / states[s].norm()) < bound, s
     assert torch.equal(got[3], state[3].double())
+
+
+@pytest.mark.parametrize("silu", [True, False])
+def test_sequences_without_rows_have_no_slot(silu):
+    """Their slots lie far outside the state, which is neither read nor written for them: outputs and states as without them."""
+    from vllm_hymeta import hip_ops
+    D, H, g = 64, 2, gen(9)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    qkv, state, decay = torch.randn(75, 3 * H * D, generator=g).bfloat16().cuda(), torch.randn(2, H, D, D, generator=g).cuda(), torch.tensor([0.9, 0.99]).cuda()
+    q, k, v = (x.unflatten(1, (H, D)) for x in qkv.split([H * D] * 3, 1))
+    results = []
+    for starts, slots in (([0, 5, 75], [0, 1]), ([0, 0, 5, 5, 75, 75], [1 << 30, 0, 1 << 30, 1, 1 << 30])):
+        got, where = state.clone(), (i32(starts), i32([3] * len(slots)), i32(slots), 70)
+        out = hip_ops.lightning_attention(qkv, got, decay, H, D, D, *where) if silu else hip_ops.decay_scan(q, k, v, got, *where, decay=decay)
+        results.append((out, got))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])

@@ -214,6 +214,7 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
     seg.row0 = a.query_start_loc[seg.seq], seg.rows = a.query_start_loc[seg.seq + 1] - seg.row0;
   }
   const int s = seg.seq, r0 = seg.row0, rows_all = seg.rows;
+  if (rows_all <= 0) return;                           // (a sequence without rows: its slot may be anything)
   if constexpr (!Summarise) {
     static_assert(sizeof(s_k) >= 8 * D && sizeof(s_v) >= 2 * 16 * 64 * NW, "the scratch of single rows");
     if (rows_all < kScanMinRows) {                     // (a segment has more)
