@@ -56,3 +56,18 @@ def test_every_slice_against_64_bits(D, Dv, H, Hk, lens, shift):
         assert float((out[a:b] - want[a:b]).norm() / want[a:b].norm()) < 2e-5, s
     assert float((got - states).norm() / states.norm()) < 2e-5
     assert torch.equal(got[3:4], state[3:4].double()) if n > 3 else True
+
+
+def test_a_portion_longer_than_the_bound_says():
+    """A bound of fewer rows than a chunk takes asks for no workspace: every row goes token by token, however many there are."""
+    from vllm_hymeta import hip_ops
+    H, D, lens, g = 4, 128, [3, 70, 1, 130], gen(7)
+    T, n, starts = sum(lens), len(lens), [sum(lens[:i]) for i in range(len(lens) + 1)]
+    q, k, v = (torch.randn(T, H, D, generator=g).bfloat16() for _ in range(3))
+    beta, l2, state = torch.randn(T, H, generator=g).bfloat16(), -torch.rand(T, H, generator=g) * 0.2, torch.randn(n, H, D, D, generator=g) * 0.1
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    got = state.cuda()
+    out = hip_ops.delta_rule(q.cuda(), k.cuda(), v.cuda(), beta.cuda(), l2.cuda(), got, i32(starts), i32([1] * n), i32(list(range(n))), 4, D ** -0.5, 1e-6)
+    want, states = _recurrence(q, k, v, beta, l2, state, starts, [1] * n, list(range(n)), D ** -0.5, 1e-6)
+    assert float((out.view(T, H, D).double().cpu() - want).norm() / want.norm()) < 2e-6        # (fp32 throughout)
+    assert float((got.double().cpu() - states).norm() / states.norm()) < 2e-6

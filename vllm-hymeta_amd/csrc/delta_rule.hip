@@ -259,10 +259,12 @@ __device__ __forceinline__ void split4(const float* v, u32x2& hi, u32x2& lo) {
 __host__ __device__ inline size_t rows_at(int64_t chunks, int heads) { return static_cast<size_t>(chunks) * heads * sizeof(ChunkPlace); }
 
 // grid = (chunk numbers, heads), 4 waves with 16 rows of the chunk each.
-// Portions shorter than kChunkMinRows go token by token here (short_too: the state fits the threads' registers), so that they
-// need no launch of their own: two launches with nothing to do took 9 of the 280 us of five portions of 1801 rows.
+// Portions of up to short_rows rows go token by token here (0: none do; the state fits the threads' registers), so that they need
+// no launch of their own: two launches with nothing to do took 9 of the 280 us of five portions of 1801 rows.  The caller's bound
+// of the rows says whether there are chunks, and with them a workspace: below kChunkMinRows every portion goes token by token,
+// however long it turns out to be.
 template <int D, bool Pack>
-__global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hymeta_delta_rule_args a, int64_t chunks, int short_too) {
+__global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hymeta_delta_rule_args a, int64_t chunks, int short_rows) {
   constexpr int PK = D + 8, PF = kChunk + 4;
   // (the keys and T share their place where nothing asks for the keys again: four workgroups to a compute unit)
   constexpr int kKeyBytes = kChunk * PK * 2, kMatrixBytes = kChunk * PF * 4;
@@ -282,9 +284,9 @@ __global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hy
   const int r0 = a.query_start_loc[s], rows = a.query_start_loc[s + 1] - r0;
   const int c0 = (number - (r0 / kChunk + s)) * kChunk;
   if (c0 >= rows) return;
-  if (rows < kChunkMinRows) {
+  if (rows < kChunkMinRows || rows <= short_rows) {
     static_assert(sizeof(StepScratch) <= sizeof(sA), "the scratch lies where A would");
-    if (short_too) delta_rows<ActBf16, false>(a, blockIdx.y, s, r0, r0 + rows, *reinterpret_cast<StepScratch*>(sA));
+    if (rows <= short_rows && c0 == 0) delta_rows<ActBf16, false>(a, blockIdx.y, s, r0, r0 + rows, *reinterpret_cast<StepScratch*>(sA));
     return;
   }
   const int nrow = min(kChunk, rows - c0), h = blockIdx.y, H = a.num_heads, group = H / a.num_qk_heads, g = h / group;
@@ -958,18 +960,19 @@ void launch_rows(const hymeta_delta_rule_args& a, hipStream_t st, int min_rows, 
 
 template <int D>
 void launch_chunks(const hymeta_delta_rule_args& a, hipStream_t st, int64_t chunks, bool short_too) {
+  const int short_rows = !short_too ? 0 : a.max_query_len < kChunkMinRows ? 0x7fffffff : kChunkMinRows - 1;
   const int64_t portions = long_portions(a.num_tokens, a.num_seqs, a.max_query_len), lanes = a.num_heads * portions;
   const int64_t idle = a.num_heads * (a.num_seqs - portions) * (a.v_dim / 32);
   const bool narrow = D % 64 == 0 && lanes * (a.v_dim / 32) <= kFewGroups && idle <= static_cast<int64_t>(kIdleGroupsPerRow) * a.max_query_len;
   const dim3 solve(static_cast<unsigned>(chunks), a.num_heads);
   if constexpr (D % 64 == 0) {
     if (narrow && a.max_query_len >= kChunkMinRows) {
-      hipLaunchKernelGGL((delta_chunk_solve_kernel<D, true>), solve, dim3(256), 0, st, a, chunks, short_too ? 1 : 0);
+      hipLaunchKernelGGL((delta_chunk_solve_kernel<D, true>), solve, dim3(256), 0, st, a, chunks, short_rows);
       hipLaunchKernelGGL(delta_chunk_narrow_kernel<D>, dim3(a.num_heads, a.num_seqs, a.v_dim / 16), dim3(256), 0, st, a, chunks);
       return;
     }
   }
-  hipLaunchKernelGGL((delta_chunk_solve_kernel<D, false>), solve, dim3(256), 0, st, a, chunks, short_too ? 1 : 0);
+  hipLaunchKernelGGL((delta_chunk_solve_kernel<D, false>), solve, dim3(256), 0, st, a, chunks, short_rows);
   if (a.max_query_len < kChunkMinRows) return;
   auto launch = [&](auto nw) {
     constexpr int NW = decltype(nw)::value;
