@@ -25,6 +25,7 @@ def _recurrence(q, k, v, w, decay, state, starts, context, slots):
 @pytest.mark.parametrize("D,Dv,H,lens", [
     (128, 128, 14, MIXED + [100] * 6), (64, 64, 4, MIXED), (32, 96, 4, MIXED), (128, 256, 4, [2, 7, 1, 3]),
     (64, 128, 2, [700, 1, 5, 300]),               # cut into segments
+    (64, 128, 32, [40] * 4 + [1] * 26 + [7, 2, 3, 6, 5]),         # in a launch beside the chunks'
 ])
 def test_short_portions(D, Dv, H, lens, silu):
     """Rows of portions of up to 7 stay in fp32: 1e-6 of the norm.  The others' operands enter as two bf16 parts, 2e-5, behind a
@@ -71,3 +72,26 @@ def test_sequences_without_rows_have_no_slot(silu):
         out = hip_ops.lightning_attention(qkv, got, decay, H, D, D, *where) if silu else hip_ops.decay_scan(q, k, v, got, *where, decay=decay)
         results.append((out, got))
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
+@pytest.mark.parametrize("silu", [True, False])
+@pytest.mark.parametrize("D,Dv,H", [(128, 128, 28), (64, 128, 64)])
+def test_single_rows_whose_states_do_not_fit_the_cache(D, Dv, H, silu):
+    """256 sequences, one of them of two rows: a launch of its own, fewer workgroups of which share a compute unit.  In 64 bits on
+    the GPU."""
+    from vllm_hymeta import hip_ops
+    n, g = 256, torch.Generator(device="cuda").manual_seed(D + H)
+    new = lambda *shape: torch.empty(*shape, device="cuda").normal_(generator=g)  # noqa: E731
+    qkv, state, decay = new(n + 1, H * (2 * D + Dv)).bfloat16(), new(n, H, D, Dv) * 0.1, 1 - 0.1 * new(H).abs().clamp_max(1)
+    q, k, v = (x.unflatten(1, (H, d)) for x, d in zip(qkv.split([H * D, H * D, H * Dv], 1), (D, D, Dv)))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    where, S = (i32([0, 2] + list(range(3, n + 2))), i32([4] * n), i32(list(range(n))), 2), state.double()
+    out = (hip_ops.lightning_attention(qkv, state, decay, H, D, Dv, *where) if silu else hip_ops.decay_scan(q, k, v, state, *where, decay=decay)).view(n + 1, H, Dv)
+    q, k, v = (torch.nn.functional.silu(x.double()) if silu else x.double() for x in (q, k, v))
+    d = decay.double()[:, None, None]
+    first = S[0] * d + k[0][:, :, None] * v[0][:, None]
+    assert float((out[0] - torch.matmul(q[0][:, None], first)[:, 0]).norm() / out[0].norm()) < 1e-6
+    S[0] = first
+    S = S * d + k[1:][..., None] * v[1:][:, :, None]
+    want = torch.matmul(q[1:][:, :, None], S)[:, :, 0]
+    assert float((out[1:] - want).norm() / want.norm()) < 1e-6 and float((state - S).norm() / S.norm()) < 1e-6

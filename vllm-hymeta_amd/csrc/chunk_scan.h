@@ -125,13 +125,11 @@ __device__ __forceinline__ PieceAt segment_at(const ChunkScanArgs& a, int seg_ro
 }
 
 // A portion too short for a chunk, row by row in fp32 by the 64 NW threads of a workgroup: a thread holds 4 value columns of the
-// rows d0, d0 + 16, ... of the state (16-byte loads, all in flight together), the 16 partial outputs of a column meet in LDS.
-// Launches of their own, which most steps have no use for, cost about 4 us each, and a thread per value column reads the state 4
-// bytes at a time: one prompt of 8192 rows, 28 heads, lightning 160 -> 156 us, four of 108 rows 23.8 -> 17.2; plain decays, five
-// portions of 3 rows 43.8 -> 18.8, four of 7 71 -> 19.6; 300 rows beside 63 single ones 61 -> 41.
+// rows d0, d0 + 16, ... of the state (16-byte loads, all in flight together), the 16 partial outputs of a column meet in LDS.  The
+// next row is on its way while one is worked on.  LDS for two rows each: queries and keys, 2 D floats a row, and partial outputs, 256 NW floats a row.
 template <int D, int NW, bool Silu>
 __device__ __forceinline__ void scan_single_rows(const ChunkScanArgs& a, int h, int s, int r0, int rows, int col0, float* s_row, float* s_part) {
-  constexpr int NT = 64 * NW, C4 = 4 * NW, U = D / 16;
+  constexpr int NT = 64 * NW, C4 = 4 * NW, U = D / 16, kEach = (2 * D + NT - 1) / NT;
   const int c4 = threadIdx.x % C4, d0 = threadIdx.x / C4, H = a.num_heads, Dv = a.v_dim, g = h / (H / a.num_qk_heads);
   const int slot = a.slot_idx[s];
   float* st = slot >= 0 ? a.state + (static_cast<int64_t>(slot) * H + h) * D * Dv + col0 : nullptr;
@@ -139,28 +137,43 @@ __device__ __forceinline__ void scan_single_rows(const ChunkScanArgs& a, int h, 
   const bool carry = st != nullptr && a.context_lens[s] > 0;
   const float constant = a.decay ? a.decay[h] : 1.f, skip = a.skip ? a.skip[h] : 0.f;
   auto act = [](float x) __attribute__((always_inline)) { return Silu ? x / (1.f + expf(-x)) : x; };
+  uint16_t qk[kEach];
+  u32x2 vraw;
+  float decay, b;
+  auto fetch = [&](int64_t t) __attribute__((always_inline)) {
+    const uint16_t *q = a.q + t * a.q_stride + static_cast<int64_t>(g) * D, *k = a.k + t * a.k_stride + static_cast<int64_t>(g) * D;
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+      const int d = threadIdx.x + NT * j;
+      if (d < 2 * D) qk[j] = d < D ? q[d] : k[d - D];
+    }
+    vraw = *reinterpret_cast<const u32x2*>(a.v + t * a.v_stride + static_cast<int64_t>(h) * Dv + col0 + 4 * c4);
+    decay = a.log2_decay ? __builtin_amdgcn_exp2f(a.log2_decay[t * H + h]) : constant;
+    b = a.v_scale ? a.v_scale[t * H + h] : 1.f;
+  };
   f32x4s S[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) S[u] = carry ? *reinterpret_cast<const f32x4s*>(st + static_cast<int64_t>(16 * u) * Dv + at) : f32x4s{0.f, 0.f, 0.f, 0.f};
+  fetch(r0);
   for (int i = 0; i < rows; ++i) {
-    const int64_t t = r0 + i;
-    const uint16_t *q = a.q + t * a.q_stride + static_cast<int64_t>(g) * D, *k = a.k + t * a.k_stride + static_cast<int64_t>(g) * D;
-    float v[4];
-    ActBf16::ld4(a.v + t * a.v_stride + static_cast<int64_t>(h) * Dv + col0 + 4 * c4, v);
-    const float decay = a.log2_decay ? __builtin_amdgcn_exp2f(a.log2_decay[t * H + h]) : constant;
-    const float b = a.v_scale ? a.v_scale[t * H + h] : 1.f;
-    float* part = s_part + (i & 1) * 16 * 16 * NW;
-    if (i > 0) __syncthreads();                        // (the last row's queries and keys are read)
-    for (int d = threadIdx.x; d < D; d += NT) s_row[d] = act(bf2f(q[d])), s_row[D + d] = act(bf2f(k[d]));
+    float *row = s_row + (i & 1) * 2 * D, *part = s_part + (i & 1) * 256 * NW;
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+      const int d = threadIdx.x + NT * j;
+      if (d < 2 * D) row[d] = act(bf2f(qk[j]));
+    }
+    float v[4] = {act(lo_bf(vraw[0])), act(hi_bf(vraw[0])), act(lo_bf(vraw[1])), act(hi_bf(vraw[1]))};
+    const float row_decay = decay, row_b = b;
     __syncthreads();
+    if (i + 1 < rows) fetch(r0 + i + 1);
     f32x4s acc = f32x4s{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = act(v[e]), acc[e] = d0 == 0 ? skip * v[e] : 0.f, v[e] *= b;
+    for (int e = 0; e < 4; ++e) acc[e] = d0 == 0 ? skip * v[e] : 0.f, v[e] *= row_b;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const float qd = s_row[d0 + 16 * u], kd = s_row[D + d0 + 16 * u];
+      const float qd = row[d0 + 16 * u], kd = row[D + d0 + 16 * u];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) S[u][e] = fmaf(decay, S[u][e], kd * v[e]), acc[e] = fmaf(S[u][e], qd, acc[e]);
+      for (int e = 0; e < 4; ++e) S[u][e] = fmaf(row_decay, S[u][e], kd * v[e]), acc[e] = fmaf(S[u][e], qd, acc[e]);
     }
     *reinterpret_cast<f32x4s*>(part + d0 * 16 * NW + 4 * c4) = acc;
     __syncthreads();
@@ -168,13 +181,22 @@ __device__ __forceinline__ void scan_single_rows(const ChunkScanArgs& a, int h, 
       float o = 0.f;
 #pragma unroll
       for (int d = 0; d < 16; ++d) o += part[d * 16 * NW + c];
-      a.out[(t * H + h) * Dv + col0 + c] = o;
+      a.out[(static_cast<int64_t>(r0 + i) * H + h) * Dv + col0 + c] = o;
     }
   }
-  if (st != nullptr && rows > 0) {
+  if (st != nullptr) {
 #pragma unroll
     for (int u = 0; u < U; ++u) *reinterpret_cast<f32x4s*>(st + static_cast<int64_t>(16 * u) * Dv + at) = S[u];
   }
+}
+
+// Portions of 1 to max_rows rows in a launch of their own.  grid = (heads, value columns in slices of 16 NW, sequences).
+template <int D, int NW, bool Silu>
+__global__ __launch_bounds__(64 * NW) void scan_short_kernel(ChunkScanArgs a, int max_rows) {
+  __shared__ __attribute__((aligned(16))) float s_row[2 * 2 * D], s_part[2 * 256 * NW];
+  const int s = blockIdx.z, r0 = a.query_start_loc[s], rows = a.query_start_loc[s + 1] - r0;
+  if (rows <= 0 || rows > max_rows) return;
+  scan_single_rows<D, NW, Silu>(a, blockIdx.x, s, r0, rows, blockIdx.y * 16 * NW, s_row, s_part);
 }
 
 // grid = (heads, value columns in slices of 16 NW, segments + sequences (Summarise: segments)); NW waves.  A workgroup takes a
@@ -194,7 +216,7 @@ __device__ __forceinline__ void scan_single_rows(const ChunkScanArgs& a, int h, 
 // decays per row 316 -> 131; before, 4 waves to 32 value columns, each such workgroup with its own staging, weights and an
 // image of the state in LDS.
 template <int D, int NW, bool Silu, bool Summarise>
-__global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(ChunkScanArgs a, int seg_rows, int segments) {
+__global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(ChunkScanArgs a, int seg_rows, int segments, bool short_too) {
   constexpr int NT = 64 * NW, KC = D / 8, VC = 2 * NW, KP = 2 * D, VP = 32 * NW, SD = D / 32, DB = D / 16;
   constexpr int KPT = (kScanRows * KC + NT - 1) / NT, VPT = 2;
   typedef ChunkOrder<KC> KOrder;
@@ -216,9 +238,9 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
   const int s = seg.seq, r0 = seg.row0, rows_all = seg.rows;
   if (rows_all <= 0) return;                           // (a sequence without rows: its slot may be anything)
   if constexpr (!Summarise) {
-    static_assert(sizeof(s_k) >= 8 * D && sizeof(s_v) >= 2 * 16 * 64 * NW, "the scratch of single rows");
+    static_assert(sizeof(s_k) >= 16 * D && sizeof(s_v) >= 2048 * NW, "the scratch of single rows");
     if (rows_all < kScanMinRows) {                     // (a segment has more)
-      scan_single_rows<D, NW, Silu>(a, h, s, r0, rows_all, vs * 16 * NW, reinterpret_cast<float*>(s_k), reinterpret_cast<float*>(s_v));
+      if (short_too) scan_single_rows<D, NW, Silu>(a, h, s, r0, rows_all, vs * 16 * NW, reinterpret_cast<float*>(s_k), reinterpret_cast<float*>(s_v));
       return;
     }
   }
@@ -533,28 +555,67 @@ __global__ __launch_bounds__(256) void chunk_scan_chain_kernel(ChunkScanArgs a, 
 }
 
 template <int D, int NW, bool Silu>
-void launch_chunk_scan_as(const ChunkScanArgs& a, ScanSegments sg, hipStream_t st) {
+void launch_chunk_scan_as(const ChunkScanArgs& a, ScanSegments sg, bool short_too, hipStream_t st) {
   const dim3 block(64 * NW);
   const unsigned slices = a.v_dim / (16 * NW);
   if (sg.count > 0) {
-    hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, true>), dim3(a.num_heads, slices, sg.count), block, 0, st, a, sg.rows, sg.count);
+    hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, true>), dim3(a.num_heads, slices, sg.count), block, 0, st, a, sg.rows, sg.count, false);
     hipLaunchKernelGGL(chunk_scan_chain_kernel, dim3(a.num_heads, sg.count, (D * a.v_dim + 3071) / 3072), dim3(256), 0, st, a, D, sg.rows, sg.count);
   }
-  hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, false>), dim3(a.num_heads, slices, sg.count + a.num_seqs), block, 0, st, a, sg.rows, sg.count);
+  hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, false>), dim3(a.num_heads, slices, sg.count + a.num_seqs), block, 0, st, a, sg.rows, sg.count, short_too);
 }
 
+// Portions too short for a chunk run in the chunks' launch, where they cost no launch (about 4 us) and fill what a long portion
+// leaves idle.  That launch has registers for 8 waves on a compute unit, though: with states of 64 x 128 that is one workgroup's
+// 32 KB, and (head, short portion) pairs take 11.1 ns each where a launch of their own takes 10.  So those have one where there are
+// more pairs than kManyShort and the chunks fill half of the chip by themselves, or three times as many: 28 heads, 2048 rows beside
+// 255 single ones 139 -> 120 us, 40 portions of 40 beside 200 112 -> 97, but 300 beside 255 85 (91 apart).  Portions of one chunk that
+// seem to fill the chip may be many short ones of several rows, which gain more: a quarter as many pairs (60 of 7 rows beside 40).
+// States of 128 rows are level (23.4 and 25.6 ns).
+//
+// Where no portion has a chunk, theirs is the only launch, and its occupancy hides a row's round trips: 28 heads of 128 x 128, 64
+// portions of 7 rows 102 -> 58 us, 20 43 -> 25; of 64 x 128, 64 portions of 7 rows 77 -> 40 (a thread per value column, before: 156, 80,
+// 55).
+constexpr int kManyShort = 3584;
+// Single rows whose states do not fit the chip's last-level cache (256 MB) pass through memory fastest with 64 KB a compute unit on
+// their way: unused LDS keeps more workgroups away.  28 heads of 128 x 128, 512 single rows 363 -> 315 us; states of 268 MB are faster
+// without (81 against 88 us).
+constexpr int64_t kManyStateBytes = 384ll << 20;
+inline unsigned spare_lds(int head_dim, int used) {
+  const int together = 256 / head_dim;     // workgroups of 64 value columns
+  return 163840 / (together + 1) + 1024 - used;
+}
+
+// A step's rows, of portions of up to max_query_len rows (below kScanMinRows: every portion goes row by row, however long).
 template <bool Silu>
-void launch_chunk_scan(const ChunkScanArgs& a, int head_dim, ScanSegments sg, hipStream_t st) {
+void launch_chunk_scan(const ChunkScanArgs& a, int num_tokens, int head_dim, int max_query_len, ScanSegments sg, hipStream_t st) {
   const int nw = scan_waves(sg.lanes, a.v_dim);
-  auto waves = [&](auto d) {
+  const bool chunks = max_query_len >= kScanMinRows;
+  const int64_t shorts = static_cast<int64_t>(a.num_heads) * (chunks ? a.num_seqs - long_portions(num_tokens, a.num_seqs, max_query_len) : a.num_seqs);
+  const bool filled = sg.lanes * (a.v_dim / (16 * nw)) >= 128;
+  const int most = !filled ? 3 * kManyShort : max_query_len <= kScanRows ? kManyShort / 4 : kManyShort;
+  const bool apart = !chunks || (head_dim <= 64 && nw == 8 && shorts > most);
+  const bool single = !chunks && num_tokens - a.num_seqs <= a.num_seqs / 4;
+  auto launch = [&](auto d) {
     constexpr int D = decltype(d)::value;
-    if (nw == 8) launch_chunk_scan_as<D, 8, Silu>(a, sg, st);
-    else if (nw == 4) launch_chunk_scan_as<D, 4, Silu>(a, sg, st);
-    else launch_chunk_scan_as<D, 2, Silu>(a, sg, st);
+    auto launch_short = [&](auto w) {
+      constexpr int NW = decltype(w)::value, used = 16 * D + 2048 * NW;
+      const unsigned spare = single && shorts * D * a.v_dim * 4 > kManyStateBytes && NW == 4 ? spare_lds(D, used) : 0;
+      hipLaunchKernelGGL((scan_short_kernel<D, NW, Silu>), dim3(a.num_heads, a.v_dim / (16 * NW), a.num_seqs), dim3(64 * NW), spare, st, a,
+                         chunks ? kScanMinRows - 1 : 0x7fffffff);
+    };
+    if (apart) {
+      if (a.v_dim % 64 == 0) launch_short(std::integral_constant<int, 4>{});
+      else launch_short(std::integral_constant<int, 2>{});
+    }
+    if (!chunks) return;
+    if (nw == 8) launch_chunk_scan_as<D, 8, Silu>(a, sg, !apart, st);
+    else if (nw == 4) launch_chunk_scan_as<D, 4, Silu>(a, sg, !apart, st);
+    else launch_chunk_scan_as<D, 2, Silu>(a, sg, !apart, st);
   };
-  if (head_dim == 32) waves(std::integral_constant<int, 32>{});
-  else if (head_dim == 64) waves(std::integral_constant<int, 64>{});
-  else waves(std::integral_constant<int, 128>{});
+  if (head_dim == 32) launch(std::integral_constant<int, 32>{});
+  else if (head_dim == 64) launch(std::integral_constant<int, 64>{});
+  else launch(std::integral_constant<int, 128>{});
 }
 
 }  // namespace

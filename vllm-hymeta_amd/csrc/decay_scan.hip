@@ -191,7 +191,7 @@ extern "C" int hymeta_decay_scan(const hymeta_decay_scan_args* args, hymeta_stre
     const ChunkScanArgs c{static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.k), static_cast<const uint16_t*>(a.v), a.q_stride_t, a.k_stride_t,
                           a.v_stride_t, a.log2_decay ? nullptr : a.decay, a.log2_decay, a.v_scale, a.skip, a.state, a.out, static_cast<float*>(a.workspace),
                           a.query_start_loc, a.context_lens, a.slot_idx, a.num_seqs, a.num_heads, a.num_qk_heads, a.v_dim};
-    launch_chunk_scan<false>(c, a.head_dim, sg, st);
+    launch_chunk_scan<false>(c, a.num_tokens, a.head_dim, a.max_query_len, sg, st);
     return launch_status();
   }
   int min_rows = 1;

@@ -257,7 +257,7 @@ extern "C" int hymeta_lightning_attention(const hymeta_lightning_attention_args*
     const ChunkScanArgs c{qkv, qkv + keys, qkv + 2 * keys, a.qkv_stride_t, a.qkv_stride_t, a.qkv_stride_t, a.decay, nullptr, nullptr, nullptr,
                           a.state, a.out, static_cast<float*>(a.workspace), a.query_start_loc, a.context_lens, a.slot_idx,
                           a.num_seqs, a.num_heads, a.num_heads, a.v_dim};
-    launch_chunk_scan<true>(c, a.head_dim, sg, st);
+    launch_chunk_scan<true>(c, a.num_tokens, a.head_dim, a.max_query_len, sg, st);
     return launch_status();
   }
   int min_rows = 1;
