@@ -1724,10 +1724,11 @@ int hymeta_scaled_key_cache(const hymeta_scaled_key_cache_args* args, hymeta_str
  * query / key head of head h: h / (num_heads / num_qk_heads).  Without norm_weight: out fp32 = o.  With it (every sequence
  * of the step brings one row, max_query_len == 1, v_dim in whole fours that divide 256 fours):
  *   out act_dtype = o / sqrt(mean(o^2) + norm_eps) * norm_weight * silu(gate[t, h])
- * Sequences with one row run a step kernel (beside longer ones part of the first launch); bf16 portions of 8 rows and more run HYMETA_DELTA_CHUNK rows at a time on the
- * matrix cores where head_dim is 32 / 64 / 96 / 128 and v_dim in whole 32s (a launch over all chunks that solves each
- * chunk's triangular system, then one that carries the state through them, products of fp32 quantities in hi + lo bf16
- * parts); everything else token by token. */
+ * bf16 portions of 8 rows and more run HYMETA_DELTA_CHUNK rows at a time on the matrix cores where head_dim is 32 / 64 / 96 / 128
+ * and v_dim in whole 32s (a launch over all chunks that solves each chunk's triangular system, then one that carries the state
+ * through them, products of fp32 quantities in hi + lo bf16 parts); shorter ones go token by token in fp32, beside the chunks or
+ * in a launch of their own; so does everything else, decode steps in a kernel of single rows.  max_query_len: bound of the
+ * portions' rows; below 8 every portion goes token by token, however long. */
 #define HYMETA_DELTA_CHUNK 64
 typedef struct hymeta_delta_rule_args {
   uint32_t struct_size;

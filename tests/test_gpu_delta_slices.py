@@ -35,6 +35,10 @@ def _recurrence(q, k, v, beta, l2, state, starts, context, slots, scale, eps):
     (64, 128, 24, 8, EDGES, 0), (128, 256, 16, 8, EDGES, 0),          # slices of 128
     (64, 128, 2, 1, [200], 0), (128, 32, 2, 2, [65, 5], 0),           # slices of 16
     (128, 128, 4, 2, [2, 7, 1, 3, 6], 0), (256, 64, 2, 2, [2, 5], 0),  # nothing long enough for a chunk
+    (32, 64, 4, 4, [5, 1, 7], 1), (64, 32, 2, 1, [3, 7], 0), (96, 64, 2, 2, [1, 6, 2], 0), (96, 32, 2, 2, [2, 4], 0),
+    # short portions in a launch of their own beside chunks: by their number, as the others fill the chip, by their rows
+    (96, 64, 32, 8, [70, 8] + [1, 3, 7] * 46, 0), (128, 128, 32, 8, [40] + [1] * 36, 0), (64, 64, 16, 16, [40] + [7] * 25, 0),
+    (32, 64, 32, 8, [70, 8] + [1, 3, 7] * 46, 0),        # ... and as many that stay
 ])
 def test_every_slice_against_64_bits(D, Dv, H, Hk, lens, shift):
     """Operands from fp32 enter as two bf16 parts, 2^-17 of the operand each, a few such roundings on the way to an output and

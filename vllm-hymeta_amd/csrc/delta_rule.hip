@@ -78,18 +78,19 @@ __global__ __launch_bounds__(256) void delta_rule_rows_kernel(hymeta_delta_rule_
   }
 }
 
-// The rows t0 .. t1 - 1 of a sequence, one after the other, by 256 threads over the state in fours of value columns: a thread
-// takes the columns 4 c4 .. 4 c4 + 3 of the rows d0, d0 + dstep, ... of S and keeps them in registers (16-byte loads, all in
-// flight together).  S^T k and S^T q of the OLD state are reduced over the row groups in one go; what the token's own write
-// adds to the output is u (k . q), so the state is read once and written once with one reduction per row between.  Norm: the
-// head's output rows go through their RMS norm, weight and silu gate as well.
+// Sequences with one row (decode).  grid = (heads, sequences), 256 threads over the state in fours of value columns: a
+// thread takes the columns 4 c4 .. 4 c4 + 3 of the rows d0, d0 + dstep, ... of S and keeps them in registers (16-byte loads,
+// all in flight together).  S^T k and S^T q of the OLD state are reduced over the row groups in one go; what the token's own
+// write adds to the output is u (k . q), so the state is read once and written once with one reduction between.  Norm: the
+// head's output row goes through its RMS norm, weight and silu gate in the same launch.
 constexpr int kStepMaxD = 256, kStepRows = 16;
-struct StepScratch {
-  __attribute__((aligned(16))) float a[256 * 4], c[256 * 4], u[1024];
-  float q[kStepMaxD], k[kStepMaxD], red[4];
-};
 template <typename A, bool Norm>
-__device__ __forceinline__ void delta_rows(const hymeta_delta_rule_args& a, int h, int s, int t0, int t1, StepScratch& m) {
+__global__ __launch_bounds__(256) void delta_rule_step_kernel(hymeta_delta_rule_args a) {
+  __shared__ float s_q[kStepMaxD], s_k[kStepMaxD];
+  __shared__ __attribute__((aligned(16))) float s_a[256 * 4], s_c[256 * 4], s_u[1024];
+  __shared__ float red[4];
+  const int h = blockIdx.x, s = blockIdx.y, t = a.query_start_loc[s];
+  if (a.query_start_loc[s + 1] - t != 1) return;
   typedef typename A::elem elem;
   const int H = a.num_heads, D = a.head_dim, Dv = a.v_dim, Dv4 = Dv / 4;
   const int g = h / (H / a.num_qk_heads);
@@ -104,91 +105,195 @@ __device__ __forceinline__ void delta_rows(const hymeta_delta_rule_args& a, int 
     const int d = d0 + u * dstep;
     S[u] = (carry && d < D) ? *reinterpret_cast<const f32x4*>(st + u * dstep * Dv + lane_at) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  for (int t = t0; t < t1; ++t) {
-    const elem* q = static_cast<const elem*>(a.q) + static_cast<int64_t>(t) * a.q_stride_t + static_cast<int64_t>(g) * D;
-    const elem* k = static_cast<const elem*>(a.k) + static_cast<int64_t>(t) * a.k_stride_t + static_cast<int64_t>(g) * D;
-    const float decay = exp2_act<A>(fmaxf(a.log2_decay[static_cast<int64_t>(t) * H + h], kMinLog2));
-    const float beta = sigmoid_exact(A::ld(static_cast<const elem*>(a.beta_logit) + static_cast<int64_t>(t) * a.beta_stride_t + h));
-    if (t > t0) __syncthreads();                                  // (the state's update reads the last row's key)
-    // every wave sums the lengths and the product for itself
-    float kk = 0.f, qq = 0.f, kq = 0.f;
-    for (int d = lane; d < D; d += 64) {
-      const float kd = A::ld(k + d), qd = A::ld(q + d);
-      if (threadIdx.x < 64) m.k[d] = kd, m.q[d] = qd;
-      kk = fmaf(kd, kd, kk);
-      qq = fmaf(qd, qd, qq);
-      kq = fmaf(kd, qd, kq);
-    }
-    kk = wave_sum(kk), qq = wave_sum(qq), kq = wave_sum(kq);
-    const float ik = 1.f / sqrtf(kk + a.unit_eps), iq = a.q_scale / sqrtf(qq + a.unit_eps);
-    __syncthreads();
-    f32x4 pa = f32x4{0.f, 0.f, 0.f, 0.f}, pc = pa;
+  const elem* q = static_cast<const elem*>(a.q) + static_cast<int64_t>(t) * a.q_stride_t + static_cast<int64_t>(g) * D;
+  const elem* k = static_cast<const elem*>(a.k) + static_cast<int64_t>(t) * a.k_stride_t + static_cast<int64_t>(g) * D;
+  const float decay = exp2_act<A>(fmaxf(a.log2_decay[static_cast<int64_t>(t) * H + h], kMinLog2));
+  const float beta = sigmoid_exact(A::ld(static_cast<const elem*>(a.beta_logit) + static_cast<int64_t>(t) * a.beta_stride_t + h));
+  // every wave sums the lengths and the product for itself
+  float kk = 0.f, qq = 0.f, kq = 0.f;
+  for (int d = lane; d < D; d += 64) {
+    const float kd = A::ld(k + d), qd = A::ld(q + d);
+    if (threadIdx.x < 64) s_k[d] = kd, s_q[d] = qd;
+    kk = fmaf(kd, kd, kk);
+    qq = fmaf(qd, qd, qq);
+    kq = fmaf(kd, qd, kq);
+  }
+  kk = wave_sum(kk), qq = wave_sum(qq), kq = wave_sum(kq);
+  const float ik = 1.f / sqrtf(kk + a.unit_eps), iq = a.q_scale / sqrtf(qq + a.unit_eps);
+  __syncthreads();
+  f32x4 pa = f32x4{0.f, 0.f, 0.f, 0.f}, pc = pa;
+#pragma unroll
+  for (int u = 0; u < kStepRows; ++u) {
+    const int d = d0 + u * dstep;
+    if (d >= D) continue;
+    const float kd = s_k[d], qd = s_q[d];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) pa[e] = fmaf(S[u][e], kd, pa[e]), pc[e] = fmaf(S[u][e], qd, pc[e]);
+  }
+  *reinterpret_cast<f32x4*>(&s_a[threadIdx.x * 4]) = pa;        // [d0][4 c4 + e]
+  *reinterpret_cast<f32x4*>(&s_c[threadIdx.x * 4]) = pc;
+  __syncthreads();
+  float o[4] = {0.f, 0.f, 0.f, 0.f}, ss = 0.f;                  // columns threadIdx.x, + 256, ...
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    if (c >= Dv) continue;
+    float da = 0.f, dc = 0.f;
+    for (int gg = 0; gg < dstep; ++gg) da += s_a[gg * Dv + c], dc += s_c[gg * Dv + c];
+    const float v = A::ld(static_cast<const elem*>(a.v) + static_cast<int64_t>(t) * a.v_stride_t + static_cast<int64_t>(h) * Dv + c);
+    const float u = beta * (v - decay * (da * ik)) * ik;        // (with the key's length: what multiplies the raw key)
+    s_u[c] = u;
+    o[i] = iq * fmaf(u, kq, decay * dc);
+    ss = fmaf(o[i], o[i], ss);
+  }
+  __syncthreads();
+  if (st != nullptr) {
+    const f32x4 u4 = *reinterpret_cast<const f32x4*>(&s_u[4 * c4]);
 #pragma unroll
     for (int u = 0; u < kStepRows; ++u) {
       const int d = d0 + u * dstep;
       if (d >= D) continue;
-      const float kd = m.k[d], qd = m.q[d];
+      const float kd = s_k[d];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) pa[e] = fmaf(S[u][e], kd, pa[e]), pc[e] = fmaf(S[u][e], qd, pc[e]);
+      for (int e = 0; e < 4; ++e) S[u][e] = fmaf(decay, S[u][e], kd * u4[e]);
+      *reinterpret_cast<f32x4*>(st + u * dstep * Dv + lane_at) = S[u];
     }
-    *reinterpret_cast<f32x4*>(&m.a[threadIdx.x * 4]) = pa;        // [d0][4 c4 + e]
-    *reinterpret_cast<f32x4*>(&m.c[threadIdx.x * 4]) = pc;
-    __syncthreads();
-    float o[4] = {0.f, 0.f, 0.f, 0.f}, ss = 0.f;                  // columns threadIdx.x, + 256, ...
+  }
+  const int64_t at = (static_cast<int64_t>(t) * H + h) * Dv;
+  if constexpr (Norm) {
+    ss = block_sum<4>(ss, red);
+    const float inv = 1.f / sqrtf(ss / static_cast<float>(Dv) + a.norm_eps);
+    const elem* gate = static_cast<const elem*>(a.gate) + static_cast<int64_t>(t) * a.gate_stride_t + static_cast<int64_t>(h) * Dv;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int c = threadIdx.x + 256 * i;
       if (c >= Dv) continue;
-      float da = 0.f, dc = 0.f;
-      for (int gg = 0; gg < dstep; ++gg) da += m.a[gg * Dv + c], dc += m.c[gg * Dv + c];
-      const float v = A::ld(static_cast<const elem*>(a.v) + static_cast<int64_t>(t) * a.v_stride_t + static_cast<int64_t>(h) * Dv + c);
-      const float u = beta * (v - decay * (da * ik)) * ik;        // (with the key's length: what multiplies the raw key)
-      m.u[c] = u;
-      o[i] = iq * fmaf(u, kq, decay * dc);
-      ss = fmaf(o[i], o[i], ss);
+      const float gv = A::ld(gate + c);
+      A::st(static_cast<elem*>(a.out) + at + c, o[i] * inv * a.norm_weight[c] * gv * sigmoid_exact(gv));
     }
-    __syncthreads();
-    if (st != nullptr || t + 1 < t1) {
-      const f32x4 u4 = *reinterpret_cast<const f32x4*>(&m.u[4 * c4]);
+  } else {
 #pragma unroll
-      for (int u = 0; u < kStepRows; ++u) {
-        const int d = d0 + u * dstep;
-        if (d >= D) continue;
-        const float kd = m.k[d];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) S[u][e] = fmaf(decay, S[u][e], kd * u4[e]);
-        if (st != nullptr && t + 1 == t1) *reinterpret_cast<f32x4*>(st + u * dstep * Dv + lane_at) = S[u];
-      }
-    }
-    const int64_t at = (static_cast<int64_t>(t) * H + h) * Dv;
-    if constexpr (Norm) {
-      ss = block_sum<4>(ss, m.red);
-      const float inv = 1.f / sqrtf(ss / static_cast<float>(Dv) + a.norm_eps);
-      const elem* gate = static_cast<const elem*>(a.gate) + static_cast<int64_t>(t) * a.gate_stride_t + static_cast<int64_t>(h) * Dv;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = threadIdx.x + 256 * i;
-        if (c >= Dv) continue;
-        const float gv = A::ld(gate + c);
-        A::st(static_cast<elem*>(a.out) + at + c, o[i] * inv * a.norm_weight[c] * gv * sigmoid_exact(gv));
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = threadIdx.x + 256 * i;
-        if (c < Dv) static_cast<float*>(a.out)[at + c] = o[i];
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      if (c < Dv) static_cast<float*>(a.out)[at + c] = o[i];
     }
   }
 }
 
-// Sequences with one row (decode).  grid = (heads, sequences).
-template <typename A, bool Norm>
-__global__ __launch_bounds__(256) void delta_rule_step_kernel(hymeta_delta_rule_args a) {
-  __shared__ StepScratch m;
-  const int h = blockIdx.x, s = blockIdx.y, t = a.query_start_loc[s];
-  if (a.query_start_loc[s + 1] - t != 1) return;
-  delta_rows<A, Norm>(a, h, s, t, t + 1, m);
+// A portion too short for a chunk, row by row in fp32 by NT threads over 4 C4 value columns of one head: a thread holds 4 columns of
+// U rows of the state.  S^T k and S^T q of the state in front of a row are reduced together, over a wave's lanes and,
+// in LDS, over the waves, whose sums every thread adds up for itself; the next row is on its way while one is worked on.  Two
+// barriers a row, or none with one wave.
+template <int D, int NT>
+struct ShortScratch {
+  __attribute__((aligned(16))) float dots[2][NT / 64][2][64];        // [row parity][wave][k, q][column]
+  __attribute__((aligned(16))) float q[2][D], k[2][D];
+};
+template <int D, int C4, int NT>
+__device__ __forceinline__ void delta_short_rows(const hymeta_delta_rule_args& a, int h, int s, int r0, int rows, int col0, ShortScratch<D, NT>& m) {
+  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+  constexpr int kGroups = NT / C4, U = D / kGroups, kEach = (D + 63) / 64, kWaves = NT / 64;
+  static_assert(D % kGroups == 0 && 4 * C4 <= 64, "the state deals evenly over the threads");
+  // (rows side by side where a thread has many: their queries and keys come four to a read)
+  constexpr int kFirst = NT < 256 ? U : 1, kNext = NT < 256 ? 1 : kGroups;
+  const int c4 = threadIdx.x % C4, d0 = threadIdx.x / C4 * kFirst, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int H = a.num_heads, Dv = a.v_dim, g = h / (H / a.num_qk_heads);
+  const int slot = a.slot_idx[s];
+  float* st = slot >= 0 ? a.state + (static_cast<int64_t>(slot) * H + h) * D * Dv + col0 : nullptr;
+  const bool carry = st != nullptr && a.context_lens[s] > 0;
+  const uint32_t at = d0 * Dv + 4 * c4;
+  f32x4 S[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) S[u] = carry ? *reinterpret_cast<const f32x4*>(st + u * kNext * Dv + at) : f32x4{0.f, 0.f, 0.f, 0.f};
+  uint16_t kr[kEach], qr[kEach], vr[4], br;
+  float l2;
+  auto fetch = [&](int64_t t) __attribute__((always_inline)) {
+    const uint16_t* q = static_cast<const uint16_t*>(a.q) + t * a.q_stride_t + static_cast<int64_t>(g) * D;
+    const uint16_t* k = static_cast<const uint16_t*>(a.k) + t * a.k_stride_t + static_cast<int64_t>(g) * D;
+    const uint16_t* v = static_cast<const uint16_t*>(a.v) + t * a.v_stride_t + static_cast<int64_t>(h) * Dv + col0 + 4 * c4;
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+      const int d = min(lane + 64 * j, D - 1);
+      kr[j] = k[d], qr[j] = q[d];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) vr[e] = v[e];
+    l2 = a.log2_decay[t * H + h];
+    br = static_cast<const uint16_t*>(a.beta_logit)[t * a.beta_stride_t + h];
+  };
+  fetch(r0);
+  for (int i = 0; i < rows; ++i) {
+    const int at_row = i & 1;
+    float kk = 0.f, qq = 0.f, kq = 0.f, v[4];
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+      const int d = lane + 64 * j;
+      const bool in = D % 64 == 0 || d < D;
+      const float kd = in ? bf2f(kr[j]) : 0.f, qd = in ? bf2f(qr[j]) : 0.f;
+      if (wave == 0 && in) m.k[at_row][d] = kd, m.q[at_row][d] = qd;
+      kk = fmaf(kd, kd, kk), qq = fmaf(qd, qd, qq), kq = fmaf(kd, qd, kq);
+    }
+    kk = wave_sum(kk), qq = wave_sum(qq), kq = wave_sum(kq);         // (every wave for itself)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = bf2f(vr[e]);
+    const float decay = __builtin_amdgcn_exp2f(fmaxf(l2, kMinLog2)), beta = sigmoid_exact(bf2f(br));
+    const float ik = 1.f / sqrtf(kk + a.unit_eps), iq = a.q_scale / sqrtf(qq + a.unit_eps);
+    __syncthreads();                                                 // the row's queries and keys are there
+    if (i + 1 < rows) fetch(r0 + i + 1);
+    float kd[U];
+    f32x4 pa = f32x4{0.f, 0.f, 0.f, 0.f}, pc = pa;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      kd[u] = m.k[at_row][d0 + u * kNext];
+      const float qd = m.q[at_row][d0 + u * kNext];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pa[e] = fmaf(S[u][e], kd[u], pa[e]), pc[e] = fmaf(S[u][e], qd, pc[e]);
+    }
+#pragma unroll
+    for (int x = C4; x < 64; x <<= 1)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pa[e] += __shfl_xor(pa[e], x, 64), pc[e] += __shfl_xor(pc[e], x, 64);
+    if constexpr (kWaves > 1) {
+      if (lane < C4) {
+        *reinterpret_cast<f32x4*>(&m.dots[at_row][wave][0][4 * c4]) = pa;
+        *reinterpret_cast<f32x4*>(&m.dots[at_row][wave][1][4 * c4]) = pc;
+      }
+      __syncthreads();
+      pa = pc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int x = 0; x < kWaves; ++x) pa += *reinterpret_cast<const f32x4*>(&m.dots[at_row][x][0][4 * c4]);
+      if (d0 == 0) {
+#pragma unroll
+        for (int x = 0; x < kWaves; ++x) pc += *reinterpret_cast<const f32x4*>(&m.dots[at_row][x][1][4 * c4]);
+      }
+    }
+    f32x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = beta * (v[e] - decay * (pa[e] * ik)) * ik;       // (with the key's length: what multiplies the raw key)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[u][e] = fmaf(decay, S[u][e], kd[u] * w[e]);
+    if (d0 == 0) {
+      f32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = iq * fmaf(w[e], kq, decay * pc[e]);
+      *reinterpret_cast<f32x4_any*>(static_cast<float*>(a.out) + (static_cast<int64_t>(r0 + i) * H + h) * Dv + col0 + 4 * c4) = o;
+    }
+  }
+  if (st != nullptr) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) *reinterpret_cast<f32x4*>(st + u * kNext * Dv + at) = S[u];
+  }
+}
+
+// Portions of 1 to max_rows rows in a launch of their own.  grid = (heads, value columns in slices of 4 C4, sequences).
+template <int D, int C4, int NT>
+__global__ __launch_bounds__(NT) void delta_short_kernel(hymeta_delta_rule_args a, int max_rows) {
+  __shared__ ShortScratch<D, NT> m;
+  const int s = blockIdx.z, r0 = a.query_start_loc[s], rows = a.query_start_loc[s + 1] - r0;
+  if (rows <= 0 || rows > max_rows) return;
+  delta_short_rows<D, C4, NT>(a, blockIdx.x, s, r0, rows, blockIdx.y * 4 * C4, m);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -217,9 +322,22 @@ constexpr int kChunk = HYMETA_DELTA_CHUNK;
 // 177 us, 301 before; five of 1801 (280, in slices of 128) 182, 280 before.
 // All count the portions that the step's rows are worth (long_portions): single rows leave the chip to a long prompt.
 constexpr int kFewGroups = 128, kIdleGroupsPerRow = 10, kManyGroups = 256;
-// (head, short portion) pairs up to which those run in the first launch and not in their own, which have more workgroups on a
-// compute unit: 28 heads, 2048 rows beside 63 single ones (1764 pairs) 129 against 141 us, 40 beside 255 (7140) 246 against 230.
-constexpr int kManyShort = 4096;
+// Whether portions too short for a chunk have a launch of their own and do not run in the chunks' first one, where they cost no
+// launch (about 4 us) and stand beside the chunks' work, but go through a head's value columns 64 at a time with the registers of
+// that kernel.  `shorts`: the (head, short portion) pairs that there may be.  Us in the first launch / in their own:
+//   28 heads of 128 x 128: 40 rows beside 15 single ones (420 pairs) 24.6 / 27.9, beside 63 56.7 / 55.0, beside 127 105 / 92; 2048
+//   beside 63 127 / 131, beside 255 330 / 294; 16 heads, 2048 beside 255 (4080) 184 / 196: with few rows in chunks from 1000 pairs on,
+//   else from 4096.
+//   28 heads of 64 x 128: 40 beside 63 29.7 / 36.8, beside 255 85 / 97, 2048 beside 255 179 / 176: single rows stay.
+//   60 portions of 7 rows beside 40: 64 x 128 79 / 52, 128 x 128 98 / 80: where the longest fits a chunk and the others have two rows
+//   each, apart.
+//   Three or four times through the columns, four portions of 600 beside three of 5: 8 heads of 128 x 256 72 / 55, 16 of 32 x 96 55 / 49.
+inline bool short_apart(const hymeta_delta_rule_args& a, int64_t shorts) {
+  if (a.v_dim > 128 || a.v_dim % 64 != 0 || (a.head_dim > 64 && shorts > 4096)) return true;
+  const int64_t chunks = static_cast<int64_t>(a.num_heads) * (a.num_tokens / kChunk);
+  if (a.head_dim > 64 && shorts > 1000 && 10 * chunks < shorts) return true;
+  return shorts > 256 && a.max_query_len <= kChunk && a.num_tokens - a.max_query_len >= 2 * (a.num_seqs - 1);
+}
 constexpr int kChunkMinRows = 8;            // shorter portions go token by token
 constexpr int kMat = kChunk * kChunk;
 // Where the second launch reads 64 x 64 matrices (or the chunk's keys) as matrix operands, they lie in the operand's own
@@ -259,12 +377,9 @@ __device__ __forceinline__ void split4(const float* v, u32x2& hi, u32x2& lo) {
 __host__ __device__ inline size_t rows_at(int64_t chunks, int heads) { return static_cast<size_t>(chunks) * heads * sizeof(ChunkPlace); }
 
 // grid = (chunk numbers, heads), 4 waves with 16 rows of the chunk each.
-// Portions of up to short_rows rows go token by token here (0: none do; the state fits the threads' registers), so that they need
-// no launch of their own: two launches with nothing to do took 9 of the 280 us of five portions of 1801 rows.  The caller's bound
-// of the rows says whether there are chunks, and with them a workspace: below kChunkMinRows every portion goes token by token,
-// however long it turns out to be.
+// Portions shorter than kChunkMinRows go row by row here (short_too), all of a head's value columns in turn.
 template <int D, bool Pack>
-__global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hymeta_delta_rule_args a, int64_t chunks, int short_rows) {
+__global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hymeta_delta_rule_args a, int64_t chunks, bool short_too) {
   constexpr int PK = D + 8, PF = kChunk + 4;
   // (the keys and T share their place where nothing asks for the keys again: four workgroups to a compute unit)
   constexpr int kKeyBytes = kChunk * PK * 2, kMatrixBytes = kChunk * PF * 4;
@@ -284,9 +399,15 @@ __global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hy
   const int r0 = a.query_start_loc[s], rows = a.query_start_loc[s + 1] - r0;
   const int c0 = (number - (r0 / kChunk + s)) * kChunk;
   if (c0 >= rows) return;
-  if (rows < kChunkMinRows || rows <= short_rows) {
-    static_assert(sizeof(StepScratch) <= sizeof(sA), "the scratch lies where A would");
-    if (rows <= short_rows && c0 == 0) delta_rows<ActBf16, false>(a, blockIdx.y, s, r0, r0 + rows, *reinterpret_cast<StepScratch*>(sA));
+  if (rows < kChunkMinRows) {
+    static_assert(sizeof(ShortScratch<D, 256>) <= sizeof(sA), "the scratch lies where A would");
+    if (!short_too) return;
+    ShortScratch<D, 256>& m = *reinterpret_cast<ShortScratch<D, 256>*>(sA);
+    if (a.v_dim % 64 == 0) {
+      for (int col0 = 0; col0 < a.v_dim; col0 += 64) delta_short_rows<D, 16, 256>(a, blockIdx.y, s, r0, rows, col0, m), __syncthreads();
+    } else {
+      for (int col0 = 0; col0 < a.v_dim; col0 += 32) delta_short_rows<D, 8, 256>(a, blockIdx.y, s, r0, rows, col0, m), __syncthreads();
+    }
     return;
   }
   const int nrow = min(kChunk, rows - c0), h = blockIdx.y, H = a.num_heads, group = H / a.num_qk_heads, g = h / group;
@@ -959,21 +1080,26 @@ void launch_rows(const hymeta_delta_rule_args& a, hipStream_t st, int min_rows, 
 }
 
 template <int D>
+void launch_short(const hymeta_delta_rule_args& a, hipStream_t st, int max_rows) {
+  constexpr int NT = D <= 64 ? 64 : 128;
+  if (a.v_dim % 64 == 0) hipLaunchKernelGGL((delta_short_kernel<D, 16, NT>), dim3(a.num_heads, a.v_dim / 64, a.num_seqs), dim3(NT), 0, st, a, max_rows);
+  else hipLaunchKernelGGL((delta_short_kernel<D, 8, NT>), dim3(a.num_heads, a.v_dim / 32, a.num_seqs), dim3(NT), 0, st, a, max_rows);
+}
+
+template <int D>
 void launch_chunks(const hymeta_delta_rule_args& a, hipStream_t st, int64_t chunks, bool short_too) {
-  const int short_rows = !short_too ? 0 : a.max_query_len < kChunkMinRows ? 0x7fffffff : kChunkMinRows - 1;
   const int64_t portions = long_portions(a.num_tokens, a.num_seqs, a.max_query_len), lanes = a.num_heads * portions;
   const int64_t idle = a.num_heads * (a.num_seqs - portions) * (a.v_dim / 32);
   const bool narrow = D % 64 == 0 && lanes * (a.v_dim / 32) <= kFewGroups && idle <= static_cast<int64_t>(kIdleGroupsPerRow) * a.max_query_len;
   const dim3 solve(static_cast<unsigned>(chunks), a.num_heads);
   if constexpr (D % 64 == 0) {
-    if (narrow && a.max_query_len >= kChunkMinRows) {
-      hipLaunchKernelGGL((delta_chunk_solve_kernel<D, true>), solve, dim3(256), 0, st, a, chunks, short_rows);
+    if (narrow) {
+      hipLaunchKernelGGL((delta_chunk_solve_kernel<D, true>), solve, dim3(256), 0, st, a, chunks, short_too);
       hipLaunchKernelGGL(delta_chunk_narrow_kernel<D>, dim3(a.num_heads, a.num_seqs, a.v_dim / 16), dim3(256), 0, st, a, chunks);
       return;
     }
   }
-  hipLaunchKernelGGL((delta_chunk_solve_kernel<D, false>), solve, dim3(256), 0, st, a, chunks, short_rows);
-  if (a.max_query_len < kChunkMinRows) return;
+  hipLaunchKernelGGL((delta_chunk_solve_kernel<D, false>), solve, dim3(256), 0, st, a, chunks, short_too);
   auto launch = [&](auto nw) {
     constexpr int NW = decltype(nw)::value;
     hipLaunchKernelGGL((delta_chunk_wide_kernel<D, NW>), dim3(a.num_heads, a.num_seqs, a.v_dim / (16 * NW)), dim3(64 * NW), 0, st, a);
@@ -1017,17 +1143,27 @@ extern "C" int hymeta_delta_rule(const hymeta_delta_rule_args* args, hymeta_stre
   hipStream_t st = begin_launches(stream);
   const bool bf = a.act_dtype == HYMETA_BF16;
   int min_rows = 1, max_rows = 0x7fffffff;
-  const int64_t idle = static_cast<int64_t>(a.num_heads) * (a.num_seqs - long_portions(a.num_tokens, a.num_seqs, a.max_query_len));
-  const bool short_too = step && idle <= kManyShort;
-  if (chunk_shape(a) && a.max_query_len >= (short_too ? 2 : kChunkMinRows)) {
+  const bool rows_too = reinterpret_cast<uintptr_t>(a.state) % 16 == 0;          // (the kernels of short portions read the state in fours)
+  if (chunk_shape(a) && a.max_query_len >= (rows_too ? 2 : kChunkMinRows)) {
+    auto dims = [&](auto&& run) {
+      if (a.head_dim == 32) run(std::integral_constant<int, 32>{});
+      else if (a.head_dim == 64) run(std::integral_constant<int, 64>{});
+      else if (a.head_dim == 96) run(std::integral_constant<int, 96>{});
+      else run(std::integral_constant<int, 128>{});
+    };
+    if (a.max_query_len < kChunkMinRows) {
+      dims([&](auto d) { launch_short<decltype(d)::value>(a, st, max_rows); });
+      return launch_status();
+    }
     const size_t need = hymeta_delta_rule_workspace_bytes(a.num_tokens, a.num_seqs, a.num_heads, a.num_qk_heads, a.head_dim, a.v_dim, a.act_dtype, a.max_query_len);
-    if (need > 0 && (!a.workspace || a.workspace_bytes < need || reinterpret_cast<uintptr_t>(a.workspace) % 16 != 0)) return HYMETA_ERR_WORKSPACE;
-    const int64_t chunks = chunk_numbers(a.num_tokens, a.num_seqs);
-    if (a.head_dim == 32) launch_chunks<32>(a, st, chunks, short_too);
-    else if (a.head_dim == 64) launch_chunks<64>(a, st, chunks, short_too);
-    else if (a.head_dim == 96) launch_chunks<96>(a, st, chunks, short_too);
-    else launch_chunks<128>(a, st, chunks, short_too);
-    if (short_too) return launch_status();
+    if (!a.workspace || a.workspace_bytes < need || reinterpret_cast<uintptr_t>(a.workspace) % 16 != 0) return HYMETA_ERR_WORKSPACE;
+    const int64_t shorts = static_cast<int64_t>(a.num_heads) * (a.num_seqs - long_portions(a.num_tokens, a.num_seqs, a.max_query_len));
+    const bool apart = rows_too && short_apart(a, shorts);
+    dims([&](auto d) {
+      if (apart) launch_short<decltype(d)::value>(a, st, kChunkMinRows - 1);
+      launch_chunks<decltype(d)::value>(a, st, chunk_numbers(a.num_tokens, a.num_seqs), rows_too && !apart);
+    });
+    if (rows_too) return launch_status();
     max_rows = kChunkMinRows - 1;
   }
   if (step) {
