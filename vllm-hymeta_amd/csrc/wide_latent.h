@@ -453,6 +453,11 @@ __global__ __launch_bounds__(64 * kLatentWaves) void latent_decode_kernel(hymeta
   const int v_lo = split * per, v_hi = min(tiles, v_lo + per) - 1;
   auto key0 = [&](int v) { return (v < kept ? v * kTile : from + (v - kept) * kTile) + kLatentKeys * wave; };
 
+  // (in front of the queries, whose loads the first tile's copies would otherwise wait for)
+  LatentCopy<D, kLatentKeys, 1> copy(a, a.block_tables + static_cast<int64_t>(s) * a.block_table_stride, g, 0);
+  const bool fits = copy.fits();
+  const int looked_up = fits ? v_hi + 1 : 0;
+  if (v_lo <= v_hi) copy.refill(v_lo, looked_up, pos, key0, true);
   bf16x8 qf[kSteps];
   f32x4v o[C / 16];
   float m = -INFINITY, l = 0.f;
@@ -466,7 +471,6 @@ __global__ __launch_bounds__(64 * kLatentWaves) void latent_decode_kernel(hymeta
   }
 #pragma unroll
   for (int cb = 0; cb < C / 16; ++cb) o[cb] = f32x4v{0.f, 0.f, 0.f, 0.f};
-  LatentCopy<D, kLatentKeys, 1> copy(a, a.block_tables + static_cast<int64_t>(s) * a.block_table_stride, g, 0);
   constexpr int kLoads = LatentCopy<D, kLatentKeys, 1>::kInstr;
   char* ring = sm.bytes + wave * 2 * Smem::kStage;
   const int swz = (n >> 1) & 7;
@@ -479,15 +483,13 @@ __global__ __launch_bounds__(64 * kLatentWaves) void latent_decode_kernel(hymeta
   }
 
   // (a wave whose 16 keys lie past the last one copies the last one and skips them)
-  const bool fits = copy.fits();
-  const int whole = key0(tiles - 1) + kLatentKeys - 1 <= pos ? tiles : tiles - 1, looked_up = fits ? v_hi + 1 : 0;
+  const int whole = key0(tiles - 1) + kLatentKeys - 1 <= pos ? tiles : tiles - 1;
   auto copy_tile = [&](int v, char* image) __attribute__((always_inline)) {
     if (!fits) copy.issue(min(key0(v), pos), pos, image);
     else if (v < whole) copy.issue_whole(v, image);
     else copy.issue_part(v, max(1, pos + 1 - key0(v)), image);
   };
   if (v_lo <= v_hi) {
-    copy.refill(v_lo, looked_up, pos, key0, true);
     copy_tile(v_lo, ring);
     if (v_lo < v_hi) copy_tile(v_lo + 1, ring + Smem::kStage);
   }
