@@ -197,3 +197,14 @@ def test_advance_step_updates_device_metadata():
     assert md.seq_lens == [5, 6] and md.seq_lens_tensor.tolist() == [5, 6] and md.max_decode_seq_len == 6
     assert mi.input_tokens.tolist() == [11, 12] and mi.input_positions.tolist() == [4, 5]
     assert md.slot_mapping.tolist() == [1 * 4 + 0, 5 * 4 + 1]
+
+
+@pytest.mark.parametrize("index", [0, None])
+def test_current_stream_without_torchs_private_name(monkeypatch, index):
+    """A torch without it: the public Stream object's handle, of the tensor's device."""
+    from vllm_hymeta import hip_ops
+    asked = []
+    monkeypatch.setattr(hip_ops, "_current_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: asked.append(device) or types.SimpleNamespace(cuda_stream=4096))
+    device = torch.device("cuda") if index is None else torch.device("cuda", index)
+    assert hip_ops._raw_stream(device) == 4096 and asked == [device]

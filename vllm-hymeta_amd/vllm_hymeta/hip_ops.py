@@ -21,8 +21,13 @@ _DT = {torch.bfloat16: _C.HYMETA_BF16, torch.float32: _C.HYMETA_F32}
 # What stands around every call.  A small step's kernels take less than the call does (attention over two portions of 125 rows 22 us
 # of host time against 15 on the GPU), so addresses go into the structs as plain numbers, the current stream is asked for
 # without building a Stream object, and messages are put together when they are needed.
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)       # (not a public name of torch)
+
+
 def _raw_stream(device: torch.device) -> int:
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
+    if _current_raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _current_raw_stream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def _stream(t: torch.Tensor) -> int:
