@@ -26,13 +26,14 @@ def _dense(q, keys, values, ctx, window, meta_k, meta_v):
     return torch.einsum("hnl,lhd->nhd", p, v)
 
 
+@pytest.mark.parametrize("splits", [0, 1])                    # (by the rule, and one that walks all tiles)
 @pytest.mark.parametrize("page", [16, 48, 64, 192, 256])
 @pytest.mark.parametrize("rows,lens,H,G,M,window", [
     ([3, 40, 1], [4500, 100, 64], 7, 1, 0, -1),              # more tiles than a lane table holds; rows over two waves
     ([19, 37], [83, 4300], 14, 2, 32, 200),                  # half a tile of meta keys, a window far into a sequence
     ([129, 65], [129, 1000], 4, 4, 64, 63),                  # one head per key: a block of 128 queries and one more
 ])
-def test_paged_rows(page, rows, lens, H, G, M, window):
+def test_paged_rows(page, rows, lens, H, G, M, window, splits):
     from vllm_hymeta import hip_ops
 
     g_ = gen(3)
@@ -56,7 +57,7 @@ def test_paged_rows(page, rows, lens, H, G, M, window):
     cache[:, ~live] = float("nan")                           # rows behind a sequence's end are nobody's
     kv = cache.cuda()
     out = hip_ops.meta_swa_prefill(q.cuda(), cu.cuda(), max(rows), key_cache=kv[0], value_cache=kv[1], block_tables=table.cuda(),
-                                   seq_lens_k=torch.tensor(lens, dtype=torch.int32).cuda(), window_left=window, max_seqlen_k=max(lens),
+                                   seq_lens_k=torch.tensor(lens, dtype=torch.int32).cuda(), window_left=window, max_seqlen_k=max(lens), num_splits=splits,
                                    **(dict(meta_key=meta[0].cuda(), meta_value=meta[1].cuda()) if M else {}))
     assert_bf16_close(out.cpu(), torch.cat(want), f"pages of {page}")
 
