@@ -1,5 +1,5 @@
-// Prompts' portions of the attention over paged rows, keys of up to 192 elements, where the value lies inside the key or a cap
-// meets a bias (the others: row_pipe.h): included by sink_attn.hip.
+// Prompts' portions of the attention over paged rows, keys of up to 192 elements, where the value lies inside the key or is it, one
+// key for all heads meets a cap or a bias, or a cap meets a bias (the others: row_pipe.h): included by sink_attn.hip.
 #pragma once
 
 #include "row_copy.h"
@@ -24,10 +24,8 @@ constexpr float kLazyMax2 = 8.f;     // the softmax reference may trail a row's 
 // kernel needs the port for its scores (measured level, with less to read from LDS and fewer registers).  The scores are
 // formed relative to the row's running reference, which moves only when a score exceeds it by 2^8 (or at the row's first
 // visible key): no maximum across lanes, no subtraction and no pass over the output registers on most tiles.
-// Bound by the vector and the matrix pipe in turn: with a logarithm and an exponential per score they are busy 56 and 43 % of
-// the time and hardly at once, whatever the number of waves (one row block a wave and four waves a SIMD: 785 us).  8192 rows x
-// 28 heads of 128 with 4 key/value heads, logarithmic bias: 1398 -> 759 us; a latent of 128 + 64: 1629 -> 745; a window of 1024:
-// 406 -> 198; key and value in one vector, window of 1024: 357 -> 230; chunks of 2048: 414 -> 199.
+// Bound by the vector and the matrix pipe in turn, hardly ever busy at once.  8192 rows x 28 heads on a latent of 128 + 64: 1629 ->
+// 745 us; key and value in one vector, 4 key/value heads of 128, window of 1024: 357 -> 230.
 template <int D, int DV, int Layout>
 struct RowShape {
   static constexpr bool Scaled = Layout == HYMETA_KV_SCALED_KEY, Inside = Layout == HYMETA_KV_VALUE_IN_KEY || Scaled, Shared = Layout == HYMETA_KV_SHARED_KEY;
@@ -38,11 +36,12 @@ struct RowShape {
 };
 
 // How a score follows from its product, in kernels of their own where a design's every layer asks for it: a branch per row
-// block in the middle of a tile keeps the compiler from overlapping what stands on its two sides.
+// block in the middle of a tile keeps the compiler from overlapping what stands on its two sides.  (kLogBias, kCapped: row_pipe.h)
 enum ScoreRule { kPlain, kLogBias, kCapped, kAnyRule };
 
 template <int D, int DV, int Layout, int Rule>
 __global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attention_args a, PortionSlices ps) {
+  static_assert(Rule == kPlain || Rule == kAnyRule, "the others are row_pipe_kernel's");
   typedef RowShape<D, DV, Layout> S;
   constexpr int kSteps = D / 16, CB = DV / 32;
   __shared__ __attribute__((aligned(16))) char s_rows[2][S::kImage];
@@ -148,7 +147,6 @@ __global__ __launch_bounds__(256, 2) void row_prefill_kernel(hymeta_sink_attenti
           float x = sc[t][4 * i + e];
           const float away = static_cast<float>(32 * t + 8 * i + e);
           if (S::Scaled) x = fmaf(x, f[e], fmaf(-ba, away, slope));
-          else if (Rule == kLogBias) x = fmaf(x, scale2, fmaf(ba, __builtin_amdgcn_logf(fmaf(bb, d0 - away, 1.f)), -ref));
           else if (Rule == kPlain) x = fmaf(x, scale2, -ref);
           sc[t][4 * i + e] = x;
         }

@@ -12,8 +12,8 @@ namespace {
 // The matrix pipe so runs under the wave's own vector work.  Keys and values lie in images of their own, two each; what a tile's
 // bookkeeping needs is worked out in front of the loop.
 //
-// Bound by power: with a logarithmic bias the vector pipe is 71 % and the matrix pipe 53 % busy at 1.84 GHz, and a quarter fewer
-// vector instructions (a weight's low part through v_dot2_f32_bf16) change nothing.  Row_prefill_kernel -> here on one box:
+// Bound by the vector and the matrix pipe together: with a logarithmic bias they are busy 69 and 56 % of the time, the waves wait 15 %
+// of theirs, and the clock is 1.9 GHz, where kernels that use either pipe less run at 2.4.  Row_prefill_kernel -> here on one box:
 // 8192 rows x 28 heads of 128 with 4 key/value heads, logarithmic bias 754 -> 695 us, a window of 1024 201 -> 184; three portions
 // of 700 behind 1000 94.8 -> 75; six of 324 behind 818, window 1024, 60.6 -> 49; four of 1500 behind 3000, 16 heads, chunks of
 // 2048, 120 -> 111; 4000 rows capped, window 1024, 115 -> 108.

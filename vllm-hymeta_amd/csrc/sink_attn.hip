@@ -1119,7 +1119,8 @@ inline dim3 portion_grid(const hymeta_sink_attention_args& a, const PortionSlice
 // the single rows' are as well; few of them, as a slice of theirs has a workgroup of 128 rows to itself: 7 rows behind 6000 26.8 ->
 // 20.6 us, 40 beside 8 single ones 50.3 -> 46.4 (latents of 128 + 64: 48.0 -> 38.3), 8 beside 15 behind 3000 40.7 -> 34.5 (of each
 // about 5 the host's shorter call).  With one key/value head, whose single rows fill a fifth of a block, a quarter as many: 300 rows beside 8
-// single ones of 4096 keys on latents of 128 + 64 46 -> 49, beside 63 75 -> 86.
+// single ones of 4096 keys on latents of 128 + 64 46 -> 49, beside 63 75 -> 86.  A logarithm per score makes them dearer: 40 rows with nothing
+// in front beside 15 single ones of 4096 keys 39.7 -> 42.3, but 2 behind 3000 beside 15 of 3000 40.3 -> 37.0.
 constexpr int kFewTiles = 16, kFewWideTiles = 2, kManySingleRows = 512, kFewSingleRows = 4;
 inline bool one_launch(const hymeta_sink_attention_args& a, const PortionSlices& ps, int most) {
   const int64_t singles = a.num_seqs - long_portions(a.num_tokens, a.num_seqs, a.max_query_len);

@@ -22,7 +22,7 @@
 // with everything 359 (1.0 PFLOP/s); copies cost 6 %, barriers and the look at
 // the reference 3 % each.  Against a workgroup per head with operands through
 // registers, one tile at a time: 647 -> 359 us here, a chunk of 2048 at 32k of
-// 7 heads on one kv-head 368 -> 248, one prompt of 32768 (window 4097) 1968 ->
+// 7 heads on one kv-head 365 -> 238, one prompt of 32768 (window 4097) 1968 ->
 // 1709, eight of 4096 1739 -> 962, four chunks of 5 tokens behind 7922 65 -> 26.
 // Eight waves to a workgroup, which read the keys half as often: level at
 // prompts of 8192 and more, 3 to 20 % slower below and with few heads.  The
@@ -488,8 +488,11 @@ static size_t prefill_partial_bytes(int64_t rows, int heads, int splits) {
   return static_cast<size_t>(splits) * rows * heads * (kHeadDim + 2) * sizeof(float);
 }
 
-// Key slices for a call: only when 128-query workgroups leave most compute units idle and every
-// slice still walks a fair number of tiles (a bound from the window or max_seqlen_k; unknown: 1).
+// Key slices for a call: only where the rows would leave most compute units idle and every slice
+// still walks a fair number of tiles (a bound from the window or max_seqlen_k; unknown: 1).  Rows are
+// counted in blocks of 128 (256) queries of one head.  The blocks launched are fewer where a kv-head
+// has several heads and a sequence few queries, as those lie side by side: 8 queries of 7 heads behind
+// 32768 keys are one block in 8 slices (77 us).
 extern "C" int hymeta_meta_swa_prefill_splits(int32_t total_q, int32_t num_heads, int32_t num_meta, int32_t meta_rows,
                                               int32_t window_left, int32_t max_seqlen_k) {
   if (total_q <= 0 || num_heads <= 0) return 1;
@@ -500,7 +503,7 @@ extern "C" int hymeta_meta_swa_prefill_splits(int32_t total_q, int32_t num_heads
   if (window_left >= 0 && (keys < 0 || window_left + 128 < keys)) keys = window_left + 128;
   if (keys < 0) return 1;
   const int64_t tiles = (keys + kTileK - 1) / kTileK + 1 + (num_meta + kTileK - 1) / kTileK;
-  int64_t splits = 512 / (wgs128 > 0 ? wgs128 : 1);          // two 128-query workgroups fit a compute unit
+  int64_t splits = 512 / (wgs128 > 0 ? wgs128 : 1);          // two workgroups fit a compute unit
   if (splits > tiles / 8) splits = tiles / 8;
   if (splits > kMaxPrefillSplits) splits = kMaxPrefillSplits;
   return splits < 2 ? 1 : static_cast<int>(splits);

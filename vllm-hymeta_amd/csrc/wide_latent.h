@@ -46,8 +46,7 @@ __device__ __forceinline__ void finish_scores(const hymeta_sink_attention_args& 
 // places of 8 rows are enough.  Where a tile's first row lies is looked up for 64 tiles at once:
 // a load in front of every tile's copies waits for all that are on their way.  So does a register that lies in scratch memory;
 // with 512 + 64 the prompts' form has none left over, works its places out on every tile and parks the queries' last two steps in
-// LDS.  8192 rows x 16 heads on 512 + 64 1614 -> 1404 us, a decode step of 64 sequences x 4096 71.2 -> 66.4 (the look-ups and
-// places alone 1615 -> 1441 and all of 5 us).
+// LDS.  8192 rows x 16 heads on 512 + 64 1618 -> 1440 us, a decode step of 64 sequences x 4096 70.8 -> 64.4.
 template <int D, int Keys, int Waves>
 struct LatentCopy {
   static constexpr int kChunks = D / 8, kInstr = Keys * kChunks / 64, kEight = kChunks / 8;
@@ -152,9 +151,9 @@ struct WideSmem {
 // Per tile of 32 keys a workgroup issues 800 matrix instructions (C = 512) against 480 LDS reads of 1 KB; a step computes
 // the scores of tile t + 1 and adds tile t's values, which do not depend on each other: the two waves of a SIMD do them in
 // opposite order, so that one's softmax runs under the other's products.  One barrier per tile.  Bound by the matrix
-// and the vector pipes, busy 51 and 40 % of the time at 2.05 GHz: 8192 rows x 16 heads on 512 + 64: 1.40 ms = 1.23 PFLOP/s of the
-// products issued (both parts of the weights counted), where launches over value slices of 128, each repeating the scores, took
-// 11.3 ms.  Fragments of the keys three ahead (two: 1.408, five: 1.406).  Plain: neither a bias nor a cap on the scores.
+// and the vector pipes, busy 51 and 40 % of the time (the waves wait 29 % of theirs): 8192 rows x 16 heads on 512 + 64: 1.44 ms = 1.20
+// PFLOP/s of the products issued (both parts of the weights counted), where launches over value slices of 128, each repeating the
+// scores, took 11.3 ms.  Fragments of the keys three ahead (two and five: level).  Plain: neither a bias nor a cap on the scores.
 template <int C, bool Plain>
 __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_sink_attention_args a, PortionSlices ps) {
   constexpr int D = C + 64, kRowB = 2 * D, kSteps = D / 32, CB = C / 128, kParked = WideSmem<C>::kParked, kAhead = 3;
@@ -419,7 +418,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void latent_prefill_kernel(hymeta_
 // heads) need 400 registers, of which 256 can be addressed by everything but the matrix instructions: the compiler spills
 // 460.  The head slices of a (sequence, slice of keys) follow each other on one die instead, whose L2 has the keys for the
 // second.  Bound by memory, and by what stands around a slice's few tiles (queries, first tile, merge): 64 sequences x 4096 keys
-// of 512 + 64, 16 heads: 66 us = 4.6 TB/s, where four launches over value slices took 280.
+// of 512 + 64, 16 heads: 64 us, 53 of them this kernel (4.8 TB/s), where four launches over value slices took 280.
 constexpr int kLatentWaves = 4, kLatentKeys = 16, kLatentHeads = 16;
 
 template <int C>
