@@ -34,6 +34,8 @@ def _recurrence(q, k, v, beta, l2, state, starts, context, slots, scale, eps):
     (128, 128, 4, 1, [300, 7, 1] + [70] * 12, 0),
     (64, 128, 24, 8, EDGES, 0), (128, 256, 16, 8, EDGES, 0),          # slices of 128
     (64, 128, 2, 1, [200], 0), (128, 32, 2, 2, [65, 5], 0),           # slices of 16
+    (96, 96, 16, 4, EDGES, 0), (96, 128, 24, 8, EDGES, 0), (32, 128, 24, 8, EDGES, 0),        # slices of 32, and of 128 with other heads
+    (96, 96, 4, 2, [300, 65], 0), (32, 32, 4, 4, [200, 9, 1], 0),      # slices of 16 whose blocks do not deal evenly over the waves
     (128, 128, 4, 2, [2, 7, 1, 3, 6], 0), (256, 64, 2, 2, [2, 5], 0),  # nothing long enough for a chunk
     (32, 64, 4, 4, [5, 1, 7], 1), (64, 32, 2, 1, [3, 7], 0), (96, 64, 2, 2, [1, 6, 2], 0), (96, 32, 2, 2, [2, 4], 0),
     # short portions in a launch of their own beside chunks: by their number, as the others fill the chip, by their rows

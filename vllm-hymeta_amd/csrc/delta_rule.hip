@@ -314,7 +314,8 @@ typedef float f32x4v __attribute__((ext_vector_type(4)));
 constexpr int kChunk = HYMETA_DELTA_CHUNK;
 // Workgroups with slices of 32 value columns up to which the second launch runs slices of 16 whose waves share a chunk's rows
 // (delta_chunk_narrow_kernel), about 2 us a chunk against 2.6 where a wave takes all rows of its columns: one prompt of 8192
-// rows with 28 heads of 128 x 128 (112 workgroups) 327 us against 388, with 16 heads 216 against 345.  They also double the
+// rows with 28 heads of 128 x 128 (112 workgroups) 327 us against 388, with 16 heads 216 against 345, of 96 x 96 190 against 319, of 32 x 32
+// 157 against 248.  They also double the
 // workgroups of the sequences without a chunk, which end at once but take about 0.65 ns each to come and go, and save about 0.6
 // us a chunk of 64 rows: not where those are more than 10 per row of the longest portion.
 // Workgroups with slices of 64 columns up to which the other kernel takes those: its images leave room for one workgroup on a
@@ -331,9 +332,12 @@ constexpr int kFewGroups = 128, kIdleGroupsPerRow = 10, kManyGroups = 256;
 //   28 heads of 64 x 128: 40 beside 63 29.7 / 36.8, beside 255 85 / 97, 2048 beside 255 179 / 176: single rows stay.
 //   60 portions of 7 rows beside 40: 64 x 128 79 / 52, 128 x 128 98 / 80: where the longest fits a chunk and the others have two rows
 //   each, apart.
-//   Three or four times through the columns, four portions of 600 beside three of 5: 8 heads of 128 x 256 72 / 55, 16 of 32 x 96 55 / 49.
+//   Three or four times through the columns, four portions of 600 beside three of 5: 8 heads of 128 x 256 72 / 55, 16 of 32 x 96 55 / 49;
+//   where none are to be expected, the launch is saved: 16 heads of 96 x 96, 64 rows 18.9 -> 16.0.
 inline bool short_apart(const hymeta_delta_rule_args& a, int64_t shorts) {
-  if (a.v_dim > 128 || a.v_dim % 64 != 0 || (a.head_dim > 64 && shorts > 4096)) return true;
+  const int passes = a.v_dim / (a.v_dim % 64 == 0 ? 64 : 32);
+  if (shorts == 0) return false;
+  if (passes > 2 || (a.head_dim > 64 && shorts > 4096)) return true;
   const int64_t chunks = static_cast<int64_t>(a.num_heads) * (a.num_tokens / kChunk);
   if (a.head_dim > 64 && shorts > 1000 && 10 * chunks < shorts) return true;
   return shorts > 256 && a.max_query_len <= kChunk && a.num_tokens - a.max_query_len >= 2 * (a.num_seqs - 1);
@@ -576,8 +580,10 @@ __global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hy
 // write, is 0 there), and the last chunk fetches itself once more, so that no load stands under a condition.
 template <int D>
 __global__ __launch_bounds__(256) void delta_chunk_narrow_kernel(hymeta_delta_rule_args a, int64_t chunks) {
-  constexpr int SV = 16, PK = D + 8, PT = kChunk + 8, NBW = D / 16 / 4;
-  static_assert(D / 16 % 4 == 0, "the state's blocks deal evenly over the waves");
+  constexpr int SV = 16, PK = D + 8, PT = kChunk + 8, DB = D / 16, NBW = (DB + 3) / 4;
+  // (what is left over of the deal, with heads of 32 and 96: the last block again, whose owner alone writes it)
+  auto block_of = [](int wave, int ib) __attribute__((always_inline)) { return DB % 4 == 0 ? wave + 4 * ib : min(wave + 4 * ib, DB - 1); };
+  auto owned = [](int wave, int ib) __attribute__((always_inline)) { return DB % 4 == 0 || wave + 4 * ib < DB; };
   __shared__ __attribute__((aligned(16))) uint16_t sst[2][SV * PK];                                      // state, [c][d]
   __shared__ __attribute__((aligned(16))) uint16_t srt[2][SV * PT], su[2][SV * PT], sw[2][SV * PT];      // [c][row]
   const int h = blockIdx.x, s = blockIdx.y, vs = blockIdx.z;
@@ -591,14 +597,15 @@ __global__ __launch_bounds__(256) void delta_chunk_narrow_kernel(hymeta_delta_ru
   f32x4v S[NBW];
 #pragma unroll
   for (int ib = 0; ib < NBW; ++ib) {
-    const int db = wave + 4 * ib;
+    const int db = block_of(wave, ib);
 #pragma unroll
     for (int r = 0; r < 4; ++r) S[ib][r] = carry ? st[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + n] : 0.f;
   }
   auto state_to_lds = [&]() {
 #pragma unroll
     for (int ib = 0; ib < NBW; ++ib) {
-      const int db = wave + 4 * ib;
+      if (!owned(wave, ib)) continue;
+      const int db = block_of(wave, ib);
       const float v[4] = {S[ib][0], S[ib][1], S[ib][2], S[ib][3]};
       u32x2 hi, lo;
       split4(v, hi, lo);
@@ -652,7 +659,7 @@ __global__ __launch_bounds__(256) void delta_chunk_narrow_kernel(hymeta_delta_ru
     m.total = places[static_cast<int64_t>(c) * H].total;
 #pragma unroll
     for (int ib = 0; ib < NBW; ++ib) {
-      const int db = wave + 4 * ib;
+      const int db = block_of(wave, ib);
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) m.wf[ib][kk] = ld16g(kt + (2 * db + kk) * 512);
     }
@@ -764,7 +771,8 @@ __global__ __launch_bounds__(256) void delta_chunk_narrow_kernel(hymeta_delta_ru
   if (st != nullptr) {
 #pragma unroll
     for (int ib = 0; ib < NBW; ++ib) {
-      const int db = wave + 4 * ib;
+      if (!owned(wave, ib)) continue;
+      const int db = block_of(wave, ib);
 #pragma unroll
       for (int r = 0; r < 4; ++r) st[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + n] = S[ib][r];
     }
@@ -1090,14 +1098,12 @@ template <int D>
 void launch_chunks(const hymeta_delta_rule_args& a, hipStream_t st, int64_t chunks, bool short_too) {
   const int64_t portions = long_portions(a.num_tokens, a.num_seqs, a.max_query_len), lanes = a.num_heads * portions;
   const int64_t idle = a.num_heads * (a.num_seqs - portions) * (a.v_dim / 32);
-  const bool narrow = D % 64 == 0 && lanes * (a.v_dim / 32) <= kFewGroups && idle <= static_cast<int64_t>(kIdleGroupsPerRow) * a.max_query_len;
+  const bool narrow = lanes * (a.v_dim / 32) <= kFewGroups && idle <= static_cast<int64_t>(kIdleGroupsPerRow) * a.max_query_len;
   const dim3 solve(static_cast<unsigned>(chunks), a.num_heads);
-  if constexpr (D % 64 == 0) {
-    if (narrow) {
-      hipLaunchKernelGGL((delta_chunk_solve_kernel<D, true>), solve, dim3(256), 0, st, a, chunks, short_too);
-      hipLaunchKernelGGL(delta_chunk_narrow_kernel<D>, dim3(a.num_heads, a.num_seqs, a.v_dim / 16), dim3(256), 0, st, a, chunks);
-      return;
-    }
+  if (narrow) {
+    hipLaunchKernelGGL((delta_chunk_solve_kernel<D, true>), solve, dim3(256), 0, st, a, chunks, short_too);
+    hipLaunchKernelGGL(delta_chunk_narrow_kernel<D>, dim3(a.num_heads, a.num_seqs, a.v_dim / 16), dim3(256), 0, st, a, chunks);
+    return;
   }
   hipLaunchKernelGGL((delta_chunk_solve_kernel<D, false>), solve, dim3(256), 0, st, a, chunks, short_too);
   auto launch = [&](auto nw) {
