@@ -953,6 +953,14 @@ typedef struct hymeta_moe_gemm_args {
 } hymeta_moe_gemm_args;
 
 int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t stream);
+/* hymeta_moe_gemm with an activation over pairs of output columns: the weights' rows are N / 2 gate rows, then N / 2 up rows,
+ * out has N / 2 columns.  HYMETA_GEMM_ACT_SILU: silu(gate) up as hymeta_silu_and_mul gives it; _SILU_EXACT: as
+ * hymeta_activation's HYMETA_ACT_SILU_MUL; _CLAMPED_GLU: its HYMETA_ACT_CLAMPED_GLU with limit and alpha -- of the bf16 rows
+ * that hymeta_moe_gemm would write.  Problems that hymeta_moe_gemm_activates answers with 1 (many rows per expert), else
+ * HYMETA_ERR_UNSUPPORTED. */
+enum hymeta_gemm_act { HYMETA_GEMM_ACT_NONE = 0, HYMETA_GEMM_ACT_SILU = 1, HYMETA_GEMM_ACT_SILU_EXACT = 2, HYMETA_GEMM_ACT_CLAMPED_GLU = 3 };
+int hymeta_moe_gemm_act(const hymeta_moe_gemm_args* args, int32_t act, float limit, float alpha, hymeta_stream_t stream);
+int hymeta_moe_gemm_activates(const hymeta_moe_gemm_args* args);
 /* 1 when hymeta_moe_gemm runs a problem of these sizes in the kernel that has the fused combine (K in bf16 elements:
  * pass K / 2 for int8 operands, the choice goes by the bytes of a row). */
 int hymeta_moe_gemm_fuses(int32_t max_rows, int32_t experts, int32_t K, int32_t N);

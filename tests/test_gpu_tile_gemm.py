@@ -1,0 +1,110 @@
+"""The tiled matrix products of prompts (256 x 256 tiles, halves of 128 rows), bit for bit: operands are small integers and
+scales powers of two, so that every fp32 sum is exact in any order and one rounding to bf16 remains."""
+import ctypes as C
+
+import pytest
+import torch
+
+from _util import gen
+
+pytestmark = pytest.mark.gpu
+
+NONE, SILU, SILU_EXACT, CLAMPED = 0, 1, 2, 3
+
+
+def _ints(g, lo, hi, *shape):
+    return torch.randint(lo, hi + 1, shape, generator=g)
+
+
+def _activate(h, act):
+    from vllm_hymeta import hip_ops
+    if act == NONE:
+        return h
+    if act == SILU:
+        return hip_ops.silu_and_mul(h)
+    return hip_ops.silu_mul(h) if act == SILU_EXACT else hip_ops.clamped_glu(h, 7.0, 1.702)
+
+
+@pytest.mark.parametrize("sizes,K,N,div,local,act,int8", [
+    # rows at the edges of tiles and halves, an expert without rows; the fewest steps; more than a round of tiles
+    ((1, 255, 256, 257, 0, 511, 129, 128), 256, 10240, 1, (0, 8), NONE, False),
+    ((1, 255, 256, 257, 0, 511, 129, 128), 320, 10240, 2, (0, 8), SILU, False),      # an odd number of steps; two slots a source row
+    ((700, 3, 1100), 256, 8704, 1, (0, 3), CLAMPED, False),                          # a last round of at most half the units: halves
+    ((700, 3, 1100), 512, 5120, 1, (0, 3), SILU_EXACT, False),
+    ((640, 333, 200, 515), 512, 5120, 1, (1, 3), SILU, True),                        # a rank's share of the experts
+    ((1, 255, 256, 257, 0, 511, 129, 128), 640, 10240, 2, (0, 8), NONE, True),
+    ((2600,), 1024, 5120, 1, (0, 1), NONE, True),                                    # more row tiles than a block of neighbours holds
+    ((5, 900), 256, 10240, 1, (0, 1), SILU, False),                                  # halves that hold no rows
+    ((2600, 1300), 448, 2560, 3, (0, 2), NONE, False),
+])
+def test_grouped_products(sizes, K, N, div, local, act, int8):
+    from vllm_hymeta import _C
+    lib, E, P = _C.load(), len(sizes), sum(sizes)
+    g = gen(7)
+    kind = torch.int8 if int8 else torch.bfloat16
+    T = (P + div - 1) // div
+    x, w = _ints(g, -3, 3, T, K), _ints(g, -2, 2, E, N, K)
+    slots = torch.randperm(T * div, generator=g)[:P]
+    factor = 2.0 ** _ints(g, -2, 1, P).float()
+    order = torch.randperm(P, generator=g)
+    offsets = torch.tensor([0] + list(sizes)).cumsum(0)
+    x_scale, w_scale = 2.0 ** _ints(g, -3, 0, T).float(), 2.0 ** _ints(g, -2, 1, E, N).float()
+    d = {n: t.cuda() for n, t in dict(x=x.to(kind), w=w.to(kind), slots=slots.int(), factor=factor, order=order.int(),
+                                      offsets=offsets.int(), x_scale=x_scale, w_scale=w_scale).items()}
+    cols = N // 2 if act else N
+    out = torch.full((P + 1, cols), 7.0, dtype=torch.bfloat16, device="cuda")
+    a = _C.MoeGemmArgs()
+    ptr = lambda t: C.c_void_p(t.data_ptr())      # noqa: E731
+    a.x, a.weights, a.out, a.expert_offsets = ptr(d["x"]), ptr(d["w"]), ptr(out), ptr(d["offsets"])
+    a.a_rows, a.a_rows_div, a.scale_rows, a.row_scale = ptr(d["slots"]), div, ptr(d["order"]), ptr(d["factor"])
+    a.max_rows, a.K, a.N = P, K, N
+    a.local_expert_begin, a.local_expert_end = local
+    a.x_stride_m, a.out_stride_m, a.w_stride_e = K, cols, N * K
+    if int8:
+        a.operand_dtype, a.x_scale, a.w_scale = _C.HYMETA_I8, ptr(d["x_scale"]), ptr(d["w_scale"])
+    assert lib.hymeta_moe_gemm_activates(C.byref(a)) == 1            # these sizes are the tiles'
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    if act:
+        assert lib.hymeta_moe_gemm_act(C.byref(a), act, 7.0, 1.702, stream) == 0
+    else:
+        assert lib.hymeta_moe_gemm(C.byref(a), stream) == 0
+    torch.cuda.synchronize()
+    source = slots // div
+    for e in range(E):
+        lo, hi = int(offsets[e]), int(offsets[e + 1])
+        if not local[0] <= e < local[1]:
+            assert bool((out[lo:hi] == 7.0).all())                   # other ranks' rows stay as they are
+            continue
+        if lo == hi:
+            continue
+        s = source[lo:hi].cuda()
+        h = d["x"][s].float() @ d["w"][e].float().t()                # exact: |sums| < 2^24
+        if int8:
+            h = h * d["x_scale"][s][:, None] * d["w_scale"][e]
+        h = (h * d["factor"][d["order"][lo:hi].long()][:, None]).to(torch.bfloat16)
+        assert torch.equal(out[lo:hi], _activate(h, act)), f"expert {e}"
+    assert bool((out[P] == 7.0).all())
+
+
+def test_what_the_tiles_do_not_take():
+    """No activation for a problem of few rows; int8 knows the quantised path's silu only."""
+    from vllm_hymeta import _C
+    lib = _C.load()
+    x = torch.zeros(4096, 512, dtype=torch.int8, device="cuda")
+    w = torch.zeros(4, 5120, 512, dtype=torch.int8, device="cuda")
+    scale = torch.ones(4 * 5120, device="cuda")
+    out = torch.zeros(4096, 2560, dtype=torch.bfloat16, device="cuda")
+    offsets = torch.tensor([0, 4, 8, 12, 16], dtype=torch.int32, device="cuda")
+    ptr = lambda t: C.c_void_p(t.data_ptr())      # noqa: E731
+    a = _C.MoeGemmArgs()
+    a.x, a.weights, a.out, a.expert_offsets = ptr(x), ptr(w), ptr(out), ptr(offsets)
+    a.max_rows, a.K, a.N, a.local_expert_end = 16, 512, 5120, 4
+    a.x_stride_m, a.out_stride_m, a.w_stride_e = 512, 2560, 5120 * 512
+    a.operand_dtype, a.x_scale, a.w_scale = _C.HYMETA_I8, ptr(scale), ptr(scale)
+    unsupported = -2
+    assert lib.hymeta_moe_gemm_activates(C.byref(a)) == 0
+    assert lib.hymeta_moe_gemm_act(C.byref(a), SILU, 0.0, 0.0, None) == unsupported
+    a.max_rows = 4096
+    assert lib.hymeta_moe_gemm_activates(C.byref(a)) == 1
+    assert lib.hymeta_moe_gemm_act(C.byref(a), CLAMPED, 7.0, 1.702, None) == unsupported
+    assert lib.hymeta_moe_gemm_act(C.byref(a), 4, 0.0, 0.0, None) == -1

@@ -121,4 +121,10 @@ __device__ __forceinline__ PieceAt piece_at(const int32_t* query_start_loc, int 
 
 __device__ __forceinline__ float sigmoid_exact(float x) { return 1.f / (1.f + expf(-x)); }
 
+__device__ __forceinline__ float clamped_glu(float gate, float up, float limit, float alpha) {
+  const float g = fminf(gate, limit);
+  const float u = fminf(fmaxf(up, -limit), limit);
+  return g * sigmoid_exact(alpha * g) * (u + 1.f);
+}
+
 }  // namespace hymeta

@@ -7,12 +7,6 @@ namespace hymeta {
 
 namespace {
 
-__device__ __forceinline__ float clamped_glu(float gate, float up, float limit, float alpha) {
-  const float g = fminf(gate, limit);
-  const float u = fminf(fmaxf(up, -limit), limit);
-  return g * sigmoid_exact(alpha * g) * (u + 1.f);
-}
-
 __device__ __forceinline__ float xielu(float z, float a_pos, float a_neg) {
   return z > 0.f ? fmaf(a_pos * z, z, 0.5f * z) : fmaf(a_neg, expm1f(z) - z, 0.5f * z);
 }

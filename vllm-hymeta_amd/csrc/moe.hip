@@ -13,7 +13,7 @@
 //   combine  out[t] = sum_k y[pos[t,k]] (+ shared[t]), y weighted in the down GEMM; pairs of non-local experts
 //            (expert parallelism) carry pos = -1 and add nothing
 #include "common.h"
-#include "lds_copy.h"
+#include "tile_gemm.h"
 #include "w8a8_quant.h"
 
 #include <algorithm>
@@ -529,20 +529,18 @@ __global__ __launch_bounds__(256) void moe_gemm_lines_kernel(hymeta_moe_gemm_arg
   }
 }
 
-// Prefill regime (many rows per expert): BM rows x BN columns per workgroup, WM x WN waves that own
+// Prompts of few rows per expert (tile_gemm.hip takes the long ones): BM rows x BN columns per workgroup, WM x WN waves that own
 // (BM / WM) x (BN / WN) each.  Both operands are K-contiguous; a 64-deep step of each (128 bytes per
 // row) is staged once per workgroup through double-buffered LDS images (16-byte chunks XOR-ed with
 // the row, so the sixteen rows of a fragment read hit distinct banks): registers -> LDS right
-// behind the barrier that frees the buffer, the next step's loads issued at once.  LDS stores run
-// at a third of the read rate, so the tile sets the ceiling: 128 x 128 spends more LDS time than
-// matrix time per step, 256 x 256 (64 x 128 per wave) about three quarters of it.
+// behind the barrier that frees the buffer, the next step's loads issued at once.
 // grid = (N / BN, row tiles); the row tiles of all local experts are numbered consecutively and a
 // workgroup finds its (expert, tile) from the offsets on the device -- the host only knows the
 // bound ceil(max_rows / BM) + experts.
 constexpr int kTK = 64;
 constexpr int kTilePitch = 2 * kTK;                 // bytes per staged row
 constexpr int kTiledMinRowsPerExpert = 8;           // measured: level at 4 rows per expert, 15 % ahead at 16, 2.6x at 512
-constexpr int kBigTileMinRowsPerExpert = 192;
+constexpr int kBigTileMinRowsPerExpert = 128, kBigTileMinTiles = 160;
 
 template <int BM, int BN, int WM, int WN, bool I8>
 __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void moe_gemm_tiled_kernel(hymeta_moe_gemm_args a) {
@@ -693,156 +691,6 @@ __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void moe_gemm_t
   }
 }
 
-// int8 in tiles of 256 x 256 (8 waves of 64 rows x 128 columns), both operands copied from memory straight into LDS: nothing
-// of a step passes registers, so the fragments of the next quarter of a step are read while this one's are multiplied, and
-// v_mfma_i32_32x32x32_i8 needs 6 fragments of 1 KB for 8 instructions.  Two images of a step (128 bytes of every row); a
-// step's copies are asked for a whole step ahead.  The barrier that frees an image stands in front of the step's last
-// quarter: the first reads of the next image go out under that quarter's products.  The weights are the first operand: a
-// lane then holds four neighbouring columns of ONE row, which share its scales and go to the staged output together.
-// Bound by the matrix pipe and its power: 16 int8 experts on 8192 rows of 3584 columns took 779 us through
-// moe_gemm_tiled_kernel's 256 x 256 tile, 732 through this one (quantisation and activation included).  In bf16 the same structure takes 4% fewer cycles at a lower
-// clock: 0.99 to 1.02 of the tiled kernel's speed over 1500 to 8192 rows, so bf16 stays there.
-typedef int i32x16 __attribute__((ext_vector_type(16)));
-constexpr int kBig = 256;                            // rows and columns of the tile
-constexpr int kBigImage = kBig * kTilePitch;         // bytes of one operand's step
-
-__global__ __launch_bounds__(512, 2) void moe_gemm_big_i8_kernel(hymeta_moe_gemm_args a) {
-  __shared__ __attribute__((aligned(16))) char sm[2][2 * kBigImage];   // [step parity][x | w]
-
-  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hh = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
-
-  // which expert, which of its row tiles
-  int e = -1, row_lo = 0, row_hi = 0;
-  {
-    int t = blockIdx.y;
-    for (int i = a.local_expert_begin; i < a.local_expert_end; ++i) {
-      const int lo = a.expert_offsets[i], hi = a.expert_offsets[i + 1];
-      const int tiles = (hi - lo + kBig - 1) / kBig;
-      if (t < tiles) {
-        e = i;
-        row_lo = lo + t * kBig;
-        row_hi = hi;
-        break;
-      }
-      t -= tiles;
-    }
-  }
-  if (e < 0) return;                                 // workgroup-uniform
-  const int col0 = blockIdx.x * kBig;
-
-  // copies: an instruction of a wave brings 8 rows x 128 bytes; a row's 16-byte chunks lie XOR-ed with (row / 2) % 8, which
-  // with the pitch of 128 bytes spreads the rows of a fragment read over all banks
-  const int64_t kb = a.K;                          // bytes of an operand row
-  const char *xp[4], *wp[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int row = 8 * (4 * wave + j) + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
-    const int slot = min(row_lo + row, row_hi - 1);    // rows past the expert's end re-read its last row
-    xp[j] = static_cast<const char*>(a.x) + static_cast<int64_t>(moe_src_row(a, slot)) * a.x_stride_m + 16 * chunk;
-    wp[j] = static_cast<const char*>(a.weights) + static_cast<int64_t>(e) * a.w_stride_e + (col0 + row) * kb + 16 * chunk;
-  }
-  
-  auto issue = [&](int it, char* image) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      copy16_to_lds(xp[j] + it * kTilePitch, image + 1024 * (4 * wave + j));
-      copy16_to_lds(wp[j] + it * kTilePitch, image + kBigImage + 1024 * (4 * wave + j));
-    }
-  };
-  int off[4];                                        // a fragment's place for this lane: row r, chunk 2 ks + hh
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) off[ks] = r * kTilePitch + 16 * ((2 * ks + hh) ^ ((r >> 1) & 7));
-  const int xat = 64 * wm * kTilePitch, wat = kBigImage + 128 * wn * kTilePitch;
-
-  i32x16 acc[2][4];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int k = 0; k < 16; ++k) acc[i][j][k] = 0;
-
-  i32x4 xf[2][2], wf[2][4];                          // [parity of the quarter]
-  auto read = [&](const char* image, int ks) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) xf[ks & 1][i] = __builtin_bit_cast(i32x4, ld16(image + xat + off[ks] + 32 * i * kTilePitch));
-#pragma unroll
-    for (int j = 0; j < 4; ++j) wf[ks & 1][j] = __builtin_bit_cast(i32x4, ld16(image + wat + off[ks] + 32 * j * kTilePitch));
-  };
-  const int nk = static_cast<int>(kb / kTilePitch);
-  issue(0, sm[0]);
-  copies_landed_barrier();
-  if (nk > 1) issue(1, sm[1]);
-  read(sm[0], 0);
-  auto multiply = [&](int ks) {
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[ks & 1][j], xf[ks & 1][i], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  // (the last step stands behind the loop: a branch around the barrier and the next step's reads would make the compiler
-  // wait for those reads in front of the last quarter's products)
-  for (int it = 0; it + 1 < nk; ++it) {
-    char* image = sm[it & 1];
-#pragma unroll
-    for (int ks = 0; ks < 3; ++ks) {
-      read(image, ks + 1);
-      multiply(ks);
-    }
-    copies_landed_barrier();                         // this step's last fragments are in registers, the next step's rows in LDS
-    read(sm[(it + 1) & 1], 0);
-    if (it + 2 < nk) issue(it + 2, image);
-    multiply(3);
-  }
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    if (ks < 3) read(sm[(nk - 1) & 1], ks + 1);
-    multiply(ks);
-  }
-  __syncthreads();
-
-  // acc[i][j][4 q + p] = C[row 64 wm + 32 i + r][col 128 wn + 32 j + 8 q + 4 hh + p]: routing weight on the fp32 sums, one
-  // rounding, staged through LDS 128 rows at a time and stored as whole rows
-  constexpr int kCPitch = 2 * kBig + 16, kStageRows = 128;
-  static_assert(kStageRows * kCPitch <= static_cast<int>(sizeof(sm)), "output staging fits the operand images");
-  char* cst = &sm[0][0];
-#pragma unroll
-  for (int half = 0; half < kBig / kStageRows; ++half) {
-    if (wm >> 1 == half) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int row = 64 * wm + 32 * i + r, slot = min(row_lo + row, row_hi - 1);
-        const float sc_row = a.row_scale != nullptr ? a.row_scale[a.scale_rows != nullptr ? a.scale_rows[slot] : slot] : 1.f;
-        const float xs = a.x_scale[moe_src_row(a, slot)];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int col = 128 * wn + 32 * j + 8 * q + 4 * hh;
-            const f32x4 ws = *reinterpret_cast<const f32x4*>(a.w_scale + static_cast<int64_t>(e) * a.N + col0 + col);
-            f32x4 v;
-#pragma unroll
-            for (int p = 0; p < 4; ++p) v[p] = w8a8_scaled(acc[i][j][4 * q + p], xs, ws[p], 0.f);
-            *reinterpret_cast<u32x2*>(cst + (row - kStageRows * half) * kCPitch + 2 * col) =
-                u32x2{pack_bf16x2(v[0] * sc_row, v[1] * sc_row), pack_bf16x2(v[2] * sc_row, v[3] * sc_row)};
-          }
-      }
-    }
-    __syncthreads();
-    constexpr int kChunksPerRow = kBig / 8;
-    for (int id = tid; id < kStageRows * kChunksPerRow; id += 512) {
-      const int row = id / kChunksPerRow, ch = id % kChunksPerRow, slot = row_lo + kStageRows * half + row;
-      if (slot < row_hi)
-        st16(reinterpret_cast<uint16_t*>(a.out) + static_cast<int64_t>(slot) * a.out_stride_m + col0 + 8 * ch, ld16(cst + row * kCPitch + 16 * ch));
-    }
-    if (half + 1 < kBig / kStageRows) __syncthreads();
-  }
-}
-
 // out[r, j] = silu(in[r, j]) * in[r, inter + j]; the product is formed in fp32 and rounded once.
 __global__ __launch_bounds__(256) void silu_and_mul_kernel(const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
                                                            const int32_t* __restrict__ num_rows_dev, int num_rows,
@@ -985,7 +833,11 @@ enum class MoeGemmKind { kBigTiles, kTiles, kLines, kFragments };
 MoeGemmKind moe_gemm_kind(int64_t max_rows, int experts, int K, int N) {
   // tiled grouped GEMM once the experts average more than a few rows (prefill chunks); the large tile when they fill it
   if (max_rows > static_cast<int64_t>(kTiledMinRowsPerExpert) * experts && K % kTK == 0) {
-    if (max_rows >= static_cast<int64_t>(kBigTileMinRowsPerExpert) * experts && N % 256 == 0) return MoeGemmKind::kBigTiles;
+    // tiles of 256 where the experts fill half of one on average and the tiles (an expert's rows scatter around the average)
+    // nearly fill the chip once: 16 experts on 2048 tokens of 3584 columns 560 -> 516 us, 8 on 1400 936 -> 705; with 112 rows
+    // an expert 424 -> 459, with 64 to 128 tiles 215 -> 226
+    const int64_t rows = max_rows / experts, tiles = (rows + 64 + 255) / 256 * experts * (N / 256);
+    if (rows >= kBigTileMinRowsPerExpert && tiles >= kBigTileMinTiles && N % 256 == 0) return MoeGemmKind::kBigTiles;
     if (N % 128 == 0) return MoeGemmKind::kTiles;
   }
   static const bool lines = [] {
@@ -1001,12 +853,33 @@ extern "C" int hymeta_moe_gemm_fuses(int32_t max_rows, int32_t experts, int32_t 
   return experts > 0 && hymeta::moe_gemm_kind(max_rows, experts, K, N) == hymeta::MoeGemmKind::kLines ? 1 : 0;
 }
 
-extern "C" int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t stream) {
-  using namespace hymeta;
-  if (!hymeta::args_ok(args)) return HYMETA_ERR_INVALID_ARG;
+namespace hymeta {
+namespace {
+
+TileGemmArgs tile_args(const hymeta_moe_gemm_args& a) {
+  const int esize = a.operand_dtype == HYMETA_I8 ? 1 : 2;
+  TileGemmArgs t = {};
+  t.x = static_cast<const char*>(a.x), t.w = static_cast<const char*>(a.weights), t.out = static_cast<uint16_t*>(a.out);
+  t.expert_offsets = a.expert_offsets, t.a_rows = a.a_rows, t.scale_rows = a.scale_rows, t.row_scale = a.row_scale;
+  t.x_scale = a.x_scale, t.w_scale = a.w_scale;
+  t.x_stride = a.x_stride_m * esize, t.w_stride_e = a.w_stride_e * esize, t.out_stride = a.out_stride_m;
+  t.a_rows_div = a.a_rows_div, t.max_rows = a.max_rows, t.N = a.N, t.k_bytes = a.K * esize;
+  t.expert_begin = a.local_expert_begin, t.expert_end = a.local_expert_end;
+  return t;
+}
+
+MoeGemmKind moe_gemm_kind(const hymeta_moe_gemm_args& a) {
+  // the kind goes by the bytes of a row
+  const MoeGemmKind kind = moe_gemm_kind(a.max_rows, a.local_expert_end - a.local_expert_begin, a.operand_dtype == HYMETA_I8 ? a.K / 2 : a.K, a.N);
+  return kind == MoeGemmKind::kBigTiles && !tile_gemm_fits(tile_args(a)) ? MoeGemmKind::kTiles : kind;
+}
+
+int moe_gemm(const hymeta_moe_gemm_args* args, int act, float limit, float alpha, hymeta_stream_t stream) {
+  if (!args_ok(args)) return HYMETA_ERR_INVALID_ARG;
   const hymeta_moe_gemm_args& a = *args;
   if (a.max_rows < 0 || a.K <= 0 || a.N <= 0) return HYMETA_ERR_INVALID_ARG;
   if (a.local_expert_begin < 0 || a.local_expert_end < a.local_expert_begin) return HYMETA_ERR_INVALID_ARG;
+  if (act < HYMETA_GEMM_ACT_NONE || act > HYMETA_GEMM_ACT_CLAMPED_GLU) return HYMETA_ERR_INVALID_ARG;
   if (a.max_rows == 0 || a.local_expert_end == a.local_expert_begin) return HYMETA_OK;
   if (!a.x || !a.weights || !a.out || !a.expert_offsets) return HYMETA_ERR_INVALID_ARG;
   if (a.a_rows != nullptr && a.a_rows_div <= 0) return HYMETA_ERR_INVALID_ARG;
@@ -1018,7 +891,9 @@ extern "C" int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t
   if ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.weights) | reinterpret_cast<uintptr_t>(a.out)) % 16 != 0)
     return HYMETA_ERR_UNSUPPORTED;
   const int experts = a.local_expert_end - a.local_expert_begin;
-  const MoeGemmKind kind = moe_gemm_kind(a.max_rows, experts, i8 ? a.K / 2 : a.K, a.N);   // the kind goes by the bytes of a row
+  const MoeGemmKind kind = moe_gemm_kind(a);
+  if (act != HYMETA_GEMM_ACT_NONE && hymeta_moe_gemm_activates(args) != 1) return HYMETA_ERR_UNSUPPORTED;
+  if (i8 && act > HYMETA_GEMM_ACT_SILU) return HYMETA_ERR_UNSUPPORTED;
   if (a.combine_tokens != nullptr || a.combine_shared != nullptr) {
     // the fused combine exists in the decode-sized kernel with whole-line loads only (hymeta_moe_gemm_fuses)
     if (kind != MoeGemmKind::kLines) return HYMETA_ERR_UNSUPPORTED;
@@ -1032,9 +907,9 @@ extern "C" int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t
   const bool small = static_cast<int64_t>(a.max_rows) <= 8LL * experts;
 #define HYMETA_MOE_BY_TYPE(LAUNCH_BF16, LAUNCH_I8) do { if (i8) { LAUNCH_I8; } else { LAUNCH_BF16; } } while (0)
   if (kind == MoeGemmKind::kBigTiles) {
-    const dim3 tgrid(a.N / 256, (a.max_rows + 255) / 256 + experts);
-    HYMETA_MOE_BY_TYPE(hipLaunchKernelGGL((moe_gemm_tiled_kernel<256, 256, 4, 2, false>), tgrid, dim3(512), 0, s, a),
-                       hipLaunchKernelGGL(moe_gemm_big_i8_kernel, tgrid, dim3(512), 0, s, a));
+    TileGemmArgs t = tile_args(a);
+    t.act = act, t.act_limit = limit, t.act_alpha = alpha;
+    tile_gemm_launch(t, i8, s);
     return launch_status();
   }
   if (kind == MoeGemmKind::kTiles) {
@@ -1058,6 +933,25 @@ extern "C" int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t
                           hipLaunchKernelGGL((moe_gemm_kernel<4, true>), grid, block, red4, s, a));
 #undef HYMETA_MOE_BY_TYPE
   return launch_status();
+}
+
+}  // namespace
+}  // namespace hymeta
+
+extern "C" int hymeta_moe_gemm_activates(const hymeta_moe_gemm_args* args) {
+  if (!hymeta::args_ok(args)) return HYMETA_ERR_INVALID_ARG;
+  if (args->a_rows != nullptr && args->a_rows_div <= 0) return 0;
+  TileGemmArgs t = hymeta::tile_args(*args);
+  t.act = HYMETA_GEMM_ACT_SILU;
+  return args->local_expert_end > args->local_expert_begin && hymeta::moe_gemm_kind(*args) == hymeta::MoeGemmKind::kBigTiles && tile_gemm_fits(t) ? 1 : 0;
+}
+
+extern "C" int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t stream) {
+  return hymeta::moe_gemm(args, HYMETA_GEMM_ACT_NONE, 0.f, 0.f, stream);
+}
+
+extern "C" int hymeta_moe_gemm_act(const hymeta_moe_gemm_args* args, int32_t act, float limit, float alpha, hymeta_stream_t stream) {
+  return hymeta::moe_gemm(args, act, limit, alpha, stream);
 }
 
 extern "C" int hymeta_silu_and_mul(const void* in, void* out, const int32_t* num_rows_dev, int32_t num_rows,

@@ -281,6 +281,9 @@ class MoeGemmArgs(_Args):
     ]
 
 
+GEMM_ACT_SILU, GEMM_ACT_SILU_EXACT, GEMM_ACT_CLAMPED_GLU = 1, 2, 3
+
+
 class MoeGptqGemmArgs(_Args):
     _fields_ = [
         _SIZE,
@@ -672,6 +675,8 @@ _SIGNATURES = {
     "hymeta_moe_router": (C.c_int, [C.POINTER(MoeRouterArgs), _ptr]),
     "hymeta_moe_gemm_fuses": (C.c_int, [_i32, _i32, _i32, _i32]),
     "hymeta_moe_gemm": (C.c_int, [C.POINTER(MoeGemmArgs), _ptr]),
+    "hymeta_moe_gemm_act": (C.c_int, [C.POINTER(MoeGemmArgs), _i32, C.c_float, C.c_float, _ptr]),
+    "hymeta_moe_gemm_activates": (C.c_int, [C.POINTER(MoeGemmArgs)]),
     "hymeta_silu_and_mul": (C.c_int, [_ptr, _ptr, _ptr, _i32, _i32, _i64, _i64, _ptr]),
     "hymeta_moe_gptq_gemm": (C.c_int, [C.POINTER(MoeGptqGemmArgs), _ptr]),
     "hymeta_moe_gptq_expand": (C.c_int, [_ptr, _ptr, _ptr, _ptr, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _ptr]),

@@ -1376,8 +1376,8 @@ def moe_forward(x: torch.Tensor, router_logits: Optional[torch.Tensor], w13: tor
         r.logits_stride_t = router_logits.stride(0)
         _C.check(lib.hymeta_moe_route(C.byref(r), st), "hymeta_moe_route")
 
-    h13 = torch.empty(P, two_i, dtype=torch.bfloat16, device=dev)
     if gptq:
+        h13 = torch.empty(P, two_i, dtype=torch.bfloat16, device=dev)
         if shared is not None:
             _require(shared.shape == (T, H) and shared.dtype == torch.bfloat16 and shared.stride(1) == 1,
                      "shared must be bf16 [T, H]")
@@ -1425,11 +1425,19 @@ def moe_forward(x: torch.Tensor, router_logits: Optional[torch.Tensor], w13: tor
         xin, xs = w8a8_quantize(x)              # per token, once for all its experts
         g.operand_dtype, g.x_scale = _C.HYMETA_I8, _p(xs)
         g.w_scale = C.c_void_p(w13_scale.data_ptr() - (lo * two_i * 4 if compact else 0))
-    g.x, g.weights, g.out, g.expert_offsets = _p(xin), w13_base, _p(h13), _p(offsets)
+    g.x, g.weights, g.expert_offsets = _p(xin), w13_base, _p(offsets)
     g.a_rows, g.a_rows_div, g.max_rows, g.K, g.N = _p(sorted_pair), top_k, P, H, two_i
     g.local_expert_begin, g.local_expert_end = lo, hi
-    g.x_stride_m, g.out_stride_m, g.w_stride_e = xin.stride(0), h13.stride(0), w13.stride(0)
-    _C.check(lib.hymeta_moe_gemm(C.byref(g), st), "hymeta_moe_gemm (w13)")
+    g.x_stride_m, g.out_stride_m, g.w_stride_e = xin.stride(0), inter, w13.stride(0)
+    activates = lib.hymeta_moe_gemm_activates(C.byref(g)) == 1      # many rows per expert: silu and mul in the GEMM's epilogue
+    if activates:
+        hact = torch.empty(P, inter, dtype=torch.bfloat16, device=dev)
+        g.out = _p(hact)
+        _C.check(lib.hymeta_moe_gemm_act(C.byref(g), _C.GEMM_ACT_SILU, 0.0, 0.0, st), "hymeta_moe_gemm_act (w13)")
+    else:
+        h13 = torch.empty(P, two_i, dtype=torch.bfloat16, device=dev)
+        g.out, g.out_stride_m = _p(h13), h13.stride(0)
+        _C.check(lib.hymeta_moe_gemm(C.byref(g), st), "hymeta_moe_gemm (w13)")
 
     if shared is not None:
         _require(shared.shape == (T, H) and shared.dtype == torch.bfloat16 and shared.stride(1) == 1,
@@ -1442,12 +1450,12 @@ def moe_forward(x: torch.Tensor, router_logits: Optional[torch.Tensor], w13: tor
     # slots in use are a prefix only when lo == 0; otherwise act on all P rows (unused rows are never read)
     d = _C.MoeGemmArgs()
     if i8:
-        hact, hs = silu_and_mul_int8(h13)       # activation and per-row quantisation in one launch
+        # activation and per-row quantisation in one launch, or the rows of the activating GEMM quantised
+        hact, hs = w8a8_quantize(hact) if activates else silu_and_mul_int8(h13)
         d.operand_dtype, d.x_scale = _C.HYMETA_I8, _p(hs)
         d.w_scale = C.c_void_p(w2_scale.data_ptr() - (lo * H * 4 if compact else 0))
-    else:
-        hact = torch.empty(P, inter, dtype=torch.bfloat16, device=dev)
-        silu_and_mul(h13, out=hact)
+    elif not activates:
+        hact = silu_and_mul(h13)
     d.x, d.x_stride_m = _p(hact), hact.stride(0)
     y = out if fuse_combine else torch.empty(P, H, dtype=torch.bfloat16, device=dev)
     d.weights, d.out, d.expert_offsets = w2_base, _p(y), _p(offsets)
@@ -2129,14 +2137,21 @@ def moe_routed_forward(x: torch.Tensor, router_weight: torch.Tensor, router_bias
         return o if choice is None else (o, identity_weight, gate)
 
     if (x.dtype == torch.bfloat16 and moe_mfma_shapes(H, inter) and n1 % 64 == 0 and E <= 64 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0):
-        h1 = torch.empty(P, n1, dtype=torch.bfloat16, device=dev)
         g = _C.MoeGemmArgs()
-        g.x, g.weights, g.out, g.expert_offsets = _p(x), _p(w1), _p(h1), _p(offsets)
+        g.x, g.weights, g.expert_offsets = _p(x), _p(w1), _p(offsets)
         g.a_rows, g.a_rows_div, g.max_rows, g.K, g.N = _p(sorted_pair), top_k, P, H, n1
         g.local_expert_begin, g.local_expert_end = 0, E
-        g.x_stride_m, g.out_stride_m, g.w_stride_e = x.stride(0), h1.stride(0), w1.stride(0)
-        _C.check(lib.hymeta_moe_gemm(C.byref(g), st), "hymeta_moe_gemm (w1)")
-        hact = clamped_glu(h1, limit, alpha) if expert_act == "clamped_glu" else silu_mul(h1) if gated else relu_squared(h1, out=h1)
+        g.x_stride_m, g.out_stride_m, g.w_stride_e = x.stride(0), inter, w1.stride(0)
+        if gated and lib.hymeta_moe_gemm_activates(C.byref(g)) == 1:      # many rows per expert: the activation in the GEMM's epilogue
+            hact = torch.empty(P, inter, dtype=torch.bfloat16, device=dev)
+            g.out = _p(hact)
+            act = _C.GEMM_ACT_CLAMPED_GLU if expert_act == "clamped_glu" else _C.GEMM_ACT_SILU_EXACT
+            _C.check(lib.hymeta_moe_gemm_act(C.byref(g), act, limit, alpha, st), "hymeta_moe_gemm_act (w1)")
+        else:
+            h1 = torch.empty(P, n1, dtype=torch.bfloat16, device=dev)
+            g.out, g.out_stride_m = _p(h1), h1.stride(0)
+            _C.check(lib.hymeta_moe_gemm(C.byref(g), st), "hymeta_moe_gemm (w1)")
+            hact = clamped_glu(h1, limit, alpha) if expert_act == "clamped_glu" else silu_mul(h1) if gated else relu_squared(h1, out=h1)
         y = torch.empty(P, H, dtype=torch.bfloat16, device=dev)
         d = _C.MoeGemmArgs()
         d.x, d.x_stride_m, d.weights, d.out, d.expert_offsets = _p(hact), hact.stride(0), _p(w2), _p(y), _p(offsets)
