@@ -738,7 +738,7 @@ int hymeta_advance_step(int32_t num_seqs, int32_t num_queries, int32_t block_siz
                         const int64_t* sampled_token_ids, int64_t* input_positions, int32_t* seq_lens, int64_t* slot_mapping,
                         const int32_t* block_tables, int64_t block_table_stride, hymeta_stream_t stream);
 
-/* The gate/up projection of a gated MLP with its activation in the GEMM's epilogue, for decode-sized batches:
+/* The gate/up projection of a gated MLP with its activation in the GEMM's epilogue, for decode-sized batches and prompts:
  * weight = [gate rows | up rows] (N rows in all, the fused gate_up_proj), out bf16 [M, N / 2] =
  * silu(x gate^T) * (x up^T), both factors rounded to bf16 before the product -- the arithmetic of
  * hymeta_bf16_gemm followed by hymeta_silu_and_mul (the same bits whenever that call sums K in one slice),
@@ -746,7 +746,8 @@ int hymeta_advance_step(int32_t num_seqs, int32_t num_queries, int32_t block_siz
  * Replaces MergedColumnParallelLinear + SiluAndMul in the MLP forward
  * (vllm_hymeta/model_for_7B/modeling_gla_swa.py:108-121, vllm_hymeta/models/modeling_hymeta.py:262-271).
  * bias must be NULL, the workspace fields are ignored.  Takes M <= 128, K % 64 == 0, N % 128 == 0, and from 129 to
- * 256 rows the shapes for which hymeta_bf16_gemm_takes(M, K, N, 1) says so (matrices wide enough for 128 whole tiles);
+ * 256 rows the shapes for which hymeta_bf16_gemm_takes(M, K, N, 1) says so (matrices wide enough for 128 whole tiles); with
+ * more rows likewise (513 to 2048 tiles of 256 x 256; then w_stride_n == K, and x within 4 GiB);
  * other shapes are HYMETA_ERR_UNSUPPORTED: run the two calls. */
 int hymeta_bf16_gemm_silu_mul(const hymeta_bf16_gemm_args* args, hymeta_stream_t stream);
 

@@ -108,3 +108,46 @@ def test_what_the_tiles_do_not_take():
     assert lib.hymeta_moe_gemm_activates(C.byref(a)) == 1
     assert lib.hymeta_moe_gemm_act(C.byref(a), CLAMPED, 7.0, 1.702, None) == unsupported
     assert lib.hymeta_moe_gemm_act(C.byref(a), 4, 0.0, 0.0, None) == -1
+
+
+@pytest.mark.parametrize("M,N,K", [(1030, 32768, 256), (2307, 14336, 320)])      # ragged last row tiles; whole rounds and halves behind them
+def test_gate_up_of_a_prompt(M, N, K):
+    """The activation in the epilogue: the bits of the exact sums, rounded, then the activation's own launch."""
+    from vllm_hymeta import hip_ops
+    g = gen(5)
+    x = _ints(g, -3, 3, M, K).to(torch.bfloat16).cuda()
+    w = _ints(g, -2, 2, N, K).to(torch.bfloat16).cuda()
+    assert hip_ops.gemm_silu_mul_supported(x, w)
+    out = hip_ops.gemm_silu_mul(x, w)
+    assert torch.equal(out, hip_ops.silu_and_mul((x.float() @ w.float().t()).to(torch.bfloat16)))
+    # a view of wider rows; a shape of too few tiles is left to the library
+    wide = torch.zeros(M, K + 64, dtype=torch.bfloat16, device="cuda")
+    wide[:, :K] = x
+    assert torch.equal(hip_ops.gemm_silu_mul(wide[:, :K], w), out)
+    assert not hip_ops.gemm_silu_mul_supported(x[:300], w[:8192])
+
+
+@pytest.mark.parametrize("M,N,K", [(1030, 4608, 512), (300, 16384, 640), (5000, 1024, 1024)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_w8a8_linear_of_a_prompt(M, N, K, gated):
+    """Exact int32 sums, (sum * x_scale) * w_scale + bias in one fused step, one rounding: powers of two keep all of it exact
+    but the bias's sum, which fp64 gives to the same bf16 (24 + 8 bits)."""
+    from vllm_hymeta import hip_ops
+    g = gen(6)
+    xq = _ints(g, -127, 127, M, K).to(torch.int8)
+    xq[:, 0] = 127                                                   # the row's largest: its scale is exactly the one chosen
+    scale = 2.0 ** _ints(g, -9, -5, M).float()
+    x = (xq.float() * scale[:, None]).to(torch.bfloat16).cuda()      # 7 bits: exact
+    w = _ints(g, -127, 127, N, K).to(torch.int8).cuda()
+    ws = (2.0 ** _ints(g, -9, -6, N).float()).cuda()
+    bias = _ints(g, -64, 64, N).to(torch.bfloat16).cuda()
+    q, s = hip_ops.w8a8_quantize(x)
+    assert torch.equal(q.cpu(), xq) and torch.equal(s.cpu(), scale)
+    sums = (q.double() @ w.double().t()) * s.double()[:, None] * ws.double()
+    if gated:
+        out = hip_ops.gemm_silu_mul(x, w, ws)
+        ref = hip_ops.silu_and_mul(sums.to(torch.bfloat16))
+    else:
+        out = hip_ops.w8a8_gemm(x, w, ws, bias=bias)
+        ref = (sums + bias.double()).float().to(torch.bfloat16)
+    assert torch.equal(out, ref)

@@ -88,7 +88,7 @@ struct Place {
 // The tiles of all experts stand in one order, a lane per expert.  An expert's tiles go in blocks of up to kDeep row tiles x
 // kWide column tiles, the blocks of one run of columns next to each other: 32 tiles in a row are about one block, which a die's
 // units take together (12 panels a step where a row of tiles would read 33), and the eight blocks of a round share what they
-// read from memory.  In a last, incomplete round of at most half the units every tile is cut into halves of 128 rows, which take
+// read from memory.  The columns are swept once for every 32 row tiles, whose x stays in the last-level cache.  In a last, incomplete round of at most half the units every tile is cut into halves of 128 rows, which take
 // 0.6 of a tile's time.  Wave-uniform; false: nothing to do.
 __device__ __forceinline__ bool find_place(const TileGemmArgs& a, int lane, Place* p) {
   constexpr int kRound = kDies * kUnits;
@@ -120,9 +120,12 @@ __device__ __forceinline__ bool find_place(const TileGemmArgs& a, int lane, Plac
     t = whole + first + j;
   }
   const int at = __popcll(__ballot(upto <= t));              // experts whose tiles all lie in front of t
-  const int in = t - (at > 0 ? __builtin_amdgcn_readlane(upto, at - 1) : 0);
+  const int of_expert = t - (at > 0 ? __builtin_amdgcn_readlane(upto, at - 1) : 0);
   lo = __builtin_amdgcn_readlane(lo, at), hi = __builtin_amdgcn_readlane(hi, at);
-  const int row_tiles = (hi - lo + kTile - 1) / kTile;
+  constexpr int kSweep = kDeep * kDies;
+  const int sweep = of_expert / (kSweep * cols), in = of_expert - sweep * kSweep * cols;
+  lo += sweep * kSweep * kTile;
+  const int row_tiles = min(kSweep, (hi - lo + kTile - 1) / kTile);
   const int col0 = in / (kWide * row_tiles) * kWide, wide = min(kWide, cols - col0), in_cols = in - col0 * row_tiles;
   const int deep = (row_tiles + (row_tiles + kDeep - 1) / kDeep - 1) / ((row_tiles + kDeep - 1) / kDeep);
   const int row0 = in_cols / (deep * wide) * deep, in_block = in_cols - row0 * wide;

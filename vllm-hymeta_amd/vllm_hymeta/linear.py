@@ -29,10 +29,10 @@ def w8a8_use_library(rows: int, in_features: int, out_features: int) -> bool:
     epilogue (``hymeta_w8a8_gemm``: K in whole 128-deep steps, N in whole 128-column tiles) or quantise -> library int8
     GEMM -> scale (three launches, the int32 sums through memory); both give the same bits.  The tiled kernel takes the
     shapes where it was measured ahead (7B shapes, us, tiled / library): gate_up 70 / 72 at 129 rows, 68 / 101 at 256,
-    331 / 412 at 2048, 4400 / 5568 at 32768 (up to 256 rows the streaming kernel has since taken over: 59 at 256, the
-    down projection 48 against 118); qkv 67 / 71 at 2048, 601 / 736 at 32768; o 51 / 57 and 481 / 594; the deep
-    narrow down projection (K = 5.3 N: few tiles, long K loops) 587 / 683 at 8192 and level at 32768 -- and leaves the
-    rest to the library (qkv / o below 1024 rows, down below 4096: 210 / 189 at 2048)."""
+    271 / 412 at 2048, 3920 / 5568 at 32768 (up to 256 rows the streaming kernel has since taken over: 59 at 256, the
+    down projection 48 against 118); qkv 57 / 71 at 2048; o 45 / 57; the deep
+    narrow down projection (K = 5.3 N: few tiles, long K loops) 247 / 299 at 4096, 496 / 683 at 8192 -- and leaves the
+    rest to the library (qkv / o below 1024 rows; down to 2048 rows, where 157 / 173 would be ahead but 1024 are 147 / 104)."""
     if rows <= W8A8_STREAM_ROWS:
         return False
     if in_features % 128 != 0 or out_features % 128 != 0:
@@ -42,7 +42,7 @@ def w8a8_use_library(rows: int, in_features: int, out_features: int) -> bool:
     if out_features >= 16384:
         return False
     if in_features >= 4 * out_features:
-        return rows < 4096
+        return rows <= 2048
     return rows < 1024
 
 
@@ -76,13 +76,21 @@ class HymetaLinear(torch.nn.Module):
 
     def forward_silu_mul(self, x: torch.Tensor) -> torch.Tensor:
         """``silu(y[:, :I]) * y[:, I:]`` of ``y = self(x)`` for a fused gate/up projection (output rows = gate, then up):
-        decode-sized batches of a bf16 or W8A8 projection run it in the GEMM's epilogue (same bits, one launch, no
-        ``[M, 2 I]`` intermediate)."""
+        decode-sized batches and prompts of a bf16 or W8A8 projection, and prompts of an expanded GPTQ one, run it
+        in the GEMM's epilogue (one launch, no ``[M, 2 I]`` intermediate)."""
         if self.bias is None and self.kind in ("bf16", "w8a8"):
             w = self.weight if self.kind == "bf16" else self.qweight
             if hip_ops.gemm_silu_mul_supported(x, w):
                 return hip_ops.gemm_silu_mul(x, w, None if self.kind == "bf16" else self.w_scale)
+        if self.bias is None and self.kind == "gptq" and x.shape[0] > GPTQ_EXPAND_ROWS and hip_ops.gptq_dequant_nk_supported(self.qweight, self.meta["bits"]):
+            w = self._expanded(True)
+            return hip_ops.gemm_silu_mul(x, w) if hip_ops.gemm_silu_mul_supported(x, w) else hip_ops.silu_and_mul(torch.nn.functional.linear(x, w))
         return hip_ops.silu_and_mul(self(x))
+
+    def _expanded(self, transposed: bool) -> torch.Tensor:
+        """A GPTQ linear's weights in bf16: [in, out], or ``transposed`` [out, in]."""
+        return hip_ops.gptq_dequant(self.qweight, self.qzeros, self.scales, self.meta["bits"], self.meta["group_size"],
+                                    zero_offset=self.meta.get("zero_offset", 1), transposed=transposed)
 
     def forward(self, x: torch.Tensor, defer: bool = False):
         """``defer``: the caller passes the result straight to a fused add + RMS norm (``HymetaRMSNorm`` with a
@@ -109,8 +117,7 @@ class HymetaLinear(torch.nn.Module):
                 # prefill regime: expand the weights once, plain library bf16 GEMM on them -- as W^T [N, K] where the
                 # expansion kernel's tiles cover the matrix, the layout the library runs 12 % faster at 32768 rows
                 nk = hip_ops.gptq_dequant_nk_supported(self.qweight, self.meta["bits"])
-                w = hip_ops.gptq_dequant(self.qweight, self.qzeros, self.scales, self.meta["bits"],
-                                         self.meta["group_size"], zero_offset=self.meta.get("zero_offset", 1), transposed=nk)
+                w = self._expanded(nk)
                 if nk:
                     return torch.nn.functional.linear(x, w, self.bias)
                 y = torch.matmul(x, w)
