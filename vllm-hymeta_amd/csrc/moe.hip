@@ -3,16 +3,16 @@
 // expert GEMMs straight from the per-expert weight stacks, SiLU-and-multiply, and the combine
 // with the shared expert.  Everything stays on the device: no host read of the expert counts.
 //
-//   route    one lane-group per token: softmax over E <= 64 logits, k <= 2 picks, histogram
-//   offsets  exclusive prefix over the experts (one workgroup)
-//   scatter  pair -> slot offsets[e] + ticket; the order inside an expert is arbitrary, which
-//            cannot change a result: rows of a GEMM are independent
+//   route    one thread per token: softmax over E <= 64 logits, k <= 2 picks
+//   sort     one workgroup: pairs counted, offsets, slots (pair_sort.h); the order inside an expert cannot change a result: rows
+//            of a GEMM are independent
 //   gemm     out[row] = x[a_rows[row]] W[e]^T for the rows of expert e; 64 columns per workgroup,
 //            the 4 waves take alternate 32-deep k-steps (bf16 MFMA 16x16x32, operands straight
 //            from global memory: both x rows and W rows are K-contiguous), LDS reduce
 //   combine  out[t] = sum_k y[pos[t,k]] (+ shared[t]), y weighted in the down GEMM; pairs of non-local experts
 //            (expert parallelism) carry pos = -1 and add nothing
 #include "common.h"
+#include "pair_sort.h"
 #include "tile_gemm.h"
 #include "w8a8_quant.h"
 
@@ -68,80 +68,56 @@ __device__ __forceinline__ f32x4 moe_sums_to_f32(const hymeta_moe_gemm_args& a, 
 
 }  // namespace
 
-// One thread per token (E is small).  counts[e] += 1 per pair.
-__global__ __launch_bounds__(256) void moe_route_kernel(hymeta_moe_route_args a) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
+// One thread per token, its logits in registers (MaxE >= num_experts of them, read at once); 64 threads a workgroup, so that a
+// prompt's tokens spread over the chip.  Bound by one trip to memory: 8192 tokens of 16 experts 6 us, 35 with a logit at a time
+// into scratch memory and a counter in memory for every pair.
+template <int MaxE>
+__global__ __launch_bounds__(64) void moe_route_kernel(hymeta_moe_route_args a) {
+  const int t = blockIdx.x * 64 + threadIdx.x;
   if (t >= a.num_tokens) return;
-  float logit[kMaxExperts];
+  float logit[MaxE];
+  const int64_t row = static_cast<int64_t>(t) * a.logits_stride_t;
+#pragma unroll
+  for (int e = 0; e < MaxE; ++e) {
+    const int64_t i = row + min(e, a.num_experts - 1);
+    logit[e] = a.logits_dtype == HYMETA_F32 ? static_cast<const float*>(a.router_logits)[i] : bf2f(static_cast<const uint16_t*>(a.router_logits)[i]);
+  }
   float mx = -INFINITY;
-  for (int e = 0; e < a.num_experts; ++e) {
-    const int64_t i = static_cast<int64_t>(t) * a.logits_stride_t + e;
-    logit[e] = a.logits_dtype == HYMETA_F32 ? reinterpret_cast<const float*>(a.router_logits)[i]
-                                            : bf2f(reinterpret_cast<const uint16_t*>(a.router_logits)[i]);
-    mx = fmaxf(mx, logit[e]);
-  }
+#pragma unroll
+  for (int e = 0; e < MaxE; ++e)
+    if (e < a.num_experts) mx = fmaxf(mx, logit[e]);
   float denom = 0.f;
-  for (int e = 0; e < a.num_experts; ++e) {
-    logit[e] = expf(logit[e] - mx);
-    denom += logit[e];
-  }
+#pragma unroll
+  for (int e = 0; e < MaxE; ++e)
+    if (e < a.num_experts) {
+      logit[e] = expf(logit[e] - mx);
+      denom += logit[e];
+    }
   int pick[2] = {0, 0};
   float pw[2] = {0.f, 0.f};
-  for (int j = 0; j < a.top_k; ++j) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if (j >= a.top_k) break;
     // starts from the first expert not taken: a row of NaN logits compares false everywhere and keeps it, with a NaN
-    // weight -- a valid index for the counters below and a NaN row out, never index -1
-    int best = (j == 1 && pick[0] == 0) ? 1 : 0;
-    float bv = logit[best];
-    for (int e = 0; e < a.num_experts; ++e) {
-      const bool taken = j == 1 && e == pick[0];
-      if (!taken && logit[e] > bv) {   // first maximum wins, as torch.topk on ties of distinct indices
-        bv = logit[e];
-        best = e;
-      }
-    }
+    // weight -- a valid index for the counters behind and a NaN row out, never index -1
+    const bool second = j == 1 && pick[0] == 0;
+    int best = second ? 1 : 0;
+    float bv = second && MaxE > 1 ? logit[MaxE > 1 ? 1 : 0] : logit[0];
+#pragma unroll
+    for (int e = 0; e < MaxE; ++e)
+      if (e < a.num_experts && !(j == 1 && e == pick[0]) && logit[e] > bv) bv = logit[e], best = e;   // first maximum wins, as torch.topk on ties of distinct indices
     pick[j] = best;
     pw[j] = bv / denom;
   }
   if (a.renormalize) {
-    float s = 0.f;
-    for (int j = 0; j < a.top_k; ++j) s += pw[j];
-    for (int j = 0; j < a.top_k; ++j) pw[j] /= s;
+    float s = pw[0];
+    if (a.top_k == 2) s += pw[1];
+    pw[0] /= s, pw[1] /= s;
   }
   for (int j = 0; j < a.top_k; ++j) {
     a.topk_ids[t * a.top_k + j] = pick[j];
     a.topk_weights[t * a.top_k + j] = pw[j];
-    atomicAdd(a.counts + pick[j], 1);
   }
-}
-
-__global__ __launch_bounds__(64) void moe_zero_counts_kernel(hymeta_moe_route_args a) {
-  if (static_cast<int>(threadIdx.x) < a.num_experts) a.counts[threadIdx.x] = 0;
-}
-
-// offsets[0..E] = exclusive prefix of counts; cursors zeroed.
-__global__ __launch_bounds__(64) void moe_offsets_kernel(hymeta_moe_route_args a) {
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int e = 0; e < a.num_experts; ++e) {
-      a.expert_offsets[e] = run;
-      run += a.counts[e];
-      a.cursors[e] = 0;
-    }
-    a.expert_offsets[a.num_experts] = run;
-  }
-}
-
-__global__ __launch_bounds__(256) void moe_scatter_kernel(hymeta_moe_route_args a) {
-  const int p = blockIdx.x * 256 + threadIdx.x;   // pair index = token * top_k + choice
-  if (p >= a.num_tokens * a.top_k) return;
-  const int e = a.topk_ids[p];
-  const bool local = e >= a.local_expert_begin && e < a.local_expert_end;
-  int pos = -1;
-  if (local) {
-    pos = a.expert_offsets[e] + atomicAdd(a.cursors + e, 1);
-    a.sorted_pair[pos] = p;
-  }
-  a.pair_pos[p] = pos;
 }
 
 // Decode-sized batches: the router's linear layer, the routing, the expert offsets and the scatter in ONE launch.
@@ -540,7 +516,7 @@ __global__ __launch_bounds__(256) void moe_gemm_lines_kernel(hymeta_moe_gemm_arg
 constexpr int kTK = 64;
 constexpr int kTilePitch = 2 * kTK;                 // bytes per staged row
 constexpr int kTiledMinRowsPerExpert = 8;           // measured: level at 4 rows per expert, 15 % ahead at 16, 2.6x at 512
-constexpr int kBigTileMinRowsPerExpert = 128, kBigTileMinTiles = 160;
+constexpr int kBigTileMinTiles = 160;
 
 template <int BM, int BN, int WM, int WN, bool I8>
 __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void moe_gemm_tiled_kernel(hymeta_moe_gemm_args a) {
@@ -793,14 +769,15 @@ extern "C" int hymeta_moe_route(const hymeta_moe_route_args* args, hymeta_stream
     return HYMETA_ERR_INVALID_ARG;
   if (!a.counts || !a.expert_offsets || !a.cursors) return HYMETA_ERR_INVALID_ARG;
   hipStream_t s = begin_launches(stream);
-  hipLaunchKernelGGL(moe_zero_counts_kernel, dim3(1), dim3(64), 0, s, a);      // a kernel, not a memset node: see the header
   if (a.num_tokens > 0) {
     if (!a.router_logits || !a.topk_ids || !a.topk_weights || !a.sorted_pair || !a.pair_pos) return HYMETA_ERR_INVALID_ARG;
-    hipLaunchKernelGGL(moe_route_kernel, dim3((a.num_tokens + 255) / 256), dim3(256), 0, s, a);
+    const dim3 grid((a.num_tokens + 63) / 64), block(64);
+    if (a.num_experts <= 8) hipLaunchKernelGGL(moe_route_kernel<8>, grid, block, 0, s, a);
+    else if (a.num_experts <= 16) hipLaunchKernelGGL(moe_route_kernel<16>, grid, block, 0, s, a);
+    else hipLaunchKernelGGL(moe_route_kernel<kMaxExperts>, grid, block, 0, s, a);
   }
-  hipLaunchKernelGGL(moe_offsets_kernel, dim3(1), dim3(64), 0, s, a);
-  if (a.num_tokens > 0)
-    hipLaunchKernelGGL(moe_scatter_kernel, dim3((a.num_tokens * a.top_k + 255) / 256), dim3(256), 0, s, a);
+  const PairSort sort = {a.topk_ids, a.num_tokens * a.top_k, a.num_experts, a.local_expert_begin, a.local_expert_end, a.expert_offsets, a.sorted_pair, a.pair_pos};
+  hipLaunchKernelGGL(sort_pairs_kernel, dim3(1), dim3(kSortThreads), 0, s, sort);
   return launch_status();
 }
 
@@ -833,11 +810,11 @@ enum class MoeGemmKind { kBigTiles, kTiles, kLines, kFragments };
 MoeGemmKind moe_gemm_kind(int64_t max_rows, int experts, int K, int N) {
   // tiled grouped GEMM once the experts average more than a few rows (prefill chunks); the large tile when they fill it
   if (max_rows > static_cast<int64_t>(kTiledMinRowsPerExpert) * experts && K % kTK == 0) {
-    // tiles of 256 where the experts fill half of one on average and the tiles (an expert's rows scatter around the average)
-    // nearly fill the chip once: 16 experts on 2048 tokens of 3584 columns 560 -> 516 us, 8 on 1400 936 -> 705; with 112 rows
-    // an expert 424 -> 459, with 64 to 128 tiles 215 -> 226
+    // tiles of 256 where the experts fill half of one on average (a little more with many columns, whose tiles fill the chip either
+    // way) and the tiles (an expert's rows scatter around the average) nearly fill the chip once: 16 experts on 2048 tokens of 3584
+    // columns 560 -> 497 us, 8 on 1400 936 -> 705; with 112 rows an expert 424 -> 459, with 64 to 128 tiles 215 -> 226
     const int64_t rows = max_rows / experts, tiles = (rows + 64 + 255) / 256 * experts * (N / 256);
-    if (rows >= kBigTileMinRowsPerExpert && tiles >= kBigTileMinTiles && N % 256 == 0) return MoeGemmKind::kBigTiles;
+    if (rows >= (N > 4096 ? 144 : 128) && tiles >= kBigTileMinTiles && N % 256 == 0) return MoeGemmKind::kBigTiles;
     if (N % 128 == 0) return MoeGemmKind::kTiles;
   }
   static const bool lines = [] {

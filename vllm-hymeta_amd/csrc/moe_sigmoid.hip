@@ -2,13 +2,11 @@
 // (sigmoid scores normalised over the chosen and scaled, a softmax over the chosen logits alone, or a softmax over all
 // outputs with a corrected, group-limited choice and identity experts); then the counting sort by expert that the grouped
 // GEMMs of the routed block read.
-#include "act_types.h"
+#include "pair_sort.h"
 
 namespace hymeta {
 
 namespace {
-
-constexpr int kSortThreads = 1024;
 
 // grid = tokens in fours, 256 threads.  The experts' dot products over the workgroup, eight experts and four tokens a
 // round (a weight is loaded once for the four tokens; the loads of a round are independent of each other; the partial
@@ -171,43 +169,6 @@ __global__ __launch_bounds__(256) void moe_scores_topk_kernel(hymeta_moe_route_s
   for (int k = lane; k < a.top_k; k += 64) a.topk_weights[t * a.top_k + k] = s_top[wave][k] * inv;
 }
 
-// One workgroup: count the pairs per expert in LDS, prefix, scatter (the order inside an expert's run depends on the
-// atomics' arrival; every pair's row is computed on its own, so the results do not).
-__global__ __launch_bounds__(kSortThreads) void moe_sort_pairs_kernel(hymeta_moe_route_sigmoid_args a) {
-  __shared__ int s_count[HYMETA_MOE_TABLE_MAX_EXPERTS];
-  __shared__ int s_off[HYMETA_MOE_TABLE_MAX_EXPERTS + 1];
-  // identity experts have no rows: their pairs are left out (pair_pos -1), and the offsets cover the experts before them
-  const bool has_identity = a.score_mode == HYMETA_ROUTE_SOFTMAX_GROUPED && a.first_identity > 0;
-  const int tid = threadIdx.x, E = has_identity ? a.first_identity : a.num_experts, P = a.num_tokens * a.top_k;
-  for (int e = tid; e < E; e += kSortThreads) s_count[e] = 0;
-  __syncthreads();
-  for (int p = tid; p < P; p += kSortThreads)
-    if (a.topk_ids[p] < E) atomicAdd(&s_count[a.topk_ids[p]], 1);
-  __syncthreads();
-  if (tid == 0) {
-    int run = 0;
-    for (int e = 0; e < E; ++e) {
-      s_off[e] = run;
-      run += s_count[e];
-    }
-    s_off[E] = run;
-  }
-  __syncthreads();
-  for (int e = tid; e <= E; e += kSortThreads) a.expert_offsets[e] = s_off[e];
-  for (int e = tid; e < E; e += kSortThreads) s_count[e] = 0;
-  __syncthreads();
-  for (int p = tid; p < P; p += kSortThreads) {
-    const int e = a.topk_ids[p];
-    if (e >= E) {
-      a.pair_pos[p] = -1;
-      continue;
-    }
-    const int pos = s_off[e] + atomicAdd(&s_count[e], 1);
-    a.sorted_pair[pos] = p;
-    a.pair_pos[p] = pos;
-  }
-}
-
 }  // namespace
 
 }  // namespace hymeta
@@ -237,6 +198,10 @@ extern "C" int hymeta_moe_route_sigmoid(const hymeta_moe_route_sigmoid_args* arg
     if (a.act_dtype == HYMETA_BF16) hipLaunchKernelGGL(moe_scores_topk_kernel<ActBf16>, dim3((a.num_tokens + kRouteTokens - 1) / kRouteTokens), dim3(256), 0, st, a);
     else hipLaunchKernelGGL(moe_scores_topk_kernel<ActF32>, dim3((a.num_tokens + kRouteTokens - 1) / kRouteTokens), dim3(256), 0, st, a);
   }
-  hipLaunchKernelGGL(moe_sort_pairs_kernel, dim3(1), dim3(kSortThreads), 0, st, a);
+  // identity experts have no rows: their pairs are left out (pair_pos -1), and the offsets cover the experts before them
+  const bool has_identity = a.score_mode == HYMETA_ROUTE_SOFTMAX_GROUPED && a.first_identity > 0;
+  const int experts = has_identity ? a.first_identity : a.num_experts;
+  const PairSort sort = {a.topk_ids, a.num_tokens * a.top_k, experts, 0, experts, a.expert_offsets, a.sorted_pair, a.pair_pos};
+  hipLaunchKernelGGL(sort_pairs_kernel, dim3(1), dim3(kSortThreads), 0, st, sort);
   return launch_status();
 }
