@@ -1261,7 +1261,8 @@ typedef struct hymeta_sink_attention_args {
 size_t hymeta_sink_attention_workspace_bytes(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads, int32_t v_dim,
                                              int32_t max_seq_len);
 /* The most a call whose longest portion has max_query_len > 1 rows can use, no less than the above: the keys of short portions are
- * cut into slices, whose partials lie behind those of single rows.  span: the keys a row sees before keep_first, by a window (window_left + 1) or a chunk, 0: all.  With less, but at
+ * cut into slices, whose partials lie behind those of single rows (HYMETA_KV_SHARED_KEY with keys of more than 192 elements: in
+ * their place, so that the larger of the two is enough).  span: the keys a row sees before keep_first, by a window (window_left + 1) or a chunk, 0: all.  With less, but at
  * least the above, the call cuts them into fewer. */
 size_t hymeta_sink_attention_portion_workspace_bytes(int32_t num_tokens, int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads, int32_t v_dim,
                                                      int32_t max_query_len, int32_t max_seq_len, int64_t span, int32_t keep_first);

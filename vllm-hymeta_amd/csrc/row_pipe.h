@@ -1,4 +1,5 @@
-// Prompts' portions of the attention over paged rows, key and value apart and up to 128 elements each: included by sink_attn.hip.
+// Prompts' portions of the attention over paged rows, key and value apart, up to 128 elements each, or one key of 256 or 512
+// for all heads: included by sink_attn.hip.
 #pragma once
 
 #include "row_attn.h"
@@ -17,15 +18,26 @@ namespace {
 // 8192 rows x 28 heads of 128 with 4 key/value heads, logarithmic bias 754 -> 695 us, a window of 1024 201 -> 184; three portions
 // of 700 behind 1000 94.8 -> 75; six of 324 behind 818, window 1024, 60.6 -> 49; four of 1500 behind 3000, 16 heads, chunks of
 // 2048, 120 -> 111; 4000 rows capped, window 1024, 115 -> 108.
+//
+// Long keys (256 or 512 elements, which all heads share): one wave on a SIMD, whose registers then hold the queries (128), the
+// weighted values and two tiles' scores (64 each); the images of 64 keys fill the LDS.  All weights of a tile are formed under the
+// products of the next scores, four fifths of the step.  A wave of 16 rows that read the whole tile for them was bound by LDS; with
+// 32 rows the matrix pipe (1.45 us a tile of 64 keys of 512) and the lone wave's issue add up: 2.76 us a tile, of which the copies'
+// issue takes 0.36, exponentials and rounding 0.30, half of the key reads 0.09; around a block's tiles lie about 12 us, half of them
+// its queries' 128 KB from memory, which all compute units ask for at once.  28 heads, 4 value heads of 128, window 1024, with a
+// workgroup per 64 rows and head -> here: 8192 rows 1275 -> 450 us; 2048 behind 4096 390 -> 134; four of 300 behind 2000 208 -> 71; five
+// of 10 behind 5955, keys cut into slices, 97 -> 26; 300 rows alone 33 -> 26.  Level or slower: copies issued among the slots (459),
+// fragments read 10 slots ahead (452), no barrier to the compiler's order between slots (a sixth slower).
 template <int D, int DV, int Layout, int Rule>
-__global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_args a, PortionSlices ps) {
+__global__ __launch_bounds__(256, D > 192 ? 1 : 2) void row_pipe_kernel(hymeta_sink_attention_args a, PortionSlices ps) {
   static_assert(Layout == HYMETA_KV_KEY_THEN_VALUE || Layout == HYMETA_KV_SHARED_KEY, "the value lies apart from the key");
-  constexpr bool Shared = Layout == HYMETA_KV_SHARED_KEY;
+  constexpr bool Shared = Layout == HYMETA_KV_SHARED_KEY, Wide = D > 192;
   constexpr int kSteps = D / 16, CB = DV / 32, kWaves = 4, kRows = 32 * kWaves;
   constexpr int kKeyChunks = D / 8, kValueChunks = DV / 8, kKeyPitch = 2 * D, kValuePitch = 2 * DV;
-  static_assert(kRows == kPortionRows && (D == 64 || D == 128) && (DV == 64 || DV == 128), "an instruction copies whole rows");
-  __shared__ __attribute__((aligned(16))) char s_k[2][kTileKeys * kKeyPitch];
-  __shared__ __attribute__((aligned(16))) char s_v[2][kTileKeys * kValuePitch];
+  static_assert(kRows == kPortionRows && (D == 64 || D == 128 || D == 256 || D == 512) && (DV == 64 || DV == 128), "an instruction copies whole rows");
+  constexpr int kKeyImage = kTileKeys * kKeyPitch, kValueImage = kTileKeys * kValuePitch;
+  __shared__ __attribute__((aligned(16))) char s_k[2][kKeyImage];
+  __shared__ __attribute__((aligned(16))) char s_v[2][kValueImage];
 
   auto uniform = [](int x) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane(x); };
   const int group = uniform(a.num_heads / a.num_kv_heads);
@@ -60,7 +72,7 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
   const float scale = a.scale == 0.f ? 1.f : fabsf(a.scale), scale2 = scale * 1.4426950408889634f;
   const float cap_in = a.softcap > 0.f ? scale / a.softcap : 0.f, cap2 = a.softcap * 1.4426950408889634f;
   u32x4 qf[kSteps];                                   // (with the scale's sign, so that scores grow with their products)
-  {
+  auto load_queries = [&]() __attribute__((always_inline)) {
     const uint16_t* qrow = static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(row0 + qi) * a.q_stride_t + static_cast<int64_t>(h) * D + 8 * hh;
     const uint32_t sign = a.scale < 0.f ? 0x80008000u : 0u, kept_bits = a.scale == 0.f ? 0u : ~0u;
 #pragma unroll
@@ -69,7 +81,8 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
 #pragma unroll
       for (int e = 0; e < 4; ++e) qf[st][e] = (qf[st][e] & kept_bits) ^ sign;
     }
-  }
+  };
+  if (!Wide) load_queries();
   f32x16 o[CB];                                       // O^T: columns 32 cb + 8 i + 4 hh + e of the lane's row, i, e < 4
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb)
@@ -90,11 +103,13 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
   const int32_t* bt = a.block_tables + static_cast<int64_t>(s) * a.block_table_stride;
   const int shift = __builtin_ctz(a.block_size), mask = a.block_size - 1;
   auto value_twist = [](int row) __attribute__((always_inline)) { return kValueChunks == 16 ? (row & 3) << 2 : (row & 2) << 1; };
-  auto key_chunk = [&](int ln) __attribute__((always_inline)) -> uint32_t {
-    return 16 * ((ln % kKeyChunks) ^ ChunkOrder<kKeyChunks>::twist(kKeyRows * wave + ln / kKeyChunks));
+  // (long keys: an instruction's few rows leave the chunk order to its number as well, in bits that no row's offset has)
+  auto key_chunk = [&](int ln, int i) __attribute__((always_inline)) -> uint32_t {
+    return 16 * ((ln % kKeyChunks) ^ ChunkOrder<kKeyChunks>::twist(kKeyRows * (wave + kWaves * i) + ln / kKeyChunks));
   };
+  auto turn = [](int i) __attribute__((always_inline)) -> uint32_t { return 16 * ((kKeyRows * kWaves * i >> 2) & 3); };
   auto value_chunk = [&](int ln) __attribute__((always_inline)) -> uint32_t { return 16 * ((ln % kValueChunks) ^ value_twist(ln / kValueChunks)); };
-  const uint32_t kplace = static_cast<uint32_t>(lane / kKeyChunks * row_bytes) + key_chunk(lane);
+  const uint32_t kplace = static_cast<uint32_t>(lane / kKeyChunks * row_bytes) + key_chunk(lane, 0);
   const uint32_t vplace = static_cast<uint32_t>(lane / kValueChunks * row_bytes) + value_chunk(lane);
   const char* kwave = kglob + kKeyRows * wave * row_bytes;
   const char* vwave = vglob + kValueRows * wave * row_bytes;
@@ -116,7 +131,7 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
       const char* base = (value ? vwave : kwave) + ((static_cast<int64_t>(hi) << 32) | lo);
 #pragma unroll
       for (int i = 0; i < copies; ++i) {
-        copy16_to_lds(base, value ? vplace : kplace, image + 1024 * (wave + kWaves * i));
+        copy16_to_lds(base, value ? vplace : kplace ^ turn(i), image + 1024 * (wave + kWaves * i));
         base += kWaves * each * row_bytes;
       }
       return;
@@ -125,29 +140,53 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
     int ln = lane;
     asm volatile("" : "+v"(ln));                      // (nothing of this is kept in registers over the other tiles)
     const int j0 = key0(t), row_in = ln / (value ? kValueChunks : kKeyChunks);
+#pragma unroll Wide ? 4 : 1
     for (int i = 0; i < copies; ++i) {
       const int j = min(j0 + each * (wave + kWaves * i) + row_in, p_hi);
       const int64_t row = (static_cast<int64_t>(bt[j >> shift]) << shift) + (j & mask);
-      copy16_to_lds((value ? vglob : kglob) + row * row_bytes + (value ? value_chunk(ln) : key_chunk(ln)), image + 1024 * (wave + kWaves * i));
+      copy16_to_lds((value ? vglob : kglob) + row * row_bytes + (value ? value_chunk(ln) : key_chunk(ln, i)), image + 1024 * (wave + kWaves * i));
     }
   };
 
   // ---- LDS offsets of this lane's fragments.  Keys: row n, chunk 2 st + hh.  Values: a tile's 16-key step i takes its keys
   // 8 i + 4 hh + e and 32 keys further on, which are the keys whose weights the lane holds
-  int koff[kSteps], voff[CB];
+  constexpr int kOffsets = kSteps < 8 ? kSteps : 8;   // (those of a chunk 16 further on lie 256 bytes behind)
+  int koff[kOffsets], voff[CB];
 #pragma unroll
-  for (int st = 0; st < kSteps; ++st) koff[st] = n * kKeyPitch + 16 * ((2 * st + hh) ^ ChunkOrder<kKeyChunks>::twist(n));
+  for (int st = 0; st < kOffsets; ++st) koff[st] = n * kKeyPitch + 16 * ((2 * st + hh) ^ ChunkOrder<kKeyChunks>::twist(n));
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb) {
     const int R = 4 * hh + ((lane & 15) >> 2), chunk = 4 * cb + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
     voff[cb] = R * kValuePitch + 16 * (chunk ^ value_twist(R)) + 8 * (lane & 1);
   }
+  // (long keys: LDS addresses, of which the images' are out of an instruction's reach, moved from image to image behind each tile)
+  uint32_t kat[kOffsets], vat[CB];
+#pragma unroll
+  for (int i = 0; i < kOffsets; ++i) kat[i] = lds_address(s_k[0]) + koff[i];
+#pragma unroll
+  for (int i = 0; i < CB; ++i) vat[i] = lds_address(s_v[0]) + voff[i];
+  auto other_image = [&](auto& at, int count, int by) __attribute__((always_inline)) {
+    if (!Wide) return;
+#pragma unroll
+    for (int i = 0; i < count; ++i) {
+      at[i] += by;
+      asm volatile("" : "+v"(at[i]));                 // (not formed from the first image's for every read)
+    }
+  };
   f32x16 sa[2], sb[2];                                // scores: keys 32 x + 8 i + 4 hh + e of a tile, element 4 i + e of [x]
   // Fragment f of a step: f < 2 kSteps of the keys (step f / 2 of the head, half f % 2 of the tile), else of the values (16 keys
   // (f - 2 kSteps) / CB, columns 32 (f % CB) ..)
-  constexpr int NQ = 2 * kSteps, NF = NQ + 4 * CB, kAhead = 3;
+  constexpr int NQ = 2 * kSteps, NF = NQ + 4 * CB, kAhead = Wide ? 6 : 3;
+  constexpr int kUnder = Wide ? 16 : 7;               // of a tile's 16 slices of weights: under the products of the scores
   auto fragment = [&](const char* kimg, const char* vimg, int f) __attribute__((always_inline)) {
-    if (f < NQ) return ld16(kimg + koff[f >> 1] + (f & 1) * 32 * kKeyPitch);
+    if (Wide && f < NQ) return *(const __attribute__((address_space(3))) u32x4*)(kat[(f >> 1) % kOffsets] + (f >> 1) / kOffsets * 256 + (f & 1) * 32 * kKeyPitch);
+    if (Wide) {
+      const uint32_t v = vat[(f - NQ) % CB] + (f - NQ) / CB * 8 * kValuePitch;
+      const u32x2 v0 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4*)v));
+      const u32x2 v1 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4*)(v + 32 * kValuePitch)));
+      return u32x4{v0[0], v0[1], v1[0], v1[1]};
+    }
+    if (f < NQ) return ld16(kimg + koff[(f >> 1) % kOffsets] + (f >> 1) / kOffsets * 256 + (f & 1) * 32 * kKeyPitch);
     const char* v = vimg + voff[(f - NQ) % CB] + (f - NQ) / CB * 8 * kValuePitch;
     const u32x2 v0 = __builtin_bit_cast(u32x2, read_transposed(v)), v1 = __builtin_bit_cast(u32x2, read_transposed(v + 32 * kValuePitch));
     return u32x4{v0[0], v0[1], v1[0], v1[1]};
@@ -163,7 +202,10 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
       const float away = static_cast<float>(32 * x + 8 * (e >> 2) + (e & 3));
-      if (Rule == kLogBias) sc[x][e] = fmaf(ba, __builtin_amdgcn_logf(fmaf(bb, d0 - away, 1.f)), fmaf(sc[x][e], scale2, -ref));
+      if (Rule == kAnyRule) {                         // (no cap: the product scaled; no bias: ba = bb = 0)
+        const float plain = fmaf(sc[x][e], scale2, -ref), capped = fmaf(cap2, tanh_fast(sc[x][e] * cap_in), -ref);
+        sc[x][e] = fmaf(ba, __builtin_amdgcn_logf(fmaf(bb, d0 - away, 1.f)), a.softcap > 0.f ? capped : plain);
+      } else if (Rule == kLogBias) sc[x][e] = fmaf(ba, __builtin_amdgcn_logf(fmaf(bb, d0 - away, 1.f)), fmaf(sc[x][e], scale2, -ref));
       else sc[x][e] = fmaf(cap2, tanh_fast(sc[x][e] * cap_in), -ref);
     }
   };
@@ -218,7 +260,7 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
     settle(t, next, mx);
   };
   // Weights of tile t (scores `cur`) times its values, and the scores of tile t + 1.  A slot is a fragment's products, the read of
-  // one a few slots ahead and a slice of the vector work: pairs of weights (7 of 16 under the scores' products), then scores
+  // one a few slots ahead and a slice of the vector work: pairs of weights (kUnder of 16 under the scores' products), then scores
   auto step = [&](int t, const char* kimg, const char* vimg, f32x16 (&cur)[2], f32x16 (&next)[2]) __attribute__((always_inline)) {
     u32x4 fr[NF], hi[4], lo[4];                       // a weight's bf16 parts, of 16 keys, as the second product's operand
     const float d0 = distance(t + 1);
@@ -237,7 +279,8 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
         o[cb] = product(fr[f], hi[i], o[cb]);
         o[cb] = product(fr[f], lo[i], o[cb]);
       }
-      const int p_lo = f < NQ ? f * 7 / NQ : 7 + (f - NQ) * 9 / (5 * CB / 2), p_hi_ = f < NQ ? (f + 1) * 7 / NQ : 7 + (f + 1 - NQ) * 9 / (5 * CB / 2);
+      const int p_lo = f < NQ ? f * kUnder / NQ : kUnder + (f - NQ) * (16 - kUnder) / (5 * CB / 2);
+      const int p_hi_ = f < NQ ? (f + 1) * kUnder / NQ : kUnder + (f + 1 - NQ) * (16 - kUnder) / (5 * CB / 2);
 #pragma unroll
       for (int p = p_lo; p < (p_hi_ < 16 ? p_hi_ : 16); ++p) {
         const int i = p >> 2, e = p & 3, x = 4 * i + 2 * (e & 1);
@@ -252,10 +295,17 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
       const int e_lo = f <= NQ ? 0 : (f - NQ - 1) * 16 / (NF - NQ - 1), e_hi = f <= NQ ? 0 : (f - NQ) * 16 / (NF - NQ - 1);
 #pragma unroll
       for (int e = e_lo; e < e_hi; ++e) {
+        if (Rule != kAnyRule) bend(next, e, d0);
+        if (Rule != kAnyRule) mx = top_of(next, mx, e);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (Rule == kAnyRule) {                           // (in the slots it takes the loop past what the compiler unrolls)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
         bend(next, e, d0);
         mx = top_of(next, mx, e);
       }
-      __builtin_amdgcn_sched_barrier(0);
     }
     asm volatile("" : "+v"(mx), "+v"(l));
     if (t + 1 < t_hi) settle(t + 1, next, mx);
@@ -266,29 +316,36 @@ __global__ __launch_bounds__(256, 2) void row_pipe_kernel(hymeta_sink_attention_
   if (t_lo < t_hi) {
     refill(t_lo);
     copy_tile(t_lo, false, s_k[0]);
+    if (Wide) load_queries();                         // (32 KB a wave, which the first keys don't wait for)
     copies_landed_barrier();
     copy_tile(t_lo, true, s_v[0]);
     if (t_lo + 1 < t_hi) copy_tile(t_lo + 1, false, s_k[1]);
     lead(t_lo, s_k[0], sa);
+    other_image(kat, kOffsets, kKeyImage);
     // tile t: images (t - t_lo) & 1
-    auto iterate = [&](int t, int even, f32x16 (&cur)[2], f32x16 (&next)[2]) __attribute__((always_inline)) {
+    auto iterate = [&](int t, auto image, f32x16 (&cur)[2], f32x16 (&next)[2]) __attribute__((always_inline)) {
+      constexpr int even = decltype(image)::value;
       copies_landed_barrier();                        // keys of t + 1 and values of t are there, and nobody reads the images they leave
       if (t + 2 < t_hi) copy_tile(t + 2, false, s_k[even]);
       if (t + 1 < t_hi) copy_tile(t + 1, true, s_v[1 - even]);
       if (t + 1 < seen_lo || t > seen_hi) {
 #pragma unroll
         for (int i = 0; i < 32; ++i) next[i >> 4][i & 15] = -INFINITY;
-        return;
+      } else {
+        step(t, s_k[1 - even], s_v[even], cur, next);
       }
-      step(t, s_k[1 - even], s_v[even], cur, next);
+      other_image(kat, kOffsets, even ? kKeyImage : -kKeyImage);
+      other_image(vat, CB, even ? -kValueImage : kValueImage);
     };
+    constexpr std::integral_constant<int, 0> first{};
+    constexpr std::integral_constant<int, 1> second{};
     int t = t_lo;
     for (; t + 1 < t_hi; t += 2) {
-      iterate(t, 0, sa, sb);
-      iterate(t + 1, 1, sb, sa);
+      iterate(t, first, sa, sb);
+      iterate(t + 1, second, sb, sa);
       if (((t - t_lo) & 31) == 30) refill(t + 2);
     }
-    if (t < t_hi) iterate(t, 0, sa, sb);
+    if (t < t_hi) iterate(t, first, sa, sb);
   }
   l += __shfl_xor(l, 32, 64);
   if (!ok) return;
