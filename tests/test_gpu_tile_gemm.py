@@ -151,3 +151,39 @@ def test_w8a8_linear_of_a_prompt(M, N, K, gated):
         out = hip_ops.w8a8_gemm(x, w, ws, bias=bias)
         ref = (sums + bias.double()).float().to(torch.bfloat16)
     assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("M,N,K,slices,bias,pitch", [
+    (257, 3584, 18944, 9, False, 18944),      # a last row tile of one row
+    (512, 256, 24704, 16, True, 24720),       # the most slices, of 24 and 25 steps; x in rows of a wider tensor
+    (1025, 3584, 7232, 3, True, 7232),        # slices of 37 and 38 steps, a die's tiles from two of them
+    (2048, 1024, 12352, 8, False, 12352),
+    (2048, 3584, 14336, 2, False, 14336),     # two slices: K of four times the weight rows
+])
+def test_a_product_cut_along_k(M, N, K, slices, bias, pitch):
+    from vllm_hymeta import hip_ops
+    from vllm_hymeta.linear import HymetaLinear
+    g = gen(11)
+    x, w = _ints(g, -3, 3, M, pitch).bfloat16().cuda()[:, :K], _ints(g, -2, 2, N, K).bfloat16().cuda()
+    b = _ints(g, -9, 9, N).bfloat16().cuda() if bias else None
+    sums = hip_ops.bf16_gemm_sliced(x, w, b)
+    assert sums.desc.splits == slices
+    ref = x.float() @ w.float().t()           # sums below 2^24: exact in any order
+    want = (ref if b is None else ref + b.float()).bfloat16()
+    assert torch.equal(sums.tensor(), want)
+    layer = HymetaLinear.from_weight(w, b)
+    assert torch.equal(layer(x), want)
+    residual, weight = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda"), torch.ones(N, dtype=torch.bfloat16, device="cuda")
+    deferred = layer(x, defer=True)
+    assert isinstance(deferred, hip_ops.PartialSums)
+    hip_ops.add_rmsnorm(deferred, weight, residual=residual)
+    assert torch.equal(residual, want)
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 3584, 18944), (300, 3584, 3584), (2048, 3584, 9472), (300, 3520, 18944), (300, 3584, 18976), (4096, 3584, 18944)])
+def test_products_that_are_not_cut(M, N, K):
+    from vllm_hymeta import hip_ops
+    x, w = torch.ones(M, K, dtype=torch.bfloat16, device="cuda"), torch.zeros(N, K, dtype=torch.bfloat16, device="cuda")
+    assert hip_ops.bf16_gemm_sliced(x, w) is None
+    if M > 256 and K % 64 == 0:
+        assert hip_ops.bf16_gemm_sliced(x[:, : K - 64], w[:, : K - 64]) is None      # weight rows that are not next to each other

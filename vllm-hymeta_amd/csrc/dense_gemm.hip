@@ -178,8 +178,16 @@ static bool gated_tiles(int32_t M, int32_t K, int32_t N) {
   return tiles > 512 && tiles <= 2048 && tile_gemm_fits(gated_tile_args(M, K, N));
 }
 
+// A product whose K is cut (tile_gemm_slices has the rule and what it measured).
+static TileGemmArgs sliced_args(int32_t M, int32_t K, int32_t N, int64_t x_stride) {
+  TileGemmArgs t = {};
+  t.x_stride = x_stride * 2, t.out_stride = 8, t.a_rows_div = 1, t.max_rows = M, t.N = N, t.k_bytes = K * 2;
+  return t;
+}
+
 extern "C" int hymeta_bf16_gemm_takes(int32_t M, int32_t K, int32_t N, int32_t form) {
   if (M <= 0 || K <= 0 || N <= 0 || K % 32 != 0 || N % kCols != 0 || K > (1 << 28)) return 0;
+  if (form == 3) return M > 256 && tile_gemm_slices(sliced_args(M, K, N, K)) > 1 ? 1 : 0;
   if (M > 256) return form == 1 && gated_tiles(M, K, N) ? 1 : 0;
   StreamPlan plan;
   if (form == 1) return stream_gemm_plan_gated(M, K * 2, N, &plan) ? 1 : 0;
@@ -251,6 +259,27 @@ extern "C" int hymeta_bf16_gemm_deferred(const hymeta_bf16_gemm_args* args, hyme
                                          hymeta_stream_t stream) {
   if (!hymeta::args_ok(partials)) return HYMETA_ERR_INVALID_ARG;
   return bf16_gemm_impl(args, stream, partials);
+}
+
+extern "C" int hymeta_bf16_gemm_sliced(const hymeta_bf16_gemm_args* args, hymeta_gemm_partials* partials, hymeta_stream_t stream) {
+  using namespace hymeta;
+  if (!hymeta::args_ok(args) || !hymeta::args_ok(partials)) return HYMETA_ERR_INVALID_ARG;
+  const hymeta_bf16_gemm_args& a = *args;
+  *partials = hymeta::make_args<hymeta_gemm_partials>();
+  if (a.M < 0 || a.K <= 0 || a.N <= 0 || a.K > (1 << 28)) return HYMETA_ERR_INVALID_ARG;
+  if (a.M == 0) return HYMETA_OK;
+  TileGemmArgs t = sliced_args(a.M, a.K, a.N, a.x_stride_m);
+  t.x = static_cast<const char*>(a.x), t.w = static_cast<const char*>(a.weight);
+  t.slices = tile_gemm_slices(t);
+  if (a.M <= 256 || a.w_stride_n != a.K || t.slices == 1) return HYMETA_ERR_UNSUPPORTED;
+  if (!a.x || !a.weight) return HYMETA_ERR_INVALID_ARG;
+  if ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.weight) | reinterpret_cast<uintptr_t>(a.bias) | reinterpret_cast<uintptr_t>(a.workspace)) % 16 != 0)
+    return HYMETA_ERR_UNSUPPORTED;
+  if (a.workspace == nullptr || a.workspace_bytes < static_cast<size_t>(t.slices) * a.M * a.N * sizeof(float)) return HYMETA_ERR_WORKSPACE;
+  partials->splits = t.slices, partials->M = a.M, partials->N = a.N, partials->bias = a.bias, partials->slabs = a.workspace;
+  t.slabs = static_cast<float*>(a.workspace);
+  tile_gemm_launch(t, false, begin_launches(stream));
+  return launch_status();
 }
 
 // fp32 result of bf16 operands, unrounded: the logits of a bf16 lm_head.  The streaming kernel without K slices only.

@@ -21,12 +21,16 @@ struct TileGemmArgs {
   int32_t a_rows_div, max_rows, N, k_bytes, expert_begin, expert_end;
   int32_t act;                      // HYMETA_GEMM_ACT_*: out has N / 2 columns, weight rows are gate rows, then up rows
   float act_limit, act_alpha;
+  float* slabs;                     // slices > 1 (bf16): the sums of K's slices, [slices][max_rows][N], instead of out
+  int32_t slices;
   uint32_t a_rows_inv;              // the launch's: 2^32 / a_rows_div, rounded up
 };
 
 // Whether the tiles take the problem: whole steps of 128 bytes, whole 16-byte stores, 32-bit offsets into x and an expert's
 // weights, as many experts as a wave has lanes.  (Alignment of the pointers to 16 bytes is the caller's to check.)
 bool tile_gemm_fits(const TileGemmArgs& a);
+// Slices that K is cut into where one bf16 matrix has so few tiles that they leave the chip idle; 1: none.  At most 64 MiB of sums.
+int tile_gemm_slices(const TileGemmArgs& a);
 void tile_gemm_launch(const TileGemmArgs& a, bool int8, hipStream_t s);
 
 }  // namespace hymeta

@@ -19,6 +19,8 @@
 //  * neighbours share the fetching of what comes from beyond their L2: each touches every 8th step of its x panel and every
 //    deep-th of its w panel, ahead of the copies, as loads whose 4 bytes a line go to a scrap of LDS (1790 -> 1610 us;
 //    all lines by all workgroups: 1880).
+// One matrix of so few tiles that they leave the chip idle is cut along K instead (tile_gemm_slices): every unit takes a slice of
+// one tile, whose fp32 sums a reducing consumer adds.
 // Workgroups that walk their tiles as one stream of steps, the next one's copies ahead of the present one's sums, were built:
 // 2 % slower in bf16 and level in int8 on 8192 rows, 6 % slower on 2048 rows of 8 experts (what is done once a tile costs every step,
 // and nobody evens out tiles of few rows).
@@ -27,6 +29,7 @@
 #include "act_types.h"
 #include "lds_copy.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace hymeta {
@@ -41,6 +44,7 @@ constexpr int kMaxTileExperts = 64;              // a lane each
 constexpr int kHalfRows = 128;                   // tiles of at most these rows take half the products
 constexpr int kAhead = 3;                        // steps between a touched line and its products
 constexpr int kMinSteps = 4;
+constexpr int kMaxSlices = 16, kSliceSteps = 24;   // tile_gemm_slice_plan
 
 // f(0), f(1) .. f(N - 1) with the numbers as constants
 template <int N, int I = 0, typename F>
@@ -83,6 +87,7 @@ __device__ __forceinline__ void copy4(const char* base, uint32_t offset, uint32_
 struct Place {
   int e, row, rows, col;
   int deep, depth;
+  int slice, step0, steps;          // the steps of K it takes: all, or those of a slice
 };
 
 // The tiles of all experts stand in one order, a lane per expert.  An expert's tiles go in blocks of up to kDeep row tiles x
@@ -135,7 +140,22 @@ __device__ __forceinline__ bool find_place(const TileGemmArgs& a, int lane, Plac
   p->e = a.expert_offsets != nullptr ? a.expert_begin + at : 0;
   p->row = lo + (row0 + p->deep) * kTile + (half > 0 ? kHalfRows : 0);
   p->rows = min(half >= 0 ? kHalfRows : kTile, hi - p->row);
+  p->slice = 0, p->step0 = 0, p->steps = a.k_bytes / kStep;
   return p->rows > 0;
+}
+
+// One matrix cut along K, a slice's tiles stand next to each other, the row tiles of a column first, and
+// a die takes an eighth of the row: about one slice, whose x its L2 then reads once and whose weights no other die asks for.
+__device__ __forceinline__ bool find_slice(const TileGemmArgs& a, Place* p) {
+  const int row_tiles = (a.max_rows + kTile - 1) / kTile, tiles = row_tiles * (a.N / kTile), total = tiles * a.slices;
+  const int block = blockIdx.x, die = block % kDies, first = total * die / kDies, count = total * (die + 1) / kDies - first, j = block / kDies;
+  if (j >= count) return false;
+  const int all = a.k_bytes / kStep, in = (first + j) % tiles;
+  p->slice = (first + j) / tiles;
+  p->step0 = all * p->slice / a.slices, p->steps = all * (p->slice + 1) / a.slices - p->step0;
+  p->deep = in % row_tiles, p->depth = row_tiles, p->col = in / row_tiles;
+  p->e = 0, p->row = p->deep * kTile, p->rows = min(kTile, a.max_rows - p->row);
+  return true;
 }
 
 __device__ __forceinline__ int divided(const TileGemmArgs& a, int r) {
@@ -148,7 +168,8 @@ struct TileTables {
   uint16_t bias[kTile];
 };
 
-template <int Act> constexpr bool kGatedAct = Act != HYMETA_GEMM_ACT_NONE;
+constexpr int kSums = -1;                        // in an activation's place: the sums themselves, a slice's into its slab
+template <int Act> constexpr bool kGatedAct = Act != HYMETA_GEMM_ACT_NONE && Act != kSums;
 
 template <int Act>
 __device__ __forceinline__ float apply_act(const TileGemmArgs& a, float gate, float up) {
@@ -176,7 +197,8 @@ __device__ __forceinline__ void tile_body(const TileGemmArgs& a, const Place& p,
   const int tid = threadIdx.x, lane = tid & 63, c = lane >> 4, n = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  const int steps = a.k_bytes / kStep;
+  const int steps = p.steps;
+  const char* const xb = a.x + static_cast<int64_t>(p.step0) * kStep;
 
   // A copy of a wave brings 8 rows x 128 bytes; a row's 16-byte chunks lie XOR-ed with (row / 2) % 8, which with the pitch of
   // 128 bytes spreads the sixteen rows of a fragment read over all banks.  Rows past the end re-read the last row.
@@ -190,10 +212,10 @@ __device__ __forceinline__ void tile_body(const TileGemmArgs& a, const Place& p,
     xo[j] = static_cast<uint32_t>(source(32 * j + 8 * wave + l3)) * static_cast<uint32_t>(a.x_stride) + 16 * (swizzled ^ (wave & 1 ? 4 : 0));
   const uint32_t touch_x = static_cast<uint32_t>(source(tid)) * static_cast<uint32_t>(a.x_stride), touch_w = static_cast<uint32_t>(lane) * a.k_bytes;
   const int64_t weight_row = Gated ? static_cast<int64_t>(wave & 1) * (a.N / 2) + p.col * (kTile / 2) + 64 * (wave >> 1) : p.col * kTile + 64 * wave;
-  const char* const wb = a.w + static_cast<int64_t>(p.e) * a.w_stride_e + weight_row * a.k_bytes;
+  const char* const wb = a.w + static_cast<int64_t>(p.e) * a.w_stride_e + weight_row * a.k_bytes + static_cast<int64_t>(p.step0) * kStep;
   auto copy1 = [&](int step, int j, int image) {             // x and w by turns while both last
     if (j < 2 * XC && j % 2 == 0) {
-      copy16(a.x + step * kStep, xo[j / 2], lds + image + 1024 * (4 * (j / 2) + wave));
+      copy16(xb + step * kStep, xo[j / 2], lds + image + 1024 * (4 * (j / 2) + wave));
     } else {
       const int i = j < 2 * XC ? j / 2 : j - XC;
       copy16(wb + step * kStep + static_cast<int64_t>(8 * i) * a.k_bytes, wo[i & 1], lds + image + kImage + 1024 * (8 * wave + i));
@@ -251,7 +273,7 @@ __device__ __forceinline__ void tile_body(const TileGemmArgs& a, const Place& p,
           copy1(h == 1 ? fresh : coming, (h == 1 ? 0 : kEarly) + k / kCopyEvery, h == 1 ? image : other);
         }
         if constexpr (h == 1 && k == kProducts / 4 + 1) {
-          if (it == touch_x_at) copy4(a.x + ahead * kStep, touch_x, scrap), touch_x_at += kWide;
+          if (it == touch_x_at) copy4(xb + ahead * kStep, touch_x, scrap), touch_x_at += kWide;
         }
         if constexpr (h == 1 && k == kProducts / 2 + 1) {
           if (it == touch_w_at) copy4(wb + ahead * kStep, touch_w, scrap), touch_w_at += p.depth;
@@ -265,6 +287,18 @@ __device__ __forceinline__ void tile_body(const TileGemmArgs& a, const Place& p,
   }
   copies_landed_barrier();
 
+  if constexpr (Act == kSums) {
+    acc_t* out = reinterpret_cast<acc_t*>(a.slabs) + ((static_cast<int64_t>(p.slice) * a.max_rows + p.row) * a.N + p.col * kTile + 128 * wn + 4 * c) / 4;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int row = 16 * (MI * wm + i) + n;
+      if (row < p.rows) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) out[static_cast<int64_t>(row) * (a.N / 4) + 4 * j] = acc[i][j];
+      }
+    }
+    return;
+  }
   // acc[i][j][r] = C[row 16 (MI wm + i) + n][tile column 128 wn + 16 j + 4 c + r].  Scales on the sums, one rounding, an
   // activation over the rounded pairs; lanes trade with the next 16 so that each stores 16 bytes of a row.
   const bool scaled = a.row_scale != nullptr, biased = !Gated && a.bias != nullptr;
@@ -316,7 +350,7 @@ template <bool I8, int Act>
 __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(TileGemmArgs a) {
   __shared__ __attribute__((aligned(16))) char sm[4 * kImage + sizeof(TileTables) + 256];
   Place p;
-  if (!find_place(a, threadIdx.x & 63, &p)) return;
+  if (Act == kSums ? !find_slice(a, &p) : !find_place(a, threadIdx.x & 63, &p)) return;
   if (p.rows > kHalfRows) tile_body<I8, Act, 8>(a, p, sm);
   else tile_body<I8, Act, 4>(a, p, sm);
 }
@@ -333,8 +367,29 @@ bool tile_gemm_fits(const TileGemmArgs& a) {
          (a.expert_offsets == nullptr || a.expert_end - a.expert_begin <= kMaxTileExperts) && row_tiles * (a.N / kTile) < (int64_t{1} << 26);
 }
 
+// The partial sums go to memory and back: 9 slices of 512 x 3584 are 66 MB, 25 of 83 us.  Bf16, the product and a residual norm that
+// adds its slices, us against the library's product and the norm, weight rows x K and rows (slices, steps of a slice):
+//   3584 x 18944: 300 rows 110 -> 74 (9, 32), 512 205 -> 88, 768 189 -> 106 (6, 49), 1024 202 -> 133, 1536 290 -> 183, 2048 382 -> 242 (2, 148)
+//   3584 x 9472: 300 49 -> 48 (9, 16), 640 66 -> 62 (6, 24), 1024 91 -> 81 (4, 37), 1536 116 -> 104, 2048 137 -> 133 (2, 74)
+//   8192 x 28672: 300 239 -> 190 (4, 112), 512 323 -> 227, 640 277 -> 315 (2, 224), 1024 389 -> 382
+//   8192 x 7168: 512 81 -> 78 (4, 28), 1024 122 -> 122 (2, 56); 3584 x 3584: 300 38 -> 35 (7, 8), 1024 43 -> 49 (4, 14)
+// so: deep and narrow, 24 steps of a slice or more, two slices only where the matrix is deep enough that the library does not fill the
+// chip.  Tiles of 128 rows: 4 % to 14 % slower on the first, 7 % to 11 % faster on the second up to 512 rows.
+int tile_gemm_slices(const TileGemmArgs& a) {
+  if (a.expert_offsets != nullptr || a.a_rows != nullptr || a.act != HYMETA_GEMM_ACT_NONE || !tile_gemm_fits(a)) return 1;
+  const int64_t tiles = static_cast<int64_t>((a.max_rows + kTile - 1) / kTile) * (a.N / kTile), k = a.k_bytes / 2;
+  const int slices = static_cast<int>(std::min<int64_t>(kDies * kUnits / tiles, kMaxSlices));
+  return slices > 1 && a.k_bytes / kStep / slices >= kSliceSteps && k >= (slices == 2 ? 4 : 2) * static_cast<int64_t>(a.N) ? slices : 1;
+}
+
 void tile_gemm_launch(const TileGemmArgs& args, bool int8, hipStream_t s) {
   TileGemmArgs a = args;
+  if (a.slices > 1) {
+    const int total = (a.max_rows + kTile - 1) / kTile * (a.N / kTile) * a.slices;
+    const dim3 all((total + kDies - 1) / kDies * kDies);
+    hipLaunchKernelGGL((tile_gemm_kernel<false, kSums>), all, dim3(256), 0, s, a);
+    return;
+  }
   if (a.a_rows != nullptr) a.a_rows_inv = a.a_rows_div > 1 ? static_cast<uint32_t>((uint64_t{1} << 32) / a.a_rows_div + 1) : 0;
   // the host knows the rows, not how the experts share them; and the halves of a last round
   const int64_t row_tiles = (a.max_rows + kTile - 1) / kTile + (a.expert_offsets != nullptr ? a.expert_end - a.expert_begin : 0);

@@ -980,6 +980,33 @@ def bf16_gemm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor
     return out
 
 
+_SLICED_BYTES = 64 << 20        # the most a sliced product's partial sums take: one size, so that the buffer never grows
+
+
+def bf16_gemm_sliced(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> Optional[PartialSums]:
+    """``PartialSums`` of x bf16 [M, K] @ weight bf16 [N, K]^T (+ bias bf16 [N]) cut along K: prompts of more rows than
+    ``bf16_gemm`` takes through deep, narrow matrices whose tiles would leave the chip idle.  None: not such a product."""
+    N, K = weight.shape
+    if not (x.dim() == 2 and x.shape[0] > BF16_GEMM_TALL_ROWS and K >= 2 * N and x.is_cuda and x.dtype == torch.bfloat16
+            and weight.dtype == torch.bfloat16 and x.shape[1] == K and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and 2 * x.shape[0] * x.stride(0) < 1 << 32 and weight.is_contiguous() and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+            and (x.data_ptr() | weight.data_ptr()) % 16 == 0):
+        return None
+    if bias is not None and not (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
+        return None
+    lib = _C.load()
+    if not lib.hymeta_bf16_gemm_takes(x.shape[0], K, N, 3):
+        return None
+    _dev(x, weight, bias)
+    a, desc = _C.Bf16GemmArgs(), _C.GemmPartials()
+    a.x, a.weight, a.bias, a.M, a.K, a.N = _p(x), _p(weight), _p(bias), x.shape[0], K, N
+    a.x_stride_m, a.w_stride_n = x.stride(0), weight.stride(0)
+    ws = _workspace(x.device, _SLICED_BYTES, "bf16_gemm_sliced")
+    a.workspace, a.workspace_bytes = _p(ws), _SLICED_BYTES
+    _C.check(lib.hymeta_bf16_gemm_sliced(C.byref(a), C.byref(desc), _stream(x)), "hymeta_bf16_gemm_sliced")
+    return _partials(desc, x.shape[0], N, x.device, "bf16_gemm_sliced", bias)
+
+
 def logits_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Shapes ``bf16_logits`` takes (any number of rows: they go 64 at a time)."""
     return (x.dim() == 2 and x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.is_cuda

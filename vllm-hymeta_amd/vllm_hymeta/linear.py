@@ -92,9 +92,16 @@ class HymetaLinear(torch.nn.Module):
         return hip_ops.gptq_dequant(self.qweight, self.qzeros, self.scales, self.meta["bits"], self.meta["group_size"],
                                     zero_offset=self.meta.get("zero_offset", 1), transposed=transposed)
 
+    def _prompt(self, x: torch.Tensor, weight: torch.Tensor, defer: bool):
+        """Prompts: deep, narrow matrices cut along K where their tiles would leave the chip idle, else a plain library GEMM."""
+        y = hip_ops.bf16_gemm_sliced(x, weight, self.bias)
+        if y is None:
+            return torch.nn.functional.linear(x, weight, self.bias)
+        return y if defer else y.tensor()
+
     def forward(self, x: torch.Tensor, defer: bool = False):
         """``defer``: the caller passes the result straight to a fused add + RMS norm (``HymetaRMSNorm`` with a
-        residual); a decode-sized bf16 / W8A8 linear whose K is cut into slices then returns their
+        residual); a bf16 / W8A8 linear whose K is cut into slices then returns their
         ``hip_ops.PartialSums`` and the norm adds them as it reads its input.  Everything else returns the tensor."""
         if self.kind == "bf16":
             # decode-sized batches: the weight-streaming kernel; prefill-sized ones: a plain library GEMM
@@ -111,7 +118,7 @@ class HymetaLinear(torch.nn.Module):
                 hip_ops.bf16_gemm(x[:half], self.weight, self.bias, out=out[:half])
                 hip_ops.bf16_gemm(x[half:], self.weight, self.bias, out=out[half:])
                 return out
-            return torch.nn.functional.linear(x, self.weight, self.bias)
+            return self._prompt(x, self.weight, defer)
         if self.kind == "gptq":
             if x.shape[0] > GPTQ_EXPAND_ROWS:
                 # prefill regime: expand the weights once, plain library bf16 GEMM on them -- as W^T [N, K] where the
@@ -119,7 +126,7 @@ class HymetaLinear(torch.nn.Module):
                 nk = hip_ops.gptq_dequant_nk_supported(self.qweight, self.meta["bits"])
                 w = self._expanded(nk)
                 if nk:
-                    return torch.nn.functional.linear(x, w, self.bias)
+                    return self._prompt(x, w, defer)
                 y = torch.matmul(x, w)
                 return y if self.bias is None else y.add_(self.bias)
             return hip_ops.gptq_gemm(x, self.qweight, self.qzeros, self.scales, self.meta["bits"],
