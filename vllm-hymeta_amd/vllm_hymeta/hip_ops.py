@@ -1251,7 +1251,7 @@ class GptqExperts(NamedTuple):
 # Rows per local expert (on average) up to which GPTQ experts run the fused de-quantising grouped GEMM; above, the local
 # experts are expanded to bf16 once per call and the tiled bf16 grouped GEMM runs on the expansion (the fused kernel
 # re-reads an expert's weights per 32-row tile).  Measured on the 70B TP=4 shapes (16 experts, us per block, fused /
-# expanded): 1024 tokens 466 / 796, 2048: 777 / 943, 4096: 1373 / 1164, 8192: 2569 / 1557.
+# expanded): 1024 tokens 466 / 796, 2048: 777 / 943, 4096: 1373 / 1041, 8192: 2569 / 1303.
 MOE_GPTQ_FUSED_ROWS_PER_EXPERT = int(os.environ.get("HYMETA_MOE_GPTQ_FUSED_ROWS", "160"))
 
 

@@ -104,7 +104,7 @@ class HymetaLinear(torch.nn.Module):
         residual); a bf16 / W8A8 linear whose K is cut into slices then returns their
         ``hip_ops.PartialSums`` and the norm adds them as it reads its input.  Everything else returns the tensor."""
         if self.kind == "bf16":
-            # decode-sized batches: the weight-streaming kernel; prefill-sized ones: a plain library GEMM
+            # decode-sized batches: the weight-streaming kernel; prefill-sized ones: _prompt
             if hip_ops.bf16_gemm_supported(x, self.weight):
                 return hip_ops.bf16_gemm(x, self.weight, self.bias, defer=defer)
             M, (N, K) = x.shape[0], self.weight.shape
@@ -121,7 +121,7 @@ class HymetaLinear(torch.nn.Module):
             return self._prompt(x, self.weight, defer)
         if self.kind == "gptq":
             if x.shape[0] > GPTQ_EXPAND_ROWS:
-                # prefill regime: expand the weights once, plain library bf16 GEMM on them -- as W^T [N, K] where the
+                # prefill regime: expand the weights once, a bf16 product on them -- as W^T [N, K] where the
                 # expansion kernel's tiles cover the matrix, the layout the library runs 12 % faster at 32768 rows
                 nk = hip_ops.gptq_dequant_nk_supported(self.qweight, self.meta["bits"])
                 w = self._expanded(nk)
