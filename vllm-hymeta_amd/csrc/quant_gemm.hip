@@ -284,8 +284,12 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
 // emits); a wave owns 32 rows x 64 columns of one chunk, software-pipelines its k-steps by hand
 // (operands of step t + 1 are fetched and de-quantised while the matrix cores work on step t) and
 // keeps its weights eight k-steps ahead in registers; the K halves meet in LDS at the end.
+// Neither issue nor memory bounds it alone: vector instructions 55 % of a wave's cycles, the matrix pipe 21 %, waits 35 %, and with
+// the weights in the last-level cache it gains 7 %.  What stands behind the last whole round of tiles weighs most (NI = 5).  A wave of
+// 64 rows x 32 columns, a third fewer vector instructions and twice the LDS reads, is 6 % slower.
 // ---------------------------------------------------------------------------------------------
-constexpr int kWideCols = 128;
+constexpr int kWideCols = 128, kWideCols5 = 160;
+constexpr int kTailQuarters = 3;
 constexpr int kWideThreads = 512;
 constexpr int kChunkK = 128;                    // k per staged activation chunk = 4 MFMA k-steps
 constexpr int kXPitch = kChunkK * 2 + 16;       // bytes per LDS row: 16 rows x 16 B hit 64 distinct banks
@@ -306,14 +310,19 @@ __device__ __forceinline__ void static_for(F&& f) {
 //           w, w + wgs, ... of the first full_rounds * wgs tiles, and the `left` tiles that remain
 //           are cut into left_slices K slices each, one per workgroup, so that the last round costs
 //           1 / left_slices of a tile instead of a whole one; their slabs are compact:
-//           [left tile][slice][64][128].
+//           [left tile][slice][64][128].  Tiles of 160 columns: left_slices = 1, whole tiles.
 struct WidePlan {
   int mode, tiles_n, splits, cps, wgs, full_rounds, left, left_slices, left_cps;
 };
 
-template <int BITS, int KSTEPS>
+// NI: 16-column fragments of a wave.  4: 64 columns, 4n .. 4n + 3 a lane.  5 (4-bit, whole K only): 16 more behind them, one a lane;
+// columns past the matrix re-read its last ones and are not written.
+template <int BITS, int KSTEPS, int NI>
 __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gptq_gemm_args a, WidePlan plan,
                                                                       float* slabs, int* counters) {
+  static_assert(NI == 4 || (NI == 5 && BITS == 4), "a quad of columns a lane, or a quad and one");
+  constexpr bool kExtra = NI == 5;
+  constexpr int kCols = 32 * NI;                  // of the tile
   __shared__ __attribute__((aligned(16))) char smem[2 * 2 * kXBuf];   // [buffer][K half][row][pitch]
   const int njobs = plan.mode == 0 ? 1 : plan.full_rounds + (static_cast<int>(blockIdx.x) < plan.left * plan.left_slices ? 1 : 0);
   for (int job = 0; job < njobs; ++job) {
@@ -331,11 +340,11 @@ __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gpt
   }
   const int nb = tile % plan.tiles_n, mb = tile / plan.tiles_n;
   if (plan.mode == 0) {
-    sbase = slabs + static_cast<int64_t>(mb) * 64 * a.N + nb * kWideCols;
+    sbase = slabs + static_cast<int64_t>(mb) * 64 * a.N + nb * kCols;
     s_split_stride = static_cast<int64_t>(a.M) * a.N, s_row_stride = a.N;
   } else {
-    sbase = slabs + static_cast<int64_t>(tile - plan.wgs * plan.full_rounds) * plan.left_slices * (64 * kWideCols);
-    s_split_stride = 64 * kWideCols, s_row_stride = kWideCols;
+    sbase = slabs + static_cast<int64_t>(tile - plan.wgs * plan.full_rounds) * plan.left_slices * (64 * kCols);
+    s_split_stride = 64 * kCols, s_row_stride = kCols;
   }
   const bool active = split < splits;          // a slice past the end of K (mode 1, uneven cut) has nothing to do
   if (job > 0) __syncthreads();                // the previous tile's last LDS reads
@@ -351,18 +360,19 @@ __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gpt
   const int ch_lo = split * cps;
   const int ch_hi = min(a.K / kChunkK, ch_lo + cps);
   const int nch = ch_hi - ch_lo;                  // >= 1
-  const int lcol0 = wc * 64 + 4 * n;              // column inside the tile
-  const int col0 = nb * kWideCols + lcol0;
+  const int lcol0 = wc * 16 * NI + 4 * n;         // column inside the tile
+  const int own0 = nb * kCols + lcol0, own1 = nb * kCols + wc * 16 * NI + 64 + n;
+  const int col0 = kExtra ? min(own0, a.N - 4) : own0, col1 = min(own1, a.N - 1);
   constexpr int PACK = 32 / BITS;
   constexpr int QL = BITS == 4 ? 1 : 2;
   constexpr int GPC = 4 / KSTEPS;                 // groups per chunk
-  constexpr int kRing = 8;                        // weight k-steps in flight
+  constexpr int kRing = kExtra ? 4 : 8;           // weight k-steps in flight (five fragments leave registers for four)
 
-  f32x4 acc_tot[2][4];
+  f32x4 acc_tot[2][NI];
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc_tot[mt][i] = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < NI; ++i) acc_tot[mt][i] = {0.f, 0.f, 0.f, 0.f};
   const u32x4 ones_raw = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
   const bf16x8 ones = as_frag(ones_raw);
 
@@ -406,22 +416,30 @@ __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gpt
   const int nrounds = (nch + 1) / 2;
   const int last_step = 4 * nrounds - 1;
   u32x4 qring[kRing][QL];
+  uint32_t qextra[kRing] = {};
   u32x2 sraw[2][GPC];
   uint32_t zraw[2][GPC];
-  auto load_w = [&](int t, u32x4 (&q)[QL]) {
+  uint16_t sextra[2][GPC];
+  uint32_t zextra[2][GPC];
+  auto load_w = [&](int t, u32x4 (&q)[QL], uint32_t& extra) {
     const int tt = min(t, last_step);
     const int k = (ch_lo + min(2 * (tt >> 2) + kh, nch - 1)) * kChunkK + 32 * (tt & 3) + 8 * c;
     const int32_t* qp = a.qweight + static_cast<int64_t>(k / PACK) * a.N + col0;
 #pragma unroll
     for (int i = 0; i < QL; ++i) q[i] = ld16g(qp + static_cast<int64_t>(i) * a.N);
+    if (kExtra) extra = *(const __attribute__((address_space(1))) uint32_t*)(qp + (col1 - col0));
   };
-  auto load_params = [&](int ci, u32x2 (&sr)[GPC], uint32_t (&zr)[GPC]) {
+  auto load_params = [&](int ci, u32x2 (&sr)[GPC], uint32_t (&zr)[GPC], uint16_t (&se)[GPC], uint32_t (&ze)[GPC]) {
     const int g0 = (ch_lo + min(2 * min(ci, nrounds - 1) + kh, nch - 1)) * GPC;
 #pragma unroll
     for (int gq = 0; gq < GPC; ++gq) {
       const int64_t g = g0 + gq;
       sr[gq] = *(const __attribute__((address_space(1))) u32x2*)(reinterpret_cast<const uint16_t*>(a.scales) + g * a.N + col0);
       zr[gq] = *(const __attribute__((address_space(1))) uint32_t*)(a.qzeros + g * (a.N / PACK) + col0 / PACK);
+      if (kExtra) {
+        se[gq] = *(const __attribute__((address_space(1))) uint16_t*)(reinterpret_cast<const uint16_t*>(a.scales) + g * a.N + col1);
+        ze[gq] = *(const __attribute__((address_space(1))) uint32_t*)(a.qzeros + g * (a.N / PACK) + col1 / PACK);
+      }
     }
   };
 
@@ -429,27 +447,27 @@ __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gpt
   // cores work on set t & 1, the same wave reads the next A fragments from LDS, turns the next
   // packed weights into set (t + 1) & 1 and refills their ring slot.  One barrier per chunk,
   // ahead of the MFMAs of the chunk's last step.
-  u32x4 bq[2][4];
+  u32x4 bq[2][NI];
   bf16x8 af[2][2];
-  f32x4 acc_g[2][4], acc_x[2];
+  f32x4 acc_g[2][NI], acc_x[2];
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt) {
     acc_x[mt] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc_g[mt][i] = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < NI; ++i) acc_g[mt][i] = {0.f, 0.f, 0.f, 0.f};
   }
   // (q >> 4w) & 0x000F000F | 0x43004300 as shift + v_and_or_b32: the mask rides in an SGPR and the
   // exponent pattern in a VGPR (two 32-bit constants do not fit one instruction, and left to
   // itself the compiler spends three instructions per word).
   uint32_t exp_pattern = 0x43004300u;
   asm volatile("" : "+v"(exp_pattern));
-  auto dequant = [&](const u32x4 (&q)[QL], u32x4 (&b)[4]) {
+  auto dequant = [&](const u32x4 (&q)[QL], uint32_t extra, u32x4 (&b)[NI]) {
     if constexpr (BITS == 4) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < NI; ++i)
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-          const uint32_t sh = w == 0 ? q[0][i] : q[0][i] >> (4 * w);
+          const uint32_t word = i < 4 ? q[0][i & 3] : extra, sh = w == 0 ? word : word >> (4 * w);
           asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(b[i][w]) : "v"(sh), "s"(0x000F000Fu), "v"(exp_pattern));
         }
     } else {
@@ -474,18 +492,18 @@ __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gpt
     for (int mt = 0; mt < 2; ++mt)
       f[mt] = as_frag(*reinterpret_cast<const u32x4*>(smem + buf * 2 * kXBuf + afrag_off + 16 * mt * kXPitch + 64 * step));
   };
-  // Half-dequantisation: B fragments i0, i0 + 1 of the four.
-  auto dequant2 = [&](const u32x4 (&q)[QL], u32x4 (&b)[4], int i0) {
-    u32x4 full[4];
-    dequant(q, full);
-    b[i0] = full[i0];
-    b[i0 + 1] = full[i0 + 1];
+  // Half of it: B fragments from i0 on, two or (the last) three.
+  auto dequant2 = [&](const u32x4 (&q)[QL], uint32_t extra, u32x4 (&b)[NI], int i0) {
+    u32x4 full[NI];
+    dequant(q, extra, full);
+#pragma unroll
+    for (int i = i0; i < (i0 == 0 ? 2 : NI); ++i) b[i] = full[i];
   };
   // Scalar FMAs on purpose: beside MFMAs a packed fp32 FMA costs several times its issue slot.
-  float pend_sc[4] = {0.f, 0.f, 0.f, 0.f}, pend_nzs[4] = {0.f, 0.f, 0.f, 0.f};   // s and -s * (c + z)
+  float pend_sc[NI] = {}, pend_nzs[NI] = {};   // s and -s * (c + z)
   auto epilogue = [&](int mt) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         float t = acc_tot[mt][i][r];
@@ -521,28 +539,28 @@ __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gpt
       } else {
         read_af(PAR, S + 1, af[SP ^ 1]);
       }
-      if constexpr (S == 0) load_params(ci + 1, sraw[PAR ^ 1], zraw[PAR ^ 1]);
-      load_w(4 * ci + S + kRing, qring[slot]);
+      if constexpr (S == 0) load_params(ci + 1, sraw[PAR ^ 1], zraw[PAR ^ 1], sextra[PAR ^ 1], zextra[PAR ^ 1]);
+      load_w(4 * ci + S + kRing, qring[slot], qextra[slot]);
       if constexpr (kFirst) epilogue(1);              // the previous group's row tile 1, before its sums are overwritten
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc_g[0][i] = mfma16(af[SP][0], as_frag(bq[SP][i]), kFirst ? zero : acc_g[0][i]);
+      for (int i = 0; i < NI; ++i) acc_g[0][i] = mfma16(af[SP][0], as_frag(bq[SP][i]), kFirst ? zero : acc_g[0][i]);
       acc_x[0] = mfma16(af[SP][0], ones, kFirst ? zero : acc_x[0]);
-      dequant2(qring[nslot], bq[SP ^ 1], 0);
+      dequant2(qring[nslot], qextra[nslot], bq[SP ^ 1], 0);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc_g[1][i] = mfma16(af[SP][1], as_frag(bq[SP][i]), kFirst ? zero : acc_g[1][i]);
+      for (int i = 0; i < NI; ++i) acc_g[1][i] = mfma16(af[SP][1], as_frag(bq[SP][i]), kFirst ? zero : acc_g[1][i]);
       acc_x[1] = mfma16(af[SP][1], ones, kFirst ? zero : acc_x[1]);
-      dequant2(qring[nslot], bq[SP ^ 1], 2);
+      dequant2(qring[nslot], qextra[nslot], bq[SP ^ 1], 2);
       if constexpr (kLast) {
         // s * (sum x (c + q) - (c + z) * sum x); zero scale for a padding chunk
         const uint32_t zw = zraw[PAR][GQ];
         const int first = col0 % PACK;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint16_t raw = static_cast<uint16_t>(sraw[PAR][GQ][i >> 1] >> (16 * (i & 1)));
+        for (int i = 0; i < NI; ++i) {
+          const uint16_t raw = i < 4 ? static_cast<uint16_t>(sraw[PAR][GQ][(i & 3) >> 1] >> (16 * (i & 1))) : sextra[PAR][GQ];
           const float sv = a.scales_dtype == HYMETA_F16 ? static_cast<float>(__builtin_bit_cast(_Float16, raw)) : bf2f(raw);
           const float scl = real ? sv : 0.f;
-          const uint32_t z = (zw >> (BITS * (first + i))) & ((1u << BITS) - 1u);
+          const uint32_t z = (i < 4 ? zw >> (BITS * (first + i)) : zextra[PAR][GQ] >> (BITS * (col1 % PACK))) & ((1u << BITS) - 1u);
           const float zf = static_cast<float>(z + a.zero_offset) + (BITS == 4 ? 128.f : 0.f);
           pend_sc[i] = scl;
           pend_nzs[i] = -scl * zf;
@@ -555,13 +573,13 @@ __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gpt
 
   load_x(0, xs);
 #pragma unroll
-  for (int p = 0; p < kRing; ++p) load_w(p, qring[p]);
-  load_params(0, sraw[0], zraw[0]);
+  for (int p = 0; p < kRing; ++p) load_w(p, qring[p], qextra[p]);
+  load_params(0, sraw[0], zraw[0], sextra[0], zextra[0]);
   write_x(0, xs);
   load_x(1, xs);
   __syncthreads();
   read_af(0, 0, af[0]);
-  dequant(qring[0], bq[0]);
+  dequant(qring[0], qextra[0], bq[0]);
   for (int ci = 0; ci < nrounds; ci += 2) {
     do_chunk(ci, std::integral_constant<int, 0>{});
     if (ci + 1 < nrounds) do_chunk(ci + 1, std::integral_constant<int, 1>{});
@@ -574,8 +592,8 @@ __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gpt
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<f32x4*>(smem + (((mt * 4 + i) * 4 + (wave & 3)) * 64 + lane) * 16) = acc_tot[mt][i];
+      for (int i = 0; i < NI; ++i)
+        *reinterpret_cast<f32x4*>(smem + (((mt * NI + i) * 4 + (wave & 3)) * 64 + lane) * 16) = acc_tot[mt][i];
   }
   __syncthreads();
   const bool owner = kh == 0;
@@ -584,12 +602,12 @@ __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gpt
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        acc_tot[mt][i] += *reinterpret_cast<const f32x4*>(smem + (((mt * 4 + i) * 4 + (wave & 3)) * 64 + lane) * 16);
+      for (int i = 0; i < NI; ++i)
+        acc_tot[mt][i] += *reinterpret_cast<const f32x4*>(smem + (((mt * NI + i) * 4 + (wave & 3)) * 64 + lane) * 16);
   }
 
   // ---- acc_tot[mt][i][r] = C[m0 + 32 wr + 16 mt + 4c + r][col0 + i]: 16 lanes x 4 columns per row
-  if (splits > 1) {
+  if (!kExtra && splits > 1) {
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
@@ -633,6 +651,7 @@ __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gpt
     const u32x2 bw = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(a.bias) + col0);
     bias = f32x4{lo_bf(bw[0]), hi_bf(bw[0]), lo_bf(bw[1]), hi_bf(bw[1])};
   }
+  const float bias1 = kExtra && a.bias != nullptr ? bf2f(static_cast<const uint16_t*>(a.bias)[col1]) : 0.f;
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
@@ -641,7 +660,9 @@ __global__ __launch_bounds__(kWideThreads) void gptq_gemm_wide_kernel(hymeta_gpt
       if (grow >= a.M) continue;
       const u32x2 o = {pack_bf16x2(acc_tot[mt][0][r] + bias[0], acc_tot[mt][1][r] + bias[1]),
                        pack_bf16x2(acc_tot[mt][2][r] + bias[2], acc_tot[mt][3][r] + bias[3])};
-      *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(a.out) + static_cast<int64_t>(grow) * a.out_stride_m + col0) = o;
+      uint16_t* row = reinterpret_cast<uint16_t*>(a.out) + static_cast<int64_t>(grow) * a.out_stride_m;
+      if (!kExtra || own0 < a.N) *reinterpret_cast<u32x2*>(row + col0) = o;
+      if (kExtra && own1 < a.N) row[col1] = static_cast<uint16_t>(pack_bf16x2(acc_tot[mt][NI - 1][r] + bias1, 0.f));
     }
   }
   }   // active
@@ -1225,13 +1246,31 @@ static int gptq_gemm_impl(const hymeta_gptq_gemm_args* args, hymeta_stream_t str
       }
     }
   }
+  // ... or tiles of 160 columns, where their whole rounds are cheaper: a cut remainder costs its share of a round and, for the second
+  // prologue, the slabs, the ticket and the last arriver's sums one after the other, about three quarters of one (3584 x 32768 at 64
+  // rows, 256 tiles, 29 us; 37888, 296, 47).  128 -> 160 columns, us, K = 3584: 37888 at 33 / 64 / 128 rows 41.6 -> 31.7 / 43.6 -> 32.5 /
+  // 67.7 -> 62.7; 33024 at 64 41.4 -> 37.2; 40960 at 64 45.9 -> 34.4; 18944 at 128 42.4 -> 32.5.  By one quarter: 33024 at 96 63.9 -> 66.4.
+  bool five = false;
+  if (plan.mode == 1 && a.bits == 4) {
+    const int tiles_n = (a.N + kWideCols5 - 1) / kWideCols5, rounds = (tiles_n * ((a.M + 63) / 64) + plan.wgs - 1) / plan.wgs;
+    const int four = 4 * plan.full_rounds + (plan.left == 0 ? 0 : plan.left_slices > 1 ? 4 / plan.left_slices + kTailQuarters : 4);
+    five = 5 * rounds + 1 < four;
+    if (five) {
+      const int tiles = tiles_n * ((a.M + 63) / 64);
+      plan.tiles_n = tiles_n, plan.full_rounds = tiles / plan.wgs, plan.left = tiles % plan.wgs, plan.left_slices = plan.left > 0 ? 1 : 0, plan.left_cps = units;
+    }
+  }
   hipStream_t s = begin_launches(stream);
   int* counters = reinterpret_cast<int*>(a.workspace);
   float* slabs = a.workspace == nullptr ? nullptr : reinterpret_cast<float*>(reinterpret_cast<char*>(a.workspace) + counter_bytes);
   if (wide) {
     dim3 grid(plan.tiles_n * ((a.M + 63) / 64), splits), block(kWideThreads);
     if (plan.mode == 1) grid = dim3(plan.wgs);
-#define HYMETA_LAUNCH_WIDE(B, KS) hipLaunchKernelGGL((gptq_gemm_wide_kernel<B, KS>), grid, block, 0, s, a, plan, slabs, counters)
+#define HYMETA_LAUNCH_WIDE(B, KS)                                                                                        \
+  do {                                                                                                                   \
+    if (B == 4 && five) hipLaunchKernelGGL((gptq_gemm_wide_kernel<4, KS, 5>), grid, block, 0, s, a, plan, slabs, counters); \
+    else hipLaunchKernelGGL((gptq_gemm_wide_kernel<B, KS, 4>), grid, block, 0, s, a, plan, slabs, counters);             \
+  } while (0)
 #define HYMETA_LAUNCH_WIDE_KS(B)                     \
   do {                                               \
     if (a.group_size == 128) HYMETA_LAUNCH_WIDE(B, 4); \
