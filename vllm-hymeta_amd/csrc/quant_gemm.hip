@@ -46,14 +46,19 @@ constexpr int kColsPerBlock = 64;  // output columns per workgroup: lane n owns 
 
 }  // namespace
 
-// grid = (N / 64, ceil(M / (16 MT)), splits); 256 threads: the 4 waves take alternate groups of
+// grid = (N / (16 NI) rounded up, ceil(M / (16 MT)), splits); 256 threads: the 4 waves take alternate groups of
 // the workgroup's K slice; each wave's (group, k-step) sequence is software-pipelined one step
 // deep (next step's packed weights and activation fragments are in flight during the MFMAs).
-template <int BITS, int MT, int KSTEPS>
+// NI: 16-column fragments.  4: 64 columns, 4n .. 4n + 3 a lane.  5 (4-bit, whole K only): 16 more behind them, one a lane; columns
+// past the matrix re-read its last ones and are not written.
+template <int BITS, int MT, int KSTEPS, int NI>
 __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a, int splits, int groups_per_split,
                                                         float* slabs, int* counters) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  float* s_red = reinterpret_cast<float*>(smem_raw);  // [4 waves][16 MT rows][64 cols]
+  float* s_red = reinterpret_cast<float*>(smem_raw);  // [4 waves][16 MT rows][16 NI cols]
+  static_assert(NI == 4 || (NI == 5 && BITS == 4), "a quad of columns a lane, or a quad and one");
+  constexpr bool kExtra = NI == 5;
+  constexpr int kCols = 16 * NI;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -65,15 +70,16 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
   const int G = a.K / a.group_size;
   const int g_lo = split * groups_per_split;
   const int g_hi = min(G, g_lo + groups_per_split);
-  const int col0 = nb * kColsPerBlock + 4 * n;   // this lane's first output column
+  // this lane's first output column, and (kExtra) its fifth
+  const int col0 = kExtra ? min(nb * kCols + 4 * n, a.N - 4) : nb * kCols + 4 * n, col1 = min(nb * kCols + 64 + n, a.N - 1);
   constexpr int PACK = 32 / BITS;
   constexpr int QL = BITS == 4 ? 1 : 2;          // 16-byte weight loads per k-step
 
-  f32x4 acc_tot[MT][4];
+  f32x4 acc_tot[MT][NI];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc_tot[mt][i] = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < NI; ++i) acc_tot[mt][i] = {0.f, 0.f, 0.f, 0.f};
 
   const u32x4 ones_raw = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
   const bf16x8 ones = as_frag(ones_raw);
@@ -100,36 +106,45 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
   u32x4 qring[kWDepth][QL], xring[kXDepth][MT];
   u32x2 sraw[2];     // 4 scales (16-bit) of the lane's columns
   uint32_t zraw[2];  // packed zeros word holding the lane's columns
+  uint32_t qextra[kWDepth] = {}, zextra[2];
+  uint16_t sextra[2];
   auto step_k0 = [&](int t) {
     const int g = first_g + 4 * (t / KSTEPS);
     return g * a.group_size + 32 * (t % KSTEPS);   // + 8c inside the pointers
   };
-  auto load_w = [&](int t, u32x4 (&q)[QL]) {
+  auto load_w = [&](int t, u32x4 (&q)[QL], uint32_t& extra) {
     const int32_t* qp = a.qweight + static_cast<int64_t>((step_k0(min(t, last_step)) + 8 * c) / PACK) * a.N + col0;
 #pragma unroll
     for (int i = 0; i < QL; ++i) q[i] = ld16(qp + static_cast<int64_t>(i) * a.N);
+    if (kExtra) extra = static_cast<uint32_t>(qp[col1 - col0]);
   };
   auto load_x = [&](int t, u32x4 (&x)[MT]) {
     const int k0 = step_k0(min(t, last_step));
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) x[mt] = ld16(xrow[mt] + k0);
   };
-  auto load_params = [&](int gi, u32x2& sr, uint32_t& zr) {
+  auto load_params = [&](int gi, u32x2& sr, uint32_t& zr, uint16_t& se, uint32_t& ze) {
     const int g = first_g + 4 * min(gi, ng - 1);
     sr = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(a.scales) + static_cast<int64_t>(g) * a.N + col0);
     zr = static_cast<uint32_t>(a.qzeros[static_cast<int64_t>(g) * (a.N / PACK) + col0 / PACK]);
+    if (kExtra) {
+      se = reinterpret_cast<const uint16_t*>(a.scales)[static_cast<int64_t>(g) * a.N + col1];
+      ze = static_cast<uint32_t>(a.qzeros[static_cast<int64_t>(g) * (a.N / PACK) + col1 / PACK]);
+    }
   };
 
+  uint32_t exp_pattern = 0x43004300u;            // (one instruction with the mask in a scalar register, see gptq_gemm_wide_kernel)
+  asm volatile("" : "+v"(exp_pattern));
   auto do_group = [&](int gi, auto parity) {
     constexpr int PAR = decltype(parity)::value;
-    load_params(gi + 1, sraw[PAR ^ 1], zraw[PAR ^ 1]);
+    load_params(gi + 1, sraw[PAR ^ 1], zraw[PAR ^ 1], sextra[PAR ^ 1], zextra[PAR ^ 1]);
     __builtin_amdgcn_sched_barrier(0);
-    f32x4 acc_g[MT][4], acc_x[MT];
+    f32x4 acc_g[MT][NI], acc_x[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       acc_x[mt] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc_g[mt][i] = {0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < NI; ++i) acc_g[mt][i] = {0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
@@ -139,12 +154,15 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
       const int wslot = PAR * KSTEPS + ks;
       const int xslot = wslot % kXDepth;
       // ---- weights: 8 k-values x 4 columns per lane
-      u32x4 bq[4];
+      u32x4 bq[NI];
       if constexpr (BITS == 4) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < NI; ++i)
 #pragma unroll
-          for (int w = 0; w < 4; ++w) bq[i][w] = ((qring[wslot][0][i] >> (4 * w)) & 0x000F000Fu) | 0x43004300u;
+          for (int w = 0; w < 4; ++w) {
+            const uint32_t word = i < 4 ? qring[wslot][0][i & 3] : qextra[wslot], sh = w == 0 ? word : word >> (4 * w);
+            asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(bq[i][w]) : "v"(sh), "s"(0x000F000Fu), "v"(exp_pattern));
+          }
       } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -161,7 +179,7 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
           }
         }
       }
-      load_w(t + kWDepth, qring[wslot]);
+      load_w(t + kWDepth, qring[wslot], qextra[wslot]);
       __builtin_amdgcn_sched_barrier(0);   // keep the refill here: the scheduler would sink it to its use
       // ---- activations: 16 rows x 8 k per m-tile
       bf16x8 af[MT];
@@ -184,7 +202,7 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc_g[mt][i] = mfma16(af[mt], as_frag(bq[i]), acc_g[mt][i]);
+        for (int i = 0; i < NI; ++i) acc_g[mt][i] = mfma16(af[mt], as_frag(bq[i]), acc_g[mt][i]);
         acc_x[mt] = mfma16(af[mt], ones, acc_x[mt]);
       }
     }
@@ -192,19 +210,19 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
     const bool real = gi < ng;
     const uint32_t zw = zraw[PAR];
     const int first = col0 % PACK;
-    float sc[4], zf[4];
+    float sc[NI], zf[NI];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint16_t raw = static_cast<uint16_t>(sraw[PAR][i >> 1] >> (16 * (i & 1)));
+    for (int i = 0; i < NI; ++i) {
+      const uint16_t raw = i < 4 ? static_cast<uint16_t>(sraw[PAR][(i & 3) >> 1] >> (16 * (i & 1))) : sextra[PAR];
       const float sv = a.scales_dtype == HYMETA_F16 ? static_cast<float>(__builtin_bit_cast(_Float16, raw)) : bf2f(raw);
       sc[i] = real ? sv : 0.f;
-      const uint32_t z = (zw >> (BITS * (first + i))) & ((1u << BITS) - 1u);
+      const uint32_t z = (i < 4 ? zw >> (BITS * (first + i)) : zextra[PAR] >> (BITS * (col1 % PACK))) & ((1u << BITS) - 1u);
       zf[i] = static_cast<float>(z + a.zero_offset) + (BITS == 4 ? 128.f : 0.f);
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < NI; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           acc_tot[mt][i][r] += sc[i] * (acc_g[mt][i][r] - zf[i] * acc_x[mt][r]);
@@ -212,10 +230,10 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
 
   if (ng > 0) {
 #pragma unroll
-    for (int p = 0; p < kWDepth; ++p) load_w(p, qring[p]);
+    for (int p = 0; p < kWDepth; ++p) load_w(p, qring[p], qextra[p]);
 #pragma unroll
     for (int p = 0; p < kXDepth; ++p) load_x(p, xring[p]);
-    load_params(0, sraw[0], zraw[0]);
+    load_params(0, sraw[0], zraw[0], sextra[0], zextra[0]);
     for (int gi = 0; gi < ngp; gi += 2) {
       do_group(gi, std::integral_constant<int, 0>{});
       do_group(gi + 1, std::integral_constant<int, 1>{});
@@ -227,22 +245,28 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      float* p = s_red + (static_cast<size_t>(wave) * 16 * MT + 16 * mt + 4 * c + r) * kColsPerBlock + 4 * n;
+      float* p = s_red + (static_cast<size_t>(wave) * 16 * MT + 16 * mt + 4 * c + r) * kCols + 4 * n;
       *reinterpret_cast<f32x4*>(p) = f32x4{acc_tot[mt][0][r], acc_tot[mt][1][r], acc_tot[mt][2][r], acc_tot[mt][3][r]};
+      if (kExtra) p[64 - 3 * n] = acc_tot[mt][NI - 1][r];
     }
   __syncthreads();
   const int cg = tid & 15;          // 4 columns per thread
-  const int col = nb * kColsPerBlock + 4 * cg;
+  const int col = nb * kCols + 4 * cg, fifth = nb * kCols + 64 + cg;
   f32x4 sum[MT];
+  float extra[MT];
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
     const int row = (tid >> 4) + 16 * j;
     sum[j] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < 4; ++w)
-      sum[j] += *reinterpret_cast<const f32x4*>(s_red + (static_cast<size_t>(w) * 16 * MT + row) * kColsPerBlock + 4 * cg);
+      sum[j] += *reinterpret_cast<const f32x4*>(s_red + (static_cast<size_t>(w) * 16 * MT + row) * kCols + 4 * cg);
+    extra[j] = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      if (kExtra) extra[j] += s_red[(static_cast<size_t>(w) * 16 * MT + row) * kCols + 64 + cg];
   }
-  if (splits > 1) {
+  if (!kExtra && splits > 1) {
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
       const int grow = m0 + (tid >> 4) + 16 * j;
@@ -259,7 +283,7 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
     }
   }
   f32x4 bias = {0.f, 0.f, 0.f, 0.f};
-  if (a.bias != nullptr) {
+  if (a.bias != nullptr && (!kExtra || col < a.N)) {
     const u32x2 bw = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(a.bias) + col);
     bias = f32x4{lo_bf(bw[0]), hi_bf(bw[0]), lo_bf(bw[1]), hi_bf(bw[1])};
   }
@@ -269,7 +293,10 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
     if (grow >= a.M) continue;
     const f32x4 y = sum[j] + bias;
     const u32x2 o = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
-    *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(a.out) + static_cast<int64_t>(grow) * a.out_stride_m + col) = o;
+    uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + static_cast<int64_t>(grow) * a.out_stride_m;
+    if (!kExtra || col < a.N) *reinterpret_cast<u32x2*>(out + col) = o;
+    if (kExtra && fifth < a.N)
+      out[fifth] = static_cast<uint16_t>(pack_bf16x2(extra[j] + (a.bias != nullptr ? bf2f(static_cast<const uint16_t*>(a.bias)[fifth]) : 0.f), 0.f));
   }
 }
 
@@ -288,7 +315,7 @@ __global__ __launch_bounds__(256) void gptq_gemm_kernel(hymeta_gptq_gemm_args a,
 // the weights in the last-level cache it gains 7 %.  What stands behind the last whole round of tiles weighs most (NI = 5).  A wave of
 // 64 rows x 32 columns, a third fewer vector instructions and twice the LDS reads, is 6 % slower.
 // ---------------------------------------------------------------------------------------------
-constexpr int kWideCols = 128, kWideCols5 = 160;
+constexpr int kWideCols = 128, kWideCols5 = 160, kCols5 = 80;
 constexpr int kTailQuarters = 3;
 constexpr int kWideThreads = 512;
 constexpr int kChunkK = 128;                    // k per staged activation chunk = 4 MFMA k-steps
@@ -1284,9 +1311,21 @@ static int gptq_gemm_impl(const hymeta_gptq_gemm_args* args, hymeta_stream_t str
   }
   const int mt = mt_for(a.M);
   dim3 grid(a.N / kColsPerBlock, (a.M + 16 * mt - 1) / (16 * mt), splits), block(256);
-  const size_t lds = static_cast<size_t>(4) * 16 * mt * kColsPerBlock * sizeof(float);
-#define HYMETA_LAUNCH_GPTQ(B, T, KS) \
-  hipLaunchKernelGGL((gptq_gemm_kernel<B, T, KS>), grid, block, lds, s, a, splits, gps, slabs, counters)
+  size_t lds = static_cast<size_t>(4) * 16 * mt * kColsPerBlock * sizeof(float);
+  // Up to 16 rows, whole K: workgroups of 80 columns where the fullest compute unit has two of them, as many as its registers hold at
+  // once, in place of three or more of 64.  64 -> 80 columns (and one instruction less a pair of weights), us, K = 3584: 37888 at 1 / 8 / 16 rows
+  // 21.2 -> 19.5 / 22.9 -> 20.9 / 27.4 -> 23.2.  18944, one in place of two: 15.9 -> 16.1; 57344, three of 80: 28.3 -> 28.7 at one row.
+  bool five80 = false;
+  if (a.bits == 4 && mt == 1 && splits == 1 && grid.y == 1) {
+    const int wgs = compute_units(), four = (a.N / kColsPerBlock + wgs - 1) / wgs, five = ((a.N + kCols5 - 1) / kCols5 + wgs - 1) / wgs;
+    five80 = five == 2 && 5 * five < 4 * four;
+    if (five80) grid.x = (a.N + kCols5 - 1) / kCols5, lds = static_cast<size_t>(4) * 16 * kCols5 * sizeof(float);
+  }
+#define HYMETA_LAUNCH_GPTQ(B, T, KS)                                                                                                  \
+  do {                                                                                                                                \
+    if (B == 4 && T == 1 && five80) hipLaunchKernelGGL((gptq_gemm_kernel<4, 1, KS, 5>), grid, block, lds, s, a, splits, gps, slabs, counters); \
+    else hipLaunchKernelGGL((gptq_gemm_kernel<B, T, KS, 4>), grid, block, lds, s, a, splits, gps, slabs, counters);                 \
+  } while (0)
 #define HYMETA_LAUNCH_GPTQ_KS(B, T)                   \
   do {                                                \
     if (a.group_size == 128) HYMETA_LAUNCH_GPTQ(B, T, 4); \
