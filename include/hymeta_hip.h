@@ -750,6 +750,9 @@ int hymeta_advance_step(int32_t num_seqs, int32_t num_queries, int32_t block_siz
  * more rows likewise (513 to 2048 tiles of 256 x 256; then w_stride_n == K, and x within 4 GiB);
  * other shapes are HYMETA_ERR_UNSUPPORTED: run the two calls. */
 int hymeta_bf16_gemm_silu_mul(const hymeta_bf16_gemm_args* args, hymeta_stream_t stream);
+/* The same for more than 256 rows with the activation of hymeta_activation's HYMETA_ACT_SILU_MUL in place of hymeta_silu_and_mul's
+ * (they differ in how exactly the exponential is formed); fewer rows: HYMETA_ERR_UNSUPPORTED. */
+int hymeta_bf16_gemm_silu_mul_exact(const hymeta_bf16_gemm_args* args, hymeta_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * W8A8 int8 linear: per-output-channel int8 weights, dynamic per-token int8

@@ -127,6 +127,27 @@ def test_gate_up_of_a_prompt(M, N, K):
     assert not hip_ops.gemm_silu_mul_supported(x[:300], w[:8192])
 
 
+@pytest.mark.parametrize("M", [300, 1030, 5000])      # too few tiles, a prompt in tiles, too many
+def test_gated_block_of_a_prompt(M):
+    """The side families' gated block has one activation for prompts of any length: silu_mul of the rounded exact sums (in
+    sixteenths, up to +-24: an exponential formed less exactly gives other bits in some of them)."""
+    from vllm_hymeta import hip_ops
+    from vllm_hymeta.linear import HymetaLinear
+    from vllm_hymeta.models.feed_forward import SiluGluMLP
+    g = gen(13)
+    K, N = 256, 32768
+    x, w = (_ints(g, -3, 3, M, K) / 16).bfloat16().cuda(), _ints(g, -3, 3, N, K).bfloat16().cuda()
+    assert hip_ops.gemm_silu_mul_supported(x, w) == (M == 1030)
+    h = (x.float() @ w.float().t()).bfloat16()
+    want, fast = hip_ops.silu_mul(h), hip_ops.silu_and_mul(h)
+    assert not torch.equal(want, fast)
+    down = HymetaLinear.from_weight(torch.eye(256, N // 2, dtype=torch.bfloat16, device="cuda"))      # the first 256 columns
+    out = SiluGluMLP(HymetaLinear.from_weight(w), down)(x)
+    assert torch.equal(out, want[:, :256])
+    if M == 1030:
+        assert torch.equal(hip_ops.gemm_silu_mul(x, w, exact=True), want) and torch.equal(hip_ops.gemm_silu_mul(x, w), fast)
+
+
 @pytest.mark.parametrize("M,N,K", [(1030, 4608, 512), (300, 16384, 640), (5000, 1024, 1024)])
 @pytest.mark.parametrize("gated", [False, True])
 def test_w8a8_linear_of_a_prompt(M, N, K, gated):

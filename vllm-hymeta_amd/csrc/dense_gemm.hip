@@ -307,7 +307,7 @@ extern "C" int hymeta_bf16_gemm_f32out(const hymeta_bf16_gemm_args* args, hymeta
 // Gate/up projection with the activation in the epilogue: out [M, N / 2] = silu(x gate^T) * (x up^T), weight = [gate rows |
 // up rows].  Only the shapes the streaming kernel takes whole (no K slices); others are HYMETA_ERR_UNSUPPORTED and the
 // caller runs hymeta_bf16_gemm + hymeta_silu_and_mul, which give the same bits.
-extern "C" int hymeta_bf16_gemm_silu_mul(const hymeta_bf16_gemm_args* args, hymeta_stream_t stream) {
+static int gemm_silu_mul(const hymeta_bf16_gemm_args* args, int32_t act, hymeta_stream_t stream) {
   using namespace hymeta;
   if (!hymeta::args_ok(args)) return HYMETA_ERR_INVALID_ARG;
   const hymeta_bf16_gemm_args& a = *args;
@@ -317,11 +317,11 @@ extern "C" int hymeta_bf16_gemm_silu_mul(const hymeta_bf16_gemm_args* args, hyme
   if ((a.x_stride_m | a.w_stride_n | a.out_stride_m) % 8 != 0) return HYMETA_ERR_UNSUPPORTED;
   if ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.weight) | reinterpret_cast<uintptr_t>(a.out)) % 16 != 0)
     return HYMETA_ERR_UNSUPPORTED;
-  if (a.K > (1 << 28)) return HYMETA_ERR_UNSUPPORTED;
+  if (a.K > (1 << 28) || (a.M <= 256 && act != HYMETA_GEMM_ACT_SILU)) return HYMETA_ERR_UNSUPPORTED;
   if (a.M > 256) {
     TileGemmArgs t = gated_tile_args(a.M, a.K, a.N);
     t.x = static_cast<const char*>(a.x), t.w = static_cast<const char*>(a.weight), t.out = static_cast<uint16_t*>(a.out);
-    t.x_stride = a.x_stride_m * 2, t.out_stride = a.out_stride_m;
+    t.x_stride = a.x_stride_m * 2, t.out_stride = a.out_stride_m, t.act = act;
     if (!gated_tiles(a.M, a.K, a.N) || a.w_stride_n != a.K || !tile_gemm_fits(t)) return HYMETA_ERR_UNSUPPORTED;
     tile_gemm_launch(t, false, begin_launches(stream));
     return launch_status();
@@ -334,4 +334,12 @@ extern "C" int hymeta_bf16_gemm_silu_mul(const hymeta_bf16_gemm_args* args, hyme
   sa.M = a.M, sa.N = a.N, sa.k_bytes = a.K * 2, sa.gated = 1;
   sa.x_stride_bytes = a.x_stride_m * 2, sa.w_stride_bytes = a.w_stride_n * 2, sa.out_stride = a.out_stride_m;
   return stream_gemm_launch<false>(sa, plan, begin_launches(stream));
+}
+
+extern "C" int hymeta_bf16_gemm_silu_mul(const hymeta_bf16_gemm_args* args, hymeta_stream_t stream) {
+  return gemm_silu_mul(args, HYMETA_GEMM_ACT_SILU, stream);
+}
+
+extern "C" int hymeta_bf16_gemm_silu_mul_exact(const hymeta_bf16_gemm_args* args, hymeta_stream_t stream) {
+  return gemm_silu_mul(args, HYMETA_GEMM_ACT_SILU_EXACT, stream);
 }

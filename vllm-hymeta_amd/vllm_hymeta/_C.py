@@ -645,6 +645,7 @@ _SIGNATURES = {
     "hymeta_gptq_dequant_nk": (C.c_int, [_ptr, _ptr, _ptr, _ptr, _i32, _i32, _i32, _i32, _i32, _i32, _ptr]),
     "hymeta_bf16_gemm": (C.c_int, [C.POINTER(Bf16GemmArgs), _ptr]),
     "hymeta_bf16_gemm_silu_mul": (C.c_int, [C.POINTER(Bf16GemmArgs), _ptr]),
+    "hymeta_bf16_gemm_silu_mul_exact": (C.c_int, [C.POINTER(Bf16GemmArgs), _ptr]),
     "hymeta_bf16_gemm_f32out": (C.c_int, [C.POINTER(Bf16GemmArgs), _ptr]),
     "hymeta_argmax_rows": (C.c_int, [_ptr, _i64, _i32, _i32, _ptr, _ptr, _sz, _ptr]),
     "hymeta_argmax_rows_workspace_bytes": (_sz, [_i32]),

@@ -1133,12 +1133,13 @@ def gemm_silu_mul_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 
 def gemm_silu_mul(x: torch.Tensor, weight: torch.Tensor, w_scale: Optional[torch.Tensor] = None,
-                  out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                  out: Optional[torch.Tensor] = None, exact: bool = False) -> torch.Tensor:
     """``silu(x gate^T) * (x up^T)`` in one launch: x bf16 [M, K]; weight [2 I, K] bf16 (M <= 128, wide ones to 256, prompts of
     513 to 2048 tiles), or int8 with ``w_scale``
     fp32 [2 I] (dynamic per-token int8 activations; any M) -> bf16 [M, I].  Bit for bit the linear followed by
-    ``silu_and_mul``."""
+    ``silu_and_mul``, or for ``exact`` (bf16 prompts only) by ``silu_mul``."""
     _dev(x, weight, w_scale, out)
+    _require(not exact or (weight.dtype == torch.bfloat16 and x.shape[0] > BF16_GEMM_TALL_ROWS), "the exact activation is for bf16 prompts")
     M, K = x.shape
     N = weight.shape[0]
     _require(gemm_silu_mul_supported(x, weight) and weight.shape == (N, K), "shape not covered: run the linear and silu_and_mul")
@@ -1152,7 +1153,8 @@ def gemm_silu_mul(x: torch.Tensor, weight: torch.Tensor, w_scale: Optional[torch
         a.x, a.weight, a.out = _p(x), _p(weight), _p(out)
         a.M, a.K, a.N = M, K, N
         a.x_stride_m, a.w_stride_n, a.out_stride_m = x.stride(0), weight.stride(0), out.stride(0)
-        _C.check(lib.hymeta_bf16_gemm_silu_mul(C.byref(a), _stream(x)), "hymeta_bf16_gemm_silu_mul")
+        call = lib.hymeta_bf16_gemm_silu_mul_exact if exact else lib.hymeta_bf16_gemm_silu_mul
+        _C.check(call(C.byref(a), _stream(x)), "hymeta_bf16_gemm_silu_mul")
         return out
     _require(w_scale is not None and w_scale.dtype == torch.float32 and w_scale.is_contiguous() and w_scale.numel() == N,
              "w_scale must be contiguous fp32 [2 I]")

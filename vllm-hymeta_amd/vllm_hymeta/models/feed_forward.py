@@ -78,8 +78,9 @@ class SiluGluMLP(torch.nn.Module):
     def forward(self, h: torch.Tensor, defer: bool = False):
         """``defer``: the down projection may leave its slices' sum to the caller (``HymetaLinear.forward``)."""
         gu = self.gate_up_proj
-        if gu.bias is None and hip_ops.gemm_silu_mul_supported(h, gu.weight):      # decode-sized bf16 batches: in the GEMM's epilogue
-            return self.down_proj(hip_ops.gemm_silu_mul(h, gu.weight), defer=defer)
+        # decode-sized bf16 batches and prompts: in the GEMM's epilogue; prompts with silu_mul's own arithmetic, whatever their length
+        if gu.bias is None and hip_ops.gemm_silu_mul_supported(h, gu.weight):
+            return self.down_proj(hip_ops.gemm_silu_mul(h, gu.weight, exact=h.shape[0] > hip_ops.BF16_GEMM_TALL_ROWS), defer=defer)
         return self.down_proj(hip_ops.silu_mul(gu(h)), defer=defer)
 
 
