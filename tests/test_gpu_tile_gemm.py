@@ -201,6 +201,21 @@ def test_a_product_cut_along_k(M, N, K, slices, bias, pitch):
     assert torch.equal(residual, want)
 
 
+def test_a_linear_that_is_more_than_its_kernel():
+    """What torch's linear does beside the product stays: a bias that is broadcast or does not fit.  (Sums of small integers: exact.)"""
+    from vllm_hymeta import hip_ops
+    from vllm_hymeta.linear import HymetaLinear
+    M, N, K = 300, 3584, 18944
+    g = gen(17)
+    x, w = _ints(g, -3, 3, M, K).bfloat16().cuda(), _ints(g, -2, 2, N, K).bfloat16().cuda()
+    ref = x.float() @ w.float().t()
+    assert hip_ops.bf16_gemm_sliced(x, w) is not None
+    one = torch.full((1,), 5.0, dtype=torch.bfloat16, device="cuda")
+    assert torch.equal(HymetaLinear.from_weight(w, one)(x), (ref + 5).bfloat16())
+    with pytest.raises(RuntimeError):
+        HymetaLinear.from_weight(w, torch.zeros(N - 1, dtype=torch.bfloat16, device="cuda"))(x)
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 3584, 18944), (300, 3584, 3584), (2048, 3584, 9472), (300, 3520, 18944), (300, 3584, 18976), (4096, 3584, 18944)])
 def test_products_that_are_not_cut(M, N, K):
     from vllm_hymeta import hip_ops

@@ -992,7 +992,7 @@ def bf16_gemm_sliced(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
             and 2 * x.shape[0] * x.stride(0) < 1 << 32 and weight.is_contiguous() and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
             and (x.data_ptr() | weight.data_ptr()) % 16 == 0):
         return None
-    if bias is not None and not (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
+    if bias is not None and not (bias.shape == (N,) and bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
         return None
     lib = _C.load()
     if not lib.hymeta_bf16_gemm_takes(x.shape[0], K, N, 3):
