@@ -202,7 +202,8 @@ def test_a_product_cut_along_k(M, N, K, slices, bias, pitch):
 
 
 def test_a_linear_that_is_more_than_its_kernel():
-    """What torch's linear does beside the product stays: a bias that is broadcast or does not fit.  (Sums of small integers: exact.)"""
+    """What torch's linear does beside the product stays: a bias that is broadcast or does not fit, gradients of either direction,
+    autocast's type.  (Sums of small integers: exact.)"""
     from vllm_hymeta import hip_ops
     from vllm_hymeta.linear import HymetaLinear
     M, N, K = 300, 3584, 18944
@@ -214,6 +215,15 @@ def test_a_linear_that_is_more_than_its_kernel():
     assert torch.equal(HymetaLinear.from_weight(w, one)(x), (ref + 5).bfloat16())
     with pytest.raises(RuntimeError):
         HymetaLinear.from_weight(w, torch.zeros(N - 1, dtype=torch.bfloat16, device="cuda"))(x)
+    bias = torch.zeros(N, dtype=torch.bfloat16, device="cuda", requires_grad=True)
+    HymetaLinear.from_weight(w, bias)(x).sum().backward()
+    assert torch.equal(bias.grad, torch.full_like(bias, M))
+    layer, ad = HymetaLinear.from_weight(w), torch.autograd.forward_ad
+    with torch.no_grad(), ad.dual_level():
+        y = ad.unpack_dual(layer(ad.make_dual(x, 2 * x)))
+    assert torch.equal(y.primal, ref.bfloat16()) and torch.equal(y.tangent, (2 * ref).bfloat16())
+    with torch.no_grad(), torch.autocast("cuda", torch.float16):
+        assert layer(x).dtype == torch.float16
 
 
 @pytest.mark.parametrize("M,N,K", [(256, 3584, 18944), (300, 3584, 3584), (2048, 3584, 9472), (300, 3520, 18944), (300, 3584, 18976), (4096, 3584, 18944)])

@@ -208,3 +208,32 @@ def test_current_stream_without_torchs_private_name(monkeypatch, index):
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: asked.append(device) or types.SimpleNamespace(cuda_stream=4096))
     device = torch.device("cuda") if index is None else torch.device("cuda", index)
     assert hip_ops._raw_stream(device) == 4096 and asked == [device]
+
+
+def test_what_may_stand_for_a_torch_operation(monkeypatch):
+    """Everything under which a linear is more than its kernel is told apart."""
+    from torch._subclasses import FakeTensorMode
+    from torch.autograd import forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from vllm_hymeta import hip_ops
+    x, seen = torch.randn(4, 8), []
+
+    def look(t):
+        seen.append(hip_ops.plain(t))
+        return t * 2
+
+    assert hip_ops.plain(x, None, torch.nn.Parameter(x, requires_grad=False))
+    asks = torch.nn.Parameter(x.clone())
+    assert not hip_ops.plain(x, asks)
+    with torch.no_grad():
+        assert hip_ops.plain(x, asks)
+        with forward_ad.dual_level():
+            assert hip_ops.plain(x) and not hip_ops.plain(forward_ad.make_dual(x, x))
+        torch.func.vmap(look)(x), torch.func.jvp(look, (x,), (x,)), torch.func.grad(lambda t: look(t).sum())(x)
+        make_fx(look)(x), torch.jit.trace(look, (x,), check_trace=False)
+    assert seen == [False] * 5
+    with FakeTensorMode() as mode:
+        assert not hip_ops.plain(torch.empty(3))
+    assert not hip_ops.plain(mode.from_tensor(x))
+    monkeypatch.setattr(hip_ops, "_wrapped", None)
+    assert not hip_ops.plain(x)

@@ -12,6 +12,7 @@ import os
 from typing import NamedTuple, Optional, Sequence, Tuple
 
 import torch
+from torch.autograd import forward_ad as _forward_ad
 
 from . import _C
 
@@ -55,6 +56,27 @@ def _dev(*ts):
             _require(t.is_cuda, "hymeta ops need HIP device tensors")
             _require(False, "all tensors must live on one device")
     return dev
+
+
+def plain(*ts: Optional[torch.Tensor]) -> bool:
+    """Whether a torch operation on ``ts`` is its kernel and nothing else, so that a kernel of ours may stand for it: no gradient
+    is asked for in either direction, nothing records, transforms or re-types operations (a trace, vmap, a dispatch mode,
+    autocast), and no tensor is a subclass that does."""
+    if (_wrapped is None or _modes is None or torch.jit.is_tracing() or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")
+            or _modes() > 0):
+        return False
+    backward, forward = torch.is_grad_enabled(), getattr(_forward_ad, "_current_level", 0) >= 0
+    for t in ts:
+        if t is not None and (type(t) not in _PLAIN_TYPES or (backward and t.requires_grad) or _wrapped(t)
+                              or (forward and _forward_ad.unpack_dual(t).tangent is not None)):
+            return False
+    return True
+
+
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+# not public names of torch; without them no tensor counts as plain
+_wrapped = getattr(getattr(torch._C, "_functorch", None), "is_functorch_wrapped_tensor", None)      # (vmap's, grad's, jvp's)
+_modes = getattr(torch._C, "_len_torch_dispatch_stack", None)
 
 
 def _inner_contig(t: torch.Tensor, name: str) -> None:
@@ -987,9 +1009,9 @@ def bf16_gemm_sliced(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
     """``PartialSums`` of x bf16 [M, K] @ weight bf16 [N, K]^T (+ bias bf16 [N]) cut along K: prompts of more rows than
     ``bf16_gemm`` takes through deep, narrow matrices whose tiles would leave the chip idle.  None: not such a product."""
     N, K = weight.shape
-    if not (x.dim() == 2 and x.shape[0] > BF16_GEMM_TALL_ROWS and K >= 2 * N and x.is_cuda and x.dtype == torch.bfloat16
+    if not (K >= 2 * N and x.dim() == 2 and x.shape[0] > BF16_GEMM_TALL_ROWS and x.is_cuda and x.dtype == torch.bfloat16
             and weight.dtype == torch.bfloat16 and x.shape[1] == K and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and 2 * x.shape[0] * x.stride(0) < 1 << 32 and weight.is_contiguous() and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+            and 2 * x.shape[0] * x.stride(0) < 1 << 32 and weight.is_contiguous() and plain(x, weight, bias)
             and (x.data_ptr() | weight.data_ptr()) % 16 == 0):
         return None
     if bias is not None and not (bias.shape == (N,) and bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
