@@ -700,7 +700,7 @@ size_t hymeta_bf16_gemm_workspace_bytes(int32_t M, int32_t N, int32_t split_k);
 int hymeta_bf16_gemm(const hymeta_bf16_gemm_args* args, hymeta_stream_t stream);
 /* 1 when the entry point named by `form` -- 0: hymeta_bf16_gemm (split_k 0, workspace of
  * hymeta_bf16_gemm_workspace_bytes(M, N, 0)); 1: hymeta_bf16_gemm_silu_mul (N counts the gate and the up rows);
- * 2: hymeta_bf16_gemm_f32out; 3: hymeta_bf16_gemm_sliced -- takes the shape, 0 when it would answer
+ * 2: hymeta_bf16_gemm_f32out; 3: hymeta_bf16_gemm_sliced; 4: the same where it is worth it with hymeta_gemm_partials_reduce behind it -- takes the shape, 0 when it would answer
  * HYMETA_ERR_UNSUPPORTED and the caller runs a library GEMM: every covered shape up to 128 rows; from 129 to 256
  * rows what the 129..256-row streaming kernel cuts into at least 128 workgroups (tiles of 112 to 160 columns; K
  * slices of at least 512 bytes for narrow matrices).  No counterpart in the reference (its linears are vLLM's):

@@ -201,6 +201,26 @@ def test_a_product_cut_along_k(M, N, K, slices, bias, pitch):
     assert torch.equal(residual, want)
 
 
+@pytest.mark.parametrize("M,N,K,deferred,reduced", [
+    (3072, 1024, 8192, False, False), (1536, 2048, 8192, False, False), (900, 3072, 8192, False, False),      # not deep
+    (2561, 1536, 8960, False, False), (2560, 1536, 8960, True, True),             # rows that leave units idle, of a narrow matrix
+    (1025, 3584, 9472, True, False), (1024, 3584, 9472, True, True),              # ... and of a wider one, where a launch reduces them
+    (1025, 3584, 18944, True, True),                                              # deep enough
+    (3072, 2048, 16384, False, False), (1500, 4096, 16384, False, False),         # two slices of too few tiles or columns
+    (330, 8192, 16384, False, False), (330, 8192, 16448, True, True),             # rows whole 32 KB apart
+    (2048, 1024, 16384, True, True),                                              # few tiles
+])
+def test_products_that_the_library_has_sooner(M, N, K, deferred, reduced):
+    from vllm_hymeta import hip_ops
+    from vllm_hymeta.linear import HymetaLinear
+    x, w = torch.ones(M, K, dtype=torch.bfloat16, device="cuda"), torch.ones(N, K, dtype=torch.bfloat16, device="cuda")
+    assert (hip_ops.bf16_gemm_sliced(x, w) is not None) == deferred
+    assert (hip_ops.bf16_gemm_sliced(x, w, reduced=True) is not None) == reduced
+    layer = HymetaLinear.from_weight(w)
+    assert isinstance(layer(x, defer=True), hip_ops.PartialSums) == deferred
+    assert bool((layer(x) == K).all()) or K % 256 != 0                             # (exact in bf16 where K is)
+
+
 def test_a_linear_that_is_more_than_its_kernel():
     """What torch's linear does beside the product stays: a bias that is broadcast or does not fit, gradients of either direction,
     autocast's type.  (Sums of small integers: exact.)"""

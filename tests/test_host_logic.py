@@ -237,3 +237,13 @@ def test_what_may_stand_for_a_torch_operation(monkeypatch):
     assert not hip_ops.plain(mode.from_tensor(x))
     monkeypatch.setattr(hip_ops, "_wrapped", None)
     assert not hip_ops.plain(x)
+
+
+def test_partial_sums_go_into_the_exchange_only_where_the_message_fits(monkeypatch):
+    """Else a launch reduces them, which the linear has to know beforehand."""
+    from vllm_hymeta import parallel
+    monkeypatch.setattr(parallel, "_active", lambda group: group is not None)
+    monkeypatch.setattr(parallel, "_exchange_of", lambda group: types.SimpleNamespace(max_bytes=4096) if group == "exchange" else None)
+    assert parallel.defers_into_all_reduce("exchange") and parallel.defers_into_all_reduce("exchange", 4096)
+    assert not parallel.defers_into_all_reduce("exchange", 4097)
+    assert not parallel.defers_into_all_reduce("library", 16) and not parallel.defers_into_all_reduce(None, 16)

@@ -187,7 +187,7 @@ static TileGemmArgs sliced_args(int32_t M, int32_t K, int32_t N, int64_t x_strid
 
 extern "C" int hymeta_bf16_gemm_takes(int32_t M, int32_t K, int32_t N, int32_t form) {
   if (M <= 0 || K <= 0 || N <= 0 || K % 32 != 0 || N % kCols != 0 || K > (1 << 28)) return 0;
-  if (form == 3) return M > 256 && tile_gemm_slices(sliced_args(M, K, N, K)) > 1 ? 1 : 0;
+  if (form == 3 || form == 4) return M > 256 && tile_gemm_slices(sliced_args(M, K, N, K), form == 4) > 1 ? 1 : 0;
   if (M > 256) return form == 1 && gated_tiles(M, K, N) ? 1 : 0;
   StreamPlan plan;
   if (form == 1) return stream_gemm_plan_gated(M, K * 2, N, &plan) ? 1 : 0;
@@ -270,7 +270,7 @@ extern "C" int hymeta_bf16_gemm_sliced(const hymeta_bf16_gemm_args* args, hymeta
   if (a.M == 0) return HYMETA_OK;
   TileGemmArgs t = sliced_args(a.M, a.K, a.N, a.x_stride_m);
   t.x = static_cast<const char*>(a.x), t.w = static_cast<const char*>(a.weight);
-  t.slices = tile_gemm_slices(t);
+  t.slices = tile_gemm_slices(t, false);
   if (a.M <= 256 || a.w_stride_n != a.K || t.slices == 1) return HYMETA_ERR_UNSUPPORTED;
   if (!a.x || !a.weight) return HYMETA_ERR_INVALID_ARG;
   if ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.weight) | reinterpret_cast<uintptr_t>(a.bias) | reinterpret_cast<uintptr_t>(a.workspace)) % 16 != 0)

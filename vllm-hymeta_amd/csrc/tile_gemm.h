@@ -30,7 +30,8 @@ struct TileGemmArgs {
 // weights, as many experts as a wave has lanes.  (Alignment of the pointers to 16 bytes is the caller's to check.)
 bool tile_gemm_fits(const TileGemmArgs& a);
 // Slices that K is cut into where one bf16 matrix has so few tiles that they leave the chip idle; 1: none.  At most 64 MiB of sums.
-int tile_gemm_slices(const TileGemmArgs& a);
+// reduced: a launch of its own adds the slices, else the consumer does while it reads them.
+int tile_gemm_slices(const TileGemmArgs& a, bool reduced);
 void tile_gemm_launch(const TileGemmArgs& a, bool int8, hipStream_t s);
 
 }  // namespace hymeta

@@ -44,7 +44,7 @@ constexpr int kMaxTileExperts = 64;              // a lane each
 constexpr int kHalfRows = 128;                   // tiles of at most these rows take half the products
 constexpr int kAhead = 3;                        // steps between a touched line and its products
 constexpr int kMinSteps = 4;
-constexpr int kMaxSlices = 16, kSliceSteps = 24;   // tile_gemm_slice_plan
+constexpr int kMaxSlices = 16, kSliceSteps = 24, kFewSliceTiles = 32, kSliceSums = 14 << 20;      // tile_gemm_slices' rule
 
 // f(0), f(1) .. f(N - 1) with the numbers as constants
 template <int N, int I = 0, typename F>
@@ -367,19 +367,31 @@ bool tile_gemm_fits(const TileGemmArgs& a) {
          (a.expert_offsets == nullptr || a.expert_end - a.expert_begin <= kMaxTileExperts) && row_tiles * (a.N / kTile) < (int64_t{1} << 26);
 }
 
-// The partial sums go to memory and back: 9 slices of 512 x 3584 are 66 MB, 25 of 83 us.  Bf16, the product and a residual norm that
-// adds its slices, us against the library's product and the norm, weight rows x K and rows (slices, steps of a slice):
-//   3584 x 18944: 300 rows 110 -> 74 (9, 32), 512 205 -> 88, 768 189 -> 106 (6, 49), 1024 202 -> 133, 1536 290 -> 183, 2048 382 -> 242 (2, 148)
-//   3584 x 9472: 300 49 -> 48 (9, 16), 640 66 -> 62 (6, 24), 1024 91 -> 81 (4, 37), 1536 116 -> 104, 2048 137 -> 133 (2, 74)
-//   8192 x 28672: 300 239 -> 190 (4, 112), 512 323 -> 227, 640 277 -> 315 (2, 224), 1024 389 -> 382
-//   8192 x 7168: 512 81 -> 78 (4, 28), 1024 122 -> 122 (2, 56); 3584 x 3584: 300 38 -> 35 (7, 8), 1024 43 -> 49 (4, 14)
-// so: deep and narrow, 24 steps of a slice or more, two slices only where the matrix is deep enough that the library does not fill the
-// chip.  Tiles of 128 rows: 4 % to 14 % slower on the first, 7 % to 11 % faster on the second up to 512 rows.
-int tile_gemm_slices(const TileGemmArgs& a) {
+// The partial sums go to memory and back: 9 slices of 512 x 3584 are 66 MB, 25 of 83 us.  Bf16 with weights from memory, the
+// product and a residual norm that adds its slices, us against the library's product and the norm; in brackets with a launch that
+// reduces them; weight rows x K and rows (slices, steps of a slice):
+//   3584 x 18944: 300 rows 104 -> 70 (100 -> 69) (9, 32), 512 201 -> 86, 768 184 -> 103, 1024 194 -> 129, 1536 284 -> 172, 2048 374 -> 238 (2, 148)
+//   3584 x 9472: 513 66 -> 59 (61 -> 56) (6, 24), 768 80 -> 65, 1025 89 -> 86 (82 -> 88) (3, 49), 1536 112 -> 99 (104 -> 96)
+//   8192 x 28672: 300 227 -> 185 (214 -> 180) (4, 112), 512 320 -> 225; 5120 x 13824: 300 83 -> 72 (79 -> 69) (6, 36), 1024 154 -> 132
+//   2048 x 11008: 1280 92 -> 68 (86 -> 66) (6, 28); 1024 x 16384: 2048 103 -> 76 (97 -> 73) (8, 32)
+// Few tiles are cut whatever the matrix.  With more, the library fills the chip by itself on matrices that are not deep (2048 x 8192 at
+// 1536 rows 62 -> 64, reduced 56 -> 62; 3072 x 8192 at 900 63 -> 64), that have few columns, whose sums the norm reads a short row at a time
+// (512 x 9216 at 6000 73 -> 79), where the tiles' last rows or the slices leave units idle and a launch reduces them (the two of
+// 1025 rows above; 1536 x 8960 at 2561 79 -> 82; kSliceSums floats of sums are 7 / 8 of the chip), in two slices that do not fill it or of
+// narrow matrices (2048 x 16384 at 3072 185 -> 189, 4096 x 16384 at 1500 191 -> 193), and where the rows of wide ones lie whole 32 KB apart
+// (8192 x 16384 at 330 rows 121 -> 138, 6144 x 16384 at 513 138 -> 140): those are left to it.  Weights that the last-level cache still holds
+// favour the library by a tenth.  Tiles of 128 rows: 4 % to 14 % slower on 3584 x 18944, 7 % to 11 % faster on 3584 x 9472 up to 512 rows.
+int tile_gemm_slices(const TileGemmArgs& a, bool reduced) {
   if (a.expert_offsets != nullptr || a.a_rows != nullptr || a.act != HYMETA_GEMM_ACT_NONE || !tile_gemm_fits(a)) return 1;
   const int64_t tiles = static_cast<int64_t>((a.max_rows + kTile - 1) / kTile) * (a.N / kTile), k = a.k_bytes / 2;
   const int slices = static_cast<int>(std::min<int64_t>(kDies * kUnits / tiles, kMaxSlices));
-  return slices > 1 && a.k_bytes / kStep / slices >= kSliceSteps && k >= (slices == 2 ? 4 : 2) * static_cast<int64_t>(a.N) ? slices : 1;
+  if (slices < 2 || a.k_bytes / kStep / slices < kSliceSteps || k < 2 * static_cast<int64_t>(a.N)) return 1;
+  if (tiles <= kFewSliceTiles) return slices;
+  const bool deep = k >= 8704, filled = static_cast<int64_t>(a.max_rows) * a.N * slices >= kSliceSums;
+  if (a.N < 1280 || !(deep || (!reduced && a.N >= 3584 && k >= 7168))) return 1;
+  if (!filled && (a.N < 2048 || (reduced && k < 13824))) return 1;
+  if (a.N >= 6144 && k % 16384 == 0) return 1;
+  return slices > 2 || (tiles >= 100 && a.N >= 2560 && k >= 4 * static_cast<int64_t>(a.N)) ? slices : 1;
 }
 
 void tile_gemm_launch(const TileGemmArgs& args, bool int8, hipStream_t s) {

@@ -8,6 +8,7 @@ runs in libhymeta_hip.so.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import os
 from typing import NamedTuple, Optional, Sequence, Tuple
 
@@ -1005,11 +1006,18 @@ def bf16_gemm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor
 _SLICED_BYTES = 64 << 20        # the most a sliced product's partial sums take: one size, so that the buffer never grows
 
 
-def bf16_gemm_sliced(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> Optional[PartialSums]:
+@functools.lru_cache(maxsize=4096)
+def _slices_pay(M: int, K: int, N: int, reduced: bool) -> bool:
+    return bool(_C.load().hymeta_bf16_gemm_takes(M, K, N, 4 if reduced else 3))
+
+
+def bf16_gemm_sliced(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, reduced: bool = False) -> Optional[PartialSums]:
     """``PartialSums`` of x bf16 [M, K] @ weight bf16 [N, K]^T (+ bias bf16 [N]) cut along K: prompts of more rows than
-    ``bf16_gemm`` takes through deep, narrow matrices whose tiles would leave the chip idle.  None: not such a product."""
+    ``bf16_gemm`` takes through deep, narrow matrices whose tiles would leave the chip idle.  None: not such a product.
+    ``reduced``: the caller asks for their ``tensor()`` at once, which pays for fewer shapes than a consumer that adds them."""
     N, K = weight.shape
-    if not (K >= 2 * N and x.dim() == 2 and x.shape[0] > BF16_GEMM_TALL_ROWS and x.is_cuda and x.dtype == torch.bfloat16
+    # (the sizes first: other linears pay nothing for the rest)
+    if not (K >= 2 * N and x.is_cuda and x.dim() == 2 and x.shape[0] > BF16_GEMM_TALL_ROWS and _slices_pay(x.shape[0], K, N, reduced) and x.dtype == torch.bfloat16
             and weight.dtype == torch.bfloat16 and x.shape[1] == K and x.stride(1) == 1 and x.stride(0) % 8 == 0
             and 2 * x.shape[0] * x.stride(0) < 1 << 32 and weight.is_contiguous() and plain(x, weight, bias)
             and (x.data_ptr() | weight.data_ptr()) % 16 == 0):
@@ -1017,8 +1025,6 @@ def bf16_gemm_sliced(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
     if bias is not None and not (bias.shape == (N,) and bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
         return None
     lib = _C.load()
-    if not lib.hymeta_bf16_gemm_takes(x.shape[0], K, N, 3):
-        return None
     _dev(x, weight, bias)
     a, desc = _C.Bf16GemmArgs(), _C.GemmPartials()
     a.x, a.weight, a.bias, a.M, a.K, a.N = _p(x), _p(weight), _p(bias), x.shape[0], K, N

@@ -94,10 +94,12 @@ class HymetaLinear(torch.nn.Module):
 
     def _prompt(self, x: torch.Tensor, weight: torch.Tensor, defer: bool):
         """Prompts: deep, narrow matrices cut along K where their tiles would leave the chip idle, else a plain library GEMM."""
-        y = hip_ops.bf16_gemm_sliced(x, weight, self.bias)
-        if y is None:
-            return torch.nn.functional.linear(x, weight, self.bias)
-        return y if defer else y.tensor()
+        bias = self.bias
+        if weight.shape[1] >= 2 * weight.shape[0]:
+            y = hip_ops.bf16_gemm_sliced(x, weight, bias, reduced=not defer)
+            if y is not None:
+                return y if defer else y.tensor()
+        return torch.nn.functional.linear(x, weight, bias)
 
     def forward(self, x: torch.Tensor, defer: bool = False):
         """``defer``: the caller passes the result straight to a fused add + RMS norm (``HymetaRMSNorm`` with a
@@ -105,20 +107,21 @@ class HymetaLinear(torch.nn.Module):
         ``hip_ops.PartialSums`` and the norm adds them as it reads its input.  Everything else returns the tensor."""
         if self.kind == "bf16":
             # decode-sized batches: the weight-streaming kernel; prefill-sized ones: _prompt
-            if hip_ops.bf16_gemm_supported(x, self.weight):
-                return hip_ops.bf16_gemm(x, self.weight, self.bias, defer=defer)
-            M, (N, K) = x.shape[0], self.weight.shape
+            weight = self.weight                     # (a buffer: every look at it costs half a microsecond)
+            if hip_ops.bf16_gemm_supported(x, weight):
+                return hip_ops.bf16_gemm(x, weight, self.bias, defer=defer)
+            M, (N, K) = x.shape[0], weight.shape
             if (x.dim() == 2 and hip_ops.BF16_GEMM_MAX_ROWS < M <= 2 * hip_ops.BF16_GEMM_MAX_ROWS and K >= 4 * N
-                    and hip_ops.bf16_gemm_supported(x[:hip_ops.BF16_GEMM_MAX_ROWS], self.weight)):
+                    and hip_ops.bf16_gemm_supported(x[:hip_ops.BF16_GEMM_MAX_ROWS], weight)):
                 # deep, narrow matrices (the MLP's down projection) at 129 .. 256 rows: two passes of the streaming kernel
                 # over the two halves of the rows (the second finds most of the weights in the last-level cache) against
                 # a library GEMM that has too few tiles to fill the chip: measured 90 against 126 us at 256 rows
                 out = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
                 half = hip_ops.BF16_GEMM_MAX_ROWS
-                hip_ops.bf16_gemm(x[:half], self.weight, self.bias, out=out[:half])
-                hip_ops.bf16_gemm(x[half:], self.weight, self.bias, out=out[half:])
+                hip_ops.bf16_gemm(x[:half], weight, self.bias, out=out[:half])
+                hip_ops.bf16_gemm(x[half:], weight, self.bias, out=out[half:])
                 return out
-            return self._prompt(x, self.weight, defer)
+            return self._prompt(x, weight, defer)
         if self.kind == "gptq":
             if x.shape[0] > GPTQ_EXPAND_ROWS:
                 # prefill regime: expand the weights once, a bf16 product on them -- as W^T [N, K] where the

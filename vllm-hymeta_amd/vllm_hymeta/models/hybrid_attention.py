@@ -232,6 +232,6 @@ class IntraHybridAttention(torch.nn.Module):
         reduce = parallel._active(self.tp_group)
         # the K slices' sum is left to whoever reads the result next: the fused add + norm (no all-reduce), or the
         # group's one-shot exchange
-        defer = parallel.defers_into_all_reduce(self.tp_group) if reduce else defer_out
+        defer = parallel.defers_into_all_reduce(self.tp_group, 2 * hidden_states.numel()) if reduce else defer_out
         y = self.out_proj(self.combine(out_attn, out_linear), defer=defer)
         return all_reduce_sum(y, self.tp_group) if reduce else y

@@ -41,7 +41,7 @@ class HymetaMLP(torch.nn.Module):
         reduce = self.reduce_results and parallel._active(self.tp_group)
         # the K slices' sum is left to whoever reads the result next: the fused add + norm (no all-reduce), or the
         # group's one-shot exchange
-        defer = parallel.defers_into_all_reduce(self.tp_group) if reduce else defer_out
+        defer = parallel.defers_into_all_reduce(self.tp_group, 2 * x.numel()) if reduce else defer_out
         y = self.down_proj(self.gate_up_proj.forward_silu_mul(x), defer=defer)
         return all_reduce_sum(y, self.tp_group) if reduce else y
 

@@ -417,10 +417,13 @@ def backend_group(group):
     return group
 
 
-def defers_into_all_reduce(group) -> bool:
+def defers_into_all_reduce(group, nbytes: int = 0) -> bool:
     """Whether a row-parallel linear in front of ``all_reduce_sum(…, group)`` may hand over its K slices' partial sums
-    (``defer=True``): the group's one-shot exchange adds them while it reads its message."""
-    return _active(group) and _exchange_of(group) is not None
+    (``defer=True``): the group's one-shot exchange adds them while it reads its message of ``nbytes``."""
+    if not _active(group):
+        return False
+    comm = _exchange_of(group)
+    return comm is not None and nbytes <= comm.max_bytes
 
 
 def all_reduce_sum(x, group: Optional[dist.ProcessGroup] = None) -> torch.Tensor:
