@@ -815,8 +815,9 @@ typedef struct hymeta_gemm_partials {
 
 int hymeta_bf16_gemm_deferred(const hymeta_bf16_gemm_args* args, hymeta_gemm_partials* partials, hymeta_stream_t stream);
 /* The same for prompts of so few tiles that a product of theirs leaves the chip idle: weight rows next to each other, N a multiple
- * of 256, K of 64, more than 256 rows.  workspace: splits x M x N floats, at most 64 MiB.  HYMETA_ERR_UNSUPPORTED: not to be cut (the caller runs a
- * library GEMM).  out, split_k and out_stride_m are unused. */
+ * of 256, K of 64, more than 256 rows.  workspace: splits x M x N floats, at most 64 MiB; _workspace_bytes: that, 0 where the product is
+ * not to be cut.  HYMETA_ERR_UNSUPPORTED: likewise (the caller runs a library GEMM).  out, split_k and out_stride_m are unused. */
+size_t hymeta_bf16_gemm_sliced_workspace_bytes(int32_t M, int32_t K, int32_t N);
 int hymeta_bf16_gemm_sliced(const hymeta_bf16_gemm_args* args, hymeta_gemm_partials* partials, hymeta_stream_t stream);
 int hymeta_w8a8_gemm_deferred(const hymeta_w8a8_gemm_args* args, hymeta_gemm_partials* partials, hymeta_stream_t stream);
 int hymeta_gptq_gemm_deferred(const hymeta_gptq_gemm_args* args, hymeta_gemm_partials* partials, hymeta_stream_t stream);

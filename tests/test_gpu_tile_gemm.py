@@ -221,6 +221,40 @@ def test_products_that_the_library_has_sooner(M, N, K, deferred, reduced):
     assert bool((layer(x) == K).all()) or K % 256 != 0                             # (exact in bf16 where K is)
 
 
+def test_the_slices_memory():
+    """Two prompts' partial sums beside each other, on their own stream and on another one; given back afterwards."""
+    from vllm_hymeta import hip_ops
+    M, N, K = 512, 3584, 18944
+    g = gen(19)
+    x, w = _ints(g, -3, 3, M, K).bfloat16().cuda(), _ints(g, -2, 2, N, K).bfloat16().cuda()
+    want = (x.float() @ w.float().t()).bfloat16()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    one, two = hip_ops.bf16_gemm_sliced(x, w), hip_ops.bf16_gemm_sliced(-x, w)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        first = one.tensor()
+        del one
+    hip_ops.bf16_gemm_sliced(2 * x, w)                     # (does not land in memory that the other stream still reads)
+    torch.cuda.current_stream().wait_stream(side)
+    second = two.tensor()
+    assert torch.equal(first, want) and torch.equal(second, -want)
+    torch.cuda.synchronize()
+    del first, second, two, side
+    again = hip_ops.bf16_gemm_sliced(x, w).tensor()        # (the allocator looks for blocks that other streams are done with)
+    assert torch.equal(again, want)
+    del again
+    assert torch.cuda.memory_allocated() == before
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = hip_ops.bf16_gemm_sliced(x, w).tensor()
+    for sign in (1, -1, 1):
+        x.mul_(sign)
+        graph.replay()
+        assert torch.equal(out, hip_ops.bf16_gemm_sliced(x, w).tensor())
+
+
 def test_a_linear_that_is_more_than_its_kernel():
     """What torch's linear does beside the product stays: a bias that is broadcast or does not fit, gradients of either direction,
     autocast's type.  (Sums of small integers: exact.)"""

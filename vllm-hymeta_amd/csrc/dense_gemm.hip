@@ -261,6 +261,11 @@ extern "C" int hymeta_bf16_gemm_deferred(const hymeta_bf16_gemm_args* args, hyme
   return bf16_gemm_impl(args, stream, partials);
 }
 
+extern "C" size_t hymeta_bf16_gemm_sliced_workspace_bytes(int32_t M, int32_t K, int32_t N) {
+  if (hymeta_bf16_gemm_takes(M, K, N, 3) != 1) return 0;
+  return static_cast<size_t>(tile_gemm_slices(sliced_args(M, K, N, K), false)) * M * N * sizeof(float);
+}
+
 extern "C" int hymeta_bf16_gemm_sliced(const hymeta_bf16_gemm_args* args, hymeta_gemm_partials* partials, hymeta_stream_t stream) {
   using namespace hymeta;
   if (!hymeta::args_ok(args) || !hymeta::args_ok(partials)) return HYMETA_ERR_INVALID_ARG;

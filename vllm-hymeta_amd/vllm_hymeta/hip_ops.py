@@ -438,14 +438,19 @@ class PartialSums:
     """Result of a K-sliced linear whose slice sum is left to its consumer (``bf16_gemm`` / ``w8a8_gemm`` with
     ``defer=True``): ``add_rmsnorm`` takes it in place of ``x`` and adds the slices while it reads them, ``tensor()``
     runs the linear's own reduce launch.  The partial sums live in the linear's workspace: they must be consumed
-    before the next linear of that kind on the stream (checked)."""
+    before the next linear of that kind on the stream (checked).  A prompt's (``bf16_gemm_sliced``, ``key`` None) are
+    memory of their own, given back with this object."""
 
     def __init__(self, desc, shape, device, key, keep):
         self.desc, self.shape, self.device = desc, shape, device
         self._key, self._keep = key, keep            # keep: tensors the descriptor points into
-        self._uses = _workspaces[key].uses
+        self._uses, self._stream = (0, _raw_stream(device)) if key is None else (_workspaces[key].uses, 0)
 
     def check_live(self) -> None:
+        if self._key is None:
+            if _raw_stream(self.device) != self._stream:       # read on another stream than the one they are given back on
+                self._keep[0].record_stream(torch.cuda.current_stream(self.device))
+            return
         ws = _workspaces.get(self._key)
         _require(ws is not None and ws.uses == self._uses and ws.buf is self._keep[0],
                  "partial sums were overwritten: another linear used the workspace before they were consumed")
@@ -1003,12 +1008,11 @@ def bf16_gemm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor
     return out
 
 
-_SLICED_BYTES = 64 << 20        # the most a sliced product's partial sums take: one size, so that the buffer never grows
-
-
 @functools.lru_cache(maxsize=4096)
-def _slices_pay(M: int, K: int, N: int, reduced: bool) -> bool:
-    return bool(_C.load().hymeta_bf16_gemm_takes(M, K, N, 4 if reduced else 3))
+def _sliced_bytes(M: int, K: int, N: int, reduced: bool) -> int:
+    """Bytes of a sliced product's partial sums (64 MiB at most); 0: not to be cut."""
+    lib = _C.load()
+    return int(lib.hymeta_bf16_gemm_sliced_workspace_bytes(M, K, N)) if not reduced or lib.hymeta_bf16_gemm_takes(M, K, N, 4) else 0
 
 
 def bf16_gemm_sliced(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, reduced: bool = False) -> Optional[PartialSums]:
@@ -1017,7 +1021,7 @@ def bf16_gemm_sliced(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
     ``reduced``: the caller asks for their ``tensor()`` at once, which pays for fewer shapes than a consumer that adds them."""
     N, K = weight.shape
     # (the sizes first: other linears pay nothing for the rest)
-    if not (K >= 2 * N and x.is_cuda and x.dim() == 2 and x.shape[0] > BF16_GEMM_TALL_ROWS and _slices_pay(x.shape[0], K, N, reduced) and x.dtype == torch.bfloat16
+    if not (K >= 2 * N and x.is_cuda and x.dim() == 2 and x.shape[0] > BF16_GEMM_TALL_ROWS and _sliced_bytes(x.shape[0], K, N, reduced) and x.dtype == torch.bfloat16
             and weight.dtype == torch.bfloat16 and x.shape[1] == K and x.stride(1) == 1 and x.stride(0) % 8 == 0
             and 2 * x.shape[0] * x.stride(0) < 1 << 32 and weight.is_contiguous() and plain(x, weight, bias)
             and (x.data_ptr() | weight.data_ptr()) % 16 == 0):
@@ -1029,10 +1033,10 @@ def bf16_gemm_sliced(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
     a, desc = _C.Bf16GemmArgs(), _C.GemmPartials()
     a.x, a.weight, a.bias, a.M, a.K, a.N = _p(x), _p(weight), _p(bias), x.shape[0], K, N
     a.x_stride_m, a.w_stride_n = x.stride(0), weight.stride(0)
-    ws = _workspace(x.device, _SLICED_BYTES, "bf16_gemm_sliced")
-    a.workspace, a.workspace_bytes = _p(ws), _SLICED_BYTES
+    slabs = torch.empty(_sliced_bytes(x.shape[0], K, N, reduced), dtype=torch.uint8, device=x.device)
+    a.workspace, a.workspace_bytes = _p(slabs), slabs.numel()
     _C.check(lib.hymeta_bf16_gemm_sliced(C.byref(a), C.byref(desc), _stream(x)), "hymeta_bf16_gemm_sliced")
-    return _partials(desc, x.shape[0], N, x.device, "bf16_gemm_sliced", bias)
+    return PartialSums(desc, (x.shape[0], N), x.device, None, (slabs, bias))
 
 
 def logits_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
