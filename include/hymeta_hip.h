@@ -934,7 +934,7 @@ typedef struct hymeta_moe_gemm_args {
   const int32_t* scale_rows;   /* index into row_scale per slot, or NULL: s */
   const float* row_scale;      /* or NULL */
   int32_t a_rows_div;
-  int32_t max_rows;            /* upper bound on the slots in use (num_tokens * top_k) */
+  int32_t max_rows;            /* upper bound on the slots in use and on the values in a_rows (num_tokens * top_k) */
   int32_t K, N;
   int32_t local_expert_begin, local_expert_end;
   int64_t x_stride_m, out_stride_m, w_stride_e;

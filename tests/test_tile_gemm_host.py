@@ -1,5 +1,6 @@
 """The tiled products' matrix instructions are inline assembly, whose results the compiler does not know to be late: no
 accumulator may be moved between the instructions of a run and the wait that ends it."""
+import ctypes as C
 import os
 import re
 import shutil
@@ -39,3 +40,22 @@ def test_nothing_touches_an_accumulator_in_flight(tmp_path):
             # the source fixes; a block that ends in flight must not hold anything else
         assert runs >= 192
         assert not re.search(r"scratch_(load|store)", body), "a spill would wait for every copy in flight"
+
+
+def test_rows_of_x_that_run_backwards():
+    """Their offsets are unsigned in the tiles: grouped products leave such rows to the kernel with 64-bit addresses, products of one
+    matrix refuse them (before anything is launched)."""
+    from vllm_hymeta import _C
+    lib, unsupported = _C.load(), -2
+    a = _C.MoeGemmArgs()
+    a.max_rows, a.K, a.N, a.local_expert_end, a.x_stride_m, a.out_stride_m, a.w_stride_e = 4096, 512, 5120, 4, 512, 2560, 5120 * 512
+    assert lib.hymeta_moe_gemm_activates(C.byref(a)) == 1
+    a.x_stride_m = -512
+    assert lib.hymeta_moe_gemm_activates(C.byref(a)) == 0
+    b, partials = _C.Bf16GemmArgs(), _C.GemmPartials()
+    b.x = b.weight = b.out = b.workspace = 1 << 20
+    b.workspace_bytes, b.M, b.K, b.N, b.x_stride_m, b.w_stride_n, b.out_stride_m = 64 << 20, 512, 18944, 3584, -18944, 18944, 3584
+    assert lib.hymeta_bf16_gemm_sliced(C.byref(b), C.byref(partials), None) == unsupported
+    b.M, b.K, b.N, b.x_stride_m, b.w_stride_n, b.out_stride_m = 1280, 3584, 37888, -3584, 3584, 18944
+    assert lib.hymeta_bf16_gemm_takes(1280, 3584, 37888, 1) == 1
+    assert lib.hymeta_bf16_gemm_silu_mul(C.byref(b), None) == unsupported

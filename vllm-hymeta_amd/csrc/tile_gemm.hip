@@ -362,7 +362,7 @@ bool tile_gemm_fits(const TileGemmArgs& a) {
   const int64_t row_tiles = a.max_rows / kTile + 1 + kMaxTileExperts;
   constexpr int64_t kReach = int64_t{1} << 32;               // of a 32-bit offset
   return a.max_rows > 0 && a.k_bytes % kStep == 0 && a.k_bytes >= kMinSteps * kStep && a.N > 0 && a.N % kTile == 0 && (a.act == HYMETA_GEMM_ACT_NONE || a.bias == nullptr) && a.out_stride % 8 == 0 &&
-         a.x_stride % 16 == 0 && a.w_stride_e % 16 == 0 && source * a.x_stride < kReach && int64_t{64} * a.k_bytes < kReach / 2 &&
+         a.x_stride % 16 == 0 && a.w_stride_e % 16 == 0 && a.x_stride >= 0 && source * a.x_stride < kReach && int64_t{64} * a.k_bytes < kReach / 2 &&
          (a.a_rows == nullptr || (a.a_rows_div >= 1 && static_cast<int64_t>(a.max_rows) * a.a_rows_div < kReach / 2)) &&
          (a.expert_offsets == nullptr || a.expert_end - a.expert_begin <= kMaxTileExperts) && row_tiles * (a.N / kTile) < (int64_t{1} << 26);
 }
