@@ -403,9 +403,9 @@ __device__ __forceinline__ const uint16_t* vt_group(const MfmaSmem<D, DV>& sm, i
   return &sm.vt[c * MfmaSmem<D, DV>::kPitchV + 4 * (grp ^ ((c >> 3) & 15))];
 }
 
-// The rows of one wave against the staged tile.  RB row blocks of 16 (row = 16 rb + lane % 16); the wave takes 16-key
-// subtile ks of the tile's four (the waves of a decode workgroup split every tile between them and each keeps statistics of
-// its own).
+// The rows of one wave against the staged tile.  RB row blocks of 16 (row = 16 rb + lane % 16); the wave takes NKS of the
+// tile's four 16-key subtiles, from ks_lo on (a prompt's wave all four, a decode wave one: the four waves of a decode
+// workgroup split every tile between them and each keeps statistics of its own).
 template <int D, int DV, int RB>
 struct WaveRows {
   bf16x8 q[RB][D / 32];
@@ -423,21 +423,26 @@ __device__ __forceinline__ float tanh_fast(float x) {
 
 // Scaled (SCALED_KEY rows): `scales` holds a factor per key of the tile, the bias is linear in the distance (its
 // coefficient, in the base-2 domain, in w.ba) and there is no cap.
-template <int D, int DV, int RB, bool Masked, bool Scaled>
+template <int D, int DV, int RB, int NKS, bool Masked, bool Scaled>
 __device__ __forceinline__ void attend_tile(WaveRows<D, DV, RB>& w, const MfmaSmem<D, DV>& sm, const float* scales,
-                                            const hymeta_sink_attention_args& a, int j0, int ks) {
+                                            const hymeta_sink_attention_args& a, int j0, int ks_lo) {
+  static_assert(NKS == 4 || NKS == 1, "all of a tile's subtiles or one");
   const int lane = threadIdx.x & 63, n = lane & 15, g4 = lane >> 4;
   constexpr int PK = MfmaSmem<D, DV>::kPitchK;
-  f32x4v s[RB];
+  f32x4v s[RB][NKS];
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) s[rb] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-  for (int st = 0; st < D / 32; ++st) {
-    const bf16x8 kf = __builtin_bit_cast(bf16x8, ld16(&sm.k[(16 * ks + n) * PK + 32 * st + 8 * g4]));
+    for (int ks = 0; ks < NKS; ++ks) s[rb][ks] = f32x4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) s[rb] = mfma16(kf, w.q[rb][st], s[rb]);
-  }
-  // lane holds, per row block, the scores of its row (n) against keys j0 + 16 ks + 4 g4 + r.  Everything from
+  for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+    for (int st = 0; st < D / 32; ++st) {
+      const bf16x8 kf = __builtin_bit_cast(bf16x8, ld16(&sm.k[(16 * (ks_lo + ks) + n) * PK + 32 * st + 8 * g4]));
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) s[rb][ks] = mfma16(kf, w.q[rb][st], s[rb][ks]);
+    }
+  // lane holds, per row block, the scores of its row (n) against keys j0 + 16 (ks_lo + ks) + 4 g4 + r.  Everything from
   // here to the weights is in the base-2 domain (scores times log2 e; the bias' coefficient is unchanged, as
   // a ln x * log2 e = a log2 x): one v_log and one v_exp per score and no multiplications around them.  The running
   // maximum, and with it the sink's score 0, mean the same in both domains.
@@ -446,32 +451,35 @@ __device__ __forceinline__ void attend_tile(WaveRows<D, DV, RB>& w, const MfmaSm
   // capped scores: softcap tanh(score / softcap), moved into the base-2 domain like the others
   const bool capped = a.softcap > 0.f;
   const float cap2 = a.softcap * 1.4426950408889634f, cap_in = capped ? a.scale / a.softcap : 0.f;
-  uint32_t phi[RB][2], plo[RB][2];       // the weights' bf16 high and low parts, two per dword
+  uint32_t phi[RB][NKS][2], plo[RB][NKS][2];       // the weights' bf16 high and low parts, two per dword
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     const int pos = w.pos[rb];
-    // distance of the lane's key r: fd0 - r
-    const float fd0 = static_cast<float>(pos - j0 - 16 * ks - 4 * g4);
+    // distance of the lane's key r of subtile ks: fd0 - (16 ks + r)
+    const float fd0 = static_cast<float>(pos - j0 - 16 * ks_lo - 4 * g4);
     float mx = -INFINITY;
     const float near = -w.ba[rb] * fd0;            // (Scaled) the linear bias of the lane's first key, sign included
-    f32x4v kscale = f32x4v{0.f, 0.f, 0.f, 0.f};
-    if (Scaled) kscale = *reinterpret_cast<const f32x4v*>(scales + 16 * ks + 4 * g4) * scale2;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float sc;
-      if (Scaled) {
-        sc = fmaf(s[rb][r], kscale[r], fmaf(w.ba[rb], static_cast<float>(r), near));
-      } else {
-        sc = s[rb][r] * scale2;
-        if (capped) sc = cap2 * tanh_fast(s[rb][r] * cap_in);
-        if (bias) sc = fmaf(-w.ba[rb], __log2f(fmaf(w.bb[rb], fd0 - static_cast<float>(r), 1.f)), sc);
+    for (int ks = 0; ks < NKS; ++ks) {
+      f32x4v kscale = f32x4v{0.f, 0.f, 0.f, 0.f};
+      if (Scaled) kscale = *reinterpret_cast<const f32x4v*>(scales + 16 * (ks_lo + ks) + 4 * g4) * scale2;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float sc;
+        if (Scaled) {
+          sc = fmaf(s[rb][ks][r], kscale[r], fmaf(w.ba[rb], static_cast<float>(16 * ks + r), near));
+        } else {
+          sc = s[rb][ks][r] * scale2;
+          if (capped) sc = cap2 * tanh_fast(s[rb][ks][r] * cap_in);
+          if (bias) sc = fmaf(-w.ba[rb], __log2f(fmaf(w.bb[rb], fd0 - static_cast<float>(16 * ks + r), 1.f)), sc);
+        }
+        if (Masked) {
+          const int j = j0 + 16 * (ks_lo + ks) + 4 * g4 + r;
+          sc = (j <= pos && (j >= w.first[rb] || j < a.keep_first)) ? sc : -INFINITY;
+        }
+        s[rb][ks][r] = sc;
+        mx = fmaxf(mx, sc);
       }
-      if (Masked) {
-        const int j = j0 + 16 * ks + 4 * g4 + r;
-        sc = (j <= pos && (j >= w.first[rb] || j < a.keep_first)) ? sc : -INFINITY;
-      }
-      s[rb][r] = sc;
-      mx = fmaxf(mx, sc);
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
@@ -481,31 +489,52 @@ __device__ __forceinline__ void attend_tile(WaveRows<D, DV, RB>& w, const MfmaSm
     const float corr = empty ? 0.f : __builtin_amdgcn_exp2f(w.m[rb] - m_new);
     float sum = 0.f;
 #pragma unroll
-    for (int r2 = 0; r2 < 2; ++r2) {
-      float p[2];
+    for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        p[u] = empty ? 0.f : __builtin_amdgcn_exp2f(s[rb][2 * r2 + u] - m_new);
-        sum += p[u];
+      for (int r2 = 0; r2 < 2; ++r2) {
+        float p[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          p[u] = empty ? 0.f : __builtin_amdgcn_exp2f(s[rb][ks][2 * r2 + u] - m_new);
+          sum += p[u];
+        }
+        const uint32_t hi = pack_bf16x2(p[0], p[1]);
+        phi[rb][ks][r2] = hi;
+        plo[rb][ks][r2] = pack_bf16x2(p[0] - lo_bf(hi), p[1] - hi_bf(hi));
       }
-      const uint32_t hi = pack_bf16x2(p[0], p[1]);
-      phi[rb][r2] = hi;
-      plo[rb][r2] = pack_bf16x2(p[0] - lo_bf(hi), p[1] - hi_bf(hi));
-    }
     w.l[rb] = w.l[rb] * corr + sum;
     w.m[rb] = m_new;
 #pragma unroll
     for (int cb = 0; cb < DV / 16; ++cb) w.o[rb][cb] *= corr;
   }
+  if constexpr (NKS == 4) {
 #pragma unroll
-  for (int cb = 0; cb < DV / 16; ++cb) {
-    const bf16x4 vf = __builtin_bit_cast(bf16x4, *reinterpret_cast<const u32x2*>(vt_group<D, DV>(sm, 16 * cb + n, 4 * ks + g4)));
+    for (int cb = 0; cb < DV / 16; ++cb)
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      const bf16x4 ph = __builtin_bit_cast(bf16x4, (u32x2{phi[rb][0], phi[rb][1]}));
-      const bf16x4 pl = __builtin_bit_cast(bf16x4, (u32x2{plo[rb][0], plo[rb][1]}));
-      w.o[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf, ph, w.o[rb][cb], 0, 0, 0);
-      w.o[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf, pl, w.o[rb][cb], 0, 0, 0);
+      for (int kp = 0; kp < 2; ++kp) {
+        // k index 8 g4 + e of the product: keys 16 (2 kp) + 4 g4 + e for e < 4, 16 (2 kp + 1) + 4 g4 + e - 4 after
+        const u32x2 v0 = *reinterpret_cast<const u32x2*>(vt_group<D, DV>(sm, 16 * cb + n, 8 * kp + g4));
+        const u32x2 v1 = *reinterpret_cast<const u32x2*>(vt_group<D, DV>(sm, 16 * cb + n, 8 * kp + 4 + g4));
+        const bf16x8 vf = __builtin_bit_cast(bf16x8, (u32x4{v0[0], v0[1], v1[0], v1[1]}));
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+          const bf16x8 ph = __builtin_bit_cast(bf16x8, (u32x4{phi[rb][2 * kp][0], phi[rb][2 * kp][1], phi[rb][2 * kp + 1][0], phi[rb][2 * kp + 1][1]}));
+          const bf16x8 pl = __builtin_bit_cast(bf16x8, (u32x4{plo[rb][2 * kp][0], plo[rb][2 * kp][1], plo[rb][2 * kp + 1][0], plo[rb][2 * kp + 1][1]}));
+          w.o[rb][cb] = mfma16(vf, ph, w.o[rb][cb]);
+          w.o[rb][cb] = mfma16(vf, pl, w.o[rb][cb]);
+        }
+      }
+  } else {
+#pragma unroll
+    for (int cb = 0; cb < DV / 16; ++cb) {
+      const bf16x4 vf = __builtin_bit_cast(bf16x4, *reinterpret_cast<const u32x2*>(vt_group<D, DV>(sm, 16 * cb + n, 4 * ks_lo + g4)));
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        const bf16x4 ph = __builtin_bit_cast(bf16x4, (u32x2{phi[rb][0][0], phi[rb][0][1]}));
+        const bf16x4 pl = __builtin_bit_cast(bf16x4, (u32x2{plo[rb][0][0], plo[rb][0][1]}));
+        w.o[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf, ph, w.o[rb][cb], 0, 0, 0);
+        w.o[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf, pl, w.o[rb][cb], 0, 0, 0);
+      }
     }
   }
 }
@@ -519,8 +548,11 @@ __device__ __forceinline__ void load_q(WaveRows<D, DV, RB>& w, int rb, const uin
 }
 
 // Whether every key of the tile from j0 on is visible to every query position in [p_lo, p_hi] (first_hi: the first key p_hi
-// sees).
+// sees) / none of them to any (first_lo: the first key p_lo sees).
 __device__ __forceinline__ bool tile_open(int j0, int p_lo, int first_hi) { return j0 + kTileKeys - 1 <= p_lo && j0 >= first_hi; }
+__device__ __forceinline__ bool tile_shut(const hymeta_sink_attention_args& a, int j0, int first_lo) {
+  return j0 + kTileKeys - 1 < first_lo && j0 >= a.keep_first;
+}
 
 // The bias' constants of head h as attend_tile wants them.
 template <int D, int DV, int RB>
@@ -528,6 +560,105 @@ __device__ __forceinline__ void load_bias(WaveRows<D, DV, RB>& w, int rb, const 
   w.ba[rb] = a.bias_mode ? a.bias_a[h] : 0.f;
   if (a.bias_mode == HYMETA_BIAS_LINEAR_DISTANCE) w.ba[rb] *= 1.4426950408889634f;
   w.bb[rb] = a.bias_mode == HYMETA_BIAS_LOG_DISTANCE ? a.bias_b[h] : 0.f;
+}
+
+// Short portions of prompts over few keys, rows of HYMETA_KV_SHARED_KEY with keys of more than 192 elements (more of either:
+// row_pipe.h, few_long_keys has the line; shorter keys and other rows: row_attn.h, wide_latent.h): grid = (tiles of 16 rows per wave,
+// heads, sequences); sequences of fewer than `least` rows are left to the decode form.  4 waves: the query fragments (D / 8
+// registers) and the staging registers do not leave a wave of 8 its accumulators within 256 registers.  Bound by LDS, whose tile
+// every wave reads whole for 16 rows: about 5 us a tile of 64 keys of 512, but 5 around them, where row_pipe.h's blocks take 2.8 and 14.
+constexpr int kPrefillWaves = 4, kPrefillRows = 16 * kPrefillWaves;
+
+template <int D, int DV>
+__global__ __launch_bounds__(64 * kPrefillWaves) void sink_attention_prefill_shared_kernel(hymeta_sink_attention_args a, int least) {
+  constexpr int kRows = kPrefillRows;
+  constexpr int kImages = 2 * sizeof(MfmaSmem<D, DV>) <= 159 * 1024 ? 2 : 1;        // (160 KB of LDS)
+  __shared__ MfmaSmem<D, DV> sm[kImages];
+  // (a prompt's later rows see more keys: the row blocks are handed out from the last on, all heads of a block side by side)
+  const int lin = blockIdx.x + gridDim.x * blockIdx.y;
+  const int s = blockIdx.z, h = lin % gridDim.y, tile = gridDim.x - 1 - lin / gridDim.y;
+  const int row0 = a.query_start_loc[s];
+  const int q = a.query_start_loc[s + 1] - row0;
+  if (q < least || tile * kRows >= q) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g4 = lane >> 4;
+  const int g = h / (a.num_heads / a.num_kv_heads);
+  const int ctx = a.seq_lens[s] - q;
+  const int32_t* bt = a.block_tables + static_cast<int64_t>(s) * a.block_table_stride;
+  WaveRows<D, DV, 1> w;
+  const int wrow = tile * kRows + wave * 16, r = wrow + n;
+  const bool ok = r < q;
+  w.pos[0] = ok ? ctx + r : -1;
+  w.first[0] = first_key(a, ctx + r);
+  load_bias<D, DV, 1>(w, 0, a, h);
+  w.m[0] = a.sink ? (a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f) : -INFINITY;
+  w.l[0] = (a.sink && g4 == 0) ? 1.f : 0.f;          // the sink's exp(m - m), counted once per row
+  load_q<D, DV, 1>(w, 0, ok ? static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(row0 + r) * a.q_stride_t + static_cast<int64_t>(h) * D : nullptr);
+#pragma unroll
+  for (int cb = 0; cb < DV / 16; ++cb) w.o[0][cb] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  const int block_last = ctx + min(q, tile * kRows + kRows) - 1;      // last key any row of the block sees
+  const int wave_last = ctx + min(q, wrow + 16) - 1;
+  const int first_lo = first_key(a, ctx + wrow), first_hi = first_key(a, wave_last);           // of the wave's rows
+  const int j_first = first_key(a, ctx + tile * kRows) / kTileKeys * kTileKeys;
+  // the tiles of the kept first keys that lie before the window's first tile come first, then the window's
+  const int keep_end = bounded(a) ? min((a.keep_first + kTileKeys - 1) / kTileKeys * kTileKeys, j_first) : 0;
+  const int j_start = keep_end > 0 ? 0 : j_first;
+  auto next = [&](int j0) { return (j0 < keep_end && j0 + kTileKeys >= keep_end) ? j_first : j0 + kTileKeys; };
+  // two LDS images: while the waves multiply tile t out of one, tile t + 1 goes into the other and the loads of tile
+  // t + 2 are in flight; one barrier per tile
+  TileStage<D, DV, 64 * kPrefillWaves, HYMETA_KV_SHARED_KEY> stage;
+  stage.value_at = D + g * DV;
+  stage.issue(a, bt, g, j_start, block_last);
+  stage.commit(sm[0], nullptr);
+  if (kImages == 2 && next(j_start) <= block_last) stage.issue(a, bt, g, next(j_start), block_last);
+  __syncthreads();
+  if constexpr (kImages == 2) {
+    int buf = 0;
+    for (int j0 = j_start; j0 <= block_last; j0 = next(j0), buf ^= 1) {
+      const int j1 = next(j0), j2 = next(j1);
+      if (j1 <= block_last) stage.commit(sm[buf ^ 1], nullptr);
+      if (j2 <= block_last) stage.issue(a, bt, g, j2, block_last);
+      if (wrow < q && j0 <= wave_last && !tile_shut(a, j0, first_lo)) {
+        // tiles whose every key is visible to every row of the wave need no mask
+        if (tile_open(j0, ctx + wrow, first_hi)) attend_tile<D, DV, 1, 4, false, false>(w, sm[buf], nullptr, a, j0, 0);
+        else attend_tile<D, DV, 1, 4, true, false>(w, sm[buf], nullptr, a, j0, 0);
+      }
+      __syncthreads();
+    }
+  } else {
+    // one image (tiles of long rows): the next tile's loads are in flight while this one is multiplied and go into LDS
+    // behind a barrier
+    for (int j0 = j_start; j0 <= block_last; j0 = next(j0)) {
+      const bool more = next(j0) <= block_last;
+      if (more) stage.issue(a, bt, g, next(j0), block_last);
+      if (wrow < q && j0 <= wave_last && !tile_shut(a, j0, first_lo)) {
+        if (tile_open(j0, ctx + wrow, first_hi)) attend_tile<D, DV, 1, 4, false, false>(w, sm[0], nullptr, a, j0, 0);
+        else attend_tile<D, DV, 1, 4, true, false>(w, sm[0], nullptr, a, j0, 0);
+      }
+      __syncthreads();
+      if (more) {
+        stage.commit(sm[0], nullptr);
+        __syncthreads();
+      }
+    }
+  }
+  float l = w.l[0];
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (r >= q) return;
+  float inv = l > 0.f ? 1.f / l : 0.f;
+  if (a.head_gate) inv *= sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.head_gate)[static_cast<int64_t>(row0 + r) * a.head_gate_stride_t + h]));
+  uint16_t* out = static_cast<uint16_t*>(a.out) + (static_cast<int64_t>(row0 + r) * a.num_heads + h) * DV;
+#pragma unroll
+  for (int cb = 0; cb < DV / 16; ++cb) {
+    f32x4v o = w.o[0][cb] * inv;
+    if (a.elem_gate) {
+      float gate[4];
+      ActBf16::ld4(static_cast<const uint16_t*>(a.elem_gate) + static_cast<int64_t>(row0 + r) * a.elem_gate_stride_t + static_cast<int64_t>(h) * DV + 16 * cb + 4 * g4, gate);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] *= ActBf16::sigmoid(gate[e]);
+    }
+    *reinterpret_cast<u32x2*>(out + 16 * cb + 4 * g4) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+  }
 }
 
 // Partial of a (sequence, key/value head, slice, wave): per query head of the group DV weighted values, then the
@@ -622,8 +753,8 @@ __global__ __launch_bounds__(64 * kDecodeWaves) void sink_attention_decode_mfma_
       if (v + 1 <= v_hi) stage.commit(sm[buf ^ 1], s_scale[buf ^ 1]);
       if (v + 2 <= v_hi) stage.issue(a, bt, g, tile(v + 2), pos);
       if (j0 + 16 * wave <= pos) {
-        if (tile_open(j0, pos, first)) attend_tile<D, DV, RB, false, kScaled>(w, sm[buf], s_scale[buf], a, j0, wave);
-        else attend_tile<D, DV, RB, true, kScaled>(w, sm[buf], s_scale[buf], a, j0, wave);
+        if (tile_open(j0, pos, first)) attend_tile<D, DV, RB, 1, false, kScaled>(w, sm[buf], s_scale[buf], a, j0, wave);
+        else attend_tile<D, DV, RB, 1, true, kScaled>(w, sm[buf], s_scale[buf], a, j0, wave);
       }
       __syncthreads();
     }
@@ -634,8 +765,8 @@ __global__ __launch_bounds__(64 * kDecodeWaves) void sink_attention_decode_mfma_
       const bool more = v + 1 <= v_hi;
       if (more) stage.issue(a, bt, g, tile(v + 1), pos);
       if (j0 + 16 * wave <= pos) {
-        if (tile_open(j0, pos, first)) attend_tile<D, DV, RB, false, kScaled>(w, sm[0], s_scale[0], a, j0, wave);
-        else attend_tile<D, DV, RB, true, kScaled>(w, sm[0], s_scale[0], a, j0, wave);
+        if (tile_open(j0, pos, first)) attend_tile<D, DV, RB, 1, false, kScaled>(w, sm[0], s_scale[0], a, j0, wave);
+        else attend_tile<D, DV, RB, 1, true, kScaled>(w, sm[0], s_scale[0], a, j0, wave);
       }
       __syncthreads();
       if (more) {
@@ -965,13 +1096,14 @@ inline PortionSlices portion_slices(int num_tokens, int num_seqs, int num_heads,
   return ps;
 }
 inline bool one_launch(const hymeta_sink_attention_args& a, const PortionSlices& ps, int most);
+inline bool long_shared_keys(const hymeta_sink_attention_args& a);
 inline PortionSlices portion_slices(const hymeta_sink_attention_args& a) {
   PortionSlices ps;
   if (a.max_query_len <= 1) return ps;
   ps = portion_slices(a.num_tokens, a.num_seqs, a.num_heads, a.num_kv_heads, a.v_dim, a.max_query_len, decode_tiles(a), a.head_dim);
   // Long keys are cut only where the portions' launch takes the single rows as well (one_launch): the slices then have the room
   // of the decode form's partials, which a caller brings anyway.
-  const bool long_keys = a.kv_layout == HYMETA_KV_SHARED_KEY && a.head_dim > 192;
+  const bool long_keys = long_shared_keys(a);
   if (long_keys && ps.splits > 1 && !one_launch(a, ps, 0)) ps.splits = 1;
   const int64_t decode = long_keys ? 0 : decode_partial_bytes(a.num_seqs, a.num_heads, a.num_kv_heads, a.v_dim, a.max_seq_len);
   const int64_t room = (static_cast<int64_t>(a.workspace_bytes) - decode) / portion_partial_bytes(a.num_tokens, a.num_heads, a.v_dim);
@@ -993,11 +1125,28 @@ inline dim3 portion_grid(const hymeta_sink_attention_args& a, const PortionSlice
 // about 5 the host's shorter call).  With one key/value head, whose single rows fill a fifth of a block, a quarter as many: 300 rows beside 8
 // single ones of 4096 keys on latents of 128 + 64 46 -> 49, beside 63 75 -> 86.  A logarithm per score makes them dearer: 40 rows with nothing
 // in front beside 15 single ones of 4096 keys 39.7 -> 42.3, but 2 behind 3000 beside 15 of 3000 40.3 -> 37.0.
-constexpr int kFewTiles = 16, kFewWideTiles = 2, kManySingleRows = 512, kFewSingleRows = 4;
+// Long keys have one workgroup on a compute unit, so single rows go along where they take no more rounds of units than the portions do
+// without them: 40 rows beside 63 single ones of 100 keys of 512, 28 heads, in 264 workgroups 23.9, in two launches 22.0; beside 127
+// 53.9 and 43.6, 40 beside 127 of 400 keys of 256 68 and 57; 40 beside 48 of 60 keys, 204 workgroups, 17 and 22.
+constexpr int kFewTiles = 16, kFewWideTiles = 2, kManySingleRows = 512, kLongKeyUnits = 256, kFewSingleRows = 4;
+inline bool long_shared_keys(const hymeta_sink_attention_args& a) { return a.kv_layout == HYMETA_KV_SHARED_KEY && a.head_dim > 192; }
 inline bool one_launch(const hymeta_sink_attention_args& a, const PortionSlices& ps, int most) {
-  const int64_t singles = a.num_seqs - long_portions(a.num_tokens, a.num_seqs, a.max_query_len);
+  const int64_t portions = long_portions(a.num_tokens, a.num_seqs, a.max_query_len), singles = a.num_seqs - portions;
   if (a.max_query_len <= 1) return false;
-  return ps.splits > 1 ? singles <= kFewSingleRows * std::min(a.num_kv_heads, 4) : decode_tiles(a) <= most && singles * a.num_kv_heads <= kManySingleRows;
+  if (ps.splits > 1) return singles <= kFewSingleRows * std::min(a.num_kv_heads, 4);
+  if (decode_tiles(a) > most) return false;
+  if (!long_shared_keys(a)) return singles * a.num_kv_heads <= kManySingleRows;
+  const int64_t each = (static_cast<int64_t>(a.max_query_len) * (a.num_heads / a.num_kv_heads) + kPortionRows - 1) / kPortionRows;
+  const int64_t units = each * portions * a.num_kv_heads;
+  return units + singles * a.num_kv_heads <= (units + kLongKeyUnits - 1) / kLongKeyUnits * kLongKeyUnits || singles == 0;
+}
+// Long keys: whether sink_attention_prefill_shared_kernel takes the portions (and, `alone`, the single rows): keys of four tiles at most
+// and all workgroups at once.  Its time -> row_pipe.h's, us, 28 heads of 512, 48 rows: one tile 10.4 -> 16.6, two 14.9 -> 22.8, four
+// 25.0 -> 27.3, six 34.8 -> 32.5; four tiles, four portions of 128 rows (224 workgroups) 26.9 -> 28.1, of 200 (448) 48.2 -> 28.2.
+constexpr int kFewLongTiles = 4;
+inline bool few_long_keys(const hymeta_sink_attention_args& a, bool alone) {
+  const int64_t portions = long_portions(a.num_tokens, a.num_seqs, a.max_query_len), each = (a.max_query_len + kPrefillRows - 1) / kPrefillRows;
+  return decode_tiles(a) <= kFewLongTiles && (each * portions + (alone ? a.num_seqs - portions : 0)) * a.num_heads <= kLongKeyUnits;
 }
 void launch_combine(const hymeta_sink_attention_args& a, hipStream_t st, int splits, HeadSlice hs, const PortionSlices& ps) {
   const int heads = hs.count ? hs.count * a.num_kv_heads : a.num_heads;
@@ -1044,9 +1193,19 @@ int launch_mfma(const hymeta_sink_attention_args& a, hipStream_t st) {
     const bool alone = one_launch(a, ps, kFewTiles);
     if (alone) ps.least = 1;
     const dim3 grid = portion_grid(a, ps);
+    bool done = false;
+    if constexpr (D > 192) {
+      done = few_long_keys(a, alone);
+      if (done) {
+        ps.splits = 1;
+        const dim3 all((a.max_query_len + kPrefillRows - 1) / kPrefillRows, a.num_heads, a.num_seqs);
+        hipLaunchKernelGGL((sink_attention_prefill_shared_kernel<D, DV>), all, dim3(64 * kPrefillWaves), 0, st, a, ps.least);
+      }
+    }
     // a kernel per rule of the scores; a cap and a bias together, which no design has, in the general one
     auto launch = [&](auto rule) {
       constexpr int Rule = decltype(rule)::value;
+      if (done) return;
       if constexpr (D > 192 || ((Layout == HYMETA_KV_KEY_THEN_VALUE || Layout == HYMETA_KV_SHARED_KEY) && Rule != kAnyRule))
         hipLaunchKernelGGL((row_pipe_kernel<D, DV, Layout, Rule>), grid, dim3(256), 0, st, a, ps);
       else hipLaunchKernelGGL((row_prefill_kernel<D, DV, Layout, Rule>), grid, dim3(256), 0, st, a, ps);
