@@ -86,6 +86,31 @@ def test_grouped_products(sizes, K, N, div, local, act, int8):
     assert bool((out[P] == 7.0).all())
 
 
+@pytest.mark.parametrize("sizes,K,N,local,total", [
+    ((1, 255, 256, 257, 0, 511, 129, 200), 2048, 5120, (0, 8), 0),               # 201 rows an expert on average, tiles of eight waves
+    ((200, 140, 160, 141) * 2, 2080, 5120, (0, 8), 0),                           # 160; an odd number of steps
+    ((239,) * 8, 2048, 5120, (0, 8), 0),
+    ((200, 3, 0, 260, 130, 190, 300, 129, 17), 2112, 5376, (1, 9), 9),           # eight of nine
+])
+def test_grouped_products_by_the_rows_of_an_expert(sizes, K, N, local, total):
+    from vllm_hymeta import _C
+    lib, E, P = _C.load(), len(sizes), sum(sizes)
+    g = gen(23)
+    x, w = _ints(g, -3, 3, P, K).bfloat16().cuda(), _ints(g, -2, 2, E, N, K).bfloat16().cuda()
+    offsets = torch.tensor([0] + list(sizes)).cumsum(0)
+    on_card, out = offsets.int().cuda(), torch.full((P + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    a = _C.MoeGemmArgs()
+    a.x, a.weights, a.out, a.expert_offsets = x.data_ptr(), w.data_ptr(), out.data_ptr(), on_card.data_ptr()
+    a.a_rows_div, a.max_rows, a.K, a.N, a.x_stride_m, a.out_stride_m, a.w_stride_e = 1, P, K, N, K, N, N * K
+    a.local_expert_begin, a.local_expert_end = local
+    assert lib.hymeta_moe_gemm(C.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+    for e in range(E):
+        lo, hi = int(offsets[e]), int(offsets[e + 1])
+        want = (x[lo:hi].float() @ w[e].float().t()).bfloat16() if local[0] <= e < local[1] else torch.full_like(out[lo:hi], 7.0)
+        assert torch.equal(out[lo:hi], want), f"expert {e}"
+    assert bool((out[P] == 7.0).all())
+
+
 def test_what_the_tiles_do_not_take():
     """No activation for a problem of few rows; int8 knows the quantised path's silu only."""
     from vllm_hymeta import _C

@@ -505,7 +505,7 @@ __global__ __launch_bounds__(256) void moe_gemm_lines_kernel(hymeta_moe_gemm_arg
   }
 }
 
-// Prompts of few rows per expert (tile_gemm.hip takes the long ones): BM rows x BN columns per workgroup, WM x WN waves that own
+// Prompts of few rows per expert (tile_gemm.hip takes the long ones), and those whose experts nearly fill a tile of 256: BM rows x BN columns per workgroup, WM x WN waves that own
 // (BM / WM) x (BN / WN) each.  Both operands are K-contiguous; a 64-deep step of each (128 bytes per
 // row) is staged once per workgroup through double-buffered LDS images (16-byte chunks XOR-ed with
 // the row, so the sixteen rows of a fragment read hit distinct banks): registers -> LDS right
@@ -805,16 +805,25 @@ extern "C" int hymeta_moe_router(const hymeta_moe_router_args* args, hymeta_stre
 
 namespace hymeta {
 namespace {
-enum class MoeGemmKind { kBigTiles, kTiles, kLines, kFragments };
+enum class MoeGemmKind { kBigTiles, kTallTiles, kTiles, kLines, kFragments };
 
-MoeGemmKind moe_gemm_kind(int64_t max_rows, int experts, int K, int N) {
+// total: the experts that max_rows pairs are spread over, of which a rank holds `experts`; act: with an activation behind
+MoeGemmKind moe_gemm_kind(int64_t max_rows, int experts, int total, int K, int N, bool i8, bool act) {
   // tiled grouped GEMM once the experts average more than a few rows (prefill chunks); the large tile when they fill it
   if (max_rows > static_cast<int64_t>(kTiledMinRowsPerExpert) * experts && K % kTK == 0) {
-    // tiles of 256 where the experts fill half of one on average (a little more with many columns, whose tiles fill the chip either
+    // Tiles of 256 where the experts fill half of one on average (a little more with many columns, whose tiles fill the chip either
     // way) and the tiles (an expert's rows scatter around the average) nearly fill the chip once: 16 experts on 2048 tokens of 3584
-    // columns 560 -> 497 us, 8 on 1400 936 -> 705; with 112 rows an expert 424 -> 459, with 64 to 128 tiles 215 -> 226
-    const int64_t rows = max_rows / experts, tiles = (rows + 64 + 255) / 256 * experts * (N / 256);
-    if (rows >= (N > 4096 ? 144 : 128) && tiles >= kBigTileMinTiles && N % 256 == 0) return MoeGemmKind::kBigTiles;
+    // columns 560 -> 497 us, 8 on 1400 936 -> 705; with 112 rows an expert 424 -> 459, with 64 to 128 tiles 215 -> 226.  Up to 192 rows it is
+    // those that a rank's experts can expect, not all pairs (8 of 16 experts of 14336 x 8192 at 300 tokens, top 4, 73 rows an expert, 602 ->
+    // 675); from 192 on half-empty tiles are level or better (the same at 512 tokens, 128 rows, 800 -> 735).
+    const int64_t rows = max_rows / total, most = max_rows / experts, tiles = (most + 64 + 255) / 256 * experts * (N / 256);
+    // One row tile an expert, nearly full, and tiles for most of the chip: every weight is fetched once, and eight waves that hold their
+    // rows in registers keep more of them in flight than the copies.  Tiles of tile_gemm.hip -> these, bf16, 196 rows an expert: 8 experts
+    // of 8192 x 8192 301 -> 270 us, of 5120 x 4736 137 -> 125, 16 of 14336 x 8192 1029 -> 968, 4 of 9472 x 5120 152 -> 143 (of 5120 x 4736, 80
+    // tiles, 80 -> 109); whole blocks of 8 experts with 162 rows 478 -> 430 (8192, 4096 wide) and 314 -> 314 (3584, 4736); with 235 rows, where an
+    // expert or two has a second tile, 16 of 8192 x 8192 712 -> 669, 8 of 14336 x 8192 636 -> 643.  Below a K of 5120 the other kernel's epilogue saves more than that where an activation follows.
+    if (!i8 && rows >= 160 && rows < 240 && N % 256 == 0 && experts * (N / 256) >= 148 && K >= (act ? 5120 : 2048)) return MoeGemmKind::kTallTiles;
+    if ((rows >= (N > 4096 ? 144 : 128) || most >= 192) && tiles >= kBigTileMinTiles && N % 256 == 0) return MoeGemmKind::kBigTiles;
     if (N % 128 == 0) return MoeGemmKind::kTiles;
   }
   static const bool lines = [] {
@@ -827,7 +836,7 @@ MoeGemmKind moe_gemm_kind(int64_t max_rows, int experts, int K, int N) {
 }  // namespace hymeta
 
 extern "C" int hymeta_moe_gemm_fuses(int32_t max_rows, int32_t experts, int32_t K, int32_t N) {
-  return experts > 0 && hymeta::moe_gemm_kind(max_rows, experts, K, N) == hymeta::MoeGemmKind::kLines ? 1 : 0;
+  return experts > 0 && hymeta::moe_gemm_kind(max_rows, experts, experts, K, N, false, false) == hymeta::MoeGemmKind::kLines ? 1 : 0;
 }
 
 namespace hymeta {
@@ -845,13 +854,22 @@ TileGemmArgs tile_args(const hymeta_moe_gemm_args& a) {
   return t;
 }
 
-MoeGemmKind moe_gemm_kind(const hymeta_moe_gemm_args& a) {
+MoeGemmKind moe_gemm_kind(const hymeta_moe_gemm_args& a, int num_experts, bool act) {
   // the kind goes by the bytes of a row
-  const MoeGemmKind kind = moe_gemm_kind(a.max_rows, a.local_expert_end - a.local_expert_begin, a.operand_dtype == HYMETA_I8 ? a.K / 2 : a.K, a.N);
+  const bool i8 = a.operand_dtype == HYMETA_I8;
+  const int experts = a.local_expert_end - a.local_expert_begin;
+  const MoeGemmKind kind = moe_gemm_kind(a.max_rows, experts, std::max(experts, num_experts), i8 ? a.K / 2 : a.K, a.N, i8, act);
   return kind == MoeGemmKind::kBigTiles && !tile_gemm_fits(tile_args(a)) ? MoeGemmKind::kTiles : kind;
 }
 
-int moe_gemm(const hymeta_moe_gemm_args* args, int act, float limit, float alpha, hymeta_stream_t stream) {
+bool moe_gemm_activates(const hymeta_moe_gemm_args& a, int num_experts) {
+  if (a.local_expert_end <= a.local_expert_begin || (a.a_rows != nullptr && a.a_rows_div <= 0)) return false;
+  TileGemmArgs t = tile_args(a);
+  t.act = HYMETA_GEMM_ACT_SILU;
+  return moe_gemm_kind(a, num_experts, true) == MoeGemmKind::kBigTiles && tile_gemm_fits(t);
+}
+
+int moe_gemm(const hymeta_moe_gemm_args* args, int num_experts, int act, float limit, float alpha, hymeta_stream_t stream) {
   if (!args_ok(args)) return HYMETA_ERR_INVALID_ARG;
   const hymeta_moe_gemm_args& a = *args;
   if (a.max_rows < 0 || a.K <= 0 || a.N <= 0) return HYMETA_ERR_INVALID_ARG;
@@ -868,8 +886,8 @@ int moe_gemm(const hymeta_moe_gemm_args* args, int act, float limit, float alpha
   if ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.weights) | reinterpret_cast<uintptr_t>(a.out)) % 16 != 0)
     return HYMETA_ERR_UNSUPPORTED;
   const int experts = a.local_expert_end - a.local_expert_begin;
-  const MoeGemmKind kind = moe_gemm_kind(a);
-  if (act != HYMETA_GEMM_ACT_NONE && hymeta_moe_gemm_activates(args) != 1) return HYMETA_ERR_UNSUPPORTED;
+  const MoeGemmKind kind = moe_gemm_kind(a, num_experts, act != HYMETA_GEMM_ACT_NONE);
+  if (act != HYMETA_GEMM_ACT_NONE && !moe_gemm_activates(a, num_experts)) return HYMETA_ERR_UNSUPPORTED;
   if (i8 && act > HYMETA_GEMM_ACT_SILU) return HYMETA_ERR_UNSUPPORTED;
   if (a.combine_tokens != nullptr || a.combine_shared != nullptr) {
     // the fused combine exists in the decode-sized kernel with whole-line loads only (hymeta_moe_gemm_fuses)
@@ -887,6 +905,11 @@ int moe_gemm(const hymeta_moe_gemm_args* args, int act, float limit, float alpha
     TileGemmArgs t = tile_args(a);
     t.act = act, t.act_limit = limit, t.act_alpha = alpha;
     tile_gemm_launch(t, i8, s);
+    return launch_status();
+  }
+  if (kind == MoeGemmKind::kTallTiles) {
+    const dim3 tgrid(a.N / 256, (a.max_rows + 255) / 256 + experts);
+    hipLaunchKernelGGL((moe_gemm_tiled_kernel<256, 256, 4, 2, false>), tgrid, dim3(512), 0, s, a);
     return launch_status();
   }
   if (kind == MoeGemmKind::kTiles) {
@@ -916,19 +939,15 @@ int moe_gemm(const hymeta_moe_gemm_args* args, int act, float limit, float alpha
 }  // namespace hymeta
 
 extern "C" int hymeta_moe_gemm_activates(const hymeta_moe_gemm_args* args) {
-  if (!hymeta::args_ok(args)) return HYMETA_ERR_INVALID_ARG;
-  if (args->a_rows != nullptr && args->a_rows_div <= 0) return 0;
-  TileGemmArgs t = hymeta::tile_args(*args);
-  t.act = HYMETA_GEMM_ACT_SILU;
-  return args->local_expert_end > args->local_expert_begin && hymeta::moe_gemm_kind(*args) == hymeta::MoeGemmKind::kBigTiles && tile_gemm_fits(t) ? 1 : 0;
+  return hymeta::moe_gemm_activates(*args, 0) ? 1 : 0;
 }
 
 extern "C" int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t stream) {
-  return hymeta::moe_gemm(args, HYMETA_GEMM_ACT_NONE, 0.f, 0.f, stream);
+  return hymeta::moe_gemm(args, 0, HYMETA_GEMM_ACT_NONE, 0.f, 0.f, stream);
 }
 
 extern "C" int hymeta_moe_gemm_act(const hymeta_moe_gemm_args* args, int32_t act, float limit, float alpha, hymeta_stream_t stream) {
-  return hymeta::moe_gemm(args, act, limit, alpha, stream);
+  return hymeta::moe_gemm(args, 0, act, limit, alpha, stream);
 }
 
 extern "C" int hymeta_silu_and_mul(const void* in, void* out, const int32_t* num_rows_dev, int32_t num_rows,
