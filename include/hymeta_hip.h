@@ -970,6 +970,10 @@ int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t stream);
 enum hymeta_gemm_act { HYMETA_GEMM_ACT_NONE = 0, HYMETA_GEMM_ACT_SILU = 1, HYMETA_GEMM_ACT_SILU_EXACT = 2, HYMETA_GEMM_ACT_CLAMPED_GLU = 3 };
 int hymeta_moe_gemm_act(const hymeta_moe_gemm_args* args, int32_t act, float limit, float alpha, hymeta_stream_t stream);
 int hymeta_moe_gemm_activates(const hymeta_moe_gemm_args* args);
+/* Both for a rank that holds [local_expert_begin, local_expert_end) of num_experts experts, over all of which the max_rows pairs are
+ * spread: the kernel is chosen by the rows that its experts can expect of them (the calls above take all pairs to be theirs). */
+int hymeta_moe_gemm_rank(const hymeta_moe_gemm_args* args, int32_t num_experts, int32_t act, float limit, float alpha, hymeta_stream_t stream);
+int hymeta_moe_gemm_rank_activates(const hymeta_moe_gemm_args* args, int32_t num_experts);
 /* 1 when hymeta_moe_gemm runs a problem of these sizes in the kernel that has the fused combine (K in bf16 elements:
  * pass K / 2 for int8 operands, the choice goes by the bytes of a row). */
 int hymeta_moe_gemm_fuses(int32_t max_rows, int32_t experts, int32_t K, int32_t N);

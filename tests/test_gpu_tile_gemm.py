@@ -91,6 +91,7 @@ def test_grouped_products(sizes, K, N, div, local, act, int8):
     ((200, 140, 160, 141) * 2, 2080, 5120, (0, 8), 0),                           # 160; an odd number of steps
     ((239,) * 8, 2048, 5120, (0, 8), 0),
     ((200, 3, 0, 260, 130, 190, 300, 129, 17), 2112, 5376, (1, 9), 9),           # eight of nine
+    ((20, 80, 0, 300, 75, 129, 5, 64) * 2, 256, 10240, (8, 16), 16),             # a rank's half of 1346 pairs: 84 rows an expert, tiles of 128
 ])
 def test_grouped_products_by_the_rows_of_an_expert(sizes, K, N, local, total):
     from vllm_hymeta import _C
@@ -103,7 +104,7 @@ def test_grouped_products_by_the_rows_of_an_expert(sizes, K, N, local, total):
     a.x, a.weights, a.out, a.expert_offsets = x.data_ptr(), w.data_ptr(), out.data_ptr(), on_card.data_ptr()
     a.a_rows_div, a.max_rows, a.K, a.N, a.x_stride_m, a.out_stride_m, a.w_stride_e = 1, P, K, N, K, N, N * K
     a.local_expert_begin, a.local_expert_end = local
-    assert lib.hymeta_moe_gemm(C.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+    assert lib.hymeta_moe_gemm_rank(C.byref(a), total, NONE, 0.0, 0.0, torch.cuda.current_stream().cuda_stream) == 0
     for e in range(E):
         lo, hi = int(offsets[e]), int(offsets[e + 1])
         want = (x[lo:hi].float() @ w[e].float().t()).bfloat16() if local[0] <= e < local[1] else torch.full_like(out[lo:hi], 7.0)

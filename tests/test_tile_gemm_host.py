@@ -59,3 +59,16 @@ def test_rows_of_x_that_run_backwards():
     b.M, b.K, b.N, b.x_stride_m, b.w_stride_n, b.out_stride_m = 1280, 3584, 37888, -3584, 3584, 18944
     assert lib.hymeta_bf16_gemm_takes(1280, 3584, 37888, 1) == 1
     assert lib.hymeta_bf16_gemm_silu_mul(C.byref(b), None) == unsupported
+
+
+def test_rows_that_a_ranks_experts_can_expect():
+    """8 experts of 14336 x 8192 and 1200 pairs: 150 rows each fill the tiles, 75 each, where 16 share the pairs, do not; from 192 pairs an
+    expert the tiles are used either way, and experts that nearly fill one tile go without the activation."""
+    from vllm_hymeta import _C
+    lib = _C.load()
+    a = _C.MoeGemmArgs()
+    a.K, a.N, a.local_expert_end, a.x_stride_m, a.out_stride_m, a.w_stride_e = 8192, 14336, 8, 8192, 7168, 14336 * 8192
+    for pairs, own, of16 in ((1100, 0, 0), (1200, 1, 0), (1535, 0, 0), (1536, 0, 1), (1919, 0, 1), (1920, 1, 1), (3000, 1, 0), (4000, 1, 1)):
+        a.max_rows = pairs
+        assert (lib.hymeta_moe_gemm_activates(C.byref(a)), lib.hymeta_moe_gemm_rank_activates(C.byref(a), 16)) == (own, of16), pairs
+        assert lib.hymeta_moe_gemm_rank_activates(C.byref(a), 8) == own, pairs

@@ -939,7 +939,7 @@ int moe_gemm(const hymeta_moe_gemm_args* args, int num_experts, int act, float l
 }  // namespace hymeta
 
 extern "C" int hymeta_moe_gemm_activates(const hymeta_moe_gemm_args* args) {
-  return hymeta::moe_gemm_activates(*args, 0) ? 1 : 0;
+  return hymeta_moe_gemm_rank_activates(args, 0);
 }
 
 extern "C" int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t stream) {
@@ -948,6 +948,15 @@ extern "C" int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t
 
 extern "C" int hymeta_moe_gemm_act(const hymeta_moe_gemm_args* args, int32_t act, float limit, float alpha, hymeta_stream_t stream) {
   return hymeta::moe_gemm(args, 0, act, limit, alpha, stream);
+}
+
+extern "C" int hymeta_moe_gemm_rank(const hymeta_moe_gemm_args* args, int32_t num_experts, int32_t act, float limit, float alpha, hymeta_stream_t stream) {
+  return hymeta::moe_gemm(args, num_experts, act, limit, alpha, stream);
+}
+
+extern "C" int hymeta_moe_gemm_rank_activates(const hymeta_moe_gemm_args* args, int32_t num_experts) {
+  if (!hymeta::args_ok(args)) return HYMETA_ERR_INVALID_ARG;
+  return hymeta::moe_gemm_activates(*args, num_experts) ? 1 : 0;
 }
 
 extern "C" int hymeta_silu_and_mul(const void* in, void* out, const int32_t* num_rows_dev, int32_t num_rows,

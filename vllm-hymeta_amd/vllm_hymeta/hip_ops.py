@@ -1492,15 +1492,15 @@ def moe_forward(x: torch.Tensor, router_logits: Optional[torch.Tensor], w13: tor
     g.a_rows, g.a_rows_div, g.max_rows, g.K, g.N = _p(sorted_pair), top_k, P, H, two_i
     g.local_expert_begin, g.local_expert_end = lo, hi
     g.x_stride_m, g.out_stride_m, g.w_stride_e = xin.stride(0), inter, w13.stride(0)
-    activates = lib.hymeta_moe_gemm_activates(C.byref(g)) == 1      # many rows per expert: silu and mul in the GEMM's epilogue
+    activates = lib.hymeta_moe_gemm_rank_activates(C.byref(g), E) == 1      # many rows per expert: silu and mul in the GEMM's epilogue
     if activates:
         hact = torch.empty(P, inter, dtype=torch.bfloat16, device=dev)
         g.out = _p(hact)
-        _C.check(lib.hymeta_moe_gemm_act(C.byref(g), _C.GEMM_ACT_SILU, 0.0, 0.0, st), "hymeta_moe_gemm_act (w13)")
+        _C.check(lib.hymeta_moe_gemm_rank(C.byref(g), E, _C.GEMM_ACT_SILU, 0.0, 0.0, st), "hymeta_moe_gemm_rank (w13)")
     else:
         h13 = torch.empty(P, two_i, dtype=torch.bfloat16, device=dev)
         g.out, g.out_stride_m = _p(h13), h13.stride(0)
-        _C.check(lib.hymeta_moe_gemm(C.byref(g), st), "hymeta_moe_gemm (w13)")
+        _C.check(lib.hymeta_moe_gemm_rank(C.byref(g), E, _C.GEMM_ACT_NONE, 0.0, 0.0, st), "hymeta_moe_gemm_rank (w13)")
 
     if shared is not None:
         _require(shared.shape == (T, H) and shared.dtype == torch.bfloat16 and shared.stride(1) == 1,
@@ -1530,7 +1530,7 @@ def moe_forward(x: torch.Tensor, router_logits: Optional[torch.Tensor], w13: tor
         d.combine_tokens = _p(sorted_pair)       # one choice per token: the pair index is the token
         if shared is not None:
             d.combine_shared, d.combine_shared_stride_m = _p(shared), shared.stride(0)
-    _C.check(lib.hymeta_moe_gemm(C.byref(d), st), "hymeta_moe_gemm (w2)")
+    _C.check(lib.hymeta_moe_gemm_rank(C.byref(d), E, _C.GEMM_ACT_NONE, 0.0, 0.0, st), "hymeta_moe_gemm_rank (w2)")
     if fuse_combine:
         return out
 
