@@ -72,3 +72,15 @@ def test_rows_that_a_ranks_experts_can_expect():
         a.max_rows = pairs
         assert (lib.hymeta_moe_gemm_activates(C.byref(a)), lib.hymeta_moe_gemm_rank_activates(C.byref(a), 16)) == (own, of16), pairs
         assert lib.hymeta_moe_gemm_rank_activates(C.byref(a), 8) == own, pairs
+
+
+@pytest.mark.parametrize("M,K,N,takes", [
+    (896, 3584, 37888, 1), (2048, 3584, 37888, 1), (3328, 3584, 37888, 1), (700, 3584, 37888, 0), (4097, 3584, 37888, 0),      # 513 to 2048 tiles
+    (1030, 256, 32768, 1), (2307, 320, 14336, 1), (8192, 960, 6144, 1),      # a short K
+    (2048, 8192, 57344, 0), (1280, 5120, 27648, 0),                          # a long one
+    (800, 1600, 35072, 0), (1024, 1600, 35072, 1),                           # rows that leave a fifth of the rounds empty
+    (5000, 3584, 7168, 0),                                                   # few columns
+])
+def test_gate_up_projections_that_run_in_tiles(M, K, N, takes):
+    from vllm_hymeta import _C
+    assert _C.load().hymeta_bf16_gemm_takes(M, K, N, 1) == takes

@@ -165,17 +165,24 @@ extern "C" size_t hymeta_bf16_gemm_workspace_bytes(int32_t M, int32_t N, int32_t
 }
 
 // The gate / up projection of a prompt in tiles (tile_gemm.hip), from two to eight rounds of tiles, us against the library's
-// product and the activation's launch, 7B: 896 rows 239 / 300, 1280 281 / 391, 2048 462 / 556, 3328 729 / 846.  Below, the library
+// product and the activation's launch, 37888 x 3584: 896 rows 223 / 291, 1280 277 / 385, 2048 444 / 548, 3328 701 / 813.  Below, the library
 // cuts K: 768 rows 189 / 186, 512 164 / 152.  Above, its product fills the chip as well: alone 4096 rows 879 / 893 and 8192
-// 1713 / 1826, but a whole prompt of 4096 7466 / 7375, of 8192 13877 / 13990.
+// 1713 / 1826, but a whole prompt of 4096 7466 / 7375, of 8192 13877 / 13990.  Over 840 sizes of 92 matrices: from a K of 4096 on the
+// library reaches 1.3 to 1.4 PFLOP/s on many that the tiles do not (57344 x 8192 at 2048 rows 1375 / 1304, 32000 x 5184 at 1113 1.08 of its time), and
+// where rows and rounds are left a fifth empty, of a long K a third (45312 x 4864 at 520 1.13, 35072 x 1600 at 800 1.12, 11264 x 2048 at 2900
+// 1.05), or the columns are few (7168 x 3584 at 5000 228 / 218); the rest are 0.65 to 1.03 of it, 0.87 on average.  A K below 1024 is the
+// epilogue's.
 static TileGemmArgs gated_tile_args(int32_t M, int32_t K, int32_t N) {
   TileGemmArgs t = {};
   t.x_stride = static_cast<int64_t>(K) * 2, t.out_stride = N / 2, t.a_rows_div = 1, t.max_rows = M, t.N = N, t.k_bytes = K * 2, t.act = HYMETA_GEMM_ACT_SILU;
   return t;
 }
 static bool gated_tiles(int32_t M, int32_t K, int32_t N) {
-  const int64_t tiles = static_cast<int64_t>(N / 256) * ((static_cast<int64_t>(M) + 255) / 256);
-  return tiles > 512 && tiles <= 2048 && tile_gemm_fits(gated_tile_args(M, K, N));
+  const int64_t tiles = static_cast<int64_t>(N / 256) * ((static_cast<int64_t>(M) + 255) / 256), units = 256, rest = tiles % units;
+  if (tiles <= 512 || tiles > 2048 || K >= 4096 || !tile_gemm_fits(gated_tile_args(M, K, N))) return false;
+  if (K < 1024) return true;
+  const int64_t tenths = tiles / units * 10 + (rest == 0 ? 0 : rest <= units / 2 ? 6 : 10);      // of a round (a last one of halves: 0.6)
+  return N >= 9216 && 1000 * static_cast<int64_t>(M) * N >= (K >= 3584 ? 66 : 80) * tenths * units * 65536;
 }
 
 // A product whose K is cut (tile_gemm_slices has the rule and what it measured).

@@ -1150,7 +1150,8 @@ def w8a8_gemm(x: torch.Tensor, qweight: torch.Tensor, w_scale: torch.Tensor,
 
 def gemm_silu_mul_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Shapes the gate/up projection with the activation in its epilogue takes: decode-sized batches of a bf16
-    ``[2 I, K]`` weight (gate rows, then up rows) and prompts of 513 to 2048 tiles, any batch of an int8 one."""
+    ``[2 I, K]`` weight (gate rows, then up rows) and prompts of 513 to 2048 tiles of 256 x 256 where the library's product is
+    slower (``hymeta_bf16_gemm_takes``), any batch of an int8 one."""
     esize = 1 if weight.dtype == torch.int8 else 2
     if not (x.dim() == 2 and 0 < x.shape[0] < 1 << 30 and x.is_cuda and x.dtype == torch.bfloat16
             and weight.dtype in (torch.bfloat16, torch.int8) and x.stride(1) == 1 and weight.is_contiguous()
@@ -1166,8 +1167,7 @@ def gemm_silu_mul_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 def gemm_silu_mul(x: torch.Tensor, weight: torch.Tensor, w_scale: Optional[torch.Tensor] = None,
                   out: Optional[torch.Tensor] = None, exact: bool = False) -> torch.Tensor:
-    """``silu(x gate^T) * (x up^T)`` in one launch: x bf16 [M, K]; weight [2 I, K] bf16 (M <= 128, wide ones to 256, prompts of
-    513 to 2048 tiles), or int8 with ``w_scale``
+    """``silu(x gate^T) * (x up^T)`` in one launch: x bf16 [M, K]; weight [2 I, K] bf16 (``gemm_silu_mul_supported``), or int8 with ``w_scale``
     fp32 [2 I] (dynamic per-token int8 activations; any M) -> bf16 [M, I].  Bit for bit the linear followed by
     ``silu_and_mul``, or for ``exact`` (bf16 prompts only) by ``silu_mul``."""
     _dev(x, weight, w_scale, out)
