@@ -174,7 +174,12 @@ def test_gated_block_of_a_prompt(M):
         assert torch.equal(hip_ops.gemm_silu_mul(x, w, exact=True), want) and torch.equal(hip_ops.gemm_silu_mul(x, w), fast)
 
 
-@pytest.mark.parametrize("M,N,K", [(1030, 4608, 512), (300, 16384, 640), (5000, 1024, 1024)])
+@pytest.mark.parametrize("M,N,K", [
+    (1030, 4608, 512), (300, 16384, 640), (5000, 1024, 1024),
+    (1024, 4096, 512), (1025, 4096, 512),        # a tile of 128 x 128 for every unit, and more
+    (640, 11264, 512), (1025, 11264, 512),       # more large tiles than are cut in halves, small ones for every place, and more
+    (400, 8192, 3072), (300, 9472, 3072),        # halves with an activation behind a longer K
+])
 @pytest.mark.parametrize("gated", [False, True])
 def test_w8a8_linear_of_a_prompt(M, N, K, gated):
     """Exact int32 sums, (sum * x_scale) * w_scale + bias in one fused step, one rounding: powers of two keep all of it exact

@@ -1093,10 +1093,16 @@ __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void w8a8_tiled
 constexpr int kW8A8TiledFromRows = 129;
 static bool w8a8_tiled_fits(int M, int K, int N) { return M >= kW8A8TiledFromRows && K % kI8StepBytes == 0 && N % 128 == 0; }
 
-// Tiles of 256 x 256 (tile_gemm.hip) once there are enough of them or of their halves to fill the chip, 128 x 128 (4 waves of
-// 64 x 64) below: 3584 -> 3584 columns, us without the quantisation, 1536 rows (84 tiles) 38 -> 34, 1024 (56) 26 against 32;
-// gate / up 1024 rows 172 -> 138, 8192 1167 -> 978, the down projection of 8192 rows 518 -> 412.
-constexpr int kW8A8TileFrom = 64;
+// Tiles of 256 x 256 (tile_gemm.hip; halves of them up to 128) or of 128 x 128 (4 waves of 64 x 64, two workgroups on a compute unit),
+// us without the quantisation.  The small ones are sooner while every unit has at most one of them (1024 rows of 4096 x 4096, 256: 37
+// against 42; 2048 x 2048 at 2048 25 / 28), and where the large ones are too many to be cut and the small ones still go at once (gate / up of
+// 18944 x 3584 at 300 rows, 148 and 444: 43 / 53; 11264 x 2048 at 640 30 / 39); of short rows the halves' epilogue with an activation takes
+// longer (16384 x 2048 at 257 27 / 29).  Else the large ones: 3584 x 3584 at 1536 rows 43 -> 41, 4096 x 11008 at 2048 120 -> 97, gate / up of
+// 9472 x 3584 at 512 42 -> 40 and at 769 61 -> 54, of 37888 x 3584 at 8192 1167 -> 978.
+static bool w8a8_large_tiles(int M, int K, int N, bool gated) {
+  const int64_t large = static_cast<int64_t>((M + 255) / 256) * (N / 256), small = static_cast<int64_t>((M + 127) / 128) * (N / 128);
+  return small > 512 || (small > 256 && large <= 128 && (!gated || K >= 3072));
+}
 
 template <bool GATED>
 static void w8a8_tiled_launch(const hymeta_w8a8_gemm_args& a, hipStream_t s) {
@@ -1105,8 +1111,7 @@ static void w8a8_tiled_launch(const hymeta_w8a8_gemm_args& a, hipStream_t s) {
   t.x_scale = a.x_scale, t.w_scale = a.w_scale, t.bias = static_cast<const uint16_t*>(a.bias);
   t.x_stride = a.K, t.out_stride = a.out_stride_m, t.a_rows_div = 1, t.max_rows = a.M, t.N = a.N, t.k_bytes = a.K;
   t.act = GATED ? HYMETA_GEMM_ACT_SILU : HYMETA_GEMM_ACT_NONE;
-  const int64_t tiles = static_cast<int64_t>(a.N / 256) * ((a.M + 255) / 256);
-  if (tiles >= kW8A8TileFrom && reinterpret_cast<uintptr_t>(a.bias) % 4 == 0 && tile_gemm_fits(t)) tile_gemm_launch(t, true, s);
+  if (w8a8_large_tiles(a.M, a.K, a.N, GATED) && reinterpret_cast<uintptr_t>(a.bias) % 4 == 0 && tile_gemm_fits(t)) tile_gemm_launch(t, true, s);
   else hipLaunchKernelGGL((w8a8_tiled_kernel<128, 128, 2, 2, GATED>), dim3(a.N / 128, (a.M + 127) / 128), dim3(256), 0, s, a);
 }
 
