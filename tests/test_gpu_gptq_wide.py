@@ -20,6 +20,7 @@ pytestmark = pytest.mark.gpu
     (37888, 512, 128, 128, False, True),      # two rounds
     (32768, 512, 128, 64, True, True),        # whole rounds of 128 columns
     (41088, 512, 128, 64, True, False),       # one tile of 160 too many: 128 columns and slices
+    (57344, 512, 64, 65, True, True),         # three rounds of 160 in place of three and a half: 128 columns and slices
     # up to 16 rows, tiles of 80: the last one with 48, 64, 32, 16 and all of its columns
     (37888, 512, 128, 1, True, True),
     (33024, 1152, 64, 16, False, False),      # an odd number of groups a wave
