@@ -36,6 +36,10 @@ def _activate(h, act):
     ((2600,), 1024, 5120, 1, (0, 1), NONE, True),                                    # more row tiles than a block of neighbours holds
     ((5, 900), 256, 10240, 1, (0, 1), SILU, False),                                  # halves that hold no rows
     ((2600, 1300), 448, 2560, 3, (0, 2), NONE, False),
+    ((8500, 3, 700), 256, 1280, 1, (0, 3), NONE, False),                             # more row tiles than the columns are swept once for
+    ((16640, 300), 512, 1536, 1, (0, 2), SILU, True),                                # three sweeps of one expert, the last of one row tile
+    ((128, 140, 0, 126, 150, 257, 1, 250) * 8, 256, 1024, 1, (0, 64), NONE, False),  # an expert for every lane
+    ((128, 140, 0, 126, 150, 257, 1, 250) * 8, 512, 1024, 2, (3, 61), SILU, True),
 ])
 def test_grouped_products(sizes, K, N, div, local, act, int8):
     from vllm_hymeta import _C
@@ -179,6 +183,7 @@ def test_gated_block_of_a_prompt(M):
     (1024, 4096, 512), (1025, 4096, 512),        # a tile of 128 x 128 for every unit, and more
     (640, 11264, 512), (1025, 11264, 512),       # more large tiles than are cut in halves, small ones for every place, and more
     (400, 8192, 3072), (300, 9472, 3072),        # halves with an activation behind a longer K
+    (8493, 1024, 512), (16641, 1024, 512),       # row tiles of two and of three sweeps over the columns
 ])
 @pytest.mark.parametrize("gated", [False, True])
 def test_w8a8_linear_of_a_prompt(M, N, K, gated):
