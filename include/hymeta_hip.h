@@ -875,8 +875,8 @@ typedef struct hymeta_moe_route_args {
   const void* router_logits;   /* logits_dtype [num_tokens, num_experts] */
   int32_t* topk_ids;           /* out [num_tokens, top_k] */
   float* topk_weights;         /* out [num_tokens, top_k] */
-  int32_t* counts;             /* scratch [num_experts] */
-  int32_t* cursors;            /* scratch [num_experts] */
+  int32_t* counts;             /* not read or written any more; must not be NULL */
+  int32_t* cursors;            /* likewise */
   int32_t* expert_offsets;     /* out [num_experts + 1] */
   int32_t* sorted_pair;        /* out [num_tokens * top_k] */
   int32_t* pair_pos;           /* out [num_tokens * top_k] */

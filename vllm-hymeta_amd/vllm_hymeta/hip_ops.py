@@ -1401,8 +1401,7 @@ def moe_forward(x: torch.Tensor, router_logits: Optional[torch.Tensor], w13: tor
     P = T * top_k
     ids = torch.empty(T, top_k, dtype=torch.int32, device=dev)
     wts = torch.empty(T, top_k, dtype=torch.float32, device=dev)
-    meta = torch.empty(3 * (E + 1), dtype=torch.int32, device=dev)
-    counts, cursors, offsets = meta[: E + 1], meta[E + 1: 2 * (E + 1)], meta[2 * (E + 1):]
+    offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
     sorted_pair = torch.empty(max(P, 1), dtype=torch.int32, device=dev)
     pair_pos = torch.empty(max(P, 1), dtype=torch.int32, device=dev)
     if out is None:
@@ -1431,7 +1430,7 @@ def moe_forward(x: torch.Tensor, router_logits: Optional[torch.Tensor], w13: tor
     else:
         r = _C.MoeRouteArgs()
         r.router_logits, r.topk_ids, r.topk_weights = _p(router_logits), _p(ids), _p(wts)
-        r.counts, r.cursors, r.expert_offsets = _p(counts), _p(cursors), _p(offsets)
+        r.counts = r.cursors = r.expert_offsets = _p(offsets)          # (the first two are not used any more)
         r.sorted_pair, r.pair_pos = _p(sorted_pair), _p(pair_pos)
         r.num_tokens, r.num_experts, r.top_k, r.renormalize = T, E, top_k, int(bool(renormalize))
         r.logits_dtype = _DT[router_logits.dtype]
