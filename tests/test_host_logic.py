@@ -247,3 +247,14 @@ def test_partial_sums_go_into_the_exchange_only_where_the_message_fits(monkeypat
     assert parallel.defers_into_all_reduce("exchange") and parallel.defers_into_all_reduce("exchange", 4096)
     assert not parallel.defers_into_all_reduce("exchange", 4097)
     assert not parallel.defers_into_all_reduce("library", 16) and not parallel.defers_into_all_reduce(None, 16)
+
+
+@pytest.mark.parametrize("rows,K,N,library", [
+    (2048, 18944, 3584, True), (2049, 18944, 3584, False),                             # deep, many columns
+    (2049, 8192, 1024, True), (4095, 8192, 1024, True), (4096, 8192, 1024, False),     # few
+    (2049, 6144, 1536, False), (3000, 7680, 1920, True), (4096, 7680, 1920, False),    # whole tiles of 256, or not
+    (1023, 3584, 4608, True), (1024, 3584, 4608, False), (300, 3584, 37888, False),
+])
+def test_w8a8_prompts_that_the_library_has_sooner(rows, K, N, library):
+    from vllm_hymeta.linear import w8a8_use_library
+    assert w8a8_use_library(rows, K, N) == library

@@ -28,11 +28,13 @@ def w8a8_use_library(rows: int, in_features: int, out_features: int) -> bool:
     """Above the streaming kernels' rows a W8A8 linear is either ONE tiled int8-MFMA launch with the scales in its
     epilogue (``hymeta_w8a8_gemm``: K in whole 128-deep steps, N in whole 128-column tiles) or quantise -> library int8
     GEMM -> scale (three launches, the int32 sums through memory); both give the same bits.  The tiled kernel takes the
-    shapes where it was measured ahead (7B shapes, us, tiled / library): gate_up 70 / 72 at 129 rows, 68 / 101 at 256,
-    271 / 412 at 2048, 3920 / 5568 at 32768 (up to 256 rows the streaming kernel has since taken over: 59 at 256, the
-    down projection 48 against 118); qkv 57 / 71 at 2048; o 45 / 57; the deep
-    narrow down projection (K = 5.3 N: few tiles, long K loops) 247 / 299 at 4096, 496 / 683 at 8192 -- and leaves the
-    rest to the library (qkv / o below 1024 rows; down to 2048 rows, where 157 / 173 would be ahead but 1024 are 147 / 104)."""
+    shapes where it was measured ahead (7B shapes, the quantisation included, weights from memory, us on the GPU, tiled /
+    library): gate_up 92 / 101 at 257 rows, 160 / 239 at 1024, 297 / 407 at 2048, 4042 / 5788 at 32768; qkv 42 / 45 at 1024,
+    60 / 69 at 2048, 585 / 755 at 32768; o 34 / 34 at 1024, 45 / 52 at 2048; the deep narrow down projection (K = 5.3 N: few
+    tiles, long K loops) 256 / 258 at 3072, 285 / 319 at 4096, 551 / 676 at 8192 -- and leaves the rest to the library: qkv / o
+    below 1024 rows (o 28.6 / 22.1 at 257, 32.0 / 32.4 at 768), down up to 2048 (119 / 66 at 257, 138 / 117 at 1024, 181 / 191 at
+    2048) and below 4096 where it has few columns or they are no whole tiles of 256 (2049 rows: 512 x 4096 36 / 27, 1024 x 8192
+    64 / 55, but 1536 x 8960 72 / 81; 2817 rows: 1920 x 7680 93 / 82; 2048 x 8192 82 / 88).  Up to 256 rows the streaming kernels run: 52 / 93 for gate_up, 45 / 57 for down, 27 / 24 and 26 / 19 for qkv and o."""
     if rows <= W8A8_STREAM_ROWS:
         return False
     if in_features % 128 != 0 or out_features % 128 != 0:
@@ -42,7 +44,7 @@ def w8a8_use_library(rows: int, in_features: int, out_features: int) -> bool:
     if out_features >= 16384:
         return False
     if in_features >= 4 * out_features:
-        return rows <= 2048
+        return rows <= 2048 or (rows < 4096 and (out_features < 1536 or out_features % 256 != 0))
     return rows < 1024
 
 
