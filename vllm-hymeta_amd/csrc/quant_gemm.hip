@@ -945,23 +945,23 @@ __global__ __launch_bounds__(256) void w8a8_gemm_kernel(hymeta_w8a8_gemm_args a,
 // W8A8 at prefill-sized row counts: out = bf16( (xq wq^T) * x_scale[m] * w_scale[n] + bias ) as ONE tiled launch.
 // The library path it replaces runs an int8 GEMM that writes its int32 sums to memory and a second launch that reads
 // them back to scale them: 10 bytes of traffic per output element that this kernel never makes.
-// 128 rows x 128 columns per workgroup, four waves that own 64 x 64 each, v_mfma_i32_16x16x64_i8.  Both
+// BM rows x BN columns per workgroup, WM x WN waves that own (BM / WM) x (BN / WN) each, v_mfma_i32_16x16x64_i8.  Both
 // operands are K-contiguous int8; a 128-deep step of each (128 bytes per row) is staged once per workgroup through
 // double-buffered LDS images (16-byte chunks XOR-ed with the row, so the sixteen rows of a fragment read hit distinct
 // banks): registers -> LDS right behind the barrier that frees the buffer, the next step's loads issued at once.  The
 // epilogue applies the scales to the exact int32 sums with the rounding rule of every W8A8 kernel here (w8a8_scaled),
-// stages the bf16 tile through LDS and stores whole rows.  grid = (N / 128, ceil(M / 128)), column tiles fastest: the
+// stages the bf16 tile through LDS and stores whole rows.  grid = (N / BN, ceil(M / BM)), column tiles fastest: the
 // workgroups that share a row tile of x run together.
-// GATED (a fused gate / up projection, weight rows = gate, then up): the tile's first 64 weight rows are gate rows
-// and the other half the up rows of the same output columns, so the staged bf16 tile holds both factors of 64 output
+// GATED (a fused gate / up projection, weight rows = gate, then up): the tile's first BN / 2 weight rows are gate rows
+// and the other half the up rows of the same output columns, so the staged bf16 tile holds both factors of BN / 2 output
 // columns side by side and the store pass writes silu(bf16 gate) * bf16 up -- the bits of this kernel followed by
 // silu_and_mul, without the [M, N] intermediate (2.5 GB written and read back at 32768 rows of the 7B MLP).
 // ---------------------------------------------------------------------------------------------
 constexpr int kI8StepBytes = 128;                  // bytes of one staged row = 128 k
 
-template <bool GATED>
-__global__ __launch_bounds__(256, 2) void w8a8_tiled_kernel(hymeta_w8a8_gemm_args a) {
-  constexpr int BM = 128, BN = 128, WM = 2, WN = 2, kThreads = 64 * WM * WN;
+template <int BM, int BN, int WM, int WN, bool GATED>
+__global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void w8a8_tiled_kernel(hymeta_w8a8_gemm_args a) {
+  constexpr int kThreads = 64 * WM * WN;
   constexpr int MT = BM / WM / 16, NT = BN / WN / 16;       // 16 x 16 tiles per wave
   constexpr int kXBytes = BM * kI8StepBytes, kWBytes = BN * kI8StepBytes;
   constexpr int kRowsPerPass = kThreads / 8;
@@ -1041,9 +1041,11 @@ __global__ __launch_bounds__(256, 2) void w8a8_tiled_kernel(hymeta_w8a8_gemm_arg
   }
 
   // acc[mt][nt][r] = C[row 16 MT wm + 16 mt + 4c + r][col 16 NT wn + 16 nt + n]: scales and bias on the exact int32 sums,
-  // one rounding, staged through LDS (the operand images are free) and stored as whole rows
+  // one rounding, staged through LDS (the operand images are free) 128 rows at a time and stored as whole rows
   constexpr int kCPitch = 2 * BN + 16;
-  static_assert(BM * kCPitch <= 2 * (kXBytes + kWBytes), "output staging fits the operand images");
+  constexpr int kStageRows = BM < 128 ? BM : 128;
+  static_assert(kStageRows * kCPitch <= 2 * (kXBytes + kWBytes), "output staging fits the operand images");
+  static_assert(kStageRows % (16 * MT) == 0 && BM % kStageRows == 0, "a wave's rows fall into one staging pass");
   char* cst = &sm[0][0];
   float wsc[NT], bia[NT];
 #pragma unroll
@@ -1053,31 +1055,37 @@ __global__ __launch_bounds__(256, 2) void w8a8_tiled_kernel(hymeta_w8a8_gemm_arg
     bia[nt] = a.bias != nullptr ? bf2f(static_cast<const uint16_t*>(a.bias)[col]) : 0.f;
   }
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+  for (int half = 0; half < BM / kStageRows; ++half) {
+    if ((16 * MT * wm) / kStageRows == half) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * MT * wm + 16 * mt + 4 * c + r;
-      const float xs = a.x_scale[min(row0 + row, a.M - 1)];
-      uint16_t* crow = reinterpret_cast<uint16_t*>(cst + row * kCPitch) + 16 * NT * wn + n;
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) crow[16 * nt] = f2bf(w8a8_scaled(acc[mt][nt][r], xs, wsc[nt], bia[nt]));
+        for (int r = 0; r < 4; ++r) {
+          const int row = 16 * MT * wm + 16 * mt + 4 * c + r;
+          const float xs = a.x_scale[min(row0 + row, a.M - 1)];
+          uint16_t* crow = reinterpret_cast<uint16_t*>(cst + (row - kStageRows * half) * kCPitch) + 16 * NT * wn + n;
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) crow[16 * nt] = f2bf(w8a8_scaled(acc[mt][nt][r], xs, wsc[nt], bia[nt]));
+        }
     }
-  __syncthreads();
-  constexpr int kChunksPerRow = (GATED ? BN / 2 : BN) / 8;      // 8-column pieces of a row of the output tile
-  for (int id = tid; id < BM * kChunksPerRow; id += kThreads) {
-    const int row = id / kChunksPerRow, ch = id % kChunksPerRow;
-    const int grow = row0 + row;
-    if (grow >= a.M) continue;
-    u32x4 o = ld16(cst + row * kCPitch + 16 * ch);
-    if constexpr (GATED) {
-      const u32x4 up = ld16(cst + row * kCPitch + BN + 16 * ch);    // the up factors sit BN / 2 columns on
+    __syncthreads();
+    constexpr int kChunksPerRow = (GATED ? BN / 2 : BN) / 8;      // 8-column pieces of a row of the output tile
+    for (int id = tid; id < kStageRows * kChunksPerRow; id += kThreads) {
+      const int row = id / kChunksPerRow, ch = id % kChunksPerRow;
+      const int grow = row0 + kStageRows * half + row;
+      if (grow >= a.M) continue;
+      u32x4 o = ld16(cst + row * kCPitch + 16 * ch);
+      if constexpr (GATED) {
+        const u32x4 up = ld16(cst + row * kCPitch + BN + 16 * ch);    // the up factors sit BN / 2 columns on
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float g0 = lo_bf(o[e]), g1 = hi_bf(o[e]);
-        o[e] = pack_bf16x2(g0 * sigmoidf(g0) * lo_bf(up[e]), g1 * sigmoidf(g1) * hi_bf(up[e]));
+        for (int e = 0; e < 4; ++e) {
+          const float g0 = lo_bf(o[e]), g1 = hi_bf(o[e]);
+          o[e] = pack_bf16x2(g0 * sigmoidf(g0) * lo_bf(up[e]), g1 * sigmoidf(g1) * hi_bf(up[e]));
+        }
       }
+      st16(static_cast<uint16_t*>(a.out) + static_cast<int64_t>(grow) * a.out_stride_m + col0 + 8 * ch, o);
     }
-    st16(static_cast<uint16_t*>(a.out) + static_cast<int64_t>(grow) * a.out_stride_m + col0 + 8 * ch, o);
+    if (half + 1 < BM / kStageRows) __syncthreads();
   }
 }
 
@@ -1104,7 +1112,7 @@ static void w8a8_tiled_launch(const hymeta_w8a8_gemm_args& a, hipStream_t s) {
   t.x_stride = a.K, t.out_stride = a.out_stride_m, t.a_rows_div = 1, t.max_rows = a.M, t.N = a.N, t.k_bytes = a.K;
   t.act = GATED ? HYMETA_GEMM_ACT_SILU : HYMETA_GEMM_ACT_NONE;
   if (w8a8_large_tiles(a.M, a.K, a.N, GATED) && reinterpret_cast<uintptr_t>(a.bias) % 4 == 0 && tile_gemm_fits(t)) tile_gemm_launch(t, true, s);
-  else hipLaunchKernelGGL(w8a8_tiled_kernel<GATED>, dim3(a.N / 128, (a.M + 127) / 128), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((w8a8_tiled_kernel<128, 128, 2, 2, GATED>), dim3(a.N / 128, (a.M + 127) / 128), dim3(256), 0, s, a);
 }
 
 }  // namespace hymeta
