@@ -182,8 +182,13 @@ def test_gated_block_of_a_prompt(M):
     (1030, 4608, 512), (300, 16384, 640), (5000, 1024, 1024),
     (1024, 4096, 512), (1025, 4096, 512),        # a tile of 128 x 128 for every unit, and more
     (640, 11264, 512), (1025, 11264, 512),       # more large tiles than are cut in halves, small ones for every place, and more
-    (400, 8192, 3072), (300, 9472, 3072),        # halves with an activation behind a longer K
+    (400, 8192, 3072), (300, 9472, 3072),        # a longer K, few rows
+    (600, 8192, 3072),                           # halves with an activation
     (8493, 1024, 512), (16641, 1024, 512),       # row tiles of two and of three sweeps over the columns
+    (1025, 4096, 2048), (520, 14336, 3072),      # a K that pays for the large tiles
+    (300, 50944, 512), (500, 50944, 512),        # half-empty large tiles, and nearly filled ones
+    (150, 50944, 512), (256, 49152, 640),        # one row tile: eight waves
+    (200, 12544, 3072), (130, 49280, 512),       # ... too few of them, and columns that are no whole tiles
 ])
 @pytest.mark.parametrize("gated", [False, True])
 def test_w8a8_linear_of_a_prompt(M, N, K, gated):

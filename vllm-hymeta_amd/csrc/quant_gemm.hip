@@ -1093,15 +1093,25 @@ __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void w8a8_tiled
 constexpr int kW8A8TiledFromRows = 129;
 static bool w8a8_tiled_fits(int M, int K, int N) { return M >= kW8A8TiledFromRows && K % kI8StepBytes == 0 && N % 128 == 0; }
 
-// Tiles of 256 x 256 (tile_gemm.hip; halves of them up to 128) or of 128 x 128 (4 waves of 64 x 64, two workgroups on a compute unit),
-// us without the quantisation.  The small ones are sooner while every unit has at most one of them (1024 rows of 4096 x 4096, 256: 37
-// against 42; 2048 x 2048 at 2048 25 / 28), and where the large ones are too many to be cut and the small ones still go at once (gate / up of
-// 18944 x 3584 at 300 rows, 148 and 444: 43 / 53; 11264 x 2048 at 640 30 / 39); of short rows the halves' epilogue with an activation takes
-// longer (16384 x 2048 at 257 27 / 29).  Else the large ones: 3584 x 3584 at 1536 rows 43 -> 41, 4096 x 11008 at 2048 120 -> 97, gate / up of
-// 9472 x 3584 at 512 42 -> 40 and at 769 61 -> 54, of 37888 x 3584 at 8192 1167 -> 978.
-static bool w8a8_large_tiles(int M, int K, int N, bool gated) {
+// Tiles of 256 x 256 of tile_gemm.hip (halves of them up to 128), of this kernel's eight waves (kTall), or of 128 x 128 (4 waves of 64 x 64,
+// two workgroups on a compute unit); us with weights from memory, the quantisation included.  The small ones are sooner
+//  * while every unit has at most one of them (1024 rows of 4096 x 4096, 256: 37 against 42 of the large; 2048 x 2048 at 2048 25 / 28);
+//  * while they go at once where the large ones are too many to be cut (gate / up of 18944 x 3584 at 300 rows, 148 and 444: 43 / 53), or
+//    where the rows are few, so that the halves leave units idle (gate / up of 11264 x 3072 at 300 35 / 39, of 9472 x 3072 at 400 36 / 39);
+//  * with a short K, whose steps do not pay for the large ones' beginning and end, while these leave units idle (4096 x 768 at 1025 15 / 17, x 2048
+//    level, x 4096 45 / 42; gate / up of 14336 x 768 at 520 22 / 25, x 2048 level; 41984 x 2048 at 148 40 / 43) or are three quarters filled at most (50944 x 1024 at 300 42 / 53).
+// Eight waves: one row tile, every weight is fetched once, and rows held in registers keep more of them in flight than copies to LDS
+// (57344 x 3584 at 200 rows 60 against 68, gate / up 64 / 71; x 8192 127 / 136); and of a short K, whose few steps the copies do not get ahead
+// of (43776 x 512 at 4078 179 / 208, 46592 x 768 at 4346 264 / 277).  Else the large ones of tile_gemm.hip: 3584 x 3584 at 1536
+// rows 43 -> 41, 4096 x 11008 at 2048 120 -> 97, gate / up of 9472 x 3584 at 769 61 -> 54, of 37888 x 3584 at 8192 1167 -> 978.
+enum class W8A8Tiles { kSmall, kTall, kLarge };
+static W8A8Tiles w8a8_tiles(int M, int K, int N, bool gated) {
+  if (N % 256 != 0) return W8A8Tiles::kSmall;
   const int64_t large = static_cast<int64_t>((M + 255) / 256) * (N / 256), small = static_cast<int64_t>((M + 127) / 128) * (N / 128);
-  return small > 512 || (small > 256 && large <= 128 && (!gated || K >= 3072));
+  const bool deep = K >= (M <= 256 ? 3584 : gated ? 3072 : 2048);
+  if (large >= 192) return M <= 256 || K < 1024 ? W8A8Tiles::kTall : deep || 4 * static_cast<int64_t>(M) * N >= 3 * large * 65536 ? W8A8Tiles::kLarge : W8A8Tiles::kSmall;
+  if (!deep || small <= 256) return W8A8Tiles::kSmall;
+  return small > 512 || (large <= 128 && M > 512) ? W8A8Tiles::kLarge : W8A8Tiles::kSmall;
 }
 
 template <bool GATED>
@@ -1111,7 +1121,10 @@ static void w8a8_tiled_launch(const hymeta_w8a8_gemm_args& a, hipStream_t s) {
   t.x_scale = a.x_scale, t.w_scale = a.w_scale, t.bias = static_cast<const uint16_t*>(a.bias);
   t.x_stride = a.K, t.out_stride = a.out_stride_m, t.a_rows_div = 1, t.max_rows = a.M, t.N = a.N, t.k_bytes = a.K;
   t.act = GATED ? HYMETA_GEMM_ACT_SILU : HYMETA_GEMM_ACT_NONE;
-  if (w8a8_large_tiles(a.M, a.K, a.N, GATED) && reinterpret_cast<uintptr_t>(a.bias) % 4 == 0 && tile_gemm_fits(t)) tile_gemm_launch(t, true, s);
+  const W8A8Tiles tiles = w8a8_tiles(a.M, a.K, a.N, GATED);
+  if (tiles == W8A8Tiles::kLarge && reinterpret_cast<uintptr_t>(a.bias) % 4 == 0 && tile_gemm_fits(t)) tile_gemm_launch(t, true, s);
+  else if (tiles == W8A8Tiles::kTall)
+    hipLaunchKernelGGL((w8a8_tiled_kernel<256, 256, 4, 2, GATED>), dim3(a.N / 256, (a.M + 255) / 256), dim3(512), 0, s, a);
   else hipLaunchKernelGGL((w8a8_tiled_kernel<128, 128, 2, 2, GATED>), dim3(a.N / 128, (a.M + 127) / 128), dim3(256), 0, s, a);
 }
 
