@@ -747,7 +747,7 @@ int hymeta_advance_step(int32_t num_seqs, int32_t num_queries, int32_t block_siz
  * (vllm_hymeta/model_for_7B/modeling_gla_swa.py:108-121, vllm_hymeta/models/modeling_hymeta.py:262-271).
  * bias must be NULL, the workspace fields are ignored.  Takes M <= 128, K % 64 == 0, N % 128 == 0, and from 129 to
  * 256 rows the shapes for which hymeta_bf16_gemm_takes(M, K, N, 1) says so (matrices wide enough for 128 whole tiles); with
- * more rows likewise (513 to 2048 tiles of 256 x 256, K < 4096; then w_stride_n == K, and x within 4 GiB);
+ * more rows likewise (513 to 2048 tiles of 256 x 256, K <= 3712; then w_stride_n == K, and x within 4 GiB);
  * other shapes are HYMETA_ERR_UNSUPPORTED: run the two calls. */
 int hymeta_bf16_gemm_silu_mul(const hymeta_bf16_gemm_args* args, hymeta_stream_t stream);
 /* The same for more than 256 rows with the activation of hymeta_activation's HYMETA_ACT_SILU_MUL in place of hymeta_silu_and_mul's

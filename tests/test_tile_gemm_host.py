@@ -79,6 +79,12 @@ def test_rows_that_a_ranks_experts_can_expect():
     (2048, 8192, 57344, 0), (1280, 5120, 27648, 0),                          # a long one
     (800, 1600, 35072, 0), (1024, 1600, 35072, 1),                           # rows that leave a fifth of the rounds empty
     (5000, 3584, 7168, 0),                                                   # few columns
+    (3328, 3584, 10496, 0), (2816, 3584, 19200, 1), (3000, 2048, 12800, 1), (4451, 2048, 9216, 0),
+    (1024, 2816, 36864, 0), (1024, 2816, 37120, 1),                          # a multiple of 2048 columns, and none
+    (4474, 4032, 9984, 0), (2560, 3840, 18944, 0), (2560, 3584, 18944, 1),   # a long K
+    (2231, 3584, 18944, 0), (1900, 3584, 37888, 1),                          # a last round of half to three quarters of the units, of three and of five
+    (1152, 3584, 52480, 0), (769, 3584, 37888, 1), (1694, 2048, 28672, 0),   # rounds filled to 78 %; to 67 % where they are few; to 80 %
+    (769, 2560, 37888, 1), (1600, 3584, 19200, 0), (769, 2048, 37888, 0),    # ... few with few tiles in the last one; a short K
 ])
 def test_gate_up_projections_that_run_in_tiles(M, K, N, takes):
     from vllm_hymeta import _C

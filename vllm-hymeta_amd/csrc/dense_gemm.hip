@@ -167,11 +167,16 @@ extern "C" size_t hymeta_bf16_gemm_workspace_bytes(int32_t M, int32_t N, int32_t
 // The gate / up projection of a prompt in tiles (tile_gemm.hip), from two to eight rounds of tiles, us against the library's
 // product and the activation's launch, 37888 x 3584: 896 rows 223 / 291, 1280 277 / 385, 2048 444 / 548, 3328 701 / 813.  Below, the library
 // cuts K: 768 rows 189 / 186, 512 164 / 152.  Above, its product fills the chip as well: alone 4096 rows 879 / 893 and 8192
-// 1713 / 1826, but a whole prompt of 4096 7466 / 7375, of 8192 13877 / 13990.  Over 840 sizes of 92 matrices: from a K of 4096 on the
-// library reaches 1.3 to 1.4 PFLOP/s on many that the tiles do not (57344 x 8192 at 2048 rows 1375 / 1304, 32000 x 5184 at 1113 1.08 of its time), and
-// where rows and rounds are left a fifth empty, of a long K a third (45312 x 4864 at 520 1.13, 35072 x 1600 at 800 1.12, 11264 x 2048 at 2900
-// 1.05), or the columns are few (7168 x 3584 at 5000 228 / 218); the rest are 0.65 to 1.03 of it, 0.87 on average.  A K below 1024 is the
-// epilogue's.
+// 1713 / 1826, but a whole prompt of 4096 7466 / 7375, of 8192 13877 / 13990.  Over 1600 sizes, of the library's time:
+//  * K below 1024, whose epilogue counts: 0.6 to 0.99.
+//  * Longer ones cost what their rounds cost, so these must be filled to 82 % (28672 x 2048 at 1694 rows, 80 %, 1.06; 35072 x 1600 at 800
+//    1.12), to 66 % where they are few and the library's no fuller (37888 x 3584 at 769 0.89, x 2560 0.92; 19200 x 3584 at 1600, with 13 tiles in the
+//    third round, 1.13), and a last round of half to three quarters of the
+//    units costs a whole one (18944 x 3584 at 2231 1.08; of more than four rounds it matters less: 37888 x 3584 at 2048 0.81).
+//  * The library has products of its own at 1.2 to 1.4 PFLOP/s for many a matrix of longer K: 57344 x 8192 at 2048 rows 1.05, 9984 x 4032 at 4474
+//    1.10, 10240 x 3840 at 4410 1.09; where the columns are a multiple of 2048 (36864 x 2816 at 1024 1.06, 20480 x 3840 at 4387 1.07); or
+//    few (10496 x 3584 at 3328 1.10, 13056 x 3584 at 2867 1.08; of a K up to 2048 9216 x 2048 at 4451 1.08).
+// What is left runs in 0.66 to 1.06 of its time, 0.91 on average; one size in 40 is above 1.03.
 static TileGemmArgs gated_tile_args(int32_t M, int32_t K, int32_t N) {
   TileGemmArgs t = {};
   t.x_stride = static_cast<int64_t>(K) * 2, t.out_stride = N / 2, t.a_rows_div = 1, t.max_rows = M, t.N = N, t.k_bytes = K * 2, t.act = HYMETA_GEMM_ACT_SILU;
@@ -179,10 +184,13 @@ static TileGemmArgs gated_tile_args(int32_t M, int32_t K, int32_t N) {
 }
 static bool gated_tiles(int32_t M, int32_t K, int32_t N) {
   const int64_t tiles = static_cast<int64_t>(N / 256) * ((static_cast<int64_t>(M) + 255) / 256), units = 256, rest = tiles % units;
-  if (tiles <= 512 || tiles > 2048 || K >= 4096 || !tile_gemm_fits(gated_tile_args(M, K, N))) return false;
+  if (tiles <= 512 || tiles > 2048 || K > 3712 || !tile_gemm_fits(gated_tile_args(M, K, N))) return false;
   if (K < 1024) return true;
+  if (K > 2048 ? N < 18432 || N % 2048 == 0 : N < 9472) return false;
+  if (tiles < 4 * units && rest > units / 2 && rest <= 3 * units / 4) return false;
   const int64_t tenths = tiles / units * 10 + (rest == 0 ? 0 : rest <= units / 2 ? 6 : 10);      // of a round (a last one of halves: 0.6)
-  return N >= 9216 && 1000 * static_cast<int64_t>(M) * N >= (K >= 3584 ? 66 : 80) * tenths * units * 65536;
+  const int filled = K > 2048 && tiles <= 3 * units && rest >= units / 4 ? 66 : 82;
+  return 1000 * static_cast<int64_t>(M) * N >= filled * tenths * units * 65536;
 }
 
 // A product whose K is cut (tile_gemm_slices has the rule and what it measured).
