@@ -25,7 +25,7 @@ namespace {
 // 32 rows the matrix pipe (1.45 us a tile of 64 keys of 512) and the lone wave's issue add up: 2.76 us a tile, of which the copies'
 // issue takes 0.36, exponentials and rounding 0.30, half of the key reads 0.09; around a block's tiles lie about 12 us, half of them
 // its queries' 128 KB from memory, which all compute units ask for at once.  28 heads, 4 value heads of 128, window 1024, with a
-// workgroup per 64 rows and head -> here: 8192 rows 1275 -> 450 us; 2048 behind 4096 390 -> 134; four of 300 behind 2000 208 -> 71; five
+// workgroup per 64 rows and head -> here, back to back: 8192 rows 1275 -> 450 us; 2048 behind 4096 390 -> 134; four of 300 behind 2000 208 -> 71; five
 // of 10 behind 5955, keys cut into slices, 97 -> 26; 300 rows alone 33 -> 26.  Level or slower: copies issued among the slots (459),
 // fragments read 10 slots ahead (452), no barrier to the compiler's order between slots (a sixth slower).
 template <int D, int DV, int Layout, int Rule>

@@ -1,6 +1,7 @@
 """Linear layers of the attention blocks: bf16 or one of the fused dequant-GEMMs (GPTQ 4/8-bit, W8A8).
-Decode-sized batches (up to 256 rows; GPTQ: up to 64 and 129 to 256) run on this package's weight-streaming kernels; prefill-sized
-batches of bf16 / expanded GPTQ / int8 weights go to the library GEMM.  Stands where the reference puts vLLM's
+Decode-sized batches (up to 256 rows; GPTQ: up to 64 and 129 to 256) run on this package's weight-streaming kernels.  Prompts run in
+this package's tiles where those were measured ahead -- gate / up projections with the activation behind them, deep and narrow matrices
+cut along K, int8 products of enough tiles -- and as plain library products elsewhere, GPTQ ones on weights expanded to bf16.  Stands where the reference puts vLLM's
 ``QKVParallelLinear`` / ``RowParallelLinear`` / ``ReplicatedLinear`` with a ``quant_config``
 (``vllm_hymeta/model_for_7B/gla_attention.py:147-176``): a tensor-parallel shard is simply a
 ``HymetaLinear`` built from the shard's rows (column parallel) or columns (row parallel)."""
@@ -14,8 +15,8 @@ import torch
 from . import hip_ops
 
 
-# Rows above which a GPTQ linear expands its weights and calls the library GEMM (measured on the 7B
-# projection shapes: the fused kernel wins up to a few hundred rows, the library from there on).
+# Rows above which a GPTQ linear expands its weights and runs a bf16 product on them (measured on the 7B
+# projection shapes: the fused kernel wins up to a few hundred rows, the expansion from there on).
 GPTQ_EXPAND_ROWS = 256
 # Rows above which a W8A8 linear may put the library int8 GEMM between its own quantisation and
 # scaling kernels: the streaming int8 kernels cover up to 256 rows (one pass over the weights); both
