@@ -32,6 +32,12 @@ pytestmark = pytest.mark.gpu
     (512, 64, 4, 2, 64, [65] * 40, [100] * 40, {}),                                              # 320
     (512, 128, 4, 2, 64, [70, 9], [300, 900], dict(window=100, keep=4)),                         # a window: few tiles of many
     (512, 64, 4, 2, 64, [63, 3], [-40, -2], dict(sink=True, chunk=50)),
+    # few single rows beside cut keys: slices of 19 tiles, which their own launch takes, in front of whole and of cut portions; of 10, in
+    # pages of a tile along with the portions, in smaller pages not
+    (256, 64, 8, 2, 64, [700, 300, 1, 1], [0, 200, 2400, 1300], dict(sink=True)),
+    (512, 128, 8, 2, 64, [700, 300, 1, 1], [1700, 2100, 2400, 1], dict(sink=True, gate=True)),
+    (256, 128, 8, 2, 64, [339, 190, 1, 1], [0, 2500, 3000, 1300], {}),
+    (256, 128, 8, 2, 16, [339, 190, 1, 1], [0, 2500, 3000, 1300], {}),
 ])
 def test_portions_over_long_shared_keys(D, Dv, H, G, page, lens, ctxs, opts):
     portions.test_against_64_bits("shared", D, Dv, H, G, page, lens, ctxs, opts)

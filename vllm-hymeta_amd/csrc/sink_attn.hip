@@ -1097,17 +1097,19 @@ inline PortionSlices portion_slices(int num_tokens, int num_seqs, int num_heads,
 }
 inline bool one_launch(const hymeta_sink_attention_args& a, const PortionSlices& ps, int most);
 inline bool long_shared_keys(const hymeta_sink_attention_args& a);
+inline bool few_single_rows(const hymeta_sink_attention_args& a);
 inline PortionSlices portion_slices(const hymeta_sink_attention_args& a) {
   PortionSlices ps;
   if (a.max_query_len <= 1) return ps;
   ps = portion_slices(a.num_tokens, a.num_seqs, a.num_heads, a.num_kv_heads, a.v_dim, a.max_query_len, decode_tiles(a), a.head_dim);
-  // Long keys are cut only where the portions' launch takes the single rows as well (one_launch): the slices then have the room
-  // of the decode form's partials, which a caller brings anyway.
-  const bool long_keys = long_shared_keys(a);
-  if (long_keys && ps.splits > 1 && !one_launch(a, ps, 0)) ps.splits = 1;
-  const int64_t decode = long_keys ? 0 : decode_partial_bytes(a.num_seqs, a.num_heads, a.num_kv_heads, a.v_dim, a.max_seq_len);
+  // Long keys are cut beside few single rows only.  Where the portions' launch takes those as well (one_launch), the slices have the
+  // room of the decode form's partials.
+  const bool long_keys = long_shared_keys(a), along = ps.splits > 1 && one_launch(a, ps, 0);
+  if (long_keys && ps.splits > 1 && !few_single_rows(a)) ps.splits = 1;
+  const int64_t decode = long_keys && along ? 0 : decode_partial_bytes(a.num_seqs, a.num_heads, a.num_kv_heads, a.v_dim, a.max_seq_len);
   const int64_t room = (static_cast<int64_t>(a.workspace_bytes) - decode) / portion_partial_bytes(a.num_tokens, a.num_heads, a.v_dim);
   ps.splits = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(ps.splits, room)));
+  if (long_keys && along && ps.splits > 1 && !one_launch(a, ps, 0)) ps.splits = 1;      // (fewer, longer slices, which no longer do)
   ps.parts = static_cast<float*>(a.workspace) + decode / 4;
   return ps;
 }
@@ -1128,12 +1130,25 @@ inline dim3 portion_grid(const hymeta_sink_attention_args& a, const PortionSlice
 // Long keys have one workgroup on a compute unit, so single rows go along where they take no more rounds of units than the portions do
 // without them: 40 rows beside 63 single ones of 100 keys of 512, 28 heads, in 264 workgroups 23.9, in two launches 22.0; beside 127
 // 53.9 and 43.6, 40 beside 127 of 400 keys of 256 68 and 57; 40 beside 48 of 60 keys, 204 workgroups, 17 and 22.
+// Of their cut keys a single row's workgroup walks a slice alone while portions that begin their sequence are done with their few tiles:
+// up to 16 tiles of 64 keys, or 8 where a tile takes several pages (a copy's addresses are looked up row by row).  All of it by the
+// portions' launch -> in two: 190 and 339 rows of 16 heads of 256 beside four of up to 7552 keys in pages of 16 262 -> 59 us, 513 beside six of
+// up to 7311 142 -> 57, 346 beside three of up to 3208 140 -> 49; rows of portions behind many keys lose the other launch, 129 and 18 behind 2000
+// beside twelve 54 -> 71.  520 steps of one to four
+// portions and up to 16 single rows: 0.29 to 1.39 of the time, 0.96 on average.
 constexpr int kFewTiles = 16, kFewWideTiles = 2, kManySingleRows = 512, kLongKeyUnits = 256, kFewSingleRows = 4;
+constexpr int kAlongTiles = 16, kAlongPagedTiles = 8;
 inline bool long_shared_keys(const hymeta_sink_attention_args& a) { return a.kv_layout == HYMETA_KV_SHARED_KEY && a.head_dim > 192; }
+inline bool few_single_rows(const hymeta_sink_attention_args& a) {
+  return a.num_seqs - long_portions(a.num_tokens, a.num_seqs, a.max_query_len) <= kFewSingleRows * std::min(a.num_kv_heads, 4);
+}
 inline bool one_launch(const hymeta_sink_attention_args& a, const PortionSlices& ps, int most) {
   const int64_t portions = long_portions(a.num_tokens, a.num_seqs, a.max_query_len), singles = a.num_seqs - portions;
   if (a.max_query_len <= 1) return false;
-  if (ps.splits > 1) return singles <= kFewSingleRows * std::min(a.num_kv_heads, 4);
+  if (ps.splits > 1) {
+    const int along = a.block_size < kTileKeys ? kAlongPagedTiles : kAlongTiles;
+    return few_single_rows(a) && (!long_shared_keys(a) || singles == 0 || (decode_tiles(a) + ps.splits - 1) / ps.splits <= along);
+  }
   if (decode_tiles(a) > most) return false;
   if (!long_shared_keys(a)) return singles * a.num_kv_heads <= kManySingleRows;
   const int64_t each = (static_cast<int64_t>(a.max_query_len) * (a.num_heads / a.num_kv_heads) + kPortionRows - 1) / kPortionRows;
