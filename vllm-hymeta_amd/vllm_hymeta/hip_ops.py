@@ -1799,6 +1799,9 @@ def sink_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_tables: torch.
     if max_query_len > 1 and q.dtype == torch.bfloat16:
         nbytes = int(lib.hymeta_sink_attention_portion_workspace_bytes(T, S, H, num_kv_heads, v_dim, max_query_len, max_seq_len,
                                                                        chunk if chunk > 0 else window_left + 1, keep_first))
+        if shared_key and head_dim > 192 and S == 1:      # (no single rows beside the portion: its slices' partials have their room)
+            single = int(lib.hymeta_sink_attention_workspace_bytes(S, H, num_kv_heads, v_dim, max_seq_len))
+            nbytes = max(single, nbytes - single)
     else:
         nbytes = int(lib.hymeta_sink_attention_workspace_bytes(S, H, num_kv_heads, v_dim, max_seq_len))
     if nbytes:
