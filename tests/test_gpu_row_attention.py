@@ -70,6 +70,8 @@ def reference(q, k, v, scale, ctx, o, sink, a, gate):
     *[("rows", 128, 128, 8, 2, 64, [8, 2], [c, 63], dict(sink=True, gate=True)) for c in (184, 185, 248, 249)],
     # single rows: as many partials as a thread of the merge holds, and one more; head groups that are not full
     *[("rows", 64, 64, 10, 2, 64, [1, 0, 1, 1], [64 * n - 1, 5, 0, 70], dict(sink=True, gate=True, elem=True)) for n in (2, 3, 4, 5, 8, 9)],
+    # and as many as its threads take at once, four or eight each, and one more; statistics for two each
+    *[("rows", 64, 64, 10, 2, 64, [1], [64 * n - 1], dict(sink=True, gate=True, elem=True)) for n in (32, 33, 64, 65, 129)],
     ("rows", 64, 128, 3, 1, 64, [1, 1], [63, -1], {}),
     ("latent", 192, 128, 37, 1, 64, [1, 1], [127, 3], dict(sink=True, elem=True)),
     ("scaled", 96, 96, 7, 7, 64, [1, 1], [200, 3], dict(sink=True, bias="linear")),

@@ -51,6 +51,8 @@ def reference(q, rows, C, scale, sink, window, keep, chunk, softcap, bias, gate,
     (256, 40, 16, [1, 5, 1], [900, 1400, 31], dict(chunk=700, gate=True)),
     (256, 33, 64, [1] * 5, [0, 15, 16, 1000, 63], dict(sink=True, window=33)),
     *[(c, 16, 64, [1, 1], [64 * n - 1, 20], dict(sink=True, gate=True)) for c, n in ((384, 2), (512, 3), (256, 8), (512, 9))],      # partials of a row
+    # as many of 128 columns as a thread takes at once, four or eight, and one more; statistics for two each
+    *[(c, 16, 64, [1], [64 * n - 1], dict(sink=True, gate=True)) for c, n in ((512, 16), (384, 17), (256, 32), (512, 33), (512, 129))],
 ])
 def test_against_64_bits(C, H, page, lens, ctxs, opts):
     from vllm_hymeta import hip_ops

@@ -830,15 +830,20 @@ __global__ __launch_bounds__(64 * kDecodeWaves) void sink_attention_decode_mfma_
 }
 
 // Merge a row's partials (`splits` of them, `stride` floats apart from `base` on), add the sink, normalise, store bf16: one
-// workgroup per (row, head).  Two round trips to memory: the threads read the partials' statistics side by side (one each),
-// agree on the row's maximum, and leave every partial's factor in LDS; then groups of v_dim / 4 threads take the partials
-// in turn, four columns a thread.  (One serial loop over the partials per column and statistic: 3 rows of 28 heads with 20
-// partials of 128 columns 25.7 us with the kernel in front of it, so 21.3.)
+// workgroup per (row, head) and part of the columns.  Bound by round trips to memory: the threads read the partials' statistics
+// side by side (one each) and, with them in flight, their first partials' values, agree on the row's maximum, and leave every
+// partial's factor in LDS; groups of a thread per four columns take the partials in turn.  Values asked for behind the statistics,
+// four at a time around a branch -> so, us: 28 heads of 128, 3 rows at 20000 keys 31.7 -> 28.8, 9 at 5000 13.9 -> 12.0; 16 heads of 128
+// on a latent, a row at 20000 41.1 -> 18.5.
 constexpr int kCombineThreads = 128;
 constexpr int kMaxPartials = 512 * kDecodeWaves;
 // Up to as many partials a (row, head) goes to the kernel that holds them all in registers: more partials are for few rows, which
 // leave the chip room for a workgroup each.
 constexpr int kFewPartials = 8;
+// Columns of a workgroup where a row has more partials: a row of 512 then has four workgroups that take the partials four at
+// a time, and not one whose threads all take every partial.  16 heads on 512 + 64, 3 rows at 9600 keys 47.3 -> 23.5 us, 12 at 5000
+// 42 -> 36; 28 heads, a row at 30000 60 -> 25.
+constexpr int kPartColumns = 128;
 
 // Columns c .. c + 3 of row t's head h, from the weighted values and the weights' sum.
 __device__ __forceinline__ void store_row(const hymeta_sink_attention_args& a, f32x4v acc, float l, int64_t t, int h, int c) {
@@ -859,49 +864,68 @@ __device__ __forceinline__ void store_row(const hymeta_sink_attention_args& a, f
 // maximum either, but a NaN for a sum, which the row's result keeps.
 __device__ __forceinline__ bool no_keys(float m, float l) { return m == -INFINITY && l == 0.f; }
 
-__device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a, const float* base, size_t stride, int splits, int64_t t, int h) {
-  __shared__ float s_f[kMaxPartials];
-  __shared__ float s_red[2][kCombineThreads / 64];
-  __shared__ __attribute__((aligned(16))) f32x4v s_acc[kCombineThreads];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, DV = a.v_dim;
+struct CombineScratch {
+  __attribute__((aligned(16))) f32x4v acc[kCombineThreads];
+  float f[kMaxPartials], red[2][kCombineThreads / 64];
+};
+// Batch: partials whose values a thread has in flight together, the first ones beside the statistics.
+template <int Batch>
+__device__ __forceinline__ void combine_row_in(CombineScratch& lds, const hymeta_sink_attention_args& a, const float* base, size_t stride, int splits, int64_t t, int h) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, DV = a.v_dim, cols = DV / gridDim.z;
+  const int quads = cols / 4, turns = kCombineThreads / quads, turn = tid / quads, c = blockIdx.z * cols + 4 * (tid % quads);
+  auto stat = [&](int sp) { return *reinterpret_cast<const float2*>(base + sp * stride + DV); };
+  f32x4v x[Batch];
+  auto fetch = [&](int sp0) __attribute__((always_inline)) {         // (past the last one: read again)
+#pragma unroll
+    for (int u = 0; u < Batch; ++u) x[u] = *reinterpret_cast<const f32x4v*>(base + min(sp0 + u * turns, splits - 1) * stride + c);
+  };
   // (the partials' maxima are in the base-2 domain, as the waves kept them)
   const float sink2 = a.sink_logits ? a.sink_logits[h] * 1.4426950408889634f : 0.f;
   float m = a.sink ? sink2 : -INFINITY;
-  for (int sp = tid; sp < splits; sp += kCombineThreads) {
-    const float ms = base[sp * stride + DV];
-    s_f[sp] = ms;
-    m = fmaxf(m, ms);
-  }
+  const float2 own = stat(min(tid, splits - 1));       // this thread's first partial
+  fetch(turn);
+  if (tid < splits) m = fmaxf(m, own.x);
+  for (int sp = tid + kCombineThreads; sp < splits; sp += kCombineThreads) m = fmaxf(m, stat(sp).x);
   m = wave_max(m);
-  if (lane == 0) s_red[0][wave] = m;
+  if (lane == 0) lds.red[0][wave] = m;
   __syncthreads();
-  m = fmaxf(s_red[0][0], s_red[0][1]);
+  m = fmaxf(lds.red[0][0], lds.red[0][1]);
   float l = 0.f;
-  for (int sp = tid; sp < splits; sp += kCombineThreads) {      // (each thread's own entries of s_f)
-    const float lp = base[sp * stride + DV + 1], f = no_keys(s_f[sp], lp) ? -1.f : __builtin_amdgcn_exp2f(s_f[sp] - m);
-    s_f[sp] = f;
-    if (!(f < 0.f)) l = fmaf(lp, f, l);
+  for (int sp = tid; sp < splits; sp += kCombineThreads) {
+    const float2 p = sp == tid ? own : stat(sp);
+    const float f = no_keys(p.x, p.y) ? -1.f : __builtin_amdgcn_exp2f(p.x - m);
+    lds.f[sp] = f;
+    if (!(f < 0.f)) l = fmaf(p.y, f, l);
   }
   l = wave_sum(l);
-  if (lane == 0) s_red[1][wave] = l;
+  if (lane == 0) lds.red[1][wave] = l;
   __syncthreads();
-  l = (s_red[1][0] + s_red[1][1]) + (a.sink ? __builtin_amdgcn_exp2f(sink2 - m) : 0.f);
-  const int quads = DV / 4, turns = kCombineThreads / quads, turn = tid / quads, c = 4 * (tid % quads);
+  l = (lds.red[1][0] + lds.red[1][1]) + (a.sink ? __builtin_amdgcn_exp2f(sink2 - m) : 0.f);
   f32x4v acc = f32x4v{0.f, 0.f, 0.f, 0.f};
-  if (turn < turns) {
-#pragma unroll 4
-    for (int sp = turn; sp < splits; sp += turns) {
-      const float f = s_f[sp];
-      if (!(f < 0.f)) acc += *reinterpret_cast<const f32x4v*>(base + sp * stride + c) * f;
+  for (int sp0 = turn; sp0 < splits;) {
+#pragma unroll
+    for (int u = 0; u < Batch; ++u) {
+      const int sp = sp0 + u * turns;
+      const float f = sp < splits ? lds.f[sp] : -1.f;
+      if (!(f < 0.f)) acc += x[u] * f;
     }
+    sp0 += Batch * turns;
+    if (sp0 < splits) fetch(sp0);
   }
   if (turns > 1) {
-    s_acc[tid] = acc;
+    lds.acc[tid] = acc;
     __syncthreads();
     if (turn == 0)
-      for (int k = 1; k < turns; ++k) acc += s_acc[tid + k * quads];
+      for (int k = 1; k < turns; ++k) acc += lds.acc[tid + k * quads];
   }
   if (turn == 0) store_row(a, acc, l, t, h, c);
+}
+__device__ __forceinline__ void combine_row(const hymeta_sink_attention_args& a, const float* base, size_t stride, int splits, int64_t t, int h) {
+  __shared__ CombineScratch lds;
+  const int work = splits * (a.v_dim / gridDim.z), each = 4 * kCombineThreads;       // (values, and how many one partial per thread is)
+  if (work <= each) combine_row_in<1>(lds, a, base, stride, splits, t, h);
+  else if (work <= 4 * each) combine_row_in<4>(lds, a, base, stride, splits, t, h);
+  else combine_row_in<8>(lds, a, base, stride, splits, t, h);
 }
 
 // How the keys of portions are cut: into `splits` slices at most, whose partials lie at `parts`, [row][head][splits]; blocks of
@@ -938,7 +962,7 @@ __device__ __forceinline__ PieceAt portion_block(const hymeta_sink_attention_arg
 }
 constexpr int kWideKeys = 32;                  // a tile of the kernels over wide latents
 
-// grid = (sequences + rows where portions' keys were cut, heads): the rows of single-row sequences, and the rows of portions whose
+// grid = (sequences + rows where portions' keys were cut, heads, parts of the columns): the rows of single-row sequences, and the rows of portions whose
 // blocks were cut.  One launch for both: a step of both takes no more launches than without slices.  A row's portion is found in
 // one round trip for 64 sequences (one read behind the other: 300 whole rows beside 63 single ones took 78.2 us, so 76.2).
 __global__ __launch_bounds__(kCombineThreads) void sink_attention_combine_kernel(hymeta_sink_attention_args a, int splits, HeadSlice hs, PortionSlices ps) {
@@ -1173,7 +1197,8 @@ void launch_combine(const hymeta_sink_attention_args& a, hipStream_t st, int spl
     else hipLaunchKernelGGL(sink_attention_combine_few_kernel<kFewPartials>, grid, dim3(kCombineThreads), 0, st, a, splits, hs);
     return;
   }
-  const dim3 grid((ps.least > 1 ? a.num_seqs : 0) + (ps.splits > 1 ? a.num_tokens : 0), heads);
+  const unsigned parts = a.v_dim > kPartColumns && std::max(splits, ps.splits) > kFewPartials ? a.v_dim / kPartColumns : 1;
+  const dim3 grid((ps.least > 1 ? a.num_seqs : 0) + (ps.splits > 1 ? a.num_tokens : 0), heads, parts);
   hipLaunchKernelGGL(sink_attention_combine_kernel, grid, dim3(kCombineThreads), 0, st, a, splits, hs, ps);
 }
 
