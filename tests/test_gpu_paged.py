@@ -78,6 +78,8 @@ W = 64  # test window (keys visible incl. self), so window_left = W - 1
     (14, 2, 64, 64, 127, [700, 130, 1], 1),                      # forced single pass
     (14, 2, 64, 64, 127, [700, 130, 1], 5),                      # forced 5 splits
     (32, 1, 16, 0, -1, [77, 300], 3),                            # 32 q-heads per kv-head: two head groups
+    # the merge's forms: splits in registers, a split or two to a thread, one loop; some splits without a key
+    *[(7, 1, 16, 32, -1, [2500, 70], n) for n in (16, 17, 33, 128, 129, 256, 257)],
 ])
 def test_paged_decode(H, Hkv, bs, M, window_left, seq_lens, splits):
     from oracle import meta_swa_paged_decode_ref

@@ -31,7 +31,7 @@
 #include <cstdlib>
 #include <mutex>
 
-#include "common.h"
+#include "act_types.h"
 
 namespace hymeta {
 
@@ -411,6 +411,51 @@ __global__ __launch_bounds__(128) void paged_decode_merge_kernel(hymeta_paged_de
         l_tot += f * ls[i];
         acc += f * os[i];
       }
+  } else if (num_splits <= 256) {
+    // few rows of many splits, bound by round trips: a split's statistics to a thread, then four groups of 32 threads take the
+    // splits in turn, four columns a thread, eight splits in flight (the first ones beside the statistics).  7 heads on one, one
+    // split behind the other in two loops -> so, with the kernel in front, us: a row at 32000 keys 43.9 -> 13.4, three at 20000
+    // 33.5 -> 14.1; 28 heads on 4, a row of 4097 keys 15.1 -> 11.2.
+    constexpr int kGroups = 4, kBatch = 8;
+    __shared__ float s_f[256], s_red[2][2];
+    __shared__ __attribute__((aligned(16))) f32x4 s_acc[128];
+    const int turn = d / 32, c = 4 * (d % 32), wave = d / 64;
+    f32x4 x[kBatch];
+    auto fetch = [&](int s0) __attribute__((always_inline)) {         // (past the last one: read again)
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) x[u] = *reinterpret_cast<const f32x4*>(wo + (unit0 + min(s0 + kGroups * u, num_splits - 1)) * D + c);
+    };
+    float2 stat[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) stat[i] = *reinterpret_cast<const float2*>(ml + 2 * min(d + 128 * i, num_splits - 1));
+    fetch(turn);
+    m_tot = wave_max(fmaxf(stat[0].x, stat[1].x));
+    if ((d & 63) == 0) s_red[0][wave] = m_tot;
+    __syncthreads();
+    m_tot = fmaxf(s_red[0][0], s_red[0][1]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const bool own = d + 128 * i < num_splits;
+      const float f = own && stat[i].x != -INFINITY ? __builtin_amdgcn_exp2f(stat[i].x - m_tot) : 0.f;
+      if (own) s_f[d + 128 * i] = f;
+      l_tot += own ? f * stat[i].y : 0.f;
+    }
+    l_tot = wave_sum(l_tot);
+    if ((d & 63) == 0) s_red[1][wave] = l_tot;
+    __syncthreads();
+    l_tot = s_red[1][0] + s_red[1][1];
+    f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = turn; s0 < num_splits;) {
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)
+        if (s0 + kGroups * u < num_splits) sum += x[u] * s_f[s0 + kGroups * u];
+      s0 += kGroups * kBatch;
+      if (s0 < num_splits) fetch(s0);
+    }
+    s_acc[d] = sum;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kGroups; ++k) acc += reinterpret_cast<const float*>(s_acc + 32 * k)[d];
   } else {
     for (int s = 0; s < num_splits; ++s) m_tot = fmaxf(m_tot, ml[2 * s]);
     for (int s = 0; s < num_splits; ++s) {
