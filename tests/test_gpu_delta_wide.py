@@ -15,7 +15,11 @@ EDGES = [8, 63, 64, 65, 130, 7, 128, 129, 20, 1, 130, 97, 126, 127, 128]        
 @pytest.mark.parametrize("D,Dv,H,Hk,lens", [
     (32, 128, 16, 4, EDGES), (64, 256, 8, 8, EDGES), (96, 128, 16, 16, EDGES), (128, 128, 16, 8, EDGES),
     (128, 128, 16, 8, [1] * 20 + [300] + [1] * 12 + [9, 130]), (96, 128, 12, 12, [1] * 20 + [300] + [1] * 12 + [9, 130]),
-    (128, 128, 16, 8, [1] * 60 + [300] + [1] * 30)])
+    (128, 128, 16, 8, [1] * 60 + [300] + [1] * 30),
+    # more pairs than half of the compute units: the shortest sequences whole, the others' halves side by side; 80, 136 and 104 whole
+    (128, 128, 28, 14, [300, 257, 299, 260, 321, 270]), (128, 128, 28, 14, [300, 290, 257, 260, 299, 270, 5]), (64, 256, 15, 15, [257] * 6),
+    (32, 128, 28, 28, [300] * 5), (96, 128, 28, 28, [300] * 6 + [7]),      # and a portion too short for a chunk where none is expected:
+    (128, 128, 28, 14, [300] * 6 + [7]), (64, 128, 28, 7, [64] * 8 + [3]), (128, 128, 16, 16, [64, 64, 64, 5]), (128, 96, 12, 4, [64, 64, 64, 5])])
 def test_wide_slices_equal_narrow_ones(D, Dv, H, Hk, lens):
     """Both multiply the same operands (fp32 as two bf16 parts, 2^-17 of the operand) and add in another order: 1e-5 of the
     norm covers what that rounding grows to over a few chunks.  Rows at a chunk's edges, several chunks, a portion that goes

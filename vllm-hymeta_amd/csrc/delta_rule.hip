@@ -190,13 +190,13 @@ struct ShortScratch {
   __attribute__((aligned(16))) float q[2][D], k[2][D];
 };
 template <int D, int C4, int NT>
-__device__ __forceinline__ void delta_short_rows(const hymeta_delta_rule_args& a, int h, int s, int r0, int rows, int col0, ShortScratch<D, NT>& m) {
+__device__ __forceinline__ void delta_short_rows(const hymeta_delta_rule_args& a, int tid, int h, int s, int r0, int rows, int col0, ShortScratch<D, NT>& m) {
   typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
   constexpr int kGroups = NT / C4, U = D / kGroups, kEach = (D + 63) / 64, kWaves = NT / 64;
   static_assert(D % kGroups == 0 && 4 * C4 <= 64, "the state deals evenly over the threads");
   // (rows side by side where a thread has many: their queries and keys come four to a read)
   constexpr int kFirst = NT < 256 ? U : 1, kNext = NT < 256 ? 1 : kGroups;
-  const int c4 = threadIdx.x % C4, d0 = threadIdx.x / C4 * kFirst, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c4 = tid % C4, d0 = tid / C4 * kFirst, lane = tid & 63, wave = tid >> 6;
   const int H = a.num_heads, Dv = a.v_dim, g = h / (H / a.num_qk_heads);
   const int slot = a.slot_idx[s];
   float* st = slot >= 0 ? a.state + (static_cast<int64_t>(slot) * H + h) * D * Dv + col0 : nullptr;
@@ -293,7 +293,7 @@ __global__ __launch_bounds__(NT) void delta_short_kernel(hymeta_delta_rule_args 
   __shared__ ShortScratch<D, NT> m;
   const int s = blockIdx.z, r0 = a.query_start_loc[s], rows = a.query_start_loc[s + 1] - r0;
   if (rows <= 0 || rows > max_rows) return;
-  delta_short_rows<D, C4, NT>(a, blockIdx.x, s, r0, rows, blockIdx.y * 4 * C4, m);
+  delta_short_rows<D, C4, NT>(a, threadIdx.x, blockIdx.x, s, r0, rows, blockIdx.y * 4 * C4, m);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -320,7 +320,8 @@ constexpr int kChunk = HYMETA_DELTA_CHUNK;
 // us a chunk of 64 rows: not where those are more than 10 per row of the longest portion.
 // Workgroups with slices of 64 columns up to which the other kernel takes those: its images leave room for one workgroup on a
 // compute unit, where four waves take 2.6 us a chunk and eight (slices of 128) 4.4.  28 heads: three portions of 2700 (168)
-// 177 us, 301 before; five of 1801 (280, in slices of 128) 182, 280 before.
+// 177 us, 301 before; five of 1801 (280, in slices of 128) 182, 280 before (154 with some sequences'
+// slices of 64: delta_chunk_mixed_kernel).
 // All count the portions that the step's rows are worth (long_portions): single rows leave the chip to a long prompt.
 constexpr int kFewGroups = 128, kIdleGroupsPerRow = 10, kManyGroups = 256;
 // Whether portions too short for a chunk have a launch of their own and do not run in the chunks' first one, where they cost no
@@ -367,6 +368,19 @@ __device__ __forceinline__ void unrolled(const F& f) { unrolled<N>(f, std::make_
 __device__ __forceinline__ f32x4v mfma16(bf16x8 a, bf16x8 b, f32x4v c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ bf16x8 frag(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
+// Inclusive sums over a wave's lanes in double precision (lane_sums, a word at a time).
+__device__ __forceinline__ double lane_sums64(double x) {
+  auto add = [&](auto ctrl, auto rows_mask) {
+    const uint64_t bits = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(bits), decltype(ctrl)::value, decltype(rows_mask)::value, 0xf, false);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(bits >> 32), decltype(ctrl)::value, decltype(rows_mask)::value, 0xf, false);
+    x += __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+  };
+  add(Const<0x111>{}, Const<0xf>{}), add(Const<0x112>{}, Const<0xf>{}), add(Const<0x114>{}, Const<0xf>{}), add(Const<0x118>{}, Const<0xf>{});
+  add(Const<0x142>{}, Const<0xa>{}), add(Const<0x143>{}, Const<0xc>{});
+  return x;
+}
+
 // four fp32 values as hi + lo bf16 parts
 __device__ __forceinline__ void split4(const float* v, u32x2& hi, u32x2& lo) {
 #pragma unroll
@@ -381,42 +395,48 @@ __device__ __forceinline__ void split4(const float* v, u32x2& hi, u32x2& lo) {
 __host__ __device__ inline size_t rows_at(int64_t chunks, int heads) { return static_cast<size_t>(chunks) * heads * sizeof(ChunkPlace); }
 
 // grid = (chunk numbers, heads), 4 waves with 16 rows of the chunk each.
-// Portions shorter than kChunkMinRows go row by row here (short_too), all of a head's value columns in turn.
-template <int D, bool Pack>
-__global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hymeta_delta_rule_args a, int64_t chunks, bool short_too) {
-  constexpr int PK = D + 8, PF = kChunk + 4;
-  // (the keys and T share their place where nothing asks for the keys again: four workgroups to a compute unit)
+// Bound by vector instructions and the latency of its phases: A stays in the registers that the elimination multiplies it from, and only
+// a wave's diagonal block passes through LDS, to the wave itself, so that six workgroups are on a compute unit (four with all of A in
+// LDS); the sequence is found in one round trip.  28 heads, five portions of 1801 rows 53 -> 46 us.
+// Short: portions shorter than kChunkMinRows go row by row here, all of a head's value columns in turn, at the price of registers.
+template <int D, bool Pack, bool Short>
+__global__ __launch_bounds__(256, Pack ? 3 : Short ? 4 : 6) void delta_chunk_solve_kernel(hymeta_delta_rule_args a, int64_t chunks) {
+  constexpr int PK = D + 8, PF = kChunk + 4, PD = 20;
+  // (the keys and T share their place where nothing asks for the keys again: six workgroups to a compute unit)
   constexpr int kKeyBytes = kChunk * PK * 2, kMatrixBytes = kChunk * PF * 4;
   __shared__ __attribute__((aligned(16))) char s_keys[Pack ? kKeyBytes + kMatrixBytes : kKeyBytes > kMatrixBytes ? kKeyBytes : kMatrixBytes];
   uint16_t* sk = reinterpret_cast<uint16_t*>(s_keys);
   float* sT = reinterpret_cast<float*>(s_keys + (Pack ? kKeyBytes : 0));
-  __shared__ __attribute__((aligned(16))) float sA[kChunk * PF];
+  __shared__ __attribute__((aligned(16))) float s_diag[4][16 * PD];                // a wave's diagonal block of A
   __shared__ float s_hi[kChunk], s_lo[kChunk], s_beta[kChunk], s_ik[kChunk], s_iq[kChunk];
-  // the sequence: the last one whose first number is not past this one
-  const int number = blockIdx.x;
-  int s = 0;
-  for (int lo = 0, hi = a.num_seqs - 1; lo <= hi;) {
-    const int mid = (lo + hi) >> 1;
-    if (a.query_start_loc[mid] / kChunk + mid <= number) s = mid, lo = mid + 1;
-    else hi = mid - 1;
+  // the sequence: the last one whose first number is not past this one (64 of them in one round trip)
+  const int number = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  int s = 0, r0 = 0, rows = 0;
+  for (int base = 0; base < a.num_seqs; base += 64) {
+    const int start = a.query_start_loc[min(base + lane, a.num_seqs)];
+    const int upto = __popcll(__ballot(base + lane < a.num_seqs && start / kChunk + base + lane <= number));
+    if (upto == 0) break;
+    s = base + upto - 1, r0 = __builtin_amdgcn_readlane(start, upto - 1);
+    rows = (upto < 64 ? __builtin_amdgcn_readlane(start, upto) : a.query_start_loc[s + 1]) - r0;
+    if (upto < 64) break;
   }
-  const int r0 = a.query_start_loc[s], rows = a.query_start_loc[s + 1] - r0;
   const int c0 = (number - (r0 / kChunk + s)) * kChunk;
   if (c0 >= rows) return;
   if (rows < kChunkMinRows) {
-    static_assert(sizeof(ShortScratch<D, 256>) <= sizeof(sA), "the scratch lies where A would");
-    if (!short_too) return;
-    ShortScratch<D, 256>& m = *reinterpret_cast<ShortScratch<D, 256>*>(sA);
-    if (a.v_dim % 64 == 0) {
-      for (int col0 = 0; col0 < a.v_dim; col0 += 64) delta_short_rows<D, 16, 256>(a, blockIdx.y, s, r0, rows, col0, m), __syncthreads();
-    } else {
-      for (int col0 = 0; col0 < a.v_dim; col0 += 32) delta_short_rows<D, 8, 256>(a, blockIdx.y, s, r0, rows, col0, m), __syncthreads();
+    if constexpr (Short) {
+      static_assert(sizeof(ShortScratch<D, 256>) <= sizeof(s_keys), "the scratch lies where the keys would");
+      ShortScratch<D, 256>& m = *reinterpret_cast<ShortScratch<D, 256>*>(s_keys);
+      if (a.v_dim % 64 == 0) {
+        for (int col0 = 0; col0 < a.v_dim; col0 += 64) delta_short_rows<D, 16, 256>(a, tid, blockIdx.y, s, r0, rows, col0, m), __syncthreads();
+      } else {
+        for (int col0 = 0; col0 < a.v_dim; col0 += 32) delta_short_rows<D, 8, 256>(a, tid, blockIdx.y, s, r0, rows, col0, m), __syncthreads();
+      }
     }
     return;
   }
   const int nrow = min(kChunk, rows - c0), h = blockIdx.y, H = a.num_heads, group = H / a.num_qk_heads, g = h / group;
   const int64_t t0 = r0 + c0;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, g4 = lane >> 4;
   const int i = 16 * wave + n;                          // this lane's row of the chunk
   ChunkPlace* place = static_cast<ChunkPlace*>(a.workspace) + static_cast<int64_t>(number) * H + h;
   u32x4 kf[D / 32], qf[D / 32];
@@ -433,12 +453,7 @@ __global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hy
     // running sums in double precision, kept as two floats: a difference of two sums is exact to its own rounding however
     // large the sums are
     const bool on = lane < nrow;
-    double cum = on ? static_cast<double>(fmaxf(a.log2_decay[(t0 + lane) * H + h], kMinLog2)) : 0.0;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const double up = __shfl_up(cum, o, 64);
-      if (lane >= o) cum += up;
-    }
+    const double cum = lane_sums64(on ? static_cast<double>(fmaxf(a.log2_decay[(t0 + lane) * H + h], kMinLog2)) : 0.0);
     s_hi[lane] = static_cast<float>(cum);
     s_lo[lane] = static_cast<float>(cum - static_cast<double>(s_hi[lane]));
     s_beta[lane] = on ? sigmoid_exact(bf2f(static_cast<const uint16_t*>(a.beta_logit)[(t0 + lane) * a.beta_stride_t + h])) : 0.f;
@@ -462,9 +477,11 @@ __global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hy
   __syncthreads();
   // A and P in blocks of 16 x 16, transposed products: a lane gets four consecutive j of its row i
   const float ch = s_hi[i], cl = s_lo[i], bk = s_beta[i] * s_ik[i], iq = s_iq[i];
+  f32x4v A[4];                                          // this lane's row, columns 16 jb + 4 g4 + r
 #pragma unroll
   for (int jb = 0; jb < 4; ++jb) {
-    float av[4] = {0.f, 0.f, 0.f, 0.f}, pv[4] = {0.f, 0.f, 0.f, 0.f};
+    float pv[4] = {0.f, 0.f, 0.f, 0.f};
+    A[jb] = f32x4v{0.f, 0.f, 0.f, 0.f};
     if (jb <= wave) {
       f32x4v xk = f32x4v{0.f, 0.f, 0.f, 0.f}, xq = xk;
 #pragma unroll
@@ -478,10 +495,10 @@ __global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hy
         const int j = 16 * jb + 4 * g4 + r;
         if (j > i) continue;
         const float w = __builtin_amdgcn_exp2f((ch - s_hi[j]) + (cl - s_lo[j])) * s_ik[j];
-        if (j < i) av[r] = bk * w * xk[r];
+        if (j < i) A[jb][r] = bk * w * xk[r];
         pv[r] = iq * w * xq[r];
       }
-      *reinterpret_cast<f32x4v*>(&sA[i * PF + 16 * jb + 4 * g4]) = f32x4v{av[0], av[1], av[2], av[3]};
+      if (jb == wave) *reinterpret_cast<f32x4v*>(&s_diag[wave][n * PD + 4 * g4]) = A[jb];
     }
     u32x2 hi, lo;
     split4(pv, hi, lo);
@@ -489,17 +506,23 @@ __global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hy
     *reinterpret_cast<u32x2*>(&place->p[0][operand_at(i, 16 * jb + 4 * g4, kChunk)]) = hi;
     *reinterpret_cast<u32x2*>(&place->p[1][operand_at(i, 16 * jb + 4 * g4, kChunk)]) = lo;
   }
-  __syncthreads();
-  // T: the diagonal blocks by forward substitution, a column per lane (the four groups of lanes do the same)
+  // T: the diagonal blocks by forward substitution, a column per lane (the four groups of lanes do the same), each by the wave
+  // that has it
   {
+    const float* diag = s_diag[wave];
     float x[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
+      f32x4v row[4];
+#pragma unroll
+      for (int j = 0; j < (r + 3) / 4; ++j) row[j] = *reinterpret_cast<const f32x4v*>(&diag[r * PD + 4 * j]);
       float v = r == n ? 1.f : 0.f;
 #pragma unroll
-      for (int j = 0; j < r; ++j) v = fmaf(-sA[(16 * wave + r) * PF + 16 * wave + j], x[j], v);
+      for (int j = 0; j < r; ++j) v = fmaf(-row[j >> 2][j & 3], x[j], v);
       x[r] = v;
+      asm volatile("" : "+v"(x[r]));                    // (here, not behind the barrier with all of A's rows in registers)
     }
+    __syncthreads();                                    // nobody reads the keys where T comes to lie
     if (g4 == 0) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) sT[(16 * wave + r) * PF + 16 * wave + n] = x[r];
@@ -514,10 +537,11 @@ __global__ __launch_bounds__(256, Pack ? 3 : 4) void delta_chunk_solve_kernel(hy
     if (wave >= below) {
       const int jb = wave - below;
       f32x4v m = f32x4v{0.f, 0.f, 0.f, 0.f}, x = m;
-      for (int lb = jb; lb < wave; ++lb) {
-        const f32x4v al = *reinterpret_cast<const f32x4v*>(&sA[i * PF + 16 * lb + 4 * g4]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) m = __builtin_amdgcn_mfma_f32_16x16x4f32(al[e], sT[(16 * lb + 4 * g4 + e) * PF + 16 * jb + n], m, 0, 0, 0);
+      for (int lb = 0; lb < 3; ++lb) {
+        if (lb < jb || lb >= wave) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m = __builtin_amdgcn_mfma_f32_16x16x4f32(A[lb][e], sT[(16 * lb + 4 * g4 + e) * PF + 16 * jb + n], m, 0, 0, 0);
       }
       const f32x4v ti = *reinterpret_cast<const f32x4v*>(&sT[i * PF + 16 * wave + 4 * g4]);
 #pragma unroll
@@ -797,17 +821,30 @@ __global__ __launch_bounds__(256) void delta_chunk_narrow_kernel(hymeta_delta_ru
 // LDS: blocks of 16 rows x 32 columns, 1 KB, in operand order but for the rows: chunk (16 bytes) ch of the block's row m lies
 // at 16 ch + (m ^ 4 ch), so that the transposed reads of 4 rows x 4 chunks spread over the banks too.
 template <int D, int NW>
-__global__ __launch_bounds__(64 * NW, NW / 4 > 0 ? NW / 4 : 1) void delta_chunk_wide_kernel(hymeta_delta_rule_args a) {
-  constexpr bool Direct = NW == 2;                          // values of any alignment, read by the lanes that want them
-  constexpr int SD = D / 32, DB = D / 16, VC = 2 * NW, kRowsBytes = kChunk * D * 2, kMatBytes = 6 * 1024;
-  constexpr int kMatsAt = 2 * kRowsBytes, kScaleAt = kMatsAt + 4 * kMatBytes, kValuesAt = kScaleAt + 1024, kImage = kValuesAt + (Direct ? 0 : kChunk * 16 * VC);
+struct WideImage {                                          // keys, queries | T hi, lo, P hi, lo | beta, rhs, read, write | values
+  static constexpr bool kDirect = NW == 2;                  // values of any alignment, read by the lanes that want them
+  static constexpr int kRowsBytes = kChunk * D * 2, kMatBytes = 6 * 1024, kMatsAt = 2 * kRowsBytes, kScaleAt = kMatsAt + 4 * kMatBytes, kValuesAt = kScaleAt + 1024;
+  static constexpr int kBytes = kValuesAt + (kDirect ? 0 : kChunk * 32 * NW);
+};
+// Columns 16 NW vs .. of head h of sequence s, by NW waves (short_too: portions shorter than kChunkMinRows as well, row by row).
+template <int D, int NW>
+__device__ __forceinline__ void delta_chunk_wide(const hymeta_delta_rule_args& a, int h, int s, int vs, char* lds, bool short_too) {
+  typedef WideImage<D, NW> Image;
+  constexpr bool Direct = Image::kDirect;
+  constexpr int SD = D / 32, DB = D / 16, VC = 2 * NW, kRowsBytes = Image::kRowsBytes, kMatBytes = Image::kMatBytes;
+  constexpr int kMatsAt = Image::kMatsAt, kScaleAt = Image::kScaleAt, kValuesAt = Image::kValuesAt, kImage = Image::kBytes;
   static_assert(NW == 2 || NW == 4 || NW == 8, "the copies deal evenly over the waves");
   typedef ChunkOrder<VC> VOrder;
   typedef f32x4v f32x4_any __attribute__((aligned(4)));
-  __shared__ __attribute__((aligned(16))) char images[2][kImage];       // keys, queries | T hi, lo, P hi, lo | beta, rhs, read, write | values
-  const int h = blockIdx.x, s = blockIdx.y, vs = blockIdx.z;
   const int r0 = a.query_start_loc[s], rows = a.query_start_loc[s + 1] - r0;
-  if (rows < kChunkMinRows) return;
+  if (rows < kChunkMinRows) {
+    constexpr int NT = NW == 2 ? 128 : 256, kCols = NW == 2 ? 32 : 64;          // (eight waves: 64 columns by four each)
+    if (!short_too || rows <= 0) return;
+    ShortScratch<D, NT>* m = reinterpret_cast<ShortScratch<D, NT>*>(lds);
+    const int part = threadIdx.x / NT;
+    delta_short_rows<D, kCols / 4, NT>(a, threadIdx.x % NT, h, s, r0, rows, vs * 16 * NW + part * kCols, m[part]);
+    return;
+  }
   const int lane = threadIdx.x & 63, n = lane & 15, g4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int H = a.num_heads, Dv = a.v_dim, g = h / (H / a.num_qk_heads), col0 = (vs * NW + wave) * 16;
@@ -857,7 +894,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4 > 0 ? NW / 4 : 1) void delta_chunk_
   {
     const Source from = source(0);
 #pragma unroll
-    for (int i = 0; i < kCopies; ++i) copy(from, images[0], i);
+    for (int i = 0; i < kCopies; ++i) copy(from, lds, i);
     fetch(from);
   }
   const int slot_ = a.slot_idx[s];
@@ -904,8 +941,8 @@ __global__ __launch_bounds__(64 * NW, NW / 4 > 0 ? NW / 4 : 1) void delta_chunk_
     if (row < live) *reinterpret_cast<f32x4_any*>(to) = y[ib];
   };
   for (int c = 0; c < num; ++c) {
-    const char* image = images[c & 1];
-    char* next = images[(c + 1) & 1];
+    const char* image = lds + (c & 1) * kImage;
+    char* next = lds + ((c + 1) & 1) * kImage;
     const Source from = source(min(c + 1, num - 1));        // (the last chunk fetches itself once more: no copy under a condition)
     copies_landed_barrier();                 // this chunk's image is there, the other's readers are done
     // what the compiler still counts as in flight has landed: it is used here, in front of the next copies, which it would
@@ -1060,6 +1097,42 @@ __global__ __launch_bounds__(64 * NW, NW / 4 > 0 ? NW / 4 : 1) void delta_chunk_
   }
 }
 
+template <int D, int NW>
+__global__ __launch_bounds__(64 * NW, NW / 4 > 0 ? NW / 4 : 1) void delta_chunk_wide_kernel(hymeta_delta_rule_args a, bool short_too) {
+  __shared__ __attribute__((aligned(16))) char images[2 * WideImage<D, NW>::kBytes];
+  delta_chunk_wide<D, NW>(a, blockIdx.x, blockIdx.y, blockIdx.z, images, short_too);
+}
+
+// More (head, sequence, 128 columns) than half of the compute units, but not more than there are: `whole` of them, of the shortest
+// sequences, by eight waves, which take 4.4 us a chunk, the others by four waves on each of two compute units, 2.6 us a chunk.  A step ends
+// with the longest of either, and lengths differ: 28 heads, five portions of 1801 to 1413 rows 128 -> 110 us, six of 1365 to 910 (80
+// pairs of 168 whole) 139.5 -> 130 with the launch in front; equal ones are level (five of 1600, 162), and so are portions of up to kMixedRows rows
+// (six of 90 27.7 and 28.3).  grid = (whole + 2 (pairs - whole)), 8 waves, of which a half needs 4; at most 64 sequences.
+constexpr int kMixedRows = 4 * kChunk;
+template <int D>
+__global__ __launch_bounds__(512, 2) void delta_chunk_mixed_kernel(hymeta_delta_rule_args a, int whole, bool short_too) {
+  __shared__ __attribute__((aligned(16))) char images[2 * WideImage<D, 8>::kBytes];
+  const int lane = threadIdx.x & 63, n = a.num_seqs, per_seq = a.num_heads * (a.v_dim / 128), halves = n * per_seq - whole;
+  int pair, half = -1;                                      // pairs numbered from the longest sequence's on
+  if (static_cast<int>(blockIdx.x) < whole) pair = n * per_seq - 1 - blockIdx.x;
+  else {                                                    // a pair's halves eight workgroups apart, on one die: they read the same keys and matrices
+    const int j = blockIdx.x - whole, first = j / 16 * 8, side = min(8, halves - first), in = j - 2 * first;
+    half = in >= side, pair = first + in - half * side;
+  }
+  // the sequence of a rank: a lane each
+  const int len = lane < n ? a.query_start_loc[lane + 1] - a.query_start_loc[lane] : -1;
+  int rank = 0;
+  for (int i = 0; i < n; ++i) {
+    const int other = __builtin_amdgcn_readlane(len, i);
+    rank += other > len || (other == len && i < lane);
+  }
+  auto uniform = [](int x) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane(x); };      // (of a division, which runs in vector registers)
+  const int place = uniform(pair / per_seq), s = __builtin_ctzll(__ballot(lane < n && rank == place));
+  const int at = pair - place * per_seq, part = uniform(at / a.num_heads), h = at - part * a.num_heads;
+  if (half < 0) delta_chunk_wide<D, 8>(a, h, s, part, images, short_too);
+  else if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 4) delta_chunk_wide<D, 4>(a, h, s, 2 * part + half, images, short_too);
+}
+
 inline bool chunk_dims(int head_dim, int v_dim, int act_dtype) {
   return act_dtype == HYMETA_BF16 && head_dim >= 32 && head_dim <= 128 && head_dim % 32 == 0 && v_dim % 32 == 0 && v_dim / 16 <= 65535;
 }
@@ -1101,18 +1174,31 @@ void launch_chunks(const hymeta_delta_rule_args& a, hipStream_t st, int64_t chun
   const bool narrow = lanes * (a.v_dim / 32) <= kFewGroups && idle <= static_cast<int64_t>(kIdleGroupsPerRow) * a.max_query_len;
   const dim3 solve(static_cast<unsigned>(chunks), a.num_heads);
   if (narrow) {
-    hipLaunchKernelGGL((delta_chunk_solve_kernel<D, true>), solve, dim3(256), 0, st, a, chunks, short_too);
+    if (short_too) hipLaunchKernelGGL((delta_chunk_solve_kernel<D, true, true>), solve, dim3(256), 0, st, a, chunks);
+    else hipLaunchKernelGGL((delta_chunk_solve_kernel<D, true, false>), solve, dim3(256), 0, st, a, chunks);
     hipLaunchKernelGGL(delta_chunk_narrow_kernel<D>, dim3(a.num_heads, a.num_seqs, a.v_dim / 16), dim3(256), 0, st, a, chunks);
     return;
   }
-  hipLaunchKernelGGL((delta_chunk_solve_kernel<D, false>), solve, dim3(256), 0, st, a, chunks, short_too);
+  // Short portions in the first launch take it registers, and with them a third of its workgroups: where none are to be expected, those
+  // that there are after all go along in the second (28 heads, portions of 6 to 9 rows 34.6 -> 26.9 us).
+  const bool later = short_too && a.num_seqs == portions;
+  if (short_too && !later) hipLaunchKernelGGL((delta_chunk_solve_kernel<D, false, true>), solve, dim3(256), 0, st, a, chunks);
+  else hipLaunchKernelGGL((delta_chunk_solve_kernel<D, false, false>), solve, dim3(256), 0, st, a, chunks);
   auto launch = [&](auto nw) {
     constexpr int NW = decltype(nw)::value;
-    hipLaunchKernelGGL((delta_chunk_wide_kernel<D, NW>), dim3(a.num_heads, a.num_seqs, a.v_dim / (16 * NW)), dim3(64 * NW), 0, st, a);
+    hipLaunchKernelGGL((delta_chunk_wide_kernel<D, NW>), dim3(a.num_heads, a.num_seqs, a.v_dim / (16 * NW)), dim3(64 * NW), 0, st, a, later);
   };
   using std::integral_constant;
   const bool aligned = a.v_stride_t % 8 == 0 && reinterpret_cast<uintptr_t>(a.v) % 16 == 0;      // (values copied to LDS)
-  if (aligned && a.v_dim % 128 == 0 && lanes * (a.v_dim / 64) > kManyGroups) launch(integral_constant<int, 8>{});
+  const int64_t pairs = static_cast<int64_t>(a.num_heads) * a.num_seqs * (a.v_dim / 128);
+  if (aligned && a.v_dim % 128 == 0 && lanes * (a.v_dim / 64) > kManyGroups) {
+    if (pairs < kManyGroups && a.num_seqs <= 64 && a.max_query_len > kMixedRows) {
+      const int whole = static_cast<int>(2 * pairs - kManyGroups);
+      hipLaunchKernelGGL((delta_chunk_mixed_kernel<D>), dim3(kManyGroups), dim3(512), 0, st, a, whole, later);
+    } else {
+      launch(integral_constant<int, 8>{});
+    }
+  }
   else if (aligned && a.v_dim % 64 == 0) launch(integral_constant<int, 4>{});
   else launch(integral_constant<int, 2>{});
 }
