@@ -38,6 +38,10 @@ SHAPES = [
     (32, 32, 2, [1, 200, 600, 7]), (64, 96, 2, [129, 701]), (32, 128, 24, [70, 64, 9, 65, 66]), (128, 64, 2, [1200]),
     # a long portion among single rows and short ones; long ones side by side, whose cuts have neighbouring numbers
     (128, 128, 2, [1] * 9 + [1300] + [1] * 20 + [600, 7, 8, 400]), (32, 32, 2, [705, 1, 700, 1, 577, 640, 1]),
+    # eight multiplying and eight staging waves over segments: with the states chained by the segments themselves, in two slices of the
+    # columns, and by a launch of their own (eleven segments)
+    (128, 128, 20, [1300, 7, 300, 1]), (64, 128, 24, [5, 1217, 600]), (128, 256, 10, [1300, 600]), (128, 128, 12, [2112]),
+    (64, 128, 40, [9, 64, 65, 128, 127, 8, 3]),
 ]
 
 

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <algorithm>
+#include <utility>
 
 #include "common.h"
 
@@ -88,6 +89,12 @@ inline int64_t long_portions(int num_tokens, int num_seqs, int max_query_len) {
 }
 
 template <int X> struct Const { static constexpr int value = X; };
+
+// f(0), f(1), ... f(N - 1) with constants
+template <int N, typename F, int... I>
+__device__ __forceinline__ void unrolled(const F& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void unrolled(const F& f) { unrolled<N>(f, std::make_integer_sequence<int, N>{}); }
 
 // Inclusive sums over a wave's lanes: within 16 lanes, then the rows of 16 lanes before.
 template <typename T>

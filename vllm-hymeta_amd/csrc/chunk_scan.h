@@ -36,8 +36,8 @@ inline int scan_waves(int64_t lanes, int v_dim) {
 
 // A sequence's chunks follow each other in one workgroup per (head, value slice).  Where that leaves most of the chip idle,
 // the portions are cut into segments that run side by side: every segment but the last is summarised from a zero state (its
-// state and the sum of its log2 decays), the summaries are chained into the states in front of the segments, then every
-// segment runs from its state.  The summaries read the keys and values a second time, so fewer than three segments do not
+// state and the sum of its log2 decays), the summaries become the states in front of the segments, and every segment runs from
+// its state.  The summaries read the keys and values a second time, so fewer than three segments do not
 // pay.  What counts is the work there is (long_portions), not the sequences: single rows and short portions leave the chip to
 // a long prompt beside them.  8192 rows of 28 heads of 128 columns beside 63 single rows: lightning 194 us (705 with the
 // sequences counted), plain decays 159 (565); 6000 rows beside six portions of 700: 218 (495) and 157 (392).
@@ -49,8 +49,14 @@ inline int scan_waves(int64_t lanes, int v_dim) {
 // The segments of the portions of more than `rows` rows are numbered one behind the other (segment_at); there are no more than
 // one per `rows` rows of the step and one per such portion.  What has no rows comes behind what has: a workgroup that ends at
 // once in front of others leaves its compute unit idle while those share one (16 heads: 90 -> 145 us).
+//
+// Up to kMostUnchained segments every one works out the state in front of it for itself, from the summaries before it, which saves a
+// launch (6 to 9 us) for at most ten reads of 64 KB: 16 heads of 128 columns, five portions of 700 rows in four segments 41 -> 31 us, of
+// 64 columns three of 2000 64 -> 57; with 16 segments level.
+constexpr int kMostUnchained = 10;
 struct ScanSegments {
   int rows = 0x7fffffff, count = 0;        // rows of a segment; bound on the segments' numbers
+  bool chained = false;                    // whether a launch of its own turns the summaries into the states in front of the segments
   int64_t lanes = 0;                       // (segment, head) pairs that run side by side
 };
 // Segments of a step of `portions` long ones: how many of a head's fit on the chip beside the others.
@@ -69,6 +75,7 @@ inline ScanSegments scan_segments(int num_tokens, int num_seqs, int num_heads, i
   const int64_t count = cuts + std::min<int64_t>(num_seqs, cuts);
   if (num_seqs + count > 65535) return sg;
   sg.rows = rows, sg.count = static_cast<int>(count), sg.lanes *= (max_query_len + rows - 1) / rows;
+  sg.chained = (max_query_len + rows - 1) / rows > kMostUnchained;
   return sg;
 }
 // The workspace: per segment and head its summary, then the state in front of it; the segments' sums of log2 decays.
@@ -122,6 +129,41 @@ struct RowBuffer {
 // segments.
 __device__ __forceinline__ PieceAt segment_at(const ChunkScanArgs& a, int seg_rows, int number) {
   return piece_at(a.query_start_loc, a.num_seqs, number, [=](int rows) { return rows > seg_rows ? (rows - 1) / seg_rows + 1 : 0; });
+}
+
+// 16 columns of a state, by a wave.
+template <int D>
+__device__ __forceinline__ void copy_columns(const float* from, float* to, int64_t v_dim, int lane) {
+  float x[D / 4];
+#pragma unroll
+  for (int u = 0; u < D / 4; ++u) x[u] = from[(4 * u + lane / 16) * v_dim + lane % 16];
+#pragma unroll
+  for (int u = 0; u < D / 4; ++u) to[(4 * u + lane / 16) * v_dim + lane % 16] = x[u];
+}
+// A lane's rows d0 + 16 db + r of a state's column n (NULL: zeros).
+template <int DB>
+__device__ __forceinline__ void load_state(f32x4s (&S)[DB], const float* from, int d0, int v_dim, int n) {
+  const RowBuffer b(from);
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[db][r] = b.load1(from != nullptr, 4 * ((16 * db + d0 + r) * v_dim + n));
+}
+// The same of the state in front of a segment: the state in front of the portion (in the last segment's place, if there is one), then
+// from segment to segment 2^(its sum of log2 decays) of it and the segment's summary.
+template <int DB>
+__device__ __forceinline__ void segment_state(f32x4s (&S)[DB], const ChunkScanArgs& a, const PieceAt& seg, int seg_rows, int segments, int number, int h,
+                                              int64_t per_head, bool carry, int col0, int d0, int v_dim, int n) {
+  const int64_t step = a.num_heads * per_head, first = static_cast<int64_t>(number - seg.index) * a.num_heads + h;
+  const float *p = a.workspace + first * per_head + col0, *totals = a.workspace + segments * step + first;
+  load_state(S, carry ? p + (seg.rows - 1) / seg_rows * step : nullptr, d0, v_dim, n);
+  for (int i = 0; i < seg.index; ++i, p += step) {
+    f32x4s summary[DB];
+    load_state(summary, p, d0, v_dim, n);
+    const float decay = __builtin_amdgcn_exp2f(totals[i * a.num_heads]);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) S[db] = decay * S[db] + summary[db];
+  }
 }
 
 // A portion too short for a chunk, row by row in fp32 by the 64 NW threads of a workgroup: a thread holds 4 value columns of the
@@ -210,12 +252,10 @@ __global__ __launch_bounds__(64 * NW) void scan_short_kernel(ChunkScanArgs a, in
 // x 32 keys per wave, and handed over in LDS as fragments.  What enters a product from fp32 goes in as hi + lo parts, two
 // products, so that it keeps 16 bits of mantissa; so do the keys behind their silu in the state's update (three products: the
 // values, rounded to bf16 as in the outputs, carry the decays).
-// Bound by vector arithmetic between the barriers of a chunk: 2 x 16 cycles of exponential and reciprocal per silu'd value,
-// splits, scales: the vector pipes are busy 45 % of the time, the matrix pipes 18 %, LDS 35 %, memory far less.  One prompt of 8192 rows, 28 heads
-// of 128 x 128: lightning 351 -> 151 us (141 with the keys in one part), plain decays 283 -> 121; with 64 value columns and
-// decays per row 316 -> 131; before, 4 waves to 32 value columns, each such workgroup with its own staging, weights and an
-// image of the state in LDS.
-template <int D, int NW, bool Silu, bool Summarise>
+// Bound by vector arithmetic between the barriers of a chunk: silu, splits, scales.  One prompt of 8192 rows of 28 heads with 64 value
+// columns and decays per row 316 -> 131 us; before, 4 waves to 32 value columns, each such workgroup with its own staging, weights
+// and an image of the state in LDS.  (Eight waves: heads of 32 only; the others by chunk_scan_piped_kernel.)
+template <int D, int NW, bool Silu, bool Summarise, bool Chained>
 __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(ChunkScanArgs a, int seg_rows, int segments, bool short_too) {
   constexpr int NT = 64 * NW, KC = D / 8, VC = 2 * NW, KP = 2 * D, VP = 32 * NW, SD = D / 32, DB = D / 16;
   constexpr int KPT = (kScanRows * KC + NT - 1) / NT, VPT = 2;
@@ -247,7 +287,8 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
   if (rows_all < kScanMinRows || (whole && rows_all > seg_rows)) return;
   const int r_lo = whole ? 0 : seg.index * seg_rows, rows = r_lo + min(rows_all - r_lo, seg_rows);        // (end of this workgroup's rows)
   const bool last = rows == rows_all;
-  if (Summarise && last) return;                       // nothing comes behind the last segment
+  const bool copies = Summarise && last;               // nothing comes behind the last segment: its place holds the state in front of the portion
+  if (copies && Chained) return;
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = a.num_heads, Dv = a.v_dim, g = h / (H / a.num_qk_heads), col0 = vs * 16 * NW + 16 * wave;
@@ -259,7 +300,12 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
   // of log2 decays lie behind all the states
   const int64_t place = static_cast<int64_t>(number) * H + h;
   float* wsp = whole ? nullptr : a.workspace + place * D * Dv + col0;
-  const float* init = Summarise ? nullptr : whole ? (st != nullptr && a.context_lens[s] > 0 ? st : nullptr) : wsp;
+  const bool carry = st != nullptr && a.context_lens[s] > 0;
+  const float* init = Summarise ? nullptr : whole ? (carry ? st : nullptr) : wsp;
+  if (copies) {
+    if (carry && threadIdx.x < NT) copy_columns<D>(st, wsp, Dv, lane);
+    return;
+  }
   float seg_total = 0.f;
 
   const uint16_t* qp = a.q + static_cast<int64_t>(g) * D;
@@ -367,10 +413,14 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
 
   fetch(r_lo);
   f32x4s S[DB];                                        // S[16 db + 4 g4 + r][col0 + n]
+  if (Summarise || Chained || whole) {
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) S[db][r] = init ? init[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + n] : 0.f;
+      for (int r = 0; r < 4; ++r) S[db][r] = init ? init[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + n] : 0.f;
+  } else {
+    segment_state(S, a, seg, seg_rows, segments, number, h, D * Dv, carry, col0, 4 * g4, Dv, n);
+  }
   stage(min(kScanRows, rows - r_lo));
   fetch(r_lo + kScanRows);
   for (int c0 = r_lo; c0 < rows; c0 += kScanRows) {
@@ -517,6 +567,384 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
   if (Summarise && vs == 0 && tid == 0) a.workspace[static_cast<int64_t>(segments) * H * D * Dv + place] = seg_total;
 }
 
+// The same with 128 columns to a workgroup and heads of 64 and 128, by eight waves that multiply and eight that stage: the rows of the
+// next chunk go through their silu and into the other image of two while this one's products run, and so do the own weights, which
+// the multiplying waves need last.  A wave issues a vector instruction every five cycles or so however simple it is, and a SIMD
+// takes one in under three: two waves on a SIMD that do both, one behind the other, leave half of it idle (the kernel above: 12400 cycles a
+// chunk; with the staging dealt among the products of the same waves 12000; so 8600), and 128 registers hold either half.
+// Two barriers a chunk (one in Summarise): behind the first the own weights and the next keys beside the state times the queries,
+// behind the second the next queries and values beside the weights times the values and the state's update.
+// Bound by vector instructions: silu and splits of 24576 values a chunk, 60 % of it.  28 heads of 128 x 128, lightning: one prompt of
+// 8192 rows 146 -> 121 us, four of 1000 91 -> 73, six of 1365 124 -> 99; plain decays: one of 8192 109 -> 95.
+template <int D, bool Silu, bool Summarise, bool Chained>
+__global__ __launch_bounds__(1024, 4) void chunk_scan_piped_kernel(ChunkScanArgs a, int seg_rows, int segments, bool short_too) {
+  constexpr int NW = 8, NT = 64 * NW, KC = D / 8, VC = 2 * NW, KP = 2 * D, VP = 32 * NW, SD = D / 32, DB = D / 16;
+  constexpr int KPT = kScanRows * KC / NT, VPT = 2, kKeyImage = kScanRows * KP, kValueImage = kScanRows * VP;
+  static_assert(kScanRows * KC % NT == 0, "every thread stages whole chunks of 16 bytes");
+  typedef ChunkOrder<KC> KOrder;
+  typedef ChunkOrder<VC> VOrder;
+  __shared__ __attribute__((aligned(16))) char s_k[2 * kKeyImage], s_v[2 * kValueImage];
+  __shared__ __attribute__((aligned(16))) char s_q[Summarise ? 16 : 2 * kKeyImage], s_klo[Silu ? 2 * kKeyImage : 16];
+  __shared__ __attribute__((aligned(16))) u32x4 s_p[Summarise ? 1 : 6][2][64];
+  __shared__ __attribute__((aligned(16))) float s_cum[2][kScanRows], s_b[2][kScanRows], s_w[2][kScanRows];
+  const int h = blockIdx.x, vs = blockIdx.y, number = blockIdx.z;
+  const bool whole = number >= segments;
+  PieceAt seg;
+  if (!whole) {
+    seg = segment_at(a, seg_rows, number);
+    if (seg.seq < 0) return;
+  } else {
+    seg.seq = number - segments, seg.index = 0;
+    seg.row0 = a.query_start_loc[seg.seq], seg.rows = a.query_start_loc[seg.seq + 1] - seg.row0;
+  }
+  const int s = seg.seq, r0 = seg.row0, rows_all = seg.rows;
+  if (rows_all <= 0) return;                           // (a sequence without rows: its slot may be anything)
+  if constexpr (!Summarise) {
+    static_assert(sizeof(s_k) >= 16 * D && sizeof(s_v) >= 2048 * NW, "the scratch of single rows");
+    if (rows_all < kScanMinRows) {                     // (a segment has more)
+      if (short_too && threadIdx.x < NT) scan_single_rows<D, NW, Silu>(a, h, s, r0, rows_all, vs * 16 * NW, reinterpret_cast<float*>(s_k), reinterpret_cast<float*>(s_v));
+      return;
+    }
+  }
+  if (rows_all < kScanMinRows || (whole && rows_all > seg_rows)) return;
+  const int r_lo = whole ? 0 : seg.index * seg_rows, rows = r_lo + min(rows_all - r_lo, seg_rows);        // (end of this workgroup's rows)
+  const bool last = rows == rows_all;
+  const bool copies = Summarise && last;               // nothing comes behind the last segment: its place holds the state in front of the portion
+  if (copies && Chained) return;
+  const int tid = threadIdx.x % NT, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
+  const int all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = all % NW;
+  const bool stager = all >= NW;
+  const int H = a.num_heads, Dv = a.v_dim, g = h / (H / a.num_qk_heads), col0 = vs * 16 * NW + 16 * wave;
+  const int slot = a.slot_idx[s];
+  float* st = slot >= 0 ? a.state + (static_cast<int64_t>(slot) * H + h) * D * Dv + col0 : nullptr;
+  const float l2_const = a.decay ? fmaxf(a.decay[h] > 0.f ? log2f(a.decay[h]) : -INFINITY, kMinLog2) : 0.f;
+  const float skip = a.skip ? a.skip[h] : 0.f;
+  // (places in the workspace: as above)
+  const int64_t place = static_cast<int64_t>(number) * H + h;
+  float* wsp = whole ? nullptr : a.workspace + place * D * Dv + col0;
+  const bool carry = st != nullptr && a.context_lens[s] > 0;
+  const float* init = Summarise ? nullptr : whole ? (carry ? st : nullptr) : wsp;
+  if (copies) {
+    if (carry && threadIdx.x < NT) copy_columns<D>(st, wsp, Dv, lane);
+    return;
+  }
+  float seg_total = 0.f;
+
+  const uint16_t* qp = a.q + static_cast<int64_t>(g) * D;
+  const uint16_t* kp = a.k + static_cast<int64_t>(g) * D;
+  const uint16_t* vp = a.v + static_cast<int64_t>(h) * Dv + vs * 16 * NW;
+  u32x4 rk[KPT], rq[Summarise ? 1 : KPT], rv[VPT];
+  float rl = 0.f, rb = 0.f;
+  auto fetch_rows = [&](auto& to, const uint16_t* base, int64_t stride, auto chunks, int c0) __attribute__((always_inline)) {
+    constexpr int kChunks = decltype(chunks)::value;
+    const int nrow = min(kScanRows, rows - c0);
+    const RowBuffer r(base + (r0 + c0) * stride);
+#pragma unroll
+    for (int u = 0; u < static_cast<int>(sizeof(to) / sizeof(to[0])); ++u) {
+      const int idx = tid + NT * u, j = idx / kChunks, ch = idx % kChunks;
+      to[u] = r.load(j < nrow, 2 * (j * static_cast<int>(stride) + 8 * ch));
+    }
+  };
+  auto fetch_keys = [&](int c0) __attribute__((always_inline)) {
+    fetch_rows(rk, kp, a.k_stride, Const<KC>{}, c0);
+    const int nrow = min(kScanRows, rows - c0), at = 4 * lane * H;
+    const int64_t t0 = r0 + c0;
+    if (a.log2_decay || a.v_scale) {
+      rl = RowBuffer(a.log2_decay + t0 * H + h).load1(a.log2_decay && lane < nrow, at);
+      rb = RowBuffer(a.v_scale + t0 * H + h).load1(a.v_scale && lane < nrow, at);
+    }
+  };
+  auto fetch_queries = [&](int c0) __attribute__((always_inline)) {
+    if constexpr (!Summarise) fetch_rows(rq, qp, a.q_stride, Const<KC>{}, c0);
+  };
+  auto fetch_values = [&](int c0) __attribute__((always_inline)) { fetch_rows(rv, vp, a.v_stride, Const<VC>{}, c0); };
+  // Half `i` of a 16-byte chunk of this thread's keys, queries or values into image `to`: four values side by side, stored with the
+  // second half.  (Rows past the portion were fetched as zeros, and silu(0) = 0.)
+  u32x4 half_hi, half_lo;
+  auto half = [&](const u32x4& raw, int i) __attribute__((always_inline)) {
+    float x[4], y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = e & 1 ? hi_bf(raw[2 * i + e / 2]) : lo_bf(raw[2 * i + e / 2]);
+    if constexpr (Silu) {                              // (silu_fast, step by step)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = -1.4426950408889634f * x[e];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = __builtin_amdgcn_exp2f(y[e]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = 1.f + y[e];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = __builtin_amdgcn_rcpf(y[e]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] *= y[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      uint32_t hi = raw[2 * i + e], lo = 0;
+      if constexpr (Silu) split_pair(x[2 * e], x[2 * e + 1], hi, lo);
+      half_hi[2 * i + e] = hi, half_lo[2 * i + e] = lo;
+    }
+  };
+  auto key_half = [&](int i, int to) __attribute__((always_inline)) {
+    half(rk[i / 2], i % 2);
+    if (i % 2 == 0) return;
+    const int idx = tid + NT * (i / 2), j = idx / KC, ch = idx % KC, at = to * kKeyImage + j * KP + 16 * (ch ^ KOrder::twist(j));
+    st16(s_k + at, half_hi);
+    if constexpr (Silu) st16(s_klo + at, half_lo);
+  };
+  auto query_half = [&](int i, int to) __attribute__((always_inline)) {
+    if constexpr (!Summarise) {
+      half(rq[i / 2], i % 2);
+      if (i % 2 == 0) return;
+      const int idx = tid + NT * (i / 2), j = idx / KC, ch = idx % KC;
+      st16(s_q + to * kKeyImage + j * KP + 16 * (ch ^ KOrder::twist(j)), half_hi);
+    }
+  };
+  auto value_half = [&](int i, int to) __attribute__((always_inline)) {
+    half(rv[i / 2], i % 2);
+    if (i % 2 == 0) return;
+    const int idx = tid + NT * (i / 2), j = idx / VC, ch = idx % VC;
+    st16(s_v + to * kValueImage + j * VP + 16 * (ch ^ VOrder::twist(j)), half_hi);
+  };
+  constexpr int kKeyHalves = 2 * KPT, kValueHalves = 2 * VPT;
+  // running sums of a chunk's log2 decays (rows past the portion add 0), by the first of the staging waves
+  auto stage_decays = [&](int nrow, int to) __attribute__((always_inline)) {
+    if (wave != 0) return;
+    const float cum = a.log2_decay ? lane_sums(fmaxf(rl, kMinLog2)) : static_cast<float>(min(lane + 1, nrow)) * l2_const;
+    const float total = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cum), 63));
+    s_cum[to][lane] = cum;
+    const float b = a.v_scale ? rb : 1.f;
+    s_b[to][lane] = b;
+    const float left = Silu ? static_cast<float>(nrow - 1 - lane) * l2_const : total - cum;
+    s_w[to][lane] = lane < nrow ? __builtin_amdgcn_exp2f(left) * b : 0.f;
+  };
+  // LDS offsets of this lane's fragments: as above
+  const int kt = KOrder::twist(n), Rt = 4 * g4 + (n >> 2), kT = KOrder::twist(Rt), vT = VOrder::twist(Rt);
+  auto row_frag = [&](const char* img, int block, int sd) { return __builtin_bit_cast(bf16x8, ld16(img + (16 * block + n) * KP + 16 * ((4 * sd + g4) ^ kt))); };
+  auto row_frag_halves = [&](const char* img, int block, int sd) {
+    const char* row = img + (16 * block + n) * KP + 8 * (g4 & 1);
+    const u32x2 x = *reinterpret_cast<const u32x2*>(row + 16 * ((4 * sd + (g4 >> 1)) ^ kt));
+    const u32x2 y = *reinterpret_cast<const u32x2*>(row + 16 * ((4 * sd + 2 + (g4 >> 1)) ^ kt));
+    return __builtin_bit_cast(bf16x8, (u32x4{x[0], x[1], y[0], y[1]}));
+  };
+  auto key_frag = [&](const char* img, int db, int kk) {
+    const char* p = img + (32 * kk + Rt) * KP + 16 * ((2 * db + ((n & 3) >> 1)) ^ kT) + 8 * (n & 1);
+    return frag_of(read_transposed(p), read_transposed(p + 16 * KP));
+  };
+  auto value_frag = [&](const char* img, int kk) {
+    const char* p = img + (32 * kk + Rt) * VP + 16 * ((2 * wave + ((n & 3) >> 1)) ^ vT) + 8 * (n & 1);
+    return frag_of(read_transposed(p), read_transposed(p + 16 * VP));
+  };
+
+  // ---- the staging waves
+  // A block of the own weights of the chunk in image `cur` as hi + lo fragments: rows 16 ib + n, keys 32 wk ..
+  auto own_weights = [&](int cur) __attribute__((always_inline)) {
+    const int ib = wave >> 1, wk = wave & 1, i = 16 * ib + n;
+    if (2 * wk > ib) return;
+    const char *kimg = s_k + cur * kKeyImage, *qimg = s_q + cur * kKeyImage;
+    bf16x8 own_q[SD], own_k[SD][2];
+#pragma unroll
+    for (int sd = 0; sd < SD; ++sd) {
+      own_q[sd] = row_frag(qimg, ib, sd);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) own_k[sd][t] = row_frag(kimg, 2 * wk + t, sd);       // (block 2 wk + 1 may lie behind the rows: masked)
+    }
+    const float cum_i = s_cum[cur][i];
+    f32x4s sc[2], cum_j[2], b_j[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      sc[t] = f32x4s{0.f, 0.f, 0.f, 0.f};
+      if constexpr (!Silu) {
+        const int j = 16 * (2 * wk + t) + 4 * g4;
+        cum_j[t] = *reinterpret_cast<const f32x4s*>(s_cum[cur] + j), b_j[t] = *reinterpret_cast<const f32x4s*>(s_b[cur] + j);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);                 // (all on their way: left to itself the compiler waits for each)
+#pragma unroll
+    for (int sd = 0; sd < SD; ++sd)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) sc[t] = scan_mfma(own_k[sd][t], own_q[sd], sc[t]);
+    u32x4 hi, lo;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      float p[2];
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        const int t = x >> 1, r = 2 * (x & 1) + y, j = 16 * (2 * wk + t) + 4 * g4 + r;
+        float span, bj = 1.f;                          // log2 of the decay between row j and row i; j's input weight
+        if constexpr (Silu) span = static_cast<float>(i - j) * l2_const;
+        else span = cum_i - cum_j[t][r], bj = b_j[t][r];
+        p[y] = j <= i ? sc[t][r] * __builtin_amdgcn_exp2f(span) * bj : 0.f;
+      }
+      uint32_t a, b;
+      split_pair(p[0], p[1], a, b);
+      hi[x] = a, lo[x] = b;
+    }
+    const int at = ib < 2 ? ib : 2 * ib - 2 + wk;
+    s_p[at][0][lane] = hi;
+    s_p[at][1][lane] = lo;
+  };
+
+  // ---- the multiplying waves
+  f32x4s S[DB], o[4];                                  // S[16 db + 4 g4 + r][col0 + n]
+  bf16x8 vf[2];
+  u32x4 wv[2][2];                                      // the values with the decays up to the chunk's end, hi and lo
+  // the state before the chunk times the queries
+  auto state_times_queries = [&](int cur) __attribute__((always_inline)) {
+    const char* qimg = s_q + cur * kKeyImage;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) o[x] = f32x4s{0.f, 0.f, 0.f, 0.f};
+    float cum[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) cum[x] = s_cum[cur][16 * x + n];
+    bf16x8 qf[6];                                      // of two blocks of rows a step of 32 d ahead
+    u32x4 sf[2][2];                                    // the state's d 32 sd + 4 g4 + e for e < 4, 32 sd + 16 + 4 g4 + e - 4 after, hi and lo
+    auto read_queries = [&](int sd, int x) __attribute__((always_inline)) { qf[x < 2 ? x + 4 * (sd & 1) : x] = row_frag_halves(qimg, x, sd); };
+    auto split_state = [&](int sd, int e) __attribute__((always_inline)) {
+      uint32_t x, y;
+      split_pair(S[2 * sd + (e >> 1)][2 * (e & 1)], S[2 * sd + (e >> 1)][2 * (e & 1) + 1], x, y);
+      sf[sd & 1][0][e] = x, sf[sd & 1][1][e] = y;
+    };
+    read_queries(0, 0), read_queries(0, 1);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) split_state(0, e);
+    __builtin_amdgcn_sched_barrier(0);
+    unrolled<8 * SD>([&](auto at) __attribute__((always_inline)) {
+      constexpr int step = decltype(at)::value, sd = step / 8, x = step % 8 < 4 ? step % 2 : 2 + step % 2, part = step / 2 % 2;
+      if constexpr (step % 8 == 0) read_queries(sd, 2), read_queries(sd, 3);
+      if constexpr (step % 8 == 4 && sd + 1 < SD) read_queries(sd + 1, 0), read_queries(sd + 1, 1);
+      o[x] = scan_mfma(__builtin_bit_cast(bf16x8, sf[sd & 1][part]), qf[x < 2 ? x + 4 * (sd & 1) : x], o[x]);
+      if constexpr (sd + 1 < SD && step % 2 == 0) split_state(sd + 1, step % 8 / 2);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+#pragma unroll
+    for (int x = 0; x < 4; ++x) o[x] *= __builtin_amdgcn_exp2f(cum[x]);
+    if (skip != 0.f) {
+      const char* vimg = s_v + cur * kValueImage;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const u32x2 vi = *reinterpret_cast<const u32x2*>(vimg + (16 * x + n) * VP + 16 * ((2 * wave + (g4 >> 1)) ^ VOrder::twist(n)) + 8 * (g4 & 1));
+        o[x][0] = fmaf(skip, lo_bf(vi[0]), o[x][0]), o[x][1] = fmaf(skip, hi_bf(vi[0]), o[x][1]);
+        o[x][2] = fmaf(skip, lo_bf(vi[1]), o[x][2]), o[x][3] = fmaf(skip, hi_bf(vi[1]), o[x][3]);
+      }
+    }
+  };
+  auto read_values = [&](int cur) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) vf[kk] = value_frag(s_v + cur * kValueImage, kk);
+  };
+  auto weigh_values = [&](int cur) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const u32x4 x = __builtin_bit_cast(u32x4, vf[kk]);
+      const f32x4s w0 = *reinterpret_cast<const f32x4s*>(s_w[cur] + 32 * kk + 4 * g4), w1 = *reinterpret_cast<const f32x4s*>(s_w[cur] + 32 * kk + 16 + 4 * g4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float wa = e < 2 ? w0[2 * e] : w1[2 * e - 4], wb = e < 2 ? w0[2 * e + 1] : w1[2 * e - 3];
+        uint32_t hi, lo;
+        split_pair(lo_bf(x[e]) * wa, hi_bf(x[e]) * wb, hi, lo);
+        wv[kk][0][e] = hi, wv[kk][1][e] = lo;
+      }
+    }
+  };
+  // the own weights times the values
+  auto finish_rows = [&](int c0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int part = 0; part < 2; ++part) {
+      u32x4 pf[6];
+#pragma unroll
+      for (int at = 0; at < 6; ++at) pf[at] = s_p[at][part][lane];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int x = 2 * kk; x < 4; ++x) o[x] = scan_mfma(vf[kk], __builtin_bit_cast(bf16x8, pf[x < 2 ? x : 2 * x - 2 + kk]), o[x]);
+    }
+    const int nrow = min(kScanRows, rows - c0);
+    const RowBuffer to(a.out + (static_cast<int64_t>(r0 + c0) * H + h) * Dv + col0);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) to.store(16 * x + n < nrow, 4 * ((16 * x + n) * H * Dv + 4 * g4), o[x]);
+  };
+  // the state after the chunk
+  auto update_state = [&](int cur, float total) __attribute__((always_inline)) {
+    const char *kimg = s_k + cur * kKeyImage, *klo = s_klo + (Silu ? cur * kKeyImage : 0);
+    const float chunk_decay = __builtin_amdgcn_exp2f(total);
+    bf16x8 kf[2][Silu ? 2 : 1];                        // fragments of 32 keys and 16 d, one set ahead of its products
+    auto read_keys = [&](int at) __attribute__((always_inline)) {
+      kf[at & 1][0] = key_frag(kimg, at / 2, at & 1);
+      if constexpr (Silu) kf[at & 1][1] = key_frag(klo, at / 2, at & 1);
+    };
+    read_keys(0);
+#pragma unroll
+    for (int at = 0; at < 2 * DB; ++at) {
+      const int db = at / 2, kk = at & 1;
+      if (at + 1 < 2 * DB) read_keys(at + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kk == 0) S[db] *= chunk_decay;
+      S[db] = scan_mfma(kf[kk][0], __builtin_bit_cast(bf16x8, wv[kk][0]), S[db]);
+      S[db] = scan_mfma(kf[kk][0], __builtin_bit_cast(bf16x8, wv[kk][1]), S[db]);
+      if constexpr (Silu) S[db] = scan_mfma(kf[kk][1], __builtin_bit_cast(bf16x8, wv[kk][0]), S[db]);
+    }
+  };
+
+  // (a loop for either kind of waves, with the same barriers: in one loop the registers of both would be alive at once)
+  if (stager) {
+    fetch_keys(r_lo), fetch_queries(r_lo), fetch_values(r_lo);
+#pragma unroll
+    for (int i = 0; i < kKeyHalves; ++i) key_half(i, 0);
+#pragma unroll
+    for (int i = 0; i < kKeyHalves; ++i) query_half(i, 0);
+#pragma unroll
+    for (int i = 0; i < kValueHalves; ++i) value_half(i, 0);
+    stage_decays(min(kScanRows, rows - r_lo), 0);
+    fetch_keys(r_lo + kScanRows), fetch_queries(r_lo + kScanRows), fetch_values(r_lo + kScanRows);      // (no row past the segment is read)
+    for (int c0 = r_lo, cur = 0; c0 < rows; c0 += kScanRows, cur ^= 1) {
+      const bool more = c0 + kScanRows < rows;
+      const int next = cur ^ 1;
+      __syncthreads();                                 // the chunk is there, and nobody reads the other image
+      if constexpr (!Summarise) own_weights(cur);
+      if (more) {
+#pragma unroll
+        for (int i = 0; i < kKeyHalves; ++i) key_half(i, next);
+        stage_decays(min(kScanRows, rows - c0 - kScanRows), next);
+        fetch_keys(c0 + 2 * kScanRows);
+      }
+      if constexpr (!Summarise) __syncthreads();       // the own weights are there
+      if (more) {
+#pragma unroll
+        for (int i = 0; i < kKeyHalves; ++i) query_half(i, next);
+        fetch_queries(c0 + 2 * kScanRows);
+#pragma unroll
+        for (int i = 0; i < kValueHalves; ++i) value_half(i, next);
+        fetch_values(c0 + 2 * kScanRows);
+      }
+    }
+    return;
+  }
+  if (Summarise || Chained || whole) load_state(S, init, 4 * g4, Dv, n);
+  else segment_state(S, a, seg, seg_rows, segments, number, h, D * Dv, carry, col0, 4 * g4, Dv, n);
+  for (int c0 = r_lo, cur = 0; c0 < rows; c0 += kScanRows, cur ^= 1) {
+    __syncthreads();
+    const float total = s_cum[cur][kScanRows - 1];
+    seg_total += total;
+    if constexpr (!Summarise) state_times_queries(cur);
+    read_values(cur);
+    if constexpr (!Summarise) {
+      __syncthreads();
+      finish_rows(c0);
+    }
+    weigh_values(cur);
+    update_state(cur, total);
+  }
+  float* to = Summarise ? wsp : (last ? st : nullptr);
+  if (to != nullptr) {
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) to[static_cast<int64_t>(16 * db + 4 * g4 + r) * Dv + n] = S[db][r];
+  }
+  if (Summarise && vs == 0 && tid == 0) a.workspace[static_cast<int64_t>(segments) * H * D * Dv + place] = seg_total;
+}
+
 // The segments' summaries (each segment's state had it started from zero) become the states in front of the segments:
 // run = carried state; per segment: place <- run, run <- 2^(segment's sum of log2 decays) run + summary.  Four elements per
 // thread.  grid = (heads, segments, parts per segment): a portion's workgroups deal the parts of 1024 elements among them.
@@ -558,11 +986,22 @@ template <int D, int NW, bool Silu>
 void launch_chunk_scan_as(const ChunkScanArgs& a, ScanSegments sg, bool short_too, hipStream_t st) {
   const dim3 block(64 * NW);
   const unsigned slices = a.v_dim / (16 * NW);
+  auto scan = [&](auto summarise, unsigned pieces, bool shorts) {
+    constexpr bool Summarise = decltype(summarise)::value;
+    const dim3 grid(a.num_heads, slices, pieces);
+    auto launch = [&](auto chained) {
+      constexpr bool Chained = decltype(chained)::value;
+      if constexpr (NW == 8 && D >= 64) hipLaunchKernelGGL((chunk_scan_piped_kernel<D, Silu, Summarise, Chained>), grid, dim3(1024), 0, st, a, sg.rows, sg.count, shorts);
+      else hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, Summarise, Chained>), grid, block, 0, st, a, sg.rows, sg.count, shorts);
+    };
+    if (sg.count > 0 && !sg.chained) launch(std::false_type{});
+    else launch(std::true_type{});
+  };
   if (sg.count > 0) {
-    hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, true>), dim3(a.num_heads, slices, sg.count), block, 0, st, a, sg.rows, sg.count, false);
-    hipLaunchKernelGGL(chunk_scan_chain_kernel, dim3(a.num_heads, sg.count, (D * a.v_dim + 3071) / 3072), dim3(256), 0, st, a, D, sg.rows, sg.count);
+    scan(std::true_type{}, sg.count, false);
+    if (sg.chained) hipLaunchKernelGGL(chunk_scan_chain_kernel, dim3(a.num_heads, sg.count, (D * a.v_dim + 3071) / 3072), dim3(256), 0, st, a, D, sg.rows, sg.count);
   }
-  hipLaunchKernelGGL((chunk_scan_kernel<D, NW, Silu, false>), dim3(a.num_heads, slices, sg.count + a.num_seqs), block, 0, st, a, sg.rows, sg.count, short_too);
+  scan(std::false_type{}, sg.count + a.num_seqs, short_too);
 }
 
 // Portions too short for a chunk run in the chunks' launch, where they cost no launch (about 4 us) and fill what a long portion

@@ -359,12 +359,6 @@ struct ChunkPlace {
 };
 static_assert(sizeof(ChunkPlace) % 16 == 0, "16-byte loads of every place");
 
-// f(0), f(1), ... f(N - 1) with constants
-template <int N, typename F, int... I>
-__device__ __forceinline__ void unrolled(const F& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
-template <int N, typename F>
-__device__ __forceinline__ void unrolled(const F& f) { unrolled<N>(f, std::make_integer_sequence<int, N>{}); }
-
 __device__ __forceinline__ f32x4v mfma16(bf16x8 a, bf16x8 b, f32x4v c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ bf16x8 frag(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
