@@ -848,7 +848,35 @@ def load() -> C.CDLL:
     if version != ABI_VERSION:
         raise RuntimeError(f"{path}: ABI version {version}, binding expects {ABI_VERSION}")
     _lib = lib
+    _load_calls(lib)
     return lib
+
+
+# The native host side of small calls (csrc/calls.cpp): None until the library is loaded, or where it is not built or the library
+# lacks a function of its.
+calls = None
+_CALLS_NAME = "hymeta_calls.so"
+_CALLED = ("hymeta_sink_attention", "hymeta_sink_attention_workspace_bytes", "hymeta_sink_attention_portion_workspace_bytes",
+           "hymeta_meta_swa_paged_decode", "hymeta_meta_swa_paged_decode_splits", "hymeta_meta_swa_paged_decode_workspace_bytes",
+           "hymeta_meta_swa_prefill", "hymeta_meta_swa_prefill_splits", "hymeta_meta_swa_prefill_workspace_bytes",
+           "hymeta_lightning_attention", "hymeta_lightning_attention_workspace_bytes", "hymeta_decay_scan", "hymeta_decay_scan_workspace_bytes",
+           "hymeta_delta_rule", "hymeta_delta_rule_workspace_bytes")
+
+
+def _load_calls(lib: C.CDLL) -> None:
+    global calls
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), _CALLS_NAME)
+    if not os.path.exists(path) or any(name in _missing for name in _CALLED):
+        return
+    import importlib.machinery
+    import importlib.util
+
+    from . import hip_ops
+    loader = importlib.machinery.ExtensionFileLoader("hymeta_calls", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("hymeta_calls", loader))
+    loader.exec_module(module)
+    module.setup(hip_ops, *(C.cast(getattr(lib, name), C.c_void_p).value for name in _CALLED))
+    calls = module
 
 
 class HymetaError(RuntimeError):

@@ -40,6 +40,22 @@ def _p(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+_empty = torch.empty
+
+
+def _native(t: torch.Tensor):
+    """The native calls (csrc/calls.cpp), where they stand for what is below them here: for device tensors, and while outputs come from
+    torch itself (what is put in ``torch.empty``'s place is asked for them)."""
+    return _C.calls if t.is_cuda and torch.empty is _empty else None
+
+
+def _answer(out, what: str) -> torch.Tensor:
+    """What a function of ``_C.calls`` answered: an output, or the library's status."""
+    if type(out) is int:
+        _C.check(out, what)
+    return out
+
+
 def _require(cond: bool, msg: str) -> None:
     if not cond:
         raise ValueError(msg)
@@ -511,6 +527,12 @@ def meta_swa_paged_decode(
     own fixed device array; no workspace is allocated or passed; pass ``out`` to allocate nothing at all).
     With ``new_key`` / ``new_value`` [B,Hkv,D] and ``slot_mapping`` int64 [B] the call first writes the
     decoded tokens' K/V rows into the cache (the fused form of ``reshape_and_cache`` + decode)."""
+    native = _native(q)
+    if native is not None and out is None and workspace is None and new_key is None and not static_scratch:
+        done = native.meta_swa_paged_decode(q, key_cache, value_cache, cache_seqlens, block_tables, meta_key, meta_value, window_left,
+                                          0.0 if scale is None else scale, max_seqlen_k, num_splits, _stream(q))
+        if done is not None:
+            return _answer(done, "hymeta_meta_swa_paged_decode")
     _dev(q, key_cache, value_cache, cache_seqlens, block_tables, meta_key, meta_value, out, workspace,
          new_key, new_value, slot_mapping)
     B, H, D = q.shape
@@ -609,6 +631,12 @@ def meta_swa_prefill(
     block_tables + seq_lens_k.  Returns [(M if meta_query)+T, H, D] bf16, meta rows first.
     ``max_seqlen_k`` (0: unknown) and ``num_splits`` (0: library's choice) steer the key slicing of
     short chunks of long sequences."""
+    native = _native(q)
+    if native is not None and block_tables is not None and key is None and value is None and cu_seqlens_k is None and meta_query is None and out is None:
+        done = native.meta_swa_prefill(q, cu_seqlens_q, max_seqlen_q, key_cache, value_cache, block_tables, seq_lens_k, meta_key, meta_value, window_left,
+                                       0.0 if scale is None else scale, max_seqlen_k, num_splits, _stream(q))
+        if done is not None:
+            return _answer(done, "hymeta_meta_swa_prefill")
     _dev(q, cu_seqlens_q, key, value, cu_seqlens_k, key_cache, value_cache, block_tables,
          seq_lens_k, meta_query, meta_key, meta_value, out)
     T, H, D = q.shape
@@ -1749,6 +1777,13 @@ def sink_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_tables: torch.
     ``bias_b``): the bias is ``slopes[h] (i - j)``.  ``chunk > 0`` (in place of ``window_left``): a query sees the keys of its own run of
     ``chunk`` positions, counted from the sequence's first token.  ``scaled_key``: cache rows as ``scaled_key_cache_`` writes them.  ``value_in_key``: a cache row holds ``D`` elements per key/value
     head, the first ``Dv`` of which are also the value (a latent that keys and values share).  Returns ``[T, H, Dv]``."""
+    native = _native(q)
+    if native is not None:
+        out = native.sink_attention(q, kv_cache, block_tables, query_start_loc, seq_lens, num_kv_heads, head_dim, v_dim, scale, max_query_len, max_seq_len,
+                                    bias_a, bias_b, sink, window_left, sink_logits, value_in_key, shared_key, keep_first, softcap, head_gate, scaled_key,
+                                    slopes, elem_gate, chunk, _stream(q))
+        if out is not None:
+            return _answer(out, "hymeta_sink_attention")
     _dev(q, kv_cache, block_tables, query_start_loc, seq_lens, bias_a, bias_b, sink_logits, slopes, elem_gate)
     _require(q.dim() == 3 and q.stride(2) == 1 and q.stride(1) == head_dim and q.shape[2] == head_dim, "q must be [T, H, D] with contiguous heads")
     T, H, _ = q.shape
@@ -2031,6 +2066,11 @@ def lightning_attention(qkv: torch.Tensor, state: torch.Tensor, decay: torch.Ten
                         query_start_loc: torch.Tensor, context_lens: torch.Tensor, slot_idx: torch.Tensor, max_query_len: int) -> torch.Tensor:
     """Linear attention with a decay per head over a step's rows: ``qkv [T, 2 H D + H Dv]`` (before their silu), ``state``
     fp32 ``[slots, H, D, Dv]`` read where ``context_lens > 0`` and written.  Returns fp32 ``[T, H Dv]``."""
+    native = _native(qkv)
+    if native is not None:
+        out = native.lightning_attention(qkv, decay, num_heads, head_dim, v_dim, state, query_start_loc, context_lens, slot_idx, max_query_len, _stream(qkv))
+        if out is not None:
+            return _answer(out, "hymeta_lightning_attention")
     _dev(qkv, state, decay, query_start_loc, context_lens, slot_idx)
     H, D, Dv = num_heads, head_dim, v_dim
     _require(qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.shape[1] >= H * (2 * D + Dv), "qkv must be row-contiguous [T, 2 H D + H Dv]")
@@ -2517,6 +2557,11 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.T
     ``v [T, H, Dv]`` (views with any row stride; head ``h`` reads query / key head ``h // (H / Hqk)``), ``state`` fp32
     ``[slots, H, D, Dv]`` read where ``context_lens > 0`` and written.  ``a_t``: ``decay [H]`` for every token, or
     ``2 ** log2_decay[t, h]``; ``b_t``: ``v_scale [T, H]`` or 1.  Returns fp32 ``[T, H Dv]``."""
+    native = _native(q)
+    if native is not None:
+        out = native.decay_scan(q, k, v, state, query_start_loc, context_lens, slot_idx, max_query_len, decay, log2_decay, v_scale, skip, _stream(q))
+        if out is not None:
+            return _answer(out, "hymeta_decay_scan")
     _dev(q, k, v, state, query_start_loc, context_lens, slot_idx, decay, log2_decay, v_scale, skip)
     _require(q.dim() == 3 and k.shape == q.shape and v.dim() == 3 and q.dtype == k.dtype == v.dtype and q.dtype in _DT, "q, k [T, Hqk, D] and v [T, H, Dv] of one type")
     T, Hqk, D = q.shape
@@ -2570,6 +2615,11 @@ def delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta_logit: to
     fp32 ``[T, H]``, ``state`` fp32 ``[slots, H, D, Dv]`` read where ``context_lens > 0`` and written.  Returns fp32 ``[T, H Dv]``;
     with ``norm_weight [Dv]`` (a step of single rows, ``delta_rule_step_supported``) ``rmsnorm(o) * norm_weight * silu(gate)``
     per head in the activations' type."""
+    native = _native(q)
+    if native is not None and norm_weight is None and gate is None:
+        out = native.delta_rule(q, k, v, beta_logit, log2_decay, state, query_start_loc, context_lens, slot_idx, max_query_len, q_scale, unit_eps, _stream(q))
+        if out is not None:
+            return _answer(out, "hymeta_delta_rule")
     _dev(q, k, v, beta_logit, log2_decay, state, query_start_loc, context_lens, slot_idx, norm_weight, gate)
     _require(q.dim() == 3 and k.shape == q.shape and v.dim() == 3 and q.dtype == k.dtype == v.dtype == beta_logit.dtype and q.dtype in _DT,
              "q, k [T, Hqk, D], v [T, H, Dv] and beta_logit [T, H] of one type")
