@@ -42,6 +42,9 @@ SHAPES = [
     # columns, and by a launch of their own (eleven segments)
     (128, 128, 20, [1300, 7, 300, 1]), (64, 128, 24, [5, 1217, 600]), (128, 256, 10, [1300, 600]), (128, 128, 12, [2112]),
     (64, 128, 40, [9, 64, 65, 128, 127, 8, 3]),
+    # the shortest segments: of one chunk, with the least rows that are cut and one fewer; beside as many single rows as leave 192 rows each
+    (128, 128, 28, [192, 1, 65]), (128, 128, 28, [191]), (64, 128, 16, [520, 40]), (128, 64, 8, [193, 192, 191, 64]), (32, 32, 64, [577] + [1] * 64),
+    (32, 32, 64, [577, 300] + [1] * 64),
 ]
 
 

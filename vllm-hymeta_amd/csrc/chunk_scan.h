@@ -43,8 +43,11 @@ inline int scan_waves(int64_t lanes, int v_dim) {
 // sequences counted), plain decays 159 (565); 6000 rows beside six portions of 700: 218 (495) and 157 (392).
 // As many segments as run at the same time, eight waves to a compute unit: one prompt of 8192 rows of 28 heads of 128
 // columns took 138 us (lightning, the keys in one part) and 120 (plain decays) in 256 workgroups of eight waves, 152 and 136 in 512, 175 and 156
-// in 1024; of 64 columns 131 us in 512 workgroups of four, 189 in 256, 147 in 1024.  At least 192 rows each: three portions
-// of 700 rows of 16 heads took 39 us in three segments, 49 in one.
+// in 1024; of 64 columns 131 us in 512 workgroups of four, 189 in 256, 147 in 1024.  At least 64 rows each (192 / 64, us): 28 heads
+// of 128 x 128, one portion of 300 rows 27.9 / 22.8, of 520 46.2 / 27.8, of 1000 40.4 / 33.3; 16 heads of 64 x 128, one of 520 34.2 / 19.0,
+// two of 400 with 128 rows of state 36.7 / 23.4.  Not beside many short portions, which fill what one segment leaves idle and wait
+// for the summaries otherwise: 28 heads of 128 x 128, one of 300 beside 32 single rows 29.5 / 27.5, beside 63 30.5 / 36.7;
+// 32 heads of 64 columns, one of 520 beside 63 37.0 / 25.8.
 //
 // The segments of the portions of more than `rows` rows are numbered one behind the other (segment_at); there are no more than
 // one per `rows` rows of the step and one per such portion.  What has no rows comes behind what has: a workgroup that ends at
@@ -53,7 +56,7 @@ inline int scan_waves(int64_t lanes, int v_dim) {
 // Up to kMostUnchained segments every one works out the state in front of it for itself, from the summaries before it, which saves a
 // launch (6 to 9 us) for at most ten reads of 64 KB: 16 heads of 128 columns, five portions of 700 rows in four segments 41 -> 31 us, of
 // 64 columns three of 2000 64 -> 57; with 16 segments level.
-constexpr int kMostUnchained = 10;
+constexpr int kMostUnchained = 10, kSegmentRows = 64, kManySegmentRows = 192, kManyColumns = 131072;
 struct ScanSegments {
   int rows = 0x7fffffff, count = 0;        // rows of a segment; bound on the segments' numbers
   bool chained = false;                    // whether a launch of its own turns the summaries into the states in front of the segments
@@ -62,11 +65,15 @@ struct ScanSegments {
 // Segments of a step of `portions` long ones: how many of a head's fit on the chip beside the others.
 inline int64_t scan_segments_wanted(int64_t portions, int num_heads, int v_dim, int max_query_len) {
   const int64_t wide = v_dim % 128 == 0 ? 128 : v_dim % 64 == 0 ? 64 : 32, slots = 256 * (128 / wide);
-  return std::min<int64_t>(slots / (portions * num_heads * std::max<int64_t>(v_dim / wide, 1)), max_query_len / 192);
+  return std::min<int64_t>(slots / (portions * num_heads * std::max<int64_t>(v_dim / wide, 1)), max_query_len / kSegmentRows);
+}
+inline int scan_segment_rows(int num_seqs, int num_heads, int v_dim) {
+  return static_cast<int64_t>(num_seqs) * num_heads * v_dim > kManyColumns ? kManySegmentRows : kSegmentRows;
 }
 inline ScanSegments scan_segments(int num_tokens, int num_seqs, int num_heads, int v_dim, int max_query_len) {
   const int64_t portions = long_portions(num_tokens, num_seqs, max_query_len);
-  const int64_t want = scan_segments_wanted(portions, num_heads, v_dim, max_query_len);
+  const int64_t want = std::min<int64_t>(scan_segments_wanted(portions, num_heads, v_dim, max_query_len),
+                                         max_query_len / scan_segment_rows(num_seqs, num_heads, v_dim));
   ScanSegments sg;
   sg.lanes = portions * num_heads;
   if (want < 3) return sg;
@@ -84,10 +91,10 @@ inline size_t scan_segment_bytes(int64_t count, int num_heads, int head_dim, int
 }
 // Enough for any number of tokens, and for fewer sequences and shorter portions too.  With p long portions of m rows at most
 // in segments of at least m / w rows there are no more than (p m + num_seqs) w / m cuts: p w is at most what one portion would
-// be cut into, w / m at most 1 / 192.
+// be cut into, w / m at most 1 / 64.
 inline size_t scan_workspace_bytes(int num_seqs, int num_heads, int head_dim, int v_dim, int max_query_len) {
   if (num_seqs <= 0 || num_heads <= 0 || head_dim <= 0 || v_dim <= 0 || scan_segments_wanted(1, num_heads, v_dim, max_query_len) < 3) return 0;
-  const int64_t cuts = scan_segments_wanted(1, num_heads, v_dim, 0x7fffffff) + num_seqs / 192 + 1;
+  const int64_t cuts = scan_segments_wanted(1, num_heads, v_dim, 0x7fffffff) + num_seqs / kSegmentRows + 1;
   return scan_segment_bytes(cuts + std::min<int64_t>(num_seqs, cuts), num_heads, head_dim, v_dim);
 }
 
