@@ -974,6 +974,10 @@ int hymeta_moe_gemm_activates(const hymeta_moe_gemm_args* args);
  * spread: the kernel is chosen by the rows that its experts can expect of them (the calls above take all pairs to be theirs). */
 int hymeta_moe_gemm_rank(const hymeta_moe_gemm_args* args, int32_t num_experts, int32_t act, float limit, float alpha, hymeta_stream_t stream);
 int hymeta_moe_gemm_rank_activates(const hymeta_moe_gemm_args* args, int32_t num_experts);
+/* hymeta_moe_gemm_rank with an activation wherever a kernel of its has it in its epilogue: the problems that
+ * hymeta_moe_gemm_glu_takes answers with 1, more than hymeta_moe_gemm_rank_activates', else HYMETA_ERR_UNSUPPORTED. */
+int hymeta_moe_gemm_glu(const hymeta_moe_gemm_args* args, int32_t num_experts, int32_t act, float limit, float alpha, hymeta_stream_t stream);
+int hymeta_moe_gemm_glu_takes(const hymeta_moe_gemm_args* args, int32_t num_experts);
 /* 1 when hymeta_moe_gemm runs a problem of these sizes in the kernel that has the fused combine (K in bf16 elements:
  * pass K / 2 for int8 operands, the choice goes by the bytes of a row). */
 int hymeta_moe_gemm_fuses(int32_t max_rows, int32_t experts, int32_t K, int32_t N);

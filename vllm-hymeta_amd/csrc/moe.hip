@@ -12,6 +12,8 @@
 //   combine  out[t] = sum_k y[pos[t,k]] (+ shared[t]), y weighted in the down GEMM; pairs of non-local experts
 //            (expert parallelism) carry pos = -1 and add nothing
 #include "common.h"
+#include "expert_tiles.h"
+#include "lds_copy.h"
 #include "pair_sort.h"
 #include "tile_gemm.h"
 #include "w8a8_quant.h"
@@ -505,8 +507,8 @@ __global__ __launch_bounds__(256) void moe_gemm_lines_kernel(hymeta_moe_gemm_arg
   }
 }
 
-// Prompts of few rows per expert (tile_gemm.hip takes the long ones), and those whose experts nearly fill a tile of 256: BM rows x BN columns per workgroup, WM x WN waves that own
-// (BM / WM) x (BN / WN) each.  Both operands are K-contiguous; a 64-deep step of each (128 bytes per
+// Experts that nearly fill one tile of 256, in bf16 (tile_gemm.hip takes longer ones, moe_gemm_deep_kernel shorter ones): BM rows x BN columns
+// per workgroup, WM x WN waves that own (BM / WM) x (BN / WN) each.  Both operands are K-contiguous; a 64-deep step of each (128 bytes per
 // row) is staged once per workgroup through double-buffered LDS images (16-byte chunks XOR-ed with
 // the row, so the sixteen rows of a fragment read hit distinct banks): registers -> LDS right
 // behind the barrier that frees the buffer, the next step's loads issued at once.
@@ -515,13 +517,11 @@ __global__ __launch_bounds__(256) void moe_gemm_lines_kernel(hymeta_moe_gemm_arg
 // bound ceil(max_rows / BM) + experts.
 constexpr int kTK = 64;
 constexpr int kTilePitch = 2 * kTK;                 // bytes per staged row
-constexpr int kTiledMinRowsPerExpert = 8;           // measured: level at 4 rows per expert, 15 % ahead at 16, 2.6x at 512
 constexpr int kBigTileMinTiles = 160;
 
-template <int BM, int BN, int WM, int WN, bool I8>
+template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void moe_gemm_tiled_kernel(hymeta_moe_gemm_args a) {
-  typedef typename MoeAcc<I8>::type acc_t;
-  constexpr int ES = I8 ? 1 : 2;
+  constexpr int ES = 2;
   constexpr int kThreads = 64 * WM * WN;
   constexpr int MT = BM / WM / 16, NT = BN / WN / 16;       // 16 x 16 tiles per wave
   constexpr int kXBytes = BM * kTilePitch, kWBytes = BN * kTilePitch;
@@ -588,11 +588,11 @@ __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void moe_gemm_t
     }
   };
 
-  acc_t acc[MT][NT];
+  f32x4 acc[MT][NT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = acc_t{0, 0, 0, 0};
+    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0, 0, 0, 0};
 
   const int nk = static_cast<int>(kb / kTilePitch);
   issue(0);
@@ -616,7 +616,7 @@ __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void moe_gemm_t
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = moe_mma<I8>(xf[mt], wf[nt], acc[mt][nt]);
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = moe_mma<false>(xf[mt], wf[nt], acc[mt][nt]);
     }
     __syncthreads();
   }
@@ -629,10 +629,6 @@ __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void moe_gemm_t
   static_assert(kStageRows * kCPitch <= 2 * (kXBytes + kWBytes), "output staging fits the operand images");
   static_assert(kStageRows % (16 * MT) == 0 && BM % kStageRows == 0, "a wave's rows fall into one staging pass");
   char* cst = &sm[0][0];
-  float wsc[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-    wsc[nt] = I8 ? a.w_scale[static_cast<int64_t>(e) * a.N + col0 + 16 * NT * wn + 16 * nt + n] : 1.f;
 #pragma unroll
   for (int half = 0; half < BM / kStageRows; ++half) {
     if ((16 * MT * wm) / kStageRows == half) {
@@ -644,14 +640,8 @@ __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void moe_gemm_t
           const int slot = min(row_lo + row, row_hi - 1);
           const float sc_row = a.row_scale != nullptr ? a.row_scale[a.scale_rows != nullptr ? a.scale_rows[slot] : slot] : 1.f;
           uint16_t* crow = reinterpret_cast<uint16_t*>(cst + (row - kStageRows * half) * kCPitch) + 16 * NT * wn + n;
-          if constexpr (I8) {
-            const float xs = a.x_scale[moe_src_row(a, slot)];
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) crow[16 * nt] = f2bf(w8a8_scaled(acc[mt][nt][r], xs, wsc[nt], 0.f) * sc_row);
-          } else {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) crow[16 * nt] = f2bf(acc[mt][nt][r] * sc_row);
-          }
+          for (int nt = 0; nt < NT; ++nt) crow[16 * nt] = f2bf(acc[mt][nt][r] * sc_row);
         }
     }
     __syncthreads();
@@ -665,6 +655,148 @@ __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void moe_gemm_t
     }
     if (half + 1 < BM / kStageRows) __syncthreads();
   }
+}
+
+// Experts whose rows do not fill a tile of tile_gemm.hip's: up to 256 slots x 128 weight rows a workgroup, eight waves of 16 MI x 64, MI
+// the slots' 64s.  Bound by the weights' way from memory: a step's 128 rows take a compute unit's share of it 0.84 us, the products of
+// 128 slots 0.35.  Hence an expert of up to 256 slots reads them once, and both operands are copied straight into LDS, 128 bytes of every
+// row a step, five (three, two) steps ahead.
+//
+// 16 experts of 3584 x 4736, a whole block on cold weights, in bf16 and int8 (tiles of 128 x 128 through registers, two steps ahead ->
+// these, us): 9 rows an expert 366 -> 339 and 241 -> 219, 40 392 -> 357 and 251 -> 237, 100 434 -> 399 and 286 -> 279; with tiles of 256 before, 150
+// 526 -> 452 and 327 -> 309, 170 515 -> 466 and 333 -> 322.  1.63 GB of bf16 are 326 us at 5 TB/s.
+constexpr int kDeepRows = 256, kDeepCols = 128, kDeepStep = 128;              // (bytes of a row in a step)
+
+constexpr int kTiledMinRowsPerExpert = 8;           // up to here the kernels of 16 rows are ahead: 5 rows an expert 333 against 335 us in bf16, 187 against 216 in int8
+
+template <int MI> constexpr int kDeepImage = (64 * MI + kDeepCols) * kDeepStep;
+template <int MI> constexpr int kDeepStages = MI == 1 ? 6 : MI == 2 ? 4 : 3;
+constexpr int kDeepLds = 144 << 10;
+static_assert(kDeepStages<1> * kDeepImage<1> <= kDeepLds && kDeepStages<2> * kDeepImage<2> <= kDeepLds &&
+              kDeepStages<3> * kDeepImage<3> <= kDeepLds && kDeepStages<4> * kDeepImage<4> <= kDeepLds, "all fit");
+
+// An activation, if one follows, over the rounded pairs of a gate column and its up column: a wave's 64 columns are 32 of each.
+struct DeepAct { int kind; float limit, alpha; };
+__device__ __forceinline__ float apply_deep_act(const DeepAct& act, float gate, float up) {
+  const float g = bf16_round(gate), u = bf16_round(up);
+  if (act.kind == HYMETA_GEMM_ACT_SILU) return g * sigmoidf(g) * u;
+  if (act.kind == HYMETA_GEMM_ACT_SILU_EXACT) return g * sigmoid_exact(g) * u;
+  return clamped_glu(g, u, act.limit, act.alpha);
+}
+
+template <bool I8, int MI, bool Gated>
+__device__ __forceinline__ void deep_body(const hymeta_moe_gemm_args& a, const DeepAct& act, const ExpertTile& p, char* sm) {
+  typedef typename MoeAcc<I8>::type acc_t;
+  constexpr int ES = I8 ? 1 : 2, NJ = 4, kStages = kDeepStages<MI>, kImage = kDeepImage<MI>, kX = 64 * MI * kDeepStep;
+  constexpr int kCopies = MI + 2;                            // a wave's of a step, 8 rows each
+  const int tid = threadIdx.x, lane = tid & 63, c = lane >> 4, n = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
+  const int col0 = p.col * kDeepCols;
+  const int64_t k_bytes = static_cast<int64_t>(a.K) * ES;
+
+  // A copy of a wave brings 8 rows x 128 bytes; a row's 16-byte chunks lie XOR-ed with (row / 2) % 8, which with the pitch of
+  // 128 bytes spreads the sixteen rows of a fragment read over all banks.  Rows past the end re-read the last one.
+  const int l3 = lane >> 3, chunk = (lane & 7) ^ (l3 >> 1) ^ (wave & 1 ? 4 : 0);
+  const char *xp[MI], *wp[2];
+#pragma unroll
+  for (int j = 0; j < MI; ++j) {
+    const int slot = p.row + min(64 * j + 8 * wave + l3, p.rows - 1);
+    xp[j] = static_cast<const char*>(a.x) + static_cast<int64_t>(moe_src_row(a, slot)) * a.x_stride_m * ES + 16 * chunk;
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    wp[j] = static_cast<const char*>(a.weights) + static_cast<int64_t>(p.e) * a.w_stride_e * ES + 16 * chunk +
+            (Gated ? (wave >> 2) * (a.N / 2) + col0 / 2 + 32 * j + 8 * (wave & 3) + l3 : col0 + 64 * j + 8 * wave + l3) * k_bytes;
+  const int steps = static_cast<int>(k_bytes / kDeepStep);
+  int asked = 0, put = 0;                                    // the step to ask for, its image; past the last step it is asked for again
+  auto ask = [&] {
+    char* const to = sm + put + 1024 * wave;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) copy16_to_lds(wp[j], to + kX + 8192 * j);
+#pragma unroll
+    for (int j = 0; j < MI; ++j) copy16_to_lds(xp[j], to + 8192 * j);
+    const int on = asked + 1 < steps ? kDeepStep : 0;
+    asked += 1;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) wp[j] += on;
+#pragma unroll
+    for (int j = 0; j < MI; ++j) xp[j] += on;
+    put = put + kImage == kStages * kImage ? 0 : put + kImage;
+  };
+
+  int off[2];                                                // a fragment's place for this lane: row n, chunk 4 half + c
+#pragma unroll
+  for (int h = 0; h < 2; ++h) off[h] = n * kDeepStep + 16 * ((4 * h + c) ^ ((n >> 1) & 7));
+  acc_t acc[MI][NJ];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+#pragma unroll
+  for (int s = 0; s + 1 < kStages; ++s) ask();
+  int image = 0;
+  for (int it = 0; it < steps; ++it) {
+    // this step's rows are in LDS and every wave is through with the image that is asked for next
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kCopies * (kStages - 2)) : "memory");
+    ask();
+    const char *xs = sm + image + 16 * MI * wm * kDeepStep, *ws = sm + image + kX + 64 * wn * kDeepStep;
+    u32x4 xf[2][MI], wf[2][NJ];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i) xf[h][i] = ld16(xs + 16 * i * kDeepStep + off[h]);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) wf[h][j] = ld16(ws + 16 * j * kDeepStep + off[h]);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < MI; ++i) acc[i][j] = moe_mma<I8>(wf[h][j], xf[h][i], acc[i][j]);
+    image = image + kImage == kStages * kImage ? 0 : image + kImage;
+  }
+
+  // acc[i][j][r] = C[slot 16 (MI wm + i) + n][column 64 wn + 16 j + 4 c + r].  Scales on the sums, one rounding; lanes trade with the
+  // next 16 so that each stores 16 bytes of a row.
+  constexpr int kOutCols = Gated ? 32 : 64;                  // of a wave
+  const int out_col = (2 * p.col + wn) * kOutCols;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int row = 16 * (MI * wm + i) + n, slot = p.row + min(row, p.rows - 1);
+    const float factor = a.row_scale != nullptr ? a.row_scale[a.scale_rows != nullptr ? a.scale_rows[slot] : slot] : 1.f;
+    uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + static_cast<int64_t>(slot) * a.out_stride_m + out_col + 16 * (c & 1) + 8 * (c >> 1);
+    auto piece = [&](int j) {                                // 4 columns of the output
+      f32x4 v = moe_sums_to_f32<I8>(a, acc[i][j], p.e, slot, out_col + 16 * j + 4 * c);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] *= factor;
+      if constexpr (Gated) {
+        const f32x4 up = moe_sums_to_f32<I8>(a, acc[i][j + 2], p.e, slot, a.N / 2 + out_col + 16 * j + 4 * c);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = apply_deep_act(act, v[r], up[r] * factor);
+      }
+      return u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    };
+#pragma unroll
+    for (int j = 0; j < kOutCols / 16; j += 2) {
+      const u32x2 even = piece(j), odd = piece(j + 1);
+      const auto first = __builtin_amdgcn_permlane16_swap(even[0], odd[0], false, false);
+      const auto second = __builtin_amdgcn_permlane16_swap(even[1], odd[1], false, false);
+      if (row < p.rows) st16(out + 16 * j, u32x4{first[0], second[0], first[1], second[1]});
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // (the copies past the last step)
+}
+
+template <bool I8, bool Gated>
+__global__ __launch_bounds__(512) void moe_gemm_deep_kernel(hymeta_moe_gemm_args a, DeepAct act, int tile_rows) {
+  __shared__ __attribute__((aligned(16))) char sm[kDeepLds];
+  ExpertTile p;
+  if (!expert_tile(a.expert_offsets, a.local_expert_begin, a.local_expert_end, a.N / kDeepCols, tile_rows, &p)) return;          // workgroup-uniform
+  if (p.rows > 192) deep_body<I8, 4, Gated>(a, act, p, sm);
+  else if (p.rows > 128) deep_body<I8, 3, Gated>(a, act, p, sm);
+  else if (p.rows > 64) deep_body<I8, 2, Gated>(a, act, p, sm);
+  else deep_body<I8, 1, Gated>(a, act, p, sm);
 }
 
 // out[r, j] = silu(in[r, j]) * in[r, inter + j]; the product is formed in fp32 and rounded once.
@@ -811,19 +943,22 @@ enum class MoeGemmKind { kBigTiles, kTallTiles, kTiles, kLines, kFragments };
 MoeGemmKind moe_gemm_kind(int64_t max_rows, int experts, int total, int K, int N, bool i8, bool act) {
   // tiled grouped GEMM once the experts average more than a few rows (prefill chunks); the large tile when they fill it
   if (max_rows > static_cast<int64_t>(kTiledMinRowsPerExpert) * experts && K % kTK == 0) {
-    // Tiles of 256 where the experts fill half of one on average (a little more with many columns, whose tiles fill the chip either
-    // way) and the tiles (an expert's rows scatter around the average) nearly fill the chip once: 16 experts on 2048 tokens of 3584
-    // columns 560 -> 497 us, 8 on 1400 936 -> 705; with 112 rows an expert 424 -> 459, with 64 to 128 tiles 215 -> 226.  Up to 192 rows it is
-    // those that a rank's experts can expect, not all pairs (8 of 16 experts of 14336 x 8192 at 300 tokens, top 4, 73 rows an expert, 602 ->
-    // 675); from 192 on half-empty tiles are level or better (the same at 512 tokens, 128 rows, 800 -> 735).
+    // An expert of fewer rows goes in one tile of the deep kernel, which is ahead while memory is the bound: until where depends on how
+    // well the tiles of 256 (`once`, a row of them an expert) fill their last round of the chip.  Whole blocks in bf16, us, tiles
+    // of 256 against these: 16 experts of 3584 x 4736 (592 and 224 tiles) 170 rows 515, 466; 190 513, 521; 8 of them (296 and 112) 190 341, 301,
+    // 235 357, 309; 8 of 8192 x 4096 (256 and 256) 150 498, 438; 170 448, 469; 4 of 5120 x 4736 (148) 150 312, 268; 170 260, 274.  The rows are
+    // those that a rank's experts can expect, not all pairs (8 of 16 experts of 3584 x 4736, 200 rows: 359, 309).
     const int64_t rows = max_rows / total, most = max_rows / experts, tiles = (most + 64 + 255) / 256 * experts * (N / 256);
+    const int64_t once = experts * (N / 256), rest = once > 0 ? (once - 1) % 256 + 1 : 0;
+    const bool few = rest < 148 && once <= 256, full = rest >= (once <= 256 ? 148 : 256);
+    const bool big = rows >= (full ? 160 : few || (once < 512 && rest <= 64) ? 240 : 176);
     // One row tile an expert, nearly full, and tiles for most of the chip: every weight is fetched once, and eight waves that hold their
     // rows in registers keep more of them in flight than the copies.  Tiles of tile_gemm.hip -> these, bf16, 196 rows an expert: 8 experts
     // of 8192 x 8192 301 -> 270 us, of 5120 x 4736 137 -> 125, 16 of 14336 x 8192 1029 -> 968, 4 of 9472 x 5120 152 -> 143 (of 5120 x 4736, 80
-    // tiles, 80 -> 109); whole blocks of 8 experts with 162 rows 478 -> 430 (8192, 4096 wide) and 314 -> 314 (3584, 4736); with 235 rows, where an
+    // tiles, 80 -> 109); whole blocks of 8 experts with 162 rows 478 -> 430 (8192, 4096 wide); with 235 rows, where an
     // expert or two has a second tile, 16 of 8192 x 8192 712 -> 669, 8 of 14336 x 8192 636 -> 643.  Below a K of 5120 the other kernel's epilogue saves more than that where an activation follows.
-    if (!i8 && rows >= 160 && rows < 240 && N % 256 == 0 && experts * (N / 256) >= 148 && K >= (act ? 5120 : 2048)) return MoeGemmKind::kTallTiles;
-    if ((rows >= (N > 4096 ? 144 : 128) || most >= 192) && tiles >= kBigTileMinTiles && N % 256 == 0) return MoeGemmKind::kBigTiles;
+    if (!i8 && big && rows < 240 && N % 256 == 0 && once >= 148 && K >= (act ? 5120 : 2048)) return MoeGemmKind::kTallTiles;
+    if (big && tiles >= kBigTileMinTiles && N % 256 == 0) return MoeGemmKind::kBigTiles;
     if (N % 128 == 0) return MoeGemmKind::kTiles;
   }
   static const bool lines = [] {
@@ -862,14 +997,29 @@ MoeGemmKind moe_gemm_kind(const hymeta_moe_gemm_args& a, int num_experts, bool a
   return kind == MoeGemmKind::kBigTiles && !tile_gemm_fits(tile_args(a)) ? MoeGemmKind::kTiles : kind;
 }
 
-bool moe_gemm_activates(const hymeta_moe_gemm_args& a, int num_experts) {
+bool moe_gemm_glu(const hymeta_moe_gemm_args& a, int num_experts) {
   if (a.local_expert_end <= a.local_expert_begin || (a.a_rows != nullptr && a.a_rows_div <= 0)) return false;
   TileGemmArgs t = tile_args(a);
   t.act = HYMETA_GEMM_ACT_SILU;
-  return moe_gemm_kind(a, num_experts, true) == MoeGemmKind::kBigTiles && tile_gemm_fits(t);
+  const MoeGemmKind kind = moe_gemm_kind(a, num_experts, true);
+  return kind == MoeGemmKind::kTiles || (kind == MoeGemmKind::kBigTiles && tile_gemm_fits(t));
 }
 
-int moe_gemm(const hymeta_moe_gemm_args* args, int num_experts, int act, float limit, float alpha, hymeta_stream_t stream) {
+// What hymeta_moe_gemm_act has always taken: problems whose experts can expect to fill half a tile of 256, but for those of one nearly
+// full tile in bf16.
+bool moe_gemm_activates(const hymeta_moe_gemm_args& a, int num_experts) {
+  if (!moe_gemm_glu(a, num_experts) || a.N % 256 != 0) return false;
+  TileGemmArgs t = tile_args(a);
+  t.act = HYMETA_GEMM_ACT_SILU;
+  if (!tile_gemm_fits(t)) return false;
+  const bool i8 = a.operand_dtype == HYMETA_I8;
+  const int experts = a.local_expert_end - a.local_expert_begin, K = i8 ? a.K / 2 : a.K;
+  const int64_t rows = a.max_rows / std::max(experts, num_experts), most = a.max_rows / experts, once = static_cast<int64_t>(experts) * (a.N / 256);
+  if (!i8 && rows >= 160 && rows < 240 && once >= 148 && K >= 5120) return false;
+  return (rows >= (a.N > 4096 ? 144 : 128) || most >= 192) && (most + 64 + 255) / 256 * once >= kBigTileMinTiles;
+}
+
+int moe_gemm(const hymeta_moe_gemm_args* args, int num_experts, int act, float limit, float alpha, bool (*takes)(const hymeta_moe_gemm_args&, int), hymeta_stream_t stream) {
   if (!args_ok(args)) return HYMETA_ERR_INVALID_ARG;
   const hymeta_moe_gemm_args& a = *args;
   if (a.max_rows < 0 || a.K <= 0 || a.N <= 0) return HYMETA_ERR_INVALID_ARG;
@@ -887,7 +1037,7 @@ int moe_gemm(const hymeta_moe_gemm_args* args, int num_experts, int act, float l
     return HYMETA_ERR_UNSUPPORTED;
   const int experts = a.local_expert_end - a.local_expert_begin;
   const MoeGemmKind kind = moe_gemm_kind(a, num_experts, act != HYMETA_GEMM_ACT_NONE);
-  if (act != HYMETA_GEMM_ACT_NONE && !moe_gemm_activates(a, num_experts)) return HYMETA_ERR_UNSUPPORTED;
+  if (act != HYMETA_GEMM_ACT_NONE && !takes(a, num_experts)) return HYMETA_ERR_UNSUPPORTED;
   if (i8 && act > HYMETA_GEMM_ACT_SILU) return HYMETA_ERR_UNSUPPORTED;
   if (a.combine_tokens != nullptr || a.combine_shared != nullptr) {
     // the fused combine exists in the decode-sized kernel with whole-line loads only (hymeta_moe_gemm_fuses)
@@ -909,13 +1059,18 @@ int moe_gemm(const hymeta_moe_gemm_args* args, int num_experts, int act, float l
   }
   if (kind == MoeGemmKind::kTallTiles) {
     const dim3 tgrid(a.N / 256, (a.max_rows + 255) / 256 + experts);
-    hipLaunchKernelGGL((moe_gemm_tiled_kernel<256, 256, 4, 2, false>), tgrid, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((moe_gemm_tiled_kernel<256, 256, 4, 2>), tgrid, dim3(512), 0, s, a);
     return launch_status();
   }
   if (kind == MoeGemmKind::kTiles) {
-    const dim3 tgrid(a.N / 128, (a.max_rows + 127) / 128 + experts);
-    HYMETA_MOE_BY_TYPE(hipLaunchKernelGGL((moe_gemm_tiled_kernel<128, 128, 2, 2, false>), tgrid, dim3(256), 0, s, a),
-                       hipLaunchKernelGGL((moe_gemm_tiled_kernel<128, 128, 2, 2, true>), tgrid, dim3(256), 0, s, a));
+    const int tile_rows = expert_tile_rows(kDeepRows, a.max_rows, experts, a.N / kDeepCols);
+    const dim3 tgrid(expert_tile_grid(a.max_rows, experts, a.N / kDeepCols, tile_rows));
+    const DeepAct then = {act, limit, alpha};
+#define HYMETA_MOE_DEEP(GATED) HYMETA_MOE_BY_TYPE(hipLaunchKernelGGL((moe_gemm_deep_kernel<false, GATED>), tgrid, dim3(512), 0, s, a, then, tile_rows), \
+                                                  hipLaunchKernelGGL((moe_gemm_deep_kernel<true, GATED>), tgrid, dim3(512), 0, s, a, then, tile_rows))
+    if (act == HYMETA_GEMM_ACT_NONE) HYMETA_MOE_DEEP(false);
+    else HYMETA_MOE_DEEP(true);
+#undef HYMETA_MOE_DEEP
     return launch_status();
   }
   const size_t red1 = 4 * 16 * kCols * sizeof(float), red4 = 4 * 64 * kCols * sizeof(float);
@@ -943,15 +1098,24 @@ extern "C" int hymeta_moe_gemm_activates(const hymeta_moe_gemm_args* args) {
 }
 
 extern "C" int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t stream) {
-  return hymeta::moe_gemm(args, 0, HYMETA_GEMM_ACT_NONE, 0.f, 0.f, stream);
+  return hymeta::moe_gemm(args, 0, HYMETA_GEMM_ACT_NONE, 0.f, 0.f, hymeta::moe_gemm_activates, stream);
 }
 
 extern "C" int hymeta_moe_gemm_act(const hymeta_moe_gemm_args* args, int32_t act, float limit, float alpha, hymeta_stream_t stream) {
-  return hymeta::moe_gemm(args, 0, act, limit, alpha, stream);
+  return hymeta::moe_gemm(args, 0, act, limit, alpha, hymeta::moe_gemm_activates, stream);
 }
 
 extern "C" int hymeta_moe_gemm_rank(const hymeta_moe_gemm_args* args, int32_t num_experts, int32_t act, float limit, float alpha, hymeta_stream_t stream) {
-  return hymeta::moe_gemm(args, num_experts, act, limit, alpha, stream);
+  return hymeta::moe_gemm(args, num_experts, act, limit, alpha, hymeta::moe_gemm_activates, stream);
+}
+
+extern "C" int hymeta_moe_gemm_glu(const hymeta_moe_gemm_args* args, int32_t num_experts, int32_t act, float limit, float alpha, hymeta_stream_t stream) {
+  return hymeta::moe_gemm(args, num_experts, act, limit, alpha, hymeta::moe_gemm_glu, stream);
+}
+
+extern "C" int hymeta_moe_gemm_glu_takes(const hymeta_moe_gemm_args* args, int32_t num_experts) {
+  if (!hymeta::args_ok(args)) return HYMETA_ERR_INVALID_ARG;
+  return hymeta::moe_gemm_glu(*args, num_experts) ? 1 : 0;
 }
 
 extern "C" int hymeta_moe_gemm_rank_activates(const hymeta_moe_gemm_args* args, int32_t num_experts) {

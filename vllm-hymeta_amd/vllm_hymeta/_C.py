@@ -682,6 +682,8 @@ _SIGNATURES = {
     "hymeta_moe_gemm_activates": (C.c_int, [C.POINTER(MoeGemmArgs)]),
     "hymeta_moe_gemm_rank": (C.c_int, [C.POINTER(MoeGemmArgs), _i32, _i32, C.c_float, C.c_float, _ptr]),
     "hymeta_moe_gemm_rank_activates": (C.c_int, [C.POINTER(MoeGemmArgs), _i32]),
+    "hymeta_moe_gemm_glu": (C.c_int, [C.POINTER(MoeGemmArgs), _i32, _i32, C.c_float, C.c_float, _ptr]),
+    "hymeta_moe_gemm_glu_takes": (C.c_int, [C.POINTER(MoeGemmArgs), _i32]),
     "hymeta_silu_and_mul": (C.c_int, [_ptr, _ptr, _ptr, _i32, _i32, _i64, _i64, _ptr]),
     "hymeta_moe_gptq_gemm": (C.c_int, [C.POINTER(MoeGptqGemmArgs), _ptr]),
     "hymeta_moe_gptq_expand": (C.c_int, [_ptr, _ptr, _ptr, _ptr, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _ptr]),

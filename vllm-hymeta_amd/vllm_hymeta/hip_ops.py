@@ -1519,11 +1519,11 @@ def moe_forward(x: torch.Tensor, router_logits: Optional[torch.Tensor], w13: tor
     g.a_rows, g.a_rows_div, g.max_rows, g.K, g.N = _p(sorted_pair), top_k, P, H, two_i
     g.local_expert_begin, g.local_expert_end = lo, hi
     g.x_stride_m, g.out_stride_m, g.w_stride_e = xin.stride(0), inter, w13.stride(0)
-    activates = lib.hymeta_moe_gemm_rank_activates(C.byref(g), E) == 1      # many rows per expert: silu and mul in the GEMM's epilogue
+    activates = lib.hymeta_moe_gemm_glu_takes(C.byref(g), E) == 1      # more than a few rows per expert: silu and mul in the GEMM's epilogue
     if activates:
         hact = torch.empty(P, inter, dtype=torch.bfloat16, device=dev)
         g.out = _p(hact)
-        _C.check(lib.hymeta_moe_gemm_rank(C.byref(g), E, _C.GEMM_ACT_SILU, 0.0, 0.0, st), "hymeta_moe_gemm_rank (w13)")
+        _C.check(lib.hymeta_moe_gemm_glu(C.byref(g), E, _C.GEMM_ACT_SILU, 0.0, 0.0, st), "hymeta_moe_gemm_glu (w13)")
     else:
         h13 = torch.empty(P, two_i, dtype=torch.bfloat16, device=dev)
         g.out, g.out_stride_m = _p(h13), h13.stride(0)
@@ -2247,11 +2247,11 @@ def moe_routed_forward(x: torch.Tensor, router_weight: torch.Tensor, router_bias
         g.a_rows, g.a_rows_div, g.max_rows, g.K, g.N = _p(sorted_pair), top_k, P, H, n1
         g.local_expert_begin, g.local_expert_end = 0, E
         g.x_stride_m, g.out_stride_m, g.w_stride_e = x.stride(0), inter, w1.stride(0)
-        if gated and lib.hymeta_moe_gemm_activates(C.byref(g)) == 1:      # many rows per expert: the activation in the GEMM's epilogue
+        if gated and lib.hymeta_moe_gemm_glu_takes(C.byref(g), E) == 1:      # more than a few rows per expert: the activation in the GEMM's epilogue
             hact = torch.empty(P, inter, dtype=torch.bfloat16, device=dev)
             g.out = _p(hact)
             act = _C.GEMM_ACT_CLAMPED_GLU if expert_act == "clamped_glu" else _C.GEMM_ACT_SILU_EXACT
-            _C.check(lib.hymeta_moe_gemm_act(C.byref(g), act, limit, alpha, st), "hymeta_moe_gemm_act (w1)")
+            _C.check(lib.hymeta_moe_gemm_glu(C.byref(g), E, act, limit, alpha, st), "hymeta_moe_gemm_glu (w1)")
         else:
             h1 = torch.empty(P, n1, dtype=torch.bfloat16, device=dev)
             g.out, g.out_stride_m = _p(h1), h1.stride(0)
