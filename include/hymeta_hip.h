@@ -1010,6 +1010,9 @@ typedef struct hymeta_moe_gptq_gemm_args {
 } hymeta_moe_gptq_gemm_args;
 
 int hymeta_moe_gptq_gemm(const hymeta_moe_gptq_gemm_args* args, hymeta_stream_t stream);
+/* The same for a rank that holds [local_expert_begin, local_expert_end) of num_experts experts, over all of which the max_rows pairs
+ * are spread: the kernel is chosen by the rows that its experts can expect of them; the results are the same. */
+int hymeta_moe_gptq_gemm_rank(const hymeta_moe_gptq_gemm_args* args, int32_t num_experts, hymeta_stream_t stream);
 
 /* `experts` stacked GPTQ matrices (layouts above, starting at the pointers given) -> bf16 W^T [experts, N, K], the
  * layout of the bf16 expert stacks: one launch.  K % (16 * (32 / bits)) == 0. */

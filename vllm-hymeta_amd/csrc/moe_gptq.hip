@@ -6,7 +6,8 @@
 //
 // Built on the dense kernel for up to 32 rows (gptq_gemm_kernel in quant_gemm.hip): a packed int32 of qweight holds 8 (4)
 // consecutive k of ONE output column, which is what the MFMA B operand wants per lane, so the weights go global -> VGPR
-// -> MFMA; 4-bit: (q >> 4w) & 0x000F000F | 0x43004300 = the bf16 pair (128 + q_w, 128 + q_{w+4}) in one VALU op, the k
+// -> MFMA; 4-bit: (q >> 4w) & 0x000F000F | 0x43004300 = the bf16 pair (128 + q_w, 128 + q_{w+4}), a shift and one VALU op (two where the
+// compiler sees both constants: 64 rows of 16 experts 126 -> 121 us), the k
 // order this induces applied to the activation fragment; scales and zeros once per group on the group's partial sums,
 //   sum_k x w = s * ( sum_k x (c + q) - (c + z) * sum_k x ),   c = 128 (4-bit) or 0,
 // with sum_k x from one extra MFMA against an all-ones fragment.  grid = (N / 64, local experts): a workgroup owns 64
@@ -18,9 +19,12 @@
 // walked all tiles of its expert would make the launch as long as the busiest expert (measured in the model, where the
 // routing is uneven: 1.12 ms per layer at 2080 rows against 0.78 for evenly spread rows).  Rows are gathered through the
 // sorted pair list as in the bf16 kernels (moe.hip).
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
+#include "expert_tiles.h"
+#include "lds_copy.h"
 
 namespace hymeta {
 namespace {
@@ -74,6 +78,8 @@ __global__ __launch_bounds__(256) void moe_gptq_gemm_kernel(hymeta_moe_gptq_gemm
   const uint16_t* scales = reinterpret_cast<const uint16_t*>(a.scales) + static_cast<int64_t>(e) * G * a.N;
   const u32x4 ones_raw = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
   const bf16x8 ones = as_frag(ones_raw);
+  uint32_t bottom = 0x000F000Fu, above = 0x43004300u;  // held in registers: an and and an or of two constants take two instructions
+  asm("" : "+s"(bottom), "+v"(above));
 
   const int first_g = wave;
   const int ng = first_g < G ? (G - first_g + 3) / 4 : 0;   // this wave's groups: wave, wave + 4, ...
@@ -146,7 +152,7 @@ __global__ __launch_bounds__(256) void moe_gptq_gemm_kernel(hymeta_moe_gptq_gemm
 #pragma unroll
           for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int w = 0; w < 4; ++w) bq[i][w] = ((qring[wslot][0][i] >> (4 * w)) & 0x000F000Fu) | 0x43004300u;
+            for (int w = 0; w < 4; ++w) bq[i][w] = ((qring[wslot][0][i] >> (4 * w)) & bottom) | above;
         } else {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -252,6 +258,174 @@ __global__ __launch_bounds__(256) void moe_gptq_gemm_kernel(hymeta_moe_gptq_gemm
   }
 }
 
+// 4-bit experts of more rows, in groups of 64 or 128: up to 64 slots x 128 columns a workgroup, eight waves of 32 x 32, two workgroups on a
+// compute unit.  Bound by vector instructions: unpacking a wave's weights of 64 k takes 28, its rows' order 16, beside 12 products.  The rows,
+// the packed weights and the groups' scales and zeros are copied straight into LDS, 64 k a step, five steps ahead, so that a weight is
+// unpacked twice for 64 slots; the kernel above unpacks it, into more columns a lane, for every 32.  The groups go in that kernel's
+// order, every fourth one first, and meet in its order: a slot's result does not depend on which of the two forms it (a rank's share of
+// the experts is the whole's, bit for bit).
+//
+// 16 experts of 3584 x 4736, a block (tiles of 32 -> this, us): 600 tokens 279 -> 224, 1150 419 -> 376, 1800 592 -> 440, 2400 751 -> 570; expanded to bf16
+// before: 3300 887 -> 712, 4100 1035 -> 837.  Waves of 16 x 64 (56 instructions of unpacking): 600 256, 1800 507; 128 slots a workgroup, one on a compute
+// unit: 600 275, 1800 518, 3300 784.
+constexpr int kDeepCols = 128, kDeepStep = 128;              // columns of a tile; bytes of a slot's row in a step, of 64 k
+constexpr int kDeepRows = 64;
+constexpr int kDeepX = kDeepRows * kDeepStep, kDeepTables = kDeepX + 8 * kDeepCols * 4;      // an image: rows, packed weights, scales and zeros
+constexpr int kDeepImage = kDeepTables + 4 * 256, kDeepStages = 6;
+static_assert(2 * kDeepStages * kDeepImage <= 160 << 10, "two workgroups on a compute unit");
+
+// 16 or 4 bytes a lane from a wave-uniform base into LDS behind `place`
+__device__ __forceinline__ void copy16(const char* base, uint32_t offset, uint32_t place) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(place), "v"(offset), "s"(base) : "memory");
+}
+__device__ __forceinline__ void copy4(const char* base, uint32_t offset, uint32_t place) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(place), "v"(offset), "s"(base) : "memory");
+}
+
+template <int kSteps>                                        // 64s of k in a group
+__global__ __launch_bounds__(512, 4) void moe_gptq_deep_kernel(hymeta_moe_gptq_gemm_args a) {
+  __shared__ __attribute__((aligned(16))) char sm[kDeepStages * kDeepImage];
+  ExpertTile p;
+  if (!expert_tile(a.expert_offsets, a.local_expert_begin, a.local_expert_end, a.N / kDeepCols, kDeepRows, &p)) return;      // workgroup-uniform
+  constexpr int MT = 2, NJ = 2;                              // a wave's tiles of 16 slots; its columns of a lane
+  constexpr int kCopies = 2;                                 // a wave's of a step
+  const int tid = threadIdx.x, lane = tid & 63, c = lane >> 4, n = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 2, wn = wave & 3;
+  const int col0 = p.col * kDeepCols, G = a.K / a.group_size;
+  const uint32_t lds = __builtin_amdgcn_readfirstlane(lds_address(sm));
+
+  // Rows: a copy of a wave brings 8 rows x 128 bytes; a row's 16-byte chunks lie XOR-ed with (row / 2) % 8, which with the pitch of
+  // 128 bytes spreads the sixteen rows of a fragment read over all banks.  Rows past the end re-read the last one.
+  const int l3 = lane >> 3, chunk = (lane & 7) ^ (l3 >> 1) ^ (wave & 1 ? 4 : 0);
+  const int copied = p.row + min(8 * wave + l3, p.rows - 1), source = a.a_rows != nullptr ? a.a_rows[copied] / a.a_rows_div : copied;
+  const char* const xp = static_cast<const char*>(a.x) + static_cast<int64_t>(source) * a.x_stride_m * 2 + 16 * chunk;
+  // The eight packed rows of a step are two each of the first four waves; the others bring its group's scales and zeros.
+  const char* const packed = reinterpret_cast<const char*>(a.qweight + (static_cast<int64_t>(p.e) * (a.K / 8) + 2 * (wave & 3)) * a.N + col0);
+  const char* const tables = wave & 1 ? reinterpret_cast<const char*>(a.qzeros + static_cast<int64_t>(p.e) * G * (a.N / 8) + col0 / 8)
+                                      : reinterpret_cast<const char*>(static_cast<const uint16_t*>(a.scales) + static_cast<int64_t>(p.e) * G * a.N + col0);
+  const int64_t table_row = wave & 1 ? a.N / 2 : 2 * a.N;    // bytes of a group
+  const uint32_t packed_at = (lane >> 5) * 4u * a.N + 16 * (lane & 31), table_at = 4 * (wave & 1 ? min(lane, kDeepCols / 8 - 1) : lane);
+  // The step to ask for, every fourth group first (past the last one: that again), and its image.
+  int group = 0, of_group = 0, put = 0;
+  const char *packed_now = packed, *tables_now = tables;
+  const int64_t packed_step = 32 * static_cast<int64_t>(a.N);
+  int row_now = 0;
+  auto ask = [&] {
+    if (wave < 4) copy16(packed_now, packed_at, lds + put + kDeepX + 1024 * wave);
+    else copy4(tables_now, table_at, lds + put + kDeepTables + 256 * (wave - 4));
+    copy16_to_lds(xp + row_now, sm + put + 1024 * wave);
+    put = put + kDeepImage == kDeepStages * kDeepImage ? 0 : put + kDeepImage;
+    if (++of_group < kSteps) {
+      packed_now += packed_step, row_now += kDeepStep;
+    } else {
+      of_group = 0;
+      group = group + 4 < G ? group + 4 : (group & 3) + 1 < min(G, 4) ? (group & 3) + 1 : group;
+      packed_now = packed + group * (kSteps * packed_step), tables_now = tables + group * table_row, row_now = group * (kSteps * kDeepStep);
+    }
+  };
+
+  int off[2];                                                // a fragment's place for this lane: row n, chunk 4 half + c
+#pragma unroll
+  for (int h = 0; h < 2; ++h) off[h] = n * kDeepStep + 16 * ((4 * h + c) ^ ((n >> 1) & 7));
+  const u32x4 ones_raw = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+  const bf16x8 ones = as_frag(ones_raw);
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  uint32_t bottom = 0x000F000Fu, above = 0x43004300u;        // (as above)
+  asm("" : "+s"(bottom), "+v"(above));
+  f32x4 all[MT][NJ], total[MT][NJ], sum[MT][NJ], sum_x[MT];     // of all groups, of every fourth one, of a group
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) all[mt][i] = zero;
+#pragma unroll
+  for (int s = 0; s + 1 < kDeepStages; ++s) ask();
+  int image = 0;
+  auto step = [&](auto opens, auto closes) {                 // whether it begins a group and ends one
+    // this step's copies are in LDS and every wave is through with the image that is asked for next
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kCopies * (kDeepStages - 2)) : "memory");
+    ask();
+    const char *xs = sm + image + 16 * MT * wm * kDeepStep, *ws = sm + image + kDeepX + c * (4 * kDeepCols) + 128 * wn + 8 * n;
+    u32x4 xf[2][MT];
+    u32x2 q[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      q[h] = *reinterpret_cast<const u32x2*>(ws + h * 16 * kDeepCols);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) xf[h][mt] = ld16(xs + 16 * mt * kDeepStep + off[h]);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bool first = decltype(opens)::value && h == 0, last = decltype(closes)::value && h == 1;
+      u32x4 bq[NJ];
+#pragma unroll
+      for (int i = 0; i < NJ; ++i)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) bq[i][w] = ((q[h][i] >> (4 * w)) & bottom) | above;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        // k in the order (0, 4, 1, 5, 2, 6, 3, 7) in which the weights come apart
+        const u32x4 x = xf[h][mt];
+        const bf16x8 af = as_frag(u32x4{__builtin_amdgcn_perm(x[2], x[0], 0x05040100u), __builtin_amdgcn_perm(x[2], x[0], 0x07060302u),
+                                        __builtin_amdgcn_perm(x[3], x[1], 0x05040100u), __builtin_amdgcn_perm(x[3], x[1], 0x07060302u)});
+#pragma unroll
+        for (int i = 0; i < NJ; ++i) sum[mt][i] = mfma16(af, as_frag(bq[i]), first ? zero : sum[mt][i]);
+        sum_x[mt] = mfma16(af, ones, first ? zero : sum_x[mt]);
+      }
+      if (last) {
+        // s * (sum x (128 + q) - (128 + z) * sum x)
+        const char* const t = sm + image + kDeepTables;
+        const uint32_t raw = *reinterpret_cast<const uint32_t*>(t + 64 * wn + 4 * n);
+        const uint32_t zeros = *reinterpret_cast<const uint32_t*>(t + 256 + 4 * (4 * wn + (n >> 2)));
+        float sc[NJ], zf[NJ];
+#pragma unroll
+        for (int i = 0; i < NJ; ++i) {
+          const uint16_t bits = static_cast<uint16_t>(raw >> (16 * i));
+          sc[i] = a.scales_dtype == HYMETA_F16 ? static_cast<float>(__builtin_bit_cast(_Float16, bits)) : bf2f(bits);
+          zf[i] = static_cast<float>(((zeros >> (8 * (n & 3) + 4 * i)) & 15u) + a.zero_offset) + 128.f;
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int i = 0; i < NJ; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) total[mt][i][r] += sc[i] * (sum[mt][i][r] - zf[i] * sum_x[mt][r]);
+      }
+    }
+    image = image + kDeepImage == kDeepStages * kDeepImage ? 0 : image + kDeepImage;
+  };
+  for (int w = 0; w < min(G, 4); ++w) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < NJ; ++i) total[mt][i] = zero;
+    for (int g = w; g < G; g += 4) {
+      if constexpr (kSteps == 2) {
+        step(std::true_type{}, std::false_type{});
+        step(std::false_type{}, std::true_type{});
+      } else {
+        step(std::true_type{}, std::true_type{});
+      }
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < NJ; ++i) all[mt][i] += total[mt][i];
+  }
+
+  // all[mt][i][r] = C[slot 16 (MT wm + mt) + 4 c + r][column 32 wn + 2 n + i]: the routing weight on the sums, one rounding
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * (MT * wm + mt) + 4 * c + r, slot = p.row + min(row, p.rows - 1);
+      const float factor = a.row_scale != nullptr ? a.row_scale[a.scale_rows != nullptr ? a.scale_rows[slot] : slot] : 1.f;
+      if (row < p.rows)
+        *reinterpret_cast<uint32_t*>(reinterpret_cast<uint16_t*>(a.out) + static_cast<int64_t>(slot) * a.out_stride_m + col0 + 32 * wn + 2 * n) =
+            pack_bf16x2(all[mt][0][r] * factor, all[mt][1][r] * factor);
+    }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // (the copies past the last step)
+}
+
 // Every local expert's matrix expanded to bf16 W^T [N, K] (the layout of the bf16 expert stacks) in one launch, for
 // prefill-sized batches: the tiled bf16 grouped GEMM then runs on the expansion.  grid = (N / 64, K / (16 PACK), experts);
 // a workgroup expands 64 columns x 16 packed rows of one expert (128 k at 4 bits: a tensor-parallel shard's K is a whole
@@ -317,7 +491,7 @@ int check_common(int K, int N, int bits, int group_size, int scales_dtype, int z
 
 using namespace hymeta;
 
-extern "C" int hymeta_moe_gptq_gemm(const hymeta_moe_gptq_gemm_args* args, hymeta_stream_t stream) {
+extern "C" int hymeta_moe_gptq_gemm_rank(const hymeta_moe_gptq_gemm_args* args, int32_t num_experts, hymeta_stream_t stream) {
   if (!hymeta::args_ok(args)) return HYMETA_ERR_INVALID_ARG;
   const hymeta_moe_gptq_gemm_args& a = *args;
   if (a.max_rows < 0) return HYMETA_ERR_INVALID_ARG;
@@ -337,6 +511,14 @@ extern "C" int hymeta_moe_gptq_gemm(const hymeta_moe_gptq_gemm_args* args, hymet
   const bool small = static_cast<int64_t>(a.max_rows) <= 8LL * experts;
   const dim3 tgrid(a.N / kCols, (a.max_rows + 31) / 32 + experts);
   if (tgrid.y > 65535u) return HYMETA_ERR_UNSUPPORTED;
+  // below, the kernel of 32-row tiles is ahead: 16 experts of 3584 x 4736 with 25 rows each 205 us, 217 in tiles of 64; with 38 279 and 224
+  const bool deep = a.max_rows > 28LL * std::max(experts, num_experts);
+  if (!small && deep && a.bits == 4 && a.group_size >= 64 && a.N % kDeepCols == 0) {
+    const dim3 dgrid(expert_tile_grid(a.max_rows, experts, a.N / kDeepCols, kDeepRows));
+    if (a.group_size == 128) hipLaunchKernelGGL(moe_gptq_deep_kernel<2>, dgrid, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL(moe_gptq_deep_kernel<1>, dgrid, dim3(512), 0, s, a);
+    return launch_status();
+  }
   const size_t lds1 = static_cast<size_t>(4) * 16 * kCols * sizeof(float), lds2 = 2 * lds1;
 #define HYMETA_MOE_GPTQ(B, KS)                                                                         \
   do {                                                                                                 \
@@ -353,6 +535,10 @@ extern "C" int hymeta_moe_gptq_gemm(const hymeta_moe_gptq_gemm_args* args, hymet
 #undef HYMETA_MOE_GPTQ_KS
 #undef HYMETA_MOE_GPTQ
   return launch_status();
+}
+
+extern "C" int hymeta_moe_gptq_gemm(const hymeta_moe_gptq_gemm_args* args, hymeta_stream_t stream) {
+  return hymeta_moe_gptq_gemm_rank(args, 0, stream);
 }
 
 extern "C" int hymeta_moe_gptq_expand(const int32_t* qweight, const int32_t* qzeros, const void* scales, void* out,

@@ -192,6 +192,8 @@ __device__ __forceinline__ void gptq_wave(const StreamGptqArgs& a, char* smem, c
   __syncthreads();
 
   const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+  uint32_t nibbles = 0x000F000Fu, exponents = 0x43004300u;      // held in registers: an and and an or of two constants are two instructions
+  asm("" : "+s"(nibbles), "+v"(exponents));
   // at the top of chunk i (counted from c_lo): the shared image i & 1 holds x of chunk i, the registers those of chunks
   // i + 1 .. i + kAheadX - 1; chunk i + kAheadX is asked for, and chunk i + 1 goes to the other image at the bottom
   for (int c0 = c_lo; c0 < c_hi; c0 += kUnroll) {
@@ -247,7 +249,7 @@ __device__ __forceinline__ void gptq_wave(const StreamGptqArgs& a, char* smem, c
               if constexpr (BITS == 4) {
                 const uint32_t w = *reinterpret_cast<const uint32_t*>(region + wsrc[s][f]);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) b[j] = ((w >> (4 * j)) & 0x000F000Fu) | 0x43004300u;
+                for (int j = 0; j < 4; ++j) b[j] = ((w >> (4 * j)) & nibbles) | exponents;
               } else {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {

@@ -686,6 +686,7 @@ _SIGNATURES = {
     "hymeta_moe_gemm_glu_takes": (C.c_int, [C.POINTER(MoeGemmArgs), _i32]),
     "hymeta_silu_and_mul": (C.c_int, [_ptr, _ptr, _ptr, _i32, _i32, _i64, _i64, _ptr]),
     "hymeta_moe_gptq_gemm": (C.c_int, [C.POINTER(MoeGptqGemmArgs), _ptr]),
+    "hymeta_moe_gptq_gemm_rank": (C.c_int, [C.POINTER(MoeGptqGemmArgs), _i32, _ptr]),
     "hymeta_moe_gptq_expand": (C.c_int, [_ptr, _ptr, _ptr, _ptr, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _ptr]),
     "hymeta_silu_and_mul_int8": (C.c_int, [_ptr, _ptr, _ptr, _ptr, _i32, _i32, _i64, _ptr]),
     "hymeta_moe_combine": (C.c_int, [C.POINTER(MoeCombineArgs), _ptr]),

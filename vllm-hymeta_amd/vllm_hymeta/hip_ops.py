@@ -1310,11 +1310,21 @@ class GptqExperts(NamedTuple):
         return (self.qweight.shape[0], self.qweight.shape[2], self.qweight.shape[1] * (32 // self.bits))
 
 
-# Rows per local expert (on average) up to which GPTQ experts run the fused de-quantising grouped GEMM; above, the local
-# experts are expanded to bf16 once per call and the tiled bf16 grouped GEMM runs on the expansion (the fused kernel
-# re-reads an expert's weights per 32-row tile).  Measured on the 70B TP=4 shapes (16 experts, us per block, fused /
-# expanded): 1024 tokens 466 / 796, 2048: 777 / 943, 4096: 1373 / 1041, 8192: 2569 / 1303.
-MOE_GPTQ_FUSED_ROWS_PER_EXPERT = int(os.environ.get("HYMETA_MOE_GPTQ_FUSED_ROWS", "160"))
+# Rows per expert (on average) up to which GPTQ experts run the fused de-quantising grouped GEMM; above, the local
+# experts are expanded to bf16 once per call and the tiled bf16 grouped GEMM runs on the expansion (the fused kernels
+# unpack an expert's weights per tile of rows).  4-bit stacks in groups of 64 or 128, in tiles of 64 rows: 16 experts of 3584 x 4736, us per block, fused /
+# expanded: 3300 tokens 712 / 887, 4100 837 / 1035, 5500 1090 / 1070.  Others, in tiles of 32 rows, by the rows of the local experts:
+# 1024 tokens 466 / 796, 2048: 777 / 943, 4096: 1373 / 1041, 8192: 2569 / 1303.
+_MOE_GPTQ_FUSED_ROWS = os.environ.get("HYMETA_MOE_GPTQ_FUSED_ROWS")
+MOE_GPTQ_FUSED_ROWS_PER_EXPERT = int(_MOE_GPTQ_FUSED_ROWS or "160")
+MOE_GPTQ_DEEP_ROWS_PER_EXPERT = int(_MOE_GPTQ_FUSED_ROWS or "256")
+
+
+def _moe_gptq_fused_rows(w13: GptqExperts, w2: GptqExperts, n_local: int, total: int) -> int:
+    """Pairs up to which GPTQ experts are not expanded."""
+    if all(w.bits == 4 and w.group_size >= 64 and w.shape[1] % 128 == 0 for w in (w13, w2)):
+        return MOE_GPTQ_DEEP_ROWS_PER_EXPERT * total
+    return MOE_GPTQ_FUSED_ROWS_PER_EXPERT * max(n_local, 1)
 
 
 def moe_gptq_expand(w: GptqExperts) -> torch.Tensor:
@@ -1368,9 +1378,10 @@ def moe_forward(x: torch.Tensor, router_logits: Optional[torch.Tensor], w13: tor
     if gptq:
         _require(isinstance(w2, GptqExperts), "w13 and w2 must both be GPTQ stacks")
         n_local = (local_experts[1] - local_experts[0]) if local_experts is not None else w13.shape[0]
-        if x.shape[0] * top_k > MOE_GPTQ_FUSED_ROWS_PER_EXPERT * max(n_local, 1):
+        _require(router_logits is not None or gate_weight is not None, "router_logits or gate_weight must be given")
+        total = gate_weight.shape[0] if gate_weight is not None else router_logits.shape[1]
+        if x.shape[0] * top_k > _moe_gptq_fused_rows(w13, w2, n_local, total):
             held = w13.shape[0]
-            total = gate_weight.shape[0] if gate_weight is not None else router_logits.shape[1]
             if held == total and local_experts is not None and tuple(local_experts) != (0, total):
                 lo_, hi_ = local_experts      # expand the rank's experts only
                 w13 = w13._replace(qweight=w13.qweight[lo_:hi_], qzeros=w13.qzeros[lo_:hi_], scales=w13.scales[lo_:hi_])
@@ -1489,13 +1500,13 @@ def moe_forward(x: torch.Tensor, router_logits: Optional[torch.Tensor], w13: tor
 
         q13 = gptq_gemm_args(w13, x, h13, H, two_i)
         q13.a_rows, q13.a_rows_div = _p(sorted_pair), top_k
-        _C.check(lib.hymeta_moe_gptq_gemm(C.byref(q13), st), "hymeta_moe_gptq_gemm (w13)")
+        _C.check(lib.hymeta_moe_gptq_gemm_rank(C.byref(q13), E, st), "hymeta_moe_gptq_gemm_rank (w13)")
         hact = torch.empty(P, inter, dtype=torch.bfloat16, device=dev)
         silu_and_mul(h13, out=hact)
         y = torch.empty(P, H, dtype=torch.bfloat16, device=dev)
         q2 = gptq_gemm_args(w2, hact, y, inter, H)
         q2.a_rows_div, q2.scale_rows, q2.row_scale = 1, _p(sorted_pair), _p(wts)
-        _C.check(lib.hymeta_moe_gptq_gemm(C.byref(q2), st), "hymeta_moe_gptq_gemm (w2)")
+        _C.check(lib.hymeta_moe_gptq_gemm_rank(C.byref(q2), E, st), "hymeta_moe_gptq_gemm_rank (w2)")
         c = _C.MoeCombineArgs()
         c.y, c.shared, c.out, c.pair_pos, c.topk_weights = _p(y), _p(shared), _p(out), _p(pair_pos), _p(wts)
         c.num_tokens, c.hidden, c.top_k = T, H, top_k
