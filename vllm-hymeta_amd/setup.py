@@ -11,7 +11,7 @@ setup(
     version="0.1.0",
     description="Hymeta hybrid-attention plugin for vLLM on AMD MI355X (gfx950): hand-written HIP kernels",
     packages=find_packages(include=["vllm_hymeta", "vllm_hymeta.*"]),
-    package_data={"vllm_hymeta": ["libhymeta_hip.so"]},
+    package_data={"vllm_hymeta": ["libhymeta_hip.so", "hymeta_calls.so"]},
     python_requires=">=3.10",
     install_requires=["torch", "transformers"],
     entry_points={
