@@ -1,4 +1,4 @@
-"""The router's scores and choice with its sums formed by halves that trade places: tokens, outputs and columns that do not fill its
+"""The routers' scores and choice with their sums formed by halves that trade places: tokens, outputs and columns that do not fill their
 rounds, against 64-bit sums."""
 import ctypes as C
 
@@ -32,3 +32,40 @@ def test_scores_and_choice(T, E, K, top):
     assert float((score.gather(1, picked) - best).abs().max()) <= slack
     assert float((weights.cpu().double() - best / (best.sum(1, keepdim=True) + 1e-20)).abs().max()) <= 4 * slack
     assert int(offsets[-1]) == T * top
+
+
+@pytest.mark.parametrize("T,E,K,top", [(1, 1, 8, 1), (3, 15, 2056, 2), (2, 17, 4104, 2), (5, 33, 256, 1), (256, 64, 520, 2)])
+def test_one_launch_router(T, E, K, top):
+    """Logits against 64 bits; choice, weights and the sort against the kernel's own bf16 logits.  The last token's row is NaN."""
+    from vllm_hymeta import _C
+    lib, g = _C.load(), gen(T * E + K)
+    x, w = torch.randn(T, K, generator=g).bfloat16(), (torch.randn(E, K, generator=g) * K ** -0.5).bfloat16()
+    x[-1, 0] = float("nan")
+    xd, wd = x.cuda(), w.cuda()
+    ids, weights, logits = torch.full((T, top), -9, dtype=torch.int32, device="cuda"), torch.zeros(T, top, device="cuda"), torch.zeros(T, E, dtype=torch.bfloat16, device="cuda")
+    offsets, pairs, pos, ticket = (torch.zeros(n, dtype=torch.int32, device="cuda") for n in (E + 1, T * top, T * top, 16))
+    a = _C.MoeRouterArgs()
+    a.x, a.gate_weight, a.logits_out, a.topk_ids, a.topk_weights, a.expert_offsets, a.sorted_pair, a.pair_pos, a.ticket = (
+        t.data_ptr() for t in (xd, wd, logits, ids, weights, offsets, pairs, pos, ticket))
+    a.x_stride_t, a.num_tokens, a.num_experts, a.top_k, a.renormalize, a.hidden = K, T, E, top, 0, K
+    a.local_expert_begin, a.local_expert_end = 0, E
+    for _ in range(2):                                       # the ticket is ready again
+        assert lib.hymeta_moe_router(C.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+    own, live = logits.cpu(), T - 1
+    exact = x[:live].double() @ w.double().t()
+    # fp32 sums of K terms in 256 strands, then one rounding to bf16
+    slack = 2.0 ** -8 * exact.abs() + 2.0 ** -24 * (K / 256 + 10) * (x[:live].double().abs() @ w.double().abs().t())
+    assert bool(((own[:live].double() - exact).abs() <= slack).all())
+    left, soft = own[:live].double().clone(), torch.softmax(own[:live].double(), 1)
+    picked = ids.cpu().long()
+    for k in range(top):
+        first = torch.tensor([int((row == row.max()).nonzero()[0]) for row in left], dtype=torch.long)
+        assert torch.equal(picked[:live, k], first)
+        assert torch.allclose(weights.cpu().double()[:live, k], soft.gather(1, first[:, None])[:, 0], rtol=2e-6, atol=0)
+        left.scatter_(1, first[:, None], -float("inf"))
+    assert picked[-1].tolist() == list(range(top)) and bool(torch.isnan(weights[-1]).all())
+    counts = torch.bincount(picked.flatten(), minlength=E)
+    assert torch.equal(offsets.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), counts.cumsum(0)]))
+    order = pairs.cpu().long()
+    assert torch.equal(order.sort().values, torch.arange(T * top)) and torch.equal(picked.flatten()[order], picked.flatten().sort().values)
+    assert torch.equal(order[pos.cpu().long()], torch.arange(T * top))

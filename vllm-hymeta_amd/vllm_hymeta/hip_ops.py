@@ -1378,9 +1378,13 @@ def moe_forward(x: torch.Tensor, router_logits: Optional[torch.Tensor], w13: tor
     if gptq:
         _require(isinstance(w2, GptqExperts), "w13 and w2 must both be GPTQ stacks")
         n_local = (local_experts[1] - local_experts[0]) if local_experts is not None else w13.shape[0]
-        _require(router_logits is not None or gate_weight is not None, "router_logits or gate_weight must be given")
-        total = gate_weight.shape[0] if gate_weight is not None else router_logits.shape[1]
-        if x.shape[0] * top_k > _moe_gptq_fused_rows(w13, w2, n_local, total):
+        if x.shape[0] * top_k > MOE_GPTQ_FUSED_ROWS_PER_EXPERT * max(n_local, 1):
+            _require(router_logits is not None or gate_weight is not None, "router_logits or gate_weight must be given")
+            total = gate_weight.shape[0] if gate_weight is not None else router_logits.shape[1]
+            expands = x.shape[0] * top_k > _moe_gptq_fused_rows(w13, w2, n_local, total)      # (never the smaller limit)
+        else:
+            expands = False
+        if expands:
             held = w13.shape[0]
             if held == total and local_experts is not None and tuple(local_experts) != (0, total):
                 lo_, hi_ = local_experts      # expand the rank's experts only
