@@ -69,3 +69,34 @@ def test_one_launch_router(T, E, K, top):
     order = pairs.cpu().long()
     assert torch.equal(order.sort().values, torch.arange(T * top)) and torch.equal(picked.flatten()[order], picked.flatten().sort().values)
     assert torch.equal(order[pos.cpu().long()], torch.arange(T * top))
+
+
+@pytest.mark.parametrize("E,top,mode", [(3, 3, "sigmoid"), (70, 9, "sigmoid"), (5, 2, "softmax"), (130, 66, "softmax")])
+def test_scores_that_are_no_numbers(E, top, mode):
+    """A token whose scores are all NaN, or -inf but for one: experts that exist, each once, with weights that say so."""
+    from vllm_hymeta import _C
+    lib, g, T, K = _C.load(), gen(E), 6, 64
+    x, w, bias = torch.randn(T, K, generator=g).bfloat16(), torch.randn(E, K, generator=g) * K ** -0.5, torch.zeros(E)
+    x[2, 5] = x[5, 0] = float("nan")
+    if mode == "softmax":
+        bias[:] = -float("inf")
+        bias[E - 2] = 0.0
+    xd, wd, bd = x.cuda(), w.cuda(), bias.cuda()
+    ids, weights = torch.full((T, top), -9, dtype=torch.int32, device="cuda"), torch.zeros(T, top, device="cuda")
+    offsets, pairs, pos = (torch.full((n,), -9, dtype=torch.int32, device="cuda") for n in (E + 1, T * top, T * top))
+    a = _C.MoeRouteSigmoidArgs()
+    a.x, a.router_weight, a.router_bias, a.topk_ids, a.topk_weights, a.expert_offsets, a.sorted_pair, a.pair_pos = (
+        t.data_ptr() for t in (xd, wd, bd, ids, weights, offsets, pairs, pos))
+    a.num_tokens, a.num_experts, a.top_k, a.hidden, a.act_dtype, a.scale, a.x_stride_t = T, E, top, K, _C.HYMETA_BF16, 1.0, K
+    a.score_mode = _C.ROUTE_SOFTMAX_CHOSEN if mode == "softmax" else _C.ROUTE_SIGMOID_SUM
+    assert lib.hymeta_moe_route_sigmoid(C.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+    picked, weights = ids.cpu(), weights.cpu()
+    assert bool(((picked >= 0) & (picked < E)).all()) and all(len(set(row)) == top for row in picked.tolist())
+    assert torch.equal(torch.isnan(weights), torch.isnan(x).any(1)[:, None].expand(T, top))
+    live = [t for t in range(T) if t not in (2, 5)]
+    if mode == "softmax":
+        assert bool((picked[live, 0] == E - 2).all()) and torch.equal(weights[live], torch.eye(1, top).expand(len(live), top))
+    else:
+        best = torch.sigmoid(x[live].double() @ w.double().t()).topk(top).values
+        assert torch.allclose(weights[live].double(), best / best.sum(1, keepdim=True), rtol=0, atol=1e-5)
+    assert int(offsets[-1]) == T * top and sorted(pos.cpu().tolist()) == list(range(T * top))

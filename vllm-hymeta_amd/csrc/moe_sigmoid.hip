@@ -14,7 +14,7 @@ namespace {
 // experts lane, lane + 64, ..., the wave reduces to the largest score and, among equals, the lowest expert.
 //
 // Bound by a round's loads on their way (four steps' at a time) and by its sums: a wave's 32 sums over 64 lanes are formed by halves that
-// trade places (wave_sums), 31 additions in place of 192.  LDS as the experts need it, so that it does not keep workgroups away.  Eight experts of
+// trade places (wave_sums), 32 additions in place of 192.  LDS as the experts need it, so that it does not keep workgroups away.  Eight experts of
 // 3584 columns, 8192 tokens 41 us (53 with 192 and room for 1024 experts), 1150 of 2048 columns 10 (13), one 9 (12).
 constexpr int kRouteTokens = 4;
 
@@ -158,6 +158,13 @@ __global__ __launch_bounds__(256) void moe_scores_topk_kernel(hymeta_moe_route_s
     return;
   }
   float total = 0.f;
+  float* taken = s_choice + wave * R;
+  for (int e = lane; e < E; e += 64) taken[e] = 0.f;
+  auto lowest = [](int x) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x = min(x, __shfl_xor(x, o, 64));
+    return x;
+  };
   for (int k = 0; k < a.top_k; ++k) {
     float best = -INFINITY;
     int arg = 0x7fffffff;
@@ -165,15 +172,23 @@ __global__ __launch_bounds__(256) void moe_scores_topk_kernel(hymeta_moe_route_s
       const float v = score[e];
       if (v > best) best = v, arg = e;            // ascending e: the first of equals stays
     }
-    const float top = wave_max(best);
-    int cand = best == top ? arg : 0x7fffffff;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) cand = min(cand, __shfl_xor(cand, o, 64));
+    float top = wave_max(best);
+    int cand = lowest(best == top ? arg : 0x7fffffff);
+    if (cand == 0x7fffffff) {
+      // every score left is NaN or -inf: the first expert not taken, with its own score, so that a row of NaN stays one
+      for (int e = lane; e < E; e += 64)
+        if (taken[e] == 0.f) {
+          arg = e;
+          break;
+        }
+      cand = lowest(arg);
+      top = score[cand];
+    }
     total += top;
     if (lane == 0) {
       a.topk_ids[t * a.top_k + k] = cand;
       top_of[k] = top;
-      if (cand != 0x7fffffff) score[cand] = -INFINITY;      // taken (none: every score left is NaN or -inf)
+      taken[cand] = 1.f, score[cand] = -INFINITY;
     }
     __builtin_amdgcn_wave_barrier();
     __threadfence_block();
