@@ -53,6 +53,8 @@ def reference(q, rows, C, scale, sink, window, keep, chunk, softcap, bias, gate,
     *[(c, 16, 64, [1, 1], [64 * n - 1, 20], dict(sink=True, gate=True)) for c, n in ((384, 2), (512, 3), (256, 8), (512, 9))],      # partials of a row
     # as many of 128 columns as a thread takes at once, four or eight, and one more; statistics for two each
     *[(c, 16, 64, [1], [64 * n - 1], dict(sink=True, gate=True)) for c, n in ((512, 16), (384, 17), (256, 32), (512, 33), (512, 129))],
+    # as many (row, head) pairs as are merged in parts of the columns, and a row more
+    (512, 16, 64, [29, 1], [2000, 300], dict(sink=True)), (384, 16, 64, [30, 1], [2000, 300], dict(sink=True, gate=True)), (512, 16, 64, [30, 1], [2000, 5], {}),
 ])
 def test_against_64_bits(C, H, page, lens, ctxs, opts):
     from vllm_hymeta import hip_ops

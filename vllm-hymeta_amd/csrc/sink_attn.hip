@@ -840,10 +840,11 @@ constexpr int kMaxPartials = 512 * kDecodeWaves;
 // Up to as many partials a (row, head) goes to the kernel that holds them all in registers: more partials are for few rows, which
 // leave the chip room for a workgroup each.
 constexpr int kFewPartials = 8;
-// Columns of a workgroup where a row has more partials: a row of 512 then has four workgroups that take the partials four at
-// a time, and not one whose threads all take every partial.  16 heads on 512 + 64, 3 rows at 9600 keys 47.3 -> 23.5 us, 12 at 5000
-// 42 -> 36; 28 heads, a row at 30000 60 -> 25.
-constexpr int kPartColumns = 128;
+// Columns of a workgroup where up to kPartRows (row, head) pairs have more partials: a row of 512 then has four workgroups that take
+// the partials four at a time, and not one whose threads all take every partial.  16 heads on 512 + 64, 3 rows at 9600 keys 47.3 ->
+// 23.5 us; 28 heads, a row at 30000 60 -> 25.  More pairs fill the chip by themselves, and the parts all read the statistics: with /
+// without parts 16 heads, 20 rows at 7000 keys 39.7 / 41.1, 40 50.5 / 48.9, six portions of 40 at 1200 49.6 / 42.8; 28 heads, 20 rows at 3500 40.2 / 39.3.
+constexpr int kPartColumns = 128, kPartRows = 512;
 
 // Columns c .. c + 3 of row t's head h, from the weighted values and the weights' sum.
 __device__ __forceinline__ void store_row(const hymeta_sink_attention_args& a, f32x4v acc, float l, int64_t t, int h, int c) {
@@ -1197,8 +1198,9 @@ void launch_combine(const hymeta_sink_attention_args& a, hipStream_t st, int spl
     else hipLaunchKernelGGL(sink_attention_combine_few_kernel<kFewPartials>, grid, dim3(kCombineThreads), 0, st, a, splits, hs);
     return;
   }
-  const unsigned parts = a.v_dim > kPartColumns && std::max(splits, ps.splits) > kFewPartials ? a.v_dim / kPartColumns : 1;
-  const dim3 grid((ps.least > 1 ? a.num_seqs : 0) + (ps.splits > 1 ? a.num_tokens : 0), heads, parts);
+  const int64_t rows = (ps.least > 1 ? a.num_seqs : 0) + static_cast<int64_t>(ps.splits > 1 ? a.num_tokens : 0);
+  const bool apart = a.v_dim > kPartColumns && rows * heads <= kPartRows && std::max(splits, ps.splits) > kFewPartials;
+  const dim3 grid(static_cast<unsigned>(rows), heads, apart ? a.v_dim / kPartColumns : 1);
   hipLaunchKernelGGL(sink_attention_combine_kernel, grid, dim3(kCombineThreads), 0, st, a, splits, hs, ps);
 }
 
