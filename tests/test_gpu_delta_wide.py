@@ -19,7 +19,9 @@ EDGES = [8, 63, 64, 65, 130, 7, 128, 129, 20, 1, 130, 97, 126, 127, 128]        
     # more pairs than half of the compute units: the shortest sequences whole, the others' halves side by side; 80, 136 and 104 whole
     (128, 128, 28, 14, [300, 257, 299, 260, 321, 270]), (128, 128, 28, 14, [300, 290, 257, 260, 299, 270, 5]), (64, 256, 15, 15, [257] * 6),
     (32, 128, 28, 28, [300] * 5), (96, 128, 28, 28, [300] * 6 + [7]),      # and a portion too short for a chunk where none is expected:
-    (128, 128, 28, 14, [300] * 6 + [7]), (64, 128, 28, 7, [64] * 8 + [3]), (128, 128, 16, 16, [64, 64, 64, 5]), (128, 96, 12, 4, [64, 64, 64, 5])])
+    (128, 128, 28, 14, [300] * 6 + [7]), (64, 128, 28, 7, [64] * 8 + [3]), (128, 128, 16, 16, [64, 64, 64, 5]), (128, 96, 12, 4, [64, 64, 64, 5]),
+    # a chunk's sequence found in two round trips and in three
+    (64, 64, 4, 4, [1] * 40 + [70] + [1] * 24 + [64, 130] + [1] * 63 + [9]), (32, 32, 2, 2, [1] * 66 + [65] + [1] * 4100 + [130, 3])])
 def test_wide_slices_equal_narrow_ones(D, Dv, H, Hk, lens):
     """Both multiply the same operands (fp32 as two bf16 parts, 2^-17 of the operand) and add in another order: 1e-5 of the
     norm covers what that rounding grows to over a few chunks.  Rows at a chunk's edges, several chunks, a portion that goes
