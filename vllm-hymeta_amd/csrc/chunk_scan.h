@@ -44,8 +44,8 @@ inline int scan_waves(int64_t lanes, int v_dim) {
 // As many segments as run at the same time, eight waves to a compute unit: one prompt of 8192 rows of 28 heads of 128
 // columns took 138 us (lightning, the keys in one part) and 120 (plain decays) in 256 workgroups of eight waves, 152 and 136 in 512, 175 and 156
 // in 1024; of 64 columns 131 us in 512 workgroups of four, 189 in 256, 147 in 1024.  At least 64 rows each (192 / 64, us): 28 heads
-// of 128 x 128, one portion of 300 rows 27.9 / 22.8, of 520 46.2 / 27.8, of 1000 40.4 / 33.3; 16 heads of 64 x 128, one of 520 34.2 / 19.0,
-// two of 400 with 128 rows of state 36.7 / 23.4.  Not beside many short portions, which fill what one segment leaves idle and wait
+// of 128 x 128, one portion of 400 rows 37.4 / 26.7, of 1000 42.2 / 35.0; 16 heads of 64 x 128, one of 577 19.3 / 15.3,
+// two of 450 with 128 rows of state 42.4 / 26.3.  Not beside many short portions, which fill what one segment leaves idle and wait
 // for the summaries otherwise: 28 heads of 128 x 128, one of 300 beside 32 single rows 29.5 / 27.5, beside 63 30.5 / 36.7;
 // 32 heads of 64 columns, one of 520 beside 63 37.0 / 25.8.
 //
@@ -56,33 +56,60 @@ inline int scan_waves(int64_t lanes, int v_dim) {
 // Up to kMostUnchained segments every one works out the state in front of it for itself, from the summaries before it, which saves a
 // launch (6 to 9 us) for at most ten reads of 64 KB: 16 heads of 128 columns, five portions of 700 rows in four segments 41 -> 31 us, of
 // 64 columns three of 2000 64 -> 57; with 16 segments level.
-constexpr int kMostUnchained = 10, kSegmentRows = 64, kManySegmentRows = 192, kManyColumns = 131072;
+// More of them take the chain's launch and more states to and fro, which single rows and short portions wait for unless the chip is
+// through with a segment at once: in segments of one chunk, or alone (at least 192 rows each otherwise, but for the first ten).  2048
+// rows of 16 heads of 128 x 128, plain decays: alone 32.2 us in 16 segments, 36.0 in 8; beside 63 single rows 47.3 and 38.2; 7 heads,
+// lightning, beside 63 37.6 in 32 of one chunk, 45.5 in 8.  Where segments of 64 columns take two places on every compute unit (32 heads) 39.1 in
+// 16, 35.0 in 8.
+constexpr int kMostUnchained = 10, kSegmentRows = 64, kManySegmentRows = 192, kManyColumns = 131072, kSomeColumns = 49152;
 struct ScanSegments {
   int rows = 0x7fffffff, count = 0;        // rows of a segment; bound on the segments' numbers
   bool chained = false;                    // whether a launch of its own turns the summaries into the states in front of the segments
   int64_t lanes = 0;                       // (segment, head) pairs that run side by side
 };
+// Columns of a segment's workgroup, and how many of them run at the same time.
+inline int scan_columns(int v_dim) { return v_dim % 128 == 0 ? 128 : v_dim % 64 == 0 ? 64 : 32; }
+inline int64_t scan_slots(int v_dim) { return 256 * (128 / scan_columns(v_dim)); }
+inline int64_t scan_slices(int num_heads, int v_dim) { return num_heads * std::max<int64_t>(v_dim / scan_columns(v_dim), 1); }
 // Segments of a step of `portions` long ones: how many of a head's fit on the chip beside the others.
 inline int64_t scan_segments_wanted(int64_t portions, int num_heads, int v_dim, int max_query_len) {
-  const int64_t wide = v_dim % 128 == 0 ? 128 : v_dim % 64 == 0 ? 64 : 32, slots = 256 * (128 / wide);
-  return std::min<int64_t>(slots / (portions * num_heads * std::max<int64_t>(v_dim / wide, 1)), max_query_len / kSegmentRows);
+  return std::min<int64_t>(scan_slots(v_dim) / (portions * scan_slices(num_heads, v_dim)), max_query_len / kSegmentRows);
 }
-inline int scan_segment_rows(int num_seqs, int num_heads, int v_dim) {
-  return static_cast<int64_t>(num_seqs) * num_heads * v_dim > kManyColumns ? kManySegmentRows : kSegmentRows;
+// Whether segments of a few chunks pay: a portion's chunks one behind the other, against those of a segment twice (summary and rows, which a
+// segment's eight staging waves halve), a launch more, and the states' way through memory, which goes with the places that the
+// segments take (and the short portions beside them, a sixteenth of one each) and is shorter where all of a head's are on one die
+// (heads in eights).  A chunk with silu takes half as long again.  Rounded to chunks there may be two segments left of three: never.
+// Us, cut / whole, plain decays: 28 heads of 128 x 128, three portions of 200 rows 23.0 / 18.8 (two segments), one of 256 18.6 / 17.2, two 23.2 / 18.4, three
+// of 260 25.4 / 22.7, one 17.4 / 20.2, three of 500 29.8 / 33.2; 16 heads, two of 256 16.4 / 17.5; lightning, 28 heads, one of 256 21.0 /
+// 23.7, two 25.3 / 24.7.  Columns in 64s or fewer, two and more workgroups on a compute unit: 56 heads, one of 256 15.5 / 17.4, three of 400 34.3 / 30.4;
+// 32 heads, three of 260 19.5 / 21.2; 28 heads of 64 x 64, five of 450 25.3 / 24.1.  192 rows with nothing to stage are level or slower: 12.4 / 10.9.
+inline bool scan_segments_pay(int64_t places, int pieces, int num_heads, int v_dim, int max_query_len, int rows, bool silu) {
+  const int64_t slots = scan_slots(v_dim), chunks = (max_query_len + kScanRows - 1) / kScanRows, each = rows / kScanRows;
+  if (pieces < 3 || (!silu && chunks < 4)) return false;
+  if (v_dim % 128 != 0) return 5 * (chunks - 2 * each) * slots > 7 * (3 * places - slots);
+  return 2 * (chunks - each) * slots > (silu ? 1 : 3) * slots + (num_heads % 8 == 0 ? 5 : 7) * places;
 }
-inline ScanSegments scan_segments(int num_tokens, int num_seqs, int num_heads, int v_dim, int max_query_len) {
-  const int64_t portions = long_portions(num_tokens, num_seqs, max_query_len);
-  const int64_t want = std::min<int64_t>(scan_segments_wanted(portions, num_heads, v_dim, max_query_len),
-                                         max_query_len / scan_segment_rows(num_seqs, num_heads, v_dim));
+inline ScanSegments scan_segments(int num_tokens, int num_seqs, int num_heads, int v_dim, int max_query_len, bool silu) {
+  const int64_t portions = long_portions(num_tokens, num_seqs, max_query_len), columns = static_cast<int64_t>(num_seqs) * num_heads * v_dim;
+  const int64_t fit = scan_segments_wanted(portions, num_heads, v_dim, max_query_len);
+  const bool many = columns > kManyColumns;
+  const int64_t want = many ? std::min<int64_t>(fit, max_query_len / kManySegmentRows) : fit;
   ScanSegments sg;
   sg.lanes = portions * num_heads;
   if (want < 3) return sg;
-  const int rows = static_cast<int>((max_query_len + want - 1) / want + kScanRows - 1) / kScanRows * kScanRows;
+  auto rows_of = [=](int64_t pieces) { return static_cast<int>((max_query_len + pieces - 1) / pieces + kScanRows - 1) / kScanRows * kScanRows; };
+  int rows = rows_of(want);
+  auto pieces = [&] { return (max_query_len + rows - 1) / rows; };
+  if (!many) {
+    const int64_t slots = scan_slots(v_dim), slices = scan_slices(num_heads, v_dim);
+    if (pieces() > kMostUnchained && rows > kScanRows && (columns > kSomeColumns || (v_dim % 128 != 0 && 8 * portions * slices * pieces() > 7 * slots)))
+      rows = rows_of(std::max<int64_t>(kMostUnchained, std::min<int64_t>(fit, max_query_len / kManySegmentRows)));
+    if (!scan_segments_pay(portions * slices * pieces() + (num_seqs - portions) * slices / 16, pieces(), num_heads, v_dim, max_query_len, rows, silu)) return sg;
+  }
   const int64_t cuts = (std::min<int64_t>(num_tokens, static_cast<int64_t>(num_seqs) * max_query_len) - 1) / rows;
   const int64_t count = cuts + std::min<int64_t>(num_seqs, cuts);
   if (num_seqs + count > 65535) return sg;
-  sg.rows = rows, sg.count = static_cast<int>(count), sg.lanes *= (max_query_len + rows - 1) / rows;
-  sg.chained = (max_query_len + rows - 1) / rows > kMostUnchained;
+  sg.rows = rows, sg.count = static_cast<int>(count), sg.lanes *= pieces(), sg.chained = pieces() > kMostUnchained;
   return sg;
 }
 // The workspace: per segment and head its summary, then the state in front of it; the segments' sums of log2 decays.

@@ -185,7 +185,7 @@ extern "C" int hymeta_decay_scan(const hymeta_decay_scan_args* args, hymeta_stre
   hipStream_t st = begin_launches(stream);
   // (portions shorter than a chunk's least run in the same launch)
   if (chunk_shape(a) && a.max_query_len >= 2) {
-    const ScanSegments sg = scan_segments(a.num_tokens, a.num_seqs, a.num_heads, a.v_dim, a.max_query_len);
+    const ScanSegments sg = scan_segments(a.num_tokens, a.num_seqs, a.num_heads, a.v_dim, a.max_query_len, false);
     const size_t need = scan_segment_bytes(sg.count, a.num_heads, a.head_dim, a.v_dim);
     if (need > 0 && (!a.workspace || a.workspace_bytes < need)) return HYMETA_ERR_WORKSPACE;
     const ChunkScanArgs c{static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.k), static_cast<const uint16_t*>(a.v), a.q_stride_t, a.k_stride_t,

@@ -249,7 +249,7 @@ extern "C" int hymeta_lightning_attention(const hymeta_lightning_attention_args*
   hipStream_t st = begin_launches(stream);
   // (portions shorter than a chunk's least run in the same launch)
   if (chunk_shape(a) && a.max_query_len >= 2) {
-    const ScanSegments sg = scan_segments(a.num_tokens, a.num_seqs, a.num_heads, a.v_dim, a.max_query_len);
+    const ScanSegments sg = scan_segments(a.num_tokens, a.num_seqs, a.num_heads, a.v_dim, a.max_query_len, true);
     const size_t need = scan_segment_bytes(sg.count, a.num_heads, a.head_dim, a.v_dim);
     if (need > 0 && (!a.workspace || a.workspace_bytes < need)) return HYMETA_ERR_WORKSPACE;
     const uint16_t* qkv = static_cast<const uint16_t*>(a.qkv);
