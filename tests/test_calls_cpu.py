@@ -1,4 +1,10 @@
 """The native host side of calls: loaded with the library, and everything but plain device tensors is left to Python."""
+import os
+import shutil
+import subprocess
+import sysconfig
+import warnings
+
 import pytest
 import torch
 
@@ -17,3 +23,33 @@ def test_native_calls_leave_the_rest_to_python():
         assert getattr(_C.calls, name)(*[q] * 26) is None and getattr(_C.calls, name)() is None
     with pytest.raises(TypeError):
         _C.calls.setup(_C)
+
+
+UNRESOLVED = "extern void not_in_this_torch(void); void *PyInit_hymeta_calls(void) { not_in_this_torch(); return 0; }"
+OLDER = """
+#include <Python.h>
+static struct PyModuleDef def = {PyModuleDef_HEAD_INIT, "hymeta_calls", 0, -1, 0};
+PyMODINIT_FUNC PyInit_hymeta_calls(void) {
+  PyObject *m = PyModule_Create(&def);
+  PyModule_AddObject(m, "built_for", Py_BuildValue("(ssi)", "2.0.0 another", "3.10", 9));
+  return m;
+}
+"""
+
+
+@pytest.mark.parametrize("source,says", [(UNRESOLVED, "does not load"), (OLDER, "is built for")], ids=["unresolved", "older"])
+def test_native_calls_of_another_torch_count_as_absent(tmp_path, monkeypatch, source, says):
+    from vllm_hymeta import _C
+    (tmp_path / "calls.c").write_text(source)
+    if shutil.which("gcc") is None or not os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h")):
+        pytest.skip("no gcc or no Python.h")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-Wl,-z,now", "-I", sysconfig.get_paths()["include"], str(tmp_path / "calls.c"), "-o", str(tmp_path / "hymeta_calls.so")], check=True)
+    monkeypatch.setattr(_C, "_CALLS_NAME", str(tmp_path / "hymeta_calls.so"))      # (an absolute path stands for itself)
+    monkeypatch.setattr(_C, "_lib", None)
+    monkeypatch.setattr(_C, "calls", None)
+    with pytest.warns(RuntimeWarning, match=says):
+        lib = _C.load()
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _C.load() is lib and _C.calls is None
+    assert lib.hymeta_abi_version() == _C.ABI_VERSION

@@ -10,6 +10,7 @@
 #include <cstring>
 #include <initializer_list>
 #include <limits>
+#include <string>
 
 #include "hymeta_hip.h"
 
@@ -450,4 +451,19 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "hymeta_calls", nullptr, -1, me
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_hymeta_calls() { return PyModule_Create(&module_def); }
+// built_for: what the loader compares (_C.py), as tensors and structs are read by their layouts at build time
+PyMODINIT_FUNC PyInit_hymeta_calls() {
+  PyObject* module = PyModule_Create(&module_def);
+  if (module == nullptr) return nullptr;
+  const std::string python = std::to_string(PY_MAJOR_VERSION) + "." + std::to_string(PY_MINOR_VERSION);
+  PyObject* built_for = Py_BuildValue("(ssinnnnnn)", HYMETA_CALLS_TORCH, python.c_str(), HYMETA_ABI_VERSION, Py_ssize_t(sizeof(hymeta_sink_attention_args)),
+                                      Py_ssize_t(sizeof(hymeta_paged_decode_args)), Py_ssize_t(sizeof(hymeta_swa_prefill_args)),
+                                      Py_ssize_t(sizeof(hymeta_lightning_attention_args)), Py_ssize_t(sizeof(hymeta_decay_scan_args)),
+                                      Py_ssize_t(sizeof(hymeta_delta_rule_args)));
+  if (built_for == nullptr || PyModule_AddObject(module, "built_for", built_for) < 0) {
+    Py_XDECREF(built_for);
+    Py_DECREF(module);
+    return nullptr;
+  }
+  return module;
+}

@@ -850,13 +850,13 @@ def load() -> C.CDLL:
     version = lib.hymeta_abi_version()
     if version != ABI_VERSION:
         raise RuntimeError(f"{path}: ABI version {version}, binding expects {ABI_VERSION}")
-    _lib = lib
     _load_calls(lib)
+    _lib = lib
     return lib
 
 
-# The native host side of small calls (csrc/calls.cpp): None until the library is loaded, or where it is not built or the library
-# lacks a function of its.
+# The native host side of small calls (csrc/calls.cpp): None until the library is loaded, where it is not built or built for another
+# torch, Python or header, or where the library lacks a function of its.
 calls = None
 _CALLS_NAME = "hymeta_calls.so"
 _CALLED = ("hymeta_sink_attention", "hymeta_sink_attention_workspace_bytes", "hymeta_sink_attention_portion_workspace_bytes",
@@ -866,6 +866,15 @@ _CALLED = ("hymeta_sink_attention", "hymeta_sink_attention_workspace_bytes", "hy
            "hymeta_delta_rule", "hymeta_delta_rule_workspace_bytes")
 
 
+def _calls_built_for():
+    """What ``hymeta_calls.so`` has to be built for: the torch and the Python that run, the header that this binding is written for."""
+    import sys
+
+    import torch
+    structs = (SinkAttentionArgs, PagedDecodeArgs, SwaPrefillArgs, LightningAttentionArgs, DecayScanArgs, DeltaRuleArgs)
+    return (f"{torch.__version__} {torch.version.git_version}", "%d.%d" % sys.version_info[:2], ABI_VERSION, *map(C.sizeof, structs))
+
+
 def _load_calls(lib: C.CDLL) -> None:
     global calls
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), _CALLS_NAME)
@@ -873,11 +882,22 @@ def _load_calls(lib: C.CDLL) -> None:
         return
     import importlib.machinery
     import importlib.util
+    import warnings
 
     from . import hip_ops
     loader = importlib.machinery.ExtensionFileLoader("hymeta_calls", path)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("hymeta_calls", loader))
-    loader.exec_module(module)
+    try:
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("hymeta_calls", loader))
+        loader.exec_module(module)
+    except ImportError as error:
+        warnings.warn(f"{path} does not load ({error}): small calls run their host side in Python; `make -C vllm-hymeta_amd` builds it again",
+                      RuntimeWarning, stacklevel=3)
+        return
+    found, wanted = getattr(module, "built_for", None), _calls_built_for()
+    if found != wanted:
+        warnings.warn(f"{path} is built for {found}, not for {wanted}: small calls run their host side in Python; `make -C vllm-hymeta_amd` builds it again",
+                      RuntimeWarning, stacklevel=3)
+        return
     module.setup(hip_ops, *(C.cast(getattr(lib, name), C.c_void_p).value for name in _CALLED))
     calls = module
 
