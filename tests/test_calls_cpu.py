@@ -53,3 +53,16 @@ def test_native_calls_of_another_torch_count_as_absent(tmp_path, monkeypatch, so
         warnings.simplefilter("error")
         assert _C.load() is lib and _C.calls is None
     assert lib.hymeta_abi_version() == _C.ABI_VERSION
+
+
+@pytest.mark.parametrize("lacks", ["CXX=no-such-compiler", "PYTHON=no-such-python"])
+def test_the_library_is_made_without_what_the_calls_need(tmp_path, lacks):
+    """The rule of the native calls alone, in a folder of its own (the library's objects are not made again)."""
+    package = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "vllm-hymeta_amd")
+    if shutil.which("make") is None:
+        pytest.skip("no make")
+    made = tmp_path / "hymeta_calls.so"
+    made.write_text("of an earlier torch")
+    os.utime(made, (1, 1))
+    run = subprocess.run(["make", "-C", package, lacks, f"OBJDIR={tmp_path}", f"CALLS={made}", str(made)], capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0 and "the package works without it" in run.stderr and not made.exists()
