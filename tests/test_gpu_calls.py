@@ -147,3 +147,27 @@ def test_refused_as_in_python(monkeypatch):
                 call()
             messages.append((type(error.value), str(error.value)))
         assert messages[0] == messages[1]
+
+
+def _long_prompt(hip_ops, rows=700, **kw):
+    g = gen(rows)
+    qkv, state, decay = _bf(g, rows, 4 * 384), torch.zeros(1, 4, 128, 128, device="cuda"), torch.full((4,), 0.9, device="cuda")
+    return hip_ops.lightning_attention(qkv, state, decay, 4, 128, 128, _i32(0, rows), _i32(0), _i32(0), kw.get("most", rows))
+
+
+@pytest.mark.parametrize("error", [KeyboardInterrupt, RuntimeError, torch.cuda.OutOfMemoryError])
+def test_an_exception_in_between_is_the_calls(monkeypatch, error):
+    """What is raised while the native side asks for a workspace is not taken for a refusal."""
+    from vllm_hymeta import _C, hip_ops
+    _C.load()
+    workspace, raised = hip_ops._workspace, []
+
+    def once(*args):
+        if not raised:
+            raised.append(args)
+            raise error("in between")
+        return workspace(*args)
+    monkeypatch.setattr(hip_ops, "_workspace", once)
+    with pytest.raises(error, match="in between"):
+        _long_prompt(hip_ops)
+    assert len(raised) == 1 and torch.isfinite(_long_prompt(hip_ops)).all()

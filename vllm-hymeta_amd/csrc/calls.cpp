@@ -3,6 +3,7 @@
 // struct).  A function here takes what its namesake in hip_ops.py accepts from plain tensors; whatever else it meets (a refused
 // shape or type, a tensor subclass, an exception) it answers with None, and the namesake goes on in Python, which raises what there
 // is to raise.  It returns the output, or the library's status if that is not 0.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
 
@@ -145,7 +146,8 @@ PyObject* launch(Args& in, F* function, const A& args, hymeta_stream_t stream, a
   return status == HYMETA_OK ? THPVariable_Wrap(std::move(out)) : PyLong_FromLong(status);
 }
 
-// What every function here is called through.
+// What every function here is called through.  A type or value that is refused is Python's to say, like whatever torch throws in front of
+// the launch; an exception from Python that runs in between (an interrupt, no memory for a workspace) is the call's.
 template <PyObject* (*F)(Args&, PyObject* const*)>
 PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Args a(args, n);
@@ -154,12 +156,13 @@ PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
       PyObject* out = F(a, args);
       if (out != nullptr || a.launched) return out;
     }
+  } catch (python_error& error) {
+    error.restore();
   } catch (...) {
-    if (a.launched) {
-      PyErr_SetString(PyExc_RuntimeError, "no tensor for an output");
-      return nullptr;
-    }
+    if (a.launched) PyErr_SetString(PyExc_RuntimeError, "no tensor for an output");
   }
+  if (PyErr_Occurred() && (a.launched || !(PyErr_ExceptionMatches(PyExc_TypeError) || PyErr_ExceptionMatches(PyExc_ValueError) || PyErr_ExceptionMatches(PyExc_OverflowError))))
+    return nullptr;
   PyErr_Clear();
   Py_RETURN_NONE;
 }
