@@ -171,3 +171,82 @@ def test_an_exception_in_between_is_the_calls(monkeypatch, error):
     with pytest.raises(error, match="in between"):
         _long_prompt(hip_ops)
     assert len(raised) == 1 and torch.isfinite(_long_prompt(hip_ops)).all()
+
+
+def _small_calls(hip_ops):
+    """Name and call of one small problem of every function but the recurrences' siblings."""
+    g = gen(11)
+    q, cache, tables = _bf(g, 2, 4, 128), _bf(g, 2, 8, 64, 2, 128), torch.arange(8, dtype=torch.int32, device="cuda").view(2, 4)
+    rows, starts, lens, slots = _bf(g, 2, 4 * 384), _i32(0, 1, 2), _i32(130, 3), _i32(0, 1)
+    state, log2, decay = torch.zeros(2, 4, 128, 128, device="cuda"), torch.zeros(2, 4, device="cuda"), torch.full((4,), 0.9, device="cuda")
+    both = _bf(g, 8, 64, 2, 256)
+    return [
+        ("sink_attention", lambda: hip_ops.sink_attention(q, both, tables, starts, lens, 2, 128, 128, 0.1, 1, 130)),
+        ("meta_swa_paged_decode", lambda: hip_ops.meta_swa_paged_decode(q, cache[0], cache[1], lens, tables)),
+        ("meta_swa_prefill", lambda: hip_ops.meta_swa_prefill(q, starts, 1, key_cache=cache[0], value_cache=cache[1], block_tables=tables, seq_lens_k=lens, max_seqlen_k=130)),
+        ("lightning_attention", lambda: hip_ops.lightning_attention(rows, state.clone(), decay, 4, 128, 128, starts, lens, slots, 1)),
+        ("decay_scan", lambda: hip_ops.decay_scan(q, q, q, state.clone(), starts, lens, slots, 1, decay=decay)),
+        ("delta_rule", lambda: hip_ops.delta_rule(q, q, q, q[:, :, 0].contiguous(), log2, state.clone(), starts, lens, slots, 1, 0.1, 1e-6)),
+    ]
+
+
+@pytest.mark.parametrize("at", range(6))
+def test_outputs_come_from_what_stands_for_torch_empty(monkeypatch, at):
+    from vllm_hymeta import _C, hip_ops
+    _C.load()
+    name, call = _small_calls(hip_ops)[at]
+    call()                                                   # (its workspace is there)
+    plain, empty, made, module, answered = call(), torch.empty, [], _C.calls, []
+
+    class Noting:
+        def __getattr__(self, attribute):
+            return lambda *args: answered.append(attribute) or getattr(module, attribute)(*args)
+
+    def filled(*size, **kw):
+        made.append(empty(*size, **kw).fill_(7))
+        return made[-1]
+    monkeypatch.setattr(_C, "calls", Noting())
+    monkeypatch.setattr(torch, "empty", filled)
+    out = call()
+    assert answered == [name] and len(made) == 1 and made[0].data_ptr() == out.data_ptr() and torch.equal(out, plain)
+
+
+@pytest.mark.parametrize("at", range(6))
+def test_on_another_stream_and_inside_a_mode(monkeypatch, at):
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from vllm_hymeta import hip_ops
+    name, call = _small_calls(hip_ops)[at]
+    plain, side = call(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        _both(monkeypatch, name, lambda: [call()])
+    torch.cuda.current_stream().wait_stream(side)
+
+    class Through(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    with Through():
+        inside = call()
+    assert torch.equal(inside, plain)
+
+
+def test_subclasses_and_transforms_are_left_to_python(monkeypatch):
+    from vllm_hymeta import _C, hip_ops
+    _C.load()
+
+    class Own(torch.Tensor):
+        pass
+    g = gen(5)
+    rows, starts, lens, slots, decay = _bf(g, 2, 4 * 384), _i32(0, 1, 2), _i32(0, 3), _i32(0, 1), torch.full((4,), 0.9, device="cuda")
+    state = torch.zeros(2, 4, 128, 128, device="cuda")
+    run = lambda x: hip_ops.lightning_attention(x, state.clone(), decay, 4, 128, 128, starts, lens, slots, 1)  # noqa: E731
+    args = (decay, 4, 128, 128, state.clone(), starts, lens, slots, 1, torch.cuda.current_stream().cuda_stream)
+    assert _C.calls.lightning_attention(rows.as_subclass(Own), *args) is None
+    assert torch.equal(run(rows.as_subclass(Own)).as_subclass(torch.Tensor), run(rows))
+    errors = []
+    for calls in (_C.calls, None):
+        with monkeypatch.context() as m, pytest.raises(RuntimeError) as error:
+            m.setattr(_C, "calls", calls)
+            torch.vmap(run)(rows[None].expand(3, -1, -1))
+        errors.append(str(error.value))
+    assert errors[0] == errors[1]

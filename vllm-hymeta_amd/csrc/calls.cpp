@@ -1,7 +1,7 @@
 // The host side of attention and recurrence calls in native code: checks of the tensors, the argument structs, the outputs.  A small
 // step's kernels take 6 to 12 us, the same checks in Python 10 to 16 (some 60 attributes of tensors at 0.1 to 0.2 us each, 40 fields of a
 // struct).  A function here takes what its namesake in hip_ops.py accepts from plain tensors; whatever else it meets (a refused
-// shape or type, a tensor subclass, an exception) it answers with None, and the namesake goes on in Python, which raises what there
+// shape or type, a tensor subclass) it answers with None, and the namesake goes on in Python, which raises what there
 // is to raise.  It returns the output, or the library's status if that is not 0.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -42,6 +42,7 @@ struct Library {
   decltype(&hymeta_delta_rule_workspace_bytes) delta_bytes;
 } lib = {};
 PyObject* ops = nullptr;                         // hip_ops, whose _workspace is asked for by name on every call
+PyObject *torch_module = nullptr, *torch_empty = nullptr, *empty_name = nullptr;      // torch, its empty() at setup, and that name
 
 // A call's arguments, read in order.
 struct Args {
@@ -133,6 +134,27 @@ Room workspace(PyObject* like, size_t bytes, const char* tag) {
   Py_DECREF(buffer);
   need(room.bytes >= bytes);
   return room;
+}
+
+// torch.empty(shape, dtype=type, device=like.device): what stands under that name is asked, directly where that is torch's own.
+at::Tensor output(PyObject* like, const at::Tensor& as, std::initializer_list<int64_t> shape, at::ScalarType type) {
+  PyObject* empty = PyObject_GetAttr(torch_module, empty_name);
+  const bool own = empty == torch_empty;
+  Py_XDECREF(empty);
+  need(empty != nullptr);
+  if (own) return at::empty(at::IntArrayRef(shape), as.options().dtype(type));
+  PyObject *sizes = PyTuple_New(static_cast<Py_ssize_t>(shape.size())), *made = nullptr;
+  need(sizes != nullptr);
+  Py_ssize_t i = 0;
+  for (const int64_t n : shape) PyTuple_SET_ITEM(sizes, i++, PyLong_FromLongLong(n));
+  if (!PyErr_Occurred()) made = PyObject_CallMethod(ops, "_output", "OOi", like, sizes, type == at::kBFloat16 ? 1 : 0);
+  Py_DECREF(sizes);
+  need(made != nullptr);
+  at::Tensor out;
+  if (THPVariable_Check(made)) out = THPVariable_Unpack(made);
+  Py_DECREF(made);
+  need(out.defined() && out.is_contiguous() && out.scalar_type() == type && out.sizes().equals(at::IntArrayRef(shape)) && out.device() == as.device());
+  return out;
 }
 
 // The call itself, without the interpreter's lock as through ctypes.
@@ -231,7 +253,7 @@ PyObject* sink_attention(Args& in, PyObject* const* args) {
   } else {
     bytes = lib.sink_bytes(a.num_seqs, a.num_heads, G, Dv, longest);
   }
-  at::Tensor out = at::empty({T, H, Dv}, q.options());
+  at::Tensor out = output(args[0], q, {T, H, Dv}, q.scalar_type());
   a.out = out.mutable_data_ptr();
   if (bytes > 0) a.workspace = workspace(args[0], bytes, "sink_attention").data, a.workspace_bytes = bytes;      // (not what the buffer has grown to: a call's slices follow from the call)
   return launch(in, lib.sink_attention, a, stream, std::move(out));
@@ -277,7 +299,7 @@ PyObject* meta_swa_paged_decode(Args& in, PyObject* const* args) {
   a.cache_stride_block = kc.stride(0), a.cache_stride_pos = kc.stride(1), a.cache_stride_h = kc.stride(2), a.block_table_stride = tables.stride(0);
   if (mk != nullptr) a.meta_stride_t = mk->stride(0), a.meta_stride_h = mk->stride(1);
   a.scale = static_cast<float>(scale);
-  at::Tensor out = at::empty({B, H, D}, q.options());
+  at::Tensor out = output(args[0], q, {B, H, D}, at::kBFloat16);
   a.out = out.mutable_data_ptr();
   if (const size_t bytes = lib.paged_bytes(a.batch, a.num_heads, a.head_dim, splits)) {
     const Room room = workspace(args[0], bytes, "paged_decode");
@@ -318,7 +340,7 @@ PyObject* meta_swa_prefill(Args& in, PyObject* const* args) {
   a.scale = static_cast<float>(scale), a.max_seqlen_k = std::max(longest, 0);
   if (splits <= 0) splits = lib.prefill_splits(a.total_q, a.num_heads, a.num_meta, 0, window_left, a.max_seqlen_k);
   a.num_splits = splits;
-  at::Tensor out = at::empty({T, H, D}, q.options());
+  at::Tensor out = output(args[0], q, {T, H, D}, at::kBFloat16);
   a.out = out.mutable_data_ptr();
   if (splits > 1) {
     const Room room = workspace(args[0], lib.prefill_bytes(a.total_q, a.num_heads, splits), "swa_prefill");
@@ -361,7 +383,7 @@ PyObject* lightning_attention(Args& in, PyObject* const* args) {
   a.query_start_loc = s.starts, a.context_lens = s.context, a.slot_idx = s.slots;
   a.num_tokens = narrow(qkv.size(0)), a.num_seqs = s.count, a.num_heads = H, a.head_dim = D, a.v_dim = Dv, a.act_dtype = act_of(qkv), a.max_query_len = s.most;
   a.qkv_stride_t = qkv.stride(0);
-  at::Tensor out = at::empty({qkv.size(0), static_cast<int64_t>(H) * Dv}, qkv.options().dtype(at::kFloat));
+  at::Tensor out = output(args[0], qkv, {qkv.size(0), static_cast<int64_t>(H) * Dv}, at::kFloat);
   a.out = static_cast<decltype(a.out)>(out.mutable_data_ptr());
   if (const size_t bytes = lib.lightning_bytes(s.count, H, D, Dv, s.most)) {
     const Room room = workspace(args[0], bytes, "lightning");
@@ -387,7 +409,7 @@ PyObject* decay_scan(Args& in, PyObject* const* args) {
   a.num_tokens = narrow(T), a.num_seqs = s.count, a.num_heads = narrow(H), a.num_qk_heads = narrow(q.size(1)), a.head_dim = narrow(D), a.v_dim = narrow(Dv);
   a.act_dtype = act_of(q), a.max_query_len = s.most;
   a.q_stride_t = q.stride(0), a.k_stride_t = k.stride(0), a.v_stride_t = v.stride(0);
-  at::Tensor out = at::empty({T, H * Dv}, q.options().dtype(at::kFloat));
+  at::Tensor out = output(args[0], q, {T, H * Dv}, at::kFloat);
   a.out = static_cast<decltype(a.out)>(out.mutable_data_ptr());
   if (const size_t bytes = lib.decay_scan_bytes(s.count, a.num_heads, a.head_dim, a.v_dim, s.most)) {
     const Room room = workspace(args[0], bytes, "decay_scan");
@@ -414,7 +436,7 @@ PyObject* delta_rule(Args& in, PyObject* const* args) {
   a.num_tokens = narrow(T), a.num_seqs = s.count, a.num_heads = narrow(H), a.num_qk_heads = narrow(q.size(1)), a.head_dim = narrow(D), a.v_dim = narrow(Dv);
   a.act_dtype = act_of(q), a.max_query_len = s.most, a.q_scale = static_cast<float>(q_scale), a.unit_eps = static_cast<float>(unit_eps);
   a.q_stride_t = q.stride(0), a.k_stride_t = k.stride(0), a.v_stride_t = v.stride(0), a.beta_stride_t = beta.stride(0);
-  at::Tensor out = at::empty({T, H * Dv}, q.options().dtype(at::kFloat));
+  at::Tensor out = output(args[0], q, {T, H * Dv}, at::kFloat);
   a.out = static_cast<decltype(a.out)>(out.mutable_data_ptr());
   if (const size_t bytes = lib.delta_bytes(a.num_tokens, s.count, a.num_heads, a.num_qk_heads, a.head_dim, a.v_dim, a.act_dtype, s.most)) {
     const Room room = workspace(args[0], bytes, "delta_rule");
@@ -438,10 +460,14 @@ PyObject* setup(PyObject*, PyObject* const* args, Py_ssize_t n) {
       return nullptr;
     }
   }
-  std::memcpy(&lib, at, sizeof(lib));
+  PyObject *name = PyUnicode_InternFromString("empty"), *torch = PyObject_GetAttrString(args[0], "torch"), *empty = PyObject_GetAttrString(args[0], "_torch_empty");
+  if (name == nullptr || torch == nullptr || empty == nullptr) {
+    Py_XDECREF(name), Py_XDECREF(torch), Py_XDECREF(empty);
+    return nullptr;
+  }
+  std::memcpy(&lib, at, sizeof(lib));                // (what an earlier setup has left is not given back: calls may be under way)
   Py_INCREF(args[0]);
-  Py_XDECREF(ops);
-  ops = args[0];
+  ops = args[0], torch_module = torch, torch_empty = empty, empty_name = name;
   Py_RETURN_NONE;
 }
 

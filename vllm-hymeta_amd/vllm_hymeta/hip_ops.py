@@ -40,13 +40,17 @@ def _p(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
-_empty = torch.empty
+_torch_empty = torch.empty
 
 
 def _native(t: torch.Tensor):
-    """The native calls (csrc/calls.cpp), where they stand for what is below them here: for device tensors, and while outputs come from
-    torch itself (what is put in ``torch.empty``'s place is asked for them)."""
-    return _C.calls if t.is_cuda and torch.empty is _empty else None
+    """The native calls (csrc/calls.cpp), which stand for what is below them here, for device tensors."""
+    return _C.calls if t.is_cuda else None
+
+
+def _output(like: torch.Tensor, shape: Tuple[int, ...], bf16: bool) -> torch.Tensor:
+    """An output of the native calls, where something else than torch's own stands for ``torch.empty``."""
+    return torch.empty(*shape, dtype=torch.bfloat16 if bf16 else torch.float32, device=like.device)
 
 
 def _answer(out, what: str) -> torch.Tensor:
