@@ -89,3 +89,27 @@ def test_rows_that_a_ranks_experts_can_expect():
 def test_gate_up_projections_that_run_in_tiles(M, K, N, takes):
     from vllm_hymeta import _C
     assert _C.load().hymeta_bf16_gemm_takes(M, K, N, 1) == takes
+
+
+@pytest.mark.parametrize("experts,total,K,N,int8,pairs,takes", [
+    # from nine rows an expert on, but not columns or a K that no tile takes
+    (16, 16, 3584, 9472, 0, 128, 0), (16, 16, 3584, 9472, 0, 129, 1), (16, 16, 3584, 9472, 1, 128, 0), (16, 16, 3584, 9472, 1, 129, 1),
+    (16, 16, 3584, 9536, 0, 600, 0), (16, 16, 3616, 9472, 0, 600, 0), (16, 16, 3616, 9472, 1, 600, 0),
+    # experts that nearly fill one tile go without from a K of 5120 on, from 176 rows (448 tiles: three quarters of their last round of the chip)
+    (8, 8, 8192, 14336, 0, 1407, 1), (8, 8, 8192, 14336, 0, 1408, 0), (8, 8, 8192, 14336, 0, 1919, 0), (8, 8, 8192, 14336, 0, 1920, 1),
+    (8, 8, 5056, 14336, 0, 1600, 1), (8, 8, 5120, 14336, 0, 1600, 0), (8, 8, 8192, 14336, 1, 1600, 1),
+    # ... those that a rank's experts can expect
+    (8, 16, 8192, 14336, 0, 2815, 1), (8, 16, 8192, 14336, 0, 2816, 0), (8, 16, 8192, 14336, 0, 3840, 1),
+    # from 160 where the tiles fill the chip once, or their last round (256 and 512 tiles); never below 148 of them (120), or with 64 and
+    # fewer in the second round (288, 320, and 324)
+    (8, 8, 8192, 8192, 0, 1279, 1), (8, 8, 8192, 8192, 0, 1280, 0), (16, 16, 8192, 8192, 0, 2559, 1), (16, 16, 8192, 8192, 0, 2560, 0),
+    (4, 4, 8192, 7680, 0, 700, 1), (4, 4, 8192, 7680, 0, 900, 1), (8, 8, 8192, 9216, 0, 1900, 1), (8, 8, 8192, 10240, 0, 1900, 1),
+    (12, 12, 8192, 6912, 0, 2111, 1), (12, 12, 8192, 6912, 0, 2112, 0),
+])
+def test_products_with_the_activation_in_the_epilogue(experts, total, K, N, int8, pairs, takes):
+    """Which grouped products have their activation inside (``hymeta_moe_gemm_glu``), on either side of every limit."""
+    from vllm_hymeta import _C
+    a = _C.MoeGemmArgs()
+    a.max_rows, a.K, a.N, a.local_expert_end, a.x_stride_m, a.out_stride_m, a.w_stride_e = pairs, K << int8, N, experts, K << int8, N // 2, (K << int8) * N
+    a.operand_dtype = _C.HYMETA_I8 if int8 else _C.HYMETA_BF16
+    assert _C.load().hymeta_moe_gemm_glu_takes(C.byref(a), total) == takes

@@ -676,7 +676,8 @@ __global__ __launch_bounds__(64 * WM * WN, 512 / (64 * WM * WN)) void moe_gemm_t
 //
 // 16 experts of 3584 x 4736, a whole block on cold weights, in bf16 and int8 (tiles of 128 x 128 through registers, two steps ahead ->
 // these, us): 9 rows an expert 366 -> 339 and 241 -> 219, 40 392 -> 357 and 251 -> 237, 100 434 -> 399 and 286 -> 279; with tiles of 256 before, 150
-// 526 -> 452 and 327 -> 309, 170 515 -> 466 and 333 -> 322.  1.63 GB of bf16 are 326 us at 5 TB/s.
+// 526 -> 452 and 327 -> 309, 170 515 -> 466 and 333 -> 322.  The weights are 1.63 GB in bf16, 326 us from memory at 5 TB/s (a loop over one block finds
+// up to 256 MB of them in the last-level cache: 160 tokens 302).
 constexpr int kDeepRows = 256, kDeepCols = 128, kDeepStep = 128;              // (bytes of a row in a step)
 
 constexpr int kTiledMinRowsPerExpert = 8;           // up to here the kernels of 16 rows are ahead: 5 rows an expert 333 against 335 us in bf16, 187 against 216 in int8
@@ -958,8 +959,11 @@ MoeGemmKind moe_gemm_kind(int64_t max_rows, int experts, int total, int K, int N
     // An expert of fewer rows goes in one tile of the deep kernel, which is ahead while memory is the bound: until where depends on how
     // well the tiles of 256 (`once`, a row of them an expert) fill their last round of the chip.  Whole blocks in bf16, us, tiles
     // of 256 against these: 16 experts of 3584 x 4736 (592 and 224 tiles) 170 rows 515, 466; 190 513, 521; 8 of them (296 and 112) 190 341, 301,
-    // 235 357, 309; 8 of 8192 x 4096 (256 and 256) 150 498, 438; 170 448, 469; 4 of 5120 x 4736 (148) 150 312, 268; 170 260, 274.  The rows are
-    // those that a rank's experts can expect, not all pairs (8 of 16 experts of 3584 x 4736, 200 rows: 359, 309).
+    // 235 357, 309; 8 of 8192 x 4096 (256 and 256) 150 498, 438; 170 448, 469; 4 of 5120 x 4736 (148) 150 312, 268; 170 260, 274; 4 of
+    // 5120 x 3840 (120 and 80) 190 219, 195, 230 260, 199; 16 of 4096 x 4096 (512 and 256) 128 521, 403, 144 505, 418 (160 505); 8 of 3584 x
+    // 4608 (288 and 112) 190 335, 299, 230 349, 303.  In int8: 16 of 3584 x 4736 144 334, 314, 160 337, 324; 8 of them 175 222, 207, 230
+    // 234, 219; 8 of 8192 x 4096 144 317, 299.  The rows are those that a rank's experts can expect, not all pairs: 8 of 16 experts of 3584 x
+    // 4736, 200 rows: 359, 309; of 8192 x 7168 (448 and 256) 128 790, 733, 144 813, 734, 160 763, 744.
     const int64_t rows = max_rows / total, most = max_rows / experts, tiles = (most + 64 + 255) / 256 * experts * (N / 256);
     const int64_t once = experts * (N / 256), rest = once > 0 ? (once - 1) % 256 + 1 : 0;
     const bool few = rest < 148 && once <= 256, full = rest >= (once <= 256 ? 148 : 256);
@@ -1018,7 +1022,7 @@ bool moe_gemm_glu(const hymeta_moe_gemm_args& a, int num_experts) {
 }
 
 // What hymeta_moe_gemm_act has always taken: problems whose experts can expect to fill half a tile of 256, but for those of one nearly
-// full tile in bf16.
+// full tile in bf16.  For callers of that entry: the package asks moe_gemm_glu.
 bool moe_gemm_activates(const hymeta_moe_gemm_args& a, int num_experts) {
   if (!moe_gemm_glu(a, num_experts) || a.N % 256 != 0) return false;
   TileGemmArgs t = tile_args(a);
