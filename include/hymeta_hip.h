@@ -966,7 +966,8 @@ int hymeta_moe_gemm(const hymeta_moe_gemm_args* args, hymeta_stream_t stream);
  * out has N / 2 columns.  HYMETA_GEMM_ACT_SILU: silu(gate) up as hymeta_silu_and_mul gives it; _SILU_EXACT: as
  * hymeta_activation's HYMETA_ACT_SILU_MUL; _CLAMPED_GLU: its HYMETA_ACT_CLAMPED_GLU with limit and alpha -- of the bf16 rows
  * that hymeta_moe_gemm would write.  Problems that hymeta_moe_gemm_activates answers with 1 (many rows per expert), else
- * HYMETA_ERR_UNSUPPORTED. */
+ * HYMETA_ERR_UNSUPPORTED.  The package asks hymeta_moe_gemm_glu, which takes these problems and more: _act, _activates and
+ * _rank_activates keep their answers for callers of their own. */
 enum hymeta_gemm_act { HYMETA_GEMM_ACT_NONE = 0, HYMETA_GEMM_ACT_SILU = 1, HYMETA_GEMM_ACT_SILU_EXACT = 2, HYMETA_GEMM_ACT_CLAMPED_GLU = 3 };
 int hymeta_moe_gemm_act(const hymeta_moe_gemm_args* args, int32_t act, float limit, float alpha, hymeta_stream_t stream);
 int hymeta_moe_gemm_activates(const hymeta_moe_gemm_args* args);

@@ -608,8 +608,9 @@ __global__ __launch_bounds__(64 * NW, Summarise ? 4 : 2) void chunk_scan_kernel(
 // chunk; with the staging dealt among the products of the same waves 12000; so 8600), and 128 registers hold either half.
 // Two barriers a chunk (one in Summarise): behind the first the own weights and the next keys beside the state times the queries,
 // behind the second the next queries and values beside the weights times the values and the state's update.
-// Bound by vector instructions: silu and splits of 24576 values a chunk, 60 % of it.  28 heads of 128 x 128, lightning: one prompt of
-// 8192 rows 146 -> 121 us, four of 1000 91 -> 73, six of 1365 124 -> 99; plain decays: one of 8192 109 -> 95.
+// Bound by vector instructions (54 % of the time, the matrix pipe 21 %; silu and splits of 24576 values a chunk are most of them) and by
+// waits at the barriers (38 %).  28 heads of 128 x 128, lightning: one prompt of 8192 rows 149 -> 133 us, four of 2000 179 -> 142, six of 1365
+// 128 -> 106; plain decays: one of 8192 118 -> 103.
 template <int D, bool Silu, bool Summarise, bool Chained>
 __global__ __launch_bounds__(1024, 4) void chunk_scan_piped_kernel(ChunkScanArgs a, int seg_rows, int segments, bool short_too) {
   constexpr int NW = 8, NT = 64 * NW, KC = D / 8, VC = 2 * NW, KP = 2 * D, VP = 32 * NW, SD = D / 32, DB = D / 16;
@@ -1039,12 +1040,13 @@ void launch_chunk_scan_as(const ChunkScanArgs& a, ScanSegments sg, bool short_to
 }
 
 // Portions too short for a chunk run in the chunks' launch, where they cost no launch (about 4 us) and fill what a long portion
-// leaves idle.  That launch has registers for 8 waves on a compute unit, though: with states of 64 x 128 that is one workgroup's
-// 32 KB, and (head, short portion) pairs take 11.1 ns each where a launch of their own takes 10.  So those have one where there are
-// more pairs than kManyShort and the chunks fill half of the chip by themselves, or three times as many: 28 heads, 2048 rows beside
-// 255 single ones 139 -> 120 us, 40 portions of 40 beside 200 112 -> 97, but 300 beside 255 85 (91 apart).  Portions of one chunk that
-// seem to fill the chip may be many short ones of several rows, which gain more: a quarter as many pairs (60 of 7 rows beside 40).
-// States of 128 rows are level (23.4 and 25.6 ns).
+// leaves idle.  A workgroup of that launch has a compute unit to itself, though, and eight waves of its sixteen (heads of 64) do nothing for a
+// short portion.  So those of states of 64 x 128 have a launch of their own where there are
+// more (head, short portion) pairs than kManyShort and the chunks fill half of the chip by themselves, or three times as many: 28 heads, lightning, 2048 rows beside
+// 255 single ones 110 -> 87 us, 40 portions of 40 beside 200 92 -> 72, ten of 300 beside 250 104 -> 87, but four of 600 beside 60 38 (48 apart);
+// 300 beside 255 is level.  Portions of one chunk that seem to fill the chip may be many short ones of several rows, which gain more: a quarter as
+// many pairs (60 of 7 rows beside 40 of 64 96 -> 75).  (Sixteen waves moved the line: 2048 beside 127 would gain apart by now, 68 and 58, four of 600
+// beside 200 77 and 67.)  States of 128 rows are level.
 //
 // Where no portion has a chunk, theirs is the only launch, and its occupancy hides a row's round trips: 28 heads of 128 x 128, 64
 // portions of 7 rows 102 -> 58 us, 20 43 -> 25; of 64 x 128, 64 portions of 7 rows 77 -> 40 (a thread per value column, before: 156, 80,
