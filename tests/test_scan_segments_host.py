@@ -74,6 +74,7 @@ def test_every_cut_has_three_pieces_and_fits_the_workspace(program):
     (1, 300, 0, 28, 128, 0, 3), (2, 300, 0, 28, 128, 0, 1), (2, 300, 0, 16, 128, 0, 3), (3, 500, 0, 28, 128, 0, 3),
     (1, 256, 0, 56, 64, 0, 4), (2, 256, 0, 56, 64, 0, 1), (3, 400, 0, 56, 64, 0, 1), (3, 260, 0, 32, 64, 0, 3), (5, 450, 0, 28, 64, 0, 1),
     (1, 8192, 0, 28, 128, 1, 9), (1, 2048, 0, 16, 128, 0, 16), (1, 2048, 31, 16, 128, 0, 8), (1, 2048, 63, 7, 128, 0, 32),      # more than ten, beside short portions
+    (1, 2048, 0, 16, 64, 0, 32), (1, 2048, 63, 16, 64, 0, 8), (1, 2048, 63, 16, 64, 1, 32), (1, 2048, 100, 16, 64, 1, 8),
     (1, 2048, 0, 32, 64, 0, 8), (1, 2048, 0, 28, 64, 0, 16), (1, 1000, 255, 28, 128, 0, 4), (1, 575, 255, 28, 128, 0, 1),
 ])
 def test_which_portions_are_cut(program, portions, rows, singles, heads, columns, silu, pieces):

@@ -59,8 +59,8 @@ inline int scan_waves(int64_t lanes, int v_dim) {
 // More of them take the chain's launch and more states to and fro, which single rows and short portions wait for unless the chip is
 // through with a segment at once: in segments of one chunk, or alone (at least 192 rows each otherwise, but for the first ten).  2048
 // rows of 16 heads of 128 x 128, plain decays: alone 32.2 us in 16 segments, 36.0 in 8; beside 63 single rows 47.3 and 38.2; 7 heads,
-// lightning, beside 63 37.6 in 32 of one chunk, 45.5 in 8.  Where segments of 64 columns take two places on every compute unit (32 heads) 39.1 in
-// 16, 35.0 in 8.
+// lightning, beside 63 37.6 in 32 of one chunk, 45.5 in 8.  Where segments of 64 columns take two places on every compute unit: 32 heads alone
+// 39.1 in 16, 35.0 in 8; 16 heads, beside 63 37.8 in 32 of one chunk, 32.9 in 8, lightning 41.4 and 44.1, beside 100 45.6 and 43.9.
 constexpr int kMostUnchained = 10, kSegmentRows = 64, kManySegmentRows = 192, kManyColumns = 131072, kSomeColumns = 49152;
 struct ScanSegments {
   int rows = 0x7fffffff, count = 0;        // rows of a segment; bound on the segments' numbers
@@ -102,7 +102,9 @@ inline ScanSegments scan_segments(int num_tokens, int num_seqs, int num_heads, i
   auto pieces = [&] { return (max_query_len + rows - 1) / rows; };
   if (!many) {
     const int64_t slots = scan_slots(v_dim), slices = scan_slices(num_heads, v_dim);
-    if (pieces() > kMostUnchained && rows > kScanRows && (columns > kSomeColumns || (v_dim % 128 != 0 && 8 * portions * slices * pieces() > 7 * slots)))
+    const bool crowded = v_dim % 128 != 0 && 8 * portions * slices * pieces() > 7 * slots;
+    const bool beside = columns > (silu ? 2 : 1) * kSomeColumns;
+    if (pieces() > kMostUnchained && (rows > kScanRows ? crowded || beside : crowded && beside))
       rows = rows_of(std::max<int64_t>(kMostUnchained, std::min<int64_t>(fit, max_query_len / kManySegmentRows)));
     if (!scan_segments_pay(portions * slices * pieces() + (num_seqs - portions) * slices / 16, pieces(), num_heads, v_dim, max_query_len, rows, silu)) return sg;
   }
